@@ -33,7 +33,7 @@ const char* lgs_last_error_string(void);
 int lgs_version(void);
 
 /* y[z] (+)= act(a[z] w[z]^T + bias) for z < batch: a[z] = a + z stride_a (M rows of K, row stride lda), w[z] = w + z stride_w
- * ([N][K]), y[z] = y + z stride_y (row stride ldy). M <= 8: streaming GEMV; otherwise 128x128 MFMA tiles (bf16) or
+ * ([N][K]), y[z] = y + z stride_y (row stride ldy). M <= 8: streaming GEMV; otherwise MFMA tiles (bf16) or
  * 64x64 FMA tiles (fp32). z_start (batch + 1 bounds, device) makes it grouped: batch z owns rows
  * [z_start[z], z_start[z+1]) of a list of at most M rows; list row i reads A row a_rows[i] (or i) and writes Y row i
  * (stride_a and stride_y are then ignored for the rows' place). a_bf16: A is a producer's bf16 copy (MFMA tiles with
@@ -44,6 +44,8 @@ int lgs_version(void);
 int lgs_linear(const void* a, long lda, long stride_a, const void* w, int w_f32, long stride_w, void* y, long ldy,
                long stride_y, int M, int N, int K, int batch, int accumulate, int act, const int* a_rows,
                const int* z_start, int a_bf16, int y_bf16, const float* bias, float* part, int ksplit, lgs_stream_t stream);
+/* ranges of K that a plain product of a bf16 A on bf16 weights (M > 8 rows) is best made in; 1: as one */
+int lgs_linear_ksplit(int M, int N, int K);
 /* x[t] = table[tokens[t]] * scale */
 int lgs_embed(const int* tokens, const void* table, int w_f32, float scale, float* x, int T, int W, int vocab,
               lgs_stream_t stream);

@@ -1,0 +1,34 @@
+// The operands of lgs_linear and its large-tile form (seq_gemm.hip).
+#pragma once
+
+#include "seq_common.h"
+
+namespace lgs {
+
+struct LinArgs {
+  const float* a;
+  long lda, sa;
+  const void* w;
+  long sw;
+  float* y;
+  long ldy, sy;
+  int M, N, K;
+  int accumulate, act;
+  const int* a_rows;   // row r of the list reads A row a_rows[r] (null: r)
+  const int* z_start;  // batch z owns list rows [z_start[z], z_start[z + 1]) (null: rows [0, M) in every batch)
+  const uint16_t* a16;  // MFMA tiles only: A as bf16 (a producer's rounded copy) instead of fp32 `a`
+  uint16_t* y16;        // MFMA tiles only: Y written as bf16 (the operand of a following bf16 product), no accumulate
+  const float* bias;    // [N] added to the product ahead of the activation (null: none)
+  float* part;          // MFMA tiles only: partial sums [ksplit][M][N] of equal ranges of K, summed by lin_sum_kernel
+  int ksplit, kper;     // (ksplit 1: none); kper: BK-deep steps per range
+};
+
+// Which tile form and how many ranges of K a product of bf16 A and W takes on the pipelined tiles (seq_gemm.hip); tile
+// -1: not one of theirs (K is no multiple of 64). Rows of A and W start on 16 bytes. ksplit 0: the plan's own choice.
+struct GemmPlan {
+  int tile, ksplit;
+};
+GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit);
+int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream);
+
+}  // namespace lgs

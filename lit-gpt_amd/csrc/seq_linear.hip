@@ -1,37 +1,20 @@
 // Linear layers, embedding and RMS norms of the layered models: fp32 activations, bf16 or fp32 weights.
 //
 //   lgs_linear     Y[z] (+)= act(A[z] W[z]^T + bias): one entry point for every projection. Up to 8 rows run a streaming
-//                  GEMV (a wave per pair of output columns, 16-B weight loads, fp32 sums); more rows run 128x128
-//                  tiles of v_mfma_f32_16x16x32_bf16 (bf16 weights; A is rounded to bf16 while it is staged into
-//                  LDS) or 64x64 fp32 FMA tiles (fp32 weights). `batch` with strides runs per-head products (the
+//                  GEMV (a wave per pair of output columns, 16-B weight loads, fp32 sums); more rows run the
+//                  pipelined tiles of seq_gemm.hip (A a producer's bf16 copy, K a multiple of 64, aligned rows), 128x128
+//                  tiles of v_mfma_f32_16x16x32_bf16 (other bf16 products; an fp32 A is rounded to bf16 while it is
+//                  staged into LDS) or 64x64 fp32 FMA tiles (fp32 weights). `batch` with strides runs per-head products (the
 //                  latent attention's absorbed key and value maps); `z_start` / `a_rows` make it a grouped product
 //                  over row ranges of a sorted list (sparse experts during a prompt).
 //   lgs_embed      x[t] = table[token[t]] * scale
 //   lgs_rmsnorm    y = x / sqrt(mean(x^2) + eps) * (offset + w), rows with strides (whole rows, or heads)
-#include "seq_common.h"
+#include "seq_gemm.h"
 
 namespace lgs {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-struct LinArgs {
-  const float* a;
-  long lda, sa;
-  const void* w;
-  long sw;
-  float* y;
-  long ldy, sy;
-  int M, N, K;
-  int accumulate, act;
-  const int* a_rows;   // row r of the list reads A row a_rows[r] (null: r)
-  const int* z_start;  // batch z owns list rows [z_start[z], z_start[z + 1]) (null: rows [0, M) in every batch)
-  const uint16_t* a16;  // MFMA tiles only: A as bf16 (a producer's rounded copy) instead of fp32 `a`
-  uint16_t* y16;        // MFMA tiles only: Y written as bf16 (the operand of a following bf16 product), no accumulate
-  const float* bias;    // [N] added to the product ahead of the activation (null: none)
-  float* part;          // MFMA tiles only: partial sums [ksplit][M][N] of equal ranges of K, summed by lin_sum_kernel
-  int ksplit, kper;     // (ksplit 1: none); kper: BK-deep steps per range
-};
 
 // ------------------------------------------------------------------------------------------------ GEMV, M <= 8
 // R output columns per wave: 4 for tall matrices (more loads in flight per lane), fewer for short ones (more waves)
@@ -510,17 +493,26 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
     lgs::lin_fma_kernel<true><<<grid, 256, 0, stream>>>(p);
     LGA_LAUNCH_RETURN();
   }
+  const int am = a_bf16 ? 8 : 4;  // elements per 16 bytes of A
+  const bool vec = K % 8 == 0 && lda % am == 0 && stride_a % am == 0 && stride_w % 8 == 0 && (uintptr_t)a % 16 == 0 &&
+                   (uintptr_t)w % 16 == 0;
   if (ksplit > 1) {
     const int nk = (K + lgs::BK - 1) / lgs::BK;
     p.part = part;
     p.kper = (nk + ksplit - 1) / ksplit;
     p.ksplit = (nk + p.kper - 1) / p.kper;  // (no empty range)
   }
+  if (a_bf16 && vec) {
+    const lgs::GemmPlan plan = lgs::gemm_plan(M, N, K, batch, z_start != nullptr, p.ksplit);
+    if (plan.tile >= 0) {
+      const int rc = lgs::gemm_launch(p, plan, batch, stream);
+      if (rc) return rc;
+      if (p.ksplit > 1) lgs::lin_sum_kernel<<<dim3((N + 255) / 256, M), 256, 0, stream>>>(p);
+      LGA_LAUNCH_RETURN();
+    }
+  }
   const dim3 grid((N + lgs::BN - 1) / lgs::BN, (M + lgs::BM - 1) / lgs::BM, p.ksplit > 1 ? p.ksplit : batch);
   LGA_CHECK_ARG(grid.y <= 65535, "lgs_linear: too many rows");
-  const int am = a_bf16 ? 8 : 4;  // elements per 16 bytes of A
-  const bool vec = K % 8 == 0 && lda % am == 0 && stride_a % am == 0 && stride_w % 8 == 0 && (uintptr_t)a % 16 == 0 &&
-                   (uintptr_t)w % 16 == 0;
   if (a_bf16) {
     if (vec) lgs::lin_mfma_kernel<true, true><<<grid, 256, 0, stream>>>(p);
     else lgs::lin_mfma_kernel<false, true><<<grid, 256, 0, stream>>>(p);
@@ -530,6 +522,11 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
   }
   if (p.ksplit > 1) lgs::lin_sum_kernel<<<dim3((N + 255) / 256, M), 256, 0, stream>>>(p);
   LGA_LAUNCH_RETURN();
+}
+
+// ranges of K that a plain product of a bf16 A on bf16 weights is best made in (1: as one)
+extern "C" int lgs_linear_ksplit(int M, int N, int K) {
+  return M > 8 && M <= 65535 && N > 0 && K > 0 ? lgs::gemm_plan(M, N, K, 1, false, 0).ksplit : 1;
 }
 
 extern "C" int lgs_embed(const int* tokens, const void* table, int w_f32, float scale, float* x, int T, int W,

@@ -273,7 +273,7 @@ class SandwichSublayer(nn.Module):
             n_in = self.w_in.shape[0]
             proj = torch.empty(T, n_in, dtype=torch.float32, device=src.device)
             seq_ops.linear(src, self.w_in, M=T, N=n_in, K=W, y=proj, lda=W, ldy=n_in, bias=self.b_in,
-                           ksplit=seq_ops.thin_ksplit(T, n_in, W, self.w_in))
+                           ksplit=0 if src.dtype == torch.bfloat16 else seq_ops.thin_ksplit(T, n_in, W, self.w_in))
         y = torch.empty(T, W, dtype=torch.float32, device=src.device)
         if cache is None:
             self.module(proj, h, y, h16=h16, accumulate=False)

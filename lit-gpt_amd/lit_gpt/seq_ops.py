@@ -32,6 +32,7 @@ SIGNATURES = {
     "lgs_version": [],
     "lgs_last_error_string": [],
     "lgs_linear": [_P, _L, _L, _P, _I, _L, _P, _L, _L, _I, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _P, _I, _P],
+    "lgs_linear_ksplit": [_I, _I, _I],
     "lgs_embed": [_P, _P, _I, _F, _P, _I, _I, _I, _P],
     "lgs_rmsnorm": [_P, _L, _P, _F, _F, _P, _L, _I, _I, _I, _P, _P],
     "lgs_gather_rows": [_P, _P, _P, _I, _I, _P],
@@ -150,12 +151,13 @@ def linear(a: torch.Tensor, w: torch.Tensor, *, M: int, N: int, K: int, y: torch
            y_off: int = 0, ldy: int, batch: int = 1, stride_a: int = 0, stride_w: int = 0, stride_y: int = 0,
            accumulate: bool = False, act: int = ACT_NONE, a_rows: Optional[torch.Tensor] = None,
            z_start: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
-           ksplit: int = 1) -> torch.Tensor:
+           ksplit: int = 0) -> torch.Tensor:
     """y[z] (+)= act(a[z] w[z]^T + bias) over ``batch`` strided operands; offsets and strides count elements. With
     ``z_start`` (batch + 1 int32 row bounds) batch z owns that range of a row list of at most M rows, whose A rows
     are ``a_rows`` (or the list places themselves) and whose Y rows are the list places. ``a`` may be a producer's
     bf16 copy (``rmsnorm(bf16_copy=True)``, ``glu(bf16=True)``) for the MFMA tiles with bf16 weights. ``ksplit`` > 1: that
-    many ranges of K side by side (MFMA tiles, one plain product), see ``thin_ksplit``."""
+    many ranges of K side by side (MFMA tiles, one plain product), see ``thin_ksplit``; 0: as many as suit a bf16 ``a``,
+    one otherwise."""
     a16 = a.dtype == torch.bfloat16
     ap = _dev(a, "a", torch.bfloat16 if a16 else F32) + (2 if a16 else 4) * a_off
     y16 = y.dtype == torch.bfloat16  # the result feeds another bf16 product
@@ -166,6 +168,9 @@ def linear(a: torch.Tensor, w: torch.Tensor, *, M: int, N: int, K: int, y: torch
         raise ValueError("linear: an operand is smaller than the sizes and strides say")
     if bias is not None and bias.numel() != N:
         raise ValueError("linear: one bias per output column")
+    if ksplit == 0:
+        plain = a16 and batch == 1 and a_rows is None and z_start is None
+        ksplit = load_library().lgs_linear_ksplit(M, N, K) if plain else 1
     part = torch.empty(ksplit * M * N, dtype=F32, device=y.device) if ksplit > 1 else None
     _check(load_library().lgs_linear(ap, lda, stride_a, _dev(w, "w"), _wf32(w, "w"), stride_w, yp, ldy, stride_y,
                                      M, N, K, batch, int(accumulate), act, _opt(a_rows, "a_rows", I32),

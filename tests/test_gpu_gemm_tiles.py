@@ -1,0 +1,81 @@
+"""The pipelined tiles of the layered models' products (csrc/seq_gemm.hip) against float64, at the edges of their forms.
+
+Every sum has K products of bf16 values, exact in fp32, added in fp32: with |a w| ~ K^-1/2 the error of a result is at
+most about K additions of half a unit in the last place of partial sums around 1, 2e-5 at the largest K here.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-5
+
+
+def operands(M, N, K, dev, seed=0):
+    g = torch.Generator(device=dev).manual_seed(seed + 7 * M + N)
+    a = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    return a, w, torch.randn(N, generator=g, device=dev)
+
+
+# one row past and one short of whole tiles of 64, 128 and 256 rows and 128 and 256 columns; the shortest K; products that
+# fill the chip with the largest form; odd columns
+@pytest.mark.parametrize("M,N,K", [(9, 1, 64), (64, 128, 64), (65, 129, 128), (127, 255, 192), (129, 257, 320),
+                                   (255, 1023, 64), (257, 4097, 256), (513, 12288, 192), (2047, 8200, 448),
+                                   (2305, 10241, 1024), (40, 6144, 4096), (700, 2048, 5632)])
+@pytest.mark.parametrize("ksplit", [0, 1, 3])
+def test_product(M, N, K, ksplit):
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    a, w, b = operands(M, N, K, dev)
+    want = a.double() @ w.double().T
+    pad = torch.full((M, N + 3), 2.0, device=dev)  # (rows apart: nothing may be written between them)
+    seq_ops.linear(a, w, M=M, N=N, K=K, y=pad, lda=K, ldy=N + 3, bias=b, accumulate=True, ksplit=ksplit)
+    assert (pad[:, :N].double() - 2.0 - b.double() - want).abs().max() < TOL
+    assert (pad[:, N:] == 2.0).all()
+    y = torch.full((M, N), float("nan"), device=dev)
+    seq_ops.linear(a, w, M=M, N=N, K=K, y=y, lda=K, ldy=N, ksplit=ksplit)
+    assert (y.double() - want).abs().max() < TOL
+    y16 = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+    seq_ops.linear(a, w, M=M, N=N, K=K, y=y16, lda=K, ldy=N, bias=b, act=seq_ops.ACT_SILU, ksplit=ksplit)
+    z = want + b.double()
+    z = z * torch.sigmoid(z)
+    assert ((y16.double() - z).abs() <= 2.0 ** -8 * z.abs() + TOL).all()  # one rounding to bf16
+
+
+@pytest.mark.parametrize("rows", [[0, 1, 0, 300], [128, 129, 127, 0], [5] * 70, [700, 0, 513, 64, 1]])
+@pytest.mark.parametrize("gather", [False, True])
+def test_grouped_product(rows, gather):
+    """Every group its own matrix and range of rows, some of them empty; rows gathered from a shorter list."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    E, M, N, K = len(rows), sum(rows), 260, 192
+    a, w, _ = operands(M, E * N, K, dev)
+    w = w.view(E, N, K)
+    start = torch.tensor([0] + rows).cumsum(0).to(torch.int32).to(dev)
+    pick = torch.randint(0, M, (M,), device=dev, dtype=torch.int32) if gather else None
+    y = torch.full((M + 1, N), 3.0, device=dev)
+    seq_ops.linear(a, w, M=M, N=N, K=K, y=y, lda=K, ldy=N, batch=E, stride_w=N * K, z_start=start, a_rows=pick)
+    src = a.double() if pick is None else a.double()[pick.long()]
+    for e in range(E):
+        lo, hi = int(start[e]), int(start[e + 1])
+        assert ((y[lo:hi].double() - src[lo:hi] @ w[e].double().T).abs() < TOL).all()
+    assert (y[M:] == 3.0).all()
+
+
+def test_strided_batch():
+    """Products side by side, A in columns of wider rows, K in one and in several stages."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    for K in (64, 512):
+        Z, M, N = 5, 130, 96
+        a, w, _ = operands(M, Z * N, K * Z, dev)
+        w = w.view(Z, N, Z * K)[:, :, :K].contiguous()
+        y = torch.zeros(M, Z * N, device=dev)
+        seq_ops.linear(a, w, M=M, N=N, K=K, y=y, lda=Z * K, ldy=Z * N, batch=Z, stride_a=K, stride_w=N * K, stride_y=N)
+        for z in range(Z):
+            want = a[:, z * K:(z + 1) * K].double() @ w[z].double().T
+            assert (y[:, z * N:(z + 1) * N].double() - want).abs().max() < TOL
