@@ -22,11 +22,12 @@
 //                         optionally rotated by their position) into the cache. In a step of one token per sequence
 //                         the workgroup whose token completes a pooled block also makes the block's means.
 //   lgs_pool_blocks       the same means for the blocks that a prompt step completes.
-//   lgs_diffattn,         QT consecutive queries of one sequence and one head per workgroup (8 with two maps, 16 with
-//   lgs_sinkattn          one) against key tiles of 256 cached rows: a thread per key for the scores, an online
+//   lgs_diffattn,         prompts over bf16 caches of the usual sizes: the matrix-core form of seq_attn_tiles.hip. Others:
+//   lgs_sinkattn          QT consecutive queries of one sequence and one head per workgroup (8 with two maps, 16 with
+//                         one) against key tiles of 256 cached rows: a thread per key for the scores, an online
 //                         softmax per (query, map), a thread per value column for the weighted sums. One query per
 //                         workgroup (decode) can spread its keys over several workgroups, merged by a second launch.
-#include "seq_common.h"
+#include "seq_attn.h"
 
 #include <type_traits>
 
@@ -233,29 +234,6 @@ __global__ void __launch_bounds__(256) pool_blocks_kernel(PoolArgs p) {
   pool_block<CF32>(p.cache_k, p.cache_v, p.pool_k, p.pool_v, (size_t)p.seq_slot[b], blk, p.pool, p.S, p.pool_rows, p.G * p.d,
                    p.G * p.dv);
 }
-
-struct AttnArgs {
-  const float* q;  // prepared queries at q + row * ld + h * MAPS d
-  long ld;
-  const void* cache_k;
-  const void* cache_v;
-  const int *seq_start, *seq_slot, *seq_pos0;
-  float* out;       // [T][H * dv]
-  uint16_t* out16;  // optional bf16 copy
-  float* part;      // splits > 1: [T][H][splits][MAPS (2 + dv)]
-  int H, G, d, dv, S, chunk, tiles;
-  float scale, cap, lambda, eps, post;
-  const float* sink;  // one map: exp(sink[h]) joins the softmax normaliser (NULL: no sink)
-  const float* gate;  // one map: the head's output is multiplied by sigmoid(gate[row * ldg + h]) (NULL: not)
-  long ldg;
-  int gate_cols;      // 1: a gate per head (above); else one per output column, gate[row * ldg + h * dv + c]
-  int window;         // one map: a query sees the last `window` positions (0: all before it)
-  const float *pool_k, *pool_v;  // one map: pooled blocks [slots][pool_rows][G][d], [..][dv] before the window
-  int pool, pool_rows;           // (pool 0: none)
-  const float* v_freq;  // one map, [dv / 2]: the finished output is turned back by the query's position (values are
-  int interleaved;      // cached rotated), pairs (2m, 2m + 1) or (m, m + dv / 2)
-  const float* score_bias;  // [H]: sigmoid weights, each sigmoid(score + score_bias[h]) (null: softmax)
-};
 
 // pooled blocks that the query at position i sees: those wholly before its window
 __device__ __forceinline__ int pooled_seen(int i, int window, int pool) {
@@ -645,6 +623,12 @@ extern "C" int lgs_diffattn(const float* q, long ld, const void* cache_k, const 
     rc = lgs::diffattn_launch<1, 2>(p, cache_f32, dim3(B, H, splits), stream);
     if (rc == 0 && splits > 1) lgs::diffattn_combine_kernel<2><<<dim3(B, H), 256, 0, stream>>>(p, splits);
   } else {
+    if (!cache_f32 && lgs::attn_tiles_fit(p, 2, 1, max_len)) {
+      const lgs::AttnTileArgs t{p, (const uint16_t*)cache_k, (const uint16_t*)cache_v, 2L * G * d, (long)G * dv, 0, 0};
+      rc = lgs::attn_tiles_launch(t, 2, 1, B, max_len, stream);
+      if (rc) return rc;
+      LGA_LAUNCH_RETURN();
+    }
     p.tiles = (max_len + 7) / 8;
     LGA_CHECK_ARG((long)B * p.tiles < (1L << 31), "lgs_diffattn: too many tiles");
     rc = lgs::diffattn_launch<8, 2>(p, cache_f32, dim3(B * p.tiles, H, 1), stream);
@@ -718,6 +702,12 @@ extern "C" int lgs_sinkattn(const float* q, long ld, const void* cache_k, const 
     rc = lgs::diffattn_launch<1, 1>(p, cache_f32, dim3(B, H, splits), stream);
     if (rc == 0 && splits > 1) lgs::diffattn_combine_kernel<1><<<dim3(B, H), 256, 0, stream>>>(p, splits);
   } else {
+    if (!cache_f32 && lgs::attn_tiles_fit(p, 1, 1, max_len)) {
+      const lgs::AttnTileArgs t{p, (const uint16_t*)cache_k, (const uint16_t*)cache_v, (long)G * d, (long)G * dv, 0, 0};
+      rc = lgs::attn_tiles_launch(t, 1, 1, B, max_len, stream);
+      if (rc) return rc;
+      LGA_LAUNCH_RETURN();
+    }
     p.tiles = (max_len + 15) / 16;
     LGA_CHECK_ARG((long)B * p.tiles < (1L << 31), "lgs_sinkattn: too many tiles");
     rc = lgs::diffattn_launch<16, 1>(p, cache_f32, dim3(B * p.tiles, H, 1), stream);

@@ -1,0 +1,424 @@
+// Prompt attention of the layered models on the bf16 matrix cores, with the results of fp32 products: every fp32
+// operand is the exact sum of bf16 summands (the upper 8 bits of its significand, the next 8, the last 8), products of
+// bf16 values are exact in fp32, and all sums are fp32. Queries and weights have three summands beside keys and values
+// that are bf16 themselves (a cache); keys and values in two summands (16 bits of their significands) meet two of the
+// query and three of the weight.
+//
+// A workgroup of 8 waves takes 32 queries (or 64, 128) of the heads that share one key head; key tiles of 64 positions
+// stream through LDS (range-checked LDS-DMA, ST stages: rows past the last visible key arrive as zeros) once for all of
+// them. Per 32 keys a wave forms S^T = K Q^T (A: key rows from LDS, B: the query summands in registers), so that a lane
+// holds the scores of one query: maximum, normaliser and rescale are its own. The weights' summands are the B operand of
+// O^T += V^T P^T as they stand: the transposed LDS reads of V take the keys in the order in which a lane holds them.
+// Unless eight (head, map) pairs share the keys, two waves split every key tile and are merged at the end.
+//
+// Bound by latency inside a wave (scores -> maximum -> exponentials -> weights), then by the matrix cores' rate at three
+// times the products that bf16 operands would take.
+#include "seq_attn.h"
+
+namespace lgs {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+typedef short i16x8_t __attribute__((ext_vector_type(8)));
+
+constexpr int kTileKeys = 64;
+
+// 16-byte chunk `ch` of row `row` in an LDS tile of `chunks` a row: permuted so that neither 32 rows' same chunk nor the
+// transposed reads meet in a bank
+__device__ __forceinline__ int chunk_swizzle(int row, int chunks) {
+  return chunks == 8 ? (((row & 3) << 1) | ((row >> 2) & 1)) : (((row & 3) << 2) | ((row >> 2) & 3));
+}
+
+// the next summands of eight fp32 values as one operand: the upper half of every value, which is taken off it
+__device__ __forceinline__ bf16x8_t take_summand(float (&x)[8]) {
+  u32x4_t o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t a = __float_as_uint(x[2 * e]), b = __float_as_uint(x[2 * e + 1]);
+    o[e] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    x[2 * e] -= __uint_as_float(a & 0xFFFF0000u);
+    x[2 * e + 1] -= __uint_as_float(b & 0xFFFF0000u);
+  }
+  return __builtin_bit_cast(bf16x8_t, o);
+}
+
+// e^x for x <= 0 (about one unit in the last place): 2^t for the rounded product, times the rounding's own power
+__device__ __forceinline__ float exp_neg(float x) {
+  const float t = x * 1.44269502f;
+  float r = fmaf(x, 1.44269502f, -t);
+  r = fmaf(x, 1.92596299e-8f, r);
+  const float e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, r * 0.69314718f, e);
+}
+
+// tanh x: below 0.625 the odd polynomial of the Cephes library's tanhf, above 1 - 2 / (e^2|x| + 1) (2e-7 relative)
+__device__ __forceinline__ float tanh_near(float x) {
+  const float z = x * x, y = fabsf(x);
+  float p = fmaf(-5.70498872745e-3f, z, 2.06390887954e-2f);
+  p = fmaf(p, z, -5.37397155531e-2f);
+  p = fmaf(p, z, 1.33314422036e-1f);
+  p = fmaf(p, z, -3.33332819422e-1f);
+  p = fmaf(p * z, x, x);
+  const float e = __builtin_amdgcn_exp2f(y * 2.88539008f);
+  const float q = copysignf(fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f), x);
+  return y < 0.625f ? p : q;
+}
+
+// 1 / (1 + e^-z) from e^-|z|
+__device__ __forceinline__ float sigmoid_near(float z) {
+  const float e = exp_neg(-fabsf(z)), d = 1.0f + e;
+  const float r = __builtin_amdgcn_rcpf(d), p = fmaf(fmaf(-d, r, 1.0f), r, r);
+  return z >= 0.0f ? p : e * p;
+}
+
+// DC: 16-wide pieces of one map's key, DT: 32-wide pieces of a value, MAPS: maps per head, PARTS: summands of keys and
+// values, SIG: sigmoid weights, ST: stages. grid (B * tiles, key heads * H / (G heads))
+template <int DC, int DT, int MAPS, int PARTS, bool SIG, int ST>
+__global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
+  constexpr int CHK = MAPS * PARTS * DC * 2, CHV = PARTS * DT * 4;  // 16-byte chunks per row
+  constexpr int STAGE = kTileKeys * 16 * (CHK + CHV);
+  constexpr int PU = (CHK + CHV) / 8;  // DMAs per wave and stage (1 KB each)
+  constexpr int QP = PARTS == 1 ? 3 : 2, DV = DT * 32;
+  static_assert(CHK % 8 == 0 && CHV % 8 == 0 && (CHK == 8 || CHK % 16 == 0) && (CHV == 8 || CHV % 16 == 0), "rows");
+  constexpr int kExchange = 4 * 64 * (DT * 16 + 2) * 4, kTurn = 4 * 32 * (DV + 4) * 4;
+  constexpr int kLds = ST * STAGE > kExchange ? (ST * STAGE > kTurn ? ST * STAGE : kTurn)
+                                              : (kExchange > kTurn ? kExchange : kTurn);
+  static_assert(kLds <= 163840, "LDS");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
+  const AttnArgs& a = p.a;
+  const int tid = threadIdx.x, lane = tid & 63, lq = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nv = p.heads * MAPS, KS = nv == 8 ? 1 : 2, QW = 8 / (nv * KS);
+  const int vh = wave % nv, ks = wave / nv % KS, qw = wave / (nv * KS);
+  const int map = MAPS == 2 ? vh & 1 : 0;
+  const int groups = a.H / p.heads, group = blockIdx.x % groups, at_b = blockIdx.x / groups, B = gridDim.x / groups / a.tiles;
+  const int h = group * p.heads + vh / MAPS, g = h / (a.H / a.G);
+  const int b = at_b % B, tile = a.tiles - 1 - at_b / B;
+  const int rfirst = a.seq_start[b] + tile * 32 * QW, rend = a.seq_start[b + 1];
+  if (rfirst >= rend) return;
+  const int wgq = min(32 * QW, rend - rfirst);
+  const int pos_first = a.seq_pos0[b] + tile * 32 * QW, pos_last = min(pos_first + wgq - 1, a.S - 1);
+  auto lowest = [&](int pos) {
+    return a.window > 0 ? max(0, pos - a.window + 1) : (a.chunk > 0 ? pos - pos % a.chunk : 0);
+  };
+  const int kt0 = lowest(pos_first) / kTileKeys, nkt = pos_last / kTileKeys + 1;
+  // this lane's query
+  const int row = rfirst + qw * 32 + lq;
+  const bool live = row < rend;
+  const int qpos = live ? pos_first + qw * 32 + lq : -1, qlo = live ? lowest(qpos) : 0;
+  // what the wave's queries see in all (positions ascend over the lanes)
+  const int nlive = min(32, max(0, rend - rfirst - qw * 32));
+  const int wfirst = pos_first + qw * 32, wlast = nlive > 0 ? wfirst + nlive - 1 : -1;
+  const int wlo = lowest(wfirst), whi_lo = nlive > 0 ? lowest(wlast) : 0;
+
+  // key and value rows: a buffer that ends after the last visible key
+  const size_t row0 = p.packed ? (size_t)a.seq_start[b] : (size_t)a.seq_slot[b] * a.S;
+  const uint16_t* kbase = p.k + row0 * p.krow + (size_t)g * (MAPS * PARTS * DC * 16);
+  const uint16_t* vbase = p.v + row0 * p.vrow + (size_t)g * (PARTS * DV);
+  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)kbase, (short)0, (int)((long)pos_last * p.krow * 2 + CHK * 16), 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)vbase, (short)0, (int)((long)pos_last * p.vrow * 2 + CHV * 16), 0x00020000);
+  int voff[PU];
+#pragma unroll
+  for (int i = 0; i < PU; ++i) {
+    const int u = wave * PU + i;
+    const bool isv = u >= CHK;
+    const int idx = (isv ? u - CHK : u) * 64 + lane, n = isv ? CHV : CHK;
+    const int r = idx / n, ch = (idx % n) ^ chunk_swizzle(r, n);
+    voff[i] = (int)((isv ? p.vrow : p.krow) * 2) * r + ch * 16;
+  }
+  auto stage = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < PU; ++i) {
+      const int u = wave * PU + i;
+      const bool isv = u >= CHK;
+      const int off = voff[i] + kt * kTileKeys * (int)((isv ? p.vrow : p.krow) * 2);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(isv ? vrs : krs,
+                                               (__attribute__((address_space(3))) void*)(lds + buf * STAGE + u * 1024), 16,
+                                               off, 0, 0, 0);
+    }
+  };
+
+  bf16x8_t q[QP][DC];
+  {
+    const float* qr = a.q + (size_t)min(row, rend - 1) * a.ld + ((size_t)h * MAPS + map) * (DC * 16) + 8 * hh;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      const float4 lo = *(const float4*)(qr + c * 16), hi = *(const float4*)(qr + c * 16 + 4);
+      float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+      for (int s = 0; s < QP; ++s) q[s][c] = take_summand(x);
+    }
+  }
+  // LDS addresses: key row lq; transposed value rows (16-lane group grp, quad qq, pair pp) of the keys that a lane's
+  // weights belong to: 4 hh + 0 .. 3 and 8 + 4 hh + 0 .. 3 of 16
+  static_assert(MAPS == 1 || (PARTS == 1 && DC == 4), "the second map's chunks are the upper eight of sixteen");
+  const int kaddr = lq * (CHK * 16) + 16 * (chunk_swizzle(lq, CHK) ^ (hh | (map * 8)));
+  const int qq = (lane & 15) >> 2, pp = lane & 3, grp = lane >> 4;
+  const int vr0 = 4 * (grp >> 1) + qq, vr1 = vr0 + 8, vch = 2 * (grp & 1) + (pp >> 1);
+  const int vaddr0 = vr0 * (CHV * 16) + 16 * (chunk_swizzle(vr0, CHV) ^ vch) + 8 * (pp & 1);
+  const int vaddr1 = vr1 * (CHV * 16) + 16 * (chunk_swizzle(vr1, CHV) ^ vch) + 8 * (pp & 1);
+  auto at = [](int addr, int ch) {  // the chunk that is ch (whose bits the lane's own chunk does not have) further
+    return (addr ^ (16 * (ch & 15))) + 256 * (ch >> 4);
+  };
+  f32x16_t o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
+  float m = SIG ? 0.0f : -INFINITY, l = 0.0f;  // l: over the keys that this lane holds
+  const float bias = SIG ? a.score_bias[h] : 0.0f, inv_cap = a.cap > 0.0f ? 1.0f / a.cap : 0.0f;
+
+  auto keys32 = [&](const unsigned char* K, const unsigned char* V, int k0) {
+    f32x16_t s, lo;  // the leading summands' products and the others'
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.0f, lo[r] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      const bf16x8_t k = *(const bf16x8_t*)(K + at(kaddr, 2 * c));
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, q[0][c], s, 0, 0, 0);
+      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, q[1][c], lo, 0, 0, 0);
+      if (PARTS == 1) {
+        lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, q[QP - 1][c], lo, 0, 0, 0);
+      } else {
+        const bf16x8_t k1 = *(const bf16x8_t*)(K + at(kaddr, DC * 2 + 2 * c));
+        lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, q[0][c], lo, 0, 0, 0);
+      }
+    }
+    const bool edge = k0 + 31 > wfirst || k0 < whi_lo;  // some query of the wave does not see all of these
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float v = (s[r] + lo[r]) * a.scale;
+      if (a.cap > 0.0f) v = a.cap * tanh_near(v * inv_cap);
+      if (edge) {
+        const int key = k0 + (r & 3) + 8 * (r >> 2) + 4 * hh;
+        if (key > qpos || key < qlo) v = -INFINITY;
+      }
+      s[r] = v;
+      if (!SIG) mx = fmaxf(mx, v);
+    }
+    float mref = 0.0f;
+    if (!SIG) {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      const float mn = fmaxf(m, mx);
+      mref = mn == -INFINITY ? 0.0f : mn;
+      if (!__all(mn == m)) {
+        const float f = m == -INFINITY ? 0.0f : exp_neg(m - mref);
+        l *= f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[t][r] *= f;
+      }
+      m = mn;
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      float w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = s[8 * kk + e];
+        w[e] = v == -INFINITY ? 0.0f : (SIG ? sigmoid_near(v + bias) : exp_neg(v - mref));
+        if (!SIG) l += w[e];
+      }
+      bf16x8_t pw[3];
+#pragma unroll
+      for (int e = 0; e < 3; ++e) pw[e] = take_summand(w);
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int part = 0; part < PARTS; ++part) {
+          typedef __attribute__((address_space(3))) i16x4_t lds_i16x4;
+          const unsigned char* vk = V + kk * 16 * (CHV * 16);
+          const i16x4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vk + at(vaddr0, part * DT * 4 + t * 4)));
+          const i16x4_t y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vk + at(vaddr1, part * DT * 4 + t * 4)));
+          const bf16x8_t vt = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+          for (int e = 0; e < 3 - part; ++e) o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vt, pw[e], o[t], 0, 0, 0);
+        }
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s) stage(kt0 + s, s);  // (past the last key: zeros)
+  int buf = 0;
+  for (int kt = kt0; kt < nkt; ++kt) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 2) * PU) : "memory");
+    __builtin_amdgcn_s_barrier();  // tile kt is whole, and no wave reads the one before
+    asm volatile("" ::: "memory");
+    const unsigned char* K = lds + buf * STAGE;
+    const unsigned char* V = lds + buf * STAGE + kTileKeys * 16 * CHK;
+    for (int st = ks; st < 2; st += KS) {
+      const int k0 = kt * kTileKeys + st * 32;
+      if (k0 <= wlast && k0 + 31 >= wlo) keys32(K + st * 32 * (CHK * 16), V + st * 32 * (CHV * 16), k0);
+    }
+    // (behind the tile's work: the transposed reads wait for every DMA in flight)
+    stage(kt + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+    buf = buf + 1 == ST ? 0 : buf + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  l += __shfl_xor(l, 32);
+
+  // ---- the two halves of the key tiles (one map), or the two maps
+  float* ex = (float*)lds;
+  constexpr int EX = 64 * (DT * 16 + 2);
+  if (KS == 2) {
+    float* mine = ex + (vh + nv * qw) * EX + lane;
+    if (ks == 1) {
+      mine[0] = m;
+      mine[64] = l;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mine[(2 + t * 16 + r) * 64] = o[t][r];
+    }
+    __syncthreads();
+    if (ks == 0) {
+      float fa = 1.0f, fb = 1.0f;
+      if (!SIG) {
+        const float m2 = mine[0], mn = fmaxf(m, m2), ref = mn == -INFINITY ? 0.0f : mn;
+        fa = m == -INFINITY ? 0.0f : exp_neg(m - ref);
+        fb = m2 == -INFINITY ? 0.0f : exp_neg(m2 - ref);
+        l = l * fa + mine[64] * fb;
+        m = mn;
+      }
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] = o[t][r] * fa + mine[(2 + t * 16 + r) * 64] * fb;
+    }
+    __syncthreads();
+  }
+  bool store = ks == 0;
+  if (MAPS == 2) {
+    float* mine = ex + (vh / 2 + p.heads * qw) * EX + lane;
+    const float inv = 1.0f / l;
+    if (store && map == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mine[(t * 16 + r) * 64] = o[t][r] * inv;
+    }
+    __syncthreads();
+    store = store && map == 0;
+    if (store) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          o[t][r] = o[t][r] * inv - a.lambda * mine[(t * 16 + r) * 64];
+          ss = fmaf(o[t][r], o[t][r], ss);
+        }
+      ss += __shfl_xor(ss, 32);
+      const float f = a.post / sqrtf(ss / (float)DV + a.eps);
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] *= f;
+    }
+    __syncthreads();
+  } else if (store) {
+    float f = a.post;
+    if (!SIG) {
+      float den = l;
+      if (a.sink) {
+        const float snk = a.sink[h], top = fmaxf(m, snk);
+        const float w = m == -INFINITY ? 0.0f : expf(m - top);
+        den = l * w + expf(snk - top);
+        f *= w;
+      }
+      f /= den;
+    }
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[t][r] *= f;
+  }
+  if (!store) return;
+  // ---- turned in LDS: a wave writes whole rows of a head
+  const int slot = MAPS == 2 ? vh / 2 + p.heads * qw : vh + nv * qw;
+  float* turn = ex + slot * 32 * (DV + 4);
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *(float4*)(turn + lq * (DV + 4) + t * 32 + 8 * (r >> 2) + 4 * hh) =
+          make_float4(o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  constexpr int LANES = DV / 4;  // a lane holds four columns
+  for (int i = lane / LANES; i < nlive; i += 64 / LANES) {
+    const int c = lane % LANES * 4;
+    const float4 got = *(const float4*)(turn + i * (DV + 4) + c);
+    float v[4] = {got.x, got.y, got.z, got.w};
+    const size_t orow = (size_t)(rfirst + qw * 32 + i);
+    if (a.v_freq) {  // turned back by the query's position
+      const int hv = DV / 2;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int ce = c + e;
+        const bool second = a.interleaved ? (ce & 1) : ce >= hv;
+        const int f = a.interleaved ? ce >> 1 : (second ? ce - hv : ce);
+        const float other = turn[i * (DV + 4) + (a.interleaved ? ce ^ 1 : (second ? ce - hv : ce + hv))];
+        const float mine = e == 0 ? got.x : (e == 1 ? got.y : (e == 2 ? got.z : got.w));
+        float sn, cs;
+        sincosf((float)(wfirst + i) * a.v_freq[f], &sn, &cs);
+        v[e] = second ? mine * cs - other * sn : mine * cs + other * sn;
+      }
+    }
+    if (a.gate) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] *= sigmoid_f(a.gate[orow * a.ldg + (a.gate_cols == 1 ? (size_t)h : (size_t)h * DV + c + e)]);
+    }
+    const size_t to = orow * a.H * DV + (size_t)h * DV + c;
+    if (a.out) *(float4*)(a.out + to) = make_float4(v[0], v[1], v[2], v[3]);
+    if (a.out16) *(uint2*)(a.out16 + to) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+  }
+}
+
+// The sizes that have a form, and queries and results in 16-byte pieces; any step with more than one token of a sequence:
+// 9 tokens after 1500 of 16 heads on 4 key heads of 128 take 75 us here and 158 with a thread per key (seq_attn.hip), 9 of
+// a new sequence 15 and 24, 2048 of one 110 and 634 (51 GFLOP of bf16 products, 17 of fp32 ones).
+bool attn_tiles_fit(const AttnArgs& a, int maps, int parts, int max_len) {
+  const bool sized = parts == 2 ? (maps == 1 && a.d == 192 && a.dv == 128)
+                                : ((a.dv == 64 || a.dv == 128) && (a.d == 64 || (a.d == 128 && maps == 1)));
+  return sized && max_len > 1 && a.pool == 0 && a.ld % 4 == 0 && (uintptr_t)a.q % 16 == 0 &&
+         (uintptr_t)a.out % 16 == 0 && (uintptr_t)a.out16 % 8 == 0;
+}
+
+template <int DC, int DT, int MAPS, int PARTS, int ST>
+static int attn_tiles_go(const AttnTileArgs& p, dim3 grid, hipStream_t stream) {
+  if (MAPS == 1 && PARTS == 1 && p.a.score_bias)
+    attn_tiles_kernel<DC, DT, MAPS, PARTS, MAPS == 1 && PARTS == 1, ST><<<grid, 512, 0, stream>>>(p);
+  else
+    attn_tiles_kernel<DC, DT, MAPS, PARTS, false, ST><<<grid, 512, 0, stream>>>(p);
+  return 0;
+}
+
+int attn_tiles_launch(const AttnTileArgs& given, int maps, int parts, int B, int max_len, hipStream_t stream) {
+  AttnTileArgs p = given;
+  AttnArgs& a = p.a;
+  const int share = a.H / a.G;
+  p.heads = share % 4 == 0 ? 4 : (share % 2 == 0 ? 2 : 1);
+  const int nv = p.heads * maps, qw = nv == 8 ? 1 : 4 / nv;
+  a.tiles = (max_len + 32 * qw - 1) / (32 * qw);
+  const long rows = p.packed ? max_len : a.S;
+  LGA_CHECK_ARG((rows + 2L * kTileKeys) * p.krow < (1L << 30) && (rows + 2L * kTileKeys) * p.vrow < (1L << 30) &&
+                    (long)B * a.tiles * (a.H / p.heads) < (1L << 31),
+                "attention: a sequence's keys or values exceed a buffer");
+  const dim3 grid((unsigned)(B * a.tiles * (a.H / p.heads)));
+  if (parts == 2) return attn_tiles_go<12, 4, 1, 2, 2>(p, grid, stream);
+  if (maps == 2) return a.dv == 64 ? attn_tiles_go<4, 2, 2, 1, 3>(p, grid, stream) : attn_tiles_go<4, 4, 2, 1, 3>(p, grid, stream);
+  if (a.d == 64) return a.dv == 64 ? attn_tiles_go<4, 2, 1, 1, 3>(p, grid, stream) : attn_tiles_go<4, 4, 1, 1, 3>(p, grid, stream);
+  return a.dv == 64 ? attn_tiles_go<8, 2, 1, 1, 3>(p, grid, stream) : attn_tiles_go<8, 4, 1, 1, 3>(p, grid, stream);
+}
+
+}  // namespace lgs

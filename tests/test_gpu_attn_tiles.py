@@ -1,0 +1,165 @@
+"""Prompt attention on the bf16 matrix cores (csrc/seq_attn_tiles.hip) against float64 and against the thread-per-key form.
+
+The same bf16 keys and values in an fp32 cache take the thread-per-key form, whose products are fp32: the matrix-core form
+has to be as close to float64 as that one. Its own bound: with scores of a few units, 2e-6 relative in the 2-norm covers
+the scores' rounding (24 bits of a sum of up to 192 products), the exponentials and up to 2000 weighted values.
+"""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-6
+
+
+def rel(x, want):
+    return float((x.double() - want).norm() / want.norm())
+
+
+def visible(pos, S, chunk, window):
+    at = torch.arange(S, device=pos.device)
+    see = at[None] <= pos[:, None]
+    if chunk:
+        see &= at[None] // chunk == pos[:, None] // chunk
+    if window:
+        see &= at[None] > pos[:, None] - window
+    return see
+
+
+def step(lengths, pos0, dev):
+    start = torch.tensor([0] + list(lengths)).cumsum(0).to(torch.int32).to(dev)
+    order = torch.randperm(len(lengths) + 1, generator=torch.Generator().manual_seed(1))[: len(lengths)]
+    return start, order.to(torch.int32).to(dev), torch.tensor(pos0, dtype=torch.int32, device=dev)
+
+
+def caches(slots, S, G, dk, dv, dev, g, filled):
+    """bf16 rows; what no sequence has written is NaN."""
+    k = torch.full((slots, S, G, dk), float("nan"), device=dev)
+    v = torch.full((slots, S, G, dv), float("nan"), device=dev)
+    for slot, n in filled:
+        k[slot, :n] = torch.randn(n, G, dk, generator=g, device=dev)
+        v[slot, :n] = torch.randn(n, G, dv, generator=g, device=dev)
+    return k.bfloat16(), v.bfloat16()
+
+
+STEPS = [([2], [61]), ([16], [0]), ([17, 1, 40], [0, 5, 100]), ([300, 64, 129], [0, 63, 31]), ([700], [513])]
+
+
+@pytest.mark.parametrize("lengths,pos0", STEPS)
+@pytest.mark.parametrize("d,dv", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("H,G,options", [
+    (4, 1, {}), (4, 4, dict(sink=True)), (6, 3, dict(chunk=48)), (8, 2, dict(window=33, gate=1)), (3, 1, dict(sigmoid=True)),
+    (8, 1, dict(sink=True, cap=5.0, rotated=True)), (4, 2, dict(gate=2, rotated=True, interleaved=True, chunk=100)),
+    (8, 2, dict(sigmoid=True, chunk=64))])
+def test_one_map(lengths, pos0, d, dv, H, G, options):
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(d + dv + H)
+    T, S, slots = sum(lengths), max(p + n for p, n in zip(pos0, lengths)) + 3, len(lengths) + 1
+    start, slot, first = step(lengths, pos0, dev)
+    ends = [p + n for p, n in zip(pos0, lengths)]
+    k, v = caches(slots, S, G, d, dv, dev, g, list(zip(slot.tolist(), ends)))
+    ld = H * d + H * dv + 8
+    proj = torch.randn(T, ld, generator=g, device=dev)
+    sink = torch.randn(H, generator=g, device=dev) if options.get("sink") else None
+    bias = torch.randn(H, generator=g, device=dev) if options.get("sigmoid") else None
+    freq = torch.rand(dv // 2, generator=g, device=dev) if options.get("rotated") else None
+    chunk, window, cap = options.get("chunk", 0), options.get("window", 0), options.get("cap", 0.0)
+    gates = {0: -1, 1: H * d, 2: H * d}[options.get("gate", 0)]
+    kw = dict(H=H, G=G, d=d, dv=dv, scale=d ** -0.5, chunk=chunk, cap=cap, post=0.7, window=window, v_freq=freq,
+              interleaved=options.get("interleaved", False), score_bias=bias, gate_off=gates,
+              gate_cols=dv if options.get("gate") == 2 else 1)
+    args = (sink, start, slot, first, max(lengths))
+    got = seq_ops.sinkattn(proj, 0, k, v, *args, **kw)
+    got16 = seq_ops.sinkattn(proj, 0, k, v, *args, bf16_copy=True, **kw)
+    plain = seq_ops.sinkattn(proj, 0, k.float(), v.float(), *args, **kw)
+    want = torch.empty(T, H, dv, dtype=torch.float64, device=dev)
+    for b, (n, p0) in enumerate(zip(lengths, pos0)):
+        rows, pos = slice(int(start[b]), int(start[b + 1])), torch.arange(p0, p0 + n, device=dev)
+        kd, vd = k[slot[b], : p0 + n].double(), v[slot[b], : p0 + n].double()
+        see = visible(pos, p0 + n, chunk, window)
+        for h in range(H):
+            s = proj[rows, h * d:(h + 1) * d].double() @ kd[:, h // (H // G)].T * d ** -0.5
+            s = cap * torch.tanh(s / cap) if cap else s
+            if bias is not None:
+                w = torch.sigmoid(s + bias[h].double()) * see
+            else:
+                s = s.masked_fill(~see, -math.inf)
+                if sink is not None:
+                    s = torch.cat([s, sink[h].double().expand(n, 1)], -1)
+                w = torch.softmax(s, -1)[:, : p0 + n]
+            o = w @ vd[:, h // (H // G)] * 0.7
+            if freq is not None:
+                ang = pos[:, None] * freq.double()
+                c, sn = torch.cos(ang), torch.sin(ang)
+                i, j = (slice(0, None, 2), slice(1, None, 2)) if kw["interleaved"] else (slice(0, dv // 2), slice(dv // 2, None))
+                x, y = o[:, i].clone(), o[:, j].clone()
+                o[:, i], o[:, j] = x * c + y * sn, y * c - x * sn
+            if gates >= 0:
+                z = proj[rows, gates + (h * dv if kw["gate_cols"] > 1 else h):][:, : kw["gate_cols"]].double()
+                o = o * torch.sigmoid(z)
+            want[rows, h] = o
+    want = want.flatten(1)
+    # (turning back by fp32 angles of up to 1200 radians: both forms take the same cosines, off by up to 1e-4)
+    bound = 1e-4 if freq is not None else TOL
+    assert rel(got, want) < bound and rel(got, want) < 1.5 * rel(plain, want) + 1e-7
+    assert torch.equal(got16, got.bfloat16())
+
+
+@pytest.mark.parametrize("lengths,pos0", STEPS)
+@pytest.mark.parametrize("dv", [64, 128])
+@pytest.mark.parametrize("H,G,chunk,cap", [(2, 2, 0, 0.0), (4, 2, 40, 30.0), (4, 1, 128, 30.0), (8, 2, 0, 3.0)])
+def test_two_maps(lengths, pos0, dv, H, G, chunk, cap):
+    from lit_gpt import seq_ops
+
+    dev, d = torch.device("cuda", 0), 64
+    g = torch.Generator(device=dev).manual_seed(dv + H)
+    T, S, slots = sum(lengths), max(p + n for p, n in zip(pos0, lengths)) + 3, len(lengths) + 1
+    start, slot, first = step(lengths, pos0, dev)
+    ends = [p + n for p, n in zip(pos0, lengths)]
+    k, v = caches(slots, S, G, 2 * d, dv, dev, g, list(zip(slot.tolist(), ends)))
+    proj = torch.randn(T, 2 * H * d + 4, generator=g, device=dev)
+    kw = dict(H=H, G=G, d=d, dv=dv, chunk=chunk, scale=0.125, cap=cap, lam=0.4, eps=1e-5, post=0.5)
+    args = (start, slot, first, max(lengths))
+    got = seq_ops.diffattn(proj, 0, k, v, *args, **kw)
+    plain = seq_ops.diffattn(proj, 0, k.float(), v.float(), *args, **kw)
+    want = torch.empty(T, H, dv, dtype=torch.float64, device=dev)
+    for b, (n, p0) in enumerate(zip(lengths, pos0)):
+        rows, pos = slice(int(start[b]), int(start[b + 1])), torch.arange(p0, p0 + n, device=dev)
+        kd, vd = k[slot[b], : p0 + n].double(), v[slot[b], : p0 + n].double()
+        see = visible(pos, p0 + n, chunk, 0)
+        for h in range(H):
+            maps = []
+            for i in range(2):
+                q = proj[rows, (2 * h + i) * d:(2 * h + i + 1) * d].double()
+                s = q @ kd[:, h // (H // G), i * d:(i + 1) * d].T * 0.125
+                s = cap * torch.tanh(s / cap) if cap else s
+                maps.append(torch.softmax(s.masked_fill(~see, -math.inf), -1) @ vd[:, h // (H // G)])
+            o = maps[0] - 0.4 * maps[1]
+            want[rows, h] = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * 0.5
+    want = want.flatten(1)
+    # (a query that sees one key has two equal maps: their difference keeps all bits here, and nothing cancels)
+    assert rel(got, want) < TOL and rel(got, want) < 1.5 * rel(plain, want) + 1e-7
+
+
+def test_large_scores_and_infinite_queries():
+    """A key that outweighs all others, scores far below it, and a query whose scores overflow: as the other form has it."""
+    from lit_gpt import seq_ops
+
+    dev, T, d = torch.device("cuda", 0), 96, 64
+    g = torch.Generator(device=dev).manual_seed(3)
+    start, slot, first = step([T], [0], dev)
+    k, v = caches(2, T, 1, d, d, dev, g, [(int(slot[0]), T)])
+    k[int(slot[0]), 40] *= 100.0
+    proj = torch.randn(T, d, generator=g, device=dev) * 10.0
+    proj[50] = 3e38
+    kw = dict(H=1, G=1, d=d, dv=d, scale=1.0)
+    got = seq_ops.sinkattn(proj, 0, k, v, None, start, slot, first, T, **kw)
+    plain = seq_ops.sinkattn(proj, 0, k.float(), v.float(), None, start, slot, first, T, **kw)
+    rest = torch.arange(T, device=dev) != 50
+    # scores of up to 1e5 carry errors of 1e-2: only weights that dominate are alike
+    assert torch.isfinite(got[rest]).all() and (got[rest] - plain[rest]).abs().max() < 0.1
+    assert not torch.isfinite(plain[50]).all() or torch.isfinite(got[50]).all()
