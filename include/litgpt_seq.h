@@ -104,6 +104,18 @@ int lgs_latent_attention_tiles(const float* qc, const float* proj, long ld, int 
                                int cache_f32, const float* cache_kr, const float* sink, const int* seq_start,
                                const int* seq_slot, const int* seq_pos0, float* out, int B, int max_len, int H, int d,
                                int dr, int r, int max_seq, float scale, int window, lgs_stream_t stream);
+/* The prompt form over expanded keys and values, for sequences that start at position 0 in this step: every key (dk values:
+ * the expanded part, then the rotated part that all heads share) and value as two bf16 summands, [T][H][2][dk] and
+ * [T][H][2][dv], which lgs_latent_split makes from a row's products kv (H keys of d, then H values of dv; row stride ld)
+ * and row rows[t] of cache_kr. lgs_split_attention: causal softmax attention (optional sink, window) of the queries q
+ * (row stride ld, head h at h dk) over them on the matrix cores; fp32 and / or bf16 results [T][H dv]. Sizes that have a
+ * form: lgs_split_attention_fits. */
+int lgs_latent_split(const float* kv, long ld, const float* cache_kr, const int* rows, void* k, void* v, int T, int H, int d,
+                     int dr, int dv, lgs_stream_t stream);
+int lgs_split_attention_fits(int dk, int dv);
+int lgs_split_attention(const float* q, long ld, const void* k, const void* v, const float* sink, const int* seq_start,
+                        const int* seq_slot, const int* seq_pos0, float* out, void* out_bf16, int B, int max_len, int H,
+                        int dk, int dv, float scale, int window, lgs_stream_t stream);
 
 /* out[t][i] = act(a[t * ld + i]) * b[t * ld + i], i < n */
 int lgs_glu(const float* a, const float* b, long ld, void* out /* fp32, or bf16 with out_bf16 */, int out_bf16, int T,

@@ -841,7 +841,8 @@ class LayeredGPT(nn.Module):
         pos = (torch.arange(T, device=dev) if input_pos is None else input_pos.to(dev)).to(torch.int32).contiguous()
         zero = torch.zeros(1, dtype=torch.int32, device=dev)
         step = StepBatch(idx.reshape(-1).to(torch.int32).contiguous(), zero.expand(T).contiguous(), pos,
-                         torch.tensor([0, T], dtype=torch.int32, device=dev), zero, pos[:1], T=T, B=1)
+                         torch.tensor([0, T], dtype=torch.int32, device=dev), zero, pos[:1], T=T, B=1,
+                         fresh=input_pos is None)
         x = self.forward_step(step)
         if last_token_only:
             x = x[-1:].contiguous()

@@ -44,6 +44,7 @@ class StepBatch:
     T: int
     B: int
     max_len: int = 0  # the most tokens any sequence brings to this step (host side; 0: unknown, taken as T)
+    fresh: bool = False  # every sequence starts at position 0 in this step (host side; False: it may not)
 
     @classmethod
     def build(cls, entries: Sequence[Tuple[int, int, Sequence[int]]], device: torch.device) -> "StepBatch":
@@ -63,7 +64,7 @@ class StepBatch:
         flat = torch.tensor(tokens + slot + pos + start + sslot + spos, dtype=torch.int32).to(device)
         cut = [T, T, T, B + 1, B, B]
         parts = torch.split(flat, cut)
-        return cls(*parts, T=T, B=B, max_len=max(len(e[2]) for e in entries))
+        return cls(*parts, T=T, B=B, max_len=max(len(e[2]) for e in entries), fresh=all(p0 == 0 for _, p0, _ in entries))
 
 
 def _f32(t: torch.Tensor, device) -> torch.Tensor:
@@ -188,7 +189,10 @@ class LatentAttention(InputReader):
             self.q_norm_w = _f32(w["dq.norm"], device)
         # per head (r, d): the key up-projection transposed, so that q_h (d values) maps to r latent coordinates
         self.register_buffer("w_ukT", w["uk"].to(device=device, dtype=dtype).view(H, d, r).transpose(1, 2).contiguous())
-        self.register_buffer("w_uv", w["uv"].to(device=device, dtype=dtype).contiguous())
+        # both up-projections as they are, one under the other: prompts expand keys and values in one product
+        up = torch.cat([w["uk"], w["uv"]]).to(device=device, dtype=dtype).contiguous()
+        self.register_buffer("w_up", up)
+        self.register_buffer("w_uv", up[H * d:])
         self.register_buffer("w_o", w["o"].to(device=device, dtype=dtype).contiguous())
         self.register_buffer("norm_w", _f32(w["dkv.norm"], device))
         self.register_buffer("sink", _f32(w["sink"], device) if spec.sink_kind == "learned" and "sink" in w else None)
@@ -214,6 +218,19 @@ class LatentAttention(InputReader):
         seq_ops.latent_prepare(q, q_off, proj, self.off["dkv"], cache.c, cache.kr, self.norm_w, self.inv_freq, step.slot,
                                step.pos, H=H, d=d, dr=dr, r=r, rot_dims=self.rot_dims, eps=self.eps,
                                rot_mult=self.rot_mult)
+        b16 = _tiles16(T, self.w_o)
+        if b16 and self._expands(step, ldq, q_off):
+            # a prompt from its start: every row's key and value are expanded once, 2 (d + dr + dv) operations per pair
+            # and head instead of 2 (2 r + dr), and the query is not rounded on its way into the latent space
+            n = H * (d + dv)
+            rows = torch.add(step.pos, step.slot, alpha=cache.c.shape[1])
+            kv = torch.empty(T, n, dtype=torch.float32, device=proj.device)
+            seq_ops.linear(cache.c, self.w_up, M=T, N=n, K=r, y=kv, lda=r, ldy=n, a_rows=rows)
+            att = seq_ops.expanded_latent_attention(q, q_off, kv, cache.kr, rows, self.sink, step.seq_start, step.seq_slot,
+                                                    step.seq_pos0, step.max_len or T, H=H, d=d, dr=dr, dv=dv, scale=self.scale,
+                                                    window=self.window, bf16=not self.out_gate)
+            self._finish(att, proj, x, accumulate, b16)
+            return
         qc = torch.empty(T, H * r, dtype=torch.float32, device=proj.device)
         seq_ops.linear(q, self.w_ukT, M=T, N=r, K=d, y=qc, a_off=q_off, lda=ldq, ldy=H * r, batch=H,
                        stride_a=d + dr, stride_w=r * d, stride_y=r)
@@ -225,14 +242,20 @@ class LatentAttention(InputReader):
             lat = seq_ops.latent_attention(qc, q, q_off, cache.c, cache.kr, self.sink, step.slot, step.pos, H=H,
                                            d=d, dr=dr, r=r, scale=self.scale, window=self.window)
         # (without a gate the per-head products leave the out-projection's operand as it reads it)
-        b16 = _tiles16(T, self.w_o)
         att = torch.empty(T, H * dv, dtype=torch.bfloat16 if b16 and not self.out_gate else torch.float32, device=proj.device)
         seq_ops.linear(lat, self.w_uv, M=T, N=dv, K=r, y=att, lda=H * r, ldy=H * dv, batch=H, stride_a=r,
                        stride_w=dv * r, stride_y=dv)
+        self._finish(att, proj, x, accumulate, b16)
+
+    def _expands(self, step: StepBatch, ldq: int, q_off: int) -> bool:
+        return step.fresh and (step.max_len or step.T) > 1 and step.T >= 8 * step.B and self.r % 64 == 0 and ldq % 4 == 0 and \
+            q_off % 4 == 0 and seq_ops.split_attention_fits(self.d + self.dr, self.dv)
+
+    def _finish(self, att: torch.Tensor, proj: torch.Tensor, x: torch.Tensor, accumulate: bool, b16: bool) -> None:
+        H, dv, W, T = self.H, self.dv, x.shape[1], x.shape[0]
         if self.out_gate:
             att = seq_ops.head_gate(att, proj, self.off["g"], H=H, dv=dv, unit_norm=False, eps=self.eps,
                                     act=seq_ops.ACT_SIGMOID, bf16_copy=b16)
-        W = x.shape[1]
         seq_ops.linear(att, self.w_o, M=T, N=W, K=H * dv, y=x, lda=H * dv, ldy=W, accumulate=accumulate)
 
 

@@ -41,6 +41,9 @@ SIGNATURES = {
     "lgs_latent_prepare": [_P, _L, _P, _L, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "lgs_latent_attention": [_P, _P, _L, _I, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _I, _P],
     "lgs_latent_attention_tiles": [_P, _P, _L, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P],
+    "lgs_latent_split": [_P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
+    "lgs_split_attention_fits": [_I, _I],
+    "lgs_split_attention": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P],
     "lgs_glu": [_P, _P, _L, _P, _I, _I, _I, _I, _P],
     "lgs_moe_route": [_P, _L, _I, _I, _I, _P, _P, _P],
     "lgs_moe_route_scores": [_P, _L, _I, _I, _I, _P, _P, _P, _I, _I, _I, _I, _F, _P],
@@ -354,6 +357,35 @@ def latent_attention_tiles(qc: torch.Tensor, proj: torch.Tensor, q_off: int, cac
         _dev(cache_kr, "cache_kr", F32), _opt(sink, "sink", F32), _dev(seq_start, "seq_start", I32),
         _dev(seq_slot, "seq_slot", I32), _dev(seq_pos0, "seq_pos0", I32), out.data_ptr(), B, int(max_len), H, d, dr, r,
         S, float(scale), int(window), _stream()))
+    return out
+
+
+def split_attention_fits(dk: int, dv: int) -> bool:
+    return bool(load_library().lgs_split_attention_fits(dk, dv))
+
+
+def expanded_latent_attention(q: torch.Tensor, q_off: int, kv: torch.Tensor, cache_kr: torch.Tensor, rows: torch.Tensor,
+                              sink: Optional[torch.Tensor], seq_start: torch.Tensor, seq_slot: torch.Tensor,
+                              seq_pos0: torch.Tensor, max_len: int, *, H: int, d: int, dr: int, dv: int, scale: float,
+                              window: int = 0, bf16: bool = False) -> torch.Tensor:
+    """``latent_attention`` of a step in which every sequence starts at position 0, over its rows' expanded keys and values
+    kv (T, H (d + dv)) and rotated parts, rows ``rows`` of ``cache_kr``; the queries (prepared) are the H (d + dr) columns
+    of ``q`` at ``q_off``. Returns (T, H dv) fp32, or with ``bf16`` its rounding."""
+    T, ld = q.shape
+    B = seq_slot.numel()
+    if tuple(kv.shape) != (T, H * (d + dv)) or q_off + H * (d + dr) > ld or rows.numel() != T or seq_start.numel() != B + 1 \
+            or not 1 < max_len <= T or (sink is not None and sink.numel() != H) or cache_kr.shape[-1] != dr:
+        raise ValueError("expanded_latent_attention: shapes")
+    k = torch.empty(T, H, 2, d + dr, dtype=torch.bfloat16, device=q.device)
+    v = torch.empty(T, H, 2, dv, dtype=torch.bfloat16, device=q.device)
+    _check(load_library().lgs_latent_split(_dev(kv, "kv", F32), kv.shape[1], _dev(cache_kr, "cache_kr", F32),
+                                           _dev(rows, "rows", I32), k.data_ptr(), v.data_ptr(), T, H, d, dr, dv, _stream()))
+    out = torch.empty(T, H * dv, dtype=torch.bfloat16 if bf16 else F32, device=q.device)
+    _check(load_library().lgs_split_attention(_dev(q, "q", F32) + 4 * q_off, ld, k.data_ptr(), v.data_ptr(),
+                                              _opt(sink, "sink", F32), _dev(seq_start, "seq_start", I32),
+                                              _dev(seq_slot, "seq_slot", I32), _dev(seq_pos0, "seq_pos0", I32),
+                                              None if bf16 else out.data_ptr(), out.data_ptr() if bf16 else None, B,
+                                              int(max_len), H, d + dr, dv, float(scale), int(window), _stream()))
     return out
 
 

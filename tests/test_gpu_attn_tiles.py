@@ -163,3 +163,37 @@ def test_large_scores_and_infinite_queries():
     # scores of up to 1e5 carry errors of 1e-2: only weights that dominate are alike
     assert torch.isfinite(got[rest]).all() and (got[rest] - plain[rest]).abs().max() < 0.1
     assert not torch.isfinite(plain[50]).all() or torch.isfinite(got[50]).all()
+
+
+@pytest.mark.parametrize("lengths", [[9], [16, 2, 40], [300, 64, 129], [1100]])
+@pytest.mark.parametrize("H,window,sink", [(1, 0, False), (3, 0, True), (4, 50, False)])
+def test_expanded_latent_attention(lengths, H, window, sink):
+    """Keys and values in two bf16 summands (16 bits of their significands: 2^-17 of a product) against float64."""
+    from lit_gpt import seq_ops
+
+    dev, d, dr, dv = torch.device("cuda", 0), 128, 64, 128
+    g = torch.Generator(device=dev).manual_seed(H)
+    T, slots, S = sum(lengths), len(lengths) + 1, max(lengths) + 5
+    start, slot, first = step(lengths, [0] * len(lengths), dev)
+    q = torch.randn(T, H * (d + dr) + 4, generator=g, device=dev)
+    kv = torch.randn(T, H * (d + dv), generator=g, device=dev)
+    kr = torch.full((slots, S, dr), float("nan"), device=dev)
+    rows = torch.cat([slot[b] * S + torch.arange(n, device=dev, dtype=torch.int32) for b, n in enumerate(lengths)])
+    kr.view(-1, dr)[rows.long()] = torch.randn(T, dr, generator=g, device=dev)
+    snk = torch.randn(H, generator=g, device=dev) if sink else None
+    args = (q, 4, kv, kr, rows, snk, start, slot, first, max(lengths))
+    kw = dict(H=H, d=d, dr=dr, dv=dv, scale=192 ** -0.5, window=window)
+    got = seq_ops.expanded_latent_attention(*args, **kw)
+    want = torch.empty(T, H, dv, dtype=torch.float64, device=dev)
+    for b, n in enumerate(lengths):
+        r, pos = slice(int(start[b]), int(start[b + 1])), torch.arange(n, device=dev)
+        see = visible(pos, n, 0, window)
+        for h in range(H):
+            k = torch.cat([kv[r, h * d:(h + 1) * d], kr[slot[b], :n]], -1).double()
+            s = q[r, 4 + h * 192:4 + (h + 1) * 192].double() @ k.T * 192 ** -0.5
+            s = s.masked_fill(~see, -math.inf)
+            s = torch.cat([s, snk[h].double().expand(n, 1)], -1) if sink else s
+            want[r, h] = torch.softmax(s, -1)[:, :n] @ kv[r, H * d + h * dv:H * d + (h + 1) * dv].double()
+    # scores of size 1 from 192 products of relative error 2^-17 each, uncorrelated; values likewise
+    assert rel(got, want.flatten(1)) < 2.0 ** -16
+    assert torch.equal(seq_ops.expanded_latent_attention(*args, bf16=True, **kw), got.bfloat16())
