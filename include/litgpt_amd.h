@@ -292,9 +292,16 @@ int lga_sample_topk(const void* logits, int n, int top_k, float temperature, con
 /* y (M, N) = x (M, K) . w (N, K)^T (+ bias[N]) (+ residual (M, N)) — F.linear (lit_gpt/model.py:519,619,656,699-702) */
 int lga_f32_linear(const float* x, const float* w, const float* bias, const float* residual, float* y, int M, int N,
                    int K, lga_stream_t stream);
+/* the same with an activation on the product + bias (act 0: none, 1: exact gelu, 2: tanh gelu), then + residual, then
+ * + residual2 (each may be NULL) */
+int lga_f32_linear_act(const float* x, const float* w, const float* bias, int act, const float* residual,
+                       const float* residual2, float* y, int M, int N, int K, lga_stream_t stream);
 /* torch.nn.LayerNorm over rows of n (config.py:137-144): two-pass mean / biased variance, (x - mean) * rstd * w + b */
 int lga_f32_layernorm(const float* x, const float* w, const float* b, float* y, int rows, int n, float eps,
                       lga_stream_t stream);
+/* two LayerNorms of the same rows in one launch (GPT-NeoX: norm_1 and norm_2 of a parallel-residual block) */
+int lga_f32_layernorm_pair(const float* x, const float* w, const float* b, float* y, float eps, const float* w2,
+                           const float* b2, float* y2, float eps2, int rows, int n, lga_stream_t stream);
 /* F.gelu (exact erf, or tanh when approximate_tanh) — GptNeoxMLP (model.py:699-702) */
 int lga_f32_gelu(const float* a, float* y, long n, int approximate_tanh, lga_stream_t stream);
 /* y = a + b (the Block residual adds, model.py:584-593) */
@@ -310,6 +317,12 @@ int lga_f32_rope_kv_append(const float* qkv, float* q_out, float* k_cache, float
 int lga_f32_attention(const float* q, const float* k_cache, const float* v_cache, const int64_t* input_pos, float* y,
                       int T, int n_head, int n_query_groups, int head_size, int max_seq, float scale,
                       lga_stream_t stream);
+/* One token's lga_f32_rope_kv_append and lga_f32_attention in one launch: qkv is its fused projection row (per group
+ * [q_0 .. q_{qpk-1}, k, v]); head_size a multiple of 4 up to 256 */
+int lga_f32_attention_decode(const float* qkv, float* k_cache, float* v_cache, const int64_t* cache_pos,
+                             const int64_t* rope_pos, const float* cos, const float* sin, int rope_rows, float* y,
+                             int n_head, int n_query_groups, int head_size, int rope_n_elem, int max_seq, float scale,
+                             lga_stream_t stream);
 /* lga_argmax over fp32 logits (generate/base.py:30-47 at temperature 0) */
 int lga_argmax_f32(const float* logits, int n, int64_t* out_idx, int32_t* token_out, int64_t* pos_inout,
                    lga_stream_t stream);

@@ -2,23 +2,36 @@
 // weights and activations in float32). BASELINE config 1 is quoted in it (pythia-160m fp32, greedy 128 tokens);
 // the bf16 kernels round every activation to bf16, which the fp32 fixture (tests/golden/g1) does not.
 //
-// Plumbing-sized, not tuned: config 1 is the reference's CPU-runnable case (a 160M model), so these kernels keep
-// the reference's per-op arithmetic — fp32 products and sums, no bf16 rounding anywhere — in simple forms:
+// A step of a 160M model is launches and their latency: what runs on one row is fused (RoPE, cache append and attention;
+// both norms of a parallel-residual block; gelu and the residual adds in the products' epilogues), 75 launches a token.
+// Per-op arithmetic is the reference's: fp32 products and sums, no bf16 rounding anywhere:
 //   lga_f32_linear          F.linear (lit_gpt/model.py:619, 656, 699-702, 519): y = x W^T (+ b) (+ residual)
 //   lga_f32_layernorm       torch.nn.LayerNorm (GPT-NeoX norm_class, config.py:137-144): two-pass mean / biased var
+//                           (lga_f32_linear_act: with gelu and a second residual, lga_f32_layernorm_pair: two norms of a row)
 //   lga_f32_gelu            F.gelu exact (erf) or tanh (GptNeoxMLP, model.py:699-702)
 //   lga_f32_add             the Block's residual adds (model.py:584-593)
 //   lga_f32_rope_kv_append  apply_rope (model.py:767-773, partial rotary) + KVCache.forward (:788-795)
 //   lga_f32_attention       SDPA over the cache with the input_pos mask rows (model.py:651, 658-665)
+//   lga_f32_attention_decode  the two above for one token in one launch
 // (the token-embedding gather is lga_embedding over the fp32 rows as pairs of 16-bit words — a byte copy; greedy
 // sampling is lga_argmax_f32 in sample.hip)
 #include "common.h"
 
 namespace lga {
 
+__device__ __forceinline__ float gelu_f32(float v, bool approximate_tanh) {
+  if (approximate_tanh) {
+    const float inner = 0.7978845608028654f * (v + 0.044715f * v * v * v);
+    return 0.5f * v * (1.0f + tanhf(inner));
+  }
+  return 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
+}
+
+// act: 0 none, 1 exact gelu, 2 tanh gelu, on the product + bias; then the residuals, one after the other
 // one wave per output (m, n): lanes stride over K (16-B loads when K % 4 == 0), then a wave sum
 __global__ void __launch_bounds__(256) f32_linear_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                         const float* __restrict__ b, const float* __restrict__ res,
+                                                         const float* __restrict__ b, int act,
+                                                         const float* __restrict__ res, const float* __restrict__ res2,
                                                          float* __restrict__ y, int N, int K) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int n = blockIdx.x * 4 + wave, m = blockIdx.y;
@@ -40,50 +53,80 @@ __global__ void __launch_bounds__(256) f32_linear_kernel(const float* __restrict
   acc = wave_sum(acc);
   if (lane == 0) {
     if (b) acc += b[n];
+    if (act) acc = gelu_f32(acc, act == 2);
     if (res) acc += res[(size_t)m * N + n];
+    if (res2) acc += res2[(size_t)m * N + n];
     y[(size_t)m * N + n] = acc;
   }
 }
 
+// two norms of one row where w2 is given (a block whose attention and MLP read the same residual): the row stays in
+// registers (up to 256 CPT columns), mean and variance are made once per eps
+template <int CPT>
 __global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const float* __restrict__ b, float* __restrict__ y, int n,
-                                                            float eps) {
+                                                            float eps, const float* __restrict__ w2,
+                                                            const float* __restrict__ b2, float* __restrict__ y2, float eps2) {
   const size_t row = blockIdx.x;
   const float* xr = x + row * n;
-  float* yr = y + row * n;
   __shared__ float red[4];
+  float r[CPT];
   float s = 0.0f;
-  for (int i = threadIdx.x; i < n; i += 256) s += xr[i];
+#pragma unroll
+  for (int e = 0; e < CPT; ++e) {
+    const int i = threadIdx.x + 256 * e;
+    r[e] = i < n ? xr[i] : 0.0f;
+    s += r[e];
+  }
+  for (int i = threadIdx.x + 256 * CPT; i < n; i += 256) s += xr[i];
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
   const float mean = ((red[0] + red[1]) + (red[2] + red[3])) / (float)n;
   __syncthreads();
   float ss = 0.0f;
-  for (int i = threadIdx.x; i < n; i += 256) {
+#pragma unroll
+  for (int e = 0; e < CPT; ++e) {
+    const float d = threadIdx.x + 256 * e < n ? r[e] - mean : 0.0f;
+    ss = fmaf(d, d, ss);
+  }
+  for (int i = threadIdx.x + 256 * CPT; i < n; i += 256) {
     const float d = xr[i] - mean;
     ss = fmaf(d, d, ss);
   }
   ss = wave_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
-  const float rstd = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)n + eps);
-  for (int i = threadIdx.x; i < n; i += 256) {
-    const float v = mul_rn(mul_rn(xr[i] - mean, rstd), w[i]);
-    yr[i] = b ? add_rn(v, b[i]) : v;
+  const float var = ((red[0] + red[1]) + (red[2] + red[3])) / (float)n;
+  auto put = [&](const float* w_, const float* b_, float rstd, float* y_, int i, float v) {
+    const float o = mul_rn(mul_rn(v - mean, rstd), w_[i]);
+    y_[row * n + i] = b_ ? add_rn(o, b_[i]) : o;
+  };
+  const float rstd = 1.0f / sqrtf(var + eps), rstd2 = w2 ? 1.0f / sqrtf(var + eps2) : 0.0f;
+#pragma unroll
+  for (int e = 0; e < CPT; ++e) {
+    const int i = threadIdx.x + 256 * e;
+    if (i < n) {
+      put(w, b, rstd, y, i, r[e]);
+      if (w2) put(w2, b2, rstd2, y2, i, r[e]);
+    }
   }
+  for (int i = threadIdx.x + 256 * CPT; i < n; i += 256) {
+    put(w, b, rstd, y, i, xr[i]);
+    if (w2) put(w2, b2, rstd2, y2, i, xr[i]);
+  }
+}
+
+static void f32_layernorm_go(const float* x, const float* w, const float* b, float* y, const float* w2, const float* b2,
+                             float* y2, int rows, int n, float eps, float eps2, hipStream_t stream) {
+  if (n <= 1024) f32_layernorm_kernel<4><<<rows, 256, 0, stream>>>(x, w, b, y, n, eps, w2, b2, y2, eps2);
+  else f32_layernorm_kernel<16><<<rows, 256, 0, stream>>>(x, w, b, y, n, eps, w2, b2, y2, eps2);
 }
 
 __global__ void __launch_bounds__(256) f32_gelu_kernel(const float* __restrict__ a, float* __restrict__ y, size_t n,
                                                        int approximate_tanh) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-    const float v = a[i];
-    if (approximate_tanh) {
-      const float inner = 0.7978845608028654f * (v + 0.044715f * v * v * v);
-      y[i] = 0.5f * v * (1.0f + tanhf(inner));
-    } else {
-      y[i] = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
-    }
+    y[i] = gelu_f32(a[i], approximate_tanh != 0);
   }
 }
 
@@ -124,8 +167,144 @@ __global__ void __launch_bounds__(256) f32_rope_kv_kernel(const float* __restric
   }
 }
 
-// grid (T, H): softmax(q . K^T * scale) . V over keys 0..input_pos[t] of the query's group; scores kept in LDS
-// (max_seq floats), exact max, fp32 exp and sums
+// x * cos + rotate_half(x) * sin of dim d on the first n_elem dims of one head vector, two roundings
+__device__ __forceinline__ float rope_f32(const float* xs, int d, int n_elem, const float* cr, const float* sr) {
+  if (d >= n_elem) return xs[d];
+  const int half = n_elem / 2;
+  const float r = d < half ? -xs[d + half] : xs[d - half];
+  return add_rn(mul_rn(xs[d], cr[d]), mul_rn(r, sr[d]));
+}
+
+struct F32AttnArgs {
+  const float* q;  // [T][H][hs] roped; fused: the token's projection, per group [q_0 .. q_{qpk-1}, k, v]
+  float *kc, *vc;  // [G][max_seq][hs] (written by the fused form only)
+  const int64_t* pos;
+  float* y;
+  int H, G, hs, max_seq;
+  float scale;
+  const int64_t* rope_pos;  // fused only
+  const float *cos, *sin;
+  int n_elem, rope_rows;
+};
+
+// grid (T, H): softmax(q . K^T * scale) . V over keys 0..pos[t] of the query's group; scores kept in LDS, exact max, fp32
+// exp and sums. LPK adjacent lanes hold a key's or value's row in pieces of four (hs <= 4 LPK), the other lanes of the 8
+// waves other keys, four rows of each in flight. FUSED (one token): RoPE on q and on the group's k, which go with v to the
+// caches at position pos[0] and into LDS, in the same launch. Latency-bound at decode sizes (300 keys of 64 per head are
+// 150 KB): one key per wave at a time took 80 us, this form 9 beside the rotation and the append.
+template <int LPK, bool FUSED>
+__global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
+  extern __shared__ float sc[];  // [max_seq] scores, then [8][hs] partial sums
+  __shared__ float red[8];
+  __shared__ __attribute__((aligned(16))) float qs[256], ks[256], vs[256];
+  constexpr int KPW = 64 / LPK, STEP = 8 * KPW;
+  const int t = blockIdx.x, h = blockIdx.y, qpk = a.H / a.G, g = h / qpk, hs = a.hs;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane % LPK, first = wave * KPW + lane / LPK;
+  const long p = a.pos[t];
+  float* kb = a.kc + (size_t)g * a.max_seq * hs;
+  float* vb = a.vc + (size_t)g * a.max_seq * hs;
+  if (FUSED) {
+    const long rp = a.rope_pos[0];
+    if (p < 0 || p >= a.max_seq || rp < 0 || rp >= a.rope_rows) return;  // host validates; never go out of bounds
+    const float* src = a.q + (size_t)g * (qpk + 2) * hs;
+    const float *cr = a.cos + (size_t)rp * a.n_elem, *sr = a.sin + (size_t)rp * a.n_elem;
+    for (int d = threadIdx.x; d < hs; d += 512) {
+      qs[d] = rope_f32(src + (size_t)(h % qpk) * hs, d, a.n_elem, cr, sr);
+      const float k = rope_f32(src + (size_t)qpk * hs, d, a.n_elem, cr, sr), v = src[(size_t)(qpk + 1) * hs + d];
+      ks[d] = k;
+      vs[d] = v;
+      if (h % qpk == 0) {
+        kb[(size_t)p * hs + d] = k;
+        vb[(size_t)p * hs + d] = v;
+      }
+    }
+  } else {
+    const float* qr = a.q + ((size_t)t * a.H + h) * hs;
+    for (int d = threadIdx.x; d < hs; d += 512) qs[d] = qr[d];
+  }
+  __syncthreads();
+  const int L = (int)min(max(p + 1, 1L), (long)a.max_seq);
+  const bool mine = sub * 4 < hs;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  const float4 q4 = mine ? *(const float4*)(qs + sub * 4) : zero;
+  auto row = [&](const float* base, const float* own, int j) {  // (the fused form's own row is not read back)
+    if (!mine) return zero;
+    if (FUSED && j == L - 1) return *(const float4*)(own + sub * 4);
+    return *(const float4*)(base + (size_t)min(j, L - 1) * hs + sub * 4);
+  };
+  float mx = -INFINITY;
+  for (int j0 = first; j0 < L; j0 += 4 * STEP) {
+    float4 k[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) k[u] = row(kb, ks, j0 + u * STEP);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float d = fmaf(q4.w, k[u].w, fmaf(q4.z, k[u].z, fmaf(q4.y, k[u].y, q4.x * k[u].x)));
+      d = group_sum<LPK>(d) * a.scale;
+      const int j = j0 + u * STEP;
+      if (j < L) {
+        mx = fmaxf(mx, d);
+        if (sub == 0) sc[j] = d;
+      }
+    }
+  }
+  mx = wave_max(mx);
+  if (lane == 0) red[wave] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 8; ++w) mx = fmaxf(mx, red[w]);
+  __syncthreads();
+  float sum = 0.0f;
+  for (int j = threadIdx.x; j < L; j += 512) {
+    const float e = expf(sc[j] - mx);
+    sc[j] = e;
+    sum += e;
+  }
+  sum = wave_sum(sum);
+  if (lane == 0) red[wave] = sum;
+  __syncthreads();
+  sum = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
+  float4 o = zero;
+  for (int j0 = first; j0 < L; j0 += 4 * STEP) {
+    float4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = row(vb, vs, j0 + u * STEP);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = j0 + u * STEP;
+      const float w = j < L ? sc[j] : 0.0f;
+      if (j < L) o.x = fmaf(w, v[u].x, o.x), o.y = fmaf(w, v[u].y, o.y), o.z = fmaf(w, v[u].z, o.z), o.w = fmaf(w, v[u].w, o.w);
+    }
+  }
+#pragma unroll
+  for (int x = 32; x >= LPK; x >>= 1) {
+    o.x += __shfl_xor(o.x, x);
+    o.y += __shfl_xor(o.y, x);
+    o.z += __shfl_xor(o.z, x);
+    o.w += __shfl_xor(o.w, x);
+  }
+  __syncthreads();  // the weights are read
+  float* part = sc;
+  if (lane < LPK && mine) *(float4*)(part + wave * hs + sub * 4) = o;
+  __syncthreads();
+  for (int d = threadIdx.x; d < hs; d += 512) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) acc += part[w * hs + d];
+    a.y[((size_t)t * a.H + h) * hs + d] = acc / sum;
+  }
+}
+
+template <bool FUSED>
+static void f32_attention_go(const F32AttnArgs& a, int T, hipStream_t stream) {
+  const size_t lds = sizeof(float) * (size_t)std::max(a.max_seq, 8 * a.hs);
+  const dim3 grid(T, a.H);
+  if (a.hs <= 64) f32_attention_vec_kernel<16, FUSED><<<grid, 512, lds, stream>>>(a);
+  else if (a.hs <= 128) f32_attention_vec_kernel<32, FUSED><<<grid, 512, lds, stream>>>(a);
+  else f32_attention_vec_kernel<64, FUSED><<<grid, 512, lds, stream>>>(a);
+}
+
+// grid (T, H): the same for head sizes that are no multiple of four (scores in LDS: max_seq floats, then partial sums)
 __global__ void __launch_bounds__(256) f32_attention_kernel(const float* __restrict__ q, const float* __restrict__ kc,
                                                             const float* __restrict__ vc,
                                                             const int64_t* __restrict__ input_pos, float* __restrict__ y,
@@ -188,18 +367,30 @@ static unsigned elementwise_blocks(size_t n) { return (unsigned)std::min<size_t>
 
 }  // namespace lga
 
+extern "C" int lga_f32_linear_act(const float* x, const float* w, const float* bias, int act, const float* residual,
+                                  const float* residual2, float* y, int M, int N, int K, hipStream_t stream) {
+  LGA_CHECK_ARG(x && w && y && M > 0 && N > 0 && K > 0 && M <= 65535 && act >= 0 && act <= 2, "lga_f32_linear: bad arguments");
+  LGA_CHECK_ARG(((uintptr_t)x | (uintptr_t)w) % 16 == 0 || K % 4 != 0, "lga_f32_linear: 16-B aligned x, w needed");
+  lga::f32_linear_kernel<<<dim3((N + 3) / 4, M), 256, 0, stream>>>(x, w, bias, act, residual, residual2, y, N, K);
+  LGA_LAUNCH_RETURN();
+}
+
 extern "C" int lga_f32_linear(const float* x, const float* w, const float* bias, const float* residual, float* y,
                               int M, int N, int K, hipStream_t stream) {
-  LGA_CHECK_ARG(x && w && y && M > 0 && N > 0 && K > 0 && M <= 65535, "lga_f32_linear: bad arguments");
-  LGA_CHECK_ARG(((uintptr_t)x | (uintptr_t)w) % 16 == 0 || K % 4 != 0, "lga_f32_linear: 16-B aligned x, w needed");
-  lga::f32_linear_kernel<<<dim3((N + 3) / 4, M), 256, 0, stream>>>(x, w, bias, residual, y, N, K);
-  LGA_LAUNCH_RETURN();
+  return lga_f32_linear_act(x, w, bias, 0, residual, nullptr, y, M, N, K, stream);
 }
 
 extern "C" int lga_f32_layernorm(const float* x, const float* w, const float* b, float* y, int rows, int n, float eps,
                                  hipStream_t stream) {
   LGA_CHECK_ARG(x && w && y && rows > 0 && n > 0, "lga_f32_layernorm: bad arguments");
-  lga::f32_layernorm_kernel<<<rows, 256, 0, stream>>>(x, w, b, y, n, eps);
+  lga::f32_layernorm_go(x, w, b, y, nullptr, nullptr, nullptr, rows, n, eps, 0.0f, stream);
+  LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lga_f32_layernorm_pair(const float* x, const float* w, const float* b, float* y, float eps, const float* w2,
+                                      const float* b2, float* y2, float eps2, int rows, int n, hipStream_t stream) {
+  LGA_CHECK_ARG(x && w && y && w2 && y2 && rows > 0 && n > 0, "lga_f32_layernorm_pair: bad arguments");
+  lga::f32_layernorm_go(x, w, b, y, w2, b2, y2, rows, n, eps, eps2, stream);
   LGA_LAUNCH_RETURN();
 }
 
@@ -238,8 +429,31 @@ extern "C" int lga_f32_attention(const float* q, const float* k_cache, const flo
                     head_size <= 256,
                 "lga_f32_attention: bad geometry (head_size <= 256)");
   LGA_CHECK_ARG(max_seq > 0 && max_seq <= 32768, "lga_f32_attention: max_seq must be in [1, 32768] (scores in LDS)");
+  if (head_size % 4 == 0 && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0) {
+    const lga::F32AttnArgs a{q, (float*)k_cache, (float*)v_cache, input_pos, y, n_head, n_query_groups, head_size, max_seq, scale,
+                             nullptr, nullptr, nullptr, 0, 0};
+    lga::f32_attention_go<false>(a, T, stream);
+    LGA_LAUNCH_RETURN();
+  }
   const size_t lds = ((size_t)max_seq + 256) * sizeof(float);
   lga::f32_attention_kernel<<<dim3(T, n_head), 256, lds, stream>>>(q, k_cache, v_cache, input_pos, y, n_head,
                                                                     n_query_groups, head_size, max_seq, scale);
+  LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lga_f32_attention_decode(const float* qkv, float* k_cache, float* v_cache, const int64_t* cache_pos,
+                                        const int64_t* rope_pos, const float* cos, const float* sin, int rope_rows, float* y,
+                                        int n_head, int n_query_groups, int head_size, int rope_n_elem, int max_seq,
+                                        float scale, hipStream_t stream) {
+  LGA_CHECK_ARG(qkv && k_cache && v_cache && cache_pos && rope_pos && cos && sin && y,
+                "lga_f32_attention_decode: null pointer");
+  LGA_CHECK_ARG(n_query_groups > 0 && n_head > 0 && n_head <= 65535 && n_head % n_query_groups == 0 && head_size > 0 &&
+                    head_size <= 256 && head_size % 4 == 0 && rope_n_elem >= 0 && rope_n_elem % 2 == 0 &&
+                    rope_n_elem <= head_size && rope_rows > 0 && max_seq > 0 && max_seq <= 32768,
+                "lga_f32_attention_decode: bad geometry (head_size a multiple of 4 up to 256, max_seq <= 32768)");
+  LGA_CHECK_ARG(((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0, "lga_f32_attention_decode: aligned caches");
+  const lga::F32AttnArgs a{qkv, k_cache, v_cache, cache_pos, y, n_head, n_query_groups, head_size, max_seq, scale,
+                           rope_pos, cos, sin, rope_n_elem, rope_rows};
+  lga::f32_attention_go<true>(a, 1, stream);
   LGA_LAUNCH_RETURN();
 }

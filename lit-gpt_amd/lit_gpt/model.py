@@ -273,11 +273,31 @@ class Block(nn.Module):
         return ops.add(self.mlp(self.norm_2(x)).contiguous(), x)
 
 
+    def _fuses_f32(self, x: torch.Tensor) -> bool:
+        """Whether the fused fp32 form computes this block: plain fp32 GPT-NeoX modules on the GPU without forward hooks."""
+        m = self.mlp
+        if not (x.is_cuda and x.dtype == torch.float32 and type(m) is GptNeoxMLP and type(self.norm_1) is LayerNorm and
+                type(self.norm_2) is LayerNorm and type(m.fc) is nn.Linear and type(m.proj) is nn.Linear):
+            return False
+        if any(mod._forward_hooks or mod._forward_pre_hooks for mod in (m, m.fc, m.proj, self.norm_1, self.norm_2)):
+            return False
+        ts = (self.norm_1.weight, self.norm_1.bias, self.norm_2.weight, self.norm_2.bias, m.fc.weight, m.fc.bias,
+              m.proj.weight, m.proj.bias)
+        return all(t is None or (t.dtype == torch.float32 and t.is_contiguous()) for t in ts) and \
+            m.config.gelu_approximate in ("none", "tanh")
+
     def _parallel_forward(self, x, cos, sin, mask, input_pos) -> torch.Tensor:
         """GPT-NeoX block (reference model.py:572-593, parallel_residual): n_1 = norm_1(x), h = attn(n_1),
         n_2 = n_1 if shared_attention_norm else norm_2(x), x = mlp(n_2) + h + x — the reference's association:
         bf16(mlp + h) (fused into the mlp.proj epilogue) then + x. Under tensor parallelism the attn / mlp outputs
         go through their all-reduce hooks first (generate/tp.py), as in the reference."""
+        if self._fuses_f32(x):  # 32-true: both norms in one launch, gelu and the two adds in the products' epilogues
+            x2 = x.reshape(-1, x.shape[-1]).contiguous()
+            a, b, mlp = self.norm_1, self.norm_2, self.mlp
+            n_1, n_2 = ops.f32_layernorm_pair(x2, a.weight, a.bias, a.eps, b.weight, b.bias, b.eps)
+            h = self.attn(n_1.view_as(x), cos, sin, mask, input_pos).contiguous()
+            g = ops.f32_linear(n_2, mlp.fc.weight, bias=mlp.fc.bias, gelu=mlp.config.gelu_approximate)
+            return ops.f32_linear(g, mlp.proj.weight, bias=mlp.proj.bias, residual=h, residual2=x2).view_as(x)
         n_1 = self.norm_1(x)
         h = self.attn(n_1, cos, sin, mask, input_pos).contiguous()
         n_2 = n_1 if self.config.shared_attention_norm else self.norm_2(x)
@@ -344,6 +364,8 @@ class CausalSelfAttention(nn.Module):
             # decode token: RoPE + KV-append + attention in a single launch
             y = ops.attention_decode_fused(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem,
                                            1.0 / math.sqrt(hs), n_splits, workspace=ws)
+        elif T == 1 and self.fuse_decode and qkv.dtype == torch.float32 and ops.f32_decode_fusable(hs, S):
+            y = ops.f32_attention_decode(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem, 1.0 / math.sqrt(hs))
         else:
             q = ops.rope_kv_append(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem)
             y = ops.attention(q, kc, vc, pos, H, G, hs, 1.0 / math.sqrt(hs), n_splits, workspace=ws)

@@ -91,11 +91,14 @@ SIGNATURES = {
     "lga_comm_trace": [_P, _I],
     "lga_allreduce_bf16": [_P, _P, _P, _I, ctypes.POINTER(_P), _I, _I, _I, _P, _P, _P],
     "lga_f32_linear": [_P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "lga_f32_linear_act": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _P],
+    "lga_f32_layernorm_pair": [_P, _P, _P, _P, _F, _P, _P, _P, _F, _I, _I, _P],
     "lga_f32_layernorm": [_P, _P, _P, _P, _I, _I, _F, _P],
     "lga_f32_gelu": [_P, _P, _L, _I, _P],
     "lga_f32_add": [_P, _P, _P, _L, _P],
     "lga_f32_rope_kv_append": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "lga_f32_attention": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P],
+    "lga_f32_attention_decode": [_P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _P],
     "lga_argmax_f32": [_P, _I, _P, _P, _P, _P],
     "lga_sample_topk": [_P, _I, _I, _F, _P, ctypes.c_ulonglong, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P],
     "lga_q4_gemv_allreduce": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, ctypes.POINTER(_P), _I, _I, _I, _P, _P, _P,
@@ -385,6 +388,24 @@ def attention(q, k_cache, v_cache, input_pos, n_head, n_query_groups, head_size,
     return y
 
 
+def f32_decode_fusable(head_size: int, max_seq: int) -> bool:
+    return head_size % 4 == 0 and head_size <= 256 and max_seq <= 32768
+
+
+def f32_attention_decode(qkv, k_cache, v_cache, cache_pos, rope_pos, cos, sin, n_head, n_query_groups, head_size,
+                         rope_n_elem, scale, out=None):
+    """One fp32 decode token: RoPE + KV-append + attention in one launch (``attention_decode_fused`` of the 32-true path)."""
+    if qkv.shape[0] != 1:
+        raise ValueError("f32_attention_decode handles exactly one token (T = 1)")
+    y = out if out is not None else torch.empty(1, n_head * head_size, dtype=torch.float32, device=qkv.device)
+    _check(load_library().lga_f32_attention_decode(
+        _dev(qkv, "qkv", torch.float32), _dev(k_cache, "k_cache", torch.float32), _dev(v_cache, "v_cache", torch.float32),
+        _dev(cache_pos, "cache_pos", torch.int64), _dev(rope_pos, "rope_pos", torch.int64), _dev(cos, "cos", torch.float32),
+        _dev(sin, "sin", torch.float32), cos.shape[0], _dev(y, "y", torch.float32), n_head, n_query_groups, head_size,
+        rope_n_elem, k_cache.shape[-2], float(scale), _stream()))
+    return y
+
+
 def attention_decode_fused(qkv, k_cache, v_cache, cache_pos, rope_pos, cos, sin, n_head, n_query_groups,
                            head_size, rope_n_elem, scale, n_splits=1, workspace: Optional[AttentionWorkspace] = None,
                            out=None):
@@ -559,15 +580,30 @@ def argmax(logits, out_idx=None, token_out=None, pos_inout=None):
     return idx
 
 
-def f32_linear(x, weight, bias=None, residual=None, out=None):
-    """y (M, N) = x (M, K) . W (N, K)^T (+ bias) (+ residual), all fp32 (--precision 32-true, csrc/fp32.hip)."""
+def f32_linear(x, weight, bias=None, residual=None, out=None, *, gelu: Optional[str] = None, residual2=None):
+    """y (M, N) = x (M, K) . W (N, K)^T (+ bias) (+ residual), all fp32 (--precision 32-true, csrc/fp32.hip). ``gelu``
+    ("none" / "tanh", F.gelu's ``approximate``): the activation of the product + bias; ``residual2`` is added last."""
     N, K = weight.shape
     M = x.numel() // K
     y = out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device)
-    _check(load_library().lga_f32_linear(_dev(x, "x", torch.float32), _dev(weight, "weight", torch.float32),
-                                         _opt(bias, "bias", torch.float32), _opt(residual, "residual", torch.float32),
-                                         _dev(y, "y", torch.float32), M, N, K, _stream()))
+    act = {None: 0, "none": 1, "tanh": 2}[gelu]
+    _check(load_library().lga_f32_linear_act(_dev(x, "x", torch.float32), _dev(weight, "weight", torch.float32),
+                                             _opt(bias, "bias", torch.float32), act,
+                                             _opt(residual, "residual", torch.float32),
+                                             _opt(residual2, "residual2", torch.float32), _dev(y, "y", torch.float32),
+                                             M, N, K, _stream()))
     return y
+
+
+def f32_layernorm_pair(x, weight, bias, eps, weight2, bias2, eps2):
+    """Two LayerNorms of the same fp32 rows in one launch."""
+    n = x.shape[-1]
+    y, y2 = torch.empty_like(x), torch.empty_like(x)
+    _check(load_library().lga_f32_layernorm_pair(
+        _dev(x, "x", torch.float32), _dev(weight, "weight", torch.float32), _opt(bias, "bias", torch.float32),
+        _dev(y, "y", torch.float32), float(eps), _dev(weight2, "weight2", torch.float32),
+        _opt(bias2, "bias2", torch.float32), _dev(y2, "y2", torch.float32), float(eps2), x.numel() // n, n, _stream()))
+    return y, y2
 
 
 def argmax_embed(logits, table, emb_out, out_idx=None, token_out=None, pos_inout=None):
