@@ -34,6 +34,7 @@
 #include <cstdlib>
 
 #include "common.h"
+#include "gemm_q4d.h"
 
 namespace lga {
 namespace pf {
@@ -740,7 +741,24 @@ int q4f_big_columns(int M, int N, int K) {
 
 int run_tiles(Args a, int fmt, bool dual, int bn, hipStream_t stream);
 
+// the product goes to the register-dequantizing form (gemm_q4d.hip); LGA_Q4F_BN / LGA_Q4F_SPLITS name a launch of the
+// tiles here
+bool q4d_takes(int M, int N, int K, int fmt, bool dual, lga::Q4dPlan* plan) {
+  if (getenv("LGA_Q4F_BN") || getenv("LGA_Q4F_SPLITS")) return false;
+  *plan = lga::q4d_plan(M, N, K, fmt, dual);
+  return plan->mf > 0;
+}
+
 int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t stream) {
+  lga::Q4dPlan dp;
+  if (q4d_takes(a.M, a.N, a.K, lga::kernel_fmt(fmt), dual, &dp)) {
+    const size_t need = lga::q4d_workspace(dp, a.M, a.N, dual);
+    LGA_CHECK_ARG(need == 0 || (ws && ws_bytes >= need),
+                  "lga_q4_gemm_fused: split-K needs the workspace lga_q4f_workspace_bytes reports");
+    const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
+                         lga::codebook_of(fmt), need ? (float*)((unsigned char*)ws + 4096) : nullptr};
+    return lga::q4d_run(d, dp, lga::kernel_fmt(fmt), dual, stream);
+  }
   if (!dual) {
     const int nb = q4f_big_columns(a.M, a.N, a.K);
     if (nb > 0) {
@@ -813,7 +831,7 @@ int lga::preload_gemm_q4f() {
   LGA_PRE(2, false);
   LGA_PRE(2, true);
 #undef LGA_PRE
-  return bad;
+  return bad + lga::preload_gemm_q4d();
 }
 
 #ifdef LGA_Q4F_TRACE
@@ -831,8 +849,13 @@ extern "C" int lga_q4f_fits(int M, int N, int K, int group, int fmt) { return q4
 
 extern "C" size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu) {
   if (M < 1 || N < 1 || K < lga::pf::BK) return 0;
+  // (the weights' format is not known here: the largest of the plans)
   const Plan p = q4f_plan(M, N, K, swiglu != 0);
-  return ws_need(p, M, N, swiglu != 0);
+  size_t need = ws_need(p, M, N, swiglu != 0);
+  lga::Q4dPlan dp;
+  for (int fmt = 0; fmt < 3; fmt += 2)
+    if (q4d_takes(M, N, K, fmt, swiglu != 0, &dp)) need = std::max(need, lga::q4d_workspace(dp, M, N, swiglu != 0));
+  return need;
 }
 
 extern "C" int lga_q4_gemm_fused(const void* x, const void* weight, const void* scales, const void* bias,

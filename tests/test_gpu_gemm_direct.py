@@ -1,0 +1,79 @@
+"""Prompt products whose weights are dequantized in registers (csrc/gemm_q4d.hip, reached through ops.q4_gemm_fused and
+ops.q4_gemm_swiglu) against the fp32 product of the bit-exact dequantized weight (lga_q4_dequantize): rows at and around
+the 16-row pieces and the 128-row tile, columns that end inside a tile and inside a wave's piece, one to many blocks of
+K, whole and split, and every epilogue. Tolerances: the two sums' bf16 roundings may each fall one place apart."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from lit_gpt import ops as _ops
+
+    _ops.load_library()
+    return _ops
+
+
+def _weight(ops, N, K, fmt, group, g):
+    w = torch.randn(N, K, generator=g, device=DEV) * 0.02
+    if fmt == 2:
+        w = w.to(torch.bfloat16)
+        return w, None, w.float()
+    qw, sc = ops.quantize(w, fmt, group)
+    return qw, sc, ops.q4_dequantize(qw, sc, N, K, group, fmt).float()
+
+
+SHAPES = [(33, 8, 128), (48, 136, 384), (64, 264, 1408), (65, 520, 4096), (96, 1032, 256),
+          (1, 8200, 2176), (16, 4104, 4224), (17, 8200, 2176), (32, 4104, 4224),
+          (97, 8712, 7808), (128, 8712, 7808), (129, 264, 1408), (200, 4096, 4096), (256, 136, 128)]
+
+
+@pytest.mark.parametrize("fmt,group", [(0, 128), (0, 64), (1, 64), (2, 64), (3, 128)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_product(ops, fmt, group, M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    w, sc, wd = _weight(ops, N, K, fmt, group, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    res = torch.randn(M, N, generator=g, device=DEV).to(torch.bfloat16)
+    bias = torch.randn(N, generator=g, device=DEV).to(torch.bfloat16)
+    h = x.float() @ wd.t()
+    plain = ops.q4_gemm_fused(x, w, sc, N, K, group, fmt)
+    assert float(((plain.float() - h).abs() - h.abs() * 2 ** -7).max()) <= 2e-3
+    assert torch.equal(plain, ops.q4_gemm_fused(x, w, sc, N, K, group, fmt))
+    h = h + bias.float()
+    y = ops.q4_gemm_fused(x, w, sc, N, K, group, fmt, bias=bias, residual=res).float()
+    ref = h.to(torch.bfloat16).float() + res.float()
+    assert float(((y - ref).abs() - (ref.abs() + h.abs()) * 2 ** -7).max()) <= 2e-3
+
+
+@pytest.mark.parametrize("fmt,group", [(0, 128), (1, 64), (2, 64)])
+@pytest.mark.parametrize("M,N,K", [(33, 8, 128), (64, 136, 1408), (80, 1032, 384), (16, 4104, 4224), (128, 8712, 7808)])
+def test_swiglu(ops, fmt, group, M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    w1, s1, d1 = _weight(ops, N, K, fmt, group, g)
+    w2, s2, d2 = _weight(ops, N, K, fmt, group, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    y = ops.q4_gemm_swiglu(x, w1, s1, w2, s2, N, K, group, fmt).float()
+    a, b = ((x.float() @ d.t()).to(torch.bfloat16).float() for d in (d1, d2))
+    ref = torch.nn.functional.silu(a).to(torch.bfloat16).float() * b
+    # |silu'| <= 1.1, a place of a and one of b, and the roundings of silu and of the result
+    tol = 2 ** -7 * (1.1 * (a * b).abs() + 2 * ref.abs()) + 2 ** -8 * ref.abs() + 2e-3
+    assert float(((y - ref).abs() - tol).max()) <= 0.0
+
+
+def test_rule_falls_back(ops):
+    """K of 64 values, small weights of few rows and long prompts stay with the tiles of gemm_q4f.hip; a split product
+    reports its workspace."""
+    lib = ops.load_library()
+    assert lib.lga_q4f_workspace_bytes(64, 12288, 4096, 0) >= 4096 + 64 * 12288 * 4
+    g = torch.Generator(device=DEV).manual_seed(5)
+    for M, N, K in ((40, 264, 192), (16, 512, 1024), (257, 264, 256)):
+        w, sc, wd = _weight(ops, N, K, 1, 64, g)
+        x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+        h = x.float() @ wd.t()
+        y = ops.q4_gemm_fused(x, w, sc, N, K, 64, 1).float()
+        assert float(((y - h).abs() - h.abs() * 2 ** -7).max()) <= 2e-3
