@@ -1,0 +1,134 @@
+// Prompt products with bf16 weights, Y = X W^T with bias / residual, and fc_1 || fc_2 + SwiGLU, on the pipelined tiles of
+// gemm_tiles.h. The weights are the tile's A: a lane then holds four neighbouring columns of one row of Y, which it
+// stores as 8 bytes, and for SwiGLU a wave's fragments alternate between the two matrices, so that the pair of a column
+// meets in one lane.
+//
+// Bound by the matrix cores' feeding, as the tiles are. Against gemm_q4f.hip's tiles of bf16 weights:
+// of 517 rows (N x K) 12288 x 4096 104 -> 65 us, 4096 x 4096 69 -> 37, 4096 x 11008 118 -> 68, 11008 x 4096 with SwiGLU
+// 183 -> 128; of 100 rows 8192 x 28672 141 -> 103, 28672 x 8192 with SwiGLU 270 -> 185.
+#include "gemm_q4d.h"
+#include "gemm_tiles.h"
+
+namespace lga {
+
+struct BfArgs {
+  Q4dArgs a;
+  int nt, mt, splits, kper;  // tiles over columns and rows; ranges of K of kper stages of 64 values
+};
+
+template <int WM, int WN, int FM, int FN, int BK, int ST, bool DUAL>
+__global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
+  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
+  constexpr int P = T::P, BN = DUAL ? T::BM / 2 : T::BM;  // columns of Y per tile
+  static_assert(FM % 2 == 0, "fragments of the two matrices in pairs");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[ST * T::STAGE];
+  const Q4dArgs& a = k.a;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // an XCD takes neighbouring tiles: the rows' tiles of up to eight columns' tiles, range after range
+  int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int per = k.nt * k.mt, split = t / per;
+  if (split >= k.splits) return;
+  t -= split * per;
+  const int g = t / (8 * k.mt), gn = min(8, k.nt - g * 8);
+  t -= g * 8 * k.mt;
+  const int n0 = (g * 8 + t % gn) * BN, m0 = t / gn * T::BN;
+  const int k0 = split * k.kper * T::RPL, nk = min(a.K / BK - k0, k.kper * T::RPL);
+  const unsigned char* src[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int piece = wave * P + i;
+    const bool of_w = piece < T::BM / T::ROWS;  // (wave-uniform)
+    int r, c;
+    gemm_dma_at<BK>((of_w ? piece : piece - T::BM / T::ROWS) * 8 + (lane >> 3), lane, &r, &c);
+    if (of_w) {  // columns past the end repeat the last one (never stored)
+      const int n = DUAL ? r / 64 * 32 + r % 32 : r;
+      const void* w = DUAL && r / 32 % 2 ? a.w2 : a.w;
+      src[i] = (const unsigned char*)((const uint16_t*)w + (size_t)min(n0 + n, a.N - 1) * a.K);
+    } else {
+      src[i] = (const unsigned char*)(a.x + (size_t)min(m0 + r, a.M - 1) * a.K);
+    }
+    src[i] += (size_t)k0 * (BK * 2) + c * 16;
+  }
+  f32x16_t acc[FM][FN];
+  gemm_tile<WM, WN, FM, FN, BK, ST>(lds, src, nk, wave, lane, acc);
+  const int wm = wave % WM, wn = wave / WM, l31 = lane & 31, hi = lane >> 5;
+  const size_t ldy = a.ldy ? a.ldy : a.N;
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int m = m0 + (wn * FN + j) * 32 + l31;
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int i = 0; i < FM; i += DUAL ? 2 : 1)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + (wm * FM + i) * (DUAL ? 16 : 32) + q * 8 + hi * 4;
+        if (n >= a.N) continue;
+        q4d_f32x4 h, h2;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = acc[i][j][q * 4 + e], h2[e] = acc[i + (DUAL ? 1 : 0)][j][q * 4 + e];
+        if (k.splits > 1) {
+          float* p = a.slabs + ((size_t)split * (DUAL ? 2 : 1) * a.M + m) * a.N + n;
+          *(q4d_f32x4*)p = h;
+          if (DUAL) *(q4d_f32x4*)(p + (size_t)a.M * a.N) = h2;
+        } else if (DUAL) {
+          *(uint2*)(a.y + m * ldy + n) = q4d_swiglu(h, h2);
+        } else {
+          q4d_store(a, m, n, ldy, h);
+        }
+      }
+  }
+}
+
+template <int WM, int WN, int FM, int FN, int BK, int ST>
+static void bf16_go(BfArgs k, bool dual, hipStream_t stream) {
+  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
+  const int bn = dual ? T::BM / 2 : T::BM;
+  k.nt = (k.a.N + bn - 1) / bn, k.mt = (k.a.M + T::BN - 1) / T::BN;
+  const unsigned grid = (unsigned)(((long)k.nt * k.mt * k.splits + 7) / 8 * 8);
+  if (dual) gemm_bf16_kernel<WM, WN, FM, FN, BK, ST, true><<<grid, T::NT, 0, stream>>>(k);
+  else gemm_bf16_kernel<WM, WN, FM, FN, BK, ST, false><<<grid, T::NT, 0, stream>>>(k);
+}
+
+// All products but two kinds (us here / on gemm_q4f.hip's tiles). Few rows and small weights, where a launch over ranges of
+// K and one that adds them are not repaid: 16 x 4096 x 4096 20 / 14, 16 x 4096 x 11008 26 / 23, against 38 / 39 for 8192 x
+// 8192 (2^26). And prompts beyond 1024 rows that fill the chip with 256 x 128 tiles: 2048 rows of 11008 x 4096 with SwiGLU
+// 362 / 349, 28672 x 8192 1698 / 1637, 3000 rows of 4096 x 4096 123 / 110; at 1000 rows 191 / 205, 931 / 902, 45 / 74.
+GemmPlan bf16_plan(int M, int N, int K, bool dual) {
+  const long cols = dual ? 2L * N : N;
+  if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1};
+  if (M > 1024 && (M + 255) / 256 * (cols / 128) >= 256) return GemmPlan{-1, 1};
+  return gemm_tile_plan((int)cols, M, K, 1, false, 0);
+}
+
+size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {
+  return p.ksplit > 1 ? 4096 + (size_t)p.ksplit * (dual ? 2 : 1) * M * N * 4 : 0;
+}
+
+int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream) {
+  const int steps = a.K / 64, kper = (steps + p.ksplit - 1) / p.ksplit;
+  const BfArgs k{a, 0, 0, (steps + kper - 1) / kper, kper};
+  switch (p.tile) {
+    case 0: bf16_go<2, 4, 4, 2, 32, 5>(k, dual, stream); break;
+    case 1: bf16_go<4, 2, 2, 2, 64, 3>(k, dual, stream); break;
+    case 2: bf16_go<2, 2, 2, 2, 64, 2>(k, dual, stream); break;
+    case 3: bf16_go<2, 4, 2, 1, 64, 4>(k, dual, stream); break;
+    default: bf16_go<1, 4, 2, 1, 64, 4>(k, dual, stream); break;
+  }
+  if (k.splits > 1) q4d_sum(a, k.splits, dual, stream);
+  LGA_LAUNCH_RETURN();
+}
+
+int preload_gemm_bf16() {
+  int bad = 0;
+#define LGA_PRE(...) bad += preload(gemm_bf16_kernel<__VA_ARGS__, false>) + preload(gemm_bf16_kernel<__VA_ARGS__, true>)
+  LGA_PRE(2, 4, 4, 2, 32, 5);
+  LGA_PRE(4, 2, 2, 2, 64, 3);
+  LGA_PRE(2, 2, 2, 2, 64, 2);
+  LGA_PRE(2, 4, 2, 1, 64, 4);
+  LGA_PRE(1, 4, 2, 1, 64, 4);
+#undef LGA_PRE
+  return bad;
+}
+
+}  // namespace lga

@@ -1,7 +1,8 @@
-// The register-dequantizing prefill GEMM (gemm_q4d.hip), called by the fused GEMM's entry points (gemm_q4f.hip).
+// The register-dequantizing prefill GEMM (gemm_q4d.hip) and the bf16 weights' tiles (gemm_bf16.hip), called by the fused
+// GEMM's entry points (gemm_q4f.hip).
 #pragma once
 
-#include "common.h"
+#include "gemm_tiles.h"
 
 namespace lga {
 
@@ -20,10 +21,17 @@ struct Q4dArgs {
 struct Q4dPlan {
   int mf, mt, nt, splits, per;
 };
-Q4dPlan q4d_plan(int M, int N, int K, int kernel_fmt, bool dual);
+Q4dPlan q4d_plan(int M, int N, int K, bool dual);
 size_t q4d_workspace(const Q4dPlan& p, int M, int N, bool dual);
 int q4d_run(const Q4dArgs& a, const Q4dPlan& p, int kernel_fmt, bool dual, hipStream_t stream);
+// the partial sums of `splits` ranges of K in order, then the epilogue
+void q4d_sum(const Q4dArgs& a, int splits, bool dual, hipStream_t stream);
 int preload_gemm_q4d();
+
+GemmPlan bf16_plan(int M, int N, int K, bool dual);
+size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual);
+int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream);
+int preload_gemm_bf16();
 
 typedef float q4d_f32x4 __attribute__((ext_vector_type(4)));
 

@@ -8,16 +8,14 @@
 // writes, straight into the A operand of v_mfma_f32_16x16x32_bf16. The products' order over K follows what a lane holds:
 // instruction m of a block takes values 32 fk + 8 m .. + 7 of each of the four lane groups fk. X (up to 128 rows a tile)
 // is shared by the eight waves through LDS (LDS-DMA, source-swizzled, D + 1 buffers), one barrier per 128 values of K.
-// bf16 weights take the same path with four 16-byte loads in the natural order.
 //
 // Ranges of K run side by side until the chip is full; their fp32 partial sums are added in order by a second launch that
 // also runs the epilogue.
 //
-// Bound: bf16 weights of few rows by memory (16 x 28672 x 8192, both matrices: 175 us, 5.4 TB/s). 4-bit weights at about
-// 1.7 us per block of 256 rows x 128 values, which neither the dequantization nor the loads' width moves, up to 64 rows,
-// and by the matrix cores' feeding from LDS beyond. Against the LDS image, 93 rows of nf4 (N x K): 10240 x 8192 97 -> 43 us,
-// 8192 x 8192 62 -> 39, 8192 x 28672 176 -> 82, 28672 x 8192 with SwiGLU 311 -> 150; int4 12288 x 4096 45 -> 29,
-// 4096 x 11008 42 -> 30, 11008 x 4096 with SwiGLU 65 -> 41.
+// Bound: up to 64 rows by about 1.7 us per block of 256 rows x 128 values, which neither the dequantization nor the loads'
+// width moves (16 x 8192 x 28672 in int4: 46 us, 2.6 TB/s), beyond by the matrix cores' feeding from LDS. Against the LDS
+// image, 93 rows of nf4 (N x K): 10240 x 8192 97 -> 43 us, 8192 x 8192 62 -> 39, 8192 x 28672 176 -> 82, 28672 x 8192 with
+// SwiGLU 311 -> 150; int4 12288 x 4096 45 -> 29, 4096 x 11008 42 -> 30, 11008 x 4096 with SwiGLU 65 -> 41.
 #include "gemm_q4d.h"
 
 namespace lga {
@@ -74,13 +72,13 @@ __device__ __forceinline__ bf16x8_t dequant8(uint32_t w, float s, const float* t
   return __builtin_bit_cast(bf16x8_t, o);
 }
 
-// FMT 0 int4-g (bf16 scales), 1 codebook (fp32 block maxima), 2 bf16 weights. MF: 16-row pieces of X. D: blocks ahead
+// FMT 0 int4-g (bf16 scales), 1 codebook (fp32 block maxima). MF: 16-row pieces of X
 template <int FMT, bool DUAL, int MF>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm_q4d_kernel(KArgs k) {
   const Q4dArgs& a = k.a;
-  constexpr int D = FMT == 2 ? 2 : 3, NS = D + 1;     // blocks of 128 values of K ahead; slots
+  constexpr int D = 3, NS = D + 1;                          // blocks of 128 values of K ahead; slots
   constexpr int XB = MF * 16 * 256, XP = (MF * 4 + 7) / 8;  // X: bytes of a block; DMAs per wave (1 KB, 4 rows)
-  constexpr int WL = FMT == 2 ? 4 : 1, WOPS = NR * (FMT == 2 ? 4 : 2);  // W: 16-byte loads per row, all loads of a block
+  constexpr int WOPS = NR * 2;                              // W: a row's loads of a block are its 16 bytes and the scale
   constexpr int JN = DUAL ? NR / 2 : NR;                    // fragments per matrix
   static_assert((D - 1) * XP + D * WOPS <= 63 && NS * XB + 64 <= 163840, "loads in flight; LDS");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * XB + 64];
@@ -93,15 +91,14 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
   if (t >= k.mt * k.nt * k.splits) return;
   const int m0 = t % k.mt * (MF * 16), split = t / k.mt % k.splits, n0 = t / k.mt / k.splits * (128 * JN);
   const int nb_all = a.K / BK, b0 = split * k.per, b1 = min(nb_all, b0 + k.per);
-  const int groups = FMT == 2 ? 0 : a.K / a.G, gshift = FMT == 2 ? 0 : 31 - __builtin_clz((unsigned)a.G);
+  const int groups = a.K / a.G, gshift = 31 - __builtin_clz((unsigned)a.G);
 
   const unsigned char* wp[NR];
   size_t srow[NR];
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
     const int n = min(n0 + (wave * JN + j % JN) * 16 + fr, a.N - 1);
-    const unsigned char* base = (const unsigned char*)(j < JN ? a.w : a.w2);
-    wp[j] = base + (FMT == 2 ? (size_t)n * a.K * 2 + fk * 16 : (size_t)n * (a.K / 2) + fk * 16);
+    wp[j] = (const unsigned char*)(j < JN ? a.w : a.w2) + (size_t)n * (a.K / 2) + fk * 16;
     srow[j] = (size_t)n * groups;
   }
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -115,7 +112,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
     xl[i] = piece * 1024;
     xp[i] = (unsigned)(min(r, a.M - 1 - m0) * a.K + c * 8) * 2;
   }
-  u32x4 w[NS][NR][WL];
+  u32x4 w[NS][NR];
   uint32_t sc[NS][NR];
   auto fetch = [&](int b, int s) {  // block b (past the range: its last, never used) into slot s; X before W, as the waits count
     const int bb = min(b, b1 - 1);
@@ -123,12 +120,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int i = 0; i < XP; ++i) dma16(xr, xp[i], bb * (BK * 2), lds + s * XB + xl[i]);
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < NR; ++j) {
-#pragma unroll
-      for (int i = 0; i < WL; ++i)
-        w[s][j][i] = *(const u32x4*)(wp[j] + (FMT == 2 ? (size_t)bb * (BK * 2) + i * 64 : (size_t)bb * (BK / 2)));
-    }
-    if (FMT == 2) return;
+    for (int j = 0; j < NR; ++j) w[s][j] = *(const u32x4*)(wp[j] + (size_t)bb * (BK / 2));
 #pragma unroll
     for (int j = 0; j < NR; ++j) {
       const void* sp = j < JN ? a.sc : a.sc2;
@@ -147,7 +139,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
     auto frags = [&](int m, bf16x8_t (&f)[MF]) {
 #pragma unroll
       for (int i = 0; i < MF; ++i)
-        f[i] = *(const bf16x8_t*)(X + i * 4096 + 16 * ((FMT == 2 ? m * 4 + fk : fk * 4 + m) ^ fr));
+        f[i] = *(const bf16x8_t*)(X + i * 4096 + 16 * ((fk * 4 + m) ^ fr));
     };
     frags(0, xf[0]);
 #pragma unroll
@@ -155,8 +147,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
       bf16x8_t wf[NR];
 #pragma unroll
       for (int j = 0; j < NR; ++j)
-        wf[j] = FMT == 2 ? __builtin_bit_cast(bf16x8_t, w[s][j][FMT == 2 ? m : 0])
-                         : dequant8<FMT>(w[s][j][0][m], __uint_as_float(FMT == 0 ? sc[s][j] << 16 : sc[s][j]), tab);
+        wf[j] = dequant8<FMT>(w[s][j][m], __uint_as_float(FMT == 0 ? sc[s][j] << 16 : sc[s][j]), tab);
       if (m < 3) frags(m + 1, xf[(m + 1) & 1]);
 #pragma unroll
       for (int i = 0; i < MF; ++i)
@@ -208,8 +199,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
 // the ranges of K in order, then the epilogue; a thread takes four columns of a row
 template <bool DUAL>
-__global__ void __launch_bounds__(256) q4d_sum_kernel(KArgs k) {
-  const Q4dArgs& a = k.a;
+__global__ void __launch_bounds__(256) q4d_sum_kernel(Q4dArgs a, int splits) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, n4 = a.N / 4;
   if (i >= (size_t)a.M * n4) return;
   const int m = (int)(i / n4), n = (int)(i % n4) * 4;
@@ -218,7 +208,7 @@ __global__ void __launch_bounds__(256) q4d_sum_kernel(KArgs k) {
   f32x4_t s = *(const f32x4_t*)p, s2 = {0.f, 0.f, 0.f, 0.f};
   if (DUAL) s2 = *(const f32x4_t*)(p + plane);
 #pragma unroll 4
-  for (int z = 1; z < k.splits; ++z) {
+  for (int z = 1; z < splits; ++z) {
     s += *(const f32x4_t*)(p + z * step);
     if (DUAL) s2 += *(const f32x4_t*)(p + z * step + plane);
   }
@@ -227,14 +217,21 @@ __global__ void __launch_bounds__(256) q4d_sum_kernel(KArgs k) {
   else q4d_store(a, m, n, ldy, s);
 }
 
+}  // namespace pd
+
+void q4d_sum(const Q4dArgs& a, int splits, bool dual, hipStream_t stream) {
+  const unsigned grid = (unsigned)(((size_t)a.M * a.N / 4 + 255) / 256);
+  if (dual) pd::q4d_sum_kernel<true><<<grid, 256, 0, stream>>>(a, splits);
+  else pd::q4d_sum_kernel<false><<<grid, 256, 0, stream>>>(a, splits);
+}
+
+namespace pd {
+
 template <int FMT, bool DUAL, int MF>
 static int go(KArgs k, hipStream_t stream) {
   const unsigned work = (unsigned)(k.mt * k.nt * k.splits);
   gemm_q4d_kernel<FMT, DUAL, MF><<<(work + 7) / 8 * 8, NT, 0, stream>>>(k);
-  if (k.splits > 1) {
-    const size_t n = (size_t)k.a.M * k.a.N / 4;
-    q4d_sum_kernel<DUAL><<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(k);
-  }
+  if (k.splits > 1) q4d_sum(k.a, k.splits, DUAL, stream);
   return 0;
 }
 
@@ -253,18 +250,16 @@ static int go_rows(const KArgs& k, int mf, hipStream_t stream) {
 
 // Which products come here (us here / on the LDS image's tiles; NK = N x K of one matrix):
 //   up to 32 rows   all but NK <= 2^24, where two launches are not repaid (int4 16 x 4096 x 4096: 18 / 15)
-//   up to 96 rows   all (int4 64 x 4096 x 4096: 19 / 23; bf16 64 x 12288 x 4096: 33 / 36)
-//   up to 128 rows  4-bit beyond 2^24 (4096 x 4096: 31 / 26; 12288 x 4096: 37 / 42); bf16 and SwiGLU from 2^26 (bf16
-//                   12288 x 4096: 44 / 37, 8192 x 8192: 50 / 57; int4 SwiGLU 11008 x 4096: 68 / 64, 28672 x 8192: 159 / 268)
-//   up to 256 rows  one matrix up to 2^27 (nf4 200 x 8192 x 8192: 56 / 71; bf16 8192 x 28672: 163 / 155); the 256-row
-//                   tiles read larger weights once
-Q4dPlan q4d_plan(int M, int N, int K, int kernel_fmt, bool dual) {
+//   up to 96 rows   all (int4 64 x 4096 x 4096: 19 / 23)
+//   up to 128 rows  beyond 2^24 (int4 4096 x 4096: 31 / 26; 12288 x 4096: 37 / 42); SwiGLU from 2^26 (int4 11008 x 4096:
+//                   68 / 64, 28672 x 8192: 159 / 268)
+//   up to 256 rows  one matrix up to 2^27 (nf4 200 x 8192 x 8192: 56 / 71; 8192 x 28672: 156 / 160, int4 142 / 148 at
+//                   160); the 256-row tiles read larger weights once
+Q4dPlan q4d_plan(int M, int N, int K, bool dual) {
   Q4dPlan p{0, 0, 0, 0, 0};
   const size_t nk = (size_t)N * K, one = 1;
   if (K % pd::BK != 0 || M > 256) return p;
-  if (M <= 32 ? nk <= one << 24 : M <= 96 ? false : M <= 128 ? nk < one << 26 && (nk <= one << 24 || kernel_fmt == 2 || dual)
-                                                             : dual || nk > one << 27)
-    return p;
+  if (M > 128 ? dual || nk > one << 27 : M > 96 ? nk <= one << (dual ? 26 : 24) : M <= 32 && nk <= one << 24) return p;
   p.mf = M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : (M <= 96 ? 6 : 8)));
   p.mt = (M + p.mf * 16 - 1) / (p.mf * 16);
   const int cols = 128 * (dual ? 1 : 2), nb = K / pd::BK;
@@ -291,9 +286,7 @@ int q4d_run(const Q4dArgs& a, const Q4dPlan& p, int kernel_fmt, bool dual, hipSt
     case 0: pd::go_rows<0, false>(k, p.mf, stream); break;
     case 1: pd::go_rows<0, true>(k, p.mf, stream); break;
     case 2: pd::go_rows<1, false>(k, p.mf, stream); break;
-    case 3: pd::go_rows<1, true>(k, p.mf, stream); break;
-    case 4: pd::go_rows<2, false>(k, p.mf, stream); break;
-    default: pd::go_rows<2, true>(k, p.mf, stream); break;
+    default: pd::go_rows<1, true>(k, p.mf, stream); break;
   }
   LGA_LAUNCH_RETURN();
 }
@@ -308,8 +301,6 @@ int preload_gemm_q4d() {
   LGA_PRE(0, true);
   LGA_PRE(1, false);
   LGA_PRE(1, true);
-  LGA_PRE(2, false);
-  LGA_PRE(2, true);
 #undef LGA_PRE
   return bad + preload(q4d_sum_kernel<false>) + preload(q4d_sum_kernel<true>);
 }

@@ -741,23 +741,22 @@ int q4f_big_columns(int M, int N, int K) {
 
 int run_tiles(Args a, int fmt, bool dual, int bn, hipStream_t stream);
 
-// the product goes to the register-dequantizing form (gemm_q4d.hip); LGA_Q4F_BN / LGA_Q4F_SPLITS name a launch of the
-// tiles here
-bool q4d_takes(int M, int N, int K, int fmt, bool dual, lga::Q4dPlan* plan) {
-  if (getenv("LGA_Q4F_BN") || getenv("LGA_Q4F_SPLITS")) return false;
-  *plan = lga::q4d_plan(M, N, K, fmt, dual);
-  return plan->mf > 0;
-}
+// LGA_Q4F_BN / LGA_Q4F_SPLITS name a launch of the tiles here
+bool tiles_named() { return getenv("LGA_Q4F_BN") || getenv("LGA_Q4F_SPLITS"); }
 
 int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t stream) {
-  lga::Q4dPlan dp;
-  if (q4d_takes(a.M, a.N, a.K, lga::kernel_fmt(fmt), dual, &dp)) {
-    const size_t need = lga::q4d_workspace(dp, a.M, a.N, dual);
-    LGA_CHECK_ARG(need == 0 || (ws && ws_bytes >= need),
-                  "lga_q4_gemm_fused: split-K needs the workspace lga_q4f_workspace_bytes reports");
-    const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
-                         lga::codebook_of(fmt), need ? (float*)((unsigned char*)ws + 4096) : nullptr};
-    return lga::q4d_run(d, dp, lga::kernel_fmt(fmt), dual, stream);
+  if (!tiles_named()) {  // 4-bit weights dequantized in registers (gemm_q4d.hip), bf16 weights on gemm_bf16.hip's tiles
+    const int kf = lga::kernel_fmt(fmt);
+    const lga::Q4dPlan dp = kf == 2 ? lga::Q4dPlan{} : lga::q4d_plan(a.M, a.N, a.K, dual);
+    const lga::GemmPlan bp = kf == 2 ? lga::bf16_plan(a.M, a.N, a.K, dual) : lga::GemmPlan{-1, 1};
+    if (dp.mf > 0 || bp.tile >= 0) {
+      const size_t need = dp.mf > 0 ? lga::q4d_workspace(dp, a.M, a.N, dual) : lga::bf16_workspace(bp, a.M, a.N, dual);
+      LGA_CHECK_ARG(need == 0 || (ws && ws_bytes >= need),
+                    "lga_q4_gemm_fused: split-K needs the workspace lga_q4f_workspace_bytes reports");
+      const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
+                           lga::codebook_of(fmt), need ? (float*)((unsigned char*)ws + 4096) : nullptr};
+      return dp.mf > 0 ? lga::q4d_run(d, dp, kf, dual, stream) : lga::bf16_run(d, bp, dual, stream);
+    }
   }
   if (!dual) {
     const int nb = q4f_big_columns(a.M, a.N, a.K);
@@ -831,7 +830,7 @@ int lga::preload_gemm_q4f() {
   LGA_PRE(2, false);
   LGA_PRE(2, true);
 #undef LGA_PRE
-  return bad + lga::preload_gemm_q4d();
+  return bad + lga::preload_gemm_q4d() + lga::preload_gemm_bf16();
 }
 
 #ifdef LGA_Q4F_TRACE
@@ -852,9 +851,10 @@ extern "C" size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu) {
   // (the weights' format is not known here: the largest of the plans)
   const Plan p = q4f_plan(M, N, K, swiglu != 0);
   size_t need = ws_need(p, M, N, swiglu != 0);
-  lga::Q4dPlan dp;
-  for (int fmt = 0; fmt < 3; fmt += 2)
-    if (q4d_takes(M, N, K, fmt, swiglu != 0, &dp)) need = std::max(need, lga::q4d_workspace(dp, M, N, swiglu != 0));
+  if (!tiles_named()) {
+    need = std::max(need, lga::q4d_workspace(lga::q4d_plan(M, N, K, swiglu != 0), M, N, swiglu != 0));
+    need = std::max(need, lga::bf16_workspace(lga::bf16_plan(M, N, K, swiglu != 0), M, N, swiglu != 0));
+  }
   return need;
 }
 

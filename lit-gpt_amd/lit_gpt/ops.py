@@ -230,14 +230,16 @@ _Q4F_WS: dict = {}
 
 
 def _q4f_workspace(M, N, K, swiglu, device):
-    """The split-K workspace of a short-prompt fused GEMM: one zeroed buffer per device, grown as needed (its
-    per-tile counters are left zeroed by every launch). Returns (ptr, bytes) or (None, 0)."""
+    """The split-K workspace of a short-prompt fused GEMM: one zeroed buffer per device and stream (products on two
+    streams may run at once), grown as needed (its per-tile counters are left zeroed by every launch). Returns
+    (ptr, bytes) or (None, 0)."""
     need = int(load_library().lga_q4f_workspace_bytes(int(M), int(N), int(K), int(bool(swiglu))))
     if need == 0:
         return None, 0
-    ws = _Q4F_WS.get(device)
+    key = device, _stream()
+    ws = _Q4F_WS.get(key)
     if ws is None or ws.numel() < need:
-        ws = _Q4F_WS[device] = torch.zeros(need, dtype=torch.uint8, device=device)
+        ws = _Q4F_WS[key] = torch.zeros(need, dtype=torch.uint8, device=device)
     return ws.data_ptr(), ws.numel()
 
 

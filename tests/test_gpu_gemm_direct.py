@@ -1,5 +1,5 @@
-"""Prompt products whose weights are dequantized in registers (csrc/gemm_q4d.hip, reached through ops.q4_gemm_fused and
-ops.q4_gemm_swiglu) against the fp32 product of the bit-exact dequantized weight (lga_q4_dequantize): rows at and around
+"""Prompt products whose 4-bit weights are dequantized in registers (csrc/gemm_q4d.hip) and those of bf16 weights on the
+pipelined tiles (csrc/gemm_bf16.hip), reached through ops.q4_gemm_fused and ops.q4_gemm_swiglu, against the fp32 product of the bit-exact dequantized weight (lga_q4_dequantize): rows at and around
 the 16-row pieces and the 128-row tile, columns that end inside a tile and inside a wave's piece, one to many blocks of
 K, whole and split, and every epilogue. Tolerances: the two sums' bf16 roundings may each fall one place apart."""
 
@@ -29,12 +29,15 @@ def _weight(ops, N, K, fmt, group, g):
 
 SHAPES = [(33, 8, 128), (48, 136, 384), (64, 264, 1408), (65, 520, 4096), (96, 1032, 256),
           (1, 8200, 2176), (16, 4104, 4224), (17, 8200, 2176), (32, 4104, 4224),
-          (97, 8712, 7808), (128, 8712, 7808), (129, 264, 1408), (200, 4096, 4096), (256, 136, 128)]
+          (97, 8712, 7808), (128, 8712, 7808), (129, 264, 1408), (200, 4096, 4096), (256, 136, 128),
+          (257, 4104, 320), (517, 520, 4160), (1024, 1032, 64), (1025, 264, 1408), (700, 24584, 192)]
 
 
 @pytest.mark.parametrize("fmt,group", [(0, 128), (0, 64), (1, 64), (2, 64), (3, 128)])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_product(ops, fmt, group, M, N, K):
+    if fmt != 2 and K % group:
+        pytest.skip("the group does not divide K")
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     w, sc, wd = _weight(ops, N, K, fmt, group, g)
     x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
@@ -51,8 +54,11 @@ def test_product(ops, fmt, group, M, N, K):
 
 
 @pytest.mark.parametrize("fmt,group", [(0, 128), (1, 64), (2, 64)])
-@pytest.mark.parametrize("M,N,K", [(33, 8, 128), (64, 136, 1408), (80, 1032, 384), (16, 4104, 4224), (128, 8712, 7808)])
+@pytest.mark.parametrize("M,N,K", [(33, 8, 128), (64, 136, 1408), (80, 1032, 384), (16, 4104, 4224), (128, 8712, 7808),
+                                   (300, 520, 4160), (517, 4104, 320)])
 def test_swiglu(ops, fmt, group, M, N, K):
+    if fmt != 2 and K % group:
+        pytest.skip("the group does not divide K")
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     w1, s1, d1 = _weight(ops, N, K, fmt, group, g)
     w2, s2, d2 = _weight(ops, N, K, fmt, group, g)
