@@ -236,7 +236,8 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
   constexpr int ROW = 3 * DP + CW + 4;   // staged floats per token: q | k | g | v | beta (rows stay 16-byte aligned)
   constexpr int kDeltaTB = DP > 256 ? 8 : (DP > 128 ? 16 : 32);  // tokens staged at a time
   constexpr int EPT = (ROW + 255) / 256;       // staged entries per thread and token
-  __shared__ __attribute__((aligned(16))) float st[kDeltaTB * ROW];
+  constexpr int KEEP = (kDeltaTB + LPC - 1) / LPC;  // outputs of a batch that a lane keeps
+  __shared__ __attribute__((aligned(16))) float st[(kDeltaTB + 1) * ROW];  // (a batch's last token reads one row ahead)
   __shared__ float os[kDeltaTB][CW];
   const int tid = threadIdx.x;
   const int r = tid % LPC, cw = tid / LPC;  // cw: column inside the workgroup
@@ -262,6 +263,11 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
       const int row = 4 * (r + LPC * j) + e;
       S[j][e] = (!fresh && live && row < d) ? sp[(size_t)row * dv + col] : 0.0f;
     }
+  // (the loads of S end here: left to the token loop's first use, every batch there would wait for the next one's loads)
+#pragma unroll
+  for (int j = 0; j < NR4; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(S[j][e]));
   // Entry e = tid + 256 i of a token's staged row comes from one place whatever the token: a pointer to it at the
   // sequence's first row, the distance to the next token's, and the value of an entry that has no source (padding).
   // (an entry without a source loads a valid address all the same, so that the loads carry no branches)
@@ -292,66 +298,118 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
     if (!has[i]) src[i] = p.kq + (size_t)r0 * p.G + g;
   }
   float pre[kDeltaTB][EPT];
-  auto prefetch = [&](int t0) {
+  auto prefetch = [&](int t0) {  // (past the end: the last token again)
 #pragma unroll
     for (int t = 0; t < kDeltaTB; ++t)
 #pragma unroll
       for (int i = 0; i < EPT; ++i) {
-        const float v = src[i][(size_t)min(t0 + t, n - 1) * step[i]];
-        pre[t][i] = has[i] ? v : pad[i];
+        pre[t][i] = *src[i];
+        src[i] += t0 + t < n - 1 ? step[i] : 0;
       }
   };
   prefetch(0);
+
+  struct Token {
+    float4 k[NR4], g[NR4], q[NR4];
+    float v, beta, kq;
+  };
+  auto fetch = [&](const float* row, Token& x) {
+#pragma unroll
+    for (int j = 0; j < NR4; ++j) {
+      const int at = 4 * (r + LPC * j);
+      x.g[j] = *(const float4*)(row + 2 * DP + at);
+      x.k[j] = *(const float4*)(row + DP + at);
+      x.q[j] = *(const float4*)(row + at);
+    }
+    x.v = row[3 * DP + cw];
+    x.beta = row[3 * DP + CW];
+    x.kq = row[3 * DP + CW + 1];
+  };
+  // With S' = diag(g) S the output is o = S'^T q + u (k . q): both products with S' run side by side and share one
+  // round of lane sums, and the write S' + k u^T leaves the output's dependent chain. Four partial sums per product
+  // keep the chains short.
+  auto one = [&](auto&& g_at, auto&& k_at, auto&& q_at, float v, float beta, float kq) {
+    float4 k4[NR4];
+    float ka = 0.0f, kb = 0.0f, kc = 0.0f, kd = 0.0f, oa = 0.0f, ob = 0.0f, oc = 0.0f, od = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NR4; ++j) {
+      k4[j] = k_at(j);
+      const float4 g4 = g_at(j), q4 = q_at(j);
+      S[j][0] *= g4.x;
+      S[j][1] *= g4.y;
+      S[j][2] *= g4.z;
+      S[j][3] *= g4.w;
+      if (DELTA) {
+        ka = fmaf(S[j][0], k4[j].x, ka);
+        kb = fmaf(S[j][1], k4[j].y, kb);
+        kc = fmaf(S[j][2], k4[j].z, kc);
+        kd = fmaf(S[j][3], k4[j].w, kd);
+      }
+      oa = fmaf(S[j][0], q4.x, oa);
+      ob = fmaf(S[j][1], q4.y, ob);
+      oc = fmaf(S[j][2], q4.z, oc);
+      od = fmaf(S[j][3], q4.w, od);
+    }
+    float ks = (ka + kb) + (kc + kd), qs = (oa + ob) + (oc + od);
+    lanes_sum2<LPC>(ks, qs);
+    const float u = DELTA ? beta * (v - ks) : v;
+#pragma unroll
+    for (int j = 0; j < NR4; ++j) {
+      S[j][0] = fmaf(k4[j].x, u, S[j][0]);
+      S[j][1] = fmaf(k4[j].y, u, S[j][1]);
+      S[j][2] = fmaf(k4[j].z, u, S[j][2]);
+      S[j][3] = fmaf(k4[j].w, u, S[j][3]);
+    }
+    return fmaf(u, kq, qs);
+  };
+  auto held = [&](const Token& x) {
+    return one([&](int j) { return x.g[j]; }, [&](int j) { return x.k[j]; }, [&](int j) { return x.q[j]; }, x.v, x.beta, x.kq);
+  };
 
   for (int t0 = 0; t0 < n; t0 += kDeltaTB) {
     const int nb = min(kDeltaTB, n - t0);
     __syncthreads();  // the previous batch's reads of st and os are done
 #pragma unroll
-    for (int t = 0; t < kDeltaTB; ++t)
+    for (int i = 0; i < EPT; ++i)
+      if (tid + 256 * i < ROW)
 #pragma unroll
-      for (int i = 0; i < EPT; ++i)
-        if (tid + 256 * i < ROW) st[t * ROW + tid + 256 * i] = pre[t][i];
+        for (int t = 0; t < kDeltaTB; ++t) st[t * ROW + tid + 256 * i] = has[i] ? pre[t][i] : pad[i];
     __syncthreads();
     if (t0 + kDeltaTB < n) prefetch(t0 + kDeltaTB);
-    // With S' = diag(g) S the output is o = S'^T q + u (k . q): both products with S' run side by side and share one
-    // round of lane sums, and the write S' + k u^T leaves the output's dependent chain. Four partial sums per product
-    // keep the chains short; two tokens per trip let one token's tail overlap the next one's decay.
-#pragma unroll 2
-    for (int t = 0; t < nb; ++t) {
-      const float* row = st + t * ROW;
-      float4 k4[NR4];
-      float ka = 0.0f, kb = 0.0f, kc = 0.0f, kd = 0.0f, oa = 0.0f, ob = 0.0f, oc = 0.0f, od = 0.0f;
+    // A full batch of up to 16 rows a lane: the next token's operands are read while one is worked on, and the output of
+    // every LPC-th token stays in one lane's register instead of a branch and a store per token. 2048 tokens of 16 heads
+    // of 128 x 128: 438 us, one token's reads after the other's work 667; with 32 rows a lane the second set of operands
+    // does not fit the registers (8 x 512 tokens of 8 heads of 256 x 256: 623 us against 462).
+    if (NR4 <= 4 && nb == kDeltaTB) {
+      Token x[2];
+      const float* row = st;
+      fetch(row, x[0]);
+      float keep[KEEP];
 #pragma unroll
-      for (int j = 0; j < NR4; ++j) {
-        const int at = 4 * (r + LPC * j);
-        k4[j] = *(const float4*)(row + DP + at);
-        const float4 g4 = *(const float4*)(row + 2 * DP + at);
-        const float4 q4 = *(const float4*)(row + at);
-        S[j][0] *= g4.x;
-        S[j][1] *= g4.y;
-        S[j][2] *= g4.z;
-        S[j][3] *= g4.w;
-        if (DELTA) {
-          ka = fmaf(S[j][0], k4[j].x, ka);
-          kb = fmaf(S[j][1], k4[j].y, kb);
-          kc = fmaf(S[j][2], k4[j].z, kc);
-          kd = fmaf(S[j][3], k4[j].w, kd);
+      for (int m = 0; m < KEEP; ++m) {
+        keep[m] = 0.0f;
+#pragma unroll 1
+        for (int t = 0; t < (kDeltaTB < LPC ? kDeltaTB : LPC); t += 2) {
+          fetch(row + ROW, x[1]);
+          float o = held(x[0]);
+          if (t == r) keep[m] = o;
+          row += 2 * ROW;
+          fetch(row, x[0]);
+          o = held(x[1]);
+          if (t + 1 == r) keep[m] = o;
         }
-        oa = fmaf(S[j][0], q4.x, oa);
-        ob = fmaf(S[j][1], q4.y, ob);
-        oc = fmaf(S[j][2], q4.z, oc);
-        od = fmaf(S[j][3], q4.w, od);
       }
-      float ks = (ka + kb) + (kc + kd), qs = (oa + ob) + (oc + od);
-      lanes_sum2<LPC>(ks, qs);
-      const float u = DELTA ? row[3 * DP + CW] * (row[3 * DP + cw] - ks) : row[3 * DP + cw];
-      if (r == 0) os[t][cw] = fmaf(u, row[3 * DP + CW + 1], qs);
 #pragma unroll
-      for (int j = 0; j < NR4; ++j) {
-        S[j][0] = fmaf(k4[j].x, u, S[j][0]);
-        S[j][1] = fmaf(k4[j].y, u, S[j][1]);
-        S[j][2] = fmaf(k4[j].z, u, S[j][2]);
-        S[j][3] = fmaf(k4[j].w, u, S[j][3]);
+      for (int m = 0; m < KEEP; ++m)
+        if (m * LPC + r < kDeltaTB) os[m * LPC + r][cw] = keep[m];
+    } else {
+#pragma unroll 2
+      for (int t = 0; t < nb; ++t) {
+        const float* row = st + t * ROW;
+        auto at = [&](int part, int j) { return *(const float4*)(row + part * DP + 4 * (r + LPC * j)); };
+        const float o = one([&](int j) { return at(2, j); }, [&](int j) { return at(1, j); }, [&](int j) { return at(0, j); },
+                            row[3 * DP + cw], row[3 * DP + CW], row[3 * DP + CW + 1]);
+        if (r == 0) os[t][cw] = o;
       }
     }
     __syncthreads();
