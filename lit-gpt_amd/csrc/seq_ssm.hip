@@ -164,12 +164,22 @@ __global__ void __launch_bounds__(256) ssm_scan_kernel(ScanArgs p) {
 // chunk's start and n its token count:
 //   y_i = exp(l_i) C_i^T S0 + sum_{j <= i} exp(l_i - l_j) dt_j (C_i . B_j) x_j + D x_i
 //   S'  = exp(l_{n-1}) S0 + sum_j exp(l_{n-1} - l_j) dt_j B_j x_j^T
-// MODE 1, grid (B * max_chunks, heads, ceil(dv / 64)): the second term of S' of every chunk -> workspace, the chunk's
-// whole decay -> wdec. ssd_carry_kernel turns these into the state at each chunk's start (an elementwise recurrence
-// over the chunks, which also leaves the final state in the slot). MODE 2: the outputs of every chunk.
-// LDS (floats): C, B [64][NP + 4], x [64][80], scores [64][66], l, dt, weights [64] each; N <= 128.
+// ssd_state_kernel: the second term of S' of every chunk -> workspace, the chunk's whole decay -> wdec. ssd_carry_kernel
+// turns these into the state at each chunk's start (an elementwise recurrence over the chunks, which also leaves the
+// final state in the slot). ssd_out_kernel: the outputs of every chunk.
+//
+// Both chunk kernels, grid (B * max_chunks, heads / HPW, ceil(dv / 64)): a workgroup takes HPW heads of one group in
+// turn. What the heads share stays in registers: B (or C) as the first operand of every product, and the scores C B^T.
+// Of a head only x and the state are staged in LDS, loaded into registers while the head before it is worked on; two
+// workgroups fit a compute unit. Four rows of the inner index at a time are one instruction: lane group q takes rows
+// 16 t + 4 q + e, so that first operands are read 16 bytes at a time. N <= 128.
+// Bound by memory and the fp32 matrix instruction in about equal parts: 2407 tokens of 128 heads of 128 x 64 take 100 us
+// and 210 us, their bytes 50 and 70 (with one head a workgroup, and B, C and four copies of the state's loads, 286 and 717).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-constexpr int kSC = 64, kXS = 80, kGS = 66;
+constexpr int kSC = 64;
+constexpr int kXS = 68;      // LDS row of x, state and scores: rows 4 apart fall 16 banks apart
+constexpr int kBS = 132;     // ... of B
+constexpr int kTiles = 8;    // 16-row pieces of N, at most
 
 struct SsdArgs {
   const float* xbc;
@@ -182,169 +192,223 @@ struct SsdArgs {
   float* y;
   float* ws;    // [B * max_chunks][heads][N][dv]
   float* wdec;  // [B * max_chunks][heads]
-  int heads, groups, N, dv, max_chunks;
+  int heads, groups, N, dv, max_chunks, hpw;  // hpw: heads per workgroup
 };
 
-template <int MODE>
-__global__ void __launch_bounds__(256) ssd_chunk_kernel(SsdArgs p) {
-  extern __shared__ float lds[];
+// four values at `at`, those from `left` on are zero. VEC: they start on 16 bytes and are all there or none
+template <bool VEC>
+__device__ __forceinline__ float4 ssd_load4(const float* at, int left) {
+  if (VEC) return left > 0 ? *(const float4*)at : make_float4(0.f, 0.f, 0.f, 0.f);
+  return make_float4(left > 0 ? at[0] : 0.0f, left > 1 ? at[1] : 0.0f, left > 2 ? at[2] : 0.0f, left > 3 ? at[3] : 0.0f);
+}
+__device__ __forceinline__ f32x4_t ssd_mma(float a, float b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// lane i's step size d and running sum of log a up to token i, from the raw step size (0 from token n on)
+__device__ __forceinline__ float ssd_decay(const SsdArgs& p, int h, int lane, int n, float raw, float* d) {
+  *d = lane < n ? softplus_f(raw + p.dt_bias[h]) : 0.0f;
+  float l = lane < n ? -expf(p.A_log[h]) * *d : 0.0f;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float v = __shfl_up(l, o);
+    if (lane >= o) l += v;
+  }
+  return l;
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(256) ssd_state_kernel(SsdArgs p) {
+  __shared__ __attribute__((aligned(16))) float Xs[kSC * kXS];
+  __shared__ float wgt[4][kSC];
   const int b = blockIdx.x / p.max_chunks, cidx = blockIdx.x % p.max_chunks;
-  const int h = blockIdx.y, col0 = blockIdx.z * 64;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int t0 = p.seq_start[b], t1 = p.seq_start[b + 1];
-  const int tc = t0 + cidx * kSC;
-  if (tc >= t1) return;
-  const int n = min(kSC, t1 - tc);
-  const int N = p.N, dv = p.dv, H = p.heads, inner = H * dv;
-  const int g = h / (H / p.groups);
-  const int NP = (N + 15) / 16 * 16, NS = NP + 4;
-  float* Cs = lds;
-  float* Bs = Cs + kSC * NS;
-  float* Xs = Bs + kSC * NS;
-  float* Gs = Xs + kSC * kXS;
-  float* la = Gs + kSC * kGS;
-  float* dts = la + kSC;
-  float* wgt = dts + kSC;
-  const int fr = lane & 15, fk = lane >> 4;
-  const size_t tile = ((size_t)blockIdx.x * H + h) * N * dv;
-  // MODE 2: this lane's share of the state at the chunk's start (the B operand of C S0), fetched before anything
-  // else so that its latency passes under the staging and the score product (one wave per SIMD: nothing else hides it)
-  float sv[32][4];
-  if (MODE == 2) {
+  const int h0 = blockIdx.y * p.hpw, col0 = blockIdx.z * 64;
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (matrix instructions stand in scalar branches only)
+  const int tc = p.seq_start[b] + cidx * kSC, n = min(kSC, p.seq_start[b + 1] - tc);
+  if (n <= 0) return;
+  const int N = p.N, dv = p.dv, H = p.heads, inner = H * dv, g = h0 / (H / p.groups);
+  const int tiles = (N + 15) / 16;
+  // wave w: rows 16 (w + 4 i) + fr of B^T, tokens 16 t + 4 fk + e
+  float ba[2][4][4];
 #pragma unroll
-    for (int kk = 0; kk < 32; ++kk)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int krow = kk * 4 + fk, col = col0 + c * 16 + fr;
-        sv[kk][c] = (krow < N && col < dv) ? p.ws[tile + (size_t)krow * dv + col] : 0.0f;
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = (wave + 4 * i) * 16 + fr, j = 16 * t + 4 * fk + e;
+        ba[i][t][e] = row < N && j < n ? p.xbc[(size_t)(tc + j) * p.ldx + inner + (size_t)g * N + row] : 0.0f;
       }
-  }
-  if (wave == 0) {
-    float d = 0.0f, l = 0.0f;
-    if (lane < n) {
-      d = softplus_f(p.dt[(size_t)(tc + lane) * p.ldd + h] + p.dt_bias[h]);
-      l = -expf(p.A_log[h]) * d;
-    }
+  float4 xr[4];
+  float raw = 0.0f;
+  auto fetch = [&](int h) {
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const float v = __shfl_up(l, o);
-      if (lane >= o) l += v;
+    for (int k = 0; k < 4; ++k) {
+      const int row = (tid >> 4) + 16 * k, c = (tid & 15) * 4;
+      xr[k] = ssd_load4<VEC>(p.xbc + (size_t)(tc + min(row, n - 1)) * p.ldx + (size_t)h * dv + col0 + c,
+                             row < n ? dv - col0 - c : 0);
     }
-    la[lane] = l;
-    dts[lane] = d;
-  }
-  const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (((N | dv | inner) & 3) == 0 && (p.ldx & 3) == 0) {  // 16-byte loads and LDS stores (NS is a multiple of 4)
-    const int q = NP / 4;
-    for (int i = tid; i < kSC * q; i += 256) {
-      const int row = i / q, k = (i - row * q) * 4;
-      const bool in = row < n && k < N;
-      const float* at = p.xbc + (size_t)(tc + row) * p.ldx + inner + (size_t)g * N + k;
-      *(float4*)(Bs + row * NS + k) = in ? *(const float4*)at : zero4;
-      if (MODE == 2) *(float4*)(Cs + row * NS + k) = in ? *(const float4*)(at + (size_t)p.groups * N) : zero4;
+    raw = p.dt[(size_t)(tc + min(lane, n - 1)) * p.ldd + h];
+  };
+  fetch(h0);
+  for (int h = h0; h < h0 + p.hpw; ++h) {
+    float d;
+    const float l = ssd_decay(p, h, lane, n, raw, &d), last = __shfl(l, n - 1);
+    wgt[wave][lane] = expf(last - l) * d;
+    __syncthreads();  // the head before is done with Xs
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = (tid >> 4) + 16 * k;
+      const float w = wgt[wave][row];
+      *(float4*)(Xs + row * kXS + (tid & 15) * 4) = make_float4(xr[k].x * w, xr[k].y * w, xr[k].z * w, xr[k].w * w);
     }
-    for (int i = tid; i < kSC * 16; i += 256) {
-      const int row = i >> 4, c = (i & 15) * 4;
-      const bool in = row < n && col0 + c < dv;
-      *(float4*)(Xs + row * kXS + c) =
-          in ? *(const float4*)(p.xbc + (size_t)(tc + row) * p.ldx + (size_t)h * dv + col0 + c) : zero4;
-    }
-  } else {
-    for (int i = tid; i < kSC * NP; i += 256) {
-      const int row = i / NP, k = i - row * NP;
-      const bool in = row < n && k < N;
-      const size_t at = (size_t)(tc + row) * p.ldx + inner + (size_t)g * N + k;
-      Bs[row * NS + k] = in ? p.xbc[at] : 0.0f;
-      if (MODE == 2) Cs[row * NS + k] = in ? p.xbc[at + (size_t)p.groups * N] : 0.0f;
-    }
-    for (int i = tid; i < kSC * 64; i += 256) {
-      const int row = i >> 6, c = i & 63;
-      Xs[row * kXS + c] = (row < n && col0 + c < dv) ? p.xbc[(size_t)(tc + row) * p.ldx + (size_t)h * dv + col0 + c] : 0.0f;
-    }
-  }
-  __syncthreads();
-  if (MODE == 1) {
-    const float lal = la[n - 1];
-    if (tid < kSC) wgt[tid] = tid < n ? expf(lal - la[tid]) * dts[tid] : 0.0f;
+    if (h + 1 < h0 + p.hpw) fetch(h + 1);
     __syncthreads();
-    for (int td = wave; td < NP / 16; td += 4) {
-      f32x4_t s[4];
+    f32x4_t s[2][4];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) s[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-      for (int k = 0; k < kSC; k += 4) {
-        const int j = k + fk;
-        const float a = Bs[j * NS + td * 16 + fr] * wgt[j];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float x = Xs[(16 * t + 4 * fk + e) * kXS + c * 16 + fr];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) s[i][c] = ssd_mma(ba[i][t][e], x, s[i][c]);
+        }
+    float* out = p.ws + ((size_t)blockIdx.x * H + h) * N * dv;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (wave + 4 * i < tiles)
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Xs[j * kXS + c * 16 + fr], s[c], 0, 0, 0);
-      }
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = td * 16 + fk * 4 + r, col = col0 + c * 16 + fr;
-          if (row < N && col < dv) p.ws[tile + (size_t)row * dv + col] = s[c][r];
-        }
-    }
-    if (tid == 0 && blockIdx.z == 0) p.wdec[(size_t)blockIdx.x * H + h] = expf(lal);
-    return;
+          for (int r = 0; r < 4; ++r) {
+            const int row = (wave + 4 * i) * 16 + fk * 4 + r, col = col0 + c * 16 + fr;
+            if (row < N && col < dv) out[(size_t)row * dv + col] = s[i][c][r];
+          }
+    if (tid == 0 && blockIdx.z == 0) p.wdec[(size_t)blockIdx.x * H + h] = expf(last);
   }
-  // ---- MODE 2: wave w owns tokens 16 w .. 16 w + 15
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(256, 2) ssd_out_kernel(SsdArgs p) {
+  __shared__ __attribute__((aligned(16))) float Xs[kSC * kXS], Ss[kTiles * 16 * kXS], Gs[kSC * kXS];
+  __shared__ float la[4][kSC], dts[4][kSC];
+  static_assert(kSC * kBS <= kTiles * 16 * kXS, "B is staged where the state will be");
+  const int b = blockIdx.x / p.max_chunks, cidx = blockIdx.x % p.max_chunks;
+  const int h0 = blockIdx.y * p.hpw, col0 = blockIdx.z * 64;
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (matrix instructions stand in scalar branches only)
+  const int tc = p.seq_start[b] + cidx * kSC, n = min(kSC, p.seq_start[b + 1] - tc);
+  if (n <= 0) return;
+  const int N = p.N, dv = p.dv, H = p.heads, inner = H * dv, g = h0 / (H / p.groups);
+  const int tiles = (N + 15) / 16;
+  const float* bc = p.xbc + (size_t)tc * p.ldx + inner + (size_t)g * N;
+  // wave w owns tokens 16 w .. + 15: C of row 16 w + fr, states 16 t + 4 fk + e
   const int ti = wave;
-  {
-    f32x4_t acc[4];
+  float4 ca[kTiles];
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj) acc[tj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const float* qa = Cs + (ti * 16 + fr) * NS + fk;
-    const float* kb = Bs + fr * NS + fk;
-#pragma unroll 2
-    for (int k = 0; k < NP; k += 4) {
-      const float a = qa[k];
+  for (int t = 0; t < kTiles; ++t) {
+    const int row = ti * 16 + fr, k = 16 * t + 4 * fk;
+    ca[t] = ssd_load4<VEC>(bc + (size_t)min(row, n - 1) * p.ldx + (size_t)p.groups * N + min(k, N - 1), row < n ? N - k : 0);
+  }
+  for (int i = tid; i < kSC * kTiles * 4; i += 256) {
+    const int row = i / (kTiles * 4), k = i % (kTiles * 4) * 4;
+    *(float4*)(Ss + row * kBS + k) = ssd_load4<VEC>(bc + (size_t)min(row, n - 1) * p.ldx + min(k, N - 1), row < n ? N - k : 0);
+  }
+  float4 xr[4], sr[kTiles];
+  float raw = 0.0f;
+  auto fetch = [&](int h) {
+    const int c = (tid & 15) * 4;
 #pragma unroll
-      for (int tj = 0; tj < 4; ++tj)
-        if (tj <= ti) acc[tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, kb[tj * 16 * NS + k], acc[tj], 0, 0, 0);
+    for (int k = 0; k < 4; ++k) {
+      const int row = (tid >> 4) + 16 * k;
+      xr[k] = ssd_load4<VEC>(p.xbc + (size_t)(tc + min(row, n - 1)) * p.ldx + (size_t)h * dv + col0 + c,
+                             row < n ? dv - col0 - c : 0);
     }
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj)
+    for (int k = 0; k < kTiles; ++k) {
+      const int row = (tid >> 4) + 16 * k;
+      sr[k] = ssd_load4<VEC>(p.ws + (((size_t)blockIdx.x * H + h) * N + min(row, N - 1)) * dv + col0 + c,
+                             row < N ? dv - col0 - c : 0);
+    }
+    raw = p.dt[(size_t)(tc + min(lane, n - 1)) * p.ldd + h];
+  };
+  fetch(h0);
+  __syncthreads();
+  f32x4_t cb[4];  // C_i . B_j of this wave's rows, j in piece tj <= ti
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj) {
+    cb[tj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (tj > ti) continue;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      if (t >= tiles) continue;
+      const float4 k4 = *(const float4*)(Ss + (tj * 16 + fr) * kBS + 16 * t + 4 * fk);
+      cb[tj] = ssd_mma(ca[t].x, k4.x, cb[tj]);
+      cb[tj] = ssd_mma(ca[t].y, k4.y, cb[tj]);
+      cb[tj] = ssd_mma(ca[t].z, k4.z, cb[tj]);
+      cb[tj] = ssd_mma(ca[t].w, k4.w, cb[tj]);
+    }
+  }
+  for (int h = h0; h < h0 + p.hpw; ++h) {
+    float d;
+    const float l = ssd_decay(p, h, lane, n, raw, &d);
+    la[wave][lane] = l, dts[wave][lane] = d;
+    __syncthreads();  // the head before is done with Xs and Ss (the first: the scores with B)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) *(float4*)(Xs + ((tid >> 4) + 16 * k) * kXS + (tid & 15) * 4) = xr[k];
+#pragma unroll
+    for (int k = 0; k < kTiles; ++k) *(float4*)(Ss + ((tid >> 4) + 16 * k) * kXS + (tid & 15) * 4) = sr[k];
+    if (h + 1 < h0 + p.hpw) fetch(h + 1);
+    float li[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) li[r] = la[wave][ti * 16 + fk * 4 + r];
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj) {  // (a wave's own rows: no barrier)
+      const int j = tj * 16 + fr;
+      const float lj = la[wave][j], dj = dts[wave][j];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = ti * 16 + fk * 4 + r, j = tj * 16 + fr;
-        Gs[i * kGS + j] = j <= i ? acc[tj][r] * expf(la[i] - la[j]) * dts[j] : 0.0f;
+        const int i = ti * 16 + fk * 4 + r;
+        if (tj <= ti) Gs[i * kXS + j] = j <= i ? cb[tj][r] * expf(li[r] - lj) * dj : 0.0f;
       }
-  }
-  f32x4_t o[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) o[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int kk = 0; kk < 32; ++kk) {
-    if (kk * 4 < NP) {
-      const float a = Cs[(ti * 16 + fr) * NS + kk * 4 + fk];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sv[kk][c], o[c], 0, 0, 0);
     }
-  }
+    __syncthreads();
+    f32x4_t o[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < 4; ++c) o[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto mul = [&](float4 a, const float* at) {  // += a . four rows
+      const float av[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[c][r] *= expf(la[ti * 16 + fk * 4 + r]);
-  __syncthreads();
-#pragma unroll 4
-  for (int k = 0; k < (ti + 1) * 16; k += 4) {
-    const float a = Gs[(ti * 16 + fr) * kGS + k + fk];
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[c] = ssd_mma(av[e], at[e * kXS + c * 16 + fr], o[c]);
+    };
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+      if (t < tiles) mul(ca[t], Ss + (16 * t + 4 * fk) * kXS);
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-      o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Xs[(k + fk) * kXS + c * 16 + fr], o[c], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[c][r] *= expf(li[r]);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (t <= ti) mul(*(const float4*)(Gs + (ti * 16 + fr) * kXS + 16 * t + 4 * fk), Xs + (16 * t + 4 * fk) * kXS);
+    const float Dh = p.D[h];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = ti * 16 + fk * 4 + r, col = col0 + c * 16 + fr;
+        if (i < n && col < dv)
+          p.y[(size_t)(tc + i) * inner + (size_t)h * dv + col] = fmaf(Dh, Xs[i * kXS + c * 16 + fr], o[c][r]);
+      }
   }
-  const float Dh = p.D[h];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = ti * 16 + fk * 4 + r, col = col0 + c * 16 + fr;
-      if (i < n && col < dv)
-        p.y[(size_t)(tc + i) * inner + (size_t)h * dv + col] = fmaf(Dh, Xs[i * kXS + c * 16 + fr], o[c][r]);
-    }
 }
 
 // grid (B, heads, ceil(N dv / 256)): one state element per thread walks its sequence's chunks: the workspace's local
@@ -364,11 +428,6 @@ __global__ void __launch_bounds__(256) ssd_carry_kernel(SsdArgs p) {
     s = fmaf(p.wdec[idx], s, local);
   }
   *st = s;
-}
-
-static size_t ssd_lds(int N) {
-  const int NP = (N + 15) / 16 * 16;
-  return sizeof(float) * ((size_t)2 * kSC * (NP + 4) + kSC * kXS + kSC * kGS + 3 * kSC);
 }
 
 // ------------------------------------------------------------------------------------------------ channel scan
@@ -605,19 +664,17 @@ extern "C" int lgs_ssm_scan(const float* xbc, long ldx, const float* dt, long ld
     LGA_CHECK_ARG(wdec && max_chunks > 0 && N <= 128, "lgs_ssm_scan: the prompt form serves state sizes up to 128");
     LGA_CHECK_ARG((long)B * max_chunks < (1L << 31) && (dv + 63) / 64 <= 65535, "lgs_ssm_scan: too many chunks");
     lgs::SsdArgs p{xbc, ldx, dt, ldd, dt_bias, A_log, D, state, seq_start, seq_slot, seq_pos0, y, ws, wdec,
-                   heads, groups, N, dv, max_chunks};
-    const size_t lds = lgs::ssd_lds(N);
-    for (auto* fn : {lgs::ssd_chunk_kernel<1>, lgs::ssd_chunk_kernel<2>}) {
-      const hipError_t e = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) {
-        lga_set_error(hipGetErrorString(e));
-        return (int)e;
-      }
-    }
-    const dim3 grid(B * max_chunks, heads, (dv + 63) / 64);
-    lgs::ssd_chunk_kernel<1><<<grid, 256, lds, stream>>>(p);
+                   heads, groups, N, dv, max_chunks, 1};
+    // heads per workgroup: up to four share the scores, as long as two workgroups for every compute unit are left
+    const int per_group = heads / groups;
+    while (p.hpw < 4 && per_group % (p.hpw * 2) == 0 && (long)B * max_chunks * heads / (p.hpw * 2) >= 512) p.hpw *= 2;
+    const dim3 grid(B * max_chunks, heads / p.hpw, (dv + 63) / 64);
+    const bool vec = N % 4 == 0 && dv % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)xbc | (uintptr_t)ws) % 16 == 0;
+    if (vec) lgs::ssd_state_kernel<true><<<grid, 256, 0, stream>>>(p);
+    else lgs::ssd_state_kernel<false><<<grid, 256, 0, stream>>>(p);
     lgs::ssd_carry_kernel<<<dim3(B, heads, (N * dv + 255) / 256), 256, 0, stream>>>(p);
-    lgs::ssd_chunk_kernel<2><<<grid, 256, lds, stream>>>(p);
+    if (vec) lgs::ssd_out_kernel<true><<<grid, 256, 0, stream>>>(p);
+    else lgs::ssd_out_kernel<false><<<grid, 256, 0, stream>>>(p);
     LGA_LAUNCH_RETURN();
   }
   lgs::ScanArgs p{xbc, ldx, dt, ldd, dt_bias, A_log, D, state, seq_start, seq_slot, seq_pos0, y, heads, groups, N, dv};

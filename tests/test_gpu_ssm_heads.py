@@ -1,0 +1,33 @@
+"""The prompt form of the selective scan where a workgroup takes several heads of a group in turn (csrc/seq_ssm.hip:
+ssd_state_kernel, ssd_out_kernel), against the token-by-token form: one, two and four heads per workgroup, sizes whose
+rows start on 16 bytes and sizes whose do not, chunks that end anywhere. Tolerance: both forms' fp32 sums, each held to
+2e-5 of the largest value against float64 by their own tests."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,groups,N,dv", [(32, 2, 128, 64), (32, 2, 23, 5), (12, 2, 40, 72), (30, 2, 16, 64), (64, 64, 8, 4)])
+def test_prompt_form_against_token_walk(heads, groups, N, dv):
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import StepBatch
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(N + dv)
+    lens, pos0 = [1500, 700, 64, 65], [0, 9, 3, 0]
+    T, inner = sum(lens), heads * dv
+    rand = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    xbc, raw = rand(T, inner + 2 * groups * N) * 0.5, rand(T, heads)
+    dt_bias, A_log, D = rand(heads) - 1.0, rand(heads), rand(heads)
+    stale = rand(len(lens) + 1, heads, N, dv)
+    step = StepBatch.build([(i, p0, [0] * n) for i, (n, p0) in enumerate(zip(lens, pos0))], dev)
+    y, state = {}, {}
+    for chunked in (False, True):
+        state[chunked] = stale.clone()
+        y[chunked] = seq_ops.ssm_scan(xbc, raw, 0, dt_bias, A_log, D, state[chunked], step.seq_start, step.seq_slot,
+                                      step.seq_pos0, heads=heads, groups=groups, N=N, dv=dv, max_len=max(lens), chunked=chunked)
+    assert float((y[True] - y[False]).abs().max()) < 4e-5 * float(y[False].abs().max())
+    assert float((state[True] - state[False]).abs().max()) < 4e-5 * max(1.0, float(state[False].abs().max()))
+    assert torch.equal(state[True][-1], stale[-1])
