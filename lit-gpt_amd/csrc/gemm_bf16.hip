@@ -98,7 +98,7 @@ GemmPlan bf16_plan(int M, int N, int K, bool dual) {
   const long cols = dual ? 2L * N : N;
   if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1};
   if (M > 1024 && (M + 255) / 256 * (cols / 128) >= 256) return GemmPlan{-1, 1};
-  return gemm_tile_plan((int)cols, M, K, 1, false, 0);
+  return gemm_tile_plan(M, (int)cols, K, 1, false, 0, true);
 }
 
 size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {

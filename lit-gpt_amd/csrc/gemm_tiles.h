@@ -157,7 +157,6 @@ __device__ __forceinline__ void gemm_dma_at(int R, int lane, int* row, int* chun
 // what a large matrix product reaches on this card), of 256 x 128 1.02, of 128 x 128 0.63 alone on a compute unit and
 // 1.14 for two, of 64 x 128 0.43. The larger tile moves fewer bytes per product, the smaller ones fill the chip when
 // rows or columns are few. A workgroup's start and end cost about 3 us.
-// M rows of A, N of B.
 struct GemmForm {
   int bm, bn, slots;  // slots: workgroups of the whole chip at a time
   float step_us;
@@ -172,16 +171,18 @@ struct GemmPlan {
 // Rounds of workgroups times what one takes; several ranges of K cost a second launch that reads them all. E.g.
 // 2048 x 2048 x 5632: 256 tiles of 128 x 128 in one round, 55 us (64 of 256 x 256: 131); 128 x 4096 x 4096: 64 tiles of
 // 64 x 128 in four ranges of K, 16 us (whole: 41); before these tiles 126 and 86 us.
-inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int ksplit) {
+// rows_b: the rows are the tile's B, the columns its A.
+inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int ksplit, bool rows_b = false) {
   GemmPlan best{-1, 1};
   if (K % 64 != 0 || M <= 0) return best;
   const int steps = K / 64;
   float best_us = 0.0f;
   for (int f = 0; f < (int)(sizeof(kGemmForms) / sizeof(kGemmForms[0])); ++f) {
     const GemmForm& t = kGemmForms[f];
-    const float nt = (float)((N + t.bn - 1) / t.bn);
+    const int rows = rows_b ? t.bn : t.bm, cols = rows_b ? t.bm : t.bn;
+    const float nt = (float)((N + cols - 1) / cols);
     // a range of the list ends somewhere in its last tile
-    const float mt = grouped ? (float)M / t.bm + 0.5f * batch : (float)((M + t.bm - 1) / t.bm) * batch;
+    const float mt = grouped ? (float)M / rows + 0.5f * batch : (float)((M + rows - 1) / rows) * batch;
     const int s_lo = ksplit > 0 ? ksplit : 1, s_hi = ksplit > 0 ? ksplit : (batch > 1 || grouped ? 1 : 16);
     for (int s = s_lo; s <= s_hi && (s == s_lo || steps / s >= 4); ++s) {
       const int per = (steps + s - 1) / s;

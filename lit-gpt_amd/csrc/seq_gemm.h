@@ -30,4 +30,22 @@ using lga::GemmPlan;
 GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit);
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream);
 
+// the gated unit on two products: act(gate) * up, or clamped: g sigmoid(alpha g) (u + shift) with g = min(gate, limit),
+// u = clamp(up, -limit, limit) (limit <= 0: no clamps)
+struct GluForm {
+  int clamped, act;
+  float alpha, limit, shift;
+  size_t up;  // where the up rows begin in W, from the gate rows (elements)
+};
+template <bool CLAMPED>
+__device__ __forceinline__ float glu_f(const GluForm& f, float g, float u) {
+  if (!CLAMPED) return act_f(f.act, g) * u;
+  if (f.limit > 0.0f) {
+    g = fminf(g, f.limit);
+    u = fminf(fmaxf(u, -f.limit), f.limit);
+  }
+  return g * sigmoid_f(f.alpha * g) * (u + f.shift);
+}
+int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream);
+
 }  // namespace lgs

@@ -524,6 +524,34 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
   LGA_LAUNCH_RETURN();
 }
 
+// whether lgs_linear_glu takes a product of M rows (the sizes of all its groups) on gate | up of n columns each: not where
+// the plain product is better made in ranges of K
+extern "C" int lgs_linear_glu_fits(int M, int n, int K, int grouped) {
+  return M > 8 && n >= 32 && n % 4 == 0 && n <= (1 << 29) && K > 0 && K % 64 == 0 &&
+                 (grouped || lgs::gemm_plan(M, 2 * n, K, 1, false, 0).ksplit == 1)
+             ? 1
+             : 0;
+}
+
+extern "C" int lgs_linear_glu(const void* a, long lda, const void* w, long stride_w, long up_rows, void* y, long ldy, int M,
+                              int n, int K, int batch, const int* a_rows, const int* z_start, int act, int clamped,
+                              float alpha, float limit, float shift, hipStream_t stream) {
+  LGA_CHECK_ARG(a && w && y, "lgs_linear_glu: null pointer");
+  LGA_CHECK_ARG(lgs_linear_glu_fits(M, n, K, z_start != nullptr), "lgs_linear_glu: not one of its sizes");
+  LGA_CHECK_ARG(batch > 0 && batch <= 65535 && (batch == 1 || z_start), "lgs_linear_glu: batches are groups of rows");
+  LGA_CHECK_ARG(lda >= K && ldy >= n && up_rows >= n, "lgs_linear_glu: row strides shorter than the rows");
+  LGA_CHECK_ARG(act >= 0 && act <= lgs::kActSigmoid, "lgs_linear_glu: unknown activation");
+  LGA_CHECK_ARG(((uintptr_t)a | (uintptr_t)w) % 16 == 0 && (uintptr_t)y % 8 == 0 && lda % 8 == 0 && stride_w % 8 == 0 &&
+                    ldy % 4 == 0,
+                "lgs_linear_glu: rows of A and W start on 16 bytes, of Y on 8");
+  lgs::LinArgs p{nullptr, lda, 0, w, stride_w, nullptr, ldy, 0, M, n, K, 0, act, a_rows, z_start, (const uint16_t*)a,
+                 (uint16_t*)y, nullptr, nullptr, 1, 0};
+  const lgs::GluForm f{clamped, act, alpha, limit, shift, (size_t)up_rows * K};
+  const int rc = lgs::gemm_glu_launch(p, f, batch, stream);
+  if (rc) return rc;
+  LGA_LAUNCH_RETURN();
+}
+
 // ranges of K that a plain product of a bf16 A on bf16 weights is best made in (1: as one)
 extern "C" int lgs_linear_ksplit(int M, int N, int K) {
   // (a few columns are a router's logits: their sums keep one order whatever the rows, so that near-ties of the choice fall

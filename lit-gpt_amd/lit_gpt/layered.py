@@ -136,10 +136,12 @@ class Sublayer(nn.Module):
     def forward(self, h: torch.Tensor, h16: Optional[torch.Tensor], step: StepBatch, cache) -> torch.Tensor:
         """h (T, width): the normed read of the streams. Returns the sublayer's output (T, width) fp32."""
         n_in, W = self.w_in.shape
+        y = torch.empty(step.T, W, dtype=torch.float32, device=h.device)
+        if cache is None and self.b_in is None and self.module.forward_in(h16, self.w_in, y):
+            return y
         proj = torch.empty(step.T, n_in, dtype=torch.float32, device=h.device)
         seq_ops.linear(h if h16 is None else h16, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in,
                        bias=self.b_in)
-        y = torch.empty(step.T, W, dtype=torch.float32, device=h.device)
         if cache is None:
             self.module(proj, h, y, h16=h16, accumulate=False)
         else:
@@ -268,13 +270,15 @@ class SandwichSublayer(nn.Module):
             y = torch.empty(T, W, dtype=torch.float32, device=src.device)
             self.module.forward_fused(h, self.w_in, self.b_in, step, cache, y, accumulate=False)
             return [(y, None)], 1.0
+        y = torch.empty(T, W, dtype=torch.float32, device=src.device)
+        if cache is None and self.w_in is not None and self.b_in is None and self.module.forward_in(h16, self.w_in, y):
+            return [(y, None)], 1.0
         proj = None
         if self.w_in is not None and self.module.wants_proj(T):
             n_in = self.w_in.shape[0]
             proj = torch.empty(T, n_in, dtype=torch.float32, device=src.device)
             seq_ops.linear(src, self.w_in, M=T, N=n_in, K=W, y=proj, lda=W, ldy=n_in, bias=self.b_in,
                            ksplit=0 if src.dtype == torch.bfloat16 else seq_ops.thin_ksplit(T, n_in, W, self.w_in))
-        y = torch.empty(T, W, dtype=torch.float32, device=src.device)
         if cache is None:
             self.module(proj, h, y, h16=h16, accumulate=False)
         elif getattr(self.module, "branch_norm", False):

@@ -98,6 +98,11 @@ class InputReader(nn.Module):
         """Whether the module makes its input projection itself in this step (``forward_fused``)."""
         return False
 
+    def forward_in(self, h16: Optional[torch.Tensor], w_in: torch.Tensor, x: torch.Tensor, accumulate: bool = False) -> bool:
+        """A module without a cache, straight from its sublayer's input (a bf16 copy) and fused input matrix; False:
+        nothing done, the input projection and ``forward`` make it."""
+        return False
+
     def reads_f32(self, rows: int) -> bool:
         """Whether a step of ``rows`` tokens needs the module's input in fp32 beside the bf16 copy its products read."""
         return False
@@ -852,6 +857,18 @@ class GatedFeedForward(InputReader):
                                     shift=shift, bf16=bf16)
         else:
             a = seq_ops.glu(proj, self.off["gate"], self.off["up"], self.ff, self.act, bf16=bf16)
+        self._down(a, x, accumulate)
+
+    def forward_in(self, h16: Optional[torch.Tensor], w_in: torch.Tensor, x: torch.Tensor, accumulate: bool = False) -> bool:
+        """Where the input product and the gated unit fit one launch (prompts, bf16 weights)."""
+        T = x.shape[0]
+        if self.off["gate"] != 0 or not _tiles16(T, self.w_down) or not seq_ops.glu_fits(h16, w_in, T, self.ff):
+            return False
+        self._down(seq_ops.linear_glu(h16, w_in, M=T, n=self.ff, up=self.off["up"], act=self.act, clamp=self.clamp), x,
+                   accumulate)
+        return True
+
+    def _down(self, a: torch.Tensor, x: torch.Tensor, accumulate: bool) -> None:
         W = x.shape[1]
         seq_ops.linear(a, self.w_down, M=a.shape[0], N=W, K=self.ff, y=x, lda=self.ff, ldy=W, accumulate=accumulate)
 
@@ -994,7 +1011,9 @@ class SparseFeedForward(InputReader):
         pairs = T * top
         z_start, tok_of, where = seq_ops.moe_sort(ids, self.n_router)
         a_dtype = torch.bfloat16 if self.w_down.dtype == torch.bfloat16 else torch.float32
-        if self.gated:
+        if self.gated and seq_ops.glu_fits(h16, self.w_up, pairs, F, grouped=True):
+            a = seq_ops.linear_glu(h16, self.w_up, M=pairs, n=F, up=F, act=self.act, a_rows=tok_of, z_start=z_start)
+        elif self.gated:
             gu = torch.empty(pairs, 2 * F, dtype=torch.float32, device=x.device)
             seq_ops.linear(h if h16 is None else h16, self.w_up, M=pairs, N=2 * F, K=W, y=gu, lda=W, ldy=2 * F, batch=E,
                            stride_w=2 * F * W, a_rows=tok_of, z_start=z_start)

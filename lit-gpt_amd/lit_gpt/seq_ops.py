@@ -33,6 +33,8 @@ SIGNATURES = {
     "lgs_last_error_string": [],
     "lgs_linear": [_P, _L, _L, _P, _I, _L, _P, _L, _L, _I, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _P, _I, _P],
     "lgs_linear_ksplit": [_I, _I, _I],
+    "lgs_linear_glu_fits": [_I, _I, _I, _I],
+    "lgs_linear_glu": [_P, _L, _P, _L, _L, _P, _L, _I, _I, _I, _I, _P, _P, _I, _I, _F, _F, _F, _P],
     "lgs_embed": [_P, _P, _I, _F, _P, _I, _I, _I, _P],
     "lgs_rmsnorm": [_P, _L, _P, _F, _F, _P, _L, _I, _I, _I, _P, _P],
     "lgs_gather_rows": [_P, _P, _P, _I, _I, _P],
@@ -386,6 +388,33 @@ def expanded_latent_attention(q: torch.Tensor, q_off: int, kv: torch.Tensor, cac
                                               _dev(seq_slot, "seq_slot", I32), _dev(seq_pos0, "seq_pos0", I32),
                                               None if bf16 else out.data_ptr(), out.data_ptr() if bf16 else None, B,
                                               int(max_len), H, d + dr, dv, float(scale), int(window), _stream()))
+    return out
+
+
+def glu_fits(a: Optional[torch.Tensor], w: torch.Tensor, M: int, n: int, grouped: bool = False) -> bool:
+    """Whether ``linear_glu`` makes a gated unit of n columns for M rows of ``a`` (rows of w.shape[-1] values)."""
+    K = w.shape[-1]
+    return a is not None and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and \
+        bool(load_library().lgs_linear_glu_fits(M, n, K, int(grouped))) and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+
+
+def linear_glu(a: torch.Tensor, w: torch.Tensor, *, M: int, n: int, up: int, act: int = 0,
+               clamp: Optional[tuple] = None, a_rows: Optional[torch.Tensor] = None,
+               z_start: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """bf16(act(A Wg^T) * (A Wu^T)) (M, n) in one launch, to the bits of ``linear`` and ``glu`` (``glu_clamped`` with
+    ``clamp`` = (alpha, limit, shift)) in turn: a bf16 rows of K values, w bf16 (rows, K) or (batch, rows, K), whose first n
+    rows are the gate's and whose rows from ``up`` on the up product's. ``a_rows`` / ``z_start``: as in ``linear``."""
+    K = w.shape[-1]
+    batch = w.shape[0] if w.dim() == 3 else 1
+    if a.shape[-1] != K or w.shape[-2] < up + n or (z_start is None) != (w.dim() == 2) or \
+            (z_start is not None and z_start.numel() <= batch) or (a_rows is None and a.shape[0] < M):
+        raise ValueError("linear_glu: shapes")
+    out = torch.empty(M, n, dtype=torch.bfloat16, device=a.device)
+    alpha, limit, shift = clamp if clamp is not None else (0.0, 0.0, 0.0)
+    _check(load_library().lgs_linear_glu(_dev(a, "a", torch.bfloat16), K, _dev(w, "w", torch.bfloat16), w.shape[-2] * K, up,
+                                         out.data_ptr(), n, M, n, K, batch, _opt(a_rows, "a_rows", I32),
+                                         _opt(z_start, "z_start", I32), act, int(clamp is not None), float(alpha),
+                                         float(limit), float(shift), _stream()))
     return out
 
 
