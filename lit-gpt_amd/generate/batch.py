@@ -14,6 +14,7 @@ import sys
 from pathlib import Path
 from typing import Dict, Hashable, List, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 wd = Path(__file__).parent.parent.resolve()
@@ -43,6 +44,26 @@ class SlotPool:
         self.free.append(slot)
 
 
+def _checked(tokens: Sequence[int], vocab: int) -> Sequence[int]:
+    """The token ids, those of long prompts of plain whole numbers as a numpy array; ValueError if one is outside the
+    vocabulary. (An id at a time, 4096 of them cost 0.3 ms here and 0.4 in the step's table.)"""
+    ids = None
+    if len(tokens) > 64:
+        try:
+            ids = np.array(tokens)
+        except Exception:
+            pass
+    if ids is None or ids.ndim != 1 or ids.dtype.kind not in "iu":
+        for t in tokens:
+            if not 0 <= int(t) < vocab:
+                raise ValueError(f"token id {t} outside the vocabulary")
+        return tokens
+    out = (ids < 0) | (ids >= vocab)
+    if out.any():
+        raise ValueError(f"token id {ids[out.argmax()]} outside the vocabulary")
+    return ids
+
+
 class BatchEngine:
     def __init__(self, model, max_seq_length: int, slots: int = 4) -> None:
         self.model = model
@@ -64,10 +85,7 @@ class BatchEngine:
             if held + len(tokens) > model.max_seq_length:
                 raise ValueError(f"request {req!r} would hold {held + len(tokens)} tokens, the cache has room for "
                                  f"{model.max_seq_length}")
-            for t in tokens:
-                if not 0 <= int(t) < model.config.vocab:
-                    raise ValueError(f"token id {t} outside the vocabulary")
-            table.append((slot, held, tokens))
+            table.append((slot, held, _checked(tokens, model.config.vocab)))
             rows += [at + int(k) for k in want]
             at += len(tokens)
             self.live[req] = (slot, held + len(tokens))

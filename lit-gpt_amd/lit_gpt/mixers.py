@@ -25,6 +25,7 @@ import math
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 import torch.nn as nn
 
@@ -49,6 +50,16 @@ class StepBatch:
     @classmethod
     def build(cls, entries: Sequence[Tuple[int, int, Sequence[int]]], device: torch.device) -> "StepBatch":
         """entries: (slot, first position, token ids) per sequence; one host -> device copy for the whole table."""
+        if any(isinstance(toks, np.ndarray) for _, _, toks in entries) and all(
+                len(toks) and (isinstance(toks, np.ndarray) or all(type(t) is int for t in toks)) for _, _, toks in entries):
+            n = np.array([len(toks) for _, _, toks in entries])
+            sslot, spos = np.array([s for s, _, _ in entries]), np.array([p0 for _, p0, _ in entries])
+            start = np.concatenate(([0], n.cumsum()))
+            T, B = int(start[-1]), len(entries)
+            pos = np.arange(T) + np.repeat(spos - start[:-1], n)
+            flat = np.concatenate([*(toks for _, _, toks in entries), np.repeat(sslot, n), pos, start, sslot, spos])
+            parts = torch.split(torch.from_numpy(flat.astype(np.int32)).to(device), [T, T, T, B + 1, B, B])
+            return cls(*parts, T=T, B=B, max_len=int(n.max()), fresh=not spos.any())
         tokens, slot, pos, start, sslot, spos = [], [], [], [0], [], []
         for s, p0, toks in entries:
             n = len(toks)
