@@ -118,6 +118,90 @@ __global__ void __launch_bounds__(256) lin_gemv_kernel(LinArgs p) {
   }
 }
 
+// the value that the lane eight further on in the row of 16 holds
+__device__ __forceinline__ uint32_t rows_up8(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false);
+}
+// Three to eight rows of A on bf16 weights, on the matrix cores: the operands are the same (A rounded to bf16), and a weight
+// costs no vector instruction however many rows there are. A workgroup owns 16 NR columns; its KW waves each take a
+// range of K, 128 values at a time: PF blocks ahead a lane loads 4 x 16 bytes of its own row of W (256 bytes of a row
+// together) and half of its row of A, of whose 32-value pieces the lanes of the upper eight rows hold every second one.
+// Sums: two instructions, then vector adds, then the ranges pairwise, so that the error against float64 is what the
+// lanes' sums of lin_gemv_kernel leave (rms of 8 rows at K 2048 / 4096 / 11008: 7.4e-8 / 8.0e-8 / 9.5e-8 of the results,
+// 7.5e-8 / 8.4e-8 / 1.1e-7 there; one chain of instructions 1.5 to 3 times as much).
+// Bound by memory, and by the loads' latency where a wave's range is a few blocks: 8 x 22016 x 4096 51 us (3.5 TB/s), 8 x
+// 4096 x 11008 28 us (3.2 TB/s); a lane's sums 84 and 85.
+template <int NR, int KW>
+__global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
+  constexpr int PF = 3;
+  __shared__ f32x4_t part[KW][NR][64];
+  const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int z = blockIdx.y, n0 = blockIdx.x * (16 * NR);
+  const int nb = p.K / 128, b0 = wave * nb / KW, b1 = (wave + 1) * nb / KW;
+  const float* a = p.a + (size_t)z * p.sa + (size_t)min(l15 & 7, p.M - 1) * p.lda + (l15 >> 3) * 32 + q4 * 8;
+  const uint16_t* w[NR];
+#pragma unroll
+  for (int j = 0; j < NR; ++j)
+    w[j] = (const uint16_t*)p.w + (size_t)z * p.sw + (size_t)min(n0 + j * 16 + l15, p.N - 1) * p.K + q4 * 8;
+  bf16x8_t wr[PF][NR][4];
+  float4 ar[PF][4];
+  auto fetch = [&](int b, int s) {  // (past the range: its last block, never used)
+    const size_t at = (size_t)max(min(b, b1 - 1), 0) * 128;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) ar[s][2 * u] = *(const float4*)(a + at + u * 64), ar[s][2 * u + 1] = *(const float4*)(a + at + u * 64 + 4);
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) wr[s][j][m] = *(const bf16x8_t*)(w[j] + at + m * 32);
+  };
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[4][NR];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < NR; ++j) acc[i][j] = zero;
+#pragma unroll
+  for (int s = 0; s < PF; ++s) fetch(b0 + s, s);
+  for (int b = b0; b < b1; b += 2 * PF) {
+#pragma unroll
+    for (int s = 0; s < 2 * PF; ++s) {
+      if (b + s < b1) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const float4 lo = ar[s % PF][2 * u], hi = ar[s % PF][2 * u + 1];
+          const uint4 x = make_uint4(pack2(lo.x, lo.y), pack2(lo.z, lo.w), pack2(hi.x, hi.y), pack2(hi.z, hi.w));
+          const uint4 t = make_uint4(rows_up8(x.x), rows_up8(x.y), rows_up8(x.z), rows_up8(x.w));
+#pragma unroll
+          for (int j = 0; j < NR; ++j) {
+            f32x4_t v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[s % PF][j][2 * u], __builtin_bit_cast(bf16x8_t, x), zero, 0, 0, 0);
+            v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[s % PF][j][2 * u + 1], __builtin_bit_cast(bf16x8_t, t), v, 0, 0, 0);
+            acc[(s & 1) * 2 + u][j] += v;
+          }
+        }
+        fetch(b + s + PF, s % PF);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NR; ++j) part[wave][j][lane] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
+  __syncthreads();
+  if (tid >= NR * 64 || l15 >= p.M) return;
+  const int j = NR > 1 ? wave : 0;
+  f32x4_t v = zero;
+#pragma unroll
+  for (int k = 0; k < KW; k += 4)
+    v += (part[k][j][lane] + part[k + 1][j][lane]) + (part[k + 2][j][lane] + part[k + 3][j][lane]);
+  float* y = p.y + (size_t)z * p.sy + (size_t)l15 * p.ldy;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int n = n0 + j * 16 + q4 * 4 + r;
+    if (n >= p.N) continue;
+    const float o = act_f(p.act, v[r] + (p.bias ? p.bias[n] : 0.0f));
+    y[n] = p.accumulate ? y[n] + o : o;
+  }
+}
+
 // ------------------------------------------------------------------------------------------------ MFMA tiles
 constexpr int BM = 128, BN = 128, BK = 64;
 constexpr int TILE_BYTES = BM * BK * 2;
@@ -463,6 +547,16 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
                  a_bf16 ? (const uint16_t*)a : nullptr, y_bf16 ? (uint16_t*)y : nullptr, bias, nullptr, 1, 0};
   LGA_CHECK_ARG(ksplit >= 1 && (ksplit == 1 || (part && !w_f32 && batch == 1 && !z_start && !a_rows && M > 8 && M <= 65535)),
                 "lgs_linear: K is split for one plain product on the MFMA tiles, with a workspace");
+  // Several rows on the matrix cores (us here / a lane's sums): 5 to 8 rows of at least 2048 columns (8 x 2048 x 2048 11.5 /
+  // 12.4, x 8256 x 2048 21 / 26, x 4096 x 11008 28 / 85, x 32000 x 4096 68 / 104; x 512 x 2048 11.4 / 6.1), 3 and 4 rows
+  // from K 4096 (4 x 4096 x 4096 12.7 / 20.8, x 20608 x 4096 45 / 55; x 10304 x 2048 21 / 19); 2 x 20608 x 4096 44 / 38
+  if (!z_start && !a_rows && !w_f32 && M > 2 && M <= 8 && N >= 2048 && (M > 4 || K >= 4096) && K % 128 == 0 && lda % 4 == 0 &&
+      stride_a % 4 == 0 && stride_w % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0) {
+    if (N > 4608) lgs::lin_rows_kernel<2, 4><<<dim3((N + 31) / 32, batch), 256, 0, stream>>>(p);
+    else if (N >= 4096) lgs::lin_rows_kernel<1, 4><<<dim3((N + 15) / 16, batch), 256, 0, stream>>>(p);
+    else lgs::lin_rows_kernel<1, 8><<<dim3((N + 15) / 16, batch), 512, 0, stream>>>(p);
+    LGA_LAUNCH_RETURN();
+  }
   if (M <= 8 && !z_start && !a_rows) {
     const int R = N >= 16384 ? 4 : (N >= 4096 ? 2 : 1);
     const bool deep = (long)N * batch <= 512 && K >= 1024;  // few columns: four waves per column
