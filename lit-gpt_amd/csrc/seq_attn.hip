@@ -524,6 +524,162 @@ __global__ void __launch_bounds__(256) diffattn_kernel(AttnArgs p) {
   }
 }
 
+// sum over the W lanes (8 or 16, aligned inside a row of 16) that share a key; every lane gets it
+template <int CTRL>
+__device__ __forceinline__ float attn_dpp(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int W>
+__device__ __forceinline__ float attn_lanes_sum(float v) {
+  v = attn_dpp<0x141>(attn_dpp<0x4E>(attn_dpp<0xB1>(v)));  // neighbours, pairs, mirrored halves of eight
+  return W == 16 ? attn_dpp<0x140>(v) : v;
+}
+
+// One token per sequence over bf16 caches whose key and value rows are 128 values (MAPS maps of 128 / MAPS, dv 128): grid
+// (B, H / HG, splits), HG query heads of one key head per workgroup. A key belongs to 16 lanes, 16 bytes of its key and
+// of its value row each; each of the workgroup's 16 such groups takes every 16th key, four at a time, whose loads are
+// in flight together and which share one rescale of the group's running maximum, normaliser and sums. These meet in
+// the wave's lanes, then in LDS, in a fixed order. Bound by the launch and the loads' latency: 8 sequences of 9 to 2047
+// keys, 16 heads on 4, 19 us, 2047 keys of two maps 9.5 (a thread a key and the scores in LDS: 53 and 15).
+template <int MAPS, int HG>
+__global__ void __launch_bounds__(256) attn_one_kernel(AttnArgs p) {
+  constexpr int U = 4, NR = HG * MAPS;
+  __shared__ float ml[4][NR][2], sums[4][NR][128];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, grp = tid >> 4;
+  const int b = blockIdx.x, h0 = blockIdx.y * HG, g = h0 / (p.H / p.G);
+  const int row = p.seq_start[b], pos = p.seq_pos0[b];
+  const size_t slot = p.seq_slot[b];
+  const int lo = p.chunk > 0 ? pos - pos % p.chunk : 0, keys = pos + 1 - lo;
+  const int per = (keys + gridDim.z - 1) / gridDim.z, from = blockIdx.z * per, to = min(keys, from + per);
+  float q[HG][8];
+#pragma unroll
+  for (int h = 0; h < HG; ++h) {
+    const float* at = p.q + (size_t)row * p.ld + (size_t)(h0 + h) * 128 + l16 * 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[h][e] = at[e];
+  }
+  float m[HG], l[HG], acc[NR][8];  // (two maps: a lane's m and l are its own map's)
+#pragma unroll
+  for (int h = 0; h < HG; ++h) m[h] = -INFINITY, l[h] = 0.0f;
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[r][e] = 0.0f;
+  const uint16_t* kc = (const uint16_t*)p.cache_k + ((slot * p.S + lo) * p.G + g) * 128 + l16 * 8;
+  const uint16_t* vc = (const uint16_t*)p.cache_v + ((slot * p.S + lo) * p.G + g) * 128 + l16 * 8;
+  const size_t step = (size_t)p.G * 128;
+  for (int u0 = from + grp; u0 < to; u0 += 16 * U) {
+    uint4 k4[U], v4[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const size_t at = (size_t)min(u0 + 16 * i, to - 1) * step;
+      k4[i] = *(const uint4*)(kc + at);
+      v4[i] = *(const uint4*)(vc + at);
+    }
+    float w[HG][U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const float kv[8] = {bflo(k4[i].x), bfhi(k4[i].x), bflo(k4[i].y), bfhi(k4[i].y),
+                           bflo(k4[i].z), bfhi(k4[i].z), bflo(k4[i].w), bfhi(k4[i].w)};
+#pragma unroll
+      for (int h = 0; h < HG; ++h) {
+        float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) s0 = fmaf(q[h][e], kv[e], s0), s1 = fmaf(q[h][e + 1], kv[e + 1], s1);
+        float s = attn_lanes_sum<16 / MAPS>(s0 + s1) * p.scale;
+        if (p.cap > 0.0f) s = p.cap * tanhf(s / p.cap);
+        w[h][i] = u0 + 16 * i < to ? s : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < HG; ++h) {
+      float mn = m[h];
+#pragma unroll
+      for (int i = 0; i < U; ++i) mn = fmaxf(mn, w[h][i]);
+      const float a = m[h] == -INFINITY ? 0.0f : expf(m[h] - mn);
+      float sum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        w[h][i] = mn == -INFINITY ? 0.0f : expf(w[h][i] - mn);
+        sum += w[h][i];
+      }
+      l[h] = l[h] * a + sum;
+      m[h] = mn;
+#pragma unroll
+      for (int f = 0; f < MAPS; ++f) {  // (the other map's weights lie with the lanes eight away)
+        const int r = h * MAPS + f;
+        const int src = (lane & ~15) | (f * 8);
+        const float ar = MAPS == 2 ? __shfl(a, src) : a;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[r][e] *= ar;
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const float wr = MAPS == 2 ? __shfl(w[h][i], src) : w[h][i];
+          const float vv[8] = {bflo(v4[i].x), bfhi(v4[i].x), bflo(v4[i].y), bfhi(v4[i].y),
+                               bflo(v4[i].z), bfhi(v4[i].z), bflo(v4[i].w), bfhi(v4[i].w)};
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[r][e] = fmaf(wr, vv[e], acc[r][e]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < HG; ++h) {  // the wave's four groups
+    const float top = fmaxf(fmaxf(m[h], __shfl_xor(m[h], 16)), fmaxf(__shfl_xor(m[h], 32), __shfl_xor(m[h], 48)));
+    const float a = m[h] == -INFINITY ? 0.0f : expf(m[h] - top);
+    float s = l[h] * a;
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+#pragma unroll
+    for (int f = 0; f < MAPS; ++f) {
+      const int r = h * MAPS + f, src = (lane & ~15) | (f * 8);
+      const float ar = MAPS == 2 ? __shfl(a, src) : a, tr = MAPS == 2 ? __shfl(top, src) : top, sr = MAPS == 2 ? __shfl(s, src) : s;
+      if (lane == 0) ml[wave][r][0] = tr, ml[wave][r][1] = sr;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float v = acc[r][e] * ar;
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+        if (lane < 16) sums[wave][r][l16 * 8 + e] = v;
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < NR * 128; i += 256) {
+    const int r = i >> 7, c = i & 127, h = h0 + r / MAPS, f = r % MAPS;
+    float top = -INFINITY, s = 0.0f, v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) top = fmaxf(top, ml[k][r][0]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float a = ml[k][r][0] == -INFINITY ? 0.0f : expf(ml[k][r][0] - top);
+      s = fmaf(ml[k][r][1], a, s);
+      v = fmaf(sums[k][r][c], a, v);
+    }
+    float* pr = p.part + (((size_t)row * p.H + h) * gridDim.z + blockIdx.z) * (MAPS * (2 + 128));
+    if (c == 0) pr[2 * f] = top, pr[2 * f + 1] = s;
+    pr[2 * MAPS + f * 128 + c] = v;
+  }
+}
+
+// query heads per workgroup of attn_one_kernel; 0: not one of its sizes
+inline int attn_one_heads(int maps, int H, int G, int d, int dv) {
+  if (maps * d != 128 || dv != 128 || H <= 0 || G <= 0 || H % G != 0) return 0;
+  const int per = H / G, most = 4 / maps;
+  return per % most == 0 ? most : (per % 2 == 0 ? 2 : 1);
+}
+template <int MAPS>
+static bool attn_one_launch(const AttnArgs& p, int cache_f32, int B, int splits, hipStream_t stream) {
+  const int hg = attn_one_heads(MAPS, p.H, p.G, p.d, p.dv);
+  if (hg == 0 || splits < 2 || cache_f32 || p.window > 0 || p.score_bias || ((uintptr_t)p.cache_k | (uintptr_t)p.cache_v) % 16 != 0)
+    return false;
+  const dim3 grid(B, p.H / hg, splits);
+  if (hg == 4) attn_one_kernel<MAPS, 4 / MAPS><<<grid, 256, 0, stream>>>(p);
+  else if (hg == 2) attn_one_kernel<MAPS, 2><<<grid, 256, 0, stream>>>(p);
+  else attn_one_kernel<MAPS, 1><<<grid, 256, 0, stream>>>(p);
+  return true;
+}
+
 // grid (T, H): merges the splits of one (token, head) in split order and finishes
 template <int MAPS>
 __global__ void __launch_bounds__(256) diffattn_combine_kernel(AttnArgs p, int splits) {
@@ -587,6 +743,9 @@ static int diffattn_launch(const AttnArgs& p, int cache_f32, dim3 grid, hipStrea
 
 }  // namespace lgs
 
+// query heads that a workgroup of the one-token form takes at a time (0: the general form)
+extern "C" int lgs_attn_one_heads(int maps, int H, int G, int d, int dv) { return lgs::attn_one_heads(maps, H, G, d, dv); }
+
 extern "C" int lgs_diffattn_prepare(float* proj, long ld, int q_off, int k_off, int v_off, void* cache_k, void* cache_v,
                                     int cache_f32, const float* inv_freq, const int* slot, const int* pos, int T, int H,
                                     int G, int d, int dv, int rot_dims, int max_seq, hipStream_t stream) {
@@ -620,7 +779,7 @@ extern "C" int lgs_diffattn(const float* q, long ld, const void* cache_k, const 
   int rc;
   if (max_len == 1) {
     p.tiles = 1;
-    rc = lgs::diffattn_launch<1, 2>(p, cache_f32, dim3(B, H, splits), stream);
+    rc = lgs::attn_one_launch<2>(p, cache_f32, B, splits, stream) ? 0 : lgs::diffattn_launch<1, 2>(p, cache_f32, dim3(B, H, splits), stream);
     if (rc == 0 && splits > 1) lgs::diffattn_combine_kernel<2><<<dim3(B, H), 256, 0, stream>>>(p, splits);
   } else {
     if (!cache_f32 && lgs::attn_tiles_fit(p, 2, 1, max_len)) {
@@ -699,7 +858,7 @@ extern "C" int lgs_sinkattn(const float* q, long ld, const void* cache_k, const 
   int rc;
   if (max_len == 1) {
     p.tiles = 1;
-    rc = lgs::diffattn_launch<1, 1>(p, cache_f32, dim3(B, H, splits), stream);
+    rc = lgs::attn_one_launch<1>(p, cache_f32, B, splits, stream) ? 0 : lgs::diffattn_launch<1, 1>(p, cache_f32, dim3(B, H, splits), stream);
     if (rc == 0 && splits > 1) lgs::diffattn_combine_kernel<1><<<dim3(B, H), 256, 0, stream>>>(p, splits);
   } else {
     if (!cache_f32 && lgs::attn_tiles_fit(p, 1, 1, max_len)) {

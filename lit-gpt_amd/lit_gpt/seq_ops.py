@@ -60,6 +60,7 @@ SIGNATURES = {
     "lgs_embed_streams": [_P, _P, _I, _F, _P, _I, _I, _I, _I, _P],
     "lgs_streams_step": [_P, _P, _P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _P],
     "lgs_diffattn_prepare": [_P, _L, _I, _I, _I, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
+    "lgs_attn_one_heads": [_I, _I, _I, _I, _I],
     "lgs_diffattn": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _F,
                      _F, _P],
     "lgs_conv_silu": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
@@ -650,6 +651,14 @@ def diffattn_prepare(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, cac
                                                _dev(pos, "pos", I32), T, H, G, d, dv, rot_dims, S, _stream()))
 
 
+def _one_token_splits(maps: int, B: int, H: int, G: int, d: int, dv: int, span: int, cache: torch.Tensor) -> int:
+    """Workgroups that share one token's keys: enough to fill the chip, at least 64 (a head at a time: 128) keys each."""
+    heads = load_library().lgs_attn_one_heads(maps, H, G, d, dv) if cache.dtype == torch.bfloat16 else 0
+    if heads:
+        return max(2, min(64, 1024 * heads // max(1, B * H), (span + 63) // 64))
+    return max(1, min(64, 512 // max(1, B * H), (span + 127) // 128))
+
+
 def diffattn(proj: torch.Tensor, q_off: int, cache_k: torch.Tensor, cache_v: torch.Tensor, seq_start: torch.Tensor,
              seq_slot: torch.Tensor, seq_pos0: torch.Tensor, max_len: int, *, H: int, G: int, d: int, dv: int,
              chunk: int, scale: float, cap: float, lam: float, eps: float, post: float, bf16_copy: bool = False,
@@ -657,7 +666,7 @@ def diffattn(proj: torch.Tensor, q_off: int, cache_k: torch.Tensor, cache_v: tor
     """Differential attention of every row of a packed batch over its sequence's cached keys and values; the
     rotated queries are the 2 H d columns of ``proj`` at ``q_off``. Returns (T, H dv) fp32, or with ``bf16_copy``
     its rounding to bf16 (the out-projection's MFMA operand). ``splits``: workgroups per (token, head) when every
-    sequence brings one token (default: enough to fill the chip, at least 128 keys each)."""
+    sequence brings one token (default: ``_one_token_splits``)."""
     T, ld = proj.shape
     B = seq_slot.numel()
     slots, S = cache_k.shape[:2]
@@ -671,7 +680,7 @@ def diffattn(proj: torch.Tensor, q_off: int, cache_k: torch.Tensor, cache_v: tor
         splits = 1
     elif splits is None:
         span = min(S, chunk) if chunk > 0 else S
-        splits = max(1, min(64, 512 // max(1, B * H), (span + 127) // 128))
+        splits = _one_token_splits(2, B, H, G, d, dv, span, cache_k)
     part = torch.empty(T * H * splits * (4 + 2 * dv), dtype=F32, device=proj.device) if splits > 1 else None
     _check(load_library().lgs_diffattn(_dev(proj, "proj", F32) + 4 * q_off, ld, _dev(cache_k, "cache_k"),
                                        _dev(cache_v, "cache_v"), _wf32(cache_k, "cache_k"),
@@ -936,7 +945,10 @@ def sinkattn(proj: torch.Tensor, q_off: int, cache_k: torch.Tensor, cache_v: tor
         splits = 1
     elif splits is None:
         span = min(S, chunk) if chunk > 0 else (min(S, window) + prow if window > 0 else S)
-        splits = max(1, min(64, 512 // max(1, B * H), (span + 63) // 64 if window > 0 else (span + 127) // 128))
+        if window > 0 or score_bias is not None:
+            splits = max(1, min(64, 512 // max(1, B * H), (span + 63) // 64 if window > 0 else (span + 127) // 128))
+        else:
+            splits = _one_token_splits(1, B, H, G, d, dv, span, cache_k)
     part = torch.empty(T * H * splits * (2 + dv), dtype=F32, device=proj.device) if splits > 1 else None
     _check(load_library().lgs_sinkattn(_dev(proj, "proj", F32) + 4 * q_off, ld, _dev(cache_k, "cache_k"),
                                        _dev(cache_v, "cache_v"), _wf32(cache_k, "cache_k"), _opt(sink, "sink", F32),
