@@ -236,6 +236,10 @@ def _q4f_workspace(M, N, K, swiglu, device):
     need = int(load_library().lga_q4f_workspace_bytes(int(M), int(N), int(K), int(bool(swiglu))))
     if need == 0:
         return None, 0
+    if torch.cuda.is_current_stream_capturing():  # a graph's own memory, its counters cleared by every replay
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        ws[:4096].zero_()
+        return ws.data_ptr(), need  # (nothing is allocated before the launch that follows in stream order)
     key = device, _stream()
     ws = _Q4F_WS.get(key)
     if ws is None or ws.numel() < need:

@@ -83,3 +83,27 @@ def test_rule_falls_back(ops):
         h = x.float() @ wd.t()
         y = ops.q4_gemm_fused(x, w, sc, N, K, 64, 1).float()
         assert float(((y - h).abs() - h.abs() * 2 ** -7).max()) <= 2e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 512, 4160), (64, 4096, 4096)])
+def test_captured(ops, M, N, K):
+    """A split product in two graphs of one stream, the later one replayed first, with eager ones between: its workspace
+    is the graph's own (64-value K: the tiles whose counters have to be clear; 128: the partial sums of this form)."""
+    g = torch.Generator(device=DEV).manual_seed(K)
+    w, sc, wd = _weight(ops, N, K, 1, 64, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    want = ops.q4_gemm_fused(x, w, sc, N, K, 64, 1).clone()
+    stream, graphs, outs = torch.cuda.Stream(), [], []
+    stream.wait_stream(torch.cuda.current_stream())
+    for _ in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = ops.q4_gemm_fused(x, w, sc, N, K, 64, 1)
+        graphs.append(graph)
+        outs.append(out)
+    for i in (1, 0, 0, 1, 1):
+        graphs[i].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[i], want)
+        outs[i].zero_()
+        assert torch.equal(ops.q4_gemm_fused(x, w, sc, N, K, 64, 1), want)
