@@ -70,9 +70,9 @@ __device__ __forceinline__ float tanh_near(float x) {
   return y < 0.625f ? p : q;
 }
 
-// 1 / (1 + e^-z) from e^-|z|
+// 1 / (1 + e^-z) from e^-|z|, which is 0 from 120 on (an infinite z has no residual in exp_neg; a NaN stays one)
 __device__ __forceinline__ float sigmoid_near(float z) {
-  const float e = exp_neg(-fabsf(z)), d = 1.0f + e;
+  const float e = exp_neg(fabsf(z) > 120.0f ? -120.0f : -fabsf(z)), d = 1.0f + e;
   const float r = __builtin_amdgcn_rcpf(d), p = fmaf(fmaf(-d, r, 1.0f), r, r);
   return z >= 0.0f ? p : e * p;
 }

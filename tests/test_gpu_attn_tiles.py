@@ -165,6 +165,26 @@ def test_large_scores_and_infinite_queries():
     assert not torch.isfinite(plain[50]).all() or torch.isfinite(got[50]).all()
 
 
+def test_sigmoid_of_infinities():
+    """Heads that a score bias switches off or on (-inf: weights 0, inf: weights 1) and biases past every exponential."""
+    from lit_gpt import seq_ops
+
+    dev, T, H, d = torch.device("cuda", 0), 70, 6, 64
+    g = torch.Generator(device=dev).manual_seed(4)
+    start, slot, first = step([T], [0], dev)
+    k, v = caches(2, T, 1, d, d, dev, g, [(int(slot[0]), T)])
+    proj = torch.randn(T, H * d, generator=g, device=dev)
+    bias = torch.tensor([-math.inf, math.inf, -3.4e38, 3.4e38, -200.0, 0.0], device=dev)
+    kw = dict(H=H, G=1, d=d, dv=d, scale=0.125, score_bias=bias)
+    got = seq_ops.sinkattn(proj, 0, k, v, None, start, slot, first, T, **kw).view(T, H, d)
+    assert float(got[:, [0, 2, 4]].abs().max()) == 0.0
+    sums = v[slot[0].item(), :T, 0].double().cumsum(0)
+    for h in (1, 3):
+        assert rel(got[:, h], sums) < TOL
+    plain = seq_ops.sinkattn(proj, 0, k.float(), v.float(), None, start, slot, first, T, **kw).view(T, H, d)
+    assert torch.isfinite(got).all() and rel(got, plain.double()) < TOL
+
+
 @pytest.mark.parametrize("lengths", [[9], [16, 2, 40], [300, 64, 129], [1100]])
 @pytest.mark.parametrize("H,window,sink", [(1, 0, False), (3, 0, True), (4, 50, False)])
 def test_expanded_latent_attention(lengths, H, window, sink):
