@@ -77,6 +77,81 @@ __device__ __forceinline__ float sigmoid_near(float z) {
   return z >= 0.0f ? p : e * p;
 }
 
+// A row of a head whose result is not finite, once more in fp32 by one wave: an infinite operand has no summands (inf - inf)
+// and an infinite value or a NaN meets weights that are 0, also those of the keys that its query does not see. A lane scores
+// every 64th visible key, then owns DV / 64 columns. Left to itself: about 0.1 ms for 4096 keys; rows of finite operands never
+// come here.
+template <int DC, int DT, int MAPS, int PARTS, bool SIG>
+__device__ __forceinline__ void attn_row_plain(const AttnTileArgs& p, const uint16_t* kbase, const uint16_t* vbase,
+                                               const float* q, int h, int qlo, int qpos, int lane, float* out) {
+  constexpr int D = DC * 16, DV = DT * 32, C = DV / 64;
+  const AttnArgs& a = p.a;
+  float o[C], m = -INFINITY, l = 0.0f;
+#pragma unroll
+  for (int map = 0; map < MAPS; ++map) {
+    auto score = [&](int key) {
+      const uint16_t* k = kbase + (size_t)min(key, qpos) * p.krow + map * D;
+      float s = 0.0f;
+#pragma unroll 1
+      for (int e = 0; e < D; e += 4) {
+        const float4 q4 = *(const float4*)(q + map * D + e);
+        const uint2 hi = *(const uint2*)(k + e);
+        float x[4] = {bflo(hi.x), bfhi(hi.x), bflo(hi.y), bfhi(hi.y)};
+        if (PARTS == 2) {
+          const uint2 lo = *(const uint2*)(k + D + e);
+          x[0] += bflo(lo.x), x[1] += bfhi(lo.x), x[2] += bflo(lo.y), x[3] += bfhi(lo.y);
+        }
+        s = fmaf(q4.w, x[3], fmaf(q4.z, x[2], fmaf(q4.y, x[1], fmaf(q4.x, x[0], s))));
+      }
+      s *= a.scale;
+      return a.cap > 0.0f ? a.cap * tanhf(s / a.cap) : s;
+    };
+    m = -INFINITY, l = 0.0f;
+    if (!SIG) {
+      for (int k0 = qlo; k0 <= qpos; k0 += 64) {
+        const float s = score(k0 + lane);
+        m = fmaxf(m, k0 + lane <= qpos ? s : -INFINITY);
+      }
+      m = wave_max(m);
+    }
+    float acc[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] = 0.0f;
+    for (int k0 = qlo; k0 <= qpos; k0 += 64) {
+      const float s = score(k0 + lane);
+      float w = 0.0f;
+      if (k0 + lane <= qpos) w = SIG ? sigmoid_f(s + a.score_bias[h]) : (m == -INFINITY ? 0.0f : expf(s - m));
+      l += w;
+      for (int j = 0; j < min(64, qpos - k0 + 1); ++j) {
+        const float wj = __shfl(w, j);
+        const uint16_t* v = vbase + (size_t)(k0 + j) * p.vrow + lane;
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          acc[c] = fmaf(wj, PARTS == 2 ? bf2f(v[c * 64]) + bf2f(v[DV + c * 64]) : bf2f(v[c * 64]), acc[c]);
+      }
+    }
+    l = wave_sum(l);
+#pragma unroll
+    for (int c = 0; c < C; ++c) o[c] = MAPS == 1 ? acc[c] : (map == 0 ? acc[c] / l : o[c] - a.lambda * (acc[c] / l));
+  }
+  float f = a.post, den = 1.0f;
+  if (MAPS == 2) {
+    float ss = 0.0f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) ss = fmaf(o[c], o[c], ss);
+    den = sqrtf(wave_sum(ss) / (float)DV + a.eps);
+  } else if (!SIG) {
+    den = l;
+    if (a.sink) {
+      const float snk = a.sink[h], top = fmaxf(m, snk), w = m == -INFINITY ? 0.0f : expf(m - top);
+      den = l * w + expf(snk - top);
+      f *= w;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) out[lane + c * 64] = o[c] / den * f;
+}
+
 // DC: 16-wide pieces of one map's key, DT: 32-wide pieces of a value, MAPS: maps per head, PARTS: summands of keys and
 // values, SIG: sigmoid weights, ST: stages. grid (B * tiles, key heads * H / (G heads))
 template <int DC, int DT, int MAPS, int PARTS, bool SIG, int ST>
@@ -347,6 +422,12 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
       for (int r = 0; r < 16; ++r) o[t][r] *= f;
   }
   if (!store) return;
+  float bad = 0.0f;  // NaN where a result of this lane's query is not finite
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bad = fmaf(o[t][r], 0.0f, bad);
+  const unsigned long long odd = __ballot(live && bad != 0.0f);
   // ---- turned in LDS: a wave writes whole rows of a head
   const int slot = MAPS == 2 ? vh / 2 + p.heads * qw : vh + nv * qw;
   float* turn = ex + slot * 32 * (DV + 4);
@@ -357,6 +438,14 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
       *(float4*)(turn + lq * (DV + 4) + t * 32 + 8 * (r >> 2) + 4 * hh) =
           make_float4(o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (odd) {
+    for (uint32_t rows = (uint32_t)odd | (uint32_t)(odd >> 32); rows; rows &= rows - 1) {
+      const int i = __ffs(rows) - 1;
+      attn_row_plain<DC, DT, MAPS, PARTS, SIG>(p, kbase, vbase, a.q + (size_t)(rfirst + qw * 32 + i) * a.ld + (size_t)h * MAPS * DC * 16,
+                                               h, lowest(wfirst + i), min(wfirst + i, a.S - 1), lane, turn + i * (DV + 4));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
   constexpr int LANES = DV / 4;  // a lane holds four columns
   for (int i = lane / LANES; i < nlive; i += 64 / LANES) {
     const int c = lane % LANES * 4;
@@ -435,8 +524,9 @@ __global__ void __launch_bounds__(256) latent_split_kernel(const float* __restri
   const float* shared = kr + (size_t)rows[t] * dr;
   auto put = [](uint16_t* hi, uint16_t* lo, const float4 x) {
     const uint32_t a = pack2(x.x, x.y), b = pack2(x.z, x.w);
+    auto left = [](float v, float top) { return fabsf(top) == INFINITY ? 0.0f : v - top; };  // (an infinity is its own sum)
     *(uint2*)hi = make_uint2(a, b);
-    *(uint2*)lo = make_uint2(pack2(x.x - bflo(a), x.y - bfhi(a)), pack2(x.z - bflo(b), x.w - bfhi(b)));
+    *(uint2*)lo = make_uint2(pack2(left(x.x, bflo(a)), left(x.y, bfhi(a))), pack2(left(x.z, bflo(b)), left(x.w, bfhi(b))));
   };
   const int dk = d + dr, nk = dk / 4, nv = dv / 4;
   for (int i = threadIdx.x; i < H * nk; i += 256) {

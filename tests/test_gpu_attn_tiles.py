@@ -185,6 +185,106 @@ def test_sigmoid_of_infinities():
     assert torch.isfinite(got).all() and rel(got, plain.double()) < TOL
 
 
+def _softmax_row(q, k, v, scale, cap=0.0, bias=None):
+    """One query over its visible keys in float64; a key of weight 0 contributes nothing."""
+    s = (q.double() * k.double()).sum(-1) * scale
+    s = cap * torch.tanh(s / cap) if cap else s
+    if bias is not None:
+        w = torch.sigmoid(s + bias)
+    else:
+        w = torch.exp(s - s.max()) if not s.isnan().any() else s
+        w = w / w.sum()
+    return (w[:, None] * v.double()).sum(0)
+
+
+def _alike(got, want, tol=1e-5):
+    """The same elements infinite (with their signs) and NaN, and the finite ones as close as fp32 sums leave them."""
+    fine = torch.isfinite(want)
+    same = torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isposinf(), want.isposinf()) and \
+        torch.equal(got.isneginf(), want.isneginf())
+    return same and (not fine.any() or float((got - want)[fine].abs().max()) < tol * float(want[fine].abs().max().clamp(min=1.0)))
+
+
+@pytest.mark.parametrize("H,G,options", [(4, 1, dict(cap=5.0)), (3, 1, dict(sigmoid=True)), (4, 4, {}), (2, 1, dict(chunk=64)),
+                                         (2, 2, dict(window=40, cap=2.0))])
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128)])
+def test_infinities_and_nan(H, G, options, d, dv):
+    """Queries with an infinity, cached keys and values with infinities and a NaN: every query has what float64 gives it over
+    the keys that it sees, and the others nothing of it."""
+    from lit_gpt import seq_ops
+
+    dev, T = torch.device("cuda", 0), 150
+    g = torch.Generator(device=dev).manual_seed(d + H)
+    start, slot, first = step([T], [0], dev)
+    at = int(slot[0])
+    k, v = caches(2, T, G, d, dv, dev, g, [(at, T)])
+    proj = torch.randn(T, H * d, generator=g, device=dev)
+    proj[20, 3], proj[33, d - 1], proj[90, 5] = math.inf, -math.inf, math.nan
+    k[at, 70, :, 2], k[at, 100, :, 0] = math.inf, math.nan
+    v[at, 45, :, 1], v[at, 80, :, dv - 1] = math.inf, -math.inf
+    v[at, 120, :, 7] = math.nan
+    bias = torch.randn(H, generator=g, device=dev) if options.get("sigmoid") else None
+    chunk, window, cap = options.get("chunk", 0), options.get("window", 0), options.get("cap", 0.0)
+    got = seq_ops.sinkattn(proj, 0, k, v, None, start, slot, first, T, H=H, G=G, d=d, dv=dv, scale=d ** -0.5, chunk=chunk,
+                           window=window, cap=cap, score_bias=bias).view(T, H, dv)
+    see = visible(torch.arange(T, device=dev), T, chunk, window)
+    for t in range(T):
+        for h in range(H):
+            keys, vals = k[at, :T, h // (H // G)][see[t]], v[at, :T, h // (H // G)][see[t]]
+            want = _softmax_row(proj[t, h * d:(h + 1) * d], keys, vals, d ** -0.5, cap, None if bias is None else bias[h].double())
+            assert _alike(got[t, h].double(), want), (t, h)
+
+
+def test_two_maps_beside_a_nan():
+    """Rows before an infinite value or a NaN are those without it, rows that see it are not finite."""
+    from lit_gpt import seq_ops
+
+    dev, T, H, d, dv = torch.device("cuda", 0), 150, 4, 64, 128
+    g = torch.Generator(device=dev).manual_seed(5)
+    start, slot, first = step([T], [0], dev)
+    k, v = caches(2, T, 2, 2 * d, dv, dev, g, [(int(slot[0]), T)])
+    proj = torch.randn(T, 2 * H * d, generator=g, device=dev)
+    kw = dict(H=H, G=2, d=d, dv=dv, chunk=0, scale=0.125, cap=0.0, lam=0.4, eps=1e-5, post=0.5)
+    run = lambda v: seq_ops.diffattn(proj, 0, k, v, start, slot, first, T, **kw).view(T, H, dv)  # noqa: E731
+    clean = run(v)
+    for value in (math.inf, math.nan):
+        dirty = v.clone()
+        dirty[int(slot[0]), 77, 0, 9] = value
+        got = run(dirty)
+        assert torch.equal(got[:, 2:], clean[:, 2:])  # the other key head's
+        assert _alike(got[:77, :2].double(), clean[:77, :2].double())
+        assert got[77:, :2, 9].isnan().all()
+    proj[30, 2] = math.inf  # with a cap an infinite score is a large one
+    kw["cap"] = 5.0
+    got = run(v)[30, 0]
+    keys, vals = k[int(slot[0]), :31, 0], v[int(slot[0]), :31, 0]
+    o = _softmax_row(proj[30, :d], keys[:, :d], vals, 0.125, 5.0) - 0.4 * _softmax_row(proj[30, d:2 * d], keys[:, d:], vals, 0.125, 5.0)
+    assert _alike(got.double(), o / torch.sqrt((o * o).mean() + 1e-5) * 0.5)
+
+
+def test_expanded_infinities():
+    """An infinite and a NaN expanded value, a key past the largest bf16: the rows that do not see them are untouched."""
+    from lit_gpt import seq_ops
+
+    dev, T, H, d, dr, dv = torch.device("cuda", 0), 130, 2, 128, 64, 128
+    g = torch.Generator(device=dev).manual_seed(6)
+    start, slot, first = step([T], [0], dev)
+    q = torch.randn(T, H * (d + dr), generator=g, device=dev)
+    kv = torch.randn(T, H * (d + dv), generator=g, device=dev)
+    kr = torch.randn(2, T, dr, generator=g, device=dev)
+    rows = slot[0] * T + torch.arange(T, device=dev, dtype=torch.int32)
+    run = lambda kv: seq_ops.expanded_latent_attention(  # noqa: E731
+        q, 0, kv, kr, rows, None, start, slot, first, T, H=H, d=d, dr=dr, dv=dv, scale=192 ** -0.5).view(T, H, dv)
+    clean = run(kv)
+    dirty = kv.clone()
+    dirty[50, H * d + 3], dirty[60, H * d + 9], dirty[99, 4] = math.inf, math.nan, 3.4e38
+    got = run(dirty)
+    assert torch.equal(got[:, 1], clean[:, 1]) and _alike(got[:50, 0].double(), clean[:50, 0].double())
+    assert got[50:99, 0, 3].isposinf().all() and got[60:, 0, 9].isnan().all()
+    rest = [c for c in range(dv) if c not in (3, 9)]
+    assert _alike(got[50:99, 0, rest].double(), clean[50:99, 0, rest].double(), 2.0 ** -14)
+
+
 @pytest.mark.parametrize("lengths", [[9], [16, 2, 40], [300, 64, 129], [1100]])
 @pytest.mark.parametrize("H,window,sink", [(1, 0, False), (3, 0, True), (4, 50, False)])
 def test_expanded_latent_attention(lengths, H, window, sink):
