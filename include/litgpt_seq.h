@@ -120,7 +120,7 @@ int lgs_latent_attention_tiles(const float* qc, const float* proj, long ld, int 
  * form: lgs_split_attention_fits. */
 int lgs_latent_split(const float* kv, long ld, const float* cache_kr, const int* rows, void* k, void* v, int T, int H, int d,
                      int dr, int dv, lgs_stream_t stream);
-int lgs_split_attention_fits(int dk, int dv);
+int lgs_split_attention_fits(int H, int dk, int dv);
 int lgs_split_attention(const float* q, long ld, const void* k, const void* v, const float* sink, const int* seq_start,
                         const int* seq_slot, const int* seq_pos0, float* out, void* out_bf16, int B, int max_len, int H,
                         int dk, int dv, float scale, int window, lgs_stream_t stream);

@@ -28,11 +28,20 @@ typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef short i16x8_t __attribute__((ext_vector_type(8)));
 
 constexpr int kTileKeys = 64;
+constexpr long kMostRow = 1 << 23;  // elements of a position's keys or values: a tile of them is one buffer (31 bits of bytes)
 
 // 16-byte chunk `ch` of row `row` in an LDS tile of `chunks` a row: permuted so that neither 32 rows' same chunk nor the
 // transposed reads meet in a bank
 __device__ __forceinline__ int chunk_swizzle(int row, int chunks) {
   return chunks == 8 ? (((row & 3) << 1) | ((row >> 2) & 1)) : (((row & 3) << 2) | ((row >> 2) & 3));
+}
+
+// 16 bytes a lane of a buffer into LDS, zeros past its end
+__device__ __forceinline__ void tile_dma16(const void* base, int bytes, int off, unsigned char* lds) {
+#ifdef __HIP_DEVICE_COMPILE__  // (device builtins: the host pass only type-checks the body)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, bytes, 0x00020000),
+                                           (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
+#endif
 }
 
 // the next summands of eight fp32 values as one operand: the upper half of every value, which is taken off it
@@ -192,14 +201,10 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
   const int wfirst = pos_first + qw * 32, wlast = nlive > 0 ? wfirst + nlive - 1 : -1;
   const int wlo = lowest(wfirst), whi_lo = nlive > 0 ? lowest(wlast) : 0;
 
-  // key and value rows: a buffer that ends after the last visible key
+  // key and value rows: a buffer per tile that ends after the last visible key (a sequence's rows may exceed one buffer)
   const size_t row0 = p.packed ? (size_t)a.seq_start[b] : (size_t)a.seq_slot[b] * a.S;
   const uint16_t* kbase = p.k + row0 * p.krow + (size_t)g * (MAPS * PARTS * DC * 16);
   const uint16_t* vbase = p.v + row0 * p.vrow + (size_t)g * (PARTS * DV);
-  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)kbase, (short)0, (int)((long)pos_last * p.krow * 2 + CHK * 16), 0x00020000);
-  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)vbase, (short)0, (int)((long)pos_last * p.vrow * 2 + CHV * 16), 0x00020000);
   int voff[PU];
 #pragma unroll
   for (int i = 0; i < PU; ++i) {
@@ -210,14 +215,15 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
     voff[i] = (int)((isv ? p.vrow : p.krow) * 2) * r + ch * 16;
   }
   auto stage = [&](int kt, int buf) {
+    const int left = min(pos_last - kt * kTileKeys, kTileKeys - 1);  // the tile's last visible row
+    const uint16_t* kat = kbase + (long)kt * kTileKeys * p.krow;
+    const uint16_t* vat = vbase + (long)kt * kTileKeys * p.vrow;
+    const int kbytes = left < 0 ? 0 : left * (int)p.krow * 2 + CHK * 16, vbytes = left < 0 ? 0 : left * (int)p.vrow * 2 + CHV * 16;
 #pragma unroll
     for (int i = 0; i < PU; ++i) {
       const int u = wave * PU + i;
       const bool isv = u >= CHK;
-      const int off = voff[i] + kt * kTileKeys * (int)((isv ? p.vrow : p.krow) * 2);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(isv ? vrs : krs,
-                                               (__attribute__((address_space(3))) void*)(lds + buf * STAGE + u * 1024), 16,
-                                               off, 0, 0, 0);
+      tile_dma16(isv ? vat : kat, isv ? vbytes : kbytes, voff[i], lds + buf * STAGE + u * 1024);
     }
   };
 
@@ -477,13 +483,14 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
   }
 }
 
-// The sizes that have a form, and queries and results in 16-byte pieces; any step with more than one token of a sequence:
-// 9 tokens after 1500 of 16 heads on 4 key heads of 128 take 75 us here and 158 with a thread per key (seq_attn.hip), 9 of
+// The sizes that have a form, and queries and results in 16-byte pieces, however many rows a cache holds; any step with more
+// than one token of a sequence: 9 tokens after 1500 of 16 heads on 4 key heads of 128 take 75 us here and 158 with a thread per key (seq_attn.hip), 9 of
 // a new sequence 15 and 24, 2048 of one 110 and 634 (51 GFLOP of bf16 products, 17 of fp32 ones).
 bool attn_tiles_fit(const AttnArgs& a, int maps, int parts, int max_len) {
   const bool sized = parts == 2 ? (maps == 1 && a.d == 192 && a.dv == 128)
                                 : ((a.dv == 64 || a.dv == 128) && (a.d == 64 || (a.d == 128 && maps == 1)));
-  return sized && max_len > 1 && a.pool == 0 && a.ld % 4 == 0 && (uintptr_t)a.q % 16 == 0 &&
+  const long row = (long)(parts == 2 ? 2 * a.H : a.G) * (maps * a.d > a.dv ? maps * a.d : a.dv);
+  return sized && row <= kMostRow && max_len > 1 && a.pool == 0 && a.ld % 4 == 0 && (uintptr_t)a.q % 16 == 0 &&
          (uintptr_t)a.out % 16 == 0 && (uintptr_t)a.out16 % 8 == 0;
 }
 
@@ -503,10 +510,8 @@ int attn_tiles_launch(const AttnTileArgs& given, int maps, int parts, int B, int
   p.heads = share % 4 == 0 ? 4 : (share % 2 == 0 ? 2 : 1);
   const int nv = p.heads * maps, qw = nv == 8 ? 1 : 4 / nv;
   a.tiles = (max_len + 32 * qw - 1) / (32 * qw);
-  const long rows = p.packed ? max_len : a.S;
-  LGA_CHECK_ARG((rows + 2L * kTileKeys) * p.krow < (1L << 30) && (rows + 2L * kTileKeys) * p.vrow < (1L << 30) &&
-                    (long)B * a.tiles * (a.H / p.heads) < (1L << 31),
-                "attention: a sequence's keys or values exceed a buffer");
+  LGA_CHECK_ARG(p.krow <= kMostRow && p.vrow <= kMostRow, "attention: a position's keys or values exceed a buffer");
+  LGA_CHECK_ARG((long)B * a.tiles * (a.H / p.heads) < (1L << 31), "attention: too many tiles");
   const dim3 grid((unsigned)(B * a.tiles * (a.H / p.heads)));
   if (parts == 2) return attn_tiles_go<12, 4, 1, 2, 2>(p, grid, stream);
   if (maps == 2) return a.dv == 64 ? attn_tiles_go<4, 2, 2, 1, 3>(p, grid, stream) : attn_tiles_go<4, 4, 2, 1, 3>(p, grid, stream);
@@ -555,8 +560,9 @@ extern "C" int lgs_latent_split(const float* kv, long ld, const float* cache_kr,
   LGA_LAUNCH_RETURN();
 }
 
-extern "C" int lgs_split_attention_fits(int dk, int dv) {
+extern "C" int lgs_split_attention_fits(int H, int dk, int dv) {
   lgs::AttnArgs a{};
+  a.H = a.G = H;
   a.d = dk;
   a.dv = dv;
   return lgs::attn_tiles_fit(a, 1, 2, 2) ? 1 : 0;

@@ -265,7 +265,7 @@ class LatentAttention(InputReader):
 
     def _expands(self, step: StepBatch, ldq: int, q_off: int) -> bool:
         return step.fresh and (step.max_len or step.T) > 1 and step.T >= 8 * step.B and self.r % 64 == 0 and ldq % 4 == 0 and \
-            q_off % 4 == 0 and seq_ops.split_attention_fits(self.d + self.dr, self.dv)
+            q_off % 4 == 0 and seq_ops.split_attention_fits(self.H, self.d + self.dr, self.dv)
 
     def _finish(self, att: torch.Tensor, proj: torch.Tensor, x: torch.Tensor, accumulate: bool, b16: bool) -> None:
         H, dv, W, T = self.H, self.dv, x.shape[1], x.shape[0]

@@ -44,7 +44,7 @@ SIGNATURES = {
     "lgs_latent_attention": [_P, _P, _L, _I, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _I, _P],
     "lgs_latent_attention_tiles": [_P, _P, _L, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "lgs_latent_split": [_P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
-    "lgs_split_attention_fits": [_I, _I],
+    "lgs_split_attention_fits": [_I, _I, _I],
     "lgs_split_attention": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P],
     "lgs_glu": [_P, _P, _L, _P, _I, _I, _I, _I, _P],
     "lgs_moe_route": [_P, _L, _I, _I, _I, _P, _P, _P],
@@ -363,8 +363,8 @@ def latent_attention_tiles(qc: torch.Tensor, proj: torch.Tensor, q_off: int, cac
     return out
 
 
-def split_attention_fits(dk: int, dv: int) -> bool:
-    return bool(load_library().lgs_split_attention_fits(dk, dv))
+def split_attention_fits(H: int, dk: int, dv: int) -> bool:
+    return bool(load_library().lgs_split_attention_fits(H, dk, dv))
 
 
 def expanded_latent_attention(q: torch.Tensor, q_off: int, kv: torch.Tensor, cache_kr: torch.Tensor, rows: torch.Tensor,

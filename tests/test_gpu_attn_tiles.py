@@ -317,3 +317,64 @@ def test_expanded_latent_attention(lengths, H, window, sink):
     # scores of size 1 from 192 products of relative error 2^-17 each, uncorrelated; values likewise
     assert rel(got, want.flatten(1)) < 2.0 ** -16
     assert torch.equal(seq_ops.expanded_latent_attention(*args, bf16=True, **kw), got.bfloat16())
+
+
+# (rows of 4096 elements: 2^30 of them and 2^31 bytes lie at row 262,144; what no sequence has written stays as it is)
+FAR = 262_400
+
+
+@pytest.mark.parametrize("n,pos0,chunk,window", [(2, 0, 0, 0), (100, 262_110, 64, 0), (70, 262_100, 0, 90), (17, 262_383, 100, 0)])
+@pytest.mark.parametrize("maps", [1, 2])
+def test_caches_past_one_buffer(n, pos0, chunk, window, maps):
+    from lit_gpt import seq_ops
+
+    if window and maps == 2:
+        pytest.skip("two maps have no window")
+    dev, H, G, d = torch.device("cuda", 0), 64 // maps, 64 // maps, 64
+    dv = 64 * maps
+    g = torch.Generator(device=dev).manual_seed(n)
+    k = torch.empty(1, FAR, G, maps * d, dtype=torch.bfloat16, device=dev)
+    v = torch.empty(1, FAR, G, dv, dtype=torch.bfloat16, device=dev)
+    lo = max(0, pos0 - 200)
+    for t in (k, v):
+        t[:, :FAR - 200] = math.nan
+        t[:, lo:pos0 + n] = torch.randn(1, pos0 + n - lo, *t.shape[2:], generator=g, device=dev).bfloat16()
+    proj = torch.randn(n, H * maps * d, generator=g, device=dev)
+    start, slot, first = (torch.tensor(x, dtype=torch.int32, device=dev) for x in ([0, n], [0], [pos0]))
+    kw = dict(H=H, G=G, d=d, dv=dv, scale=0.125, chunk=chunk)
+    if maps == 1:
+        got = seq_ops.sinkattn(proj, 0, k, v, None, start, slot, first, n, window=window, **kw)
+    else:
+        got = seq_ops.diffattn(proj, 0, k, v, start, slot, first, n, cap=0.0, lam=0.4, eps=1e-5, post=0.5, **kw)
+    kd, vd = k[0, lo:pos0 + n].double().transpose(0, 1), v[0, lo:pos0 + n].double().transpose(0, 1)
+    see = visible(torch.arange(pos0, pos0 + n, device=dev), pos0 + n, chunk, window)[:, lo:]
+    q, out = proj.double().view(n, H, maps, d), []
+    for i in range(maps):
+        s = torch.matmul(q[:, :, i].transpose(0, 1), kd[..., i * d:(i + 1) * d].transpose(1, 2).contiguous()) * 0.125
+        out.append(torch.matmul(torch.softmax(s.masked_fill(~see, -math.inf), -1), vd).transpose(0, 1))
+    want = out[0]
+    if maps == 2:
+        o = out[0] - 0.4 * out[1]
+        want = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * 0.5
+    assert rel(got, want.flatten(1)) < TOL
+
+
+def test_expanded_rows_past_one_buffer():
+    """128 heads: the summands of 21,846 tokens' keys are 2^30 elements."""
+    from lit_gpt import seq_ops
+
+    dev, T, H, d, dr, dv, window = torch.device("cuda", 0), 22_100, 128, 128, 64, 128, 33
+    g = torch.Generator(device=dev).manual_seed(7)
+    start, slot, first = (torch.tensor(x, dtype=torch.int32, device=dev) for x in ([0, T], [0], [0]))
+    q = torch.randn(T, H * (d + dr), generator=g, device=dev)
+    kv = torch.randn(T, H * (d + dv), generator=g, device=dev)
+    kr = torch.randn(1, T, dr, generator=g, device=dev)
+    got = seq_ops.expanded_latent_attention(q, 0, kv, kr, torch.arange(T, device=dev, dtype=torch.int32), None, start, slot, first,
+                                            T, H=H, d=d, dr=dr, dv=dv, scale=192 ** -0.5, window=window).view(T, H, dv)
+    assert torch.isfinite(got).all()
+    for t in (40, 21_800, 21_845, 21_846, 21_900, T - 1):
+        seen = slice(t - window + 1, t + 1)
+        for h in (0, 77, 127):
+            k = torch.cat([kv[seen, h * d:(h + 1) * d], kr[0, seen]], -1).double()
+            w = torch.softmax(k @ q[t, h * 192:(h + 1) * 192].double() * 192 ** -0.5, -1)
+            assert rel(got[t, h], w @ kv[seen, H * d + h * dv:H * d + (h + 1) * dv].double()) < 2.0 ** -14
