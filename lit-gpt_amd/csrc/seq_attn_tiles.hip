@@ -483,15 +483,16 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
   }
 }
 
-// The sizes that have a form, and queries and results in 16-byte pieces, however many rows a cache holds; any step with more
-// than one token of a sequence: 9 tokens after 1500 of 16 heads on 4 key heads of 128 take 75 us here and 158 with a thread per key (seq_attn.hip), 9 of
-// a new sequence 15 and 24, 2048 of one 110 and 634 (51 GFLOP of bf16 products, 17 of fp32 ones).
+// The sizes that have a form, where queries, keys, values and results start on the bytes that it moves at a time, however many
+// rows a cache holds; any step with more than one token of a sequence: 9 tokens after 1500 of 16 heads on 4 key heads of 128
+// take 75 us here and 158 with a thread per key (seq_attn.hip), 9 of a new sequence 15 and 24, 2048 of one 110 and 634 (51
+// GFLOP of bf16 products, 17 of fp32 ones).
 bool attn_tiles_fit(const AttnArgs& a, int maps, int parts, int max_len) {
   const bool sized = parts == 2 ? (maps == 1 && a.d == 192 && a.dv == 128)
                                 : ((a.dv == 64 || a.dv == 128) && (a.d == 64 || (a.d == 128 && maps == 1)));
   const long row = (long)(parts == 2 ? 2 * a.H : a.G) * (maps * a.d > a.dv ? maps * a.d : a.dv);
   return sized && row <= kMostRow && max_len > 1 && a.pool == 0 && a.ld % 4 == 0 && (uintptr_t)a.q % 16 == 0 &&
-         (uintptr_t)a.out % 16 == 0 && (uintptr_t)a.out16 % 8 == 0;
+         ((uintptr_t)a.cache_k | (uintptr_t)a.cache_v | (uintptr_t)a.out) % 16 == 0 && (uintptr_t)a.out16 % 8 == 0;
 }
 
 template <int DC, int DT, int MAPS, int PARTS, int ST>

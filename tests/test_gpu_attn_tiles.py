@@ -145,6 +145,28 @@ def test_two_maps(lengths, pos0, dv, H, G, chunk, cap):
     assert rel(got, want) < TOL and rel(got, want) < 1.5 * rel(plain, want) + 1e-7
 
 
+def test_caches_off_sixteen_bytes():
+    """Caches that start on 8 bytes take the form whose loads are that wide."""
+    from lit_gpt import seq_ops
+
+    dev, T, H, d = torch.device("cuda", 0), 90, 2, 64
+    g = torch.Generator(device=dev).manual_seed(8)
+    start, slot, first = step([T], [0], dev)
+    k, v = caches(2, T, 1, d, d, dev, g, [(int(slot[0]), T)])
+    proj = torch.randn(T, 2 * H * d, generator=g, device=dev)
+
+    def off(t):
+        return torch.empty(t.numel() + 4, dtype=t.dtype, device=dev)[4:].view(t.shape).copy_(t)
+
+    kw = dict(H=H, G=1, d=d, dv=d, scale=0.125)
+    want = seq_ops.sinkattn(proj, 0, k.float(), v.float(), None, start, slot, first, T, **kw)
+    for pair in ((off(k), v), (k, off(v)), (off(k), off(v))):
+        assert torch.equal(seq_ops.sinkattn(proj, 0, *pair, None, start, slot, first, T, **kw), want)
+    two, kw = torch.cat([k, k], -1), dict(kw, chunk=0, cap=0.0, lam=0.4, eps=1e-5, post=0.5)
+    want = seq_ops.diffattn(proj, 0, two.float(), v.float(), start, slot, first, T, **kw)
+    assert torch.equal(seq_ops.diffattn(proj, 0, off(two), off(v), start, slot, first, T, **kw), want)
+
+
 def test_large_scores_and_infinite_queries():
     """A key that outweighs all others, scores far below it, and a query whose scores overflow: as the other form has it."""
     from lit_gpt import seq_ops
