@@ -576,6 +576,10 @@ __global__ void __launch_bounds__(256) attn_one_kernel(AttnArgs p) {
       k4[i] = *(const uint4*)(kc + at);
       v4[i] = *(const uint4*)(vc + at);
     }
+    if (u0 + 16 * (U - 1) >= to)  // past the share: a weight of 0 does not meet the last key's value
+#pragma unroll
+      for (int i = 0; i < U; ++i)
+        if (u0 + 16 * i >= to) v4[i] = make_uint4(0, 0, 0, 0);
     float w[HG][U];
 #pragma unroll
     for (int i = 0; i < U; ++i) {
@@ -600,7 +604,7 @@ __global__ void __launch_bounds__(256) attn_one_kernel(AttnArgs p) {
       float sum = 0.0f;
 #pragma unroll
       for (int i = 0; i < U; ++i) {
-        w[h][i] = mn == -INFINITY ? 0.0f : expf(w[h][i] - mn);
+        w[h][i] = w[h][i] == -INFINITY ? 0.0f : expf(w[h][i] - (mn == -INFINITY ? 0.0f : mn));  // (a NaN stays one)
         sum += w[h][i];
       }
       l[h] = l[h] * a + sum;

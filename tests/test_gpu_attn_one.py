@@ -60,3 +60,44 @@ def test_two_maps(H, G, chunk, cap):
     want = run(1)
     for n in (2, 5, 64, None):  # (the outputs are divided by their root mean square: relative to it)
         assert float((run(n) - want).abs().max()) < 2 ** -15 * float(want.abs().max()), n
+
+
+@pytest.mark.parametrize("cap", [0.0, 5.0])
+def test_nan_and_infinity(cap):
+    """A NaN in a key that no other key of its group and share stands beside makes the result NaN; an infinite value of the
+    last key, beside which a group has no more, is infinite in its column and nowhere else."""
+    from lit_gpt import seq_ops
+
+    H, G = 4, 2
+    k, v, q, slots, step, g = _step(H, G, 128, 128, 600, 11)
+    kw = dict(H=H, G=G, d=128, dv=128, scale=128 ** -0.5, cap=cap)
+    run = lambda n: seq_ops.sinkattn(q, 0, k, v, None, step.seq_start, step.seq_slot, step.seq_pos0, 1, splits=n, **kw).view(-1, H, 128)  # noqa: E731
+    clean = run(1)
+    at = {b: p for b, p in enumerate(POS) if p >= 16}
+    for b, p in at.items():
+        v[slots[b], p, :, 5] = float("inf")
+    for n in (2, 7, 64, None):
+        got = run(n)
+        rest = [c for c in range(128) if c != 5]
+        for b in at:
+            assert got[b, :, 5].isposinf().all(), (n, b)
+        assert float((got - clean)[:, :, rest].abs().max()) < 2 ** -16
+    for b, p in at.items():
+        k[slots[b], p, 0, 9] = float("nan")
+    for n in (2, 7, 64, None):
+        got = run(n)
+        for b in at:
+            assert got[b, :2].isnan().all() and torch.isfinite(got[b, 2:, 6:]).all(), (n, b)
+
+
+def test_two_maps_nan():
+    from lit_gpt import seq_ops
+
+    H, G = 4, 2
+    k, v, q, slots, step, g = _step(H, G, 128, 128, 600, 12)
+    kw = dict(H=H, G=G, d=64, dv=128, scale=0.125, chunk=0, cap=0.0, lam=0.4, eps=1e-5, post=0.6)
+    for b, p in enumerate(POS):
+        k[slots[b], p, 0, 70] = float("nan")  # of the second map
+    for n in (2, 64, None):
+        got = seq_ops.diffattn(q, 0, k, v, step.seq_start, step.seq_slot, step.seq_pos0, 1, splits=n, **kw).view(-1, H, 128)
+        assert got[:, :2].isnan().all() and torch.isfinite(got[:, 2:]).all(), n
