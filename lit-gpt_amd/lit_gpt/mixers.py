@@ -235,7 +235,7 @@ class LatentAttention(InputReader):
                                step.pos, H=H, d=d, dr=dr, r=r, rot_dims=self.rot_dims, eps=self.eps,
                                rot_mult=self.rot_mult)
         b16 = _tiles16(T, self.w_o)
-        if b16 and self._expands(step, ldq, q_off):
+        if b16 and self._expands(step, cache, ldq, q_off):
             # a prompt from its start: every row's key and value are expanded once, 2 (d + dr + dv) operations per pair
             # and head instead of 2 (2 r + dr), and the query is not rounded on its way into the latent space
             n = H * (d + dv)
@@ -263,9 +263,11 @@ class LatentAttention(InputReader):
                        stride_w=dv * r, stride_y=dv)
         self._finish(att, proj, x, accumulate, b16)
 
-    def _expands(self, step: StepBatch, ldq: int, q_off: int) -> bool:
-        return step.fresh and (step.max_len or step.T) > 1 and step.T >= 8 * step.B and self.r % 64 == 0 and ldq % 4 == 0 and \
-            q_off % 4 == 0 and seq_ops.split_attention_fits(self.H, self.d + self.dr, self.dv)
+    def _expands(self, step: StepBatch, cache: LatentKVCache, ldq: int, q_off: int) -> bool:
+        # (latents that a caller keeps in fp32 are not rounded on their way through the bf16 product that expands them)
+        return step.fresh and (step.max_len or step.T) > 1 and step.T >= 8 * step.B and cache.c.dtype == torch.bfloat16 and \
+            self.r % 64 == 0 and ldq % 4 == 0 and q_off % 4 == 0 and \
+            seq_ops.split_attention_fits(self.H, self.d + self.dr, self.dv)
 
     def _finish(self, att: torch.Tensor, proj: torch.Tensor, x: torch.Tensor, accumulate: bool, b16: bool) -> None:
         H, dv, W, T = self.H, self.dv, x.shape[1], x.shape[0]

@@ -1,0 +1,48 @@
+"""Fresh prompts of latent attention over expanded keys and values against the form in the latent space, both on the same
+queries and caches, and against float64 over the same bf16 latents and weights."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+H, DK, DR, DV, R, W = 3, 128, 64, 128, 192, 64
+
+
+def model(seed=0, edit=None):
+    from lit_gpt.config import LayeredConfig
+    from lit_gpt.layered import LayeredGPT
+
+    cfg = {"architecture": "Fazolorn", "vocab": 50, "width": W, "norm": {"eps": 1e-5}, "layers": [
+        {"type": "latent_attention", "mixer": {"heads": H, "dim": DK, "rot_dim": DR, "vdim": DV, "kv_rank": R, "q_rank": 96,
+                                               "rot": {"dims": DR, "base": 100.0}, "scale": 192 ** -0.5}}]}
+    config = LayeredConfig.from_dict(cfg)
+    weights = LayeredGPT.random_weights(config, seed=seed)
+    if edit:
+        edit(weights)
+    return LayeredGPT(config, weights, device=torch.device("cuda", 0), dtype=torch.bfloat16)
+
+
+def heads(mix, step, cache, proj):
+    """The heads' outputs in fp32, ahead of the out-projection."""
+    kept = []
+    mix.out_gate, mix._finish = True, lambda att, *_: kept.append(att)  # (with a gate to come they are not rounded)
+    mix.forward(proj, step, cache, torch.empty(step.T, W, device=proj.device))
+    del mix._finish
+    mix.out_gate = False
+    return kept[0]
+
+
+def prompt(lengths, fresh=True, slots=(1, 0, 2)):
+    from lit_gpt.mixers import StepBatch
+
+    step = StepBatch.build([(s, 0, [1] * n) for s, n in zip(slots, lengths)], torch.device("cuda", 0))
+    step.fresh = fresh
+    return step
+
+
+def test_fp32_latents_take_the_latent_form():
+    mix = model().blocks[0].mixer
+    dev, T = torch.device("cuda", 0), 70
+    proj = torch.randn(T, 96 + R + DR, generator=torch.Generator(device=dev).manual_seed(1), device=dev)
+    out = [heads(mix, prompt([T], fresh), mix.build_cache(3, 80, dev, torch.float32), proj.clone()) for fresh in (True, False)]
+    assert torch.equal(*out)
