@@ -45,7 +45,9 @@ class StepBatch:
     T: int
     B: int
     max_len: int = 0  # the most tokens any sequence brings to this step (host side; 0: unknown, taken as T)
-    fresh: bool = False  # every sequence starts at position 0 in this step (host side; False: it may not)
+    # every sequence starts at position 0 in this step (host side, of the positions as they were when the table was made;
+    # False: it may not). Not looked at while a step is captured
+    fresh: bool = False
 
     @classmethod
     def build(cls, entries: Sequence[Tuple[int, int, Sequence[int]]], device: torch.device) -> "StepBatch":
@@ -264,9 +266,10 @@ class LatentAttention(InputReader):
         self._finish(att, proj, x, accumulate, b16)
 
     def _expands(self, step: StepBatch, cache: LatentKVCache, ldq: int, q_off: int) -> bool:
-        # (latents that a caller keeps in fp32 are not rounded on their way through the bf16 product that expands them)
-        return step.fresh and (step.max_len or step.T) > 1 and step.T >= 8 * step.B and cache.c.dtype == torch.bfloat16 and \
-            self.r % 64 == 0 and ldq % 4 == 0 and q_off % 4 == 0 and \
+        # (latents that a caller keeps in fp32 are not rounded on their way through the bf16 product that expands them; a
+        # captured step reads its positions from the device at every replay, where `fresh` need not hold any more)
+        return step.fresh and not torch.cuda.is_current_stream_capturing() and (step.max_len or step.T) > 1 and \
+            step.T >= 8 * step.B and cache.c.dtype == torch.bfloat16 and self.r % 64 == 0 and ldq % 4 == 0 and q_off % 4 == 0 and \
             seq_ops.split_attention_fits(self.H, self.d + self.dr, self.dv)
 
     def _finish(self, att: torch.Tensor, proj: torch.Tensor, x: torch.Tensor, accumulate: bool, b16: bool) -> None:

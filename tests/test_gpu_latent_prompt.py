@@ -46,3 +46,35 @@ def test_fp32_latents_take_the_latent_form():
     proj = torch.randn(T, 96 + R + DR, generator=torch.Generator(device=dev).manual_seed(1), device=dev)
     out = [heads(mix, prompt([T], fresh), mix.build_cache(3, 80, dev, torch.float32), proj.clone()) for fresh in (True, False)]
     assert torch.equal(*out)
+
+
+def test_captured_prompt_at_later_positions():
+    """A step captured from a prompt's start and replayed further on, its positions moved on the device in between."""
+    m = model(2)
+    dev, T = torch.device("cuda", 0), 24
+    m.set_kv_cache(2, 128)
+    g = torch.Generator().manual_seed(1)
+    ids = torch.randint(0, 50, (4, T), generator=g)
+
+    def table(i, fresh):
+        from lit_gpt.mixers import StepBatch
+
+        step = StepBatch.build([(1, i * T, ids[i].tolist())], dev)
+        step.fresh = fresh
+        return step
+
+    with torch.inference_mode():
+        want = [m.logits(m.forward_step(table(i, False))).clone() for i in range(4)]
+        step = table(0, True)
+        m.logits(m.forward_step(step))
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = m.logits(m.forward_step(step))
+        for i in (0, 1, 2, 3, 0, 1):
+            step.tokens.copy_(ids[i])
+            step.pos.copy_(torch.arange(i * T, (i + 1) * T))
+            step.seq_pos0.fill_(i * T)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want[i]), i

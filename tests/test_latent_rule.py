@@ -1,6 +1,12 @@
 """Which latent prompts are made over expanded keys and values (the others: in the latent space), on the host."""
 
+import pytest
 import torch
+
+
+@pytest.fixture(autouse=True)
+def eager(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)  # (asks the GPU)
 
 
 def module(kv_rank=128, vdim=128):
@@ -38,3 +44,9 @@ def test_fresh_prompts_of_the_served_sizes():
 def test_latents_kept_in_fp32_are_not_rounded():
     mix = module()
     assert not takes(mix, prompt(), torch.float32)
+
+
+def test_captured_steps_are_not_bound_to_their_start(monkeypatch):
+    mix = module()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert not takes(mix, prompt())
