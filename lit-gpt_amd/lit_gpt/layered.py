@@ -46,6 +46,7 @@ from lit_gpt.config import SOFTMAX_KINDS, LayeredConfig, LayerSpec
 from lit_gpt.mixers import (MIXERS, DenseFeedForward, GatedFeedForward, SparseFeedForward, StepBatch, StreamLinks,
                             TokenSide)
 from lit_gpt.rmsnorm import StreamRMSNorm
+from lit_gpt.utils import hooked
 
 
 def _sub(w: Dict[str, torch.Tensor], prefix: str) -> Dict[str, torch.Tensor]:
@@ -137,7 +138,7 @@ class Sublayer(nn.Module):
         """h (T, width): the normed read of the streams. Returns the sublayer's output (T, width) fp32."""
         n_in, W = self.w_in.shape
         y = torch.empty(step.T, W, dtype=torch.float32, device=h.device)
-        if cache is None and self.b_in is None and self.module.forward_in(h16, self.w_in, y):
+        if cache is None and self.b_in is None and not hooked(self.module) and self.module.forward_in(h16, self.w_in, y):
             return y
         proj = torch.empty(step.T, n_in, dtype=torch.float32, device=h.device)
         seq_ops.linear(h if h16 is None else h16, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in,
@@ -271,7 +272,8 @@ class SandwichSublayer(nn.Module):
             self.module.forward_fused(h, self.w_in, self.b_in, step, cache, y, accumulate=False)
             return [(y, None)], 1.0
         y = torch.empty(T, W, dtype=torch.float32, device=src.device)
-        if cache is None and self.w_in is not None and self.b_in is None and self.module.forward_in(h16, self.w_in, y):
+        if cache is None and self.w_in is not None and self.b_in is None and not hooked(self.module) and \
+                self.module.forward_in(h16, self.w_in, y):
             return [(y, None)], 1.0
         proj = None
         if self.w_in is not None and self.module.wants_proj(T):

@@ -31,6 +31,7 @@ import torch.nn as nn
 from lit_gpt import ops
 from lit_gpt.config import Config
 from lit_gpt.rmsnorm import RMSNorm
+from lit_gpt.utils import hooked
 
 
 
@@ -279,7 +280,7 @@ class Block(nn.Module):
         if not (x.is_cuda and x.dtype == torch.float32 and type(m) is GptNeoxMLP and type(self.norm_1) is LayerNorm and
                 type(self.norm_2) is LayerNorm and type(m.fc) is nn.Linear and type(m.proj) is nn.Linear):
             return False
-        if any(mod._forward_hooks or mod._forward_pre_hooks for mod in (m, m.fc, m.proj, self.norm_1, self.norm_2)):
+        if hooked(m, m.fc, m.proj, self.norm_1, self.norm_2):
             return False
         ts = (self.norm_1.weight, self.norm_1.bias, self.norm_2.weight, self.norm_2.bias, m.fc.weight, m.fc.bias,
               m.proj.weight, m.proj.bias)

@@ -14,6 +14,14 @@ def find_multiple(n: int, k: int) -> int:
     return n + k - (n % k)
 
 
+def hooked(*modules) -> bool:
+    """Whether calling one of these torch modules runs a forward hook: a form that computes past the call would skip it."""
+    from torch.nn.modules import module as everywhere
+
+    return bool(everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks) or \
+        any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+
+
 def check_valid_checkpoint_dir(checkpoint_dir: Path) -> None:
     """Same required files as the reference (lit_gpt/utils.py:93-124); exits with status 1 otherwise."""
     checkpoint_dir = Path(checkpoint_dir)
