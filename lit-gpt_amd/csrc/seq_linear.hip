@@ -658,9 +658,7 @@ extern "C" int lgs_linear_glu(const void* a, long lda, const void* w, long strid
 
 // ranges of K that a plain product of a bf16 A on bf16 weights is best made in (1: as one)
 extern "C" int lgs_linear_ksplit(int M, int N, int K) {
-  // (a few columns are a router's logits: their sums keep one order whatever the rows, so that near-ties of the choice fall
-  // alike in every step; 2048 x 24 x 2048 in 8 ranges would save 4 us)
-  return M > 8 && M <= 65535 && N >= 64 && K > 0 ? lgs::gemm_plan(M, N, K, 1, false, 0).ksplit : 1;
+  return M > 8 && M <= 65535 && N > 0 && K > 0 ? lgs::gemm_plan(M, N, K, 1, false, 0).ksplit : 1;
 }
 
 extern "C" int lgs_embed(const int* tokens, const void* table, int w_f32, float scale, float* x, int T, int W,

@@ -81,7 +81,8 @@ class LayeredBlock(nn.Module):
         h, h16 = self.norm1(x, bf16_copy=True) if tiles16 else (self.norm1(x), None)
         n_in, W = self.w_in.shape
         proj = torch.empty(step.T, n_in, dtype=torch.float32, device=x.device)
-        seq_ops.linear(h16 if tiles16 else h, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in, bias=self.b_in)
+        seq_ops.linear(h16 if tiles16 else h, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in, bias=self.b_in,
+                       ksplit=self.mixer.in_ksplit if self.mlp is None else self.mlp.in_ksplit)
         self.mixer(proj, step, cache, x)
         if self.mlp is not None:
             self.mlp(proj, h, x, h16=h16)
@@ -142,7 +143,7 @@ class Sublayer(nn.Module):
             return y
         proj = torch.empty(step.T, n_in, dtype=torch.float32, device=h.device)
         seq_ops.linear(h if h16 is None else h16, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in,
-                       bias=self.b_in)
+                       bias=self.b_in, ksplit=self.module.in_ksplit)
         if cache is None:
             self.module(proj, h, y, h16=h16, accumulate=False)
         else:
@@ -200,7 +201,7 @@ class PostSublayer(nn.Module):
         if self.module.wants_proj(step.T):
             proj = torch.empty(step.T, n_in, dtype=torch.float32, device=x.device)
             seq_ops.linear(x if x16 is None else x16, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in,
-                           bias=self.b_in)
+                           bias=self.b_in, ksplit=self.module.in_ksplit)
         y = torch.empty(step.T, W, dtype=torch.float32, device=x.device)
         if cache is None:
             self.module(proj, x, y, h16=x16, accumulate=False)
@@ -280,7 +281,7 @@ class SandwichSublayer(nn.Module):
             n_in = self.w_in.shape[0]
             proj = torch.empty(T, n_in, dtype=torch.float32, device=src.device)
             seq_ops.linear(src, self.w_in, M=T, N=n_in, K=W, y=proj, lda=W, ldy=n_in, bias=self.b_in,
-                           ksplit=0 if src.dtype == torch.bfloat16 else seq_ops.thin_ksplit(T, n_in, W, self.w_in))
+                           ksplit=self.module.in_ksplit if src.dtype == torch.bfloat16 else seq_ops.thin_ksplit(T, n_in, W, self.w_in))
         if cache is None:
             self.module(proj, h, y, h16=h16, accumulate=False)
         elif getattr(self.module, "branch_norm", False):

@@ -111,6 +111,10 @@ class InputReader(nn.Module):
         """Whether the module makes its input projection itself in this step (``forward_fused``)."""
         return False
 
+    # ranges of K of the input projection (0: as many as suit its size). A router's logits are whole in every step, so that a
+    # token's near ties fall alike however many rows stand beside it
+    in_ksplit = 0
+
     def forward_in(self, h16: Optional[torch.Tensor], w_in: torch.Tensor, x: torch.Tensor, accumulate: bool = False) -> bool:
         """A module without a cache, straight from its sublayer's input (a bf16 copy) and fused input matrix; False:
         nothing done, the input projection and ``forward`` make it."""
@@ -947,6 +951,8 @@ class SparseFeedForward(InputReader):
     token's choices in routing order."""
 
     STREAM_PAIRS = 48  # up to this many (token, choice) pairs the streaming form runs
+    in_ksplit = 1
+
     def __init__(self, spec: FeedForwardSpec, width: int, w: Dict[str, torch.Tensor], device, dtype,
                  act: Optional[int] = None, route: str = "top_logits") -> None:
         super().__init__()
