@@ -75,8 +75,13 @@ int lga_q4_gemm(const void* x, const uint8_t* qweight, const void* scales, const
  * weights, fp32 accumulation, one bf16 rounding (+bias), then + residual. */
 int lga_q4f_fits(int M, int N, int K, int group, int fmt);
 /* Short prompts split K across workgroups: the caller passes a zero-initialised workspace of at least this many
- * bytes (0 = none needed) and keeps it for later calls (its per-tile counters are left zeroed). */
+ * bytes (0 = none needed; the largest of all formats') and keeps it for later calls (its per-tile counters are left
+ * zeroed). */
 size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu);
+/* How a product of one format is made: 0 the LDS-image tiles, 1 4-bit weights dequantized in registers, 2 the bf16 weights'
+ * pipelined tiles. workspace_bytes: what this form needs; counters: 1 where its first 4096 bytes are counters that have to
+ * be zero (else the workspace need not be cleared nor kept). Either may be NULL. */
+int lga_q4f_plan(int M, int N, int K, int swiglu, int fmt, size_t* workspace_bytes, int* counters);
 int lga_q4_gemm_fused(const void* x, const void* weight, const void* scales, const void* bias, const void* residual,
                       void* y, int M, int N, int K, int group, int fmt, void* workspace, size_t workspace_bytes,
                       lga_stream_t stream);

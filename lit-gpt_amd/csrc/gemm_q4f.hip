@@ -744,19 +744,35 @@ int run_tiles(Args a, int fmt, bool dual, int bn, hipStream_t stream);
 // LGA_Q4F_BN / LGA_Q4F_SPLITS name a launch of the tiles here
 bool tiles_named() { return getenv("LGA_Q4F_BN") || getenv("LGA_Q4F_SPLITS"); }
 
-int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t stream) {
-  if (!tiles_named()) {  // 4-bit weights dequantized in registers (gemm_q4d.hip), bf16 weights on gemm_bf16.hip's tiles
-    const int kf = lga::kernel_fmt(fmt);
-    const lga::Q4dPlan dp = kf == 2 ? lga::Q4dPlan{} : lga::q4d_plan(a.M, a.N, a.K, dual);
-    const lga::GemmPlan bp = kf == 2 ? lga::bf16_plan(a.M, a.N, a.K, dual) : lga::GemmPlan{-1, 1};
-    if (dp.mf > 0 || bp.tile >= 0) {
-      const size_t need = dp.mf > 0 ? lga::q4d_workspace(dp, a.M, a.N, dual) : lga::bf16_workspace(bp, a.M, a.N, dual);
-      LGA_CHECK_ARG(need == 0 || (ws && ws_bytes >= need),
-                    "lga_q4_gemm_fused: split-K needs the workspace lga_q4f_workspace_bytes reports");
-      const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
-                           lga::codebook_of(fmt), need ? (float*)((unsigned char*)ws + 4096) : nullptr};
-      return dp.mf > 0 ? lga::q4d_run(d, dp, kf, dual, stream) : lga::bf16_run(d, bp, dual, stream);
+// which form makes a product, and the workspace of the form that it makes
+enum Form { kTiles = 0, kRegisters = 1, kBf16Tiles = 2 };  // here; gemm_q4d.hip (4-bit); gemm_bf16.hip
+struct Route {
+  Form form = kTiles;
+  lga::Q4dPlan d{};
+  lga::GemmPlan b{-1, 1};
+  size_t need = 0;
+};
+Route route(int M, int N, int K, int fmt, bool dual) {
+  Route r;
+  if (!tiles_named()) {
+    if (lga::kernel_fmt(fmt) == 2) {
+      r.b = lga::bf16_plan(M, N, K, dual);
+      if (r.b.tile >= 0) r.form = kBf16Tiles, r.need = lga::bf16_workspace(r.b, M, N, dual);
+    } else {
+      r.d = lga::q4d_plan(M, N, K, dual);
+      if (r.d.mf > 0) r.form = kRegisters, r.need = lga::q4d_workspace(r.d, M, N, dual);
     }
+  }
+  if (r.form == kTiles && (dual || q4f_big_columns(M, N, K) == 0)) r.need = ws_need(q4f_plan(M, N, K, dual), M, N, dual);
+  return r;
+}
+
+int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t stream) {
+  const Route r = route(a.M, a.N, a.K, fmt, dual);
+  if (r.form != kTiles && (r.need == 0 || (ws && ws_bytes >= r.need))) {  // (a smaller workspace may do for the tiles here)
+    const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
+                         lga::codebook_of(fmt), r.need ? (float*)((unsigned char*)ws + 4096) : nullptr};
+    return r.form == kRegisters ? lga::q4d_run(d, r.d, lga::kernel_fmt(fmt), dual, stream) : lga::bf16_run(d, r.b, dual, stream);
   }
   if (!dual) {
     const int nb = q4f_big_columns(a.M, a.N, a.K);
@@ -846,15 +862,18 @@ extern "C" int lga_q4f_trace_read(unsigned long long* host, int n) {
 
 extern "C" int lga_q4f_fits(int M, int N, int K, int group, int fmt) { return q4f_fits(M, N, K, group, fmt) ? 1 : 0; }
 
+extern "C" int lga_q4f_plan(int M, int N, int K, int swiglu, int fmt, size_t* workspace_bytes, int* counters) {
+  const bool ok = M >= 1 && N >= 1 && K >= lga::pf::BK && fmt >= 0 && fmt <= 3;
+  const Route r = ok ? route(M, N, K, fmt, swiglu != 0) : Route();
+  if (workspace_bytes) *workspace_bytes = r.need;
+  if (counters) *counters = r.form == kTiles && r.need > 0;
+  return r.form;
+}
+
 extern "C" size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu) {
   if (M < 1 || N < 1 || K < lga::pf::BK) return 0;
-  // (the weights' format is not known here: the largest of the plans)
-  const Plan p = q4f_plan(M, N, K, swiglu != 0);
-  size_t need = ws_need(p, M, N, swiglu != 0);
-  if (!tiles_named()) {
-    need = std::max(need, lga::q4d_workspace(lga::q4d_plan(M, N, K, swiglu != 0), M, N, swiglu != 0));
-    need = std::max(need, lga::bf16_workspace(lga::bf16_plan(M, N, K, swiglu != 0), M, N, swiglu != 0));
-  }
+  size_t need = ws_need(q4f_plan(M, N, K, swiglu != 0), M, N, swiglu != 0);
+  for (int fmt : {0, 2}) need = std::max(need, route(M, N, K, fmt, swiglu != 0).need);
   return need;
 }
 

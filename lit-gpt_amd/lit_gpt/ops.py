@@ -46,6 +46,7 @@ SIGNATURES = {
     "lga_q4_gemm": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "lga_q4f_fits": [_I, _I, _I, _I, _I],
     "lga_q4f_workspace_bytes": [_I, _I, _I, _I],
+    "lga_q4f_plan": [_I, _I, _I, _I, _I, ctypes.POINTER(_SZ), ctypes.POINTER(_I)],
     "lga_q4_gemm_fused": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P],
     "lga_q4_gemm_swiglu": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P],
     "lga_q4_dequantize": [_P, _P, _P, _I, _I, _I, _I, _P],
@@ -229,22 +230,37 @@ def q4f_fits(M, N, K, group, fmt) -> bool:
 _Q4F_WS: dict = {}
 
 
-def _q4f_workspace(M, N, K, swiglu, device):
-    """The split-K workspace of a short-prompt fused GEMM: one zeroed buffer per device and stream (products on two
-    streams may run at once), grown as needed (its per-tile counters are left zeroed by every launch). Returns
-    (ptr, bytes) or (None, 0)."""
-    need = int(load_library().lga_q4f_workspace_bytes(int(M), int(N), int(K), int(bool(swiglu))))
+def q4f_plan(M, N, K, swiglu, fmt):
+    """How a fused product of this format is made (lga_q4f_plan): (form, workspace bytes, whether it holds counters)."""
+    need, counters = _SZ(0), _I(0)
+    form = load_library().lga_q4f_plan(int(M), int(N), int(K), int(bool(swiglu)), int(fmt), ctypes.byref(need),
+                                       ctypes.byref(counters))
+    return form, need.value, bool(counters.value)
+
+
+def _q4f_workspace(M, N, K, swiglu, fmt, device):
+    """The split-K workspace of a short-prompt fused GEMM, or None: for the caller to hold until its launch. Partial sums
+    alone come from the allocator per product. The form with per-tile counters keeps a zeroed buffer per device and stream
+    (products on two streams may run at once), grown as needed: a launch leaves its counters zeroed; under
+    capture it has one of the graph's own, whose counters every replay clears."""
+    _, need, counters = q4f_plan(M, N, K, swiglu, fmt)
     if need == 0:
-        return None, 0
-    if torch.cuda.is_current_stream_capturing():  # a graph's own memory, its counters cleared by every replay
+        return None
+    if not counters:
+        return torch.empty(need, dtype=torch.uint8, device=device)
+    if torch.cuda.is_current_stream_capturing():
         ws = torch.empty(need, dtype=torch.uint8, device=device)
         ws[:4096].zero_()
-        return ws.data_ptr(), need  # (nothing is allocated before the launch that follows in stream order)
+        return ws
     key = device, _stream()
     ws = _Q4F_WS.get(key)
     if ws is None or ws.numel() < need:
         ws = _Q4F_WS[key] = torch.zeros(need, dtype=torch.uint8, device=device)
-    return ws.data_ptr(), ws.numel()
+    return ws
+
+
+def _ws_args(ws):
+    return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
 
 
 def q4_gemm_fused(x, weight, scales, N, K, group, fmt, *, bias=None, residual=None, out=None):
@@ -253,11 +269,11 @@ def q4_gemm_fused(x, weight, scales, N, K, group, fmt, *, bias=None, residual=No
     M = x.shape[0]
     y = out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
     wdt = torch.bfloat16 if fmt == 2 else torch.uint8
-    ws, nws = _q4f_workspace(M, N, K, False, x.device)
+    ws = _q4f_workspace(M, N, K, False, fmt, x.device)
     _check(load_library().lga_q4_gemm_fused(_dev(x, "x", torch.bfloat16), _dev(weight, "weight", wdt),
                                             _opt(scales, "scales"), _opt(bias, "bias", torch.bfloat16),
                                             _opt(residual, "residual", torch.bfloat16), _dev(y, "y", torch.bfloat16),
-                                            M, N, K, group, fmt, ws, nws, _stream()))
+                                            M, N, K, group, fmt, *_ws_args(ws), _stream()))
     return y
 
 
@@ -266,10 +282,10 @@ def q4_gemm_swiglu(x, w1, s1, w2, s2, N, K, group, fmt, *, out=None):
     M = x.shape[0]
     y = out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
     wdt = torch.bfloat16 if fmt == 2 else torch.uint8
-    ws, nws = _q4f_workspace(M, N, K, True, x.device)
+    ws = _q4f_workspace(M, N, K, True, fmt, x.device)
     _check(load_library().lga_q4_gemm_swiglu(_dev(x, "x", torch.bfloat16), _dev(w1, "w1", wdt), _opt(s1, "s1"),
                                              _dev(w2, "w2", wdt), _opt(s2, "s2"), _dev(y, "y", torch.bfloat16),
-                                             M, N, K, group, fmt, ws, nws, _stream()))
+                                             M, N, K, group, fmt, *_ws_args(ws), _stream()))
     return y
 
 

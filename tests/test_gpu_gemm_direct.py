@@ -107,3 +107,46 @@ def test_captured(ops, M, N, K):
         assert torch.equal(outs[i], want)
         outs[i].zero_()
         assert torch.equal(ops.q4_gemm_fused(x, w, sc, N, K, 64, 1), want)
+
+
+@pytest.mark.parametrize("M,N,K,fmt", [(64, 4096, 4096, 1), (64, 512, 4160, 1), (100, 4096, 11008, 2)])
+def test_two_streams(ops, M, N, K, fmt):
+    """Split products on two streams at once, each between others of its stream: the partial sums and counters of one are
+    never the other's."""
+    g = torch.Generator(device=DEV).manual_seed(K)
+    work = []
+    for _ in range(2):
+        w, sc, wd = _weight(ops, N, K, fmt, 64, g)
+        x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+        work.append((x, w, sc, ops.q4_gemm_fused(x, w, sc, N, K, 64, fmt).clone()))
+    assert ops.q4f_plan(M, N, K, 0, fmt)[1] > 0
+    streams = [torch.cuda.Stream() for _ in work]
+    torch.cuda.synchronize()
+    outs = [[], []]
+    for _ in range(20):
+        for i, (x, w, sc, _) in enumerate(work):
+            with torch.cuda.stream(streams[i]):
+                outs[i].append(ops.q4_gemm_fused(x, w, sc, N, K, 64, fmt))
+    torch.cuda.synchronize()
+    for got, (_, _, _, want) in zip(outs, work):
+        assert all(torch.equal(y, want) for y in got)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 12288, 11008), (200, 512, 4096)])
+def test_a_workspace_of_the_older_tiles(ops, M, N, K, monkeypatch):
+    """A caller whose workspace (none, or a smaller one) serves the older tiles has their result."""
+    g = torch.Generator(device=DEV).manual_seed(K)
+    w, _, wd = _weight(ops, N, K, 2, 64, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    form, need, _ = ops.q4f_plan(M, N, K, 0, 2)
+    monkeypatch.setenv("LGA_Q4F_BN", "128")
+    older = ops.q4f_plan(M, N, K, 0, 2)[1]
+    monkeypatch.delenv("LGA_Q4F_BN")
+    assert form == 2 and older < need
+    ws = torch.zeros(older, dtype=torch.uint8, device=DEV)
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    rc = ops.load_library().lga_q4_gemm_fused(x.data_ptr(), w.data_ptr(), None, None, None, y.data_ptr(), M, N, K, 64, 2,
+                                              ws.data_ptr() if older else None, older, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    h = x.float() @ wd.t()
+    assert float(((y.float() - h).abs() - h.abs() * 2 ** -7).max()) <= 2e-3
