@@ -15,6 +15,8 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import threading
+from collections import OrderedDict
 from pathlib import Path
 from typing import Optional
 
@@ -227,7 +229,9 @@ def q4f_fits(M, N, K, group, fmt) -> bool:
     return bool(load_library().lga_q4f_fits(int(M), int(N), int(K), int(group), int(fmt)))
 
 
-_Q4F_WS: dict = {}
+_Q4F_WS: "OrderedDict" = OrderedDict()  # (device, stream) -> workspace with counters, the last used at the end
+_Q4F_WS_MOST = 8
+_Q4F_WS_LOCK = threading.Lock()
 
 
 def q4f_plan(M, N, K, swiglu, fmt):
@@ -241,8 +245,8 @@ def q4f_plan(M, N, K, swiglu, fmt):
 def _q4f_workspace(M, N, K, swiglu, fmt, device):
     """The split-K workspace of a short-prompt fused GEMM, or None: for the caller to hold until its launch. Partial sums
     alone come from the allocator per product. The form with per-tile counters keeps a zeroed buffer per device and stream
-    (products on two streams may run at once), grown as needed: a launch leaves its counters zeroed; under
-    capture it has one of the graph's own, whose counters every replay clears."""
+    (products on two streams may run at once), grown as needed, the eight last used: a launch leaves its counters zeroed;
+    under capture it has one of the graph's own, whose counters every replay clears."""
     _, need, counters = q4f_plan(M, N, K, swiglu, fmt)
     if need == 0:
         return None
@@ -253,9 +257,13 @@ def _q4f_workspace(M, N, K, swiglu, fmt, device):
         ws[:4096].zero_()
         return ws
     key = device, _stream()
-    ws = _Q4F_WS.get(key)
-    if ws is None or ws.numel() < need:
-        ws = _Q4F_WS[key] = torch.zeros(need, dtype=torch.uint8, device=device)
+    with _Q4F_WS_LOCK:
+        ws = _Q4F_WS.pop(key, None)
+        if ws is None or ws.numel() < need:
+            ws = torch.zeros(need, dtype=torch.uint8, device=device)
+        _Q4F_WS[key] = ws
+        while len(_Q4F_WS) > _Q4F_WS_MOST:  # (given back in the order of its own stream)
+            _Q4F_WS.popitem(last=False)
     return ws
 
 

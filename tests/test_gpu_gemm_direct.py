@@ -132,6 +132,25 @@ def test_two_streams(ops, M, N, K, fmt):
         assert all(torch.equal(y, want) for y in got)
 
 
+def test_workspaces_are_given_back(ops):
+    """Workspaces with counters: of many streams the last used are kept, and a stream that comes back is served anew."""
+    M, N, K = 64, 512, 4160
+    assert ops.q4f_plan(M, N, K, 0, 1)[2]
+    g = torch.Generator(device=DEV).manual_seed(K)
+    w, sc, wd = _weight(ops, N, K, 1, 64, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    want = ops.q4_gemm_fused(x, w, sc, N, K, 64, 1).clone()
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(12)]
+    for _ in range(2):
+        for s in streams:
+            with torch.cuda.stream(s):
+                got = ops.q4_gemm_fused(x, w, sc, N, K, 64, 1)
+            s.synchronize()
+            assert torch.equal(got, want)
+    assert len(ops._Q4F_WS) <= ops._Q4F_WS_MOST
+
+
 @pytest.mark.parametrize("M,N,K", [(300, 12288, 11008), (200, 512, 4096)])
 def test_a_workspace_of_the_older_tiles(ops, M, N, K, monkeypatch):
     """A caller whose workspace (none, or a smaller one) serves the older tiles has their result."""
