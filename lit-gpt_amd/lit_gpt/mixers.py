@@ -211,15 +211,21 @@ class LatentAttention(InputReader):
             self.q_norm_w = _f32(w["dq.norm"], device)
         # per head (r, d): the key up-projection transposed, so that q_h (d values) maps to r latent coordinates
         self.register_buffer("w_ukT", w["uk"].to(device=device, dtype=dtype).view(H, d, r).transpose(1, 2).contiguous())
-        # both up-projections as they are, one under the other: prompts expand keys and values in one product
+        # both up-projections as they are, one under the other: prompts expand keys and values in one product. The key part
+        # is w_ukT's other layout (a product reads its matrix along K), not saved, and follows what is loaded
         up = torch.cat([w["uk"], w["uv"]]).to(device=device, dtype=dtype).contiguous()
-        self.register_buffer("w_up", up)
+        self.register_buffer("w_up", up, persistent=False)
         self.register_buffer("w_uv", up[H * d:])
+        self.register_load_state_dict_post_hook(LatentAttention._follow)
         self.register_buffer("w_o", w["o"].to(device=device, dtype=dtype).contiguous())
         self.register_buffer("norm_w", _f32(w["dkv.norm"], device))
         self.register_buffer("sink", _f32(w["sink"], device) if spec.sink_kind == "learned" and "sink" in w else None)
         self.register_buffer("inv_freq", torch.tensor(spec.rot.inv_freq() or [1.0], dtype=torch.float64)
                              .to(device=device, dtype=torch.float32))
+
+    def _follow(self, *_) -> None:
+        with torch.no_grad():
+            self.w_up.copy_(torch.cat([self.w_ukT.transpose(1, 2).reshape(self.H * self.d, self.r), self.w_uv]))
 
     def in_parts(self):
         return self._in
