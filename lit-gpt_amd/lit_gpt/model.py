@@ -365,7 +365,7 @@ class CausalSelfAttention(nn.Module):
             # decode token: RoPE + KV-append + attention in a single launch
             y = ops.attention_decode_fused(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem,
                                            1.0 / math.sqrt(hs), n_splits, workspace=ws)
-        elif T == 1 and self.fuse_decode and qkv.dtype == torch.float32 and ops.f32_decode_fusable(hs, S):
+        elif T == 1 and self.fuse_decode and qkv.dtype == torch.float32 and ops.f32_decode_fusable(hs, S, kc, vc):
             y = ops.f32_attention_decode(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem, 1.0 / math.sqrt(hs))
         else:
             q = ops.rope_kv_append(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem)

@@ -418,8 +418,9 @@ def attention(q, k_cache, v_cache, input_pos, n_head, n_query_groups, head_size,
     return y
 
 
-def f32_decode_fusable(head_size: int, max_seq: int) -> bool:
-    return head_size % 4 == 0 and head_size <= 256 and max_seq <= 32768
+def f32_decode_fusable(head_size: int, max_seq: int, *caches: torch.Tensor) -> bool:
+    """Whether f32_attention_decode serves these sizes over these caches (its loads are 16 bytes wide)."""
+    return head_size % 4 == 0 and head_size <= 256 and max_seq <= 32768 and all(t.data_ptr() % 16 == 0 for t in caches)
 
 
 def f32_attention_decode(qkv, k_cache, v_cache, cache_pos, rope_pos, cos, sin, n_head, n_query_groups, head_size,

@@ -57,3 +57,22 @@ def test_fused_norms_activations_and_adds(rows, n):
         lin = ops.f32_linear(x, m, bias=c[0])
         want = ops.gelu(lin, kind) + r + r2
         assert torch.equal(ops.f32_linear(x, m, bias=c[0].contiguous(), gelu=kind, residual=r, residual2=r2), want)
+
+
+def test_caches_off_sixteen_bytes():
+    """A decode step over caches that start on 4 bytes: the unfused form's."""
+    from generate.base import build_model
+    from lit_gpt import Config
+
+    dev = torch.device("cuda", 0)
+    m = build_model(Config.from_name("pythia-160m", n_layer=1), quantize=None, device=dev, seed=1, max_seq_length=64, dtype=torch.float32)
+    kv, outs = m.transformer.h[0].attn.kv_cache, []
+    idx, pos = torch.tensor([[5]], device=dev), torch.tensor([9], device=dev)
+    g = torch.Generator(device=dev).manual_seed(1)
+    filled = {n: torch.randn(getattr(kv, n).shape, generator=g, device=dev) for n in "kv"}
+    with torch.inference_mode():
+        for off in (0, 1):
+            for n, t in filled.items():
+                setattr(kv, n, torch.empty(t.numel() + off, device=dev)[off:].view(t.shape).copy_(t))
+            outs.append(m(idx, pos).clone())
+    assert float((outs[0] - outs[1]).abs().max()) < 1e-5 * float(outs[0].abs().max())
