@@ -11,6 +11,12 @@
 // O^T += V^T P^T as they stand: the transposed LDS reads of V take the keys in the order in which a lane holds them.
 // Unless eight (head, map) pairs share the keys, two waves split every key tile and are merged at the end.
 //
+// Error against float64 beside the thread-per-key form's (rms over the sizes of the tests): 0.5 to 0.9 of it with one map, 0.5
+// to 0.85 with two. The two-summand form's operands are less than fp32 (the query's two summands are cut at 16 bits, keys and
+// values rounded at 16 or 17, the product of both second summands is left out), in rotated parts too, which the latent form
+// multiplies in fp32; but that form rounds queries and weighted latents to bf16: the heads' outputs are 5e-6 to 1.8e-5 off
+// float64 here and 1.5e-3 to 3.4e-3 there, with rotated parts that outweigh the others 6e-6 and 1.5e-3.
+//
 // The two-summand form serves latent attention: expanded keys of 192 and values of 128, 4096 tokens of 16 heads in 372 us
 // (205 TFLOP/s of fp32-like products) with 26 us for the summands and 20 for the expansion; the fp32 tiles in the latent
 // space took 7.7 ms (2176 operations per pair and head instead of 640, at a sixteenth of the bf16 rate).
@@ -57,7 +63,9 @@ __device__ __forceinline__ bf16x8_t take_summand(float (&x)[8]) {
   return __builtin_bit_cast(bf16x8_t, o);
 }
 
-// e^x for x <= 0 (about one unit in the last place): 2^t for the rounded product, times the rounding's own power
+// e^x for x <= 0: 2^t for the rounded product, times the rounding's own power. 3.6e-8 rms and 1.4e-7 at most off float64,
+// where expf has 2.6e-8 and 8.3e-8; whole rows are nearer to float64 than those of the thread-per-key form with expf (0.5 to
+// 0.9 of its error over the sizes of the tests), whose scores are one long chain of fp32 sums
 __device__ __forceinline__ float exp_neg(float x) {
   const float t = x * 1.44269502f;
   float r = fmaf(x, 1.44269502f, -t);
@@ -66,7 +74,9 @@ __device__ __forceinline__ float exp_neg(float x) {
   return fmaf(e, r * 0.69314718f, e);
 }
 
-// tanh x: below 0.625 the odd polynomial of the Cephes library's tanhf, above 1 - 2 / (e^2|x| + 1) (2e-7 relative)
+// tanh x: below 0.625 the odd polynomial of the Cephes library's tanhf, above 1 - 2 e^-2|x| / (1 + e^-2|x|). Errors against
+// float64 (rms): 3.6e-8 in [0.625, 1], 1.9e-8 in [1, 3], where tanhf has 3.8e-8 and 1.9e-8. (An infinite x gives NaN, and its
+// row goes to attn_row_plain.)
 __device__ __forceinline__ float tanh_near(float x) {
   const float z = x * x, y = fabsf(x);
   float p = fmaf(-5.70498872745e-3f, z, 2.06390887954e-2f);
@@ -74,12 +84,12 @@ __device__ __forceinline__ float tanh_near(float x) {
   p = fmaf(p, z, 1.33314422036e-1f);
   p = fmaf(p, z, -3.33332819422e-1f);
   p = fmaf(p * z, x, x);
-  const float e = __builtin_amdgcn_exp2f(y * 2.88539008f);
-  const float q = copysignf(fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f), x);
-  return y < 0.625f ? p : q;
+  const float e = exp_neg(-2.0f * y), d = 1.0f + e;
+  const float r = __builtin_amdgcn_rcpf(d), q = fmaf(-2.0f * e, fmaf(fmaf(-d, r, 1.0f), r, r), 1.0f);
+  return y < 0.625f ? p : copysignf(q, x);
 }
 
-// 1 / (1 + e^-z) from e^-|z|, which is 0 from 120 on (an infinite z has no residual in exp_neg; a NaN stays one)
+// 1 / (1 + e^-z) from e^-|z| (3.8e-8 rms for z >= 0, 5.5e-8 below; sigmoid_f 3.8e-8), which is 0 from 120 on (an infinite z has no residual in exp_neg; a NaN stays one)
 __device__ __forceinline__ float sigmoid_near(float z) {
   const float e = exp_neg(fabsf(z) > 120.0f ? -120.0f : -fabsf(z)), d = 1.0f + e;
   const float r = __builtin_amdgcn_rcpf(d), p = fmaf(fmaf(-d, r, 1.0f), r, r);
@@ -309,8 +319,10 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
       for (int e = 0; e < 8; ++e) {
         const float v = s[8 * kk + e];
         w[e] = v == -INFINITY ? 0.0f : (SIG ? sigmoid_near(v + bias) : exp_neg(v - mref));
-        if (!SIG) l += w[e];
+        if (!SIG && MAPS == 1) l += w[e];
       }
+      // (a difference of two maps, scaled up to unit size, shows what their normalisers lose in one long chain)
+      if (MAPS == 2) l += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
       bf16x8_t pw[3];
 #pragma unroll
       for (int e = 0; e < 3; ++e) pw[e] = take_summand(w);
@@ -323,6 +335,18 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
           const i16x4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vk + at(vaddr0, part * DT * 4 + t * 4)));
           const i16x4_t y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vk + at(vaddr1, part * DT * 4 + t * 4)));
           const bf16x8_t vt = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+          // The least summands first, then one rounding of the sum so far: 2.4e-7 off float64 with a cap of 3 over 1213 keys,
+          // 4.3e-7 with the products one after the other, 4.0e-7 in the thread-per-key form, whose chains are shorter for
+          // values of 64. (Of 128 the chain is no worse than that form's: 4.3e-7 and 5.2e-7.)
+          if (MAPS == 2 && DT == 2) {
+            f32x16_t c;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) c[r] = 0.0f;
+#pragma unroll
+            for (int e = 2; e >= 0; --e) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vt, pw[e], c, 0, 0, 0);
+            o[t] += c;
+            continue;
+          }
 #pragma unroll
           for (int e = 0; e < 3 - part; ++e) o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vt, pw[e], o[t], 0, 0, 0);
         }

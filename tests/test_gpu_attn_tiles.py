@@ -1,7 +1,7 @@
 """Prompt attention on the bf16 matrix cores (csrc/seq_attn_tiles.hip) against float64 and against the thread-per-key form.
 
-The same bf16 keys and values in an fp32 cache take the thread-per-key form, whose products are fp32: the matrix-core form
-has to be as close to float64 as that one. Its own bound: with scores of a few units, 2e-6 relative in the 2-norm covers
+The same bf16 keys and values in an fp32 cache take the thread-per-key form, whose products are fp32: the matrix-core form's
+error against float64 is no larger than that one's. Its own bound: with scores of a few units, 2e-6 relative in the 2-norm covers
 the scores' rounding (24 bits of a sum of up to 192 products), the exponentials and up to 2000 weighted values.
 """
 
@@ -50,7 +50,7 @@ STEPS = [([2], [61]), ([16], [0]), ([17, 1, 40], [0, 5, 100]), ([300, 64, 129], 
 @pytest.mark.parametrize("lengths,pos0", STEPS)
 @pytest.mark.parametrize("d,dv", [(64, 64), (64, 128), (128, 64), (128, 128)])
 @pytest.mark.parametrize("H,G,options", [
-    (4, 1, {}), (4, 4, dict(sink=True)), (6, 3, dict(chunk=48)), (8, 2, dict(window=33, gate=1)), (3, 1, dict(sigmoid=True)),
+    (4, 1, {}), (4, 4, dict(sink=True)), (4, 2, dict(cap=3.0)), (6, 3, dict(chunk=48)), (8, 2, dict(window=33, gate=1)), (3, 1, dict(sigmoid=True)),
     (8, 1, dict(sink=True, cap=5.0, rotated=True)), (4, 2, dict(gate=2, rotated=True, interleaved=True, chunk=100)),
     (8, 2, dict(sigmoid=True, chunk=64))])
 def test_one_map(lengths, pos0, d, dv, H, G, options):
@@ -105,7 +105,7 @@ def test_one_map(lengths, pos0, d, dv, H, G, options):
     want = want.flatten(1)
     # (turning back by fp32 angles of up to 1200 radians: both forms take the same cosines, off by up to 1e-4)
     bound = 1e-4 if freq is not None else TOL
-    assert rel(got, want) < bound and rel(got, want) < 1.5 * rel(plain, want) + 1e-7
+    assert rel(got, want) < bound and rel(got, want) < 1.001 * rel(plain, want)  # (turned back: the same angles' errors)
     assert torch.equal(got16, got.bfloat16())
 
 
@@ -142,7 +142,7 @@ def test_two_maps(lengths, pos0, dv, H, G, chunk, cap):
             want[rows, h] = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * 0.5
     want = want.flatten(1)
     # (a query that sees one key has two equal maps: their difference keeps all bits here, and nothing cancels)
-    assert rel(got, want) < TOL and rel(got, want) < 1.5 * rel(plain, want) + 1e-7
+    assert rel(got, want) < TOL and rel(got, want) < rel(plain, want)
 
 
 def test_caches_off_sixteen_bytes():
