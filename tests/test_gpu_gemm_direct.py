@@ -1,7 +1,7 @@
 """Prompt products whose 4-bit weights are dequantized in registers (csrc/gemm_q4d.hip) and those of bf16 weights on the
-pipelined tiles (csrc/gemm_bf16.hip), reached through ops.q4_gemm_fused and ops.q4_gemm_swiglu, against the fp32 product of the bit-exact dequantized weight (lga_q4_dequantize): rows at and around
-the 16-row pieces and the 128-row tile, columns that end inside a tile and inside a wave's piece, one to many blocks of
-K, whole and split, and every epilogue. Tolerances: the two sums' bf16 roundings may each fall one place apart."""
+pipelined tiles (csrc/gemm_bf16.hip), reached through ops.q4_gemm_fused and ops.q4_gemm_swiglu, against the fp32 product of
+the bit-exact dequantized weight (lga_q4_dequantize): rows at and around the 16-row pieces and the 128-row tile, columns that
+end inside a tile and inside a wave's piece, one to many blocks of K, whole and split, and every epilogue. Tolerances: the two sums' bf16 roundings may each fall one place apart."""
 
 import pytest
 import torch
@@ -78,6 +78,7 @@ def test_rule_falls_back(ops):
     assert lib.lga_q4f_workspace_bytes(64, 12288, 4096, 0) >= 4096 + 64 * 12288 * 4
     g = torch.Generator(device=DEV).manual_seed(5)
     for M, N, K in ((40, 264, 192), (16, 512, 1024), (257, 264, 256)):
+        assert ops.q4f_plan(M, N, K, 0, 1)[0] == 0
         w, sc, wd = _weight(ops, N, K, 1, 64, g)
         x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
         h = x.float() @ wd.t()
