@@ -559,10 +559,14 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
                 "lgs_linear: K is split for one plain product on the MFMA tiles, with a workspace");
   // Several rows on the matrix cores (us here / a lane's sums): 5 to 8 rows of at least 2048 columns (8 x 2048 x 2048 11.5 /
   // 12.4, x 8256 x 2048 21 / 26, x 4096 x 11008 28 / 85, x 32000 x 4096 68 / 104; x 512 x 2048 11.4 / 6.1), 3 and 4 rows
-  // from K 4096 (4 x 4096 x 4096 12.7 / 20.8, x 20608 x 4096 45 / 55; x 10304 x 2048 21 / 19); 2 x 20608 x 4096 44 / 38
+  // from K 4096 (4 x 4096 x 4096 12.7 / 20.8, x 20608 x 4096 45 / 55; x 10304 x 2048 21 / 19); 2 x 20608 x 4096 44 / 38.
+  // 16 columns a workgroup while that is one to a compute unit, 32 beyond (us of 16 / 32 columns: 8 x 4096 x 4096 14.3 / 18.2,
+  // x 4608 x 4096 23.2 / 19.0, x 20608 x 4096 61 / 49; x 8256 x 2048 21.5 / 22.0), the same sums either way. Below 4096 columns
+  // eight waves share K, not four (8 x 2048 x 2048: 11.8; four would take 9.3 and add in another order). A row's bits are not
+  // those that it has alone: lin_gemv_kernel adds in another order
   if (!z_start && !a_rows && !w_f32 && M > 2 && M <= 8 && N >= 2048 && (M > 4 || K >= 4096) && K % 128 == 0 && lda % 4 == 0 &&
       stride_a % 4 == 0 && stride_w % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0) {
-    if (N > 4608) lgs::lin_rows_kernel<2, 4><<<dim3((N + 31) / 32, batch), 256, 0, stream>>>(p);
+    if (N > 4096) lgs::lin_rows_kernel<2, 4><<<dim3((N + 31) / 32, batch), 256, 0, stream>>>(p);
     else if (N >= 4096) lgs::lin_rows_kernel<1, 4><<<dim3((N + 15) / 16, batch), 256, 0, stream>>>(p);
     else lgs::lin_rows_kernel<1, 8><<<dim3((N + 15) / 16, batch), 512, 0, stream>>>(p);
     LGA_LAUNCH_RETURN();

@@ -276,6 +276,8 @@ class LatentAttention(InputReader):
         self._finish(att, proj, x, accumulate, b16)
 
     def _expands(self, step: StepBatch, cache: LatentKVCache, ldq: int, q_off: int) -> bool:
+        # From 8 rows a sequence on, as the latent form's own tiles: us of the whole mixer expanded / latent, 16 heads, 9 tokens
+        # 103 / 101, 40 106 / 103, 4 x 16 105 / 103 (bound by the launches), 100 102 / 141, 1000 160 / 823; 32 heads, 40 103 / 114
         # (latents that a caller keeps in fp32 are not rounded on their way through the bf16 product that expands them; a
         # captured step reads its positions from the device at every replay, where `fresh` need not hold any more)
         return step.fresh and not torch.cuda.is_current_stream_capturing() and (step.max_len or step.T) > 1 and \
