@@ -109,11 +109,10 @@ int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream)
   const int steps = a.K / 64, kper = (steps + p.ksplit - 1) / p.ksplit;
   const BfArgs k{a, 0, 0, (steps + kper - 1) / kper, kper};
   switch (p.tile) {
-    case 0: bf16_go<2, 4, 4, 2, 32, 5>(k, dual, stream); break;
-    case 1: bf16_go<4, 2, 2, 2, 64, 3>(k, dual, stream); break;
-    case 2: bf16_go<2, 2, 2, 2, 64, 2>(k, dual, stream); break;
-    case 3: bf16_go<2, 4, 2, 1, 64, 4>(k, dual, stream); break;
-    default: bf16_go<1, 4, 2, 1, 64, 4>(k, dual, stream); break;
+#define LGA_CASE(I, SLOTS, US, ...) \
+  case I: bf16_go<__VA_ARGS__>(k, dual, stream); break;
+    LGA_GEMM_FORMS(LGA_CASE)
+#undef LGA_CASE
   }
   if (k.splits > 1) q4d_sum(a, k.splits, dual, stream);
   LGA_LAUNCH_RETURN();
@@ -121,12 +120,9 @@ int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream)
 
 int preload_gemm_bf16() {
   int bad = 0;
-#define LGA_PRE(...) bad += preload(gemm_bf16_kernel<__VA_ARGS__, false>) + preload(gemm_bf16_kernel<__VA_ARGS__, true>)
-  LGA_PRE(2, 4, 4, 2, 32, 5);
-  LGA_PRE(4, 2, 2, 2, 64, 3);
-  LGA_PRE(2, 2, 2, 2, 64, 2);
-  LGA_PRE(2, 4, 2, 1, 64, 4);
-  LGA_PRE(1, 4, 2, 1, 64, 4);
+#define LGA_PRE(I, SLOTS, US, ...) \
+  bad += preload(gemm_bf16_kernel<__VA_ARGS__, false>) + preload(gemm_bf16_kernel<__VA_ARGS__, true>);
+  LGA_GEMM_FORMS(LGA_PRE)
 #undef LGA_PRE
   return bad;
 }

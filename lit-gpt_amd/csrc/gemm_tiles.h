@@ -157,12 +157,20 @@ __device__ __forceinline__ void gemm_dma_at(int R, int lane, int* row, int* chun
 // what a large matrix product reaches on this card), of 256 x 128 1.02, of 128 x 128 0.63 alone on a compute unit and
 // 1.14 for two, of 64 x 128 0.43. The larger tile moves fewer bytes per product, the smaller ones fill the chip when
 // rows or columns are few. A workgroup's start and end cost about 3 us.
+// X(index, workgroups of the whole chip at a time, us, waves WM x WN, fragments FM x FN, BK, stages)
+#define LGA_GEMM_FORMS(X)                  \
+  X(0, 256, 1.80f, 2, 4, 4, 2, 32, 5)      \
+  X(1, 256, 1.02f, 4, 2, 2, 2, 64, 3)      \
+  X(2, 512, 1.14f, 2, 2, 2, 2, 64, 2)      \
+  X(3, 256, 0.63f, 2, 4, 2, 1, 64, 4)      \
+  X(4, 256, 0.43f, 1, 4, 2, 1, 64, 4)
 struct GemmForm {
-  int bm, bn, slots;  // slots: workgroups of the whole chip at a time
+  int bm, bn, slots;
   float step_us;
 };
-constexpr GemmForm kGemmForms[] = {{256, 256, 256, 1.80f}, {256, 128, 256, 1.02f}, {128, 128, 512, 1.14f},
-                                  {128, 128, 256, 0.63f}, {64, 128, 256, 0.43f}};
+#define LGA_GEMM_FORM(I, SLOTS, US, ...) {GemmTile<__VA_ARGS__>::BM, GemmTile<__VA_ARGS__>::BN, SLOTS, US},
+constexpr GemmForm kGemmForms[] = {LGA_GEMM_FORMS(LGA_GEMM_FORM)};
+#undef LGA_GEMM_FORM
 
 // Which form, and how many ranges of K (ksplit 0: the plan's own choice); tile -1: K is no multiple of 64.
 struct GemmPlan {

@@ -232,13 +232,12 @@ static int glu_go(const LinArgs& p, const GluForm& f, int batch, hipStream_t str
 }
 
 int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
-  switch (lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, true).tile) {
-    case 0: return glu_go<2, 4, 4, 2, 32, 5>(p, f, batch, stream);
-    case 1: return glu_go<4, 2, 2, 2, 64, 3>(p, f, batch, stream);
-    case 2: return glu_go<2, 2, 2, 2, 64, 2>(p, f, batch, stream);
-    case 3: return glu_go<2, 4, 2, 1, 64, 4>(p, f, batch, stream);
-    default: return glu_go<1, 4, 2, 1, 64, 4>(p, f, batch, stream);
-  }
+#define LGS_CASE(I, SLOTS, US, ...) \
+  case I: return glu_go<__VA_ARGS__>(p, f, batch, stream);
+  switch (lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, true).tile) { LGA_GEMM_FORMS(LGS_CASE) }
+#undef LGS_CASE
+  lga_set_error("lgs_linear_glu: no such form");
+  return (int)hipErrorInvalidValue;
 }
 
 GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit) {
@@ -246,13 +245,12 @@ GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit) {
 }
 
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream) {
-  switch (plan.tile) {
-    case 0: return gemm_go<2, 4, 4, 2, 32, 5>(p, batch, stream);
-    case 1: return gemm_go<4, 2, 2, 2, 64, 3>(p, batch, stream);
-    case 2: return gemm_go<2, 2, 2, 2, 64, 2>(p, batch, stream);
-    case 3: return gemm_go<2, 4, 2, 1, 64, 4>(p, batch, stream);
-    default: return gemm_go<1, 4, 2, 1, 64, 4>(p, batch, stream);
-  }
+#define LGS_CASE(I, SLOTS, US, ...) \
+  case I: return gemm_go<__VA_ARGS__>(p, batch, stream);
+  switch (plan.tile) { LGA_GEMM_FORMS(LGS_CASE) }
+#undef LGS_CASE
+  lga_set_error("lgs_linear: no such form");
+  return (int)hipErrorInvalidValue;
 }
 
 }  // namespace lgs
