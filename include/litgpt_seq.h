@@ -191,7 +191,7 @@ int lgs_diffattn_prepare(float* proj, long ld, int q_off, int k_off, int v_off, 
                          int d, int dv, int rot_dims, int max_seq, lgs_stream_t stream);
 /* one token per sequence over bf16 caches: the query heads that a workgroup of lgs_diffattn (maps 2) or lgs_sinkattn (maps
  * 1) takes at a time where its splits are more than one and there is no window, score bias or fp32 cache; 0: one */
-int lgs_attn_one_heads(int maps, int H, int G, int d, int dv);
+int lgs_attn_one_heads(int maps, int B, int H, int G, int d, int dv);
 /* out[t][h] = post * unit_rms(a1 - lambda a2), a_m = softmax_j(cap(q_m . k_m,j * scale)) V over the cached rows
  * lo <= j <= position of the sequence's slot, lo = position - position % chunk (chunk 0: lo = 0);
  * cap(s) = cap tanh(s / cap) (cap 0: none); query head h reads key head h / (H / G). q: the rotated queries

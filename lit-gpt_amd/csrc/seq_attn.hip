@@ -539,8 +539,8 @@ __device__ __forceinline__ float attn_lanes_sum(float v) {
 // (B, H / HG, splits), HG query heads of one key head per workgroup. A key belongs to 16 lanes, 16 bytes of its key and
 // of its value row each; each of the workgroup's 16 such groups takes every 16th key, four at a time, whose loads are
 // in flight together and which share one rescale of the group's running maximum, normaliser and sums. These meet in
-// the wave's lanes, then in LDS, in a fixed order. Bound by the launch and the loads' latency: 8 sequences of 9 to 2047
-// keys, 16 heads on 4, 19 us, 2047 keys of two maps 9.5 (a thread a key and the scores in LDS: 53 and 15).
+// the wave's lanes, then in LDS, in a fixed order. Bound by the launch and the loads' latency: 16 heads on 4, 2047 keys, with
+// the merge 7.3 us, two maps 9.8, 8 sequences 15 and 18 (a thread a key and the scores in LDS: 11.7, 14, 38 and 49).
 template <int MAPS, int HG>
 __global__ void __launch_bounds__(256) attn_one_kernel(AttnArgs p) {
   constexpr int U = 4, NR = HG * MAPS;
@@ -666,20 +666,20 @@ __global__ void __launch_bounds__(256) attn_one_kernel(AttnArgs p) {
   }
 }
 
-// query heads per workgroup of attn_one_kernel; 0: not one of its sizes
-inline int attn_one_heads(int maps, int H, int G, int d, int dv) {
+// Query heads per workgroup of attn_one_kernel; 0: not one of its sizes. Two heads share what they read of a key, which pays
+// only where the (sequence, head) pairs alone fill the chip several times: 16 heads on 4, 2047 keys, us with one / two / four
+// heads a workgroup: 64 sequences 70 / 58 / 64, 24 sequences 33 / 37 / 47, 8 (8 splits) 15.2 / 15.7 / 19, 1 (16) 7.2 / 9.6 / 13.
+inline int attn_one_heads(int maps, int B, int H, int G, int d, int dv) {
   if (maps * d != 128 || dv != 128 || H <= 0 || G <= 0 || H % G != 0) return 0;
-  const int per = H / G, most = 4 / maps;
-  return per % most == 0 ? most : (per % 2 == 0 ? 2 : 1);
+  return H / G % 2 == 0 && (long)B * H >= 1024 ? 2 : 1;
 }
 template <int MAPS>
 static bool attn_one_launch(const AttnArgs& p, int cache_f32, int B, int splits, hipStream_t stream) {
-  const int hg = attn_one_heads(MAPS, p.H, p.G, p.d, p.dv);
+  const int hg = attn_one_heads(MAPS, B, p.H, p.G, p.d, p.dv);
   if (hg == 0 || splits < 2 || cache_f32 || p.window > 0 || p.score_bias || ((uintptr_t)p.cache_k | (uintptr_t)p.cache_v) % 16 != 0)
     return false;
   const dim3 grid(B, p.H / hg, splits);
-  if (hg == 4) attn_one_kernel<MAPS, 4 / MAPS><<<grid, 256, 0, stream>>>(p);
-  else if (hg == 2) attn_one_kernel<MAPS, 2><<<grid, 256, 0, stream>>>(p);
+  if (hg == 2) attn_one_kernel<MAPS, 2><<<grid, 256, 0, stream>>>(p);
   else attn_one_kernel<MAPS, 1><<<grid, 256, 0, stream>>>(p);
   return true;
 }
@@ -748,7 +748,9 @@ static int diffattn_launch(const AttnArgs& p, int cache_f32, dim3 grid, hipStrea
 }  // namespace lgs
 
 // query heads that a workgroup of the one-token form takes at a time (0: the general form)
-extern "C" int lgs_attn_one_heads(int maps, int H, int G, int d, int dv) { return lgs::attn_one_heads(maps, H, G, d, dv); }
+extern "C" int lgs_attn_one_heads(int maps, int B, int H, int G, int d, int dv) {
+  return lgs::attn_one_heads(maps, B, H, G, d, dv);
+}
 
 extern "C" int lgs_diffattn_prepare(float* proj, long ld, int q_off, int k_off, int v_off, void* cache_k, void* cache_v,
                                     int cache_f32, const float* inv_freq, const int* slot, const int* pos, int T, int H,

@@ -60,7 +60,7 @@ SIGNATURES = {
     "lgs_embed_streams": [_P, _P, _I, _F, _P, _I, _I, _I, _I, _P],
     "lgs_streams_step": [_P, _P, _P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _P],
     "lgs_diffattn_prepare": [_P, _L, _I, _I, _I, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
-    "lgs_attn_one_heads": [_I, _I, _I, _I, _I],
+    "lgs_attn_one_heads": [_I, _I, _I, _I, _I, _I],
     "lgs_diffattn": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _F,
                      _F, _P],
     "lgs_conv_silu": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
@@ -653,11 +653,14 @@ def diffattn_prepare(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, cac
 
 
 def _one_token_splits(maps: int, B: int, H: int, G: int, d: int, dv: int, span: int, cache: torch.Tensor) -> int:
-    """Workgroups that share one token's keys: enough to fill the chip, at least 64 (a head at a time: 128) keys each."""
-    heads = load_library().lgs_attn_one_heads(maps, H, G, d, dv) if cache.dtype == torch.bfloat16 else 0
-    if heads:
-        return max(2, min(64, 1024 * heads // max(1, B * H), (span + 63) // 64))
-    return max(1, min(64, 512 // max(1, B * H), (span + 127) // 128))
+    """Workgroups that share one token's keys: enough to fill the chip, at least 64 keys each (128 in the general form). A cache
+    of up to 64 positions is one launch of the general form. us of general / one-token form at 5 %, 30 % and all of the cache
+    filled, 16 heads on 4: 64 positions 5.5, 5.9, 7.2 / 6.8, 6.8, 6.9; 128 5.6, 6.5, 9.0 / 6.7, 6.9, 6.7; of 64 sequences 64
+    positions 6.6, 7.5, 10.4 / 8.3, 10.1, 10.9, 128 6.7, 8.6, 15.9 / 8.4, 10.7, 10.8, 300 7.1, 12.6, 37 / 9.1, 10.8, 18.8."""
+    pairs = max(1, B * H)
+    if span > 64 and cache.dtype == torch.bfloat16 and load_library().lgs_attn_one_heads(maps, B, H, G, d, dv):
+        return max(2, min(64, 1024 // pairs, (span + 63) // 64))
+    return max(1, min(64, 512 // pairs, (span + 127) // 128))
 
 
 def diffattn(proj: torch.Tensor, q_off: int, cache_k: torch.Tensor, cache_v: torch.Tensor, seq_start: torch.Tensor,

@@ -1,6 +1,6 @@
 """One-token attention over bf16 caches with 128-value rows (attn_one_kernel) against the general form (one split) and
-float64: sequences of one key to several hundred, shares that end inside a group of keys or hold none, one to four query
-heads a workgroup, masks, caps, sinks and gates. Tolerance: fp32 sums of weights that add up to one, on values of unit
+float64: sequences of one key to several hundred, shares that end inside a group of keys or hold none, one or two query
+heads a workgroup (two from 1024 pairs of sequence and head on), masks, caps, sinks and gates. Tolerance: fp32 sums of weights that add up to one, on values of unit
 variance: 2^-17."""
 
 import pytest
@@ -23,7 +23,7 @@ def _step(H, G, d2, dv, S, seed):
     return k, v, q, slots, StepBatch.build([(s, p, [0]) for s, p in zip(slots, POS)], torch.device(DEV, 0)), g
 
 
-@pytest.mark.parametrize("H,G", [(16, 4), (4, 2), (3, 3), (6, 1), (12, 2)])
+@pytest.mark.parametrize("H,G", [(16, 4), (4, 2), (3, 3), (6, 1), (12, 2), (128, 32), (128, 128)])
 @pytest.mark.parametrize("chunk,cap,sink", [(0, 0.0, False), (100, 0.0, True), (0, 5.0, True)])
 def test_sink(H, G, chunk, cap, sink):
     from lit_gpt import seq_ops
@@ -49,7 +49,7 @@ def test_sink(H, G, chunk, cap, sink):
     assert torch.equal(run(7), run(7))
 
 
-@pytest.mark.parametrize("H,G", [(8, 2), (3, 3), (6, 1)])
+@pytest.mark.parametrize("H,G", [(8, 2), (3, 3), (6, 1), (128, 64)])
 @pytest.mark.parametrize("chunk,cap", [(0, 30.0), (64, 0.0)])
 def test_two_maps(H, G, chunk, cap):
     from lit_gpt import seq_ops
