@@ -47,8 +47,9 @@ int lgs_linear(const void* a, long lda, long stride_a, const void* w, int w_f32,
 /* Y (bf16, M x n) = act(A Wg^T) * (A Wu^T) of bf16 A and W in one launch: Wg the first n rows of W, Wu the n rows that
  * begin up_rows below (per batch, stride_w elements apart); clamped != 0: g sigmoid(alpha g) (u + shift) with
  * g = min(., limit), u = clamp(., -limit, limit) (limit <= 0: no clamps). a_rows / z_start as lgs_linear's (M: the rows
- * of all groups). lgs_linear_glu_fits: whether a size is served (n % 4 == 0, K % 64 == 0, M > 8). */
-int lgs_linear_glu_fits(int M, int n, int K, int grouped);
+ * of all groups). n % 4 == 0, n >= 32, K % 64 == 0, M > 8. lgs_linear_glu_fits: whether that is the best way to make it
+ * (groups 0: one plain product). */
+int lgs_linear_glu_fits(int M, int n, int K, int groups);
 int lgs_linear_glu(const void* a, long lda, const void* w, long stride_w, long up_rows, void* y, long ldy, int M, int n,
                    int K, int batch, const int* a_rows, const int* z_start, int act, int clamped, float alpha, float limit,
                    float shift, lgs_stream_t stream);

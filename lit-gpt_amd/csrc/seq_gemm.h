@@ -30,6 +30,13 @@ using lga::GemmPlan;
 GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit);
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream);
 
+// A grouped product whose list is one tile of lgs_linear's older kernel and whose groups have two rows or less: that kernel
+// finds a group's rows by its place in the grid, where every workgroup here looks the list's groups through and most have
+// nothing to do. us there / here of top-4 routed tokens, up and down products: 64 experts of 512 x 2048, 13 tokens 45 + 30 / 60
+// + 34, 32 tokens 50 + 34 / 71 + 37, 33 tokens 92 + 57 / 68 + 36; 128 of 256 x 1024, 13 tokens 27 + 11 / 36 + 25; 40 of 1024 x
+// 4096, 13 tokens 124 + 51 / 136 + 67, 26 tokens 222 + 93 / 155 + 72; 24 of 512 x 2048, 13 tokens 41 + 19 / 32 + 16
+inline bool gemm_few_rows(int M, int groups) { return M <= 128 && M <= 2 * groups; }
+
 // the gated unit on two products: act(gate) * up, or clamped: g sigmoid(alpha g) (u + shift) with g = min(gate, limit),
 // u = clamp(up, -limit, limit) (limit <= 0: no clamps)
 struct GluForm {

@@ -241,6 +241,7 @@ int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t s
 }
 
 GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit) {
+  if (grouped && gemm_few_rows(M, batch)) return GemmPlan{-1, 1};
   return lga::gemm_tile_plan(M, N, K, batch, grouped, ksplit);
 }
 

@@ -632,20 +632,18 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
   LGA_LAUNCH_RETURN();
 }
 
-// whether lgs_linear_glu takes a product of M rows (the sizes of all its groups) on gate | up of n columns each: not where
-// the plain product is better made in ranges of K
-extern "C" int lgs_linear_glu_fits(int M, int n, int K, int grouped) {
-  return M > 8 && n >= 32 && n % 4 == 0 && n <= (1 << 29) && K > 0 && K % 64 == 0 &&
-                 (grouped || lgs::gemm_plan(M, 2 * n, K, 1, false, 0).ksplit == 1)
-             ? 1
-             : 0;
+static bool glu_served(int M, int n, int K) { return M > 8 && n >= 32 && n % 4 == 0 && n <= (1 << 29) && K > 0 && K % 64 == 0; }
+// whether a product of M rows (the sizes of all its groups; groups 0: one plain product) on gate | up of n columns each is best
+// made by lgs_linear_glu: not where the plain product is better made in ranges of K, or on the tiles for few rows of many groups
+extern "C" int lgs_linear_glu_fits(int M, int n, int K, int groups) {
+  return glu_served(M, n, K) && (groups > 0 ? !lgs::gemm_few_rows(M, groups) : lgs::gemm_plan(M, 2 * n, K, 1, false, 0).ksplit == 1) ? 1 : 0;
 }
 
 extern "C" int lgs_linear_glu(const void* a, long lda, const void* w, long stride_w, long up_rows, void* y, long ldy, int M,
                               int n, int K, int batch, const int* a_rows, const int* z_start, int act, int clamped,
                               float alpha, float limit, float shift, hipStream_t stream) {
   LGA_CHECK_ARG(a && w && y, "lgs_linear_glu: null pointer");
-  LGA_CHECK_ARG(lgs_linear_glu_fits(M, n, K, z_start != nullptr), "lgs_linear_glu: not one of its sizes");
+  LGA_CHECK_ARG(glu_served(M, n, K), "lgs_linear_glu: not one of its sizes");
   LGA_CHECK_ARG(batch > 0 && batch <= 65535 && (batch == 1 || z_start), "lgs_linear_glu: batches are groups of rows");
   LGA_CHECK_ARG(lda >= K && ldy >= n && up_rows >= n, "lgs_linear_glu: row strides shorter than the rows");
   LGA_CHECK_ARG(act >= 0 && act <= lgs::kActSigmoid, "lgs_linear_glu: unknown activation");

@@ -394,10 +394,11 @@ def expanded_latent_attention(q: torch.Tensor, q_off: int, kv: torch.Tensor, cac
 
 
 def glu_fits(a: Optional[torch.Tensor], w: torch.Tensor, M: int, n: int, grouped: bool = False) -> bool:
-    """Whether ``linear_glu`` makes a gated unit of n columns for M rows of ``a`` (rows of w.shape[-1] values)."""
+    """Whether ``linear_glu`` is to make a gated unit of n columns for M rows of ``a`` (rows of w.shape[-1] values; ``grouped``:
+    the rows of w.shape[0] groups)."""
     K = w.shape[-1]
     return a is not None and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and \
-        bool(load_library().lgs_linear_glu_fits(M, n, K, int(grouped))) and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+        bool(load_library().lgs_linear_glu_fits(M, n, K, w.shape[0] if grouped else 0)) and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 
 
 def linear_glu(a: torch.Tensor, w: torch.Tensor, *, M: int, n: int, up: int, act: int = 0,

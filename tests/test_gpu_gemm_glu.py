@@ -58,3 +58,26 @@ def test_sizes():
     w = torch.zeros(128, 192, dtype=torch.bfloat16, device=DEV)
     assert seq_ops.glu_fits(h, w, 64, 64) and not seq_ops.glu_fits(h, w, 8, 64) and not seq_ops.glu_fits(h, w, 64, 62)
     assert not seq_ops.glu_fits(h.float(), w, 64, 64) and not seq_ops.glu_fits(h[:, :96], w[:, :96], 64, 64)
+
+
+@pytest.mark.parametrize("E,pairs,fits", [(64, 52, False), (64, 128, False), (64, 129, True), (26, 52, False), (25, 52, True),
+                                          (16, 52, True), (256, 128, False)])
+def test_few_rows_of_many_groups(E, pairs, fits):
+    """The sizes that stay with the tiles made for a group's place in the grid, to the bits of the other form."""
+    from lit_gpt import seq_ops
+
+    F, K = 64, 128
+    g = torch.Generator(device=DEV).manual_seed(E + pairs)
+    sizes = torch.bincount(torch.randint(0, E, (pairs,), generator=torch.Generator().manual_seed(pairs)), minlength=E)
+    z = torch.cat([torch.zeros(1, dtype=torch.long), sizes.cumsum(0)]).to(torch.int32).to(DEV)
+    rows = torch.randint(0, 40, (pairs,), generator=g, device=DEV).to(torch.int32)
+    h = torch.randn(40, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randn(E, 2 * F, K, generator=g, device=DEV).to(torch.bfloat16)
+    assert seq_ops.glu_fits(h, w, pairs, F, grouped=True) == fits
+    gu = torch.empty(pairs, 2 * F, device=DEV)
+    seq_ops.linear(h, w, M=pairs, N=2 * F, K=K, y=gu, lda=K, ldy=2 * F, batch=E, stride_w=2 * F * K, a_rows=rows, z_start=z)
+    of = torch.repeat_interleave(torch.arange(E, device=DEV), sizes.to(DEV))
+    want = (h[rows.long()].double()[:, None] @ w[of].double().transpose(1, 2).contiguous())[:, 0]
+    assert float((gu.double() - want).abs().max()) < 2 ** -20 * float(want.abs().max()) * 8
+    made = seq_ops.linear_glu(h, w, M=pairs, n=F, up=F, act=seq_ops.ACT_SILU, a_rows=rows, z_start=z)
+    assert torch.equal(made, seq_ops.glu(gu, 0, F, F, seq_ops.ACT_SILU, bf16=True))
