@@ -253,13 +253,15 @@ static int go_rows(const KArgs& k, int mf, hipStream_t stream) {
 //   up to 96 rows   all (int4 64 x 4096 x 4096: 19 / 23)
 //   up to 128 rows  beyond 2^24 (int4 4096 x 4096: 31 / 26; 12288 x 4096: 37 / 42); SwiGLU from 2^26 (int4 11008 x 4096:
 //                   68 / 64, 28672 x 8192: 159 / 268)
-//   up to 256 rows  one matrix up to 2^27 (nf4 200 x 8192 x 8192: 56 / 71; 8192 x 28672: 156 / 160, int4 142 / 148 at
-//                   160); the 256-row tiles read larger weights once
+//   up to 256 rows  one matrix up to 2^27 of at most 16384 columns (nf4 200 x 8192 x 8192: 56 / 71; 16384 x 4096: 56 / 70,
+//                   16384 x 8192: 95 / 101; 20480 x 4096: 83 / 70, 28672 x 4096: 84 / 74, 50000 x 2048: 90 / 73; 8192 x
+//                   28672: 156 / 160, int4 142 / 148 at 160): the 256-row tiles read larger weights once, and more
+//                   columns give them more than half a round of the chip without ranges of K
 Q4dPlan q4d_plan(int M, int N, int K, bool dual) {
   Q4dPlan p{0, 0, 0, 0, 0};
   const size_t nk = (size_t)N * K, one = 1;
   if (K % pd::BK != 0 || M > 256) return p;
-  if (M > 128 ? dual || nk > one << 27 : M > 96 ? nk <= one << (dual ? 26 : 24) : M <= 32 && nk <= one << 24) return p;
+  if (M > 128 ? dual || N > 16384 || nk > one << 27 : M > 96 ? nk <= one << (dual ? 26 : 24) : M <= 32 && nk <= one << 24) return p;
   p.mf = M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : (M <= 96 ? 6 : 8)));
   p.mt = (M + p.mf * 16 - 1) / (p.mf * 16);
   const int cols = 128 * (dual ? 1 : 2), nb = K / pd::BK;

@@ -18,7 +18,8 @@ def plan(M, N, K, swiglu=0, fmt=1):
     (2, SMALL, 0, TILES), (32, SMALL, 0, TILES), (32, LARGE, 0, REGISTERS), (33, SMALL, 0, REGISTERS),
     (96, SMALL, 0, REGISTERS), (96, SMALL, 1, REGISTERS), (97, SMALL, 0, TILES), (97, LARGE, 0, REGISTERS),
     (97, LARGE, 1, TILES), (97, HUGE, 1, REGISTERS), (128, LARGE, 0, REGISTERS), (128, HUGE, 1, REGISTERS),
-    (129, HUGE, 1, TILES), (129, HUGE, 0, TILES), (129, LARGE, 0, REGISTERS), (129, SMALL, 0, REGISTERS), (256, SMALL, 0, REGISTERS),
+    (129, HUGE, 1, TILES), (129, HUGE, 0, TILES), (129, (16384, 8192), 0, REGISTERS), (256, (16384, 4096), 0, REGISTERS),
+    (129, (16392, 4096), 0, TILES), (256, (28672, 4096), 0, TILES), (128, (28672, 4096), 0, REGISTERS), (129, LARGE, 0, REGISTERS), (129, SMALL, 0, REGISTERS), (256, SMALL, 0, REGISTERS),
     (257, SMALL, 0, TILES), (64, (4096, 4160), 0, TILES), (64, (4096, 192), 0, TILES), (64, (4096, 128), 0, REGISTERS)])
 def test_four_bit_weights(fmt, M, size, swiglu, form):
     assert plan(M, *size, swiglu, fmt)[0] == form
