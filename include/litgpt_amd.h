@@ -78,10 +78,10 @@ int lga_q4f_fits(int M, int N, int K, int group, int fmt);
  * bytes (0 = none needed; the largest of all formats') and keeps it for later calls (its per-tile counters are left
  * zeroed). */
 size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu);
-/* How a product of one format is made: 0 the LDS-image tiles, 1 4-bit weights dequantized in registers, 2 the bf16 weights'
- * pipelined tiles. workspace_bytes: what this form needs; counters: 1 where its first 4096 bytes are counters that have to
- * be zero (else the workspace need not be cleared nor kept). Either may be NULL. */
-int lga_q4f_plan(int M, int N, int K, int swiglu, int fmt, size_t* workspace_bytes, int* counters);
+/* How a product of one format is made, in one number: bits 0..1 the form (0 the LDS-image tiles, 1 4-bit weights dequantized in
+ * registers, 2 the bf16 weights' pipelined tiles), bit 2 set where the first 4096 bytes of its workspace are counters that have
+ * to be zero (else it need be neither cleared nor kept), the bits above the workspace's bytes. */
+size_t lga_q4f_plan(int M, int N, int K, int swiglu, int fmt);
 int lga_q4_gemm_fused(const void* x, const void* weight, const void* scales, const void* bias, const void* residual,
                       void* y, int M, int N, int K, int group, int fmt, void* workspace, size_t workspace_bytes,
                       lga_stream_t stream);

@@ -862,12 +862,10 @@ extern "C" int lga_q4f_trace_read(unsigned long long* host, int n) {
 
 extern "C" int lga_q4f_fits(int M, int N, int K, int group, int fmt) { return q4f_fits(M, N, K, group, fmt) ? 1 : 0; }
 
-extern "C" int lga_q4f_plan(int M, int N, int K, int swiglu, int fmt, size_t* workspace_bytes, int* counters) {
-  const bool ok = M >= 1 && N >= 1 && K >= lga::pf::BK && fmt >= 0 && fmt <= 3;
-  const Route r = ok ? route(M, N, K, fmt, swiglu != 0) : Route();
-  if (workspace_bytes) *workspace_bytes = r.need;
-  if (counters) *counters = r.form == kTiles && r.need > 0;
-  return r.form;
+extern "C" size_t lga_q4f_plan(int M, int N, int K, int swiglu, int fmt) {
+  if (M < 1 || N < 1 || K < lga::pf::BK || fmt < 0 || fmt > 3) return kTiles;
+  const Route r = route(M, N, K, fmt, swiglu != 0);
+  return r.need * 8 + (r.form == kTiles && r.need > 0 ? 4 : 0) + r.form;
 }
 
 extern "C" size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu) {

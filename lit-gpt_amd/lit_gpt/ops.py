@@ -48,7 +48,7 @@ SIGNATURES = {
     "lga_q4_gemm": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "lga_q4f_fits": [_I, _I, _I, _I, _I],
     "lga_q4f_workspace_bytes": [_I, _I, _I, _I],
-    "lga_q4f_plan": [_I, _I, _I, _I, _I, ctypes.POINTER(_SZ), ctypes.POINTER(_I)],
+    "lga_q4f_plan": [_I, _I, _I, _I, _I],
     "lga_q4_gemm_fused": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P],
     "lga_q4_gemm_swiglu": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P],
     "lga_q4_dequantize": [_P, _P, _P, _I, _I, _I, _I, _P],
@@ -109,7 +109,7 @@ SIGNATURES = {
     "lga_q4_gemv_allreduce_tagged": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, ctypes.POINTER(_P), _I, _I, _I, _P, _P,
                                      _P, _P],
 }
-_RESTYPES = {"lga_q4_gemv_experts_pair_counters": ctypes.c_size_t, "lga_q4f_workspace_bytes": ctypes.c_size_t, "lga_last_error_string": ctypes.c_char_p, "lga_attention_workspace_bytes": ctypes.c_size_t,
+_RESTYPES = {"lga_q4_gemv_experts_pair_counters": ctypes.c_size_t, "lga_q4f_workspace_bytes": ctypes.c_size_t, "lga_q4f_plan": ctypes.c_size_t, "lga_last_error_string": ctypes.c_char_p, "lga_attention_workspace_bytes": ctypes.c_size_t,
              "lga_comm_mailbox_bytes": ctypes.c_size_t, "lga_q4_gemv_argmax_work_bytes": ctypes.c_size_t}
 
 _lib: Optional[ctypes.CDLL] = None
@@ -236,10 +236,8 @@ _Q4F_WS_LOCK = threading.Lock()
 
 def q4f_plan(M, N, K, swiglu, fmt):
     """How a fused product of this format is made (lga_q4f_plan): (form, workspace bytes, whether it holds counters)."""
-    need, counters = _SZ(0), _I(0)
-    form = load_library().lga_q4f_plan(int(M), int(N), int(K), int(bool(swiglu)), int(fmt), ctypes.byref(need),
-                                       ctypes.byref(counters))
-    return form, need.value, bool(counters.value)
+    plan = load_library().lga_q4f_plan(M, N, K, swiglu, fmt)
+    return plan & 3, plan >> 3, bool(plan & 4)
 
 
 def _q4f_workspace(M, N, K, swiglu, fmt, device):
