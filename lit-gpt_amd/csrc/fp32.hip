@@ -119,7 +119,8 @@ __global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restr
 
 static void f32_layernorm_go(const float* x, const float* w, const float* b, float* y, const float* w2, const float* b2,
                              float* y2, int rows, int n, float eps, float eps2, hipStream_t stream) {
-  if (n <= 1024) f32_layernorm_kernel<4><<<rows, 256, 0, stream>>>(x, w, b, y, n, eps, w2, b2, y2, eps2);
+  if (n <= 256) f32_layernorm_kernel<1><<<rows, 256, 0, stream>>>(x, w, b, y, n, eps, w2, b2, y2, eps2);
+  else if (n <= 1024) f32_layernorm_kernel<4><<<rows, 256, 0, stream>>>(x, w, b, y, n, eps, w2, b2, y2, eps2);
   else f32_layernorm_kernel<16><<<rows, 256, 0, stream>>>(x, w, b, y, n, eps, w2, b2, y2, eps2);
 }
 

@@ -455,20 +455,22 @@ __global__ void __launch_bounds__(256) embed_pos_kernel(const int* __restrict__ 
 // Layer norm of a sublayer's output joining the residual: x[r] (+)= mult * ((y - mean) / sqrt(var + eps) * w + b),
 // var = mean of the squared deviations (two passes over the row, which stays in registers up to 256 * CPT columns).
 // x16: optional copy of the new x rounded to bf16 (the next product's operand). grid (rows). Bound by latency for few rows:
-// 8 rows of 2048 take 4.7 us (8.0 with weights, bias and residual loaded after the sums).
-template <int CPT>
+// 8 rows of 2048 take 4.7 us (8.0 with weights, bias and residual loaded after the sums). AHEAD: those are on their way
+// before the sums; not for rows of which the registers hold less than half (3000 rows of 11008: 95 us, 80 without).
+template <int CPT, bool AHEAD>
 __global__ void __launch_bounds__(256) layernorm_kernel(const float* __restrict__ y, const float* __restrict__ w,
                                                         const float* __restrict__ b, float eps, float mult, int accumulate,
                                                         float* __restrict__ x, uint16_t* __restrict__ x16, int n) {
   __shared__ float red[4];
   const size_t r = blockIdx.x;
   const float* yr = y + r * n;
-  float v[CPT], wv[CPT], bv[CPT], xv[CPT];  // (everything is on its way before the first sum is needed)
+  float v[CPT], wv[CPT], bv[CPT], xv[CPT];
   float s = 0.0f;
 #pragma unroll
   for (int e = 0; e < CPT; ++e) {
     const int i = min((int)threadIdx.x + 256 * e, n - 1);
     v[e] = yr[i];
+    if (!AHEAD) continue;
     wv[e] = w[i];
     bv[e] = b ? b[i] : 0.0f;
     xv[e] = accumulate ? x[r * n + i] : 0.0f;
@@ -499,8 +501,12 @@ __global__ void __launch_bounds__(256) layernorm_kernel(const float* __restrict_
     if (x16) x16[r * n + i] = f2bf(o);
   };
 #pragma unroll
-  for (int e = 0; e < CPT; ++e)
-    if (threadIdx.x + 256 * e < n) put(threadIdx.x + 256 * e, v[e], wv[e], bv[e], xv[e]);
+  for (int e = 0; e < CPT; ++e) {
+    const int i = threadIdx.x + 256 * e;
+    if (i >= n) continue;
+    if (AHEAD) put(i, v[e], wv[e], bv[e], xv[e]);
+    else put(i, v[e], w[i], b ? b[i] : 0.0f, accumulate ? x[r * n + i] : 0.0f);
+  }
   for (int i = threadIdx.x + 256 * CPT; i < n; i += 256)
     put(i, yr[i], w[i], b ? b[i] : 0.0f, accumulate ? x[r * n + i] : 0.0f);
 }
@@ -688,12 +694,14 @@ extern "C" int lgs_embed_pos(const int* tokens, const int* pos, const void* tabl
 extern "C" int lgs_layernorm(const float* y, const float* weight, const float* bias, float eps, float mult,
                              int accumulate, float* x, void* x_bf16, int rows, int n, hipStream_t stream) {
   LGA_CHECK_ARG(y && weight && x && rows > 0 && n > 0, "lgs_layernorm: bad arguments");
-  if (n <= 1024)
-    lgs::layernorm_kernel<4><<<rows, 256, 0, stream>>>(y, weight, bias, eps, mult, accumulate, x, (uint16_t*)x_bf16, n);
-  else if (n <= 2048)
-    lgs::layernorm_kernel<8><<<rows, 256, 0, stream>>>(y, weight, bias, eps, mult, accumulate, x, (uint16_t*)x_bf16, n);
-  else
-    lgs::layernorm_kernel<16><<<rows, 256, 0, stream>>>(y, weight, bias, eps, mult, accumulate, x, (uint16_t*)x_bf16, n);
+#define LGS_NORM(CPT, AHEAD) \
+  lgs::layernorm_kernel<CPT, AHEAD><<<rows, 256, 0, stream>>>(y, weight, bias, eps, mult, accumulate, x, (uint16_t*)x_bf16, n)
+  if (n <= 256) LGS_NORM(1, true);
+  else if (n <= 1024) LGS_NORM(4, true);
+  else if (n <= 2048) LGS_NORM(8, true);
+  else if (n <= 8192) LGS_NORM(16, true);
+  else LGS_NORM(16, false);
+#undef LGS_NORM
   LGA_LAUNCH_RETURN();
 }
 
