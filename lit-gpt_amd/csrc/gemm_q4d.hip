@@ -261,7 +261,9 @@ Q4dPlan q4d_plan(int M, int N, int K, bool dual) {
   Q4dPlan p{0, 0, 0, 0, 0};
   const size_t nk = (size_t)N * K, one = 1;
   if (K % pd::BK != 0 || M > 256) return p;
-  if (M > 128 ? dual || N > 16384 || nk > one << 27 : M > 96 ? nk <= one << (dual ? 26 : 24) : M <= 32 && nk <= one << 24) return p;
+  if (M > 128 && (dual || N > 16384 || nk > one << 27)) return p;
+  if (M > 96 && M <= 128 && nk <= one << (dual ? 26 : 24)) return p;
+  if (M <= 32 && nk <= one << 24) return p;
   p.mf = M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : (M <= 96 ? 6 : 8)));
   p.mt = (M + p.mf * 16 - 1) / (p.mf * 16);
   const int cols = 128 * (dual ? 1 : 2), nb = K / pd::BK;

@@ -89,7 +89,8 @@ __device__ __forceinline__ float tanh_near(float x) {
   return y < 0.625f ? p : copysignf(q, x);
 }
 
-// 1 / (1 + e^-z) from e^-|z| (3.8e-8 rms for z >= 0, 5.5e-8 below; sigmoid_f 3.8e-8), which is 0 from 120 on (an infinite z has no residual in exp_neg; a NaN stays one)
+// 1 / (1 + e^-z) from e^-|z| (3.8e-8 rms for z >= 0, 5.5e-8 below; sigmoid_f 3.8e-8), which is 0 from 120 on (an infinite z has
+// no residual in exp_neg; a NaN stays one)
 __device__ __forceinline__ float sigmoid_near(float z) {
   const float e = exp_neg(fabsf(z) > 120.0f ? -120.0f : -fabsf(z)), d = 1.0f + e;
   const float r = __builtin_amdgcn_rcpf(d), p = fmaf(fmaf(-d, r, 1.0f), r, r);
@@ -471,8 +472,9 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
   if (odd) {
     for (uint32_t rows = (uint32_t)odd | (uint32_t)(odd >> 32); rows; rows &= rows - 1) {
       const int i = __ffs(rows) - 1;
-      attn_row_plain<DC, DT, MAPS, PARTS, SIG>(p, kbase, vbase, a.q + (size_t)(rfirst + qw * 32 + i) * a.ld + (size_t)h * MAPS * DC * 16,
-                                               h, lowest(wfirst + i), min(wfirst + i, a.S - 1), lane, turn + i * (DV + 4));
+      const float* q_at = a.q + (size_t)(rfirst + qw * 32 + i) * a.ld + (size_t)h * MAPS * DC * 16;
+      attn_row_plain<DC, DT, MAPS, PARTS, SIG>(p, kbase, vbase, q_at, h, lowest(wfirst + i), min(wfirst + i, a.S - 1), lane,
+                                               turn + i * (DV + 4));
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }

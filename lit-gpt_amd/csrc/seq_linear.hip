@@ -638,11 +638,14 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
   LGA_LAUNCH_RETURN();
 }
 
-static bool glu_served(int M, int n, int K) { return M > 8 && n >= 32 && n % 4 == 0 && n <= (1 << 29) && K > 0 && K % 64 == 0; }
+static bool glu_served(int M, int n, int K) {
+  return M > 8 && n >= 32 && n % 4 == 0 && n <= (1 << 29) && K > 0 && K % 64 == 0;
+}
 // whether a product of M rows (the sizes of all its groups; groups 0: one plain product) on gate | up of n columns each is best
 // made by lgs_linear_glu: not where the plain product is better made in ranges of K, or on the tiles for few rows of many groups
 extern "C" int lgs_linear_glu_fits(int M, int n, int K, int groups) {
-  return glu_served(M, n, K) && (groups > 0 ? !lgs::gemm_few_rows(M, groups) : lgs::gemm_plan(M, 2 * n, K, 1, false, 0).ksplit == 1) ? 1 : 0;
+  if (!glu_served(M, n, K)) return 0;
+  return (groups > 0 ? !lgs::gemm_few_rows(M, groups) : lgs::gemm_plan(M, 2 * n, K, 1, false, 0).ksplit == 1) ? 1 : 0;
 }
 
 extern "C" int lgs_linear_glu(const void* a, long lda, const void* w, long stride_w, long up_rows, void* y, long ldy, int M,

@@ -398,7 +398,8 @@ def glu_fits(a: Optional[torch.Tensor], w: torch.Tensor, M: int, n: int, grouped
     the rows of w.shape[0] groups)."""
     K = w.shape[-1]
     return a is not None and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and \
-        bool(load_library().lgs_linear_glu_fits(M, n, K, w.shape[0] if grouped else 0)) and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+        a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and \
+        bool(load_library().lgs_linear_glu_fits(M, n, K, w.shape[0] if grouped else 0))
 
 
 def linear_glu(a: torch.Tensor, w: torch.Tensor, *, M: int, n: int, up: int, act: int = 0,

@@ -1,7 +1,7 @@
 """One-token attention over bf16 caches with 128-value rows (attn_one_kernel) against the general form (one split) and
 float64: sequences of one key to several hundred, shares that end inside a group of keys or hold none, one or two query
-heads a workgroup (two from 1024 pairs of sequence and head on), masks, caps, sinks and gates. Tolerance: fp32 sums of weights that add up to one, on values of unit
-variance: 2^-17."""
+heads a workgroup (two from 1024 pairs of sequence and head on), masks, caps, sinks and gates. Tolerance: fp32 sums of weights
+that add up to one, on values of unit variance: 2^-17."""
 
 import pytest
 import torch
