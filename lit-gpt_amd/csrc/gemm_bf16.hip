@@ -3,9 +3,9 @@
 // stores as 8 bytes, and for SwiGLU a wave's fragments alternate between the two matrices, so that the pair of a column
 // meets in one lane.
 //
-// Bound by the matrix cores' feeding, as the tiles are. Against gemm_q4f.hip's tiles of bf16 weights:
-// of 517 rows (N x K) 12288 x 4096 104 -> 65 us, 4096 x 4096 69 -> 37, 4096 x 11008 118 -> 68, 11008 x 4096 with SwiGLU
-// 183 -> 128; of 100 rows 8192 x 28672 141 -> 103, 28672 x 8192 with SwiGLU 270 -> 185.
+// Bound as the tiles are; with few rows by the weights on their way from memory. With weights from memory, us on stages of 32
+// values / here: of 517 rows (N x K) 12288 x 4096 70 / 65, 4096 x 4096 36 / 35, 4096 x 11008 68 / 71, 11008 x 4096 with
+// SwiGLU 131 / 119; of 2048 rows 12288 x 4096 195 / 178, 4096 x 11008 181 / 162, 6144 x 4096 with SwiGLU 209 / 192.
 #include "gemm_q4d.h"
 #include "gemm_tiles.h"
 
@@ -16,42 +16,41 @@ struct BfArgs {
   int nt, mt, splits, kper;  // tiles over columns and rows; ranges of K of kper stages of 64 values
 };
 
-template <int WM, int WN, int FM, int FN, int BK, int ST, bool DUAL>
+template <int WM, int WN, int FM, int FN, int RA, int RB, bool DUAL>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
-  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
-  constexpr int P = T::P, BN = DUAL ? T::BM / 2 : T::BM;  // columns of Y per tile
-  static_assert(FM % 2 == 0, "fragments of the two matrices in pairs");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[ST * T::STAGE];
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
+  constexpr int BN = DUAL ? T::BM / 2 : T::BM;  // columns of Y per tile
+  static_assert(!DUAL || FM % 2 == 0, "fragments of the two matrices in pairs");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
   const Q4dArgs& a = k.a;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // an XCD takes neighbouring tiles: the rows' tiles of up to eight columns' tiles, range after range
+  // an XCD takes neighbouring tiles: of a column's weights those of up to eight row tiles, range after range (all of a
+  // column's on one XCD: 517 x 12288 x 4096 with weights from memory 70 -> 62 us)
   int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const int per = k.nt * k.mt, split = t / per;
   if (split >= k.splits) return;
   t -= split * per;
-  const int g = t / (8 * k.mt), gn = min(8, k.nt - g * 8);
-  t -= g * 8 * k.mt;
-  const int n0 = (g * 8 + t % gn) * BN, m0 = t / gn * T::BN;
-  const int k0 = split * k.kper * T::RPL, nk = min(a.K / BK - k0, k.kper * T::RPL);
-  const unsigned char* src[P];
+  const int g = t / (8 * k.nt), gm = min(8, k.mt - g * 8);
+  t -= g * 8 * k.nt;
+  const int m0 = (g * 8 + t % gm) * T::BN, n0 = t / gm * BN;
+  const int k0 = split * k.kper, nk = min(a.K / 64 - k0, k.kper);
+  const unsigned char *src_w[T::PA], *src_x[T::PB];
+  int r, c;
 #pragma unroll
-  for (int i = 0; i < P; ++i) {
-    const int piece = wave * P + i;
-    const bool of_w = piece < T::BM / T::ROWS;  // (wave-uniform)
-    int r, c;
-    gemm_dma_at<BK>((of_w ? piece : piece - T::BM / T::ROWS) * 8 + (lane >> 3), lane, &r, &c);
-    if (of_w) {  // columns past the end repeat the last one (never stored)
-      const int n = DUAL ? r / 64 * 32 + r % 32 : r;
-      const void* w = DUAL && r / 32 % 2 ? a.w2 : a.w;
-      src[i] = (const unsigned char*)((const uint16_t*)w + (size_t)min(n0 + n, a.N - 1) * a.K);
-    } else {
-      src[i] = (const unsigned char*)(a.x + (size_t)min(m0 + r, a.M - 1) * a.K);
-    }
-    src[i] += (size_t)k0 * (BK * 2) + c * 16;
+  for (int i = 0; i < T::PA; ++i) {  // columns past the end repeat the last one (never stored)
+    gemm_dma_at(wave * T::PA + i, lane, &r, &c);
+    const int n = DUAL ? r / 64 * 32 + r % 32 : r;
+    const void* w = DUAL && r / 32 % 2 ? a.w2 : a.w;
+    src_w[i] = (const unsigned char*)((const uint16_t*)w + (size_t)min(n0 + n, a.N - 1) * a.K) + (size_t)k0 * 128 + c * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < T::PB; ++i) {
+    gemm_dma_at(wave * T::PB + i, lane, &r, &c);
+    src_x[i] = (const unsigned char*)(a.x + (size_t)min(m0 + r, a.M - 1) * a.K) + (size_t)k0 * 128 + c * 16;
   }
   f32x16_t acc[FM][FN];
-  gemm_tile<WM, WN, FM, FN, BK, ST>(lds, src, nk, wave, lane, acc);
+  gemm_tile<WM, WN, FM, FN, RA, RB>(lds, src_w, src_x, nk, wave, lane, acc);
   const int wm = wave % WM, wn = wave / WM, l31 = lane & 31, hi = lane >> 5;
   const size_t ldy = a.ldy ? a.ldy : a.N;
 #pragma unroll
@@ -80,25 +79,25 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
   }
 }
 
-template <int WM, int WN, int FM, int FN, int BK, int ST>
+template <int WM, int WN, int FM, int FN, int RA, int RB>
 static void bf16_go(BfArgs k, bool dual, hipStream_t stream) {
-  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   const int bn = dual ? T::BM / 2 : T::BM;
   k.nt = (k.a.N + bn - 1) / bn, k.mt = (k.a.M + T::BN - 1) / T::BN;
   const unsigned grid = (unsigned)(((long)k.nt * k.mt * k.splits + 7) / 8 * 8);
-  if (dual) gemm_bf16_kernel<WM, WN, FM, FN, BK, ST, true><<<grid, T::NT, 0, stream>>>(k);
-  else gemm_bf16_kernel<WM, WN, FM, FN, BK, ST, false><<<grid, T::NT, 0, stream>>>(k);
+  if constexpr (FM % 2 == 0) {
+    if (dual) gemm_bf16_kernel<WM, WN, FM, FN, RA, RB, true><<<grid, T::NT, 0, stream>>>(k);
+  }
+  if (!dual) gemm_bf16_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(k);
 }
 
-// All products but two kinds (us here / on gemm_q4f.hip's tiles). Few rows and small weights, where a launch over ranges of
-// K and one that adds them are not repaid: 16 x 4096 x 4096 20 / 14, 16 x 4096 x 11008 26 / 23, against 38 / 39 for 8192 x
-// 8192 (2^26). And prompts beyond 1024 rows that fill the chip with 256 x 128 tiles: 2048 rows of 11008 x 4096 with SwiGLU
-// 362 / 349, 28672 x 8192 1698 / 1637, 3000 rows of 4096 x 4096 123 / 110; at 1000 rows 191 / 205, 931 / 902, 45 / 74.
+// All products but those of few rows and small weights, where a launch over ranges of K and one that adds them are not
+// repaid (us here / on gemm_q4f.hip's tiles): 16 x 4096 x 4096 20 / 14, 16 x 4096 x 11008 26 / 23, against 38 / 39 for 8192 x
+// 8192 (2^26).
 GemmPlan bf16_plan(int M, int N, int K, bool dual) {
   const long cols = dual ? 2L * N : N;
   if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1};
-  if (M > 1024 && (M + 255) / 256 * (cols / 128) >= 256) return GemmPlan{-1, 1};
-  return gemm_tile_plan(M, (int)cols, K, 1, false, 0, true);
+  return gemm_tile_plan(M, (int)cols, K, 1, false, 0, kGemmRowsB | (dual ? kGemmPairs : 0));
 }
 
 size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {
@@ -109,7 +108,7 @@ int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream)
   const int steps = a.K / 64, kper = (steps + p.ksplit - 1) / p.ksplit;
   const BfArgs k{a, 0, 0, (steps + kper - 1) / kper, kper};
   switch (p.tile) {
-#define LGA_CASE(I, SLOTS, US, ...) \
+#define LGA_CASE(I, SLOTS, US, FAST, ROUND, ...) \
   case I: bf16_go<__VA_ARGS__>(k, dual, stream); break;
     LGA_GEMM_FORMS(LGA_CASE)
 #undef LGA_CASE
@@ -118,10 +117,15 @@ int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream)
   LGA_LAUNCH_RETURN();
 }
 
+template <int WM, int WN, int FM, int FN, int RA, int RB>
+static int bf16_preload() {
+  int bad = preload(gemm_bf16_kernel<WM, WN, FM, FN, RA, RB, false>);
+  if constexpr (FM % 2 == 0) bad += preload(gemm_bf16_kernel<WM, WN, FM, FN, RA, RB, true>);
+  return bad;
+}
 int preload_gemm_bf16() {
   int bad = 0;
-#define LGA_PRE(I, SLOTS, US, ...) \
-  bad += preload(gemm_bf16_kernel<__VA_ARGS__, false>) + preload(gemm_bf16_kernel<__VA_ARGS__, true>);
+#define LGA_PRE(I, SLOTS, US, FAST, ROUND, ...) bad += bf16_preload<__VA_ARGS__>();
   LGA_GEMM_FORMS(LGA_PRE)
 #undef LGA_PRE
   return bad;

@@ -2,14 +2,23 @@
 // layered models' products (seq_gemm.hip) and the GPT models' (gemm_bf16.hip) share.
 //
 // A tile of BM x BN outputs belongs to one workgroup of WM x WN waves; a wave holds FM x FN accumulators of
-// v_mfma_f32_32x32x16_bf16. A and B reach LDS by LDS-DMA (global_load_lds, 16 bytes a lane, source-swizzled so that
-// fragments are read without bank conflicts) in ST stages of BK values of K. Per 16 values of K a wave reads FM + FN
-// fragments for FM * FN matrix instructions; the fragments of the next 16 are read while these run, across the stages
-// too: the one barrier of a stage stands before its last 16 values' matrix instructions, whose operands are in
-// registers by then, and the buffer that it frees is refilled between the matrix instructions that follow.
+// v_mfma_f32_32x32x16_bf16. A and B reach LDS by LDS-DMA (global_load_lds, 16 bytes a lane, whole 128-byte lines of a row,
+// source-swizzled so that fragments are read without bank conflicts) in steps of 64 values of K, A's rows into a ring of RA
+// buffers, B's into one of RB: three and two of a 256 x 256 tile fill the 160 KB. Per 16 values of K a wave reads FM + FN
+// fragments for FM * FN matrix instructions; the fragments of the next 16 are read while these run, across the steps
+// too: the one barrier of a step stands before its last 16 values' matrix instructions, whose operands are in registers by
+// then, and the buffers that it frees are refilled between the matrix instructions that follow. Where reads and DMAs stand
+// among the matrix instructions is written out (sched_barrier), not left to the scheduler, which bunches the DMAs.
+//
+// What bounds it: LDS has 128 bytes a clock for the fragments and the DMAs. Four waves of 128 x 128 read 1024 clocks' worth
+// per step of 64 and the DMAs write 512, for 2048 clocks of matrix instructions; eight waves of 128 x 64 would read 1536.
+// Measured 2340 clocks a step, 1.48 us at the 1.6 GHz that a full chip of matrix instructions is left with (power), where
+// stages of 32 values (half lines) in one ring took 3230 clocks, 1.8 us: 2048 x 22016 x 4096 355 -> 296 us, 8192 x 8192 x
+// 8192 950 -> 804. Both give the same bits.
 #pragma once
 
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 
@@ -26,149 +35,138 @@ __device__ __forceinline__ void gemm_wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int WM, int WN, int FM, int FN, int BK, int ST>
+template <int WM, int WN, int FM, int FN, int RA, int RB>
 struct GemmTile {
-  static_assert(BK == 32 || BK == 64, "a row of a stage is half or all of a 128-byte LDS row");
-  static constexpr int BM = WM * FM * 32, BN = WN * FN * 32, NW = WM * WN, NT = NW * 64;
-  static constexpr int RPL = 64 / BK;                     // matrix rows per LDS row
-  static constexpr int STAGE = (BM + BN) / RPL * 128;     // bytes
-  static constexpr int ROWS = 8 * RPL;                    // matrix rows per DMA of a wave (1 KB)
-  static constexpr int P = (BM + BN) / ROWS / NW;         // DMAs per wave and stage
-  static constexpr int H = (P + 1) / 2;                   // ... of these ahead of the next barrier but one
-  static_assert((BM + BN) % (ROWS * NW) == 0 && BM % ROWS == 0 && ST >= 2, "every wave issues the same number of DMAs");
-  static_assert((ST - 1) * P <= 63, "DMAs in flight are counted in six bits");
-  static_assert(ST * STAGE <= 163840, "LDS");
+  static constexpr int FRAGS = FM, BM = WM * FM * 32, BN = WN * FN * 32, NW = WM * WN, NT = NW * 64;
+  static constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, LDS = RA * A_BYTES + RB * B_BYTES;
+  static constexpr int PA = BM / 8 / NW, PB = BN / 8 / NW;  // DMAs (8 rows, 1 KB) per wave and step
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "every wave issues the same number of DMAs");
+  static_assert(RA >= 2 && (RB == RA || RB == RA - 1), "one buffer in use, the others on their way");
+  static_assert((RA - 1) * (PA + PB) <= 63, "DMAs in flight are counted in six bits");
+  static_assert(LDS <= 163840, "LDS");
 };
 
-// acc = the products of nk stages. src[i]: where lane's 16 bytes of DMA i of its wave begin (piece wave * P + i: eight LDS
-// rows, A's first). Accumulator [i][j] of wave (wave % WM, wave / WM): a lane holds row l31 of B's fragment j and rows
-// 8 (e / 4) + 4 hi + e % 4 of A's fragment i.
-template <int WM, int WN, int FM, int FN, int BK, int ST, int P>
-__device__ __forceinline__ void gemm_tile(unsigned char* lds, const unsigned char* const (&src)[P], int nk, int wave,
-                                          int lane, f32x16_t (&acc)[FM][FN]) {
-  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
-  static_assert(P == T::P, "DMAs per wave and stage");
-  constexpr int H = T::H;
-  // Past the last stage the last one is fetched again into a buffer that nobody reads: the count of DMAs in flight is
+// which row and 16-byte chunk of a step's 128 bytes lane `lane` of piece `piece` (8 rows) fetches
+__device__ __forceinline__ void gemm_dma_at(int piece, int lane, int* row, int* chunk) {
+  *row = piece * 8 + (lane >> 3);
+  *chunk = (lane & 7) ^ (*row & 7);
+}
+
+// acc = the products of nk steps. a[i], b[i]: where lane's 16 bytes of DMA i of its wave begin (pieces wave * PA + i of A's
+// rows, wave * PB + i of B's). Accumulator [i][j] of wave (wave % WM, wave / WM): a lane holds row l31 of B's fragment j
+// and rows 8 (e / 4) + 4 hi + e % 4 of A's fragment i.
+template <int WM, int WN, int FM, int FN, int RA, int RB, int PA, int PB>
+__device__ __forceinline__ void gemm_tile(unsigned char* lds, const unsigned char* const (&a)[PA],
+                                          const unsigned char* const (&b)[PB], int nk, int wave, int lane,
+                                          f32x16_t (&acc)[FM][FN]) {
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
+  static_assert(PA == T::PA && PB == T::PB, "DMAs per wave and step");
+  // Past the last step the last one is fetched again into a buffer that nobody reads: the count of DMAs in flight is
   // the same at every barrier, and no branch stands around them.
-  auto stage = [&](int k, int buf, int from, int to) {
-    const size_t at = (size_t)min(k, nk - 1) * (BK * 2);
-#pragma unroll
-    for (int i = 0; i < P; ++i)
-      if (i >= from && i < to) gemm_dma16(src[i] + at, lds + buf * T::STAGE + (wave * P + i) * 1024);
+  auto dma_a = [&](int i, int k, int slot) {
+    gemm_dma16(a[i] + (size_t)min(k, nk - 1) * 128, lds + slot * T::A_BYTES + (wave * PA + i) * 1024);
   };
-  const int wm = wave % WM, wn = wave / WM;
-  const int l31 = lane & 31, hi = lane >> 5;
-  // row l31 of a fragment, chunk hi: its LDS row and swizzled chunk; chunk 2 s + hi lies at that address ^ 32 s
-  const int lrow = l31 / T::RPL;
-  const int sw = lrow * 128 + 16 * (((l31 % T::RPL) * 4 + hi) ^ (lrow & 7));
-  const int abase = wm * FM * 32 / T::RPL * 128 + sw, bbase = (T::BM + wn * FN * 32) / T::RPL * 128 + sw;
+  auto dma_b = [&](int i, int k, int slot) {
+    gemm_dma16(b[i] + (size_t)min(k, nk - 1) * 128, lds + RA * T::A_BYTES + slot * T::B_BYTES + (wave * PB + i) * 1024);
+  };
+  // row l31 of a fragment, chunk hi, swizzled; chunk 2 s + hi lies at that address ^ 32 s
+  const int wm = wave % WM, wn = wave / WM, l31 = lane & 31, hi = lane >> 5;
+  const int sw = l31 * 128 + 16 * (hi ^ (l31 & 7));
+  const int a_at = wm * FM * 4096 + sw, b_at = RA * T::A_BYTES + wn * FN * 4096 + sw;
   struct Frags {
     gemm_bf16x8 a[FM], b[FN];
   };
-  auto read = [&](int buf, int s, Frags& f) {
-    const unsigned char* A = lds + buf * T::STAGE + (abase ^ (32 * s));
-    const unsigned char* B = lds + buf * T::STAGE + (bbase ^ (32 * s));
-#pragma unroll
-    for (int j = 0; j < FN; ++j) f.b[j] = *(const gemm_bf16x8*)(B + j * (4096 / T::RPL));
-#pragma unroll
-    for (int i = 0; i < FM; ++i) f.a[i] = *(const gemm_bf16x8*)(A + i * (4096 / T::RPL));
+  // fragment number n in the order of use: a0, b0, b1, .. , a1, a2, ..
+  auto read = [&](Frags& f, int n, int sa, int sb, int s) {
+    if (n >= 1 && n <= FN) {
+      f.b[n - 1] = *(const gemm_bf16x8*)(lds + sb * T::B_BYTES + (b_at ^ (32 * s)) + (n - 1) * 4096);
+    } else {
+      const int i = n == 0 ? 0 : n - FN;
+      f.a[i] = *(const gemm_bf16x8*)(lds + sa * T::A_BYTES + (a_at ^ (32 * s)) + i * 4096);
+    }
   };
+  // the matrix instructions of 16 values of K, and among them the reads of the next 16 and ND DMAs
+  auto mma = [&](const Frags& f, Frags& g, int sa, int sb, int s, auto nd, auto&& dma) {
+    constexpr int ND = decltype(nd)::value, E = FM * FN, READS = (FM + FN + E - 1) / E;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      acc[e / FN][e % FN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[e / FN], f.b[e % FN], acc[e / FN][e % FN], 0, 0, 0);
+#pragma unroll
+      for (int n = e * READS; n < (e + 1) * READS && n < FM + FN; ++n) read(g, n, sa, sb, s);
+#pragma unroll
+      for (int q = ND * e / E; q < ND * (e + 1) / E; ++q) dma(q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr std::integral_constant<int, PA> all_a{};
+  constexpr std::integral_constant<int, PB> all_b{};
+  constexpr std::integral_constant<int, 0> none{};
+  auto no_dma = [](int) {};
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  auto mma = [&](const Frags& f) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+  for (int s = 0; s < RA - 1; ++s) {
 #pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
-  };
-  // after every matrix instruction two reads of the next fragments, after every second a DMA
-#define LGS_WEAVE(DMAS)                                                \
-  do {                                                                 \
-    int rd_ = 0, dma_ = 0;                                             \
-    _Pragma("unroll") for (int e_ = 0; e_ < FM * FN; ++e_) {           \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);               \
-      _Pragma("unroll") for (int q_ = 0; q_ < 2; ++q_)                 \
-        if (rd_ < FM + FN) {                                           \
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);           \
-          ++rd_;                                                       \
-        }                                                              \
-      if (e_ % 2 == 1 && dma_ < (DMAS)) {                              \
-        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);             \
-        ++dma_;                                                        \
-      }                                                                \
-    }                                                                  \
-  } while (0)
+    for (int i = 0; i < PA; ++i) dma_a(i, s, s);
 #pragma unroll
-  for (int s = 0; s < ST; ++s) stage(s, s, 0, P);
-  gemm_wait_vm<(ST - 1) * P>();
+    for (int i = 0; i < PB; ++i) dma_b(i, s, s);
+  }
+  gemm_wait_vm<(RA - 2) * (PA + PB)>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   Frags f0, f1;
-  read(0, 0, f0);
-  int buf = 0, last = ST - 1;  // the buffers of stages k and k - 1
+#pragma unroll
+  for (int n = 0; n < FM + FN; ++n) read(f0, n, 0, 0, 0);
+  // buffers: sa, sb of this step; free_a, free_b those that the last barrier freed (at first the ones never filled)
+  int sa = 0, sb = 0, free_a = RA - 1, free_b = RB - 1;
   for (int k = 0; k < nk; ++k) {
+    const int na = sa + 1 == RA ? 0 : sa + 1, nb = sb + 1 == RB ? 0 : sb + 1;
     __builtin_amdgcn_sched_barrier(0);
-    read(buf, 1, f1);
-    stage(k - 1 + ST, last, H, P);  // (first pass: the second half of the last stage of the lead once more)
-    mma(f0);
-    LGS_WEAVE(P - H);
-    if constexpr (BK == 64) {
-      __builtin_amdgcn_sched_barrier(0);
-      read(buf, 2, f0);
-      mma(f1);
-      LGS_WEAVE(0);
-      __builtin_amdgcn_sched_barrier(0);
-      read(buf, 3, f1);
-      mma(f0);
-      LGS_WEAVE(0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    const int next = buf + 1 == ST ? 0 : buf + 1;
-    gemm_wait_vm<(ST - 2) * P>();                       // this wave's part of stage k + 1 has landed,
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and it has read all that it reads of stage k
+    mma(f0, f1, sa, sb, 1, all_a, [&](int i) { dma_a(i, k + RA - 1, free_a); });
+    if constexpr (RB == RA) mma(f1, f0, sa, sb, 2, all_b, [&](int i) { dma_b(i, k + RB - 1, free_b); });
+    else mma(f1, f0, sa, sb, 2, none, no_dma);
+    mma(f0, f1, sa, sb, 3, none, no_dma);
+    // this wave's part of step k + 1 has landed (what it issued later may still be on its way), ...
+    gemm_wait_vm<RB == RA ? (RA - 2) * (PA + PB) : (RA - 2) * PA + (RB - 2) * PB>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ... and it has read all that it reads of step k
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    read(next, 0, f0);  // (past the last stage: the repeated one, never used)
-    stage(k + ST, buf, 0, H);
-    mma(f1);
-    LGS_WEAVE(H);
-    last = buf;
-    buf = next;
+    // (past the last step: the repeated one, never used)
+    if constexpr (RB == RA) mma(f1, f0, na, nb, 0, none, no_dma);
+    else mma(f1, f0, na, nb, 0, all_b, [&](int i) { dma_b(i, k + RB, sb); });
+    free_a = sa, free_b = sb;
+    sa = na, sb = nb;
   }
-#undef LGS_WEAVE
   gemm_wait_vm<0>();  // no DMA may outlive the workgroup's LDS
 }
 
-// which row and 16-byte chunk of a stage's BK values lane `lane` of piece row R8 (LDS row) holds
-template <int BK>
-__device__ __forceinline__ void gemm_dma_at(int R, int lane, int* row, int* chunk) {
-  const int lc = (lane & 7) ^ (R & 7);
-  *row = BK == 64 ? R : 2 * R + (lc >> 2);
-  *chunk = BK == 64 ? lc : lc & 3;
-}
-// The tile forms, and what a stage of 64 values of K costs a full chip of their workgroups, measured on products of
-// 2048 x 2048 x 2048 to 2407 x 22016 x 4096: a tile of 256 x 256 runs 1.80 us per 64 values (1190 TFLOP/s, 0.79 of
-// what a large matrix product reaches on this card), of 256 x 128 1.02, of 128 x 128 0.63 alone on a compute unit and
-// 1.14 for two, of 64 x 128 0.43. The larger tile moves fewer bytes per product, the smaller ones fill the chip when
-// rows or columns are few. A workgroup's start and end cost about 3 us.
-// X(index, workgroups of the whole chip at a time, us, waves WM x WN, fragments FM x FN, BK, stages)
-#define LGA_GEMM_FORMS(X)                  \
-  X(0, 256, 1.80f, 2, 4, 4, 2, 32, 5)      \
-  X(1, 256, 1.02f, 4, 2, 2, 2, 64, 3)      \
-  X(2, 512, 1.14f, 2, 2, 2, 2, 64, 2)      \
-  X(3, 256, 0.63f, 2, 4, 2, 1, 64, 4)      \
-  X(4, 256, 0.43f, 1, 4, 2, 1, 64, 4)
+// The tile forms: what a step of 64 values of K costs a full chip of their workgroups, and what it would cost at the 2.4 GHz
+// that a chip with few of them runs at; start, end and fp32 results of a round of them. Measured on 256 tiles (512 of the
+// form of which a compute unit holds two) and K 1024 and 4096. The larger tile moves fewer bytes per product (256 x 256:
+// 1450 TFLOP/s, 256 x 128 1290, 128 x 128 1190, 64 x 128 940), the smaller ones fill the chip when rows or columns are few.
+// X(index, workgroups of the whole chip at a time, us of a step, us of it at 2.4 GHz, us of a round, waves WM x WN,
+//   fragments FM x FN, rings RA, RB)
+#define LGA_GEMM_FORMS(X)                                 \
+  X(0, 256, 1.48f, 0.98f, 15.5f, 2, 2, 4, 4, 3, 2)        \
+  X(1, 256, 1.165f, 0.745f, 10.6f, 2, 2, 4, 3, 3, 2)      \
+  X(2, 256, 0.835f, 0.547f, 8.0f, 2, 2, 4, 2, 3, 3)       \
+  X(3, 256, 0.833f, 0.544f, 7.4f, 2, 2, 2, 4, 3, 3)       \
+  X(4, 256, 0.65f, 0.439f, 5.9f, 2, 2, 2, 3, 4, 4)        \
+  X(5, 512, 0.898f, 0.593f, 7.1f, 2, 2, 2, 2, 2, 2)       \
+  X(6, 256, 0.45f, 0.38f, 5.5f, 2, 4, 2, 1, 5, 5)         \
+  X(7, 256, 0.285f, 0.275f, 4.9f, 1, 4, 2, 1, 6, 6)       \
+  X(8, 256, 1.163f, 0.745f, 10.3f, 2, 2, 3, 4, 3, 2)
 struct GemmForm {
-  int bm, bn, slots;
-  float step_us;
+  int bm, bn, fm, slots;
+  float step_us, fast_us, round_us;
 };
-#define LGA_GEMM_FORM(I, SLOTS, US, ...) {GemmTile<__VA_ARGS__>::BM, GemmTile<__VA_ARGS__>::BN, SLOTS, US},
+#define LGA_GEMM_FORM(I, SLOTS, US, FAST, ROUND, ...) \
+  {GemmTile<__VA_ARGS__>::BM, GemmTile<__VA_ARGS__>::BN, GemmTile<__VA_ARGS__>::FRAGS, SLOTS, US, FAST, ROUND},
 constexpr GemmForm kGemmForms[] = {LGA_GEMM_FORMS(LGA_GEMM_FORM)};
 #undef LGA_GEMM_FORM
 
@@ -176,27 +174,36 @@ constexpr GemmForm kGemmForms[] = {LGA_GEMM_FORMS(LGA_GEMM_FORM)};
 struct GemmPlan {
   int tile, ksplit;
 };
-// Rounds of workgroups times what one takes; several ranges of K cost a second launch that reads them all. E.g.
-// 2048 x 2048 x 5632: 256 tiles of 128 x 128 in one round, 55 us (64 of 256 x 256: 131); 128 x 4096 x 4096: 64 tiles of
-// 64 x 128 in four ranges of K, 16 us (whole: 41); before these tiles 126 and 86 us.
-// rows_b: the rows are the tile's B, the columns its A.
-inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int ksplit, bool rows_b = false) {
+// Rounds of workgroups times what one takes; several ranges of K cost a second launch that reads them all. Against all forms
+// and ranges on 24 products of 64 to 4096 rows, weights from memory, the choice is the fastest or within 7 % of it.
+enum {
+  kGemmRowsB = 1,  // the rows are the tile's B, the columns its A
+  kGemmPairs = 2,  // A's fragments are those of two matrices in turn: forms with an even number of them
+  kGemmActs = 4    // forms whose code holds activations
+};
+inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int flags) {
   GemmPlan best{-1, 1};
   if (K % 64 != 0 || M <= 0) return best;
   const int steps = K / 64;
   float best_us = 0.0f;
   for (int f = 0; f < (int)(sizeof(kGemmForms) / sizeof(kGemmForms[0])); ++f) {
     const GemmForm& t = kGemmForms[f];
-    const int rows = rows_b ? t.bn : t.bm, cols = rows_b ? t.bm : t.bn;
+    if ((flags & kGemmActs && t.bm * t.bn > 256 * 128) || (flags & kGemmPairs && t.fm % 2)) continue;
+    const int rows = flags & kGemmRowsB ? t.bn : t.bm, cols = flags & kGemmRowsB ? t.bm : t.bn;
     const float nt = (float)((N + cols - 1) / cols);
-    // a range of the list ends somewhere in its last tile
-    const float mt = grouped ? (float)M / rows + 0.5f * batch : (float)((M + rows - 1) / rows) * batch;
+    // a range of the list ends somewhere in its last tile, and has one
+    const float mt = grouped ? fmaxf((float)M / rows + 0.5f * batch, (float)min(batch, M)) : (float)((M + rows - 1) / rows) * batch;
     const int s_lo = ksplit > 0 ? ksplit : 1, s_hi = ksplit > 0 ? ksplit : (batch > 1 || grouped ? 1 : 16);
     for (int s = s_lo; s <= s_hi && (s == s_lo || steps / s >= 4); ++s) {
       const int per = (steps + s - 1) / s;
-      const float rounds = ceilf(mt * nt * (float)((steps + per - 1) / per) / (float)t.slots);
-      float us = rounds * (per * t.step_us + 3.0f);
-      if (s > 1) us += 5.0f + (float)M * N * 4.0f * (2 * s + 1) / 3.0e6f;
+      const float rounds = mt * nt * (float)((steps + per - 1) / per) / (float)t.slots, whole = floorf(rounds);
+      float us = (grouped && rounds > 1.0f ? rounds + 0.5f : whole) * (per * t.step_us + t.round_us);
+      if (grouped ? rounds <= 1.0f : rounds > whole) {
+        // few workgroups have a higher clock: 160 of 256 x 256 take 0.74 of 256's time; smaller tiles, which draw less, 0.82
+        const float most = t.bm * t.bn > 128 * 192 ? 0.7f : 0.5f;
+        us += per * fmaxf(t.fast_us, t.step_us * (1.0f - most * (1.0f - (rounds - whole)))) + t.round_us;
+      }
+      if (s > 1) us += 2.0f + (float)M * N * 4.0f * (s + 1) / 5.5e6f;
       if (best.tile < 0 || us < best_us) {
         best_us = us;
         best = GemmPlan{f, s};

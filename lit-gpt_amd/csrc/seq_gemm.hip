@@ -10,50 +10,56 @@ using lga::GemmTile;
 using lga::f32x16_t;
 using lga::gemm_tile;
 
-// grouped rows: the batch whose tiles hold number t, the batches' tiles counted side by side over the lanes; t becomes the
-// number inside the batch
+// grouped rows: this workgroup's tile, z its batch and t its number inside the batch (false: none is left). The batches'
+// tiles are counted side by side over the lanes, and every XCD takes an eighth of those that there are: the grid is the
+// largest number that the groups' sizes allow, of which a third stayed empty and with it the last XCDs (16 groups of 512
+// rows of 2 x 1408 x 2048: 3 rounds on 5 XCDs instead of 2 on all, 216 -> 125 us).
 template <int ROWS>
 __device__ __forceinline__ bool gemm_group(const int* z_start, int batch, int nt, int lane, int* t_at, int* z_at) {
-  int t = *t_at, z = 0;
-  bool found = false;
-  for (int e0 = 0; e0 < batch && !found; e0 += 64) {
+  auto count = [&](int e0, int* own) {  // tiles of lane's batch and of all up to it
     const int e = e0 + lane;
     const int rows = e < batch ? z_start[e + 1] - z_start[e] : 0;
-    const int own = (rows + ROWS - 1) / ROWS * nt;
-    int upto = own;
+    *own = (rows + ROWS - 1) / ROWS * nt;
+    int upto = *own;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const int v = __shfl_up(upto, o);
       if (lane >= o) upto += v;
     }
+    return upto;
+  };
+  int own, total = 0;
+  for (int e0 = 0; e0 < batch; e0 += 64) total += __shfl(count(e0, &own), 63);
+  const int each = (total + 7) / 8, at = blockIdx.x >> 3;
+  int t = (blockIdx.x & 7) * each + at;
+  if (at >= each || t >= total) return false;
+  for (int e0 = 0; e0 < batch; e0 += 64) {
+    const int upto = count(e0, &own);
     const unsigned long long past = __ballot(upto > t);
     if (past) {
       const int l = __ffsll(past) - 1;
-      z = e0 + l;
-      t -= __shfl(upto - own, l);
-      found = true;
-    } else {
-      t -= __shfl(upto, 63);
+      *z_at = __builtin_amdgcn_readfirstlane(e0 + l);
+      *t_at = __builtin_amdgcn_readfirstlane(t - __shfl(upto - own, l));
+      return true;
     }
+    t -= __shfl(upto, 63);
   }
-  if (!found) return false;
-  z = __builtin_amdgcn_readfirstlane(z);
-  t = __builtin_amdgcn_readfirstlane(t);
-  *t_at = t;
-  *z_at = z;
-  return true;
+  return false;
 }
 
-// Bound by the matrix cores' feeding: without its DMAs the 256 x 256 form runs 1.3 times as fast, without its fragment
-// reads 1.1 times, without both at the matrix cores' rate (2.1 PFLOP/s). Results go straight to memory, past the caches
-// (a lane's rows in 128-byte pieces): turning them in LDS into longer pieces cost 14 us a tile.
+// an activation on more accumulators than these is code past what the compiler unrolls (it then keeps them in memory)
+template <int FM, int FN>
+constexpr bool kActsFit = FM * FN <= 8;
+
+// Bound by the matrix cores and the power that they take (gemm_tiles.h); start, end and the results of a round of 256 x 256
+// tiles cost 15 us, of 256 x 128 8. Results go straight to memory, past the caches (a lane's rows in 128-byte pieces):
+// turning them in LDS into longer pieces cost 14 us a tile.
 //
 // Workgroup b runs on XCD b % 8, and an XCD takes neighbouring tiles, whose rows of A and W its L2 then holds.
-template <int WM, int WN, int FM, int FN, int BK, int ST>
+template <int WM, int WN, int FM, int FN, int RA, int RB>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, int nt, int batch) {
-  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
-  constexpr int P = T::P;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[ST * T::STAGE];
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -78,89 +84,99 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, in
     n = t / gm;
   }
   const int m0 = m * T::BM, n0 = n * T::BN;
-  int nk = p.K / BK, k0 = 0;
-  if (p.ksplit > 1) {  // (kper counts 64 values of K)
-    k0 = split * p.kper * T::RPL;
-    nk = min(nk - k0, p.kper * T::RPL);
+  int nk = p.K / 64, k0 = 0;
+  if (p.ksplit > 1) {
+    k0 = split * p.kper;
+    nk = min(nk - k0, p.kper);
   }
-  // DMA sources: lane -> LDS row lane / 8 of the piece, the 16-byte chunk of it that the swizzle places at lane % 8
-  const unsigned char* src[P];
+  const unsigned char *src_a[T::PA], *src_w[T::PB];
+  int r, c;
 #pragma unroll
-  for (int i = 0; i < P; ++i) {
-    const int piece = wave * P + i;
-    const bool of_a = piece < T::BM / T::ROWS;  // (wave-uniform)
-    int r, c;
-    lga::gemm_dma_at<BK>((of_a ? piece : piece - T::BM / T::ROWS) * 8 + (lane >> 3), lane, &r, &c);
-    if (of_a) {
-      const int lr = r_lo + min(m0 + r, Mz - 1);  // rows past the end repeat the last one (never stored)
-      src[i] = (const unsigned char*)(p.a16 + (size_t)z * p.sa + (size_t)(p.a_rows ? p.a_rows[lr] : lr) * p.lda);
-    } else {
-      src[i] = (const unsigned char*)((const uint16_t*)p.w + (size_t)z * p.sw + (size_t)min(n0 + r, p.N - 1) * p.K);
-    }
-    src[i] += (size_t)k0 * (BK * 2) + c * 16;
+  for (int i = 0; i < T::PA; ++i) {
+    lga::gemm_dma_at(wave * T::PA + i, lane, &r, &c);
+    const int lr = r_lo + min(m0 + r, Mz - 1);  // rows past the end repeat the last one (never stored)
+    src_a[i] = (const unsigned char*)(p.a16 + (size_t)z * p.sa + (size_t)(p.a_rows ? p.a_rows[lr] : lr) * p.lda) +
+               (size_t)k0 * 128 + c * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < T::PB; ++i) {
+    lga::gemm_dma_at(wave * T::PB + i, lane, &r, &c);
+    src_w[i] = (const unsigned char*)((const uint16_t*)p.w + (size_t)z * p.sw + (size_t)min(n0 + r, p.N - 1) * p.K) +
+               (size_t)k0 * 128 + c * 16;
   }
   f32x16_t acc[FM][FN];
-  gemm_tile<WM, WN, FM, FN, BK, ST>(lds, src, nk, wave, lane, acc);
+  gemm_tile<WM, WN, FM, FN, RA, RB>(lds, src_a, src_w, nk, wave, lane, acc);
+  // a lane holds column l31 of a fragment and its rows 8 (e / 4) + 4 hi + e % 4: the wave's rows and columns begin at
+  // (mw, nw); a row's address is the wave's, a lane's place in it 32 bits
   const int wm = wave % WM, wn = wave / WM, l31 = lane & 31, hi = lane >> 5;
-  // a lane holds column l31 of a fragment and its rows 8 (e / 4) + 4 hi + e % 4
-  const int row0 = m0 + wm * FM * 32 + hi * 4, col0 = n0 + wn * FN * 32 + l31;
-  auto each = [&](auto&& put) {
+  const int mw = m0 + wm * FM * 32, nw = n0 + wn * FN * 32;
+  const bool inside = mw + FM * 32 <= Mz && nw + FN * 32 <= p.N;
+  auto each = [&](auto in, auto* y, long ld, auto&& put) {  // y: (mw, nw)
+    const unsigned at = (unsigned)(hi * 4 * (int)ld + l31);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int r = i * 32 + (e >> 2) * 8 + (e & 3);
-        if (row0 + r < Mz)
+        auto* row = y + (long)r * ld;
+        if (decltype(in)::value || mw + hi * 4 + r < Mz)
 #pragma unroll
           for (int j = 0; j < FN; ++j)
-            if (col0 + j * 32 < p.N) put(r, j, acc[i][j][e]);
+            if (decltype(in)::value || nw + l31 + j * 32 < p.N) put(row + j * 32 + at, j, acc[i][j][e]);
+        __builtin_amdgcn_sched_barrier(0);  // (or all accumulators are fetched ahead, into memory)
       }
   };
+  constexpr std::true_type in{};
+  constexpr std::false_type some{};
   if (p.ksplit > 1) {
-    float* y = p.part + ((size_t)split * p.M + row0) * p.N + col0;
-    each([&](int r, int j, float v) { y[(long)r * p.N + j * 32] = v; });
+    float* y = p.part + ((size_t)split * p.M + mw) * p.N + nw;
+    auto put = [](float* o, int, float v) { *o = v; };
+    if (inside) each(in, y, p.N, put);
+    else each(some, y, p.N, put);
     return;
   }
   float bias[FN];
 #pragma unroll
-  for (int j = 0; j < FN; ++j) bias[j] = p.bias ? p.bias[min(col0 + j * 32, p.N - 1)] : 0.0f;
-  const long at = (long)z * p.sy + (long)(r_lo + row0) * p.ldy + col0;
-  if (p.act != kActNone) {  // (few products have one: a loop that keeps the code small)
-    each([&](int r, int j, float v) {
-      v = act_f(p.act, v + bias[j]);
-      const long o = at + (long)r * p.ldy + j * 32;
-      if (p.y16) p.y16[o] = f2bf(v);
-      else p.y[o] = p.accumulate ? p.y[o] + v : v;
-    });
+  for (int j = 0; j < FN; ++j) bias[j] = p.bias ? p.bias[min(nw + l31 + j * 32, p.N - 1)] : 0.0f;
+  const long at = (long)z * p.sy + (long)(r_lo + mw) * p.ldy + nw;
+  if (kActsFit<FM, FN> && p.act != kActNone) {
+    if constexpr (kActsFit<FM, FN>) {
+      if (p.y16) each(some, p.y16 + at, p.ldy, [&](uint16_t* o, int j, float v) { *o = f2bf(act_f(p.act, v + bias[j])); });
+      else each(some, p.y + at, p.ldy, [&](float* o, int j, float v) {
+        v = act_f(p.act, v + bias[j]);
+        *o = p.accumulate ? *o + v : v;
+      });
+    }
   } else if (p.y16) {
-    each([&](int r, int j, float v) { p.y16[at + (long)r * p.ldy + j * 32] = f2bf(v + bias[j]); });
+    each(some, p.y16 + at, p.ldy, [&](uint16_t* o, int j, float v) { *o = f2bf(v + bias[j]); });
   } else if (p.accumulate) {
-    each([&](int r, int j, float v) { p.y[at + (long)r * p.ldy + j * 32] += v + bias[j]; });
+    each(some, p.y + at, p.ldy, [&](float* o, int j, float v) { *o += v + bias[j]; });
   } else {
-    each([&](int r, int j, float v) { __builtin_nontemporal_store(v + bias[j], p.y + at + (long)r * p.ldy + j * 32); });
+    auto put = [&](float* o, int j, float v) { __builtin_nontemporal_store(v + bias[j], o); };
+    if (inside) each(in, p.y + at, p.ldy, put);
+    else each(some, p.y + at, p.ldy, put);
   }
 }
 
-template <int WM, int WN, int FM, int FN, int BK, int ST>
+template <int WM, int WN, int FM, int FN, int RA, int RB>
 static int gemm_go(const LinArgs& p, int batch, hipStream_t stream) {
-  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   const int mt = (p.M + T::BM - 1) / T::BM, nt = (p.N + T::BN - 1) / T::BN;
   const long tiles = p.z_start ? (long)(mt + batch) * nt : (long)mt * nt * batch * p.ksplit;
   LGA_CHECK_ARG(tiles < (1L << 30), "lgs_linear: too many tiles");
-  gemm_kernel<WM, WN, FM, FN, BK, ST><<<(unsigned)((tiles + 7) / 8 * 8), T::NT, 0, stream>>>(p, mt, nt, batch);
+  gemm_kernel<WM, WN, FM, FN, RA, RB><<<(unsigned)((tiles + 7) / 8 * 8), T::NT, 0, stream>>>(p, mt, nt, batch);
   return 0;
 }
 
 // act(gate) * up with the gate's and the up's rows of W in turn as the tile's A, 32 of each: the pair of a column meets in
 // one lane, which has four neighbouring columns of a row and stores them rounded to bf16. Two passes over fp32 results of
-// twice the width and a launch less than the product and its unit apart, whose bits it gives: 511 us for 2407 rows, twice
-// 11008 columns and K 4096 in a model's prompt, where the two took 497 and 82.
-template <int WM, int WN, int FM, int FN, int BK, int ST, bool CLAMPED>
+// twice the width and a launch less than the product and its unit apart, whose bits it gives: 403 us for 2407 rows, twice
+// 11008 columns and K 4096 in a model's prompt (511 on stages of 32 values of K).
+template <int WM, int WN, int FM, int FN, int RA, int RB, bool CLAMPED>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluForm f, int mt, int nt, int batch) {
-  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
-  constexpr int P = T::P;
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   static_assert(FM % 2 == 0, "fragments of the two matrices in pairs");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[ST * T::STAGE];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -178,75 +194,80 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluFor
     m = g * 8 + t % gm, n = t / gm;
   }
   const int m0 = m * T::BN, n0 = n * (T::BM / 2);
-  const unsigned char* src[P];
+  const unsigned char *src_w[T::PA], *src_x[T::PB];
+  int r, c;
 #pragma unroll
-  for (int i = 0; i < P; ++i) {
-    const int piece = wave * P + i;
-    const bool of_w = piece < T::BM / T::ROWS;  // (wave-uniform)
-    int r, c;
-    lga::gemm_dma_at<BK>((of_w ? piece : piece - T::BM / T::ROWS) * 8 + (lane >> 3), lane, &r, &c);
-    if (of_w) {  // columns past the end repeat the last one (never stored)
-      const int col = min(n0 + r / 64 * 32 + r % 32, p.N - 1);
-      src[i] = (const unsigned char*)((const uint16_t*)p.w + (size_t)z * p.sw + (r / 32 % 2 ? f.up : 0) + (size_t)col * p.K);
-    } else {
-      const int lr = r_lo + min(m0 + r, Mz - 1);
-      src[i] = (const unsigned char*)(p.a16 + (size_t)(p.a_rows ? p.a_rows[lr] : lr) * p.lda);
-    }
-    src[i] += c * 16;
+  for (int i = 0; i < T::PA; ++i) {  // columns past the end repeat the last one (never stored)
+    lga::gemm_dma_at(wave * T::PA + i, lane, &r, &c);
+    const int col = min(n0 + r / 64 * 32 + r % 32, p.N - 1);
+    src_w[i] = (const unsigned char*)((const uint16_t*)p.w + (size_t)z * p.sw + (r / 32 % 2 ? f.up : 0) + (size_t)col * p.K) + c * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < T::PB; ++i) {
+    lga::gemm_dma_at(wave * T::PB + i, lane, &r, &c);
+    const int lr = r_lo + min(m0 + r, Mz - 1);
+    src_x[i] = (const unsigned char*)(p.a16 + (size_t)(p.a_rows ? p.a_rows[lr] : lr) * p.lda) + c * 16;
   }
   f32x16_t acc[FM][FN];
-  gemm_tile<WM, WN, FM, FN, BK, ST>(lds, src, p.K / BK, wave, lane, acc);
+  gemm_tile<WM, WN, FM, FN, RA, RB>(lds, src_w, src_x, p.K / 64, wave, lane, acc);
   const int wm = wave % WM, wn = wave / WM, l31 = lane & 31, hi = lane >> 5;
+  auto store = [&](auto&& unit) {
 #pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    const int row = m0 + (wn * FN + j) * 32 + l31;
-    if (row >= Mz) continue;
+    for (int j = 0; j < FN; ++j) {
+      const int row = m0 + (wn * FN + j) * 32 + l31;
+      if (row >= Mz) continue;
 #pragma unroll
-    for (int i = 0; i < FM; i += 2)
+      for (int i = 0; i < FM; i += 2)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int col = n0 + (wm * FM + i) * 16 + q * 8 + hi * 4;
-        if (col >= p.N) continue;
-        uint32_t o[2];
+        for (int q = 0; q < 4; ++q) {
+          const int col = n0 + (wm * FM + i) * 16 + q * 8 + hi * 4;
+          if (col >= p.N) continue;
+          uint32_t o[2];
 #pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-          const float a = glu_f<CLAMPED>(f, acc[i][j][q * 4 + e], acc[i + 1][j][q * 4 + e]);
-          const float b = glu_f<CLAMPED>(f, acc[i][j][q * 4 + e + 1], acc[i + 1][j][q * 4 + e + 1]);
-          o[e / 2] = (uint32_t)f2bf(a) | (uint32_t)f2bf(b) << 16;
+          for (int e = 0; e < 4; e += 2) {
+            const float a = unit(acc[i][j][q * 4 + e], acc[i + 1][j][q * 4 + e]);
+            const float b = unit(acc[i][j][q * 4 + e + 1], acc[i + 1][j][q * 4 + e + 1]);
+            o[e / 2] = (uint32_t)f2bf(a) | (uint32_t)f2bf(b) << 16;
+          }
+          *(uint2*)(p.y16 + (size_t)(r_lo + row) * p.ldy + col) = make_uint2(o[0], o[1]);
         }
-        *(uint2*)(p.y16 + (size_t)(r_lo + row) * p.ldy + col) = make_uint2(o[0], o[1]);
-      }
-  }
+    }
+  };
+  // the unit that gated models have gets code of its own: a choice per result costs 18 us a round of 256 x 256 tiles
+  if (CLAMPED || f.act != kActSilu) store([&](float g, float u) { return glu_f<CLAMPED>(f, g, u); });
+  else store([](float g, float u) { return act_f(kActSilu, g) * u; });
 }
 
-template <int WM, int WN, int FM, int FN, int BK, int ST>
+template <int WM, int WN, int FM, int FN, int RA, int RB>
 static int glu_go(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
-  using T = GemmTile<WM, WN, FM, FN, BK, ST>;
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   const int mt = (p.M + T::BN - 1) / T::BN, nt = (p.N + T::BM / 2 - 1) / (T::BM / 2);
   const long tiles = p.z_start ? (long)(mt + batch) * nt : (long)mt * nt;
   LGA_CHECK_ARG(tiles < (1L << 30), "lgs_linear_glu: too many tiles");
   const unsigned grid = (unsigned)((tiles + 7) / 8 * 8);
-  if (f.clamped) gemm_glu_kernel<WM, WN, FM, FN, BK, ST, true><<<grid, T::NT, 0, stream>>>(p, f, mt, nt, batch);
-  else gemm_glu_kernel<WM, WN, FM, FN, BK, ST, false><<<grid, T::NT, 0, stream>>>(p, f, mt, nt, batch);
+  if (f.clamped) gemm_glu_kernel<WM, WN, FM, FN, RA, RB, true><<<grid, T::NT, 0, stream>>>(p, f, mt, nt, batch);
+  else gemm_glu_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(p, f, mt, nt, batch);
   return 0;
 }
 
 int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
-#define LGS_CASE(I, SLOTS, US, ...) \
-  case I: return glu_go<__VA_ARGS__>(p, f, batch, stream);
-  switch (lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, true).tile) { LGA_GEMM_FORMS(LGS_CASE) }
+#define LGS_CASE(I, SLOTS, US, FAST, ROUND, ...)                                     \
+  case I:                                                                            \
+    if constexpr (lga::GemmTile<__VA_ARGS__>::FRAGS % 2 == 0) return glu_go<__VA_ARGS__>(p, f, batch, stream); \
+    break;
+  switch (lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, lga::kGemmRowsB | lga::kGemmPairs).tile) { LGA_GEMM_FORMS(LGS_CASE) }
 #undef LGS_CASE
   lga_set_error("lgs_linear_glu: no such form");
   return (int)hipErrorInvalidValue;
 }
 
-GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit) {
+GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act) {
   if (grouped && gemm_few_rows(M, batch)) return GemmPlan{-1, 1};
-  return lga::gemm_tile_plan(M, N, K, batch, grouped, ksplit);
+  return lga::gemm_tile_plan(M, N, K, batch, grouped, ksplit, act != kActNone ? lga::kGemmActs : 0);
 }
 
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream) {
-#define LGS_CASE(I, SLOTS, US, ...) \
+#define LGS_CASE(I, SLOTS, US, FAST, ROUND, ...) \
   case I: return gemm_go<__VA_ARGS__>(p, batch, stream);
   switch (plan.tile) { LGA_GEMM_FORMS(LGS_CASE) }
 #undef LGS_CASE

@@ -9,6 +9,8 @@
 //                  over row ranges of a sorted list (sparse experts during a prompt).
 //   lgs_embed      x[t] = table[token[t]] * scale
 //   lgs_rmsnorm    y = x / sqrt(mean(x^2) + eps) * (offset + w), rows with strides (whole rows, or heads)
+#include <algorithm>
+
 #include "seq_gemm.h"
 
 namespace lgs {
@@ -616,8 +618,8 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
     p.kper = (nk + ksplit - 1) / ksplit;
     p.ksplit = (nk + p.kper - 1) / p.kper;  // (no empty range)
   }
-  if (a_bf16 && vec) {
-    const lgs::GemmPlan plan = lgs::gemm_plan(M, N, K, batch, z_start != nullptr, p.ksplit);
+  if (a_bf16 && vec && std::max(ldy, (long)N) < (1L << 28)) {  // (a lane's place in four rows of Y: 32 bits)
+    const lgs::GemmPlan plan = lgs::gemm_plan(M, N, K, batch, z_start != nullptr, p.ksplit, act);
     if (plan.tile >= 0) {
       const int rc = lgs::gemm_launch(p, plan, batch, stream);
       if (rc) return rc;

@@ -79,3 +79,31 @@ def test_strided_batch():
         for z in range(Z):
             want = a[:, z * K:(z + 1) * K].double() @ w[z].double().T
             assert (y[:, z * N:(z + 1) * N].double() - want).abs().max() < TOL
+
+
+# every tile form with a partial last tile of rows and of columns, rows as the tile's A (tests of products with rows as its
+# B: below); few values of K, so that rings are refilled past the end from the first step on
+@pytest.mark.parametrize("M,N,K", [(1279, 12031, 256), (1023, 10753, 128), (3327, 2305, 1024), (385, 12289, 256),
+                                   (257, 10943, 128), (769, 6913, 128), (257, 6529, 128), (65, 127, 128), (769, 9471, 128)])
+def test_every_form_at_its_edges(M, N, K):
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    a, w, b = operands(M, N, K, dev, seed=3)
+    want = a.double() @ w.double().T + b.double()
+    y = torch.full((M + 1, N), float("nan"), device=dev)
+    seq_ops.linear(a, w, M=M, N=N, K=K, y=y, lda=K, ldy=N, bias=b)
+    assert (y[:M].double() - want).abs().max() < TOL and y[M:].isnan().all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1279, 12032, 256), (575, 13056, 128), (769, 6656, 1024), (1023, 5376, 256), (769, 4608, 128),
+                                   (769, 6528, 128), (257, 5504, 128), (129, 64, 128), (769, 9408, 128)])
+def test_every_form_of_prompt_products(M, N, K):
+    """bf16 weights of the GPT models: one rounding of the sum to bf16."""
+    from lit_gpt import ops
+
+    dev = torch.device("cuda", 0)
+    a, w, _ = operands(M, N, K, dev, seed=5)
+    want = a.double() @ w.double().T
+    y = ops.q4_gemm_fused(a, w, None, N, K, 0, 2)
+    assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + TOL).all()
