@@ -52,30 +52,12 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
   f32x16_t acc[FM][FN];
   gemm_tile<WM, WN, FM, FN, RA, RB>(lds, src_w, src_x, nk, wave, lane, acc);
   const int wm = wave % WM, wn = wave / WM, l31 = lane & 31, hi = lane >> 5;
-  const size_t ldy = a.ldy ? a.ldy : a.N;
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     const int m = m0 + (wn * FN + j) * 32 + l31;
-    if (m >= a.M) continue;
 #pragma unroll
     for (int i = 0; i < FM; i += DUAL ? 2 : 1)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + (wm * FM + i) * (DUAL ? 16 : 32) + q * 8 + hi * 4;
-        if (n >= a.N) continue;
-        q4d_f32x4 h, h2;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = acc[i][j][q * 4 + e], h2[e] = acc[i + (DUAL ? 1 : 0)][j][q * 4 + e];
-        if (k.splits > 1) {
-          float* p = a.slabs + ((size_t)split * (DUAL ? 2 : 1) * a.M + m) * a.N + n;
-          *(q4d_f32x4*)p = h;
-          if (DUAL) *(q4d_f32x4*)(p + (size_t)a.M * a.N) = h2;
-        } else if (DUAL) {
-          *(uint2*)(a.y + m * ldy + n) = q4d_swiglu(h, h2);
-        } else {
-          q4d_store(a, m, n, ldy, h);
-        }
-      }
+      q4d_store_fragment<DUAL>(a, acc[i][j], acc[i + (DUAL ? 1 : 0)][j], m, n0 + (wm * FM + i) * (DUAL ? 16 : 32), hi, split, k.splits);
   }
 }
 
@@ -91,13 +73,19 @@ static void bf16_go(BfArgs k, bool dual, hipStream_t stream) {
   if (!dual) gemm_bf16_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(k);
 }
 
-// All products but those of few rows and small weights, where a launch over ranges of K and one that adds them are not
-// repaid (us here / on gemm_q4f.hip's tiles): 16 x 4096 x 4096 20 / 14, 16 x 4096 x 11008 26 / 23, against 38 / 39 for 8192 x
-// 8192 (2^26).
+// Products with a workspace of partial sums: all but those of few rows and small weights, where a launch over ranges of K and
+// one that adds them are not repaid (us here / on gemm_q4f.hip's tiles): 16 x 4096 x 4096 20 / 14, 16 x 4096 x 11008 26 /
+// 23, against 38 / 39 for 8192 x 8192 (2^26); and but those of more than 1024 rows that fill the chip with K whole
+static bool bf16_long(int M, long cols) { return M > 1024 && (M + 255) / 256 * (cols / 128) >= 256; }
 GemmPlan bf16_plan(int M, int N, int K, bool dual) {
   const long cols = dual ? 2L * N : N;
-  if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1};
+  if ((M <= 32 && cols * K < 1L << 26) || bf16_long(M, cols)) return GemmPlan{-1, 1};
   return gemm_tile_plan(M, (int)cols, K, 1, false, 0, kGemmRowsB | (dual ? kGemmPairs : 0));
+}
+GemmPlan bf16_long_plan(int M, int N, int K, bool dual) {
+  const long cols = dual ? 2L * N : N;
+  if (!bf16_long(M, cols)) return GemmPlan{-1, 1};
+  return gemm_tile_plan(M, (int)cols, K, 1, false, 1, kGemmRowsB | (dual ? kGemmPairs : 0));
 }
 
 size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {

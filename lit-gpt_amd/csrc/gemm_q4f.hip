@@ -13,6 +13,7 @@
 //    64 x 64 per wave = 4 x 4 `v_mfma_f32_16x16x32_bf16`), <256, 256> (64 x 128 per wave, one K-step of prefetch
 //    to fit LDS) where its rounds fill the CUs better (fc_1 || fc_2 at 2048 tokens: 11 % faster), and <64, 128> /
 //    <64, 256> for short ones (1 x 8 waves);
+//    of long prompts here: the grouped products and K of no multiple of 128 (gemm_q4r.hip and gemm_bf16.hip make the others);
 //    the weight rows are the A operand, so a lane's accumulators are 4 consecutive output columns of one row
 //    (8-byte stores).
 //  * X tiles and the packed weight / scale tiles reach LDS by LDS-DMA (`global_load_lds_dwordx4`, source-swizzled so
@@ -744,7 +745,8 @@ int run_tiles(Args a, int fmt, bool dual, int bn, hipStream_t stream);
 // LGA_Q4F_BN / LGA_Q4F_SPLITS name a launch of the tiles here
 bool tiles_named() { return getenv("LGA_Q4F_BN") || getenv("LGA_Q4F_SPLITS"); }
 
-// which form makes a product, and the workspace of the form that it makes
+// which form makes a product, and the workspace of the form that it makes. With the workspace of the tiles here (often
+// none) long prompts are made by gemm_q4r.hip and gemm_bf16.hip (run_long).
 enum Form { kTiles = 0, kRegisters = 1, kBf16Tiles = 2 };  // here; gemm_q4d.hip (4-bit); gemm_bf16.hip
 struct Route {
   Form form = kTiles;
@@ -767,13 +769,34 @@ Route route(int M, int N, int K, int fmt, bool dual) {
   return r;
 }
 
+// Long prompts on gemm_q4r.hip's tiles and, bf16 weights, gemm_bf16.hip's: faster at every size measured (their figures stand
+// there); false: not one of theirs.
+bool run_long(const lga::Q4dArgs& d, int fmt, bool dual, size_t ws_bytes, hipStream_t stream, int* rc) {
+  if (tiles_named()) return false;
+  if (lga::kernel_fmt(fmt) == 2) {
+    const lga::GemmPlan b = lga::bf16_long_plan(d.M, d.N, d.K, dual);
+    if (b.tile < 0) return false;
+    *rc = lga::bf16_run(d, b, dual, stream);
+    return true;
+  }
+  if (((uintptr_t)d.sc | (uintptr_t)d.sc2) % 8 != 0) return false;  // (scales are loaded in pairs)
+  const size_t plane = (size_t)(dual ? 2 : 1) * d.M * d.N * 4;
+  const lga::Q4rPlan l = lga::q4r_plan(
+      d.M, d.N, d.K, dual, lga::kernel_fmt(fmt), ws_bytes > 4096 ? (int)std::min<size_t>((ws_bytes - 4096) / plane, 16) : 1);
+  if (l.fn == 0) return false;
+  *rc = lga::q4r_run(d, l, lga::kernel_fmt(fmt), dual, stream);
+  return true;
+}
+
 int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t stream) {
   const Route r = route(a.M, a.N, a.K, fmt, dual);
+  const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
+                       lga::codebook_of(fmt), ws ? (float*)((unsigned char*)ws + 4096) : nullptr};
   if (r.form != kTiles && (r.need == 0 || (ws && ws_bytes >= r.need))) {  // (a smaller workspace may do for the tiles here)
-    const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
-                         lga::codebook_of(fmt), r.need ? (float*)((unsigned char*)ws + 4096) : nullptr};
     return r.form == kRegisters ? lga::q4d_run(d, r.d, lga::kernel_fmt(fmt), dual, stream) : lga::bf16_run(d, r.b, dual, stream);
   }
+  int rc;
+  if (r.form == kTiles && run_long(d, fmt, dual, ws ? ws_bytes : 0, stream, &rc)) return rc;
   if (!dual) {
     const int nb = q4f_big_columns(a.M, a.N, a.K);
     if (nb > 0) {
@@ -846,7 +869,7 @@ int lga::preload_gemm_q4f() {
   LGA_PRE(2, false);
   LGA_PRE(2, true);
 #undef LGA_PRE
-  return bad + lga::preload_gemm_q4d() + lga::preload_gemm_bf16();
+  return bad + lga::preload_gemm_q4d() + lga::preload_gemm_q4r() + lga::preload_gemm_bf16();
 }
 
 #ifdef LGA_Q4F_TRACE

@@ -170,3 +170,37 @@ def test_a_workspace_of_the_older_tiles(ops, M, N, K, monkeypatch):
     assert rc == 0
     h = x.float() @ wd.t()
     assert float(((y.float() - h).abs() - h.abs() * 2 ** -7).max()) <= 2e-3
+
+
+# the tiles of long prompts: 128, 192 and 256 rows a tile, one row past and one short of whole tiles, columns past the last whole
+# tile, one pair of steps and many, ranges of K of unequal length
+@pytest.mark.parametrize("fmt,group", [(0, 64), (0, 128), (1, 64), (1, 256), (3, 128)])
+@pytest.mark.parametrize("M,N,K", [(129, 136, 256), (257, 264, 512), (257, 4104, 1280), (385, 1032, 768), (511, 8200, 256),
+                                   (577, 520, 5632), (1025, 776, 1024)])
+@pytest.mark.parametrize("epi", ["plain", "bias+residual", "swiglu"])
+def test_long_prompts(ops, fmt, group, M, N, K, epi):
+    """Against fp32 products of the dequantized weights: the operands are bf16 and their sums fp32, so one rounding to bf16
+    (2^-9 of the value) and K roundings of partial sums, 2e-4 at the largest K here, stand between the two."""
+    g = torch.Generator(device=DEV).manual_seed(K + M)
+    w, sc, wd = _weight(ops, N, K, fmt, group, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    h = x.float() @ wd.t()
+    if epi == "swiglu":
+        w2, sc2, wd2 = _weight(ops, N, K, fmt, group, g)
+        a, b = h.to(torch.bfloat16).float(), (x.float() @ wd2.t()).to(torch.bfloat16).float()
+        ref = (a * torch.sigmoid(a)).to(torch.bfloat16).float() * b
+        y = ops.q4_gemm_swiglu(x, w, sc, w2, sc2, N, K, group, fmt).float()
+        # each factor may round to the neighbouring bf16 number
+        tol = 2 ** -7 * (1.1 * (a * b).abs() + 2 * ref.abs()) + 2 ** -8 * ref.abs() + 2e-3
+        assert float(((y - ref).abs() - tol).max()) <= 0.0
+        return
+    if epi == "plain":
+        y = ops.q4_gemm_fused(x, w, sc, N, K, group, fmt).float()
+        assert float(((y - h).abs() - h.abs() * 2 ** -8).max()) <= 2e-4
+        return
+    bias = torch.randn(N, generator=g, device=DEV).to(torch.bfloat16)
+    res = torch.randn(M, N, generator=g, device=DEV).to(torch.bfloat16)
+    h = h + bias.float()
+    ref = h.to(torch.bfloat16).float() + res.float()
+    y = ops.q4_gemm_fused(x, w, sc, N, K, group, fmt, bias=bias, residual=res).float()
+    assert float(((y - ref).abs() - (ref.abs() + h.abs()) * 2 ** -7).max()) <= 2e-3
