@@ -28,7 +28,7 @@ int q4d_run(const Q4dArgs& a, const Q4dPlan& p, int kernel_fmt, bool dual, hipSt
 void q4d_sum(const Q4dArgs& a, int splits, bool dual, hipStream_t stream);
 int preload_gemm_q4d();
 
-// long prompts (gemm_q4r.hip). fn: 32-row pieces of X per tile (0: not one of its products), per: pairs of steps of 64 values
+// long prompts and most short ones (gemm_q4r.hip). fn: 32-row pieces of X per tile (0: not one of its products), per: pairs of steps of 64 values
 struct Q4rPlan {
   int fn, mt, nt, splits, per;
 };

@@ -745,8 +745,8 @@ int run_tiles(Args a, int fmt, bool dual, int bn, hipStream_t stream);
 // LGA_Q4F_BN / LGA_Q4F_SPLITS name a launch of the tiles here
 bool tiles_named() { return getenv("LGA_Q4F_BN") || getenv("LGA_Q4F_SPLITS"); }
 
-// which form makes a product, and the workspace of the form that it makes. With the workspace of the tiles here (often
-// none) long prompts are made by gemm_q4r.hip and gemm_bf16.hip (run_long).
+// which form makes a product, and the workspace of the form that it makes. With that workspace (often none) long prompts are
+// made by gemm_q4r.hip and gemm_bf16.hip, and most short 4-bit ones by gemm_q4r.hip (run_long).
 enum Form { kTiles = 0, kRegisters = 1, kBf16Tiles = 2 };  // here; gemm_q4d.hip (4-bit); gemm_bf16.hip
 struct Route {
   Form form = kTiles;
@@ -769,8 +769,8 @@ Route route(int M, int N, int K, int fmt, bool dual) {
   return r;
 }
 
-// Long prompts on gemm_q4r.hip's tiles and, bf16 weights, gemm_bf16.hip's: faster at every size measured (their figures stand
-// there); false: not one of theirs.
+// Products on gemm_q4r.hip's tiles and, long prompts with bf16 weights, gemm_bf16.hip's: their figures stand there; false: not
+// one of theirs.
 bool run_long(const lga::Q4dArgs& d, int fmt, bool dual, size_t ws_bytes, hipStream_t stream, int* rc) {
   if (tiles_named()) return false;
   if (lga::kernel_fmt(fmt) == 2) {
@@ -792,11 +792,12 @@ int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t strea
   const Route r = route(a.M, a.N, a.K, fmt, dual);
   const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
                        lga::codebook_of(fmt), ws ? (float*)((unsigned char*)ws + 4096) : nullptr};
-  if (r.form != kTiles && (r.need == 0 || (ws && ws_bytes >= r.need))) {  // (a smaller workspace may do for the tiles here)
+  int rc;
+  const bool whole = r.need == 0 || (ws && ws_bytes >= r.need);  // (a smaller workspace may do for the tiles here)
+  if ((r.form == kTiles || (r.form == kRegisters && whole)) && run_long(d, fmt, dual, ws ? ws_bytes : 0, stream, &rc)) return rc;
+  if (r.form != kTiles && whole) {
     return r.form == kRegisters ? lga::q4d_run(d, r.d, lga::kernel_fmt(fmt), dual, stream) : lga::bf16_run(d, r.b, dual, stream);
   }
-  int rc;
-  if (r.form == kTiles && run_long(d, fmt, dual, ws ? ws_bytes : 0, stream, &rc)) return rc;
   if (!dual) {
     const int nb = q4f_big_columns(a.M, a.N, a.K);
     if (nb > 0) {

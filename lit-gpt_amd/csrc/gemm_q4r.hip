@@ -1,5 +1,5 @@
-// Prefill GEMM of long prompts with 4-bit weights: the products of gemm_q4d.hip (Y = X . bf16(dequant(W))^T with bias /
-// residual, and fc_1 || fc_2 + SwiGLU) where a tile of weights serves 128 to 256 rows.
+// Prefill GEMM with 4-bit weights: the products of gemm_q4d.hip (Y = X . bf16(dequant(W))^T with bias / residual, and fc_1 ||
+// fc_2 + SwiGLU) where a tile of weights serves 128 to 256 rows, and most of those where it serves 32 to 96.
 //
 // A workgroup of four waves makes 256 columns (SwiGLU: 128 of each matrix) of 32 FN rows; a wave 64 columns of all its rows:
 // 2 x FN accumulators of v_mfma_f32_32x32x16_bf16 with the weights as the A operand, so that no weight is dequantized
@@ -9,12 +9,18 @@
 // to the bits that bnb's dequantize_4bit writes, between the matrix instructions of the 16 values of K before. The products'
 // order over K follows what a lane holds: instruction m of a step takes values 8 m .. + 7 and 32 + 8 m .. + 7. (Weights loaded
 // straight into registers cost 64 separate addresses a load: 930 of 5600 clocks a pair of steps, scales two at a time 700.)
+//
+// Up to 96 rows a wave has too few matrix instructions to stand its 410 others of a pair of steps between (one each five
+// clocks while a wave is alone on its SIMD, half as many while two are): a second group of four waves takes the other half of
+// the workgroup's range of K, with buffers of its own, and hands its sums over in LDS. 93 rows of nf4 28672 x 8192 with SwiGLU:
+// one group 135 us, two workgroups of one group each on a CU and halves of K through memory 137, two groups 124.
 #include "gemm_q4d.h"
 
 namespace lga {
 namespace pr {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 struct KArgs {
   Q4dArgs a;
@@ -88,8 +94,9 @@ struct Dequant<1> {  // codebook in LDS, fp32 product: the lookups first, the pr
 
 template <int FN>
 struct Tile {
-  static constexpr int RX = FN == 8 ? 3 : (FN == 6 ? 5 : 6);  // X: steps of 64 values in LDS
-  static constexpr int XB = FN * 4096, WB = 16384, OFF_W = RX * XB, OFF_TAB = OFF_W + 2 * WB, LDS = OFF_TAB + 64;
+  static constexpr int KW = FN < 4 ? 2 : 1;                                              // groups of four waves: halves of K
+  static constexpr int RX = FN == 8 ? 3 : (FN == 6 ? 5 : (FN == 4 ? 6 : (FN == 3 ? 3 : 4)));  // X: steps of 64 values in LDS
+  static constexpr int XB = FN * 4096, WB = 16384, OFF_W = RX * XB, GROUP = OFF_W + 2 * WB, OFF_TAB = KW * GROUP, LDS = OFF_TAB + 64;
   static_assert(LDS <= 163840, "LDS");
   // loads younger than X of step k + 1 at the barrier of step k: what the steps since its own have issued (X, and the scales of
   // a pair in its first step, its weights in its second)
@@ -103,14 +110,15 @@ struct Tile {
 
 // FMT 0 int4-g (bf16 scales), 1 codebook (fp32 block maxima)
 template <int FMT, bool DUAL, int FN>
-__global__ void __launch_bounds__(256, 1) gemm_q4r_kernel(KArgs k) {
+__global__ void __launch_bounds__(256 * Tile<FN>::KW, Tile<FN>::KW) gemm_q4r_kernel(KArgs k) {
   using T = Tile<FN>;
-  constexpr int RX = T::RX, XB = T::XB, E = 2 * FN;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
+  constexpr int RX = T::RX, XB = T::XB, KW = T::KW, E = 2 * FN;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds_all[T::LDS];
   const Q4dArgs& a = k.a;
   const int tid = threadIdx.x, lane = tid & 63, l31 = lane & 31, hi = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const unsigned char* tab = lds + T::OFF_TAB;
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all & 3, kg = wave_all >> 2;
+  unsigned char* lds = lds_all + kg * T::GROUP;
+  const unsigned char* tab = lds_all + T::OFF_TAB;
   if (FMT == 1 && tid < 16) ((float*)tab)[tid] = kCode4[a.cb][tid];
   // an XCD takes neighbouring tiles: of a column's weights those of up to eight row tiles, range after range
   int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -120,7 +128,8 @@ __global__ void __launch_bounds__(256, 1) gemm_q4r_kernel(KArgs k) {
   const int g = t / (8 * k.nt), gm = min(8, k.mt - g * 8);
   t -= g * 8 * k.nt;
   const int m0 = (g * 8 + t % gm) * (FN * 32), n0 = t / gm * (DUAL ? 128 : 256);
-  const int p0 = split * k.per, np = min(a.K / 128 - p0, k.per), nk = 2 * np;  // pairs of steps from p0 on
+  const int range = min(a.K / 128 - split * k.per, k.per), most = (range + KW - 1) / KW;  // pairs of steps; a group's at most
+  const int p0 = split * k.per + kg * most, np = kg == 0 ? most : range - most, nk = 2 * np;  // this group's, from p0 on
   const int groups = a.K / a.G, gshift = 31 - __builtin_clz((unsigned)a.G);
 
   // this wave's 64 rows of weights: of one matrix, or 32 of each; rows past the end repeat the last one (never stored)
@@ -251,7 +260,7 @@ __global__ void __launch_bounds__(256, 1) gemm_q4r_kernel(KArgs k) {
           if constexpr (FMT == 1 && e == FN) __builtin_amdgcn_s_waitcnt(0xC07F | 8 << 8);        // the other row's 8 behind
           if constexpr (FMT == 1 && e == FN + FN / 2) __builtin_amdgcn_s_waitcnt(0xC07F | FN / 2 << 8);  // X behind
           // X beside the products of looked-up values, or else ahead of the loads
-          constexpr int x = FMT == 1 ? e - FN : e, l = FMT == 1 ? e : e - FN;
+          constexpr int x = FMT == 1 ? e - FN : e, l = FMT == 1 || FN < 3 ? e : (FN == 3 ? e - 2 : e - FN);
           if constexpr (x >= 0 && x < FN) read_x(n, x, rs, nm);
           // lookups of both rows, then their products; without lookups row after row
           constexpr int HALF = FMT == 1 ? 4 : 8, lo = 16 * e / E, up = 16 * (e + 1) / E;
@@ -265,10 +274,12 @@ __global__ void __launch_bounds__(256, 1) gemm_q4r_kernel(KArgs k) {
           };
           parts(parts, std::integral_constant<int, lo>{});
           if constexpr (q == 0 && l == 0) fetch_scales(p + 1);
-          if constexpr (q == 4 && l >= 0 && l < 4) dma_w(l, p + 2);
+          if constexpr (q == 4 && FN > 1 && l >= 0 && l < 4) dma_w(l, p + 2);
+          if constexpr (q == 4 && FN == 1) dma_w(2 * e, p + 2), dma_w(2 * e + 1, p + 2);
           if constexpr (m == 1 && l >= 0 && l < FN) dma_x(l, 2 * p + st + RX - 1, free_slot);
           if constexpr (m == 2 && l >= 0 && l < 2) read_w(p + st, 1 - st, l);
-          if constexpr (q == 6 && (l == 2 || l == 3)) spread_scales(p + 1, l - 2, sn[l - 2]);
+          if constexpr (q == 6 && FN > 1 && (l == 2 || l == 3)) spread_scales(p + 1, l - 2, sn[l - 2]);
+          if constexpr (q == 6 && FN == 1) spread_scales(p + 1, e, sn[e]);
           __builtin_amdgcn_sched_barrier(0);
           eself(eself, std::integral_constant<int, e + 1>{});
         }
@@ -282,6 +293,37 @@ __global__ void __launch_bounds__(256, 1) gemm_q4r_kernel(KArgs k) {
   }
   gemm_wait_vm<0>();  // no DMA may outlive the workgroup's LDS
 
+  if constexpr (KW > 1) {  // group 1's sums meet group 0's in LDS
+    static_assert(FN * 32768 <= T::LDS, "sums of a group");
+    if (np < most) {  // (a group with a pair less: the other's barriers)
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_s_barrier();
+    }
+    __syncthreads();
+    f32x4_t* sums = (f32x4_t*)(lds_all + wave * (FN * 8192)) + lane;
+    if (kg != 0) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sums[((j * 2 + i) * 4 + e) * 64] =
+                f32x4_t{acc[i][j][e * 4], acc[i][j][e * 4 + 1], acc[i][j][e * 4 + 2], acc[i][j][e * 4 + 3]};
+    }
+    __syncthreads();
+    if (kg != 0) return;
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x4_t o = sums[((j * 2 + i) * 4 + e) * 64];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[i][j][e * 4 + c] += o[c];
+        }
+  }
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     const int m = m0 + j * 32 + l31;
@@ -294,14 +336,17 @@ __global__ void __launch_bounds__(256, 1) gemm_q4r_kernel(KArgs k) {
 template <int FMT, bool DUAL, int FN>
 static void go(KArgs k, hipStream_t stream) {
   const unsigned work = (unsigned)(k.mt * k.nt * k.splits);
-  gemm_q4r_kernel<FMT, DUAL, FN><<<(work + 7) / 8 * 8, 256, 0, stream>>>(k);
+  gemm_q4r_kernel<FMT, DUAL, FN><<<(work + 7) / 8 * 8, 256 * Tile<FN>::KW, 0, stream>>>(k);
   if (k.splits > 1) q4d_sum(k.a, k.splits, DUAL, stream);
 }
 template <int FMT, bool DUAL>
 static void go_rows(const KArgs& k, int fn, hipStream_t stream) {
   if (fn == 8) go<FMT, DUAL, 8>(k, stream);
   else if (fn == 6) go<FMT, DUAL, 6>(k, stream);
-  else go<FMT, DUAL, 4>(k, stream);
+  else if (fn == 4) go<FMT, DUAL, 4>(k, stream);
+  else if (fn == 3) go<FMT, DUAL, 3>(k, stream);
+  else if (fn == 2) go<FMT, DUAL, 2>(k, stream);
+  else go<FMT, DUAL, 1>(k, stream);
 }
 
 }  // namespace pr
@@ -309,23 +354,35 @@ static void go_rows(const KArgs& k, int fn, hipStream_t stream) {
 // Rounds of 256 workgroups times their pairs of steps (128 values of K), at the clock of a full chip or, with few workgroups, a
 // higher one, and their start and end. us of a pair for 256, 192 and 128 rows, measured on 256 workgroups of K 4096: int4 2.93,
 // 2.30, 1.75 (4740, 3870, 3140 clocks, of which 4096, 3072, 2048 of matrix instructions), codebooks 3.22, 2.67, 2.12 (5560,
-// 5050, 4470: sixteen more instructions per eight weights). us on gemm_q4f.hip's tiles / here, int4 with weights from memory:
-// 2048 rows of 12288 x 4096 209 / 197, 4096 x 4096 75 / 68, 11008 x 4096 with SwiGLU 374 / 311, 4096 x 11008 194 / 171; 517
-// rows 118 / 65, 71 / 37, 194 / 126, 126 / 70; 300 rows 70 / 56, -, 122 / 76, 90 / 49; nf4 2048 rows 233 / 212, 82 / 82, 429 /
-// 341, 209 / 202.
+// 5050, 4470: sixteen more instructions per eight weights); for 96, 64 and 32 rows from whole products of 86 to 240 workgroups.
+// us on gemm_q4f.hip's tiles / here, int4 with weights from memory: 2048 rows of 12288 x 4096 209 / 197, 4096 x 4096 75 / 68,
+// 11008 x 4096 with SwiGLU 374 / 311, 4096 x 11008 194 / 171; 517 rows 118 / 65, 71 / 37, 194 / 126, 126 / 70; 300 rows 70 / 56,
+// -, 122 / 76, 90 / 49; nf4 2048 rows 233 / 212, 82 / 82, 429 / 341, 209 / 202.
+// Up to 128 rows against gemm_q4d.hip's form, or the tiles where that is not taken, weights from memory:
+//   nf4 93 rows    28672 x 8192 with SwiGLU 150 / 124, 8192 x 28672 84 / 71, 10240 x 8192 41 / 39, 8192 x 8192 36 / 35
+//   nf4 64 rows    28672 x 8192 with SwiGLU 133 / 105, 8192 x 28672 71 / 62; 4096 x 4096 21 / 22, 6144 x 4096 23.2 / 23.6
+//   int4 64 rows   12288 x 4096 25.5 / 24.1, 11008 x 4096 with SwiGLU 37 / 33, 4096 x 4096 20.4 / 20.4, 4096 x 11008 23.3 / 24.7
+//   int4 128 rows  11008 x 4096 with SwiGLU 63 / 42, 4096 x 11008 35 / 30, 4096 x 4096 28 / 22
+//   32 rows        int4 4096 x 4096 19.6 / 14.6, 11008 x 4096 with SwiGLU 32 / 28; 4096 x 11008 20.1 / 21.1, nf4 10240 x 8192
+//                  28.9 / 30.0, 28672 x 8192 with SwiGLU 108 / 98: beyond 2^24 values one matrix stays in gemm_q4d.hip's form
 Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, int most) {
   Q4rPlan p{0, 0, 0, 0, 0};
-  if (K % 128 != 0 || M <= 128) return p;
+  const size_t nk = (size_t)N * K, one = 1;
+  if (K % 128 != 0) return p;
+  if (!dual && M <= 32 && nk > one << 24) return p;
+  if (!dual && M > 32 && M <= 64 && nk < one << 26 && (kernel_fmt == 1 || (nk > one << 24 && N <= 8192))) return p;
   const int cols = dual ? 128 : 256, np = K / 128;
   p.nt = (N + cols - 1) / cols;
-  const float pair_us[2][3] = {{2.93f, 2.30f, 1.75f}, {3.22f, 2.67f, 2.12f}};
-  const float fast_us[2][3] = {{1.97f, 1.61f, 1.31f}, {2.32f, 2.10f, 1.86f}};
+  constexpr int forms[] = {8, 6, 4, 3, 2, 1};
+  const float pair_us[2][6] = {{2.93f, 2.30f, 1.75f, 1.65f, 1.40f, 1.05f}, {3.22f, 2.67f, 2.12f, 1.85f, 1.55f, 1.42f}};
+  const float fast_us[2][6] = {{1.97f, 1.61f, 1.31f, 1.12f, 0.97f, 0.90f}, {2.32f, 2.10f, 1.86f, 1.40f, 1.28f, 1.19f}};
   float best = 0.0f;
-  for (int i = 0; i < 3; ++i) {
-    const int fn = 8 - 2 * i, mt = (M + fn * 32 - 1) / (fn * 32);
-    const float slow = pair_us[kernel_fmt][i], fast = fast_us[kernel_fmt][i], ends = 2.0f + fn;
+  for (int i = 0; i < 6; ++i) {
+    const int fn = forms[i], mt = (M + fn * 32 - 1) / (fn * 32);
+    const float slow = pair_us[kernel_fmt][i], fast = fast_us[kernel_fmt][i], ends = fn < 4 ? 4.0f : 2.0f + fn;
     for (int s = 1; s <= most && (s == 1 || np / s >= 2); ++s) {
       const int per = (np + s - 1) / s, used = (np + per - 1) / per;
+      if (fn < 4 && np - per * (used - 1) < 2) continue;  // (a pair for each half)
       const float rounds = (float)((long)mt * p.nt * used) / 256.0f, whole = floorf(rounds);
       float us = whole * (per * slow + ends);
       if (rounds > whole) us += per * fmaxf(fast, slow * (0.3f + 0.7f * (rounds - whole))) + ends;
@@ -351,7 +408,7 @@ int preload_gemm_q4r() {
   using namespace pr;
   int bad = 0;
 #define LGA_PRE(F, D) \
-  bad += preload(gemm_q4r_kernel<F, D, 4>) + preload(gemm_q4r_kernel<F, D, 6>) + preload(gemm_q4r_kernel<F, D, 8>)
+  bad += preload(gemm_q4r_kernel<F, D, 1>) + preload(gemm_q4r_kernel<F, D, 2>) + preload(gemm_q4r_kernel<F, D, 3>) + preload(gemm_q4r_kernel<F, D, 4>) + preload(gemm_q4r_kernel<F, D, 6>) + preload(gemm_q4r_kernel<F, D, 8>)
   LGA_PRE(0, false);
   LGA_PRE(0, true);
   LGA_PRE(1, false);

@@ -204,3 +204,27 @@ def test_long_prompts(ops, fmt, group, M, N, K, epi):
     ref = h.to(torch.bfloat16).float() + res.float()
     y = ops.q4_gemm_fused(x, w, sc, N, K, group, fmt, bias=bias, residual=res).float()
     assert float(((y - ref).abs() - (ref.abs() + h.abs()) * 2 ** -7).max()) <= 2e-3
+
+
+# 32, 64 and 96 rows a tile, whose two groups of waves share a range of K: ranges of an even and an odd number of pairs of
+# steps, as few as two; a row short of, at and past whole tiles; columns past the last whole tile
+@pytest.mark.parametrize("fmt,group", [(0, 64), (0, 128), (1, 64), (3, 128)])
+@pytest.mark.parametrize("M,N,K", [(2, 136, 256), (31, 264, 384), (32, 1032, 1408), (33, 8200, 256), (64, 8712, 7808), (65, 264, 896),
+                                   (96, 1032, 384), (97, 136, 2176), (128, 264, 128)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_short_prompts(ops, fmt, group, M, N, K, swiglu):
+    """As test_long_prompts: one rounding to bf16 and K roundings of partial sums between the product and its fp32 reference."""
+    g = torch.Generator(device=DEV).manual_seed(K + M)
+    w, sc, wd = _weight(ops, N, K, fmt, group, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    h = x.float() @ wd.t()
+    if not swiglu:
+        y = ops.q4_gemm_fused(x, w, sc, N, K, group, fmt).float()
+        assert float(((y - h).abs() - h.abs() * 2 ** -8).max()) <= 2e-4
+        return
+    w2, sc2, wd2 = _weight(ops, N, K, fmt, group, g)
+    a, b = h.to(torch.bfloat16).float(), (x.float() @ wd2.t()).to(torch.bfloat16).float()
+    ref = (a * torch.sigmoid(a)).to(torch.bfloat16).float() * b
+    y = ops.q4_gemm_swiglu(x, w, sc, w2, sc2, N, K, group, fmt).float()
+    tol = 2 ** -7 * (1.1 * (a * b).abs() + 2 * ref.abs()) + 2 ** -8 * ref.abs() + 2e-3
+    assert float(((y - ref).abs() - tol).max()) <= 0.0
