@@ -307,6 +307,16 @@ int lga_f32_layernorm(const float* x, const float* w, const float* b, float* y, 
 /* two LayerNorms of the same rows in one launch (GPT-NeoX: norm_1 and norm_2 of a parallel-residual block) */
 int lga_f32_layernorm_pair(const float* x, const float* w, const float* b, float* y, float eps, const float* w2,
                            const float* b2, float* y2, float eps2, int rows, int n, lga_stream_t stream);
+/* One row: y1 = act1(norm1(x) w1^T + b1) and, where N2 > 0, y2 = act2(norm2(x) w2^T + b2) in one launch, lga_f32_linear_act of
+ * lga_f32_layernorm's row to the bit. K a multiple of 4 up to 8192 */
+int lga_f32_norm_linears(const float* x, int K, const float* nw1, const float* nb1, float eps1, const float* w1,
+                         const float* b1, int act1, float* y1, int N1, const float* nw2, const float* nb2, float eps2,
+                         const float* w2, const float* b2, int act2, float* y2, int N2, lga_stream_t stream);
+/* One row: y = ((x2 w2^T + b2) + (x1 w1^T + b1)) + residual in one launch (a parallel-residual block's output projections).
+ * parts > 1: x1 [parts][K1] and ml are those of lga_f32_attention_decode_parts with heads of hs columns */
+int lga_f32_linears_sum(const float* x1, const float* ml, int parts, int hs, const float* w1, const float* b1, int K1,
+                        const float* x2, const float* w2, const float* b2, int K2, const float* residual, float* y, int N,
+                        lga_stream_t stream);
 /* F.gelu (exact erf, or tanh when approximate_tanh) — GptNeoxMLP (model.py:699-702) */
 int lga_f32_gelu(const float* a, float* y, long n, int approximate_tanh, lga_stream_t stream);
 /* y = a + b (the Block residual adds, model.py:584-593) */
@@ -328,6 +338,13 @@ int lga_f32_attention_decode(const float* qkv, float* k_cache, float* v_cache, c
                              const int64_t* rope_pos, const float* cos, const float* sin, int rope_rows, float* y,
                              int n_head, int n_query_groups, int head_size, int rope_n_elem, int max_seq, float scale,
                              lga_stream_t stream);
+/* The same over `parts` ranges of the keys side by side (1 to 8; lga_f32_attention_parts says how many pay): y [parts][H * hs] holds
+ * each range's sums of weighted values, ml [parts][H][2] its largest score and the sum of its weights (parts 1: y as above) */
+int lga_f32_attention_parts(int n_head, int max_seq);
+int lga_f32_attention_decode_parts(const float* qkv, float* k_cache, float* v_cache, const int64_t* cache_pos,
+                                   const int64_t* rope_pos, const float* cos, const float* sin, int rope_rows, float* y,
+                                   float* ml, int parts, int n_head, int n_query_groups, int head_size, int rope_n_elem,
+                                   int max_seq, float scale, lga_stream_t stream);
 /* lga_argmax over fp32 logits (generate/base.py:30-47 at temperature 0) */
 int lga_argmax_f32(const float* logits, int n, int64_t* out_idx, int32_t* token_out, int64_t* pos_inout,
                    lga_stream_t stream);

@@ -2,12 +2,15 @@
 // weights and activations in float32). BASELINE config 1 is quoted in it (pythia-160m fp32, greedy 128 tokens);
 // the bf16 kernels round every activation to bf16, which the fp32 fixture (tests/golden/g1) does not.
 //
-// A step of a 160M model is launches and their latency: what runs on one row is fused (RoPE, cache append and attention;
-// both norms of a parallel-residual block; gelu and the residual adds in the products' epilogues), 75 launches a token.
+// A step of a 160M model is launches and their latency: what runs on one row is fused into three launches a block (both norms,
+// the attention's input product and the MLP's with gelu; RoPE, cache append and attention; both output products with the
+// residual adds), 38 a token.
 // Per-op arithmetic is the reference's: fp32 products and sums, no bf16 rounding anywhere:
 //   lga_f32_linear          F.linear (lit_gpt/model.py:619, 656, 699-702, 519): y = x W^T (+ b) (+ residual)
 //   lga_f32_layernorm       torch.nn.LayerNorm (GPT-NeoX norm_class, config.py:137-144): two-pass mean / biased var
 //                           (lga_f32_linear_act: with gelu and a second residual, lga_f32_layernorm_pair: two norms of a row)
+//   lga_f32_norm_linears    one row's norms and the products that read them (the next two lines' numbers)
+//   lga_f32_linears_sum     one row: two products and the residual adds of a parallel-residual block
 //   lga_f32_gelu            F.gelu exact (erf) or tanh (GptNeoxMLP, model.py:699-702)
 //   lga_f32_add             the Block's residual adds (model.py:584-593)
 //   lga_f32_rope_kv_append  apply_rope (model.py:767-773, partial rotary) + KVCache.forward (:788-795)
@@ -60,29 +63,23 @@ __global__ void __launch_bounds__(256) f32_linear_kernel(const float* __restrict
   }
 }
 
-// two norms of one row where w2 is given (a block whose attention and MLP read the same residual): the row stays in
-// registers (up to 256 CPT columns), mean and variance are made once per eps
+// Mean and biased variance of a row by a workgroup of 256, the first 256 CPT columns left in r
 template <int CPT>
-__global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                            const float* __restrict__ b, float* __restrict__ y, int n,
-                                                            float eps, const float* __restrict__ w2,
-                                                            const float* __restrict__ b2, float* __restrict__ y2, float eps2) {
-  const size_t row = blockIdx.x;
-  const float* xr = x + row * n;
-  __shared__ float red[4];
-  float r[CPT];
+__device__ __forceinline__ void f32_row_stats(const float* __restrict__ xr, int n, float (&r)[CPT], float (&red)[4],
+                                              float& mean, float& var) {
   float s = 0.0f;
 #pragma unroll
   for (int e = 0; e < CPT; ++e) {
     const int i = threadIdx.x + 256 * e;
     r[e] = i < n ? xr[i] : 0.0f;
-    s += r[e];
   }
+#pragma unroll
+  for (int e = 0; e < CPT; ++e) s += r[e];
   for (int i = threadIdx.x + 256 * CPT; i < n; i += 256) s += xr[i];
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  const float mean = ((red[0] + red[1]) + (red[2] + red[3])) / (float)n;
+  mean = ((red[0] + red[1]) + (red[2] + red[3])) / (float)n;
   __syncthreads();
   float ss = 0.0f;
 #pragma unroll
@@ -97,10 +94,28 @@ __global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restr
   ss = wave_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
-  const float var = ((red[0] + red[1]) + (red[2] + red[3])) / (float)n;
+  var = ((red[0] + red[1]) + (red[2] + red[3])) / (float)n;
+}
+__device__ __forceinline__ float f32_normed(float v, float mean, float rstd, float w, bool biased, float b) {
+  const float o = mul_rn(mul_rn(v - mean, rstd), w);
+  return biased ? add_rn(o, b) : o;
+}
+
+// two norms of one row where w2 is given (a block whose attention and MLP read the same residual): the row stays in
+// registers (up to 256 CPT columns), mean and variance are made once per eps
+template <int CPT>
+__global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                            const float* __restrict__ b, float* __restrict__ y, int n,
+                                                            float eps, const float* __restrict__ w2,
+                                                            const float* __restrict__ b2, float* __restrict__ y2, float eps2) {
+  const size_t row = blockIdx.x;
+  const float* xr = x + row * n;
+  __shared__ float red[4];
+  float r[CPT];
+  float mean, var;
+  f32_row_stats<CPT>(xr, n, r, red, mean, var);
   auto put = [&](const float* w_, const float* b_, float rstd, float* y_, int i, float v) {
-    const float o = mul_rn(mul_rn(v - mean, rstd), w_[i]);
-    y_[row * n + i] = b_ ? add_rn(o, b_[i]) : o;
+    y_[row * n + i] = f32_normed(v, mean, rstd, w_[i], b_, b_ ? b_[i] : 0.0f);
   };
   const float rstd = 1.0f / sqrtf(var + eps), rstd2 = w2 ? 1.0f / sqrtf(var + eps2) : 0.0f;
 #pragma unroll
@@ -114,6 +129,178 @@ __global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restr
   for (int i = threadIdx.x + 256 * CPT; i < n; i += 256) {
     put(w, b, rstd, y, i, xr[i]);
     if (w2) put(w2, b2, rstd2, y2, i, xr[i]);
+  }
+}
+
+// One row, K a multiple of 4: up to two products of a norm of the row each (f32_linear_kernel of f32_layernorm_kernel's row, to
+// the bit). A workgroup makes its norm anew, in LDS, while its first weights are on their way; a wave then one output after the
+// other. pythia-160m (768 -> 2304 and 3072): norms and products in three launches 16.2 us, in this one 7.6.
+struct F32NormLinear {
+  const float *nw, *nb;
+  float eps;
+  const float *w, *b;
+  int act;
+  float* y;
+  int N, blocks;
+};
+struct F32NormLinears {
+  const float* x;
+  int K;
+  F32NormLinear p[2];
+};
+constexpr int kF32Chunks = 4;  // 256 columns each: a wave's loads in flight
+__device__ __forceinline__ void f32_load_chunks(const float* row, int c0, int K, int lane, float4 (&v)[kF32Chunks]) {
+#pragma unroll
+  for (int c = 0; c < kF32Chunks; ++c) {
+    const int k = (c0 + c) * 256 + lane * 4;
+    if (k < K) v[c] = *(const float4*)(row + k);
+  }
+}
+__device__ __forceinline__ float f32_dot_chunks(const float* xr, int c0, int K, int lane, const float4 (&w)[kF32Chunks], float acc) {
+#pragma unroll
+  for (int c = 0; c < kF32Chunks; ++c) {
+    const int k = (c0 + c) * 256 + lane * 4;
+    if (k < K) {
+      const float4 x = *(const float4*)(xr + k);
+      acc = fmaf(x.w, w[c].w, fmaf(x.z, w[c].z, fmaf(x.y, w[c].y, fmaf(x.x, w[c].x, acc))));
+    }
+  }
+  return acc;
+}
+template <int CPT>
+__global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a) {
+  extern __shared__ __attribute__((aligned(16))) float xn[];  // [K]
+  __shared__ float red[4];
+  const bool second = (int)blockIdx.x >= a.p[0].blocks;
+  const F32NormLinear p = second ? a.p[1] : a.p[0];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, K = a.K;
+  int n = ((int)blockIdx.x - (second ? a.p[0].blocks : 0)) * 4 + wave;
+  float4 w[kF32Chunks];
+  if (n < p.N) f32_load_chunks(p.w + (size_t)n * K, 0, K, lane, w);
+  float bias = n < p.N && p.b ? p.b[n] : 0.0f;
+  float r[CPT], nw[CPT], nb[CPT], mean, var;
+#pragma unroll
+  for (int e = 0; e < CPT; ++e) {
+    const int i = threadIdx.x + 256 * e;
+    nw[e] = i < K ? p.nw[i] : 0.0f;
+    nb[e] = i < K && p.nb ? p.nb[i] : 0.0f;
+  }
+  f32_row_stats<CPT>(a.x, K, r, red, mean, var);
+  const float rstd = 1.0f / sqrtf(var + p.eps);
+#pragma unroll
+  for (int e = 0; e < CPT; ++e) {
+    const int i = threadIdx.x + 256 * e;
+    if (i < K) xn[i] = f32_normed(r[e], mean, rstd, nw[e], p.nb, nb[e]);
+  }
+  for (int i = threadIdx.x + 256 * CPT; i < K; i += 256) xn[i] = f32_normed(a.x[i], mean, rstd, p.nw[i], p.nb, p.nb ? p.nb[i] : 0.0f);
+  __syncthreads();
+  for (const int step = p.blocks * 4; n < p.N; n += step) {
+    float acc = 0.0f;
+    for (int c0 = 0; c0 * 256 < K; c0 += kF32Chunks) {
+      acc = f32_dot_chunks(xn, c0, K, lane, w, acc);
+      const bool more = (c0 + kF32Chunks) * 256 < K;
+      if (more || n + step < p.N) f32_load_chunks(p.w + (size_t)(more ? n : n + step) * K, more ? c0 + kF32Chunks : 0, K, lane, w);
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) {
+      if (p.b) acc += bias;
+      if (p.act) acc = gelu_f32(acc, p.act == 2);
+      p.y[n] = acc;
+    }
+    bias = n + step < p.N && p.b ? p.b[n + step] : 0.0f;
+  }
+}
+
+// One row: y = ((x2 W2^T + b2) + (x1 W1^T + b1)) + res, a wave per output, both products in f32_linear_kernel's order. Bound by
+// one round of latency: all loads of a block of 768 columns beside 3072 are in flight at once. Two launches 13.7 us, one 8.0 (8.9 with ranges of keys to join).
+struct F32LinearsSum {
+  const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
+  float* y;
+  int N, K1, K2;
+  // parts > 1: x1 is [parts][K1], an attention's sums over ranges of its keys, ml [parts][K1 / hs][2] (f32_attention_vec_kernel)
+  const float* ml;
+  int parts, hs;
+};
+// x1 of ranges of keys, joined in LDS: the ranges' sums weighted by exp(their largest score - the largest of all)
+__device__ __forceinline__ void f32_join_parts(const F32LinearsSum& a, float* xs, float* wt) {
+  constexpr int E = 4, P = 8;
+  const int H = a.K1 / a.hs;
+  float o[E][P];
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      const int i = threadIdx.x + 256 * e;
+      o[e][s] = i < a.K1 && s < a.parts ? a.x1[(size_t)s * a.K1 + i] : 0.0f;
+    }
+  for (int h = threadIdx.x; h < H; h += 256) {
+    float m[P], l[P], most = -INFINITY, sum = 0.0f;
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      m[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2] : -INFINITY;
+      l[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2 + 1] : -1.0f;
+      most = fmaxf(most, m[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      const bool empty = l[s] < 0.0f;
+      const float w = empty ? -1.0f : (m[s] == -INFINITY ? 0.0f : expf(m[s] - most));
+      if (!empty) sum = fmaf(w, l[s], sum);
+      wt[h * (P + 1) + s] = w;
+    }
+    wt[h * (P + 1) + P] = sum;
+  }
+  __syncthreads();
+  auto join = [&](int i, auto&& at) {
+    const float* w = wt + i / a.hs * (P + 1);
+    float acc = 0.0f;
+#pragma unroll
+    for (int s = 0; s < P; ++s)
+      if (!(w[s] < 0.0f)) acc = fmaf(w[s], at(s), acc);
+    xs[i] = acc / w[P];
+  };
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = threadIdx.x + 256 * e;
+    if (i < a.K1) join(i, [&](int s) { return o[e][s]; });
+  }
+  for (int i = threadIdx.x + 256 * E; i < a.K1; i += 256) join(i, [&](int s) { return a.x1[(size_t)s * a.K1 + i]; });
+  __syncthreads();
+}
+template <bool PARTS>
+__global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
+  extern __shared__ __attribute__((aligned(16))) float xs[];  // [K1] the joined row, then the ranges' weights
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), n = min(row, a.N - 1);
+  const float *r1 = a.w1 + (size_t)n * a.K1, *r2 = a.w2 + (size_t)n * a.K2;
+  float4 w1[kF32Chunks], w2[3][kF32Chunks];
+  f32_load_chunks(r1, 0, a.K1, lane, w1);
+#pragma unroll
+  for (int u = 0; u < 3; ++u) f32_load_chunks(r2, u * kF32Chunks, a.K2, lane, w2[u]);
+  const float b1 = a.b1 ? a.b1[n] : 0.0f, b2 = a.b2 ? a.b2[n] : 0.0f, res = a.res[n];
+  const float* x1 = a.x1;
+  if (PARTS) {
+    f32_join_parts(a, xs, xs + a.K1);
+    x1 = xs;
+  }
+  float h = 0.0f, m = 0.0f;
+  for (int c0 = 0; c0 * 256 < a.K1; c0 += kF32Chunks) {
+    if (c0 > 0) f32_load_chunks(r1, c0, a.K1, lane, w1);
+    h = f32_dot_chunks(x1, c0, a.K1, lane, w1, h);
+  }
+  for (int c0 = 0; c0 * 256 < a.K2; c0 += 3 * kF32Chunks) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      if (c0 > 0) f32_load_chunks(r2, c0 + u * kF32Chunks, a.K2, lane, w2[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 3; ++u) m = f32_dot_chunks(a.x2, c0 + u * kF32Chunks, a.K2, lane, w2[u], m);
+  }
+  h = wave_sum(h), m = wave_sum(m);
+  if (lane == 0 && row < a.N) {
+    if (a.b1) h += b1;
+    if (a.b2) m += b2;
+    m += h;
+    a.y[n] = m + res;
   }
 }
 
@@ -186,27 +373,40 @@ struct F32AttnArgs {
   const int64_t* rope_pos;  // fused only
   const float *cos, *sin;
   int n_elem, rope_rows;
+  int parts;  // ranges of the keys (fused only), beyond one:
+  float* ml;  // [parts][H][2] the largest score and the sum of the weights; y holds [parts][H * hs] sums of weighted values
 };
+
+__host__ __device__ inline int f32_attention_chunk(int keys, int parts) { return ((keys + parts - 1) / parts + 31) / 32 * 32; }
 
 // grid (T, H): softmax(q . K^T * scale) . V over keys 0..pos[t] of the query's group; scores kept in LDS, exact max, fp32
 // exp and sums. LPK adjacent lanes hold a key's or value's row in pieces of four (hs <= 4 LPK), the other lanes of the 8
 // waves other keys, four rows of each in flight. FUSED (one token): RoPE on q and on the group's k, which go with v to the
 // caches at position pos[0] and into LDS, in the same launch. Latency-bound at decode sizes (300 keys of 64 per head are
-// 150 KB): one key per wave at a time took 80 us, this form 9 beside the rotation and the append.
+// 150 KB): one key per wave at a time took 80 us, this form 9 beside the rotation and the append. A workgroup's loads bring some
+// 20 GB/s, so that the fused form takes the keys in ranges side by side (grid (parts, H)), whose sums f32_linears_sum_kernel
+// joins; pythia-160m at 301 keys 12.2 us in one range, 7.8 in five.
 template <int LPK, bool FUSED>
 __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   extern __shared__ float sc[];  // [max_seq] scores, then [8][hs] partial sums
   __shared__ float red[8];
   __shared__ __attribute__((aligned(16))) float qs[256], ks[256], vs[256];
   constexpr int KPW = 64 / LPK, STEP = 8 * KPW;
-  const int t = blockIdx.x, h = blockIdx.y, qpk = a.H / a.G, g = h / qpk, hs = a.hs;
+  const int t = FUSED ? 0 : blockIdx.x, range = FUSED ? blockIdx.x : 0, h = blockIdx.y, qpk = a.H / a.G, g = h / qpk, hs = a.hs;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane % LPK, first = wave * KPW + lane / LPK;
   const long p = a.pos[t];
   float* kb = a.kc + (size_t)g * a.max_seq * hs;
   float* vb = a.vc + (size_t)g * a.max_seq * hs;
+  const int L = (int)min(max(p + 1, 1L), (long)a.max_seq);
+  // this workgroup's keys: ranges of whole steps of the 32 keys of the narrowest rows, as many as there are keys for
+  const int chunk = FUSED && a.parts > 1 ? f32_attention_chunk(L, a.parts) : L, lo = range * chunk, hi = min(lo + chunk, L);
   if (FUSED) {
     const long rp = a.rope_pos[0];
     if (p < 0 || p >= a.max_seq || rp < 0 || rp >= a.rope_rows) return;  // host validates; never go out of bounds
+    if (lo >= L) {  // (an empty range: a sum below zero)
+      if (threadIdx.x == 0) a.ml[((size_t)range * a.H + h) * 2] = -INFINITY, a.ml[((size_t)range * a.H + h) * 2 + 1] = -1.0f;
+      return;
+    }
     const float* src = a.q + (size_t)g * (qpk + 2) * hs;
     const float *cr = a.cos + (size_t)rp * a.n_elem, *sr = a.sin + (size_t)rp * a.n_elem;
     for (int d = threadIdx.x; d < hs; d += 512) {
@@ -214,7 +414,7 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
       const float k = rope_f32(src + (size_t)qpk * hs, d, a.n_elem, cr, sr), v = src[(size_t)(qpk + 1) * hs + d];
       ks[d] = k;
       vs[d] = v;
-      if (h % qpk == 0) {
+      if (h % qpk == 0 && hi == L) {
         kb[(size_t)p * hs + d] = k;
         vb[(size_t)p * hs + d] = v;
       }
@@ -224,7 +424,6 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
     for (int d = threadIdx.x; d < hs; d += 512) qs[d] = qr[d];
   }
   __syncthreads();
-  const int L = (int)min(max(p + 1, 1L), (long)a.max_seq);
   const bool mine = sub * 4 < hs;
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
   const float4 q4 = mine ? *(const float4*)(qs + sub * 4) : zero;
@@ -234,7 +433,7 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
     return *(const float4*)(base + (size_t)min(j, L - 1) * hs + sub * 4);
   };
   float mx = -INFINITY;
-  for (int j0 = first; j0 < L; j0 += 4 * STEP) {
+  for (int j0 = lo + first; j0 < hi; j0 += 4 * STEP) {
     float4 k[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) k[u] = row(kb, ks, j0 + u * STEP);
@@ -243,9 +442,9 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
       float d = fmaf(q4.w, k[u].w, fmaf(q4.z, k[u].z, fmaf(q4.y, k[u].y, q4.x * k[u].x)));
       d = group_sum<LPK>(d) * a.scale;
       const int j = j0 + u * STEP;
-      if (j < L) {
+      if (j < hi) {
         mx = fmaxf(mx, d);
-        if (sub == 0) sc[j] = d;
+        if (sub == 0) sc[j - lo] = d;
       }
     }
   }
@@ -256,8 +455,9 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   for (int w = 0; w < 8; ++w) mx = fmaxf(mx, red[w]);
   __syncthreads();
   float sum = 0.0f;
-  for (int j = threadIdx.x; j < L; j += 512) {
-    const float e = expf(sc[j] - mx);
+  const float from = FUSED && a.parts > 1 && mx == -INFINITY ? 0.0f : mx;  // (other ranges may have finite scores)
+  for (int j = threadIdx.x; j < hi - lo; j += 512) {
+    const float e = expf(sc[j] - from);
     sc[j] = e;
     sum += e;
   }
@@ -266,15 +466,15 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   __syncthreads();
   sum = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
   float4 o = zero;
-  for (int j0 = first; j0 < L; j0 += 4 * STEP) {
+  for (int j0 = lo + first; j0 < hi; j0 += 4 * STEP) {
     float4 v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) v[u] = row(vb, vs, j0 + u * STEP);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int j = j0 + u * STEP;
-      const float w = j < L ? sc[j] : 0.0f;
-      if (j < L) o.x = fmaf(w, v[u].x, o.x), o.y = fmaf(w, v[u].y, o.y), o.z = fmaf(w, v[u].z, o.z), o.w = fmaf(w, v[u].w, o.w);
+      const float w = j < hi ? sc[j - lo] : 0.0f;
+      if (j < hi) o.x = fmaf(w, v[u].x, o.x), o.y = fmaf(w, v[u].y, o.y), o.z = fmaf(w, v[u].z, o.z), o.w = fmaf(w, v[u].w, o.w);
     }
   }
 #pragma unroll
@@ -292,14 +492,19 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
     float acc = 0.0f;
 #pragma unroll
     for (int w = 0; w < 8; ++w) acc += part[w * hs + d];
-    a.y[((size_t)t * a.H + h) * hs + d] = acc / sum;
+    a.y[((size_t)(t + range) * a.H + h) * hs + d] = FUSED && a.parts > 1 ? acc : acc / sum;
+  }
+  if (FUSED && a.parts > 1 && threadIdx.x == 0) {
+    a.ml[((size_t)range * a.H + h) * 2] = mx;
+    a.ml[((size_t)range * a.H + h) * 2 + 1] = sum;
   }
 }
 
 template <bool FUSED>
 static void f32_attention_go(const F32AttnArgs& a, int T, hipStream_t stream) {
-  const size_t lds = sizeof(float) * (size_t)std::max(a.max_seq, 8 * a.hs);
-  const dim3 grid(T, a.H);
+  const int keys = a.parts > 1 ? f32_attention_chunk(a.max_seq, a.parts) : a.max_seq;
+  const size_t lds = sizeof(float) * (size_t)std::max(keys, 8 * a.hs);
+  const dim3 grid(FUSED ? a.parts : T, a.H);
   if (a.hs <= 64) f32_attention_vec_kernel<16, FUSED><<<grid, 512, lds, stream>>>(a);
   else if (a.hs <= 128) f32_attention_vec_kernel<32, FUSED><<<grid, 512, lds, stream>>>(a);
   else f32_attention_vec_kernel<64, FUSED><<<grid, 512, lds, stream>>>(a);
@@ -376,6 +581,38 @@ extern "C" int lga_f32_linear_act(const float* x, const float* w, const float* b
   LGA_LAUNCH_RETURN();
 }
 
+extern "C" int lga_f32_norm_linears(const float* x, int K, const float* nw1, const float* nb1, float eps1, const float* w1,
+                                    const float* b1, int act1, float* y1, int N1, const float* nw2, const float* nb2,
+                                    float eps2, const float* w2, const float* b2, int act2, float* y2, int N2,
+                                    hipStream_t stream) {
+  LGA_CHECK_ARG(x && nw1 && w1 && y1 && K > 0 && N1 > 0 && N2 >= 0 && (N2 == 0 || (nw2 && w2 && y2)) && act1 >= 0 && act1 <= 2 &&
+                    act2 >= 0 && act2 <= 2,
+                "lga_f32_norm_linears: bad arguments");
+  LGA_CHECK_ARG(K % 4 == 0 && K <= 8192 && ((uintptr_t)w1 | (uintptr_t)w2) % 16 == 0,
+                "lga_f32_norm_linears: K a multiple of 4 up to 8192 and 16-B aligned weights needed");
+  // (2048 workgroups fill the chip: beyond, a workgroup's norm serves several outputs a wave)
+  auto blocks = [](int N) { return std::min((N + 3) / 4, 2048); };
+  const lga::F32NormLinears a{x, K, {{nw1, nb1, eps1, w1, b1, act1, y1, N1, blocks(N1)}, {nw2, nb2, eps2, w2, b2, act2, y2, N2, blocks(N2)}}};
+  const unsigned grid = (unsigned)(blocks(N1) + blocks(N2));
+  if (K <= 1024) lga::f32_norm_linears_kernel<4><<<grid, 256, K * sizeof(float), stream>>>(a);
+  else lga::f32_norm_linears_kernel<16><<<grid, 256, K * sizeof(float), stream>>>(a);
+  LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lga_f32_linears_sum(const float* x1, const float* ml, int parts, int hs, const float* w1, const float* b1, int K1,
+                                   const float* x2, const float* w2, const float* b2, int K2, const float* residual, float* y,
+                                   int N, hipStream_t stream) {
+  LGA_CHECK_ARG(x1 && w1 && x2 && w2 && residual && y && N > 0 && K1 > 0 && K2 > 0, "lga_f32_linears_sum: bad arguments");
+  LGA_CHECK_ARG(K1 % 4 == 0 && K2 % 4 == 0 && ((uintptr_t)x1 | (uintptr_t)w1 | (uintptr_t)x2 | (uintptr_t)w2) % 16 == 0,
+                "lga_f32_linears_sum: K in multiples of 4 and 16-B aligned operands needed");
+  LGA_CHECK_ARG(parts == 1 || (parts > 1 && parts <= 8 && ml && hs > 0 && K1 % hs == 0 && K1 <= 8192 && K1 / hs <= 256),
+                "lga_f32_linears_sum: 1 to 8 ranges of up to 256 heads, 8192 columns");
+  const lga::F32LinearsSum a{x1, w1, b1, x2, w2, b2, residual, y, N, K1, K2, ml, parts, hs};
+  if (parts > 1) lga::f32_linears_sum_kernel<true><<<(N + 3) / 4, 256, (K1 + K1 / hs * 9) * sizeof(float), stream>>>(a);
+  else lga::f32_linears_sum_kernel<false><<<(N + 3) / 4, 256, 0, stream>>>(a);
+  LGA_LAUNCH_RETURN();
+}
+
 extern "C" int lga_f32_linear(const float* x, const float* w, const float* bias, const float* residual, float* y,
                               int M, int N, int K, hipStream_t stream) {
   return lga_f32_linear_act(x, w, bias, 0, residual, nullptr, y, M, N, K, stream);
@@ -432,7 +669,7 @@ extern "C" int lga_f32_attention(const float* q, const float* k_cache, const flo
   LGA_CHECK_ARG(max_seq > 0 && max_seq <= 32768, "lga_f32_attention: max_seq must be in [1, 32768] (scores in LDS)");
   if (head_size % 4 == 0 && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0) {
     const lga::F32AttnArgs a{q, (float*)k_cache, (float*)v_cache, input_pos, y, n_head, n_query_groups, head_size, max_seq, scale,
-                             nullptr, nullptr, nullptr, 0, 0};
+                             nullptr, nullptr, nullptr, 0, 0, 1, nullptr};
     lga::f32_attention_go<false>(a, T, stream);
     LGA_LAUNCH_RETURN();
   }
@@ -442,19 +679,33 @@ extern "C" int lga_f32_attention(const float* q, const float* k_cache, const flo
   LGA_LAUNCH_RETURN();
 }
 
-extern "C" int lga_f32_attention_decode(const float* qkv, float* k_cache, float* v_cache, const int64_t* cache_pos,
-                                        const int64_t* rope_pos, const float* cos, const float* sin, int rope_rows, float* y,
-                                        int n_head, int n_query_groups, int head_size, int rope_n_elem, int max_seq,
-                                        float scale, hipStream_t stream) {
+extern "C" int lga_f32_attention_decode_parts(const float* qkv, float* k_cache, float* v_cache, const int64_t* cache_pos,
+                                              const int64_t* rope_pos, const float* cos, const float* sin, int rope_rows,
+                                              float* y, float* ml, int parts, int n_head, int n_query_groups, int head_size,
+                                              int rope_n_elem, int max_seq, float scale, hipStream_t stream) {
   LGA_CHECK_ARG(qkv && k_cache && v_cache && cache_pos && rope_pos && cos && sin && y,
                 "lga_f32_attention_decode: null pointer");
+  LGA_CHECK_ARG(parts == 1 || (parts > 1 && parts <= 8 && ml), "lga_f32_attention_decode: 1 to 8 ranges");
   LGA_CHECK_ARG(n_query_groups > 0 && n_head > 0 && n_head <= 65535 && n_head % n_query_groups == 0 && head_size > 0 &&
                     head_size <= 256 && head_size % 4 == 0 && rope_n_elem >= 0 && rope_n_elem % 2 == 0 &&
                     rope_n_elem <= head_size && rope_rows > 0 && max_seq > 0 && max_seq <= 32768,
                 "lga_f32_attention_decode: bad geometry (head_size a multiple of 4 up to 256, max_seq <= 32768)");
   LGA_CHECK_ARG(((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0, "lga_f32_attention_decode: aligned caches");
   const lga::F32AttnArgs a{qkv, k_cache, v_cache, cache_pos, y, n_head, n_query_groups, head_size, max_seq, scale,
-                           rope_pos, cos, sin, rope_n_elem, rope_rows};
+                           rope_pos, cos, sin, rope_n_elem, rope_rows, parts, ml};
   lga::f32_attention_go<true>(a, 1, stream);
   LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lga_f32_attention_parts(int n_head, int max_seq) {
+  // (ranges of 64 keys or more; eight are joined in one round of loads)
+  return n_head > 0 && max_seq > 0 ? std::min(8, (max_seq + 63) / 64) : 0;
+}
+
+extern "C" int lga_f32_attention_decode(const float* qkv, float* k_cache, float* v_cache, const int64_t* cache_pos,
+                                        const int64_t* rope_pos, const float* cos, const float* sin, int rope_rows, float* y,
+                                        int n_head, int n_query_groups, int head_size, int rope_n_elem, int max_seq,
+                                        float scale, hipStream_t stream) {
+  return lga_f32_attention_decode_parts(qkv, k_cache, v_cache, cache_pos, rope_pos, cos, sin, rope_rows, y, nullptr, 1, n_head,
+                                        n_query_groups, head_size, rope_n_elem, max_seq, scale, stream);
 }

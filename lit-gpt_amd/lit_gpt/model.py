@@ -205,7 +205,12 @@ class GPT(nn.Module):
         ln = self.transformer.ln_f
         if isinstance(ln, RMSNorm):
             return _lin(self.lm_head, x, norm_weight=ln.weight, norm_eps=ln.eps)
-        return _lin(self.lm_head, ln(x))
+        head = self.lm_head
+        if x.dtype == torch.float32 and x.shape[1] == 1 and type(ln) is LayerNorm and type(head) is nn.Linear and \
+                not hooked(ln, head) and all(t is None or (t.dtype == torch.float32 and t.is_contiguous()) for t in
+                                             (ln.weight, ln.bias, head.weight, head.bias)) and ops.f32_row_fusable(head.weight):
+            return ops.f32_norm_linears(x.contiguous(), (ln, head, None))[0].view(1, 1, -1)
+        return _lin(head, ln(x))
 
     @classmethod
     def from_name(cls, name: str, **kwargs: Any) -> "GPT":
@@ -287,6 +292,18 @@ class Block(nn.Module):
         return all(t is None or (t.dtype == torch.float32 and t.is_contiguous()) for t in ts) and \
             m.config.gelu_approximate in ("none", "tanh")
 
+    def _fuses_f32_row(self, x2: torch.Tensor) -> bool:
+        """Whether a block that fuses in fp32 (_fuses_f32) also computes past its attention's projections: one token, plain fp32
+        linears without forward hooks over the attention's cache."""
+        t = self.attn
+        if x2.shape[0] != 1 or type(t) is not CausalSelfAttention or type(t.attn) is not nn.Linear or type(t.proj) is not nn.Linear or \
+                hooked(t, t.attn, t.proj):
+            return False
+        ws = (t.attn.weight, t.proj.weight, self.mlp.fc.weight, self.mlp.proj.weight)
+        bs = (t.attn.bias, t.proj.bias)
+        return all(w.dtype == torch.float32 and w.is_contiguous() for w in ws) and \
+            all(b is None or (b.dtype == torch.float32 and b.is_contiguous()) for b in bs) and ops.f32_row_fusable(*ws)
+
     def _parallel_forward(self, x, cos, sin, mask, input_pos) -> torch.Tensor:
         """GPT-NeoX block (reference model.py:572-593, parallel_residual): n_1 = norm_1(x), h = attn(n_1),
         n_2 = n_1 if shared_attention_norm else norm_2(x), x = mlp(n_2) + h + x — the reference's association:
@@ -295,6 +312,10 @@ class Block(nn.Module):
         if self._fuses_f32(x):  # 32-true: both norms in one launch, gelu and the two adds in the products' epilogues
             x2 = x.reshape(-1, x.shape[-1]).contiguous()
             a, b, mlp = self.norm_1, self.norm_2, self.mlp
+            if self._fuses_f32_row(x2):  # one token: the norms in the input products' launch, one launch for the output products
+                qkv, g = ops.f32_norm_linears(x2, (a, self.attn.attn, None), (b, mlp.fc, mlp.config.gelu_approximate))
+                y = self.attn.attend(qkv, cos, sin, input_pos, in_parts=True)
+                return ops.f32_linears_sum(y, self.attn.proj, g, mlp.proj, x2).view_as(x)
             n_1, n_2 = ops.f32_layernorm_pair(x2, a.weight, a.bias, a.eps, b.weight, b.bias, b.eps)
             h = self.attn(n_1.view_as(x), cos, sin, mask, input_pos).contiguous()
             g = ops.f32_linear(n_2, mlp.fc.weight, bias=mlp.fc.bias, gelu=mlp.config.gelu_approximate)
@@ -329,11 +350,18 @@ class CausalSelfAttention(nn.Module):
         GEMV prologue, the residual add (and under TP the all-reduce hook ``reduce``) in the proj epilogue. Without
         them this is the reference forward."""
         B, T, C = x.size()
-        c = self.config
-        H, G, hs = c.n_head, c.n_query_groups, c.head_size
         qkv = _lin(self.attn, x, norm_weight=None if norm is None else norm.weight,
-                   norm_eps=c.norm_eps if norm is None else norm.eps).view(T, -1)
-        dev = x.device
+                   norm_eps=self.config.norm_eps if norm is None else norm.eps).view(T, -1)
+        y = self.attend(qkv, cos, sin, input_pos)
+        out = _lin(self.proj, y.view(1, T, -1), residual=residual, reduce=reduce)
+        return out.view(B, T, -1)
+
+    def attend(self, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, input_pos: Optional[torch.Tensor],
+               in_parts: bool = False):
+        """What lies between the two projections: (T, (H + 2 G) hs) -> (T, H hs), the cache extended. ``in_parts``: one fp32
+        token may come as the ranges of keys that ops.f32_linears_sum joins."""
+        c, T, dev = self.config, qkv.shape[0], qkv.device
+        H, G, hs = c.n_head, c.n_query_groups, c.head_size
         if input_pos is None:
             # no cache (training-style causal forward, model.py:510-513): a private cache of T rows
             pos = torch.arange(T, device=dev, dtype=torch.int64)
@@ -366,12 +394,13 @@ class CausalSelfAttention(nn.Module):
             y = ops.attention_decode_fused(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem,
                                            1.0 / math.sqrt(hs), n_splits, workspace=ws)
         elif T == 1 and self.fuse_decode and qkv.dtype == torch.float32 and ops.f32_decode_fusable(hs, S, kc, vc):
-            y = ops.f32_attention_decode(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem, 1.0 / math.sqrt(hs))
+            args = (qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem, 1.0 / math.sqrt(hs))
+            parts = ops.f32_attention_parts(H, S) if in_parts and H <= 256 else 1
+            y = ops.f32_attention_decode(*args) if parts == 1 else ops.f32_attention_decode_parts(*args, parts)
         else:
             q = ops.rope_kv_append(qkv, kc, vc, pos, rope_pos, cos, sin, H, G, hs, c.rope_n_elem)
             y = ops.attention(q, kc, vc, pos, H, G, hs, 1.0 / math.sqrt(hs), n_splits, workspace=ws)
-        out = _lin(self.proj, y.view(1, T, H * hs), residual=residual, reduce=reduce)
-        return out.view(B, T, -1)
+        return y
 
     def scaled_dot_product_attention(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                      mask: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -95,6 +95,10 @@ SIGNATURES = {
     "lga_allreduce_bf16": [_P, _P, _P, _I, ctypes.POINTER(_P), _I, _I, _I, _P, _P, _P],
     "lga_f32_linear": [_P, _P, _P, _P, _P, _I, _I, _I, _P],
     "lga_f32_linear_act": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _P],
+    "lga_f32_norm_linears": [_P, _I, _P, _P, _F, _P, _P, _I, _P, _I, _P, _P, _F, _P, _P, _I, _P, _I, _P],
+    "lga_f32_linears_sum": [_P, _P, _I, _I, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _P],
+    "lga_f32_attention_parts": [_I, _I],
+    "lga_f32_attention_decode_parts": [_P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P],
     "lga_f32_layernorm_pair": [_P, _P, _P, _P, _F, _P, _P, _P, _F, _I, _I, _P],
     "lga_f32_layernorm": [_P, _P, _P, _P, _I, _I, _F, _P],
     "lga_f32_gelu": [_P, _P, _L, _I, _P],
@@ -437,6 +441,25 @@ def f32_attention_decode(qkv, k_cache, v_cache, cache_pos, rope_pos, cos, sin, n
     return y
 
 
+def f32_attention_decode_parts(qkv, k_cache, v_cache, cache_pos, rope_pos, cos, sin, n_head, n_query_groups, head_size,
+                               rope_n_elem, scale, parts):
+    """``f32_attention_decode`` over ranges of the keys side by side, for ``f32_linears_sum`` to join: (their sums, their largest
+    scores and weights, head_size)."""
+    y = torch.empty(parts, n_head * head_size, dtype=torch.float32, device=qkv.device)
+    ml = torch.empty(parts, n_head, 2, dtype=torch.float32, device=qkv.device)
+    _check(load_library().lga_f32_attention_decode_parts(
+        _dev(qkv, "qkv", torch.float32), _dev(k_cache, "k_cache", torch.float32), _dev(v_cache, "v_cache", torch.float32),
+        _dev(cache_pos, "cache_pos", torch.int64), _dev(rope_pos, "rope_pos", torch.int64), _dev(cos, "cos", torch.float32),
+        _dev(sin, "sin", torch.float32), cos.shape[0], _dev(y, "y", torch.float32), _dev(ml, "ml", torch.float32), parts,
+        n_head, n_query_groups, head_size, rope_n_elem, k_cache.shape[-2], float(scale), _stream()))
+    return y, ml, head_size
+
+
+def f32_attention_parts(n_head: int, max_seq: int) -> int:
+    """How many ranges of a cache's keys pay beside one another in f32_attention_decode_parts."""
+    return load_library().lga_f32_attention_parts(n_head, max_seq)
+
+
 def attention_decode_fused(qkv, k_cache, v_cache, cache_pos, rope_pos, cos, sin, n_head, n_query_groups,
                            head_size, rope_n_elem, scale, n_splits=1, workspace: Optional[AttentionWorkspace] = None,
                            out=None):
@@ -635,6 +658,49 @@ def f32_layernorm_pair(x, weight, bias, eps, weight2, bias2, eps2):
         _dev(y, "y", torch.float32), float(eps), _dev(weight2, "weight2", torch.float32),
         _opt(bias2, "bias2", torch.float32), _dev(y2, "y2", torch.float32), float(eps2), x.numel() // n, n, _stream()))
     return y, y2
+
+
+_F32_ACT = {None: 0, "none": 1, "tanh": 2}
+
+
+def f32_row_fusable(*operands) -> bool:
+    """Whether f32_norm_linears and f32_linears_sum serve these matrices (and rows: 16-byte loads)."""
+    return all(t.shape[-1] % 4 == 0 and t.shape[-1] <= 8192 and t.data_ptr() % 16 == 0 for t in operands)
+
+
+def f32_norm_linears(x, first, second=None):
+    """One fp32 row, in one launch: for each of up to two (norm, linear, gelu) the linear of the LayerNorm of x, then gelu
+    ("none" / "tanh", None: no activation) — ``f32_linear`` of ``layernorm``, to the bit."""
+    K, args, outs = x.numel(), [], []
+    for part in (first, second):
+        if part is None:
+            args += [None, None, 0.0, None, None, 0, None, 0]
+            continue
+        norm, linear, gelu = part
+        y = torch.empty(1, linear.weight.shape[0], dtype=torch.float32, device=x.device)
+        args += [_dev(norm.weight, "norm weight", torch.float32), _opt(norm.bias, "norm bias", torch.float32), float(norm.eps),
+                 _dev(linear.weight, "weight", torch.float32), _opt(linear.bias, "bias", torch.float32), _F32_ACT[gelu],
+                 _dev(y, "y", torch.float32), y.shape[1]]
+        outs.append(y)
+    _check(load_library().lga_f32_norm_linears(_dev(x, "x", torch.float32), K, *args, _stream()))
+    return outs
+
+
+def f32_linears_sum(x1, linear1, x2, linear2, residual):
+    """One fp32 row, in one launch: (linear2(x2) + linear1(x1)) + residual. ``x1``: a row, or the ranges of
+    f32_attention_decode_parts."""
+    N, K1 = linear1.weight.shape
+    ml, parts, hs = None, 1, 0
+    if isinstance(x1, tuple):
+        x1, ml, hs = x1
+        parts = x1.shape[0]
+    y = torch.empty(1, N, dtype=torch.float32, device=x1.device)
+    _check(load_library().lga_f32_linears_sum(
+        _dev(x1, "x1", torch.float32), _opt(ml, "ml", torch.float32), parts, hs, _dev(linear1.weight, "weight1", torch.float32),
+        _opt(linear1.bias, "bias1", torch.float32), K1, _dev(x2, "x2", torch.float32),
+        _dev(linear2.weight, "weight2", torch.float32), _opt(linear2.bias, "bias2", torch.float32), linear2.weight.shape[1],
+        _dev(residual, "residual", torch.float32), _dev(y, "y", torch.float32), N, _stream()))
+    return y
 
 
 def argmax_embed(logits, table, emb_out, out_idx=None, token_out=None, pos_inout=None):

@@ -76,3 +76,106 @@ def test_caches_off_sixteen_bytes():
                 setattr(kv, n, torch.empty(t.numel() + off, device=dev)[off:].view(t.shape).copy_(t))
             outs.append(m(idx, pos).clone())
     assert float((outs[0] - outs[1]).abs().max()) < 1e-5 * float(outs[0].abs().max())
+
+
+@pytest.mark.parametrize("K,N1,N2", [(4, 1, 3), (252, 5, 0), (768, 2304, 3072), (1024, 4, 9), (1028, 6, 2), (4100, 7, 5), (8192, 3, 0),
+                                     (256, 8200, 33)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_one_row_norms_and_products(K, N1, N2, bias):
+    """One launch for two norms and their products, one for two products and the adds: the bits of the single kernels, at the edges of
+    256 columns a load, of the row's registers and of several outputs a wave."""
+    from types import SimpleNamespace as Part
+
+    from lit_gpt import ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(K + N1)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev)  # noqa: E731
+    x = draw(1, K)
+    norms = [Part(weight=draw(K), bias=draw(K) if bias else None, eps=e) for e in (1e-5, 1e-3)]
+    linears = [Part(weight=draw(n, K) * K ** -0.5, bias=draw(n) if bias else None) for n in (N1, max(N2, 1))]
+    parts = [(norms[0], linears[0], None)] + [(norms[1], linears[1], "tanh")] * (N2 > 0)
+    for y, (norm, linear, gelu) in zip(ops.f32_norm_linears(x, *parts), parts):
+        assert torch.equal(y, ops.f32_linear(ops.layernorm(x, norm.weight, norm.bias, norm.eps), linear.weight, linear.bias, gelu=gelu))
+    x2, res = draw(1, 3 * K), draw(1, N1)
+    wide = Part(weight=draw(N1, 3 * K) * K ** -0.5, bias=draw(N1) if bias else None)
+    h = ops.f32_linear(x, linears[0].weight, linears[0].bias)
+    want = ops.f32_linear(x2, wide.weight, wide.bias, residual=h, residual2=res)
+    assert torch.equal(ops.f32_linears_sum(x, linears[0], x2, wide, res), want)
+
+
+def test_one_token_past_the_modules():
+    """A block's three launches give the bits of its modules called one by one (a hook keeps them apart)."""
+    from generate.base import build_model
+    from lit_gpt import Config
+
+    dev = torch.device("cuda", 0)
+    m = build_model(Config.from_name("pythia-160m", n_layer=2), quantize=None, device=dev, seed=1, max_seq_length=64, dtype=torch.float32)
+    idx, pos, seen = torch.tensor([[5]], device=dev), torch.tensor([9], device=dev), []
+    for block in m.transformer.h:
+        block.attn.kv_cache.k.normal_(), block.attn.kv_cache.v.normal_()
+    with torch.inference_mode():
+        fused = m(idx, pos)
+        for module in (m.transformer.h[0].attn, m.transformer.h[1].attn.proj, m.transformer.ln_f):
+            handle = module.register_forward_hook(lambda mod, args, out: seen.append(type(mod).__name__))
+            assert torch.equal(m(idx, pos), fused)
+            handle.remove()
+    assert seen == ["CausalSelfAttention", "LayerNorm"]  # (a projection is no call of its module)
+
+
+@pytest.mark.parametrize("hs,H,G", [(64, 12, 12), (128, 4, 2), (4, 3, 1), (256, 9, 9)])
+@pytest.mark.parametrize("p0,S", [(0, 65), (31, 128), (32, 200), (63, 512), (300, 320), (511, 512), (1000, 2048)])
+def test_ranges_of_keys(hs, H, G, p0, S):
+    """Ranges of keys side by side, joined in the output product: ranges without keys, with one, and whole ones. Against float64: sums
+    of up to 1001 weighted values of size 1 and their products with a matrix of rows of length 1 (2e-6 and sqrt(K) 2^-24 of it)."""
+    from types import SimpleNamespace as Part
+
+    from lit_gpt import ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(hs + p0)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev)  # noqa: E731
+    k, v, qkv = draw(1, G, S, hs), draw(1, G, S, hs), draw(1, (H + 2 * G) * hs)
+    k[:, :, p0:], v[:, :, p0:] = float("nan"), float("nan")  # rows that nobody has written
+    pos = torch.tensor([p0], device=dev)
+    cos, sin = torch.ones(S, 2, device=dev), torch.zeros(S, 2, device=dev)
+    kb, vb = k.clone(), v.clone()
+    parts = ops.f32_attention_parts(H, S)
+    assert parts == min(8, -(-S // 64))
+    joined = ops.f32_attention_decode_parts(qkv, kb, vb, pos, pos, cos, sin, H, G, hs, 2, hs ** -0.5, parts)
+    y = ops.f32_attention_decode(qkv, k, v, pos, pos, cos, sin, H, G, hs, 2, hs ** -0.5)
+    assert torch.equal(k[:, :, : p0 + 1], kb[:, :, : p0 + 1]) and torch.equal(v[:, :, : p0 + 1], vb[:, :, : p0 + 1])
+    K = H * hs
+    one, two = Part(weight=draw(5, K) * K ** -0.5, bias=None), Part(weight=draw(5, 8), bias=draw(5))
+    x2, res = draw(1, 8), draw(1, 5)
+    q = qkv.view(G, H // G + 2, hs)[:, :-2].reshape(H, hs).double()
+    rows = torch.arange(H, device=dev) // (H // G)
+    s = torch.einsum("hd,hnd->hn", q, k[0, rows, : p0 + 1].double()) * hs ** -0.5
+    want = (torch.softmax(s, 1).unsqueeze(1) @ v[0, rows, : p0 + 1].double()).view(1, K)
+    end = x2.double() @ two.weight.double().T + two.bias.double() + res.double()
+    want = want @ one.weight.double().T + end
+    assert (ops.f32_linears_sum(joined, one, x2, two, res).double() - want).abs().max() < 1e-5
+    assert (ops.f32_linears_sum(y, one, x2, two, res).double() - want).abs().max() < 1e-5
+
+
+def test_ranges_of_infinite_scores():
+    """Scores of minus infinity throughout a range, and a NaN in one, as the unsplit form has them."""
+    from types import SimpleNamespace as Part
+
+    from lit_gpt import ops
+
+    dev, S, H, hs = torch.device("cuda", 0), 256, 2, 8
+    k, v = torch.ones(1, H, S, hs, device=dev), torch.rand(1, H, S, hs, device=dev)
+    k[0, 0, :64] = -float("inf")
+    k[0, 1, 70] = float("nan")
+    qkv, pos = torch.ones(1, 3 * H * hs, device=dev), torch.tensor([200], device=dev)
+    cos, sin = torch.ones(S, 2, device=dev), torch.zeros(S, 2, device=dev)
+    args = (qkv, k, v, pos, pos, cos, sin, H, H, hs, 2, 1.0)
+    eye, none = Part(weight=torch.eye(hs, device=dev), bias=None), Part(weight=torch.zeros(hs, 4, device=dev), bias=None)
+    want = ops.f32_attention_decode(*args).view(H, hs)
+    assert want[0].isfinite().all() and want[1].isnan().all()
+    y, ml, _ = ops.f32_attention_decode_parts(*args, 4)
+    for h in range(H):
+        head = y.view(4, H, hs)[:, h].contiguous(), ml[:, h: h + 1].contiguous(), hs
+        got = ops.f32_linears_sum(head, eye, torch.zeros(1, 4, device=dev), none, torch.zeros(1, hs, device=dev))[0]
+        assert got.isnan().all() if h else (got - want[0]).abs().max() < 1e-6
