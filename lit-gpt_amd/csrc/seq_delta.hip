@@ -430,6 +430,145 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
   }
 }
 
+// The same recurrence for key dims of 128 with 32 lanes a column, to the bits of gated_delta_kernel<2, 16>: of the four partial
+// sums per product there, ka + kb stand in one lane and kc + kd in its neighbour, whose sum is the first of the lane sums.
+//
+// A lone wave issues an instruction each five clocks, and a token is a chain of some 70 there, 490 clocks: with half of the rows
+// a lane has 48, 310 clocks, and a prompt of 16 heads one wave on each SIMD of the chip instead of one on every other. q, k and decays lie
+// in LDS as the lanes hold them (one 16-byte read each), v, beta and k . q of a token and column side by side. 2048 tokens of 16
+// heads of 128 x 128: 432 us before, 276 here; one token 6.6 / 5.2. Beyond 4096 columns the waves share their SIMDs and the fewer
+// instructions of the other form count: 2048 tokens of 32 heads 432 / 388, 1024 of 48 heads 259 / 302.
+//
+// grid (B * H * ceil(dv / 8) rounded up to 8). Lane l of a column: rows 64 j + 2 l + e, j, e < 2.
+template <bool DELTA>
+__global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
+  constexpr int D = 128, CW = 8, TB = 32, ROW = 3 * D + 4 * CW;  // staged floats per token: q | k | g | (v, beta, k . q, -) per column
+  __shared__ __attribute__((aligned(16))) float st[(TB + 1) * ROW];  // (a batch's last token reads one row ahead)
+  __shared__ float os[TB * CW];
+  const int tid = threadIdx.x, l = tid & 31, cw = tid >> 5;
+  const int per_xcd = (p.items + 7) / 8;  // (a head's column blocks on one XCD, as above)
+  const int item = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (item >= p.items) return;
+  const int cblk = item % p.ncb, hd = (item / p.ncb) % p.H, b = item / (p.ncb * p.H);
+  const int dv = p.dv, H = p.H, col = cblk * CW + cw;
+  const bool live = col < dv;
+  const int g = hd / (H / p.G);
+  const int r0 = p.seq_start[b], n = p.seq_start[b + 1] - r0;
+  float* sp = p.state + (((size_t)p.seq_slot[b] * H + hd) * D) * dv;
+  const bool fresh = p.seq_pos0[b] == 0;
+  auto row_of = [&](int i) { return 64 * (i >> 1) + 2 * l + (i & 1); };
+  float S[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) S[i] = !fresh && live ? sp[(size_t)row_of(i) * dv + col] : 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(S[i]));  // (as above: the loads of S end here)
+
+  // a thread stages the tokens cw, cw + 8, ... of a batch: q, k and decays of the rows of lane l; and one column's v, beta, k . q
+  // of one token
+  const float* qk = p.qkv + (size_t)r0 * p.ld;
+  const float* dec = p.dec + ((size_t)r0 * H + hd) * (p.per_channel ? D : 1);
+  const long dstep = (long)H * (p.per_channel ? D : 1);
+  const int vt = tid / CW, vc = cblk * CW + tid % CW;
+  float2 pre[TB / 8][3][2];
+  float vpre, bpre, kqpre;
+  auto prefetch = [&](int t0) {  // (past the end: the last token again)
+#pragma unroll
+    for (int u = 0; u < TB / 8; ++u) {
+      const int t = min(t0 + u * 8 + cw, n - 1);
+      const float *q = qk + t * p.ld + (size_t)g * D + 2 * l, *k = q + (size_t)p.G * D, *d = dec + t * dstep;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        pre[u][0][j] = *(const float2*)(q + 64 * j);
+        pre[u][1][j] = *(const float2*)(k + 64 * j);
+        pre[u][2][j] = p.per_channel ? *(const float2*)(d + 64 * j + 2 * l) : make_float2(d[0], d[0]);
+      }
+    }
+    const int t = min(t0 + vt, n - 1);
+    vpre = vc < dv ? qk[t * p.ld + (size_t)2 * p.G * D + (size_t)hd * dv + vc] : 0.0f;
+    bpre = DELTA ? p.beta[(size_t)(r0 + t) * H + hd] : 0.0f;
+    kqpre = p.kq[(size_t)(r0 + t) * p.G + g];
+  };
+  if (n > 0) prefetch(0);
+
+  struct Token {
+    float4 k, g, q, c;
+  };
+  auto fetch = [&](const float* row, Token& x) {
+    x.g = *(const float4*)(row + 2 * D + 4 * l);
+    x.k = *(const float4*)(row + D + 4 * l);
+    x.q = *(const float4*)(row + 4 * l);
+    x.c = *(const float4*)(row + 3 * D + 4 * cw);
+  };
+  auto one = [&](const Token& x) {
+    S[0] *= x.g.x, S[1] *= x.g.y, S[2] *= x.g.z, S[3] *= x.g.w;
+    float ks = 0.0f;
+    if (DELTA) ks = fmaf(S[2], x.k.z, fmaf(S[0], x.k.x, 0.0f)) + fmaf(S[3], x.k.w, fmaf(S[1], x.k.y, 0.0f));
+    float qs = fmaf(S[2], x.q.z, fmaf(S[0], x.q.x, 0.0f)) + fmaf(S[3], x.q.w, fmaf(S[1], x.q.y, 0.0f));
+    lanes_sum2<16>(ks, qs);
+    // the two rows of 16 lanes, both sums in one swap: even rows then hold ks of either row, odd ones qs; and back to all lanes
+    const auto halves = __builtin_amdgcn_permlane16_swap(__float_as_uint(ks), __float_as_uint(qs), false, false);
+    const float both = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+    const auto sums = __builtin_amdgcn_permlane16_swap(__float_as_uint(both), __float_as_uint(both), false, false);
+    ks = __uint_as_float(sums[0]), qs = __uint_as_float(sums[1]);
+    const float u = DELTA ? x.c.y * (x.c.x - ks) : x.c.x;
+    S[0] = fmaf(x.k.x, u, S[0]), S[1] = fmaf(x.k.y, u, S[1]), S[2] = fmaf(x.k.z, u, S[2]), S[3] = fmaf(x.k.w, u, S[3]);
+    return fmaf(u, x.c.z, qs);
+  };
+  for (int t0 = 0; t0 < n; t0 += TB) {
+    const int nb = min(TB, n - t0);
+    __syncthreads();  // the previous batch's reads of st and os are done
+#pragma unroll
+    for (int u = 0; u < TB / 8; ++u)
+#pragma unroll
+      for (int part = 0; part < 3; ++part)
+        *(float4*)(st + (u * 8 + cw) * ROW + part * D + 4 * l) =
+            make_float4(pre[u][part][0].x, pre[u][part][0].y, pre[u][part][1].x, pre[u][part][1].y);
+    *(float4*)(st + vt * ROW + 3 * D + 4 * (tid % CW)) = make_float4(vpre, bpre, kqpre, 0.0f);
+    __syncthreads();
+    if (t0 + TB < n) prefetch(t0 + TB);
+    Token x[2];
+    const float* row = st;
+    fetch(row, x[0]);
+    float keep = 0.0f;
+    if (nb == TB) {
+#pragma unroll 4
+      for (int t = 0; t < TB; t += 2) {
+        fetch(row + ROW, x[1]);
+        float o = one(x[0]);
+        if (t == l) keep = o;
+        row += 2 * ROW;
+        fetch(row, x[0]);
+        o = one(x[1]);
+        if (t + 1 == l) keep = o;
+      }
+    } else {
+      for (int t = 0; t < nb; ++t) {
+        row += ROW;
+        fetch(row, x[1]);
+        const float o = one(x[0]);
+        if (t == l) keep = o;
+        x[0] = x[1];
+      }
+    }
+    os[l * CW + cw] = keep;
+    __syncthreads();
+    if (vt < nb && vc < dv) p.out[(size_t)(r0 + t0 + vt) * H * dv + (size_t)hd * dv + vc] = os[tid];
+  }
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sp[(size_t)row_of(i) * dv + col] = S[i];
+  }
+}
+
+constexpr long kDeltaWideColumns = 4096;  // (the figures stand above)
+static void gated_delta_wide_launch(DeltaArgs p, int B, bool plain, hipStream_t stream) {
+  p.ncb = (p.dv + 7) / 8;
+  p.items = B * p.H * p.ncb;
+  const unsigned grid = (unsigned)((p.items + 7) / 8 * 8);
+  if (plain) gated_delta_wide_kernel<false><<<grid, 256, 0, stream>>>(p);
+  else gated_delta_wide_kernel<true><<<grid, 256, 0, stream>>>(p);
+}
+
 template <int LPC, bool DELTA>
 static bool gated_delta_launch(DeltaArgs p, int B, hipStream_t stream) {
   p.ncb = (p.dv + 256 / LPC - 1) / (256 / LPC);
@@ -512,6 +651,11 @@ extern "C" int lgs_gated_delta(const float* qkv, long ld, const float* dec, cons
   // lanes per column: more lanes shorten a token's dependent chain and multiply the waves; by default as many as
   // keep the launch within about two waves per SIMD, and at least enough for 32 rows per lane
   int lpc = lanes;
+  const bool pairs = ld % 2 == 0 && ((uintptr_t)qkv | (uintptr_t)dec) % 8 == 0;  // (loaded two floats at a time)
+  if (lanes == 0 && d == 128 && pairs && (long)B * H * dv <= lgs::kDeltaWideColumns) {
+    lgs::gated_delta_wide_launch(p, B, plain != 0, stream);
+    LGA_LAUNCH_RETURN();
+  }
   if (lpc == 0) {
     const long cols = (long)B * H * dv;
     lpc = cols * 16 / 64 <= 2048 ? 16 : cols * 8 / 64 <= 2048 ? 8 : 4;

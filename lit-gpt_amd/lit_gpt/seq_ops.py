@@ -1084,7 +1084,7 @@ def gated_delta(qkv: torch.Tensor, dec: torch.Tensor, beta: Optional[torch.Tenso
     """The gated delta rule over a packed batch, token by token: S <- diag(dec) S; u = beta (v - S^T k);
     S <- S + k u^T; o = S^T q. qkv (T, 2 G d + H dv) prepared rows, kq (T, G) their k . q (``delta_prepare``); state
     (slots, H, d, dv) fp32 is read unless a sequence starts at position 0 and left at the step's last token. Returns
-    o (T, H dv). ``lanes``: lanes that share one state column (4, 8, 16; 0: chosen from the sizes). ``plain``: the
+    o (T, H dv). ``lanes``: lanes that share one state column (4, 8, 16; 0: chosen from the sizes, 32 among them). ``plain``: the
     rule without the correction, S <- diag(dec) S + k v^T, o = S^T q (``beta`` None). ``qkv_off``: the first column of
     q | k | v in wider rows."""
     T, ld = qkv.shape

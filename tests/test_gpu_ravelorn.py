@@ -434,6 +434,31 @@ def test_delta_rule_kernel_every_form(H, G, d, dv, lanes, per_channel):
     assert torch.equal(sd[4].cpu(), state[4])  # a slot no sequence owns is left alone
 
 
+@pytest.mark.parametrize("per_channel,plain", [(True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("H,G,dv,extra,lens", [(2, 2, 40, 0, [1, 90, 17, 33]), (16, 16, 128, 0, [64]), (2, 1, 9, 2, [31, 32, 65]),
+                                               (3, 3, 3, 1, [5, 2]), (32, 8, 128, 0, [33])])
+def test_delta_rule_of_wide_heads_to_the_bit(H, G, dv, extra, lens, per_channel, plain):
+    """Heads of 128 rows of state, 32 lanes a column where few columns leave the chip idle: the bits of 16 lanes a column, over
+    batches of 32 tokens, columns past whole workgroups, and rows whose odd stride (extra + H dv) keeps the older form."""
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import StepBatch
+
+    dev, d, T = torch.device("cuda", 0), 128, sum(lens)
+    g = torch.Generator(device=dev).manual_seed(dv + T)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev)  # noqa: E731
+    slots, first = list(range(len(lens)))[::-1], [0, 5, 0, 40][: len(lens)]
+    step = StepBatch.build([(s, p, [0] * n) for s, p, n in zip(slots, first, lens)], dev)
+    qkv, state = draw(T, 2 * G * d + H * dv + extra) * d ** -0.5, draw(len(lens) + 1, H, d, dv)
+    dec = torch.rand(T, H * d if per_channel else H, generator=g, device=dev) * 0.5 + 0.5
+    beta, kq, res = torch.rand(T, H, generator=g, device=dev), draw(T, G), []
+    for lanes in (0, 16):
+        s = state.clone()
+        out = seq_ops.gated_delta(qkv, dec, None if plain else beta, kq, s, step.seq_start, step.seq_slot, step.seq_pos0, H=H, G=G,
+                                  d=d, dv=dv, per_channel=per_channel, lanes=lanes, plain=plain)
+        res.append((out, s))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+
+
 def test_delta_prepare():
     from lit_gpt import seq_ops
 
