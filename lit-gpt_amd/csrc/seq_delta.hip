@@ -433,14 +433,15 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
 // The same recurrence for key dims of 128 with 32 lanes a column, to the bits of gated_delta_kernel<2, 16>: of the four partial
 // sums per product there, ka + kb stand in one lane and kc + kd in its neighbour, whose sum is the first of the lane sums.
 //
-// A lone wave issues an instruction each five clocks, and a token is a chain of some 70 there, 490 clocks: with half of the rows
+// A lone wave issues an instruction each five clocks, and a token is a chain of some 70 there, 490 clocks. With half of the rows
 // a lane has 48, 310 clocks, and a prompt of 16 heads one wave on each SIMD of the chip instead of one on every other. q, k and decays lie
 // in LDS as the lanes hold them (one 16-byte read each), v, beta and k . q of a token and column side by side. 2048 tokens of 16
-// heads of 128 x 128: 432 us before, 276 here; one token 6.6 / 5.2. Beyond 4096 columns the waves share their SIMDs and the fewer
+// heads of 128 x 128: 430 us before, 270 to 280 here; one token 6.6 / 5.2. Beyond 4096 columns the waves share their SIMDs and the fewer
 // instructions of the other form count: 2048 tokens of 32 heads 432 / 388, 1024 of 48 heads 259 / 302.
 //
 // grid (B * H * ceil(dv / 8) rounded up to 8). Lane l of a column: rows 64 j + 2 l + e, j, e < 2.
-template <bool DELTA>
+// (PC: a decay per channel. The loads ahead carry no branches: behind one, every batch would wait for the next one's loads.)
+template <bool DELTA, bool PC>
 __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
   constexpr int D = 128, CW = 8, TB = 32, ROW = 3 * D + 4 * CW;  // staged floats per token: q | k | g | (v, beta, k . q, -) per column
   __shared__ __attribute__((aligned(16))) float st[(TB + 1) * ROW];  // (a batch's last token reads one row ahead)
@@ -466,11 +467,11 @@ __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
   // a thread stages the tokens cw, cw + 8, ... of a batch: q, k and decays of the rows of lane l; and one column's v, beta, k . q
   // of one token
   const float* qk = p.qkv + (size_t)r0 * p.ld;
-  const float* dec = p.dec + ((size_t)r0 * H + hd) * (p.per_channel ? D : 1);
-  const long dstep = (long)H * (p.per_channel ? D : 1);
+  const float* dec = p.dec + ((size_t)r0 * H + hd) * (PC ? D : 1);
+  const long dstep = (long)H * (PC ? D : 1);
   const int vt = tid / CW, vc = cblk * CW + tid % CW;
   float2 pre[TB / 8][3][2];
-  float vpre, bpre, kqpre;
+  float vpre, bpre = 0.0f, kqpre;
   auto prefetch = [&](int t0) {  // (past the end: the last token again)
 #pragma unroll
     for (int u = 0; u < TB / 8; ++u) {
@@ -480,12 +481,13 @@ __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
       for (int j = 0; j < 2; ++j) {
         pre[u][0][j] = *(const float2*)(q + 64 * j);
         pre[u][1][j] = *(const float2*)(k + 64 * j);
-        pre[u][2][j] = p.per_channel ? *(const float2*)(d + 64 * j + 2 * l) : make_float2(d[0], d[0]);
+        if constexpr (PC) pre[u][2][j] = *(const float2*)(d + 64 * j + 2 * l);
+        else pre[u][2][j].x = d[0];
       }
     }
     const int t = min(t0 + vt, n - 1);
-    vpre = vc < dv ? qk[t * p.ld + (size_t)2 * p.G * D + (size_t)hd * dv + vc] : 0.0f;
-    bpre = DELTA ? p.beta[(size_t)(r0 + t) * H + hd] : 0.0f;
+    vpre = qk[t * p.ld + (size_t)2 * p.G * D + (size_t)hd * dv + min(vc, dv - 1)];
+    if constexpr (DELTA) bpre = p.beta[(size_t)(r0 + t) * H + hd];
     kqpre = p.kq[(size_t)(r0 + t) * p.G + g];
   };
   if (n > 0) prefetch(0);
@@ -520,9 +522,11 @@ __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
 #pragma unroll
     for (int u = 0; u < TB / 8; ++u)
 #pragma unroll
-      for (int part = 0; part < 3; ++part)
+      for (int part = 0; part < 3; ++part) {
+        const float2 a = pre[u][part][0], c = pre[u][part][1];
         *(float4*)(st + (u * 8 + cw) * ROW + part * D + 4 * l) =
-            make_float4(pre[u][part][0].x, pre[u][part][0].y, pre[u][part][1].x, pre[u][part][1].y);
+            part < 2 || PC ? make_float4(a.x, a.y, c.x, c.y) : make_float4(a.x, a.x, a.x, a.x);
+      }
     *(float4*)(st + vt * ROW + 3 * D + 4 * (tid % CW)) = make_float4(vpre, bpre, kqpre, 0.0f);
     __syncthreads();
     if (t0 + TB < n) prefetch(t0 + TB);
@@ -565,8 +569,13 @@ static void gated_delta_wide_launch(DeltaArgs p, int B, bool plain, hipStream_t 
   p.ncb = (p.dv + 7) / 8;
   p.items = B * p.H * p.ncb;
   const unsigned grid = (unsigned)((p.items + 7) / 8 * 8);
-  if (plain) gated_delta_wide_kernel<false><<<grid, 256, 0, stream>>>(p);
-  else gated_delta_wide_kernel<true><<<grid, 256, 0, stream>>>(p);
+  if (p.per_channel) {
+    if (plain) gated_delta_wide_kernel<false, true><<<grid, 256, 0, stream>>>(p);
+    else gated_delta_wide_kernel<true, true><<<grid, 256, 0, stream>>>(p);
+  } else {
+    if (plain) gated_delta_wide_kernel<false, false><<<grid, 256, 0, stream>>>(p);
+    else gated_delta_wide_kernel<true, false><<<grid, 256, 0, stream>>>(p);
+  }
 }
 
 template <int LPC, bool DELTA>
