@@ -117,6 +117,110 @@ __global__ void __launch_bounds__(256) delta_prepare_kernel(DeltaPrepArgs p) {
   delta_prepare_row<A2F32>(p, blockIdx.x, blockIdx.y, gridDim.y == 1);
 }
 
+// Prompts: the same numbers from more waves with fewer trips to memory. Workgroups of the first `vecs` make q and k of some (token,
+// key head) pairs, a wave several side by side, and their k . q from registers; those of the next `decs` the decays of 256 entries
+// of eight tokens, each row of the low-rank map read once for all eight (a workgroup per token reads all 256 KB of a map of 2048 x
+// 64 for itself); the last ones 256 betas each. CPT: columns a lane holds. 2048 tokens, us for a workgroup per token / here:
+// 16 heads of 128 with a decay per channel 95 / 42, 8 heads with one each 12 / 12; 200 tokens 22 / 12.
+constexpr int kPrepTokens = 8;
+template <bool A2F32, int CPT>
+__global__ void __launch_bounds__(256) delta_prepare_rows_kernel(DeltaPrepArgs p, int T, int vecs, int decs) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, d = p.d;
+  int blk = blockIdx.x;
+  if (blk < vecs) {
+    constexpr int U = CPT <= 2 ? 4 : 1;  // pairs of a wave, side by side
+    const long first = ((long)blk * 4 + wave) * U, end = (long)T * p.G;
+    float qv[U][CPT], kv[U][CPT];
+    float *q[U], *k[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long at = min(first + u, end - 1), t = at / p.G;
+      q[u] = p.qkv + t * p.ld + (size_t)(at % p.G) * d, k[u] = q[u] + (size_t)p.G * d;
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) {
+        const int i = lane + 64 * c;
+        qv[u][c] = i < d ? q[u][i] : 0.0f, kv[u][c] = i < d ? k[u][i] : 0.0f;
+      }
+    }
+    float qs[U], ks[U], dot[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float qn = 0.0f, kn = 0.0f;
+      qs[u] = p.q_scale, ks[u] = 1.0f;
+      if (p.unit) {
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) qn = fmaf(qv[u][c], qv[u][c], qn), kn = fmaf(kv[u][c], kv[u][c], kn);
+        qn = wave_sum(qn), kn = wave_sum(kn);
+        qs[u] = qs[u] / sqrtf(qn + p.norm_eps), ks[u] = ks[u] / sqrtf(kn + p.norm_eps);
+      }
+      dot[u] = 0.0f;
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) {
+        qv[u][c] *= qs[u], kv[u][c] *= ks[u];
+        dot[u] = fmaf(qv[u][c], kv[u][c], dot[u]);
+      }
+      dot[u] = wave_sum(dot[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (first + u >= end) break;
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) {
+        const int i = lane + 64 * c;
+        if (i < d) q[u][i] = qv[u][c], k[u][i] = kv[u][c];
+      }
+      if (lane == 0) p.kq[first + u] = dot[u];
+    }
+    return;
+  }
+  blk -= vecs;
+  const int dc = p.per_channel ? d : 1, n = p.H * dc;
+  if (blk >= decs) {
+    const long at = (long)(blk - decs) * 256 + threadIdx.x;
+    if (at < (long)T * p.H) p.beta[at] = sigmoid_f(p.b[at / p.H * p.ldb + at % p.H]);
+    return;
+  }
+  const int cols = (n + 255) / 256, i = blk % cols * 256 + threadIdx.x;
+  const long t0 = (long)(blk / cols) * kPrepTokens;
+  float raw[kPrepTokens];
+  if (p.w_a2) {
+    __shared__ __attribute__((aligned(16))) float a1[kPrepTokens][kMaxRank];
+    for (int x = threadIdx.x; x < kPrepTokens * p.rank; x += 256) {
+      const int u = x / p.rank, r = x % p.rank;
+      a1[u][r] = aop<A2F32>(p.a[min(t0 + u, (long)T - 1) * p.lda + r]);
+    }
+    __syncthreads();
+    if (i >= n) return;
+#pragma unroll
+    for (int u = 0; u < kPrepTokens; ++u) raw[u] = 0.0f;
+    int r = 0;
+    if ((p.rank & 7) == 0)
+      for (; r < p.rank; r += 8) {
+        float w[8];
+        wload8<A2F32>(p.w_a2, (size_t)i * p.rank + r, w);
+#pragma unroll
+        for (int u = 0; u < kPrepTokens; ++u)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) raw[u] = fmaf(a1[u][r + e], w[e], raw[u]);
+      }
+    for (; r < p.rank; ++r) {
+      const float w = wload<A2F32>(p.w_a2, (size_t)i * p.rank + r);
+#pragma unroll
+      for (int u = 0; u < kPrepTokens; ++u) raw[u] = fmaf(a1[u][r], w, raw[u]);
+    }
+  } else {
+    if (i >= n) return;
+#pragma unroll
+    for (int u = 0; u < kPrepTokens; ++u) raw[u] = p.a[min(t0 + u, (long)T - 1) * p.lda + i];
+  }
+  const float bias = p.dt_bias[i], rate = p.decay_form == 1 ? 0.0f : expf(p.A_log[i / dc]);
+#pragma unroll
+  for (int u = 0; u < kPrepTokens; ++u) {
+    const float z = raw[u] + bias;
+    if (t0 + u < T) p.dec[(t0 + u) * n + i] = p.decay_form == 1 ? decay_of(p, z, 0) : expf(-rate * softplus_d(z));
+  }
+}
+
 // One channel of the short convolution for a one-token step: the weighted sum of the token's input and the slot's
 // stored inputs (zeros before the sequence's start), which are shifted by one; returns silu of the sum.
 template <bool WF32>
@@ -569,12 +673,16 @@ static void gated_delta_wide_launch(DeltaArgs p, int B, bool plain, hipStream_t 
   p.ncb = (p.dv + 7) / 8;
   p.items = B * p.H * p.ncb;
   const unsigned grid = (unsigned)((p.items + 7) / 8 * 8);
+  // Up to half as many workgroups as the chip has CUs: 28 KB that nobody uses, 84 with the kernel's own, keep a CU's LDS from two
+  // of them and from one beside an attention's 98. The rule of 8 heads runs beside its layer's attention on another stream: 354
+  // to 424 us of 2048 tokens where they share CUs, 274 on its own ones (a raised wave priority changed nothing).
+  const unsigned alone = p.items <= 128 ? 28 * 1024 : 0;
   if (p.per_channel) {
-    if (plain) gated_delta_wide_kernel<false, true><<<grid, 256, 0, stream>>>(p);
-    else gated_delta_wide_kernel<true, true><<<grid, 256, 0, stream>>>(p);
+    if (plain) gated_delta_wide_kernel<false, true><<<grid, 256, alone, stream>>>(p);
+    else gated_delta_wide_kernel<true, true><<<grid, 256, alone, stream>>>(p);
   } else {
-    if (plain) gated_delta_wide_kernel<false, false><<<grid, 256, 0, stream>>>(p);
-    else gated_delta_wide_kernel<true, false><<<grid, 256, 0, stream>>>(p);
+    if (plain) gated_delta_wide_kernel<false, false><<<grid, 256, alone, stream>>>(p);
+    else gated_delta_wide_kernel<true, false><<<grid, 256, alone, stream>>>(p);
   }
 }
 
@@ -606,8 +714,20 @@ extern "C" int lgs_delta_prepare(float* qkv, long ld, const float* a, long lda, 
   lgs::DeltaPrepArgs p{qkv, ld, a, lda, b, ldb, A_log, dt_bias, dec, beta, kq, H, G, d, per_channel ? 1 : 0, q_scale,
                        norm_eps, w_a2, rank, a2_f32, unit ? 1 : 0, decay_form, tau, nullptr, 0, nullptr, 0, 0, 0, nullptr,
                        nullptr, nullptr};
-  // few rows (decode): the decays - with a low-rank second map a product each - spread over workgroups of their own
   const int n = per_channel ? H * d : H;
+  if (T > 64 && d <= 512) {
+    const long vecs = ((long)T * G + 4 * (d <= 128 ? 4 : 1) - 1) / (4 * (d <= 128 ? 4 : 1)), decs = ((long)T + lgs::kPrepTokens - 1) / lgs::kPrepTokens * ((n + 255) / 256);
+    const long betas = b ? ((long)T * H + 255) / 256 : 0;
+    if (vecs + decs + betas < (1L << 31)) {
+      const unsigned grid = (unsigned)(vecs + decs + betas);
+      if (a2_f32 && d <= 128) lgs::delta_prepare_rows_kernel<true, 2><<<grid, 256, 0, stream>>>(p, T, (int)vecs, (int)decs);
+      else if (a2_f32) lgs::delta_prepare_rows_kernel<true, 8><<<grid, 256, 0, stream>>>(p, T, (int)vecs, (int)decs);
+      else if (d <= 128) lgs::delta_prepare_rows_kernel<false, 2><<<grid, 256, 0, stream>>>(p, T, (int)vecs, (int)decs);
+      else lgs::delta_prepare_rows_kernel<false, 8><<<grid, 256, 0, stream>>>(p, T, (int)vecs, (int)decs);
+      LGA_LAUNCH_RETURN();
+    }
+  }
+  // few rows (decode): the decays - with a low-rank second map a product each - spread over workgroups of their own
   const dim3 grid(T, T <= 64 && n > 256 ? 1 + (n + 255) / 256 : 1);
   if (a2_f32) lgs::delta_prepare_kernel<true><<<grid, 256, 0, stream>>>(p);
   else lgs::delta_prepare_kernel<false><<<grid, 256, 0, stream>>>(p);

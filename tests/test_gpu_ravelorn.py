@@ -459,6 +459,31 @@ def test_delta_rule_of_wide_heads_to_the_bit(H, G, dv, extra, lens, per_channel,
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
 
 
+@pytest.mark.parametrize("H,G,d,per_channel,rank,unit,form", [(4, 2, 128, True, 64, True, 0), (4, 4, 40, False, 0, True, 0),
+                                                              (2, 1, 130, True, 12, True, 0), (3, 3, 512, True, 3, False, 1),
+                                                              (16, 16, 64, True, 0, True, 1)])
+@pytest.mark.parametrize("T", [65, 72, 131])
+def test_delta_prepare_of_prompts_to_the_bit(H, G, d, per_channel, rank, unit, form, T):
+    """More than 64 rows: the bits of 64 at a time, over ends of eight tokens, 256 entries and four heads."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(d + T)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev)  # noqa: E731
+    n = H * d if per_channel else H
+    qkv, a, b, A_log, bias = draw(T, 2 * G * d + 5), draw(T, 2 + (rank or n)), draw(T, H + 3), draw(H), draw(n)
+    w = draw(n, rank).to(torch.bfloat16) if rank else None
+    kw = dict(H=H, G=G, d=d, per_channel=per_channel, q_scale=0.25, w_a2=w, unit=unit, decay_form=form, tau=2.0)
+    whole = qkv.clone()
+    got = [whole, *seq_ops.delta_prepare(whole, a, 2, b, 3, A_log, bias, **kw)]
+    parts = []
+    for rows in (slice(0, 64), slice(64, 128), slice(128, T))[: -(-T // 64)]:
+        q = qkv[rows].clone()
+        parts.append([q, *seq_ops.delta_prepare(q, a[rows].contiguous(), 2, b[rows].contiguous(), 3, A_log, bias, **kw)])
+    for x, *pieces in zip(got, *parts):
+        assert torch.equal(x, torch.cat(pieces))
+
+
 def test_delta_prepare():
     from lit_gpt import seq_ops
 
