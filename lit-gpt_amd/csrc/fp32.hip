@@ -30,6 +30,10 @@ __device__ __forceinline__ float gelu_f32(float v, bool approximate_tanh) {
   return 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
 }
 
+__device__ __forceinline__ void f32_fma4(const float4& x, const float4& w, float4& acc) {
+  acc.x = fmaf(x.x, w.x, acc.x), acc.y = fmaf(x.y, w.y, acc.y), acc.z = fmaf(x.z, w.z, acc.z), acc.w = fmaf(x.w, w.w, acc.w);
+}
+
 // act: 0 none, 1 exact gelu, 2 tanh gelu, on the product + bias; then the residuals, one after the other
 // one wave per output (m, n): lanes stride over K (16-B loads when K % 4 == 0), then a wave sum
 __global__ void __launch_bounds__(256) f32_linear_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -43,13 +47,9 @@ __global__ void __launch_bounds__(256) f32_linear_kernel(const float* __restrict
   const float* wr = w + (size_t)n * K;
   float acc = 0.0f;
   if ((K & 3) == 0) {
-    for (int k = lane * 4; k < K; k += 256) {
-      const float4 xv = *(const float4*)(xr + k), wv = *(const float4*)(wr + k);
-      acc = fmaf(xv.x, wv.x, acc);
-      acc = fmaf(xv.y, wv.y, acc);
-      acc = fmaf(xv.z, wv.z, acc);
-      acc = fmaf(xv.w, wv.w, acc);
-    }
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);  // (four sums of a lane are nearer to the exact one than one)
+    for (int k = lane * 4; k < K; k += 256) f32_fma4(*(const float4*)(xr + k), *(const float4*)(wr + k), a);
+    acc = (a.x + a.y) + (a.z + a.w);
   } else {
     for (int k = lane; k < K; k += 64) acc = fmaf(xr[k], wr[k], acc);
   }
@@ -156,16 +156,12 @@ __device__ __forceinline__ void f32_load_chunks(const float* row, int c0, int K,
     if (k < K) v[c] = *(const float4*)(row + k);
   }
 }
-__device__ __forceinline__ float f32_dot_chunks(const float* xr, int c0, int K, int lane, const float4 (&w)[kF32Chunks], float acc) {
+__device__ __forceinline__ void f32_dot_chunks(const float* xr, int c0, int K, int lane, const float4 (&w)[kF32Chunks], float4& acc) {
 #pragma unroll
   for (int c = 0; c < kF32Chunks; ++c) {
     const int k = (c0 + c) * 256 + lane * 4;
-    if (k < K) {
-      const float4 x = *(const float4*)(xr + k);
-      acc = fmaf(x.w, w[c].w, fmaf(x.z, w[c].z, fmaf(x.y, w[c].y, fmaf(x.x, w[c].x, acc))));
-    }
+    if (k < K) f32_fma4(*(const float4*)(xr + k), w[c], acc);
   }
-  return acc;
 }
 template <int CPT>
 __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a) {
@@ -195,13 +191,13 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
   for (int i = threadIdx.x + 256 * CPT; i < K; i += 256) xn[i] = f32_normed(a.x[i], mean, rstd, p.nw[i], p.nb, p.nb ? p.nb[i] : 0.0f);
   __syncthreads();
   for (const int step = p.blocks * 4; n < p.N; n += step) {
-    float acc = 0.0f;
+    float4 a4 = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int c0 = 0; c0 * 256 < K; c0 += kF32Chunks) {
-      acc = f32_dot_chunks(xn, c0, K, lane, w, acc);
+      f32_dot_chunks(xn, c0, K, lane, w, a4);
       const bool more = (c0 + kF32Chunks) * 256 < K;
       if (more || n + step < p.N) f32_load_chunks(p.w + (size_t)(more ? n : n + step) * K, more ? c0 + kF32Chunks : 0, K, lane, w);
     }
-    acc = wave_sum(acc);
+    float acc = wave_sum((a4.x + a4.y) + (a4.z + a4.w));
     if (lane == 0) {
       if (p.b) acc += bias;
       if (p.act) acc = gelu_f32(acc, p.act == 2);
@@ -282,10 +278,10 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
     f32_join_parts(a, xs, xs + a.K1);
     x1 = xs;
   }
-  float h = 0.0f, m = 0.0f;
+  float4 h4 = make_float4(0.f, 0.f, 0.f, 0.f), m4 = h4;
   for (int c0 = 0; c0 * 256 < a.K1; c0 += kF32Chunks) {
     if (c0 > 0) f32_load_chunks(r1, c0, a.K1, lane, w1);
-    h = f32_dot_chunks(x1, c0, a.K1, lane, w1, h);
+    f32_dot_chunks(x1, c0, a.K1, lane, w1, h4);
   }
   for (int c0 = 0; c0 * 256 < a.K2; c0 += 3 * kF32Chunks) {
 #pragma unroll
@@ -293,9 +289,9 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
       if (c0 > 0) f32_load_chunks(r2, c0 + u * kF32Chunks, a.K2, lane, w2[u]);
     }
 #pragma unroll
-    for (int u = 0; u < 3; ++u) m = f32_dot_chunks(a.x2, c0 + u * kF32Chunks, a.K2, lane, w2[u], m);
+    for (int u = 0; u < 3; ++u) f32_dot_chunks(a.x2, c0 + u * kF32Chunks, a.K2, lane, w2[u], m4);
   }
-  h = wave_sum(h), m = wave_sum(m);
+  float h = wave_sum((h4.x + h4.y) + (h4.z + h4.w)), m = wave_sum((m4.x + m4.y) + (m4.z + m4.w));
   if (lane == 0 && row < a.N) {
     if (a.b1) h += b1;
     if (a.b2) m += b2;
