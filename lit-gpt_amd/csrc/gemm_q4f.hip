@@ -766,6 +766,13 @@ Route route(int M, int N, int K, int fmt, bool dual) {
     }
   }
   if (r.form == kTiles && (dual || q4f_big_columns(M, N, K) == 0)) r.need = ws_need(q4f_plan(M, N, K, dual), M, N, dual);
+  if (r.form == kTiles && lga::kernel_fmt(fmt) != 2 && K >= 8192 && !tiles_named()) {
+    // halves of K where gemm_q4r.hip's tiles leave much of the chip idle, up to 128 MB of sums. us whole / in halves: nf4 517 rows
+    // of 8192 x 28672 363 / 289, 4096 x 11008 116 / 80, 1000 rows 518 / 420, 128 / 116, of 8192 x 8192 149 / 143; int4 1000 rows of
+    // 4096 x 11008 110 / 102 (of 4096 x 4096, where the sums cost more than they gain, 47 / 52)
+    const size_t halves = 4096 + (size_t)2 * (dual ? 2 : 1) * M * N * 4;
+    if (r.need < halves && halves <= (size_t)128 << 20 && lga::q4r_plan(M, N, K, dual, lga::kernel_fmt(fmt), 2).splits > 1) r.need = halves;
+  }
   return r;
 }
 
@@ -895,7 +902,7 @@ extern "C" size_t lga_q4f_plan(int M, int N, int K, int swiglu, int fmt) {
 extern "C" size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu) {
   if (M < 1 || N < 1 || K < lga::pf::BK) return 0;
   size_t need = ws_need(q4f_plan(M, N, K, swiglu != 0), M, N, swiglu != 0);
-  for (int fmt : {0, 2}) need = std::max(need, route(M, N, K, fmt, swiglu != 0).need);
+  for (int fmt : {0, 1, 2}) need = std::max(need, route(M, N, K, fmt, swiglu != 0).need);
   return need;
 }
 
