@@ -51,7 +51,7 @@ def test_refused_sizes_have_no_workspace():
     assert plan(0, 64, 64) == (TILES, 0, False) and plan(4, 64, 32) == (TILES, 0, False) and plan(4, 64, 64, 0, 7) == (TILES, 0, False)
 
 
-@pytest.mark.parametrize("M,N,K,halves", [(1000, 4096, 11008, True), (517, 8192, 28672, True), (1000, 4096, 4096, False),
+@pytest.mark.parametrize("M,N,K,halves", [(1000, 4096, 11008, True), (517, 8192, 28672, True), (1400, 4096, 4096, False),
                                           (2048, 28672, 8192, False)])
 def test_halves_of_long_rows(M, N, K, halves):
     """4-bit prompts past the tiles' own ranges of K ask for two ranges' sums where rows are long and tiles few."""
