@@ -21,7 +21,10 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // ------------------------------------------------------------------------------------------------ GEMV, M <= 8
 // R output columns per wave: 4 for tall matrices (more loads in flight per lane), fewer for short ones (more waves)
 // KS 4: short and deep matrices; the four waves of a workgroup share its R columns, each a quarter of K
-template <bool WF32, int MT, int R, int KS>
+// AHEAD: the weights of four passes over K on their way together, for few columns a wave, whose time is trips to memory. us before /
+// with, weights from memory: 2048 x 5632 10.7 / 10.4, two rows 16.0 / 11.4, 11264 x 2048 13.2 / 12.1; with more columns or
+// deeper rows the registers cost more waves than the trips take (22016 x 4096 38.8 / 41.6)
+template <bool WF32, int MT, int R, int KS, bool AHEAD>
 __global__ void __launch_bounds__(256) lin_gemv_kernel(LinArgs p) {
   __shared__ float shared_acc[KS > 1 ? 4 * MT * R : 1];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -46,7 +49,47 @@ __global__ void __launch_bounds__(256) lin_gemv_kernel(LinArgs p) {
     rows[r] = min(n0 + r, p.N - 1);
     bias[r] = p.bias ? p.bias[rows[r]] : 0.0f;
   }
-  if (vec) {
+  auto add = [&](int k, const float (&wv)[R][8]) {  // eight values of K of every row and column
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      if (m < p.M) {
+        const float* ar = a + (size_t)m * p.lda + k;
+        const float4 lo = *(const float4*)ar, hi = *(const float4*)(ar + 4);
+        const float av[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = aop<WF32>(av[e]);
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[m][r] = fmaf(x, wv[r][e], acc[m][r]);
+        }
+      }
+    }
+  };
+  auto spread = [](const uint4& q, float (&v)[8]) {
+    v[0] = bflo(q.x); v[1] = bfhi(q.x); v[2] = bflo(q.y); v[3] = bfhi(q.y);
+    v[4] = bflo(q.z); v[5] = bfhi(q.z); v[6] = bflo(q.w); v[7] = bfhi(q.w);
+  };
+  if (vec && AHEAD) {
+    static_assert(!AHEAD || (!WF32 && KS == 1), "bf16 weights, a wave per column");
+    constexpr int U = 4;
+    for (int k0 = kl * 8; k0 < K; k0 += 512 * U) {
+      uint4 q[U][R];
+      // (a lane past the end loads its row's last values and does not use them: behind a branch a load waits for those before it)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          q[u][r] = *(const uint4*)((const uint16_t*)p.w + wbase + (size_t)rows[r] * K + min(k0 + u * 512, K - 8));
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (k0 + u * 512 >= K) break;
+        float wv[R][8];
+#pragma unroll
+        for (int r = 0; r < R; ++r) spread(q[u][r], wv[r]);
+        add(k0 + u * 512, wv);
+      }
+    }
+  } else if (vec) {
 #pragma unroll 2
     for (int k = kl * 8; k < K; k += 512 * KS) {
       float wv[R][8];
@@ -58,25 +101,10 @@ __global__ void __launch_bounds__(256) lin_gemv_kernel(LinArgs p) {
           wv[r][0] = lo.x; wv[r][1] = lo.y; wv[r][2] = lo.z; wv[r][3] = lo.w;
           wv[r][4] = hi.x; wv[r][5] = hi.y; wv[r][6] = hi.z; wv[r][7] = hi.w;
         } else {
-          const uint4 q = *(const uint4*)((const uint16_t*)p.w + off);
-          wv[r][0] = bflo(q.x); wv[r][1] = bfhi(q.x); wv[r][2] = bflo(q.y); wv[r][3] = bfhi(q.y);
-          wv[r][4] = bflo(q.z); wv[r][5] = bfhi(q.z); wv[r][6] = bflo(q.w); wv[r][7] = bfhi(q.w);
+          spread(*(const uint4*)((const uint16_t*)p.w + off), wv[r]);
         }
       }
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        if (m < p.M) {
-          const float* ar = a + (size_t)m * p.lda + k;
-          const float4 lo = *(const float4*)ar, hi = *(const float4*)(ar + 4);
-          const float av[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float x = aop<WF32>(av[e]);
-#pragma unroll
-            for (int r = 0; r < R; ++r) acc[m][r] = fmaf(x, wv[r][e], acc[m][r]);
-          }
-        }
-      }
+      add(k, wv);
     }
   } else {
     for (int k = kl; k < K; k += 64 * KS) {
@@ -583,10 +611,10 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
     const int R = N >= 16384 ? 4 : (N >= 4096 ? 2 : 1);
     const bool deep = (long)N * batch <= 512 && K >= 1024;  // few columns: four waves per column
     const dim3 grid(deep ? N : (N + 4 * R - 1) / (4 * R), batch);
-#define LGS_GEMV_R(MT, RR, KS)                                                          \
-  do {                                                                                  \
-    if (w_f32) lgs::lin_gemv_kernel<true, MT, RR, KS><<<grid, 256, 0, stream>>>(p);     \
-    else lgs::lin_gemv_kernel<false, MT, RR, KS><<<grid, 256, 0, stream>>>(p);          \
+#define LGS_GEMV_R(MT, RR, KS)                                                                 \
+  do {                                                                                         \
+    if (w_f32) lgs::lin_gemv_kernel<true, MT, RR, KS, false><<<grid, 256, 0, stream>>>(p);     \
+    else lgs::lin_gemv_kernel<false, MT, RR, KS, false><<<grid, 256, 0, stream>>>(p);          \
   } while (0)
 #define LGS_GEMV(MT)                       \
   do {                                     \
@@ -595,6 +623,12 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
     else if (deep) LGS_GEMV_R(MT, 1, 4);   \
     else LGS_GEMV_R(MT, 1, 1);             \
   } while (0)
+    if (!w_f32 && !deep && M <= 2 && K >= 1024 && (R == 1 || (R == 2 && M == 1 && K <= 2048))) {
+      if (R == 2) lgs::lin_gemv_kernel<false, 1, 2, 1, true><<<grid, 256, 0, stream>>>(p);
+      else if (M == 1) lgs::lin_gemv_kernel<false, 1, 1, 1, true><<<grid, 256, 0, stream>>>(p);
+      else lgs::lin_gemv_kernel<false, 2, 1, 1, true><<<grid, 256, 0, stream>>>(p);
+      LGA_LAUNCH_RETURN();
+    }
     if (M == 1) LGS_GEMV(1);
     else if (M == 2) LGS_GEMV(2);
     else if (M <= 4) LGS_GEMV(4);

@@ -457,6 +457,28 @@ def test_streams_step(s, W, T):
     assert (plain.cpu().double() - u).abs().max() < 1e-5 and (xd.cpu().double() - nx).abs().max() < 1e-5
 
 
+@pytest.mark.parametrize("N,K", [(513, 1024), (2048, 2056), (700, 5640), (515, 1032), (4097, 1024), (4100, 2048), (4096, 2040), (513, 1020)])
+def test_one_and_two_rows_to_the_bit(N, K):
+    """Products of one and two rows, some with the weights of four passes over K on their way together: the bits of three rows, over
+    ends of passes, of 512 values and of columns; rows of no eight values keep the general form."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).to(torch.bfloat16)
+    x, bias = torch.randn(3, K, generator=g, device=dev), torch.randn(N, generator=g, device=dev)
+
+    def rows(M):
+        y = torch.full((M, N), 2.0, device=dev)
+        seq_ops.linear(x[:M].contiguous(), w, M=M, N=N, K=K, y=y, lda=K, ldy=N, bias=bias, accumulate=True)
+        return y
+
+    three = rows(3)
+    want = x.bfloat16().double() @ w.double().T + bias.double() + 2.0
+    assert (three.double() - want).abs().max() < 2e-5  # K products of size K^-1/2 each, summed in 32 bits
+    assert torch.equal(rows(1), three[:1]) and torch.equal(rows(2), three[:2])
+
+
 def test_clamped_unit():
     from lit_gpt import seq_ops
 
