@@ -139,7 +139,8 @@ class Sublayer(nn.Module):
         """h (T, width): the normed read of the streams. Returns the sublayer's output (T, width) fp32."""
         n_in, W = self.w_in.shape
         y = torch.empty(step.T, W, dtype=torch.float32, device=h.device)
-        if cache is None and self.b_in is None and not hooked(self.module) and self.module.forward_in(h16, self.w_in, y):
+        if cache is None and self.b_in is None and not hooked(self.module) and \
+                self.module.forward_in(h if h16 is None else h16, self.w_in, y):
             return y
         proj = torch.empty(step.T, n_in, dtype=torch.float32, device=h.device)
         seq_ops.linear(h if h16 is None else h16, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in,
@@ -274,7 +275,7 @@ class SandwichSublayer(nn.Module):
             return [(y, None)], 1.0
         y = torch.empty(T, W, dtype=torch.float32, device=src.device)
         if cache is None and self.w_in is not None and self.b_in is None and not hooked(self.module) and \
-                self.module.forward_in(h16, self.w_in, y):
+                self.module.forward_in(src, self.w_in, y):
             return [(y, None)], 1.0
         proj = None
         if self.w_in is not None and self.module.wants_proj(T):

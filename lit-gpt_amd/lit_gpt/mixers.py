@@ -115,9 +115,9 @@ class InputReader(nn.Module):
     # token's near ties fall alike however many rows stand beside it
     in_ksplit = 0
 
-    def forward_in(self, h16: Optional[torch.Tensor], w_in: torch.Tensor, x: torch.Tensor, accumulate: bool = False) -> bool:
-        """A module without a cache, straight from its sublayer's input (a bf16 copy) and fused input matrix; False:
-        nothing done, the input projection and ``forward`` make it."""
+    def forward_in(self, h: Optional[torch.Tensor], w_in: torch.Tensor, x: torch.Tensor, accumulate: bool = False) -> bool:
+        """A module without a cache, straight from its sublayer's input (its bf16 copy where there is one) and fused input matrix;
+        False: nothing done, the input projection and ``forward`` make it."""
         return False
 
     def reads_f32(self, rows: int) -> bool:
@@ -887,13 +887,18 @@ class GatedFeedForward(InputReader):
             a = seq_ops.glu(proj, self.off["gate"], self.off["up"], self.ff, self.act, bf16=bf16)
         self._down(a, x, accumulate)
 
-    def forward_in(self, h16: Optional[torch.Tensor], w_in: torch.Tensor, x: torch.Tensor, accumulate: bool = False) -> bool:
-        """Where the input product and the gated unit fit one launch (prompts, bf16 weights)."""
-        T = x.shape[0]
-        if self.off["gate"] != 0 or not _tiles16(T, self.w_down) or not seq_ops.glu_fits(h16, w_in, T, self.ff):
+    def forward_in(self, h: Optional[torch.Tensor], w_in: torch.Tensor, x: torch.Tensor, accumulate: bool = False) -> bool:
+        """Where the input product and the gated unit fit one launch (bf16 weights: prompts, and one row)."""
+        T, form = x.shape[0], dict(n=self.ff, up=self.off["up"], act=self.act, clamp=self.clamp)
+        if self.off["gate"] != 0 or h is None:
             return False
-        self._down(seq_ops.linear_glu(h16, w_in, M=T, n=self.ff, up=self.off["up"], act=self.act, clamp=self.clamp), x,
-                   accumulate)
+        if T == 1 and h.dtype == torch.float32 and w_in.dtype == torch.bfloat16 and h.is_contiguous() and \
+                w_in.shape[1] % 8 == 0 and h.data_ptr() % 16 == 0 and w_in.data_ptr() % 16 == 0:
+            self._down(seq_ops.linear_glu_row(h, w_in, **form), x, accumulate)
+            return True
+        if not _tiles16(T, self.w_down) or not seq_ops.glu_fits(h, w_in, T, self.ff):
+            return False
+        self._down(seq_ops.linear_glu(h, w_in, M=T, **form), x, accumulate)
         return True
 
     def _down(self, a: torch.Tensor, x: torch.Tensor, accumulate: bool) -> None:

@@ -34,6 +34,7 @@ SIGNATURES = {
     "lgs_linear": [_P, _L, _L, _P, _I, _L, _P, _L, _L, _I, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _P, _I, _P],
     "lgs_linear_ksplit": [_I, _I, _I],
     "lgs_linear_glu_fits": [_I, _I, _I, _I],
+    "lgs_linear_glu_row": [_P, _P, _L, _P, _I, _I, _I, _I, _F, _F, _F, _P],
     "lgs_linear_glu": [_P, _L, _P, _L, _L, _P, _L, _I, _I, _I, _I, _P, _P, _I, _I, _F, _F, _F, _P],
     "lgs_embed": [_P, _P, _I, _F, _P, _I, _I, _I, _P],
     "lgs_rmsnorm": [_P, _L, _P, _F, _F, _P, _L, _I, _I, _I, _P, _P],
@@ -419,6 +420,18 @@ def linear_glu(a: torch.Tensor, w: torch.Tensor, *, M: int, n: int, up: int, act
                                          out.data_ptr(), n, M, n, K, batch, _opt(a_rows, "a_rows", I32),
                                          _opt(z_start, "z_start", I32), act, int(clamp is not None), float(alpha),
                                          float(limit), float(shift), _stream()))
+    return out
+
+
+def linear_glu_row(a: torch.Tensor, w: torch.Tensor, *, n: int, up: int, act: int = 0, clamp: Optional[tuple] = None) -> torch.Tensor:
+    """``linear_glu`` of one fp32 row, in fp32: (1, n), to the bits of ``linear`` and ``glu`` / ``glu_clamped`` in turn."""
+    rows, K = w.shape
+    if a.numel() != K or rows < up + n:
+        raise ValueError("linear_glu_row: shapes")
+    out = torch.empty(1, n, dtype=F32, device=a.device)
+    alpha, limit, shift = clamp if clamp is not None else (0.0, 0.0, 0.0)
+    _check(load_library().lgs_linear_glu_row(_dev(a, "a", F32), _dev(w, "w", torch.bfloat16), up, out.data_ptr(), n, K, act,
+                                             int(clamp is not None), float(alpha), float(limit), float(shift), _stream()))
     return out
 
 

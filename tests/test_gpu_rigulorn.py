@@ -479,6 +479,24 @@ def test_one_and_two_rows_to_the_bit(N, K):
     assert torch.equal(rows(1), three[:1]) and torch.equal(rows(2), three[:2])
 
 
+@pytest.mark.parametrize("n,K", [(1, 8), (5, 520), (1001, 2048), (600, 2056), (9000, 4096)])
+@pytest.mark.parametrize("clamp", [None, (1.702, 2.5, 1.0)])
+def test_one_row_gated_unit_to_the_bit(n, K, clamp):
+    """A row's input product and gated unit in one launch: the bits of the two, with two and four columns a wave there."""
+    from lit_gpt import seq_ops
+
+    dev, up = torch.device("cuda", 0), n + -n % 8
+    g = torch.Generator(device=dev).manual_seed(n + K)
+    w = (torch.randn(2 * up, K, generator=g, device=dev) * 2 * K ** -0.5).to(torch.bfloat16)
+    h, proj = torch.randn(1, K, generator=g, device=dev), torch.empty(1, 2 * up, device=dev)
+    seq_ops.linear(h, w, M=1, N=2 * up, K=K, y=proj, lda=K, ldy=2 * up)
+    if clamp is None:
+        want = seq_ops.glu(proj, 0, up, n, seq_ops.ACT_SILU)
+    else:
+        want = seq_ops.glu_clamped(proj, 0, up, n, alpha=clamp[0], limit=clamp[1], shift=clamp[2])
+    assert torch.equal(seq_ops.linear_glu_row(h, w, n=n, up=up, act=seq_ops.ACT_SILU, clamp=clamp), want)
+
+
 def test_clamped_unit():
     from lit_gpt import seq_ops
 
