@@ -23,7 +23,7 @@ __global__ void __launch_bounds__(256) embed_streams_kernel(const int* __restric
                                                             float scale, float* __restrict__ x, int W, int streams) {
   const size_t t = blockIdx.x;
   const size_t src = (size_t)tokens[t] * W;
-  for (int i = threadIdx.x; i < W; i += 256) {
+  for (int i = blockIdx.y * 256 + threadIdx.x; i < W; i += gridDim.y * 256) {
     const float v = wload<WF32>(table, src + i) * scale;
     for (int j = 0; j < streams; ++j) x[(t * streams + j) * W + i] = v;
   }
@@ -396,8 +396,9 @@ extern "C" int lgs_embed_streams(const int* tokens, const void* table, int w_f32
                                  int vocab, int streams, hipStream_t stream) {
   LGA_CHECK_ARG(tokens && table && x && T > 0 && W > 0 && vocab > 0, "lgs_embed_streams: bad arguments");
   LGA_CHECK_ARG(streams >= 1 && streams <= lgs::kMaxStreams, "lgs_embed_streams: 1 to 8 streams");
-  if (w_f32) lgs::embed_streams_kernel<true><<<T, 256, 0, stream>>>(tokens, table, scale, x, W, streams);
-  else lgs::embed_streams_kernel<false><<<T, 256, 0, stream>>>(tokens, table, scale, x, W, streams);
+  const dim3 grid = lgs::embed_grid(T, W);
+  if (w_f32) lgs::embed_streams_kernel<true><<<grid, 256, 0, stream>>>(tokens, table, scale, x, W, streams);
+  else lgs::embed_streams_kernel<false><<<grid, 256, 0, stream>>>(tokens, table, scale, x, W, streams);
   LGA_LAUNCH_RETURN();
 }
 

@@ -568,3 +568,35 @@ def test_command_line_serves_a_checkpoint_folder(tmp_path, capsys):
     agree = [ids[i + 1] == int(torch.argmax(lg[i])) for i in range(6, 11)
              if float(torch.topk(lg[i], 2).values.diff().abs()) > 1e-3]
     assert agree and all(agree)
+
+
+@pytest.mark.parametrize("T,W", [(1, 1), (1, 257), (3, 2048), (64, 2049), (65, 255), (65, 300)])
+def test_embeddings_of_few_and_many_tokens(T, W):
+    """Rows spread over workgroups up to 64 tokens, one workgroup a token beyond: table rows times a power of two, exactly."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(T + W)
+    table, ptable = (torch.randn(n, W, generator=g, device=dev).to(torch.bfloat16) for n in (50, 70))
+    tok = torch.randint(0, 50, (T,), generator=g, device=dev, dtype=torch.int32)
+    pos = torch.arange(T, device=dev, dtype=torch.int32)
+    want = table[tok.long()].float() * 0.5
+    assert torch.equal(seq_ops.embed(tok, table, 0.5), want)
+    assert torch.equal(seq_ops.embed_streams(tok, table, 0.5, 3), want.unsqueeze(1).expand(T, 3, W))
+    x, x16 = seq_ops.embed_pos(tok, pos, table, ptable, 0.5, bf16_copy=True)
+    assert torch.equal(x, want + ptable[:T].float()) and torch.equal(x16, x.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("n", [1, 256, 257, 1024, 1025, 2048, 2049, 4096, 4097, 9000])
+def test_rms_norm_edges(n):
+    """Rows that the registers hold to the last column, and past them: 32-bit sums of n squares against float64."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(n)
+    x, w = torch.randn(3, n, generator=g, device=dev), torch.randn(n, generator=g, device=dev)
+    for weight, offset in ((w, 1.0), (None, 0.0)):
+        y, y16 = seq_ops.rmsnorm(x, weight, offset=offset, eps=1e-5, bf16_copy=True)
+        d = x.double()
+        want = d / (d.pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * (1.0 if weight is None else offset + w.double())
+        assert (y.double() - want).abs().max() < 4e-6 * max(1.0, float(want.abs().max())) and torch.equal(y16, y.to(torch.bfloat16))
