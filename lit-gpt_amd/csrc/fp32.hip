@@ -208,7 +208,8 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 }
 
 // One row: y = ((x2 W2^T + b2) + (x1 W1^T + b1)) + res, a wave per output, both products in f32_linear_kernel's order. Bound by
-// one round of latency: all loads of a block of 768 columns beside 3072 are in flight at once. Two launches 13.7 us, one 8.0 (8.9 with ranges of keys to join).
+// one round of latency: all loads of a block of 768 columns beside 3072 are in flight at once. Two launches 13.7 us, one 8.0
+// (8.9 with ranges of keys to join).
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
   float* y;

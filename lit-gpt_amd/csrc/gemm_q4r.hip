@@ -408,7 +408,8 @@ int preload_gemm_q4r() {
   using namespace pr;
   int bad = 0;
 #define LGA_PRE(F, D) \
-  bad += preload(gemm_q4r_kernel<F, D, 1>) + preload(gemm_q4r_kernel<F, D, 2>) + preload(gemm_q4r_kernel<F, D, 3>) + preload(gemm_q4r_kernel<F, D, 4>) + preload(gemm_q4r_kernel<F, D, 6>) + preload(gemm_q4r_kernel<F, D, 8>)
+  bad += preload(gemm_q4r_kernel<F, D, 1>) + preload(gemm_q4r_kernel<F, D, 2>) + preload(gemm_q4r_kernel<F, D, 3>) + \
+         preload(gemm_q4r_kernel<F, D, 4>) + preload(gemm_q4r_kernel<F, D, 6>) + preload(gemm_q4r_kernel<F, D, 8>)
   LGA_PRE(0, false);
   LGA_PRE(0, true);
   LGA_PRE(1, false);

@@ -716,7 +716,9 @@ extern "C" int lgs_delta_prepare(float* qkv, long ld, const float* a, long lda, 
                        nullptr, nullptr};
   const int n = per_channel ? H * d : H;
   if (T > 64 && d <= 512) {
-    const long vecs = ((long)T * G + 4 * (d <= 128 ? 4 : 1) - 1) / (4 * (d <= 128 ? 4 : 1)), decs = ((long)T + lgs::kPrepTokens - 1) / lgs::kPrepTokens * ((n + 255) / 256);
+    const int pairs = 4 * (d <= 128 ? 4 : 1);  // of a workgroup
+    const long vecs = ((long)T * G + pairs - 1) / pairs;
+    const long decs = ((long)T + lgs::kPrepTokens - 1) / lgs::kPrepTokens * ((n + 255) / 256);
     const long betas = b ? ((long)T * H + 255) / 256 : 0;
     if (vecs + decs + betas < (1L << 31)) {
       const unsigned grid = (unsigned)(vecs + decs + betas);
