@@ -179,3 +179,16 @@ def test_ranges_of_infinite_scores():
         head = y.view(4, H, hs)[:, h].contiguous(), ml[:, h: h + 1].contiguous(), hs
         got = ops.f32_linears_sum(head, eye, torch.zeros(1, 4, device=dev), none, torch.zeros(1, hs, device=dev))[0]
         assert got.isnan().all() if h else (got - want[0]).abs().max() < 1e-6
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 2999, 4), (8, 2996, 4), (9, 1501, 260), (33, 601, 1028), (65, 334, 768), (15, 1501, 255)])
+def test_rows_of_prompts_to_the_bit(M, N, K):
+    """Eight rows and two outputs a wave: the bits of one row at a time, past whole groups of rows and outputs."""
+    from lit_gpt import ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(K + M)
+    x, w, b, r, r2 = (torch.randn(m, generator=g, device=dev) for m in ((M, K), (N, K), (N,), (M, N), (M, N)))
+    for kw in (dict(), dict(bias=b, gelu="tanh", residual=r, residual2=r2)):
+        rows = [ops.f32_linear(x[i: i + 1], w, **{k: v[i: i + 1] if v is r or v is r2 else v for k, v in kw.items()}) for i in range(M)]
+        assert torch.equal(ops.f32_linear(x, w, **kw), torch.cat(rows))
