@@ -79,8 +79,10 @@ int lga_q4f_fits(int M, int N, int K, int group, int fmt);
  * zeroed). */
 size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu);
 /* How a product of one format is made, in one number: bits 0..1 the form (0 the LDS-image tiles, 1 4-bit weights dequantized in
- * registers, 2 the bf16 weights' pipelined tiles), bit 2 set where the first 4096 bytes of its workspace are counters that have
- * to be zero (else it need be neither cleared nor kept), the bits above the workspace's bytes. */
+ * registers, 2 the bf16 weights' pipelined tiles, 3 4-bit weights dequantized beside rings of X; 4-bit scales off 8 bytes take form
+ * 1 or 0 in the place of 3, without counters), bit 2 set where the first 4096 bytes of its workspace are counters that have
+ * to be zero (else it need be neither cleared nor kept), the bits above the workspace's bytes. A matter of the sizes and the format
+ * alone: a larger workspace changes nothing. */
 size_t lga_q4f_plan(int M, int N, int K, int swiglu, int fmt);
 int lga_q4_gemm_fused(const void* x, const void* weight, const void* scales, const void* bias, const void* residual,
                       void* y, int M, int N, int K, int group, int fmt, void* workspace, size_t workspace_bytes,

@@ -73,19 +73,14 @@ static void bf16_go(BfArgs k, bool dual, hipStream_t stream) {
   if (!dual) gemm_bf16_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(k);
 }
 
-// Products with a workspace of partial sums: all but those of few rows and small weights, where a launch over ranges of K and
-// one that adds them are not repaid (us here / on gemm_q4f.hip's tiles): 16 x 4096 x 4096 20 / 14, 16 x 4096 x 11008 26 /
-// 23, against 38 / 39 for 8192 x 8192 (2^26); and but those of more than 1024 rows that fill the chip with K whole
-static bool bf16_long(int M, long cols) { return M > 1024 && (M + 255) / 256 * (cols / 128) >= 256; }
+// All products but those of few rows and small weights, where a launch over ranges of K and one that adds them are not repaid
+// (us here / on gemm_q4f.hip's tiles): 16 x 4096 x 4096 20 / 14, 16 x 4096 x 11008 26 / 23, against 38 / 39 for 8192 x 8192
+// (2^26). More than 1024 rows that fill the chip keep K whole.
 GemmPlan bf16_plan(int M, int N, int K, bool dual) {
   const long cols = dual ? 2L * N : N;
-  if ((M <= 32 && cols * K < 1L << 26) || bf16_long(M, cols)) return GemmPlan{-1, 1};
-  return gemm_tile_plan(M, (int)cols, K, 1, false, 0, kGemmRowsB | (dual ? kGemmPairs : 0));
-}
-GemmPlan bf16_long_plan(int M, int N, int K, bool dual) {
-  const long cols = dual ? 2L * N : N;
-  if (!bf16_long(M, cols)) return GemmPlan{-1, 1};
-  return gemm_tile_plan(M, (int)cols, K, 1, false, 1, kGemmRowsB | (dual ? kGemmPairs : 0));
+  if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1};
+  const bool full = M > 1024 && (M + 255) / 256 * (cols / 128) >= 256;
+  return gemm_tile_plan(M, (int)cols, K, 1, false, full ? 1 : 0, kGemmRowsB | (dual ? kGemmPairs : 0));
 }
 
 size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {

@@ -28,16 +28,17 @@ int q4d_run(const Q4dArgs& a, const Q4dPlan& p, int kernel_fmt, bool dual, hipSt
 void q4d_sum(const Q4dArgs& a, int splits, bool dual, hipStream_t stream);
 int preload_gemm_q4d();
 
-// long prompts and most short ones (gemm_q4r.hip). fn: 32-row pieces of X per tile (0: not one of its products), per: pairs of steps of 64 values
+// long prompts and most short ones (gemm_q4r.hip). fn: 32-row pieces of X per tile (0: not one of its products), per: pairs of steps
+// of 64 values
 struct Q4rPlan {
   int fn, mt, nt, splits, per;
 };
-Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, int most);  // most: ranges of K that the caller's workspace holds
+Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, bool ranges);  // ranges: there is a workspace for the plan's ranges of K
+size_t q4r_workspace(const Q4rPlan& p, int M, int N, bool dual);
 int q4r_run(const Q4dArgs& a, const Q4rPlan& p, int kernel_fmt, bool dual, hipStream_t stream);
 int preload_gemm_q4r();
 
 GemmPlan bf16_plan(int M, int N, int K, bool dual);
-GemmPlan bf16_long_plan(int M, int N, int K, bool dual);  // without a workspace
 size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual);
 int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream);
 int preload_gemm_bf16();

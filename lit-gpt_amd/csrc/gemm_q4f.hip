@@ -745,70 +745,51 @@ int run_tiles(Args a, int fmt, bool dual, int bn, hipStream_t stream);
 // LGA_Q4F_BN / LGA_Q4F_SPLITS name a launch of the tiles here
 bool tiles_named() { return getenv("LGA_Q4F_BN") || getenv("LGA_Q4F_SPLITS"); }
 
-// which form makes a product, and the workspace of the form that it makes. With that workspace (often none) long prompts are
-// made by gemm_q4r.hip and gemm_bf16.hip, and most short 4-bit ones by gemm_q4r.hip (run_long).
-enum Form { kTiles = 0, kRegisters = 1, kBf16Tiles = 2 };  // here; gemm_q4d.hip (4-bit); gemm_bf16.hip
+// Which form makes a product, with its plan and its workspace: all of it a matter of the sizes and the format alone, so that a
+// product gives the same bits whatever ran before it and whatever workspace is left over.
+enum Form { kTiles = 0, kRegisters = 1, kBf16Tiles = 2, kRing = 3 };  // here; gemm_q4d.hip (4-bit); gemm_bf16.hip; gemm_q4r.hip (4-bit)
 struct Route {
   Form form = kTiles;
   lga::Q4dPlan d{};
   lga::GemmPlan b{-1, 1};
+  lga::Q4rPlan r{};
   size_t need = 0;
 };
-Route route(int M, int N, int K, int fmt, bool dual) {
+// aligned: scales start on 8 bytes (kRing loads them in pairs)
+Route route(int M, int N, int K, int fmt, bool dual, bool aligned = true) {
   Route r;
+  const int kf = lga::kernel_fmt(fmt);
   if (!tiles_named()) {
-    if (lga::kernel_fmt(fmt) == 2) {
+    if (kf == 2) {
       r.b = lga::bf16_plan(M, N, K, dual);
       if (r.b.tile >= 0) r.form = kBf16Tiles, r.need = lga::bf16_workspace(r.b, M, N, dual);
     } else {
+      if (aligned) r.r = lga::q4r_plan(M, N, K, dual, kf, true);
       r.d = lga::q4d_plan(M, N, K, dual);
-      if (r.d.mf > 0) r.form = kRegisters, r.need = lga::q4d_workspace(r.d, M, N, dual);
+      if (r.r.fn > 0) r.form = kRing, r.need = lga::q4r_workspace(r.r, M, N, dual);
+      else if (r.d.mf > 0) r.form = kRegisters, r.need = lga::q4d_workspace(r.d, M, N, dual);
     }
   }
   if (r.form == kTiles && (dual || q4f_big_columns(M, N, K) == 0)) r.need = ws_need(q4f_plan(M, N, K, dual), M, N, dual);
-  if (r.form == kTiles && lga::kernel_fmt(fmt) != 2 && K >= 8192 && !tiles_named()) {
-    // halves of K where gemm_q4r.hip's tiles leave much of the chip idle, up to 128 MB of sums. us whole / in halves: nf4 517 rows
-    // of 8192 x 28672 363 / 289, 4096 x 11008 116 / 80, 1000 rows 518 / 420, 128 / 116, of 8192 x 8192 149 / 143; int4 1000 rows of
-    // 4096 x 11008 110 / 102 (of 4096 x 4096, where the sums cost more than they gain, 47 / 52)
-    const size_t halves = 4096 + (size_t)2 * (dual ? 2 : 1) * M * N * 4;
-    if (r.need < halves && halves <= (size_t)128 << 20 && lga::q4r_plan(M, N, K, dual, lga::kernel_fmt(fmt), 2).splits > 1) r.need = halves;
-  }
   return r;
 }
 
-// Products on gemm_q4r.hip's tiles and, long prompts with bf16 weights, gemm_bf16.hip's: their figures stand there; false: not
-// one of theirs.
-bool run_long(const lga::Q4dArgs& d, int fmt, bool dual, size_t ws_bytes, hipStream_t stream, int* rc) {
-  if (tiles_named()) return false;
-  if (lga::kernel_fmt(fmt) == 2) {
-    const lga::GemmPlan b = lga::bf16_long_plan(d.M, d.N, d.K, dual);
-    if (b.tile < 0) return false;
-    *rc = lga::bf16_run(d, b, dual, stream);
-    return true;
-  }
-  if (((uintptr_t)d.sc | (uintptr_t)d.sc2) % 8 != 0) return false;  // (scales are loaded in pairs)
-  const size_t plane = (size_t)(dual ? 2 : 1) * d.M * d.N * 4;
-  const lga::Q4rPlan l = lga::q4r_plan(
-      d.M, d.N, d.K, dual, lga::kernel_fmt(fmt), ws_bytes > 4096 ? (int)std::min<size_t>((ws_bytes - 4096) / plane, 16) : 1);
-  if (l.fn == 0) return false;
-  *rc = lga::q4r_run(d, l, lga::kernel_fmt(fmt), dual, stream);
-  return true;
-}
-
 int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t stream) {
-  const Route r = route(a.M, a.N, a.K, fmt, dual);
+  const int kf = lga::kernel_fmt(fmt);
+  Route r = route(a.M, a.N, a.K, fmt, dual);
+  // Scales off 8 bytes: a form without their pairs, and without counters, for which the caller's workspace was not made
+  const bool off = r.form == kRing && ((uintptr_t)a.sc | (uintptr_t)a.sc2) % 8 != 0;
+  if (off) r = route(a.M, a.N, a.K, fmt, dual, false);
   const lga::Q4dArgs d{a.x, a.w, a.sc, a.w2, a.sc2, a.bias, a.residual, a.y, a.M, a.N, a.K, a.G, a.ldy,
                        lga::codebook_of(fmt), ws ? (float*)((unsigned char*)ws + 4096) : nullptr};
-  int rc;
   const bool whole = r.need == 0 || (ws && ws_bytes >= r.need);  // (a smaller workspace may do for the tiles here)
-  if ((r.form == kTiles || (r.form == kRegisters && whole)) && run_long(d, fmt, dual, ws ? ws_bytes : 0, stream, &rc)) return rc;
-  if (r.form != kTiles && whole) {
-    return r.form == kRegisters ? lga::q4d_run(d, r.d, lga::kernel_fmt(fmt), dual, stream) : lga::bf16_run(d, r.b, dual, stream);
-  }
+  if (r.form == kRing)  // (without its workspace: K whole)
+    return lga::q4r_run(d, whole ? r.r : lga::q4r_plan(a.M, a.N, a.K, dual, kf, false), kf, dual, stream);
+  if (r.form == kRegisters && whole) return lga::q4d_run(d, r.d, kf, dual, stream);
+  if (r.form == kBf16Tiles && whole) return lga::bf16_run(d, r.b, dual, stream);
   if (!dual) {
     const int nb = q4f_big_columns(a.M, a.N, a.K);
     if (nb > 0) {
-      const int kf = lga::kernel_fmt(fmt);
       const size_t row_bytes = kf == 2 ? (size_t)a.K * 2 : (size_t)a.K / 2;
       const size_t sc_bytes = kf == 2 ? 0 : (size_t)(a.K / a.G) * (kf == 0 ? 2 : 4);
       Args b = a, c = a;
@@ -825,7 +806,8 @@ int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t strea
       return rc ? rc : run_tiles(c, fmt, false, 128, stream);
     }
   }
-  const Plan p = q4f_plan(a.M, a.N, a.K, dual);
+  Plan p = q4f_plan(a.M, a.N, a.K, dual);
+  if (off) p.splits = 1;
   if (p.splits > 1) {
     LGA_CHECK_ARG(ws && ws_bytes >= ws_need(p, a.M, a.N, dual) && p.tiles <= 1024,
                   "lga_q4_gemm_fused: split-K needs the workspace lga_q4f_workspace_bytes reports");
@@ -833,7 +815,7 @@ int run(Args a, int fmt, bool dual, void* ws, size_t ws_bytes, hipStream_t strea
     a.slabs = (float*)((unsigned char*)ws + 4096);
   }
   a.cb = lga::codebook_of(fmt);
-  switch (lga::kernel_fmt(fmt) * 2 + (dual ? 1 : 0)) {
+  switch (kf * 2 + (dual ? 1 : 0)) {
     case 0: return launch_q4f<0, false>(a, p, stream);
     case 1: return launch_q4f<0, true>(a, p, stream);
     case 2: return launch_q4f<1, false>(a, p, stream);

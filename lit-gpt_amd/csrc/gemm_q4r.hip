@@ -16,6 +16,8 @@
 // one group 135 us, two workgroups of one group each on a CU and halves of K through memory 137, two groups 124.
 #include "gemm_q4d.h"
 
+#include <algorithm>
+
 namespace lga {
 namespace pr {
 
@@ -352,7 +354,10 @@ static void go_rows(const KArgs& k, int fn, hipStream_t stream) {
 }  // namespace pr
 
 // Rounds of 256 workgroups times their pairs of steps (128 values of K), at the clock of a full chip or, with few workgroups, a
-// higher one, and their start and end. us of a pair for 256, 192 and 128 rows, measured on 256 workgroups of K 4096: int4 2.93,
+// higher one, and their start and end; several ranges of K cost a second launch and the traffic of their sums, at a copy's rate. Of
+// 462 products of 16 to 2048 rows of twelve matrices the choice is 1.1 % from the fastest of up to ten forms and ranges in the
+// mean, and the ranges of the forms that stood here before 2.5 % (nf4 517 rows of 4096 x 11008 77 / 69 us, int4 400 of 8192 x
+// 28672 217 / 195; int4 128 of 11008 x 4096 with SwiGLU 39.0 / 40.7). us of a pair for 256, 192 and 128 rows, measured on 256 workgroups of K 4096: int4 2.93,
 // 2.30, 1.75 (4740, 3870, 3140 clocks, of which 4096, 3072, 2048 of matrix instructions), codebooks 3.22, 2.67, 2.12 (5560,
 // 5050, 4470: sixteen more instructions per eight weights); for 96, 64 and 32 rows from whole products of 86 to 240 workgroups.
 // us on gemm_q4f.hip's tiles / here, int4 with weights from memory: 2048 rows of 12288 x 4096 209 / 197, 4096 x 4096 75 / 68,
@@ -365,8 +370,11 @@ static void go_rows(const KArgs& k, int fn, hipStream_t stream) {
 //   int4 128 rows  11008 x 4096 with SwiGLU 63 / 42, 4096 x 11008 35 / 30, 4096 x 4096 28 / 22
 //   32 rows        int4 4096 x 4096 19.6 / 14.6, 11008 x 4096 with SwiGLU 32 / 28; 4096 x 11008 20.1 / 21.1, nf4 10240 x 8192
 //                  28.9 / 30.0, 28672 x 8192 with SwiGLU 108 / 98: beyond 2^24 values one matrix stays in gemm_q4d.hip's form
-Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, int most) {
+Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, bool ranges) {
   Q4rPlan p{0, 0, 0, 0, 0};
+  // up to 16 ranges, and up to 128 MB of their sums
+  const size_t plane = (size_t)(dual ? 2 : 1) * M * N * 4;
+  const int most = ranges ? (int)std::max<size_t>(std::min<size_t>(((size_t)128 << 20) / plane, 16), 1) : 1;
   const size_t nk = (size_t)N * K, one = 1;
   if (K % 128 != 0) return p;
   if (!dual && M <= 32 && nk > one << 24) return p;
@@ -386,11 +394,15 @@ Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, int most) {
       const float rounds = (float)((long)mt * p.nt * used) / 256.0f, whole = floorf(rounds);
       float us = whole * (per * slow + ends);
       if (rounds > whole) us += per * fmaxf(fast, slow * (0.3f + 0.7f * (rounds - whole))) + ends;
-      if (used > 1) us += 2.0f + (float)M * N * (dual ? 2 : 1) * 4.0f * (used + 1) / 5.5e6f;
+      if (used > 1) us += 2.0f + 0.25f * used + (float)plane * (used + 1) / 4.75e6f;
       if (p.fn == 0 || us < best) best = us, p.fn = fn, p.mt = mt, p.splits = used, p.per = per;
     }
   }
   return p;
+}
+
+size_t q4r_workspace(const Q4rPlan& p, int M, int N, bool dual) {
+  return p.splits > 1 ? 4096 + (size_t)p.splits * (dual ? 2 : 1) * M * N * 4 : 0;
 }
 
 int q4r_run(const Q4dArgs& a, const Q4rPlan& p, int kernel_fmt, bool dual, hipStream_t stream) {

@@ -247,10 +247,11 @@ def q4f_plan(M, N, K, swiglu, fmt):
 
 
 def _q4f_workspace(M, N, K, swiglu, fmt, device):
-    """The split-K workspace of a short-prompt fused GEMM, or None: for the caller to hold until its launch. Partial sums
-    alone come from the allocator per product. The form with per-tile counters keeps a zeroed buffer per device and stream
-    (products on two streams may run at once), grown as needed, the eight last used: a launch leaves its counters zeroed;
-    under capture it has one of the graph's own, whose counters every replay clears."""
+    """The split-K workspace of a fused GEMM, or None: for the caller to hold until its launch. Partial sums alone come from the
+    allocator per product (its launches are two: on a shared buffer another thread's product could stand between them). The
+    form with per-tile counters, one launch, keeps a zeroed buffer per device and stream (products on two streams may run at
+    once), grown as needed, the eight last used: a launch leaves its counters zeroed; under capture it has one of the
+    graph's own, whose counters every replay clears."""
     _, need, counters = q4f_plan(M, N, K, swiglu, fmt)
     if need == 0:
         return None

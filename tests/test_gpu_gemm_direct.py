@@ -72,13 +72,13 @@ def test_swiglu(ops, fmt, group, M, N, K):
 
 
 def test_rule_falls_back(ops):
-    """K of 64 values, small weights of few rows and long prompts stay with the tiles of gemm_q4f.hip; a split product
-    reports its workspace."""
+    """K of no multiple of 128 stays with the tiles of gemm_q4f.hip, small weights of few rows and long prompts with the rings of
+    gemm_q4r.hip; a split product reports its workspace."""
     lib = ops.load_library()
     assert lib.lga_q4f_workspace_bytes(64, 12288, 4096, 0) >= 4096 + 64 * 12288 * 4
     g = torch.Generator(device=DEV).manual_seed(5)
-    for M, N, K in ((40, 264, 192), (16, 512, 1024), (257, 264, 256)):
-        assert ops.q4f_plan(M, N, K, 0, 1)[0] == 0
+    for M, N, K, form in ((40, 264, 192, 0), (16, 512, 1024, 3), (257, 264, 256, 3)):
+        assert ops.q4f_plan(M, N, K, 0, 1)[0] == form
         w, sc, wd = _weight(ops, N, K, 1, 64, g)
         x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
         h = x.float() @ wd.t()
@@ -170,6 +170,102 @@ def test_a_workspace_of_the_older_tiles(ops, M, N, K, monkeypatch):
     assert rc == 0
     h = x.float() @ wd.t()
     assert float(((y.float() - h).abs() - h.abs() * 2 ** -7).max()) <= 2e-3
+
+
+@pytest.mark.parametrize("M,N,K,fmt,swiglu", [(702, 4096, 11008, 0, False), (300, 4096, 11008, 1, False), (16, 4096, 4096, 0, False),
+                                              (129, 1536, 12800, 1, True), (64, 8200, 4096, 0, False)])
+def test_bits_are_those_of_the_sizes(ops, M, N, K, fmt, swiglu):
+    """A product gives the same bits before and after larger ones of its stream, captured, and with a workspace larger than its own."""
+    group = 128 if fmt == 0 else 64
+    g = torch.Generator(device=DEV).manual_seed(M)
+    (w, sc, _), (w2, sc2, _) = (_weight(ops, N, K, fmt, group, g) for _ in range(2))
+    x = torch.randn(2048, K, generator=g, device=DEV).to(torch.bfloat16)
+
+    def product(rows):
+        if swiglu:
+            return ops.q4_gemm_swiglu(x[:rows], w, sc, w2, sc2, N, K, group, fmt)
+        return ops.q4_gemm_fused(x[:rows], w, sc, N, K, group, fmt)
+
+    form, need, _ = ops.q4f_plan(M, N, K, swiglu, fmt)
+    assert form == 3 and need > 0
+    first = product(M).clone()
+    product(1000), product(2048)
+    assert torch.equal(product(M), first)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=stream):
+        out = product(M)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, first) and torch.equal(product(M), first)
+    ws, y = torch.empty(4 * need, dtype=torch.uint8, device=DEV), torch.empty_like(first)
+    stream = torch.cuda.current_stream().cuda_stream
+    if swiglu:
+        rc = ops.load_library().lga_q4_gemm_swiglu(x.data_ptr(), w.data_ptr(), sc.data_ptr(), w2.data_ptr(), sc2.data_ptr(), y.data_ptr(),
+                                                   M, N, K, group, fmt, ws.data_ptr(), ws.numel(), stream)
+    else:
+        rc = ops.load_library().lga_q4_gemm_fused(x.data_ptr(), w.data_ptr(), sc.data_ptr(), None, None, y.data_ptr(), M, N, K, group,
+                                                  fmt, ws.data_ptr(), ws.numel(), stream)
+    assert rc == 0 and torch.equal(y, first)
+
+
+def test_two_threads_on_one_stream(ops):
+    """Products of two threads that share a stream: the partial sums of one never stand between the launches of the other."""
+    import threading
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    work = []
+    for M, N, K in ((300, 4096, 11008), (16, 4096, 4096)):
+        w, sc, _ = _weight(ops, N, K, 0, 128, g)
+        x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+        form, need, counters = ops.q4f_plan(M, N, K, 0, 0)
+        assert form == 3 and need > 0 and not counters
+        work.append(((x, w, sc, N, K, 128, 0), ops.q4_gemm_fused(x, w, sc, N, K, 128, 0).clone()))
+    torch.cuda.synchronize()
+    outs, errors = [[], []], []
+
+    def many(i):
+        try:
+            for _ in range(60):
+                outs[i].append(ops.q4_gemm_fused(*work[i][0]))
+        except Exception as e:  # pragma: no cover
+            errors.append(e)
+
+    threads = [threading.Thread(target=many, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for got, (_, want) in zip(outs, work):
+        assert len(got) == 60 and all(torch.equal(y, want) for y in got)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 4096, 4096), (93, 512, 1024), (300, 1032, 1408)])
+@pytest.mark.parametrize("fmt,group", [(0, 128), (1, 64)])
+@pytest.mark.parametrize("given", ["planned", "none", "small"])
+def test_scales_off_eight_bytes_and_small_workspaces(ops, M, N, K, fmt, group, given):
+    """Scales that the rings' form cannot load, and workspaces that do not hold its sums (those it asks for are not cleared): the
+    product is made in another way. Tolerance as in test_long_prompts."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    w, sc, wd = _weight(ops, N, K, fmt, group, g)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    h = x.float() @ wd.t()
+    form, need, _ = ops.q4f_plan(M, N, K, 0, fmt)
+    assert form == 3
+    size = {"planned": need, "none": 0, "small": 8192}[given]
+    ws = torch.full((max(size, 16),), 255, dtype=torch.uint8, device=DEV)
+    four = 4 // sc.element_size()  # scales that start on 4 bytes
+    off = torch.empty(sc.numel() + four, dtype=sc.dtype, device=DEV)[four:].view(sc.shape).copy_(sc)
+    for s in (sc, off):
+        y = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        rc = ops.load_library().lga_q4_gemm_fused(x.data_ptr(), w.data_ptr(), s.data_ptr(), None, None, y.data_ptr(), M, N, K, group, fmt,
+                                                  ws.data_ptr() if size else None, size, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        assert float(((y.float() - h).abs() - h.abs() * 2 ** -8).max()) <= 2e-4
 
 
 # the tiles of long prompts: 128, 192 and 256 rows a tile, one row past and one short of whole tiles, columns past the last whole
