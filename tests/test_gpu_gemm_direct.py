@@ -324,3 +324,41 @@ def test_short_prompts(ops, fmt, group, M, N, K, swiglu):
     y = ops.q4_gemm_swiglu(x, w, sc, w2, sc2, N, K, group, fmt).float()
     tol = 2 ** -7 * (1.1 * (a * b).abs() + 2 * ref.abs()) + 2 ** -8 * ref.abs() + 2e-3
     assert float(((y - ref).abs() - tol).max()) <= 0.0
+
+
+@pytest.mark.parametrize("fmt", [0, 2])
+def test_gated_unit_of_every_bf16_number(ops, fmt):
+    """The unit of unsplit SwiGLU products is ops.swiglu's, for all normal bf16 gates (identity weights, gates times 1), infinities
+    and NaN among them; and that unit is within four roundings of 2^-24 of float64, or where expf overflows 4e-37, of bf16's rounding."""
+    M, N, K = 512, 128, 256
+    v = torch.arange(65536, device=DEV, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(M, N)
+    v = torch.where(torch.isfinite(v) & (v.abs() >= 2.0 ** -126), v, torch.ones_like(v))  # (sums flush denormal products)
+    x = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
+    x[:, :N], x[:, N] = v, 1.0
+    one = torch.zeros(2, N, K, device=DEV)  # the gate's matrix and the up's
+    one[0, :, :N], one[1, :, N] = torch.eye(N, device=DEV), 1.0
+    every = torch.zeros(N, K, device=DEV)
+    every[:, 0] = 1.0
+
+    def product(x, a, b):
+        if fmt == 2:
+            return ops.q4_gemm_swiglu(x, a.to(torch.bfloat16), None, b.to(torch.bfloat16), None, N, K, 64, 2)
+        (qa, qb), sc = (((8 + m[:, ::2]) + 16 * (8 + m[:, 1::2])).to(torch.uint8).contiguous() for m in (a, b)), \
+            torch.ones(N, K // 128, dtype=torch.bfloat16, device=DEV)
+        return ops.q4_gemm_swiglu(x, qa, sc, qb, sc, N, K, 128, 0)
+
+    assert ops.q4f_plan(x.shape[0], N, K, 1, fmt)[1] == 0  # one launch: the unit stands in the product's
+    y = product(x, one[0], one[1])
+    unit = ops.swiglu(v.contiguous(), torch.ones_like(v))
+    assert torch.equal(y, unit)
+    exact = v.double() / (1 + torch.exp(-v.double()))
+    place = 2.0 ** (torch.frexp(exact.abs().clamp_min(2.0 ** -126))[1].double() - 8)  # of bf16 at that size
+    assert float(((y.double() - exact).abs() - 0.5 * place - 4 * 2 ** -24 * exact.abs()).max()) <= 4e-37
+    for special in (float("inf"), float("-inf"), float("nan")):  # (an infinite up: 0 times one is NaN in both products)
+        x = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
+        x[:, 0] = special
+        y = product(x, every, every)
+        both = torch.full((M, N), special, dtype=torch.bfloat16, device=DEV)
+        unit = ops.swiglu(both, both)
+        assert torch.equal(torch.nan_to_num(y.float(), 7.0), torch.nan_to_num(unit.float(), 7.0))
+        assert bool(torch.isinf(y).all()) == (special == float("inf"))
