@@ -669,10 +669,21 @@ def f32_row_fusable(*operands) -> bool:
     return all(t.shape[-1] % 4 == 0 and t.shape[-1] <= 8192 and t.data_ptr() % 16 == 0 for t in operands)
 
 
+def _f32_row(what: str, K: int, linear, *columns) -> None:
+    """A row of K values against a linear's matrix and bias; ``columns``: further vectors of its K columns."""
+    w, b = linear.weight, linear.bias
+    if w.dim() != 2 or w.shape[1] != K or (b is not None and b.numel() != w.shape[0]) or \
+            any(c is not None and c.numel() != K for c in columns):
+        sizes = [None if c is None else c.numel() for c in (b, *columns)]
+        raise ValueError(f"{what}: a row of {K} values, a matrix {tuple(w.shape)}, its bias and norm {sizes}")
+
+
 def f32_norm_linears(x, first, second=None):
     """One fp32 row, in one launch: for each of up to two (norm, linear, gelu) the linear of the LayerNorm of x, then gelu
     ("none" / "tanh", None: no activation) — ``f32_linear`` of ``layernorm``, to the bit."""
     K, args, outs = x.numel(), [], []
+    for norm, linear, _ in filter(None, (first, second)):
+        _f32_row("f32_norm_linears", K, linear, norm.weight, norm.bias)
     for part in (first, second):
         if part is None:
             args += [None, None, 0.0, None, None, 0, None, 0]
@@ -695,6 +706,12 @@ def f32_linears_sum(x1, linear1, x2, linear2, residual):
     if isinstance(x1, tuple):
         x1, ml, hs = x1
         parts = x1.shape[0]
+        if ml.numel() * hs != 2 * x1.numel():
+            raise ValueError(f"f32_linears_sum: {ml.numel()} scores and weights of ranges {tuple(x1.shape)} in heads of {hs}")
+    _f32_row("f32_linears_sum", x1.numel() // parts, linear1)
+    _f32_row("f32_linears_sum", x2.numel(), linear2)
+    if linear2.weight.shape[0] != N or residual.numel() != N:
+        raise ValueError(f"f32_linears_sum: {N} and {linear2.weight.shape[0]} outputs, {residual.numel()} residuals")
     y = torch.empty(1, N, dtype=torch.float32, device=x1.device)
     _check(load_library().lga_f32_linears_sum(
         _dev(x1, "x1", torch.float32), _opt(ml, "ml", torch.float32), parts, hs, _dev(linear1.weight, "weight1", torch.float32),

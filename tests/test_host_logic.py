@@ -340,3 +340,36 @@ def test_oracle_route_override_hook():
     other.route_override = swap_last
     got = other.forward(idx, torch.arange(6))
     assert torch.equal(got[:-1], want[:-1]) and not torch.equal(got[-1], want[-1])
+
+
+def test_fused_fp32_rows_check_their_shapes():
+    """The one-row launches take the length of a row from one operand: every other that does not fit it is refused before a launch."""
+    from types import SimpleNamespace as Part
+
+    from lit_gpt import ops
+
+    def linear(n, k, bias=None):
+        return Part(weight=torch.zeros(n, k), bias=None if bias is None else torch.zeros(bias))
+
+    def norm(k, bias=None):
+        return Part(weight=torch.zeros(k), bias=None if bias is None else torch.zeros(bias), eps=1e-5)
+
+    x, good = torch.zeros(1, 16), (norm(16, 16), linear(8, 16, 8), None)
+    for bad in ((norm(16), linear(8, 20), None), (norm(20), linear(8, 16), None), (norm(16, 12), linear(8, 16), None),
+                (norm(16), linear(8, 16, 4), "tanh"), (norm(16), linear(8, 12, 8), None)):
+        for parts in ((bad,), (good, bad)):
+            with pytest.raises(ValueError, match="f32_norm_linears"):
+                ops.f32_norm_linears(x, *parts)
+    row, wide, res = torch.zeros(1, 16), torch.zeros(1, 32), torch.zeros(1, 8)
+    ranges = torch.zeros(3, 16), torch.zeros(3, 4, 2), 4
+    for args in ((row, linear(8, 20), wide, linear(8, 32), res), (row, linear(8, 16), wide, linear(8, 64), res),
+                 (row, linear(8, 16), wide, linear(4, 32), res), (row, linear(8, 16), wide, linear(8, 32), res[:, :4]),
+                 (row, linear(8, 16, 9), wide, linear(8, 32), res), (ranges, linear(8, 20), wide, linear(8, 32), res),
+                 ((ranges[0], ranges[1][:2], 4), linear(8, 16), wide, linear(8, 32), res),
+                 ((ranges[0], ranges[1], 8), linear(8, 16), wide, linear(8, 32), res)):
+        with pytest.raises(ValueError, match="f32_linears_sum"):
+            ops.f32_linears_sum(*args)
+    for call in (lambda: ops.f32_norm_linears(x, good, good), lambda: ops.f32_linears_sum(row, linear(8, 16), wide, linear(8, 32), res),
+                 lambda: ops.f32_linears_sum(ranges, linear(8, 16), wide, linear(8, 32), res)):
+        with pytest.raises(RuntimeError, match="expected a GPU tensor"):  # (sound shapes come as far as the device)
+            call()
