@@ -430,7 +430,12 @@ struct F32AttnArgs {
   float* ml;  // [parts][H][2] the largest score and the sum of the weights; y holds [parts][H * hs] sums of weighted values
 };
 
-__host__ __device__ inline int f32_attention_chunk(int keys, int parts) { return ((keys + parts - 1) / parts + 31) / 32 * 32; }
+// Keys of a range, whole steps of the 32 keys of the narrowest rows: 64 at least, so that with lga_f32_attention_parts' number of
+// ranges they follow from the keys alone, and a token's bits not from the size of its cache
+__host__ __device__ inline int f32_attention_chunk(int keys, int parts) {
+  const int chunk = ((keys + parts - 1) / parts + 31) / 32 * 32;
+  return chunk < 64 ? 64 : chunk;
+}
 
 // grid (T, H): softmax(q . K^T * scale) . V over keys 0..pos[t] of the query's group; scores kept in LDS, exact max, fp32
 // exp and sums. LPK adjacent lanes hold a key's or value's row in pieces of four (hs <= 4 LPK), the other lanes of the 8
@@ -451,7 +456,7 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   float* kb = a.kc + (size_t)g * a.max_seq * hs;
   float* vb = a.vc + (size_t)g * a.max_seq * hs;
   const int L = (int)min(max(p + 1, 1L), (long)a.max_seq);
-  // this workgroup's keys: ranges of whole steps of the 32 keys of the narrowest rows, as many as there are keys for
+  // this workgroup's keys, of as many ranges as there are keys for
   const int chunk = FUSED && a.parts > 1 ? f32_attention_chunk(L, a.parts) : L, lo = range * chunk, hi = min(lo + chunk, L);
   if (FUSED) {
     const long rp = a.rope_pos[0];
@@ -753,7 +758,7 @@ extern "C" int lga_f32_attention_decode_parts(const float* qkv, float* k_cache, 
 }
 
 extern "C" int lga_f32_attention_parts(int n_head, int max_seq) {
-  // (ranges of 64 keys or more; eight are joined in one round of loads)
+  // (ranges of 64 keys or more, whatever the position; eight are joined in one round of loads)
   return n_head > 0 && max_seq > 0 ? std::min(8, (max_seq + 63) / 64) : 0;
 }
 

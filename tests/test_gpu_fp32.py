@@ -105,7 +105,7 @@ def test_one_row_norms_and_products(K, N1, N2, bias):
 
 
 def test_one_token_past_the_modules():
-    """A block's three launches give the bits of its modules called one by one (a hook keeps them apart)."""
+    """A block's three launches give the bits of its modules called one by one (a hook keeps them apart), behind up to 64 keys."""
     from generate.base import build_model
     from lit_gpt import Config
 
@@ -156,6 +156,61 @@ def test_ranges_of_keys(hs, H, G, p0, S):
     want = want @ one.weight.double().T + end
     assert (ops.f32_linears_sum(joined, one, x2, two, res).double() - want).abs().max() < 1e-5
     assert (ops.f32_linears_sum(y, one, x2, two, res).double() - want).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("p0", [0, 31, 32, 63, 64, 99, 127, 128, 200, 256, 447, 448, 600])
+def test_ranges_follow_the_keys(p0):
+    """The bits of a token's attention and output product are those of its keys, whatever the cache's size; behind up to 64 keys those
+    of the unsplit form."""
+    from types import SimpleNamespace as Part
+
+    from lit_gpt import ops
+
+    dev, H, hs, most = torch.device("cuda", 0), 3, 64, 1200
+    g = torch.Generator(device=dev).manual_seed(p0)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev)  # noqa: E731
+    k, v, qkv, pos = draw(1, H, most, hs), draw(1, H, most, hs), draw(1, 3 * H * hs), torch.tensor([p0], device=dev)
+    cos, sin = torch.ones(most, 2, device=dev), torch.zeros(most, 2, device=dev)
+    one, two = Part(weight=draw(5, H * hs), bias=draw(5)), Part(weight=draw(5, 8), bias=None)
+    x2, res, seen = draw(1, 8), draw(1, 5), []
+    for S in (p0 + 1, p0 + 2, 65, 128, 320, 448, 449, 512, most):
+        if S > p0:
+            args = (qkv, k[:, :, :S].contiguous(), v[:, :, :S].contiguous(), pos, pos, cos, sin, H, H, hs, 2, hs ** -0.5)
+            parts = ops.f32_attention_parts(H, S)
+            y = ops.f32_attention_decode(*args) if parts == 1 else ops.f32_attention_decode_parts(*args, parts)
+            seen.append(ops.f32_linears_sum(y, one, x2, two, res))
+            if p0 < 64:
+                seen.append(ops.f32_linears_sum(ops.f32_attention_decode(*args), one, x2, two, res))
+    assert len(seen) >= 3 and all(torch.equal(y, seen[0]) for y in seen)
+
+
+@pytest.mark.parametrize("S,p0", [(320, 300), (64, 40), (1024, 700)])
+def test_one_token_in_ranges_of_keys(S, p0):
+    """The model's step over a cache in ranges: within the modules' one by one, whose attention is one range (a hook keeps them
+    apart), by four roundings of 2^-24 a layer and product, and the same bits in a larger cache."""
+    from generate.base import build_model
+    from lit_gpt import Config, ops
+
+    dev = torch.device("cuda", 0)
+    assert (ops.f32_attention_parts(12, S) > 1) == (S > 64)
+    idx, pos, outs = torch.tensor([[5]], device=dev), torch.tensor([p0], device=dev), []
+    g = torch.Generator(device=dev).manual_seed(p0)
+    filled = torch.randn(2, 2, 12, p0, 64, generator=g, device=dev)
+    for size in (S, S + 448):
+        m = build_model(Config.from_name("pythia-160m", n_layer=2), quantize=None, device=dev, seed=1, max_seq_length=size, dtype=torch.float32)
+        for block, kv in zip(m.transformer.h, filled):
+            block.attn.kv_cache.k[0, :, :p0], block.attn.kv_cache.v[0, :, :p0] = kv
+        with torch.inference_mode():
+            outs.append(m(idx, pos).clone())
+    assert torch.equal(outs[0], outs[1])
+    handles = [block.attn.register_forward_hook(lambda mod, args, out: None) for block in m.transformer.h]
+    with torch.inference_mode():
+        apart = m(idx, pos)
+    for handle in handles:
+        handle.remove()
+    if S <= 64:
+        assert torch.equal(apart, outs[0])
+    assert float((apart - outs[0]).abs().max()) <= 2 * 6 * 4 * 2 ** -24 * float(apart.abs().max())
 
 
 def test_ranges_of_infinite_scores():
