@@ -53,8 +53,10 @@ int lgs_linear_glu_fits(int M, int n, int K, int groups);
 int lgs_linear_glu(const void* a, long lda, const void* w, long stride_w, long up_rows, void* y, long ldy, int M, int n,
                    int K, int batch, const int* a_rows, const int* z_start, int act, int clamped, float alpha, float limit,
                    float shift, lgs_stream_t stream);
-/* One row's unit from fp32 a [K] in one launch, in fp32: to the bits of lgs_linear and lgs_glu / lgs_glu_clamped in turn. K % 8 == 0,
- * a and w start on 16 bytes */
+/* One row's unit from fp32 a [K] in one launch, in fp32: to the bits of lgs_linear and lgs_glu / lgs_glu_clamped in turn where
+ * lgs_linear_glu_row_fits the product's columns (gate, up and what stands between); narrower ones are better made in those two, whose
+ * waves share a column's sum. K % 8 == 0, a and w start on 16 bytes */
+int lgs_linear_glu_row_fits(int columns, int K);
 int lgs_linear_glu_row(const float* a, const void* w, long up_rows, float* y, int n, int K, int act, int clamped, float alpha,
                        float limit, float shift, lgs_stream_t stream);
 /* ranges of K that a plain product of a bf16 A on bf16 weights (M > 8 rows) is best made in; 1: as one */

@@ -148,8 +148,11 @@ __global__ void __launch_bounds__(256) lin_gemv_kernel(LinArgs p) {
   }
 }
 
+static bool gemv_deep(long columns, int K) { return columns <= 512 && K >= 1024; }  // few columns: four waves per column
+
 // One row's gated unit in its input product's launch: a wave makes a gate column and the up column beside it, in lin_gemv_kernel's
-// order, and the unit of the two. One row of 2 x 5632 columns of 2048 values: product and unit 12.1 + 4.3 us and the gap between them, here 12.2.
+// order (but that of few columns: gemv_deep), and the unit of the two. us, product and unit / here: 2 x 520 columns of 2048 values
+// 5.9 / 4.1, 2 x 5632 14.2 / 11.8, of 4096 values 24.8 / 20.0, 2 x 11008 41.1 / 36.2, of 8192 75.0 / 70.5.
 template <bool AHEAD, bool CLAMPED>
 __global__ void __launch_bounds__(256) lin_glu_row_kernel(const float* __restrict__ a, const uint16_t* __restrict__ w, GluForm f,
                                                           float* __restrict__ y, int n, int K) {
@@ -662,7 +665,7 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
   }
   if (M <= 8 && !z_start && !a_rows) {
     const int R = N >= 16384 ? 4 : (N >= 4096 ? 2 : 1);
-    const bool deep = (long)N * batch <= 512 && K >= 1024;  // few columns: four waves per column
+    const bool deep = lgs::gemv_deep((long)N * batch, K);
     const dim3 grid(deep ? N : (N + 4 * R - 1) / (4 * R), batch);
 #define LGS_GEMV_R(MT, RR, KS)                                                                 \
   do {                                                                                         \
@@ -755,6 +758,8 @@ extern "C" int lgs_linear_glu(const void* a, long lda, const void* w, long strid
   if (rc) return rc;
   LGA_LAUNCH_RETURN();
 }
+
+extern "C" int lgs_linear_glu_row_fits(int columns, int K) { return columns > 0 && K > 0 && K % 8 == 0 && !lgs::gemv_deep(columns, K) ? 1 : 0; }
 
 extern "C" int lgs_linear_glu_row(const float* a, const void* w, long up_rows, float* y, int n, int K, int act, int clamped,
                                   float alpha, float limit, float shift, hipStream_t stream) {

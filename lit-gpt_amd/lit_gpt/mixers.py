@@ -892,8 +892,7 @@ class GatedFeedForward(InputReader):
         T, form = x.shape[0], dict(n=self.ff, up=self.off["up"], act=self.act, clamp=self.clamp)
         if self.off["gate"] != 0 or h is None:
             return False
-        if T == 1 and h.dtype == torch.float32 and w_in.dtype == torch.bfloat16 and h.is_contiguous() and \
-                w_in.shape[1] % 8 == 0 and h.data_ptr() % 16 == 0 and w_in.data_ptr() % 16 == 0:
+        if T == 1 and seq_ops.glu_row_fits(h, w_in):
             self._down(seq_ops.linear_glu_row(h, w_in, **form), x, accumulate)
             return True
         if not _tiles16(T, self.w_down) or not seq_ops.glu_fits(h, w_in, T, self.ff):

@@ -34,6 +34,7 @@ SIGNATURES = {
     "lgs_linear": [_P, _L, _L, _P, _I, _L, _P, _L, _L, _I, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _P, _I, _P],
     "lgs_linear_ksplit": [_I, _I, _I],
     "lgs_linear_glu_fits": [_I, _I, _I, _I],
+    "lgs_linear_glu_row_fits": [_I, _I],
     "lgs_linear_glu_row": [_P, _P, _L, _P, _I, _I, _I, _I, _F, _F, _F, _P],
     "lgs_linear_glu": [_P, _L, _P, _L, _L, _P, _L, _I, _I, _I, _I, _P, _P, _I, _I, _F, _F, _F, _P],
     "lgs_embed": [_P, _P, _I, _F, _P, _I, _I, _I, _P],
@@ -423,8 +424,15 @@ def linear_glu(a: torch.Tensor, w: torch.Tensor, *, M: int, n: int, up: int, act
     return out
 
 
+def glu_row_fits(a: Optional[torch.Tensor], w: torch.Tensor) -> bool:
+    """Whether ``linear_glu_row`` is to make the gated unit of one fp32 row ``a`` with the matrix w (rows, K)."""
+    return a is not None and a.dtype == F32 and w.dtype == torch.bfloat16 and a.is_contiguous() and a.data_ptr() % 16 == 0 and \
+        w.data_ptr() % 16 == 0 and bool(load_library().lgs_linear_glu_row_fits(w.shape[0], w.shape[1]))
+
+
 def linear_glu_row(a: torch.Tensor, w: torch.Tensor, *, n: int, up: int, act: int = 0, clamp: Optional[tuple] = None) -> torch.Tensor:
-    """``linear_glu`` of one fp32 row, in fp32: (1, n), to the bits of ``linear`` and ``glu`` / ``glu_clamped`` in turn."""
+    """``linear_glu`` of one fp32 row, in fp32: (1, n); where ``glu_row_fits``, to the bits of ``linear`` and ``glu`` /
+    ``glu_clamped`` in turn."""
     rows, K = w.shape
     if a.numel() != K or rows < up + n:
         raise ValueError("linear_glu_row: shapes")

@@ -8,17 +8,17 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
 
 
-def layered(design):
+def layered(design, width=64, ff=96):
     from lit_gpt.config import LayeredConfig
     from lit_gpt.layered import LayeredGPT
 
-    mlp = {"kind": "dense", "ff": 96, "limit": 7.0}
+    mlp = {"kind": "dense", "ff": ff, "limit": 7.0}
     if design == "Rigulorn":
         layer = {"type": "mamba2", "mixer": {"heads": 4, "vdim": 16, "state": 16, "groups": 2, "norm_groups": 2, "conv": 4}}
         more = {"embedding": {"scale": 1.0}, "streams": 2}
     else:
-        layer, more = {"type": "mingru", "mixer": {"width": 64}}, {}
-    config = LayeredConfig.from_dict(dict(architecture=design, vocab=50, width=64, norm={"eps": 1e-5}, layers=[dict(layer, mlp=mlp)],
+        layer, more = {"type": "mingru", "mixer": {"width": width}}, {}
+    config = LayeredConfig.from_dict(dict(architecture=design, vocab=50, width=width, norm={"eps": 1e-5}, layers=[dict(layer, mlp=mlp)],
                                           **more))
     return LayeredGPT(config, LayeredGPT.random_weights(config, seed=3), device=DEV, dtype=torch.bfloat16)
 
@@ -50,6 +50,29 @@ def test_gated_feed_forward(design, kind):
                 handle.remove()
             assert calls == [ff[0]], n
             assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("design", ["Rigulorn", "Fazolorn"])
+@pytest.mark.parametrize("width,ff", [(1024, 200), (1024, 256), (1024, 264), (512, 200)])
+def test_one_row_of_a_gated_feed_forward(design, width, ff):
+    """One token: the unit in its input product's launch and apart give the same bits, on both sides of the line below which
+    the product's waves share its columns."""
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import GatedFeedForward, StepBatch
+
+    m = layered(design, width, ff)
+    ff_of = [x for x in m.modules() if isinstance(x, GatedFeedForward)]
+    w = torch.empty(2 * (ff + -ff % 8), width, dtype=torch.bfloat16, device=DEV)
+    assert seq_ops.glu_row_fits(torch.zeros(1, width, device=DEV), w) == (width < 1024 or ff > 256)
+    m.set_kv_cache(1, 64)
+    with torch.inference_mode():
+        step = StepBatch.build([(0, 0, [7])], DEV)
+        want = m.logits(m.forward_step(step)).clone()
+        handle = ff_of[0].register_forward_hook(lambda *_: None)
+        try:
+            assert torch.equal(m.logits(m.forward_step(step)), want)
+        finally:
+            handle.remove()
 
 
 def test_parallel_block_in_fp32():
