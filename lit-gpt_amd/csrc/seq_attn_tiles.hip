@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(512) attn_tiles_kernel(AttnTileArgs p) {
   constexpr int kExchange = 4 * 64 * (DT * 16 + 2) * 4, kTurn = 4 * 32 * (DV + 4) * 4;
   constexpr int kLds = ST * STAGE > kExchange ? (ST * STAGE > kTurn ? ST * STAGE : kTurn)
                                               : (kExchange > kTurn ? kExchange : kTurn);
-  static_assert(kLds <= 163840, "LDS");
+  static_assert(kLds <= kCuLds && (DC != 8 || DT != 4 || MAPS != 1 || PARTS != 1 || kLds == kPromptAttnLds), "LDS");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
   const AttnArgs& a = p.a;
   const int tid = threadIdx.x, lane = tid & 63, lq = lane & 31, hh = lane >> 5;

@@ -15,6 +15,9 @@
 namespace lgs {
 using namespace lga;
 
+constexpr int kCuLds = 163840;         // bytes of a compute unit
+constexpr int kPromptAttnLds = 98304;  // ... of a workgroup of attn_tiles_kernel's form for keys and values of 128
+
 enum Act { kActNone = 0, kActRelu2 = 1, kActGeluTanh = 2, kActSilu = 3, kActSigmoid = 4 };
 
 __device__ __forceinline__ float gelu_tanh_f(float z) {

@@ -545,10 +545,16 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
 //
 // grid (B * H * ceil(dv / 8) rounded up to 8). Lane l of a column: rows 64 j + 2 l + e, j, e < 2.
 // (PC: a decay per channel. The loads ahead carry no branches: behind one, every batch would wait for the next one's loads.)
+struct DeltaWide {
+  static constexpr int D = 128, CW = 8, TB = 32, ROW = 3 * D + 4 * CW;  // staged floats per token: q | k | g | (v, beta, k . q, -) per column
+  static constexpr int STAGED = (TB + 1) * ROW, LDS = (STAGED + TB * CW) * 4;  // (a batch's last token reads one row ahead)
+  static constexpr int ALONE = 28 * 1024;  // more of it that nobody uses (gated_delta_wide_launch)
+  static_assert(2 * (LDS + ALONE) > kCuLds && LDS + ALONE + kPromptAttnLds > kCuLds, "alone on a CU");
+};
 template <bool DELTA, bool PC>
 __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
-  constexpr int D = 128, CW = 8, TB = 32, ROW = 3 * D + 4 * CW;  // staged floats per token: q | k | g | (v, beta, k . q, -) per column
-  __shared__ __attribute__((aligned(16))) float st[(TB + 1) * ROW];  // (a batch's last token reads one row ahead)
+  constexpr int D = DeltaWide::D, CW = DeltaWide::CW, TB = DeltaWide::TB, ROW = DeltaWide::ROW;
+  __shared__ __attribute__((aligned(16))) float st[DeltaWide::STAGED];
   __shared__ float os[TB * CW];
   const int tid = threadIdx.x, l = tid & 31, cw = tid >> 5;
   const int per_xcd = (p.items + 7) / 8;  // (a head's column blocks on one XCD, as above)
@@ -673,10 +679,10 @@ static void gated_delta_wide_launch(DeltaArgs p, int B, bool plain, hipStream_t 
   p.ncb = (p.dv + 7) / 8;
   p.items = B * p.H * p.ncb;
   const unsigned grid = (unsigned)((p.items + 7) / 8 * 8);
-  // Up to half as many workgroups as the chip has CUs: 28 KB that nobody uses, 84 with the kernel's own, keep a CU's LDS from two
-  // of them and from one beside an attention's 98. The rule of 8 heads runs beside its layer's attention on another stream: 354
+  // Up to half as many workgroups as the chip has CUs: LDS that nobody uses keeps a CU from two of them and from one beside a
+  // workgroup of the prompts' attention (kPromptAttnLds). The rule of 8 heads runs beside its layer's attention on another stream: 354
   // to 424 us of 2048 tokens where they share CUs, 274 on its own ones (a raised wave priority changed nothing).
-  const unsigned alone = p.items <= 128 ? 28 * 1024 : 0;
+  const unsigned alone = p.items <= 128 ? DeltaWide::ALONE : 0;
   if (p.per_channel) {
     if (plain) gated_delta_wide_kernel<false, true><<<grid, 256, alone, stream>>>(p);
     else gated_delta_wide_kernel<true, true><<<grid, 256, alone, stream>>>(p);
