@@ -189,8 +189,9 @@ __global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restr
 }
 
 // One row, K a multiple of 4: up to two products of a norm of the row each (f32_linear_kernel of f32_layernorm_kernel's row, to
-// the bit). A workgroup makes its norm anew, in LDS, while its first weights are on their way; a wave then one output after the
-// other. pythia-160m (768 -> 2304 and 3072): norms and products in three launches 16.2 us, in this one 7.6.
+// the bit). A workgroup makes its norm anew, in LDS, a wave then one output after the other. The first weights are loaded ahead of the
+// row, and loads return in order: the statistics wait for both, the sums for nothing more. pythia-160m (768 -> 2304 and 3072):
+// norms and products in three launches 16.2 us, in this one 7.6.
 struct F32NormLinear {
   const float *nw, *nb;
   float eps;
@@ -264,8 +265,8 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 }
 
 // One row: y = ((x2 W2^T + b2) + (x1 W1^T + b1)) + res, a wave per output, both products in f32_linear_kernel's order. Bound by
-// one round of latency: all loads of a block of 768 columns beside 3072 are in flight at once. Two launches 13.7 us, one 8.0
-// (8.9 with ranges of keys to join).
+// latency: the weights of a block of 768 columns beside 3072 are in flight at once, x1 and x2 come behind them, and a join of ranges
+// of keys waits for its own loads and the weights ahead of those. Two launches 13.7 us, one 8.0 (8.9 with ranges to join).
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
   float* y;

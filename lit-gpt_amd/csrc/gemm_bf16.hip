@@ -1,6 +1,6 @@
 // Prompt products with bf16 weights, Y = X W^T with bias / residual, and fc_1 || fc_2 + SwiGLU, on the pipelined tiles of
-// gemm_tiles.h. The weights are the tile's A: a lane then holds four neighbouring columns of one row of Y, which it
-// stores as 8 bytes, and for SwiGLU a wave's fragments alternate between the two matrices, so that the pair of a column
+// gemm_tiles.h. The weights are the tile's A: two lanes then hold eight neighbouring columns of one row of Y, four each, swap halves
+// and store 16 bytes, and for SwiGLU a wave's fragments alternate between the two matrices, so that the pair of a column
 // meets in one lane.
 //
 // Bound as the tiles are; with few rows by the weights on their way from memory. With weights from memory, us on stages of 32

@@ -1,5 +1,5 @@
 // Prefill GEMM with weights dequantized in registers: the same products as gemm_q4f.hip (Y = X . bf16(dequant(W))^T with
-// bias / residual, and fc_1 || fc_2 + SwiGLU) for prompts whose weight tiles serve few rows.
+// bias / residual, and fc_1 || fc_2 + SwiGLU) for prompts whose weight tiles serve few rows; what gemm_q4r.hip leaves of them.
 //
 // gemm_q4f.hip stages packed weights in LDS, dequantizes them into a bf16 image there and reads fragments back: three
 // LDS round trips and a barrier per 64 values of K, which a tile of few rows cannot hide (0.75 us a step). Here a weight

@@ -357,9 +357,10 @@ static void go_rows(const KArgs& k, int fn, hipStream_t stream) {
 // higher one, and their start and end; several ranges of K cost a second launch and the traffic of their sums, at a copy's rate. Of
 // 462 products of 16 to 2048 rows of twelve matrices the choice is 1.1 % from the fastest of up to ten forms and ranges in the
 // mean, and the ranges of the forms that stood here before 2.5 % (nf4 517 rows of 4096 x 11008 77 / 69 us, int4 400 of 8192 x
-// 28672 217 / 195; int4 128 of 11008 x 4096 with SwiGLU 39.0 / 40.7). us of a pair for 256, 192 and 128 rows, measured on 256 workgroups of K 4096: int4 2.93,
-// 2.30, 1.75 (4740, 3870, 3140 clocks, of which 4096, 3072, 2048 of matrix instructions), codebooks 3.22, 2.67, 2.12 (5560,
-// 5050, 4470: sixteen more instructions per eight weights); for 96, 64 and 32 rows from whole products of 86 to 240 workgroups.
+// 28672 217 / 195; int4 128 of 11008 x 4096 with SwiGLU 39.0 / 40.7). us of a pair for 256, 192 and 128 rows, measured on 256
+// workgroups of K 4096: int4 2.93, 2.30, 1.75 (4740, 3870, 3140 clocks, of which 4096, 3072, 2048 of matrix instructions),
+// codebooks 3.22, 2.67, 2.12 (5560, 5050, 4470: sixteen more instructions per eight weights); for 96, 64 and 32 rows from whole
+// products of 86 to 240 workgroups.
 // us on gemm_q4f.hip's tiles / here, int4 with weights from memory: 2048 rows of 12288 x 4096 209 / 197, 4096 x 4096 75 / 68,
 // 11008 x 4096 with SwiGLU 374 / 311, 4096 x 11008 194 / 171; 517 rows 118 / 65, 71 / 37, 194 / 126, 126 / 70; 300 rows 70 / 56,
 // -, 122 / 76, 90 / 49; nf4 2048 rows 233 / 212, 82 / 82, 429 / 341, 209 / 202.

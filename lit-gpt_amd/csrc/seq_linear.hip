@@ -23,7 +23,8 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // KS 4: short and deep matrices; the four waves of a workgroup share its R columns, each a quarter of K
 // AHEAD: the weights of four passes over K on their way together, for few columns a wave, whose time is trips to memory. us before /
 // with, weights from memory: 2048 x 5632 10.7 / 10.4, two rows 16.0 / 11.4, 11264 x 2048 13.2 / 12.1; with more columns or
-// deeper rows the registers cost more waves than the trips take (22016 x 4096 38.8 / 41.6)
+// deeper rows the registers cost more waves than the trips take (22016 x 4096 38.8 / 41.6). The row's own values come pass by pass,
+// behind the weights.
 template <bool WF32, int MT, int R, int KS, bool AHEAD>
 __global__ void __launch_bounds__(256) lin_gemv_kernel(LinArgs p) {
   __shared__ float shared_acc[KS > 1 ? 4 * MT * R : 1];
