@@ -111,28 +111,57 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, in
   const int wm = wave % WM, wn = wave / WM, l31 = lane & 31, hi = lane >> 5;
   const int mw = m0 + wm * FM * 32, nw = n0 + wn * FN * 32;
   const bool inside = mw + FM * 32 <= Mz && nw + FN * 32 <= p.N;
-  auto each = [&](auto in, auto* y, long ld, auto&& put) {  // y: (mw, nw)
+  // y: (mw, nw). R rows of a fragment at a time: the old values of sums on their way together, then the results, then the stores.
+  // (More, and all accumulators are fetched ahead, into memory; row by row, the latency of a load or an activation stands
+  // between any two rows.)
+  constexpr int FEW = FM * FN > 12 ? 1 : 4;
+  auto each = [&](auto in, auto sums, auto past, auto rows_at_once, auto* y, long ld, auto&& make) __attribute__((always_inline)) {
+    constexpr bool IN = decltype(in)::value, SUMS = decltype(sums)::value;
+    constexpr int R = decltype(rows_at_once)::value;
     const unsigned at = (unsigned)(hi * 4 * (int)ld + l31);
+    const int rows = Mz - 1 - mw - hi * 4, cols = p.N - 1 - nw - l31;  // a lane's last ones
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = i * 32 + (e >> 2) * 8 + (e & 3);
-        auto* row = y + (long)r * ld;
-        if (decltype(in)::value || mw + hi * 4 + r < Mz)
+      for (int q = 0; q < 16; q += R) {
+        const int r0 = i * 32 + q / 4 * 8 + q % 4;
+        float old[R][FN];
+        std::remove_reference_t<decltype(*y)> v[R][FN];
+        if constexpr (SUMS) {
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
-            if (decltype(in)::value || nw + l31 + j * 32 < p.N) put(row + j * 32 + at, j, acc[i][j][e]);
-        __builtin_amdgcn_sched_barrier(0);  // (or all accumulators are fetched ahead, into memory)
+          for (int e = 0; e < R; ++e)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)  // (past the end the last ones, not used)
+              old[e][j] = IN ? (y + (long)(r0 + e) * ld + j * 32)[at] : y[(long)(min(r0 + e, rows) + hi * 4) * ld + l31 + min(j * 32, cols)];
+        }
+#pragma unroll
+        for (int e = 0; e < R; ++e)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) v[e][j] = make(j, acc[i][j][q + e], SUMS ? old[e][j] : 0.0f);
+#pragma unroll
+        for (int e = 0; e < R; ++e) {
+          auto* row = y + (long)(r0 + e) * ld;
+          if (IN || r0 + e <= rows)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+              if (IN || j * 32 <= cols) {
+                if constexpr (decltype(past)::value) __builtin_nontemporal_store(v[e][j], row + j * 32 + at);
+                else (row + j * 32)[at] = v[e][j];
+              }
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
   };
-  constexpr std::true_type in{};
-  constexpr std::false_type some{};
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  constexpr std::integral_constant<int, 1> one{};
+  constexpr std::integral_constant<int, FEW> few{};
+  auto put = [&](auto sums, auto past, auto n, auto* y, long ld, auto&& make) __attribute__((always_inline)) {
+    if (inside) each(yes, sums, past, n, y, ld, make);
+    else each(no, sums, past, n, y, ld, make);
+  };
   if (p.ksplit > 1) {
-    float* y = p.part + ((size_t)split * p.M + mw) * p.N + nw;
-    auto put = [](float* o, int, float v) { *o = v; };
-    if (inside) each(in, y, p.N, put);
-    else each(some, y, p.N, put);
+    put(no, no, one, p.part + ((size_t)split * p.M + mw) * p.N + nw, p.N, [](int, float v, float) { return v; });
     return;
   }
   float bias[FN];
@@ -141,20 +170,24 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, in
   const long at = (long)z * p.sy + (long)(r_lo + mw) * p.ldy + nw;
   if (kActsFit<FM, FN> && p.act != kActNone) {
     if constexpr (kActsFit<FM, FN>) {
-      if (p.y16) each(some, p.y16 + at, p.ldy, [&](uint16_t* o, int j, float v) { *o = f2bf(act_f(p.act, v + bias[j])); });
-      else each(some, p.y + at, p.ldy, [&](float* o, int j, float v) {
-        v = act_f(p.act, v + bias[j]);
-        *o = p.accumulate ? *o + v : v;
-      });
+      // (a loop of its own for each activation: a choice per result keeps them from standing among one another)
+      auto act = [&](auto kind) __attribute__((always_inline)) {
+        auto f = [&](int j, float v, float) { return act_f(decltype(kind)::value, v + bias[j]); };
+        if (p.y16) each(no, no, no, few, p.y16 + at, p.ldy, [&](int j, float v, float) { return f2bf(f(j, v, 0.0f)); });
+        else each(no, no, no, few, p.y + at, p.ldy, f);
+      };
+      if (p.accumulate) each(no, yes, no, few, p.y + at, p.ldy, [&](int j, float v, float old) { return old + act_f(p.act, v + bias[j]); });
+      else if (p.act == kActRelu2) act(std::integral_constant<int, kActRelu2>{});
+      else if (p.act == kActGeluTanh) act(std::integral_constant<int, kActGeluTanh>{});
+      else if (p.act == kActSilu) act(std::integral_constant<int, kActSilu>{});
+      else act(std::integral_constant<int, kActSigmoid>{});
     }
   } else if (p.y16) {
-    each(some, p.y16 + at, p.ldy, [&](uint16_t* o, int j, float v) { *o = f2bf(v + bias[j]); });
+    put(no, no, one, p.y16 + at, p.ldy, [&](int j, float v, float) { return f2bf(v + bias[j]); });
   } else if (p.accumulate) {
-    each(some, p.y + at, p.ldy, [&](float* o, int j, float v) { *o += v + bias[j]; });
+    put(yes, no, few, p.y + at, p.ldy, [&](int j, float v, float old) { return old + (v + bias[j]); });
   } else {
-    auto put = [&](float* o, int j, float v) { __builtin_nontemporal_store(v + bias[j], o); };
-    if (inside) each(in, p.y + at, p.ldy, put);
-    else each(some, p.y + at, p.ldy, put);
+    put(no, yes, one, p.y + at, p.ldy, [&](int j, float v, float) { return v + bias[j]; });
   }
 }
 

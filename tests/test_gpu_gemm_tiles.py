@@ -65,6 +65,32 @@ def test_grouped_product(rows, gather):
     assert (y[M:] == 3.0).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(1279, 12031, 256), (1023, 10753, 128), (3327, 2305, 1024), (769, 6655, 1024), (575, 4097, 128),
+                                   (130, 1000, 192), (40, 260, 64), (256, 512, 64)])
+@pytest.mark.parametrize("act", [0, 1, 2, 3, 4])
+def test_results_of_every_kind(M, N, K, act):
+    """fp32, bf16 and sums, each activation, tiles inside and past the ends, rows apart: the activation of the plain result, which
+    test_product holds against float64, within a few roundings of 2^-24 (of tanh, exponential and products) and one to bf16."""
+    from lit_gpt import seq_ops
+
+    dev, ld = torch.device("cuda", 0), N + 5
+    a, w, b = operands(M, N, K, dev)
+    z = torch.empty(M, N, device=dev)
+    seq_ops.linear(a, w, M=M, N=N, K=K, y=z, lda=K, ldy=N, bias=b, ksplit=1)
+    z = z.double()
+    want = {0: z, 1: z.clamp_min(0) ** 2, 2: torch.nn.functional.gelu(z, approximate="tanh"), 3: torch.nn.functional.silu(z),
+            4: torch.sigmoid(z)}[act]
+    old = torch.randn(M, ld, device=dev)
+    for kind in ("fp32", "bf16", "sums"):
+        y = old.to(torch.bfloat16) if kind == "bf16" else old.clone()
+        seq_ops.linear(a, w, M=M, N=N, K=K, y=y, lda=K, ldy=ld, bias=b, act=act, accumulate=kind == "sums", ksplit=1)
+        assert torch.equal(y[:, N:], old[:, N:].to(y.dtype)), kind
+        got = y[:, :N].double() - (old[:, :N].double() if kind == "sums" else 0.0)
+        size = want.abs() + (old[:, :N].double().abs() if kind == "sums" else 0.0)
+        bound = (2.0 ** -8 if kind == "bf16" else 0.0) * want.abs() + 16 * 2.0 ** -24 * (size + z.abs().clamp_max(4.0))
+        assert bool(((got - want).abs() <= bound).all()), kind
+
+
 def test_strided_batch():
     """Products side by side, A in columns of wider rows, K in one and in several stages."""
     from lit_gpt import seq_ops
