@@ -248,8 +248,8 @@ static int go_rows(const KArgs& k, int mf, hipStream_t stream) {
 
 }  // namespace pd
 
-// Which products come here, of those that gemm_q4r.hip leaves (q4r_plan: one matrix, up to 64 rows) or has no aligned scales for (all
-// with SwiGLU; us here / on the LDS image's tiles; NK = N x K of one matrix):
+// Which products come here, of those that gemm_q4r.hip leaves (q4r_plan: up to 96 rows) or has no aligned scales for (us here / on
+// the LDS image's tiles; NK = N x K of one matrix):
 //   up to 32 rows   all but NK <= 2^24, where two launches are not repaid (int4 16 x 4096 x 4096: 18 / 15)
 //   up to 96 rows   all (int4 64 x 4096 x 4096: 19 / 23)
 //   up to 128 rows  beyond 2^24 (int4 4096 x 4096: 31 / 26; 12288 x 4096: 37 / 42); SwiGLU from 2^26 (int4 11008 x 4096:

@@ -365,12 +365,17 @@ static void go_rows(const KArgs& k, int fn, hipStream_t stream) {
 // 11008 x 4096 with SwiGLU 374 / 311, 4096 x 11008 194 / 171; 517 rows 118 / 65, 71 / 37, 194 / 126, 126 / 70; 300 rows 70 / 56,
 // -, 122 / 76, 90 / 49; nf4 2048 rows 233 / 212, 82 / 82, 429 / 341, 209 / 202.
 // Up to 128 rows against gemm_q4d.hip's form, or the tiles where that is not taken, weights from memory:
-//   nf4 93 rows    28672 x 8192 with SwiGLU 150 / 124, 8192 x 28672 84 / 71, 10240 x 8192 41 / 39, 8192 x 8192 36 / 35
-//   nf4 64 rows    28672 x 8192 with SwiGLU 133 / 105, 8192 x 28672 71 / 62; 4096 x 4096 21 / 22, 6144 x 4096 23.2 / 23.6
-//   int4 64 rows   12288 x 4096 25.5 / 24.1, 11008 x 4096 with SwiGLU 37 / 33, 4096 x 4096 20.4 / 20.4, 4096 x 11008 23.3 / 24.7
-//   int4 128 rows  11008 x 4096 with SwiGLU 63 / 42, 4096 x 11008 35 / 30, 4096 x 4096 28 / 22
-//   32 rows        int4 4096 x 4096 19.6 / 14.6, 11008 x 4096 with SwiGLU 32 / 28; 4096 x 11008 20.1 / 21.1, nf4 10240 x 8192
-//                  28.9 / 30.0, 28672 x 8192 with SwiGLU 108 / 98: beyond 2^24 values one matrix stays in gemm_q4d.hip's form
+//   97 .. 128      int4 128 rows 11008 x 4096 with SwiGLU 63 / 42, 4096 x 11008 35 / 30, 4096 x 4096 28 / 22: all here
+//   33 .. 96       nf4 93 rows 28672 x 8192 with SwiGLU 150 / 124, 8192 x 28672 84 / 71; int4 64 rows 12288 x 4096 25.5 / 24.1, 11008 x
+//                  4096 with SwiGLU 37 / 33. One matrix of up to 8192 columns between 2^24 and 2^26 values stays there: int4 80
+//                  rows 5120 x 5120 26.1 / 27.1, 8192 x 4096 24.2 / 28.3, 4096 x 8192 25.8 / 29.4, nf4 24.6 / 27.3 and 25.8 / 28.4
+//                  (4096 x 4096 23.5 / 22.1 and 24.2 / 23.2); up to 64 rows so do smaller ones of codebooks (4096 x 4096 21 / 22).
+//                  And so do 8192 columns, whose partial sums it writes faster than those of 8064 (16.1 for 18.0 us, not
+//                  explained): int4 48 rows, K 1536 11.6 / 15.6, with SwiGLU 14.9 / 19.6 (7168: 14.4 / 13.9, 18.0 / 18.1)
+//   2 .. 32        int4 4096 x 4096 19.6 / 14.6, 11008 x 4096 with SwiGLU 32 / 28, nf4 28672 x 8192 with SwiGLU 108 / 98; 4096 x 11008
+//                  20.1 / 21.1, nf4 10240 x 8192 28.9 / 30.0: beyond 2^24 values one matrix stays there, and with SwiGLU one of up
+//                  to 8192 columns and 2^26 values: int4 16 rows 4096 x 8192 21.5 / 24.3, 8192 x 8192 31.8 / 34.7, 4096 x 11008
+//                  24.8 / 26.4, nf4 24.0 / 25.0, 36.3 / 36.9, 28.4 / 30.4
 Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, bool ranges) {
   Q4rPlan p{0, 0, 0, 0, 0};
   // up to 16 ranges, and up to 128 MB of their sums
@@ -378,8 +383,11 @@ Q4rPlan q4r_plan(int M, int N, int K, bool dual, int kernel_fmt, bool ranges) {
   const int most = ranges ? (int)std::max<size_t>(std::min<size_t>(((size_t)128 << 20) / plane, 16), 1) : 1;
   const size_t nk = (size_t)N * K, one = 1;
   if (K % 128 != 0) return p;
-  if (!dual && M <= 32 && nk > one << 24) return p;
-  if (!dual && M > 32 && M <= 64 && nk < one << 26 && (kernel_fmt == 1 || (nk > one << 24 && N <= 8192))) return p;
+  const bool middle = N <= 8192 && nk > one << 24;  // columns by columns of K
+  if (M <= 32 && (dual ? middle && nk <= one << 26 : nk > one << 24)) return p;
+  if (!dual && M > 32 && M <= 64 && kernel_fmt == 1 && nk < one << 26) return p;
+  if (!dual && M > 32 && M <= 96 && middle && nk < one << 26) return p;
+  if (N == 8192 && K >= 1536 && K <= 2560 && M > 32 && M <= (dual ? 64 : 96)) return p;
   const int cols = dual ? 128 : 256, np = K / 128;
   p.nt = (N + cols - 1) / cols;
   constexpr int forms[] = {8, 6, 4, 3, 2, 1};

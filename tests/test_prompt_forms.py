@@ -15,7 +15,11 @@ def plan(M, N, K, swiglu=0, fmt=1):
 
 @pytest.mark.parametrize("fmt", [0, 1, 3])
 @pytest.mark.parametrize("M,size,swiglu,form", [
-    (2, SMALL, 0, RING), (32, SMALL, 0, RING), (32, LARGE, 0, REGISTERS), (32, LARGE, 1, RING), (65, SMALL, 0, RING),
+    (2, SMALL, 0, RING), (32, SMALL, 0, RING), (32, LARGE, 0, REGISTERS), (32, SMALL, 1, RING), (32, LARGE, 1, REGISTERS),
+    (32, (8192, 8192), 1, REGISTERS), (32, (8200, 8192), 1, RING), (32, (11008, 4096), 1, RING), (33, LARGE, 1, RING), (65, SMALL, 0, RING),
+    (96, LARGE, 0, REGISTERS), (96, (8192, 8064), 0, REGISTERS), (96, (8200, 4096), 0, RING), (97, LARGE, 0, RING),
+    (33, (8192, 2048), 0, REGISTERS), (96, (8192, 1536), 0, REGISTERS), (97, (8192, 2048), 0, RING), (64, (8192, 2560), 1, REGISTERS),
+    (65, (8192, 2560), 1, RING), (48, (8192, 2688), 1, RING), (64, (8184, 2048), 1, RING),
     (64, (8192, 8192), 0, RING), (96, SMALL, 0, RING), (96, SMALL, 1, RING), (97, SMALL, 0, RING), (97, LARGE, 1, RING),
     (97, HUGE, 1, RING), (128, LARGE, 0, RING), (128, HUGE, 1, RING), (129, HUGE, 1, RING), (129, HUGE, 0, RING),
     (256, (16384, 4096), 0, RING), (256, (28672, 4096), 0, RING), (129, SMALL, 0, RING), (257, SMALL, 0, RING),
@@ -27,7 +31,7 @@ def test_four_bit_weights(fmt, M, size, swiglu, form):
 @pytest.mark.parametrize("M,size,int4,nf4", [(33, SMALL, RING, REGISTERS), (64, SMALL, RING, REGISTERS), (64, LARGE, REGISTERS, REGISTERS),
                                              (64, (8200, 4096), RING, REGISTERS), (64, (4096, 128), RING, REGISTERS)])
 def test_formats_apart(M, size, int4, nf4):
-    """33 to 64 rows of one matrix below 2^26 values: codebooks stay in gemm_q4d.hip's form, int4 of large ones up to 8192 columns."""
+    """33 to 64 rows of one matrix below 2^26 values: codebooks stay in gemm_q4d.hip's form, int4 only between 2^24 and 2^26."""
     assert plan(M, *size, 0, 0)[0] == int4 and plan(M, *size, 0, 1)[0] == nf4 and plan(M, *size, 0, 3)[0] == nf4
 
 
