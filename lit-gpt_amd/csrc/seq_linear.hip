@@ -21,10 +21,11 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // ------------------------------------------------------------------------------------------------ GEMV, M <= 8
 // R output columns per wave: 4 for tall matrices (more loads in flight per lane), fewer for short ones (more waves)
 // KS 4: short and deep matrices; the four waves of a workgroup share its R columns, each a quarter of K
-// AHEAD: the weights of four passes over K on their way together, for few columns a wave, whose time is trips to memory. us before /
-// with, weights from memory: 2048 x 5632 10.7 / 10.4, two rows 16.0 / 11.4, 11264 x 2048 13.2 / 12.1; with more columns or
-// deeper rows the registers cost more waves than the trips take (22016 x 4096 38.8 / 41.6). The row's own values come pass by pass,
-// behind the weights.
+// AHEAD: the weights of four passes over K on their way together, for few columns a wave, whose time is trips to memory. us without /
+// with, weights from memory: 1024 x 8192 11.4 / 9.7, 2048 x 4096 8.0 / 7.7, two rows 12.3 / 8.9, 11264 x 2048 13.0 / 12.0; where more
+// waves stand side by side the registers cost more of them than the trips take: 3584 x 4096 9.2 / 9.8 (3072: 8.8 / 8.9), 4088 x 8192
+// 17.5 / 18.9, 22016 x 4096 38.8 / 41.6; and passes past a short row's end cost theirs: 2048 x 1024 3.5 / 3.6, 8192 x 1024 5.8 / 6.5,
+// 16376 x 1536 12.3 / 12.9. The row's own values come pass by pass, behind the weights.
 template <bool WF32, int MT, int R, int KS, bool AHEAD>
 __global__ void __launch_bounds__(256) lin_gemv_kernel(LinArgs p) {
   __shared__ float shared_acc[KS > 1 ? 4 * MT * R : 1];
@@ -680,7 +681,8 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
     else if (deep) LGS_GEMV_R(MT, 1, 4);   \
     else LGS_GEMV_R(MT, 1, 1);             \
   } while (0)
-    if (!w_f32 && !deep && M <= 2 && K >= 1024 && (R == 1 || (R == 2 && M == 1 && K <= 2048))) {
+    const bool ahead = M == 2 ? R == 1 && K >= 1024 : M == 1 && (R == 1 ? N <= 3072 && K >= 1536 : R == 2 && K > 1536 && K <= 2048);
+    if (!w_f32 && !deep && ahead) {
       if (R == 2) lgs::lin_gemv_kernel<false, 1, 2, 1, true><<<grid, 256, 0, stream>>>(p);
       else if (M == 1) lgs::lin_gemv_kernel<false, 1, 1, 1, true><<<grid, 256, 0, stream>>>(p);
       else lgs::lin_gemv_kernel<false, 2, 1, 1, true><<<grid, 256, 0, stream>>>(p);
