@@ -540,8 +540,9 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
 // A lone wave issues an instruction each five clocks, and a token is a chain of some 70 there, 490 clocks. With half of the rows
 // a lane has 48, 310 clocks, and a prompt of 16 heads one wave on each SIMD of the chip instead of one on every other. q, k and decays lie
 // in LDS as the lanes hold them (one 16-byte read each), v, beta and k . q of a token and column side by side. 2048 tokens of 16
-// heads of 128 x 128: 430 us before, 270 to 280 here; one token 6.6 / 5.2. Beyond 4096 columns the waves share their SIMDs and the fewer
-// instructions of the other form count: 2048 tokens of 32 heads 432 / 388, 1024 of 48 heads 259 / 302.
+// heads of 128 x 128: 430 us before, 270 to 280 here; one token 6.6 / 5.2. Beyond 512 workgroups the waves share their
+// SIMDs unevenly and the fewer instructions of the other form count: 2048 tokens of 32 heads 432 / 388, 1024 of 48 heads 259 / 302, 404
+// of 5 sequences' 8 heads of 100 columns, which are 13 workgroups each, 92 / 107.
 //
 // grid (B * H * ceil(dv / 8) rounded up to 8). Lane l of a column: rows 64 j + 2 l + e, j, e < 2.
 // (PC: a decay per channel. The loads ahead carry no branches: behind one, every batch would wait for the next one's loads.)
@@ -674,7 +675,7 @@ __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
   }
 }
 
-constexpr long kDeltaWideColumns = 4096;  // (the figures stand above)
+constexpr long kDeltaWideItems = 512;  // workgroups of eight columns (the figures stand above)
 static void gated_delta_wide_launch(DeltaArgs p, int B, bool plain, hipStream_t stream) {
   p.ncb = (p.dv + 7) / 8;
   p.items = B * p.H * p.ncb;
@@ -789,7 +790,7 @@ extern "C" int lgs_gated_delta(const float* qkv, long ld, const float* dec, cons
   // keep the launch within about two waves per SIMD, and at least enough for 32 rows per lane
   int lpc = lanes;
   const bool pairs = ld % 2 == 0 && ((uintptr_t)qkv | (uintptr_t)dec) % 8 == 0;  // (loaded two floats at a time)
-  if (lanes == 0 && d == 128 && pairs && (long)B * H * dv <= lgs::kDeltaWideColumns) {
+  if (lanes == 0 && d == 128 && pairs && (long)B * H * ((dv + 7) / 8) <= lgs::kDeltaWideItems) {
     lgs::gated_delta_wide_launch(p, B, plain != 0, stream);
     LGA_LAUNCH_RETURN();
   }
