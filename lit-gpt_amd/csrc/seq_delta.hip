@@ -122,7 +122,14 @@ __global__ void __launch_bounds__(256) delta_prepare_kernel(DeltaPrepArgs p) {
 // of eight tokens, each row of the low-rank map read once for all eight (a workgroup per token reads all 256 KB of a map of 2048 x
 // 64 for itself); the last ones 256 betas each. CPT: columns a lane holds. 2048 tokens, us for a workgroup per token / here:
 // 16 heads of 128 with a decay per channel 95 / 42, 8 heads with one each 12 / 12; 200 tokens 22 / 12.
+// Few heads keep the workgroup per token up to 2048 rows, its waves being as many as there is work: us there / here of 200 and 1200
+// rows, 4 heads with a decay each 4.3 / 6.1, 5.4 / 6.9, 8 heads 6.1 / 6.3, 7.5 / 8.5, of a low-rank map 6.9 / 8.9, 8.5 / 11.4, 2 heads of
+// 128 with a decay per channel of one 6.1 / 11.4, 13.7 / 11.8; 8 such heads 8.1 / 6.8, 12.8 / 11.5, 16 with one each 9.2 / 6.5, 11.1 /
+// 11.7; 2048 rows of 4 heads 7.3 / 7.6, of 8 11.2 / 10.9.
 constexpr int kPrepTokens = 8;
+static bool prepare_rows_pay(int T, int H, int G, int d, bool per_channel, bool low_rank) {
+  return T >= 2048 || (T > 64 && (per_channel ? H * d >= 1024 : G >= 16 && !low_rank));
+}
 template <bool A2F32, int CPT>
 __global__ void __launch_bounds__(256) delta_prepare_rows_kernel(DeltaPrepArgs p, int T, int vecs, int decs) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, d = p.d;
@@ -722,7 +729,7 @@ extern "C" int lgs_delta_prepare(float* qkv, long ld, const float* a, long lda, 
                        norm_eps, w_a2, rank, a2_f32, unit ? 1 : 0, decay_form, tau, nullptr, 0, nullptr, 0, 0, 0, nullptr,
                        nullptr, nullptr};
   const int n = per_channel ? H * d : H;
-  if (T > 64 && d <= 512) {
+  if (d <= 512 && lgs::prepare_rows_pay(T, H, G, d, per_channel != 0, w_a2 != nullptr)) {
     const int pairs = 4 * (d <= 128 ? 4 : 1);  // of a workgroup
     const long vecs = ((long)T * G + pairs - 1) / pairs;
     const long decs = ((long)T + lgs::kPrepTokens - 1) / lgs::kPrepTokens * ((n + 255) / 256);

@@ -462,9 +462,9 @@ def test_delta_rule_of_wide_heads_to_the_bit(H, G, dv, extra, lens, per_channel,
 @pytest.mark.parametrize("H,G,d,per_channel,rank,unit,form", [(4, 2, 128, True, 64, True, 0), (4, 4, 40, False, 0, True, 0),
                                                               (2, 1, 130, True, 12, True, 0), (3, 3, 512, True, 3, False, 1),
                                                               (16, 16, 64, True, 0, True, 1)])
-@pytest.mark.parametrize("T", [65, 72, 131])
+@pytest.mark.parametrize("T", [65, 72, 131, 2049])
 def test_delta_prepare_of_prompts_to_the_bit(H, G, d, per_channel, rank, unit, form, T):
-    """More than 64 rows: the bits of 64 at a time, over ends of eight tokens, 256 entries and four heads."""
+    """More than 64 rows, in both forms: the bits of 64 at a time, over ends of eight tokens, 256 entries and four heads."""
     from lit_gpt import seq_ops
 
     dev = torch.device("cuda", 0)
@@ -477,7 +477,7 @@ def test_delta_prepare_of_prompts_to_the_bit(H, G, d, per_channel, rank, unit, f
     whole = qkv.clone()
     got = [whole, *seq_ops.delta_prepare(whole, a, 2, b, 3, A_log, bias, **kw)]
     parts = []
-    for rows in (slice(0, 64), slice(64, 128), slice(128, T))[: -(-T // 64)]:
+    for rows in (slice(i, min(i + 64, T)) for i in range(0, T, 64)):
         q = qkv[rows].clone()
         parts.append([q, *seq_ops.delta_prepare(q, a[rows].contiguous(), 2, b[rows].contiguous(), 3, A_log, bias, **kw)])
     for x, *pieces in zip(got, *parts):
