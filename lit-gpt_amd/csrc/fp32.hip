@@ -113,10 +113,13 @@ __global__ void __launch_bounds__(256) f32_linear_rows_kernel(const float* __res
   y[(size_t)m * N + n] = acc;
 }
 
-// From eight rows and some six waves a CU on: 8 rows of 3072 x 768 (1536 waves) 9.2 / 8.5 us, of 2304 x 768 (1152) 7.8 / 8.4, 16 rows of
-// 768 x 3072 (768) 13.8 / 14.9; 4 rows of 3072 x 768, half of them repeated, 6.5 / 8.6
+// From eight rows and some eight waves a CU on, where few of the rows computed are repeated ones or the chip is full several times
+// over. us, a wave per output / here: 8 rows of 4096 x 768 9.3 / 8.3, of 3072 x 768 (1536 waves) 7.6 / 7.9, of 3072 x 3072 21.1 / 23.6; 9
+// rows of 2304 x 256 4.4 / 6.4, of 4096 x 768 10.5 / 11.5, of 8192 x 768 21.1 / 19.1; 12 rows of 2304 x 768 8.2 / 9.2, of 3072 x 768
+// 10.0 / 9.6; 16 rows of 2304 x 768 10.0 / 9.2; 17 of 4096 x 768 17.2 / 14.6, of 2304 x 256 6.5 / 7.5
 static bool f32_linear_in_rows(int M, int N, int K) {
-  return K % 4 == 0 && M >= 8 && (long)((N + 1) / 2) * ((M + 7) / 8) >= 1500;
+  const long live = (long)M * N / 16, padded = (long)((N + 1) / 2) * ((M + 7) / 8);  // waves' worth of rows, and waves
+  return K % 4 == 0 && M >= 8 && live >= 2000 && (live * 10 >= padded * 7 || live >= 4500);
 }
 
 // Mean and biased variance of a row by a workgroup of 256, the first 256 CPT columns left in r

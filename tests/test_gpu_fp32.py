@@ -236,7 +236,8 @@ def test_ranges_of_infinite_scores():
         assert got.isnan().all() if h else (got - want[0]).abs().max() < 1e-6
 
 
-@pytest.mark.parametrize("M,N,K", [(8, 2999, 4), (8, 2996, 4), (9, 1501, 260), (33, 601, 1028), (65, 334, 768), (15, 1501, 255)])
+@pytest.mark.parametrize("M,N,K", [(8, 2999, 4), (8, 2996, 4), (9, 1501, 260), (33, 601, 1028), (65, 334, 768), (15, 1501, 255),
+                                   (8, 4003, 4), (9, 8005, 260), (12, 2701, 1028), (33, 1001, 768), (65, 501, 260), (23, 1501, 255)])
 def test_rows_of_prompts_to_the_bit(M, N, K):
     """Eight rows and two outputs a wave: the bits of one row at a time, past whole groups of rows and outputs."""
     from lit_gpt import ops
