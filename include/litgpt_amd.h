@@ -76,7 +76,7 @@ int lga_q4_gemm(const void* x, const uint8_t* qweight, const void* scales, const
 int lga_q4f_fits(int M, int N, int K, int group, int fmt);
 /* Short prompts split K across workgroups: the caller passes a zero-initialised workspace of at least this many
  * bytes (0 = none needed; the largest of all formats') and keeps it for later calls (its per-tile counters are left
- * zeroed). */
+ * zeroed). One product at a time may use it: of one stream, and of one thread, as some are two launches. */
 size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu);
 /* How a product of one format is made, in one number: bits 0..1 the form (0 the LDS-image tiles, 1 4-bit weights dequantized in
  * registers, 2 the bf16 weights' pipelined tiles, 3 4-bit weights dequantized beside rings of X; 4-bit scales off 8 bytes take form
