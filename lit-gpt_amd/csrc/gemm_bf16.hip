@@ -13,27 +13,18 @@ namespace lga {
 
 struct BfArgs {
   Q4dArgs a;
-  int nt, mt, splits, kper;  // tiles over columns and rows; ranges of K of kper stages of 64 values
+  int nt, splits, kper;  // tiles over columns; ranges of K of kper stages of 64 values
+  bool apart;            // (gemm_at)
 };
 
+// the tile at rows m0 .. and columns n0 .. of range `split`
 template <int WM, int WN, int FM, int FN, int RA, int RB, bool DUAL>
-__global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
+__device__ __forceinline__ void bf16_rows(const BfArgs& k, unsigned char* lds, int split, int m0, int n0) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
-  constexpr int BN = DUAL ? T::BM / 2 : T::BM;  // columns of Y per tile
   static_assert(!DUAL || FM % 2 == 0, "fragments of the two matrices in pairs");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
   const Q4dArgs& a = k.a;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // an XCD takes neighbouring tiles: of a column's weights those of up to eight row tiles, range after range (all of a
-  // column's on one XCD: 517 x 12288 x 4096 with weights from memory 70 -> 62 us)
-  int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int per = k.nt * k.mt, split = t / per;
-  if (split >= k.splits) return;
-  t -= split * per;
-  const int g = t / (8 * k.nt), gm = min(8, k.mt - g * 8);
-  t -= g * 8 * k.nt;
-  const int m0 = (g * 8 + t % gm) * T::BN, n0 = t / gm * BN;
   const int k0 = split * k.kper, nk = min(a.K / 64 - k0, k.kper);
   const unsigned char *src_w[T::PA], *src_x[T::PB];
   int r, c;
@@ -61,12 +52,34 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
   }
 }
 
+template <int WM, int WN, int FM, int FN, int MOST, bool DUAL, int F = FN - 1>
+__device__ __forceinline__ void bf16_short(const BfArgs& k, unsigned char* lds, int split, int m0, int n0, int frags) {
+  if constexpr (F > 0) {
+    using S = GemmShort<WM, WN, FM, F, MOST>;
+    if (frags == F) bf16_rows<WM, WN, FM, F, S::RA, S::RB, DUAL>(k, lds, split, m0, n0);
+    else bf16_short<WM, WN, FM, FN, MOST, DUAL, F - 1>(k, lds, split, m0, n0, frags);
+  }
+}
+
+// (an XCD takes neighbouring tiles: of a column's weights those of up to eight row tiles, range after range. All of a column's on
+// one XCD: 517 x 12288 x 4096 with weights from memory 70 -> 62 us)
+template <int WM, int WN, int FM, int FN, int RA, int RB, bool DUAL>
+__global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[FN > 1 ? kGemmLds<T> : T::LDS];
+  GemmAt at;
+  if (!gemm_at<T::BN, WN * 32>(k.a.M, k.nt, k.splits, k.apart, &at)) return;
+  const int m0 = at.m * T::BN, n0 = at.n * (DUAL ? T::BM / 2 : T::BM), frags = (k.a.M - m0 + WN * 32 - 1) / (WN * 32);
+  if (frags >= FN) bf16_rows<WM, WN, FM, FN, RA, RB, DUAL>(k, lds, at.which, m0, n0);
+  else bf16_short<WM, WN, FM, FN, kGemmLds<T>, DUAL>(k, lds, at.which, m0, n0, frags);
+}
+
 template <int WM, int WN, int FM, int FN, int RA, int RB>
 static void bf16_go(BfArgs k, bool dual, hipStream_t stream) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   const int bn = dual ? T::BM / 2 : T::BM;
-  k.nt = (k.a.N + bn - 1) / bn, k.mt = (k.a.M + T::BN - 1) / T::BN;
-  const unsigned grid = (unsigned)(((long)k.nt * k.mt * k.splits + 7) / 8 * 8);
+  k.nt = (k.a.N + bn - 1) / bn;
+  const unsigned grid = gemm_grid((long)k.nt * ((k.a.M + T::BN - 1) / T::BN) * k.splits);
   if constexpr (FM % 2 == 0) {
     if (dual) gemm_bf16_kernel<WM, WN, FM, FN, RA, RB, true><<<grid, T::NT, 0, stream>>>(k);
   }
@@ -78,7 +91,7 @@ static void bf16_go(BfArgs k, bool dual, hipStream_t stream) {
 // (2^26). More than 1024 rows that fill the chip keep K whole.
 GemmPlan bf16_plan(int M, int N, int K, bool dual) {
   const long cols = dual ? 2L * N : N;
-  if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1};
+  if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1, false};
   const bool full = M > 1024 && (M + 255) / 256 * (cols / 128) >= 256;
   return gemm_tile_plan(M, (int)cols, K, 1, false, full ? 1 : 0, kGemmRowsB | (dual ? kGemmPairs : 0));
 }
@@ -89,7 +102,7 @@ size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {
 
 int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream) {
   const int steps = a.K / 64, kper = (steps + p.ksplit - 1) / p.ksplit;
-  const BfArgs k{a, 0, 0, (steps + kper - 1) / kper, kper};
+  const BfArgs k{a, 0, (steps + kper - 1) / kper, kper, p.apart};
   switch (p.tile) {
 #define LGA_CASE(I, SLOTS, US, FAST, ROUND, ...) \
   case I: bf16_go<__VA_ARGS__>(k, dual, stream); break;

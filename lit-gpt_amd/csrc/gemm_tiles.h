@@ -37,7 +37,7 @@ __device__ __forceinline__ void gemm_wait_vm() {
 
 template <int WM, int WN, int FM, int FN, int RA, int RB>
 struct GemmTile {
-  static constexpr int FRAGS = FM, BM = WM * FM * 32, BN = WN * FN * 32, NW = WM * WN, NT = NW * 64;
+  static constexpr int BM = WM * FM * 32, BN = WN * FN * 32, NW = WM * WN, NT = NW * 64;
   static constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, LDS = RA * A_BYTES + RB * B_BYTES;
   static constexpr int PA = BM / 8 / NW, PB = BN / 8 / NW;  // DMAs (8 rows, 1 KB) per wave and step
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "every wave issues the same number of DMAs");
@@ -145,6 +145,58 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const unsigned cha
   gemm_wait_vm<0>();  // no DMA may outlive the workgroup's LDS
 }
 
+// The rows past the last whole tile get a tile of their own with fewer fragments along them: the same columns, waves and
+// sums, in the LDS that the whole tile leaves, so a matrix instruction works on at most STEP - 1 rows that are not there. The
+// short tiles stand last in the grid and fill the whole ones' last round.
+template <int WM, int WN, int FM, int FN, int MOST>
+struct GemmShort {
+  static constexpr int A = WM * FM * 4096, B = WN * FN * 4096, FIT = MOST / (A + B), R = FIT < 6 ? FIT : 6;
+  static constexpr int RA = R < 3 && (R + 1) * A + R * B <= MOST ? R + 1 : R, RB = R;
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
+};
+template <class T>
+constexpr int kGemmLds = T::LDS > 81920 ? 163840 : 81920;  // (two workgroups on a CU or one)
+
+// rows: whole tiles of ROWS, a short one behind them that leaves STEP rows out at least
+template <int ROWS, int STEP>
+__host__ __device__ constexpr int gemm_whole(int rows) {
+  return rows / ROWS + (rows % ROWS > ROWS - STEP ? 1 : 0);
+}
+// Workgroup b runs on XCD b % 8, and an XCD takes neighbouring tiles, whose rows and columns its L2 then holds: of `whole` ones, then
+// of `last` ones, as many as any other XCD or one less (an XCD with a tile more than it has compute units makes them in two rounds).
+// Its place in the first list, or else (false) in the second; -1: none is left.
+__device__ __forceinline__ bool gemm_xcd(int whole, int last, int* t) {
+  const int x = blockIdx.x & 7, at = blockIdx.x >> 3, q = whole / 8, r = whole % 8, own = q + (x < r ? 1 : 0);
+  if (at < own) {
+    *t = x * q + min(x, r) + at;
+    return true;
+  }
+  const int ql = last / 8, rl = last % 8, more = x - (8 - rl);  // (the odd ones to the XCDs at the other end)
+  *t = at - own < ql + (more >= 0 ? 1 : 0) ? x * ql + max(more, 0) + at - own : -1;
+  return false;
+}
+inline unsigned gemm_grid(long tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
+// Where a workgroup's tile lies among those of `count` products (batches or ranges of K). apart: the short tiles behind all whole ones,
+// or else each beside the whole tiles of its columns
+struct GemmAt {
+  int which, m, n;
+};
+template <int ROWS, int STEP>
+__device__ __forceinline__ bool gemm_at(int rows, int nt, int count, bool apart, GemmAt* o) {
+  const int all = (rows + ROWS - 1) / ROWS, mt = apart ? gemm_whole<ROWS, STEP>(rows) : all, per = mt * nt;
+  int t;
+  if (gemm_xcd(count * per, count * (all - mt) * nt, &t)) {
+    o->which = t / per;
+    t -= o->which * per;
+    const int g = t / (8 * nt), gm = min(8, mt - g * 8);  // groups of up to 8 row tiles
+    t -= g * 8 * nt;
+    o->m = g * 8 + t % gm, o->n = t / gm;
+    return true;
+  }
+  if (t < 0) return false;
+  o->which = t / nt, o->m = mt, o->n = t % nt;
+  return true;
+}
 // The tile forms: what a step of 64 values of K costs a full chip of their workgroups, and what it would cost at the 2.4 GHz
 // that a chip with few of them runs at; start, end and fp32 results of a round of them. Measured on 256 tiles (512 of the
 // form of which a compute unit holds two) and K 1024 and 4096. The larger tile moves fewer bytes per product (256 x 256:
@@ -162,33 +214,38 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const unsigned cha
   X(7, 256, 0.285f, 0.275f, 4.9f, 1, 4, 2, 1, 6, 6)       \
   X(8, 256, 1.163f, 0.745f, 10.3f, 2, 2, 3, 4, 3, 2)
 struct GemmForm {
-  int bm, bn, fm, slots;
+  int bm, bn, fm, fn, slots;
   float step_us, fast_us, round_us;
 };
-#define LGA_GEMM_FORM(I, SLOTS, US, FAST, ROUND, ...) \
-  {GemmTile<__VA_ARGS__>::BM, GemmTile<__VA_ARGS__>::BN, GemmTile<__VA_ARGS__>::FRAGS, SLOTS, US, FAST, ROUND},
+#define LGA_GEMM_FORM(I, SLOTS, US, FAST, ROUND, WM, WN, FM, FN, ...) {WM * FM * 32, WN * FN * 32, FM, FN, SLOTS, US, FAST, ROUND},
 constexpr GemmForm kGemmForms[] = {LGA_GEMM_FORMS(LGA_GEMM_FORM)};
 #undef LGA_GEMM_FORM
+constexpr int kGemmFormCount = sizeof(kGemmForms) / sizeof(kGemmForms[0]);
 
 // Which form, and how many ranges of K (ksplit 0: the plan's own choice); tile -1: K is no multiple of 64.
 struct GemmPlan {
   int tile, ksplit;
+  bool apart;
 };
-// Rounds of workgroups times what one takes; several ranges of K cost a second launch that reads them all. Against all forms
-// and ranges on 24 products of 64 to 4096 rows, weights from memory, the choice is the fastest or within 7 % of it.
 enum {
   kGemmRowsB = 1,  // the rows are the tile's B, the columns its A
   kGemmPairs = 2,  // A's fragments are those of two matrices in turn: forms with an even number of them
   kGemmActs = 4    // forms whose code holds activations
 };
-inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int flags) {
-  GemmPlan best{-1, 1};
+inline bool gemm_form_fits(const GemmForm& t, int flags) {
+  return !((flags & kGemmActs && t.bm * t.bn > 256 * 128) || (flags & kGemmPairs && t.fm % 2));
+}
+// Counted in whole tiles: rounds of workgroups times what one takes; several ranges of K cost a second launch that reads them all.
+// Against all forms and ranges on 24 products of 64 to 4096 rows, weights from memory, the choice was the fastest or within 7 % of it
+// before there were short tiles. It still says the ranges, and with them the order of a product's sums, and the forms of grouped products.
+inline GemmPlan gemm_whole_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int flags) {
+  GemmPlan best{-1, 1, false};
   if (K % 64 != 0 || M <= 0) return best;
   const int steps = K / 64;
   float best_us = 0.0f;
-  for (int f = 0; f < (int)(sizeof(kGemmForms) / sizeof(kGemmForms[0])); ++f) {
+  for (int f = 0; f < kGemmFormCount; ++f) {
     const GemmForm& t = kGemmForms[f];
-    if ((flags & kGemmActs && t.bm * t.bn > 256 * 128) || (flags & kGemmPairs && t.fm % 2)) continue;
+    if (!gemm_form_fits(t, flags)) continue;
     const int rows = flags & kGemmRowsB ? t.bn : t.bm, cols = flags & kGemmRowsB ? t.bm : t.bn;
     const float nt = (float)((N + cols - 1) / cols);
     // a range of the list ends somewhere in its last tile, and has one
@@ -204,14 +261,48 @@ inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int
         us += per * fmaxf(t.fast_us, t.step_us * (1.0f - most * (1.0f - (rounds - whole)))) + t.round_us;
       }
       if (s > 1) us += 2.0f + (float)M * N * 4.0f * (s + 1) / 5.5e6f;
-      if (best.tile < 0 || us < best_us) {
-        best_us = us;
-        best = GemmPlan{f, s};
-      }
+      if (best.tile < 0 || us < best_us) best_us = us, best.tile = f, best.ksplit = s;
     }
   }
   return best;
 }
 
+// The form of a plain product for these ranges: whole tiles' rounds, the short ones among the last of them or behind, where they fill
+// the chip's idle part. Of 1491 products of 33 to 2600 rows, weights from memory, it is 1.1 % from the fastest form in the mean, and
+// the form that counts whole tiles 2.0 %. us of whole tiles alone / here: 2407 x 20608 x 4096 448 / 381, 517 x 11008 x 4096 with SwiGLU
+// 109 / 101, 40 rows of it 37 / 33.
+// A grouped product's short tiles stand beside the whole ones of their columns, whose weights they would otherwise fetch anew (16 groups of
+// 278 rows of twice 2752 x 4096 302 behind, 260 beside): 546 products of 16 groups, 160 to 16384 rows in all, in 0.96 of the time of
+// whole tiles (450 rows each of 2048 x 1408 70 / 67, of 4096 x 2752 227 / 210), none more than 7 % slower.
+inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int flags) {
+  GemmPlan best = gemm_whole_plan(M, N, K, batch, grouped, ksplit, flags);
+  if (best.tile < 0 || grouped) return best;
+  const int steps = K / 64, per = (steps + best.ksplit - 1) / best.ksplit, count = batch * ((steps + per - 1) / per);
+  float best_us = 0.0f;
+  best.apart = true;
+  for (int f = 0; f < kGemmFormCount; ++f) {
+    const GemmForm& t = kGemmForms[f];
+    if (!gemm_form_fits(t, flags)) continue;
+    const bool rows_b = flags & kGemmRowsB;
+    const int rows = rows_b ? t.bn : t.bm, cols = rows_b ? t.bm : t.bn, frags = rows_b ? t.fn : t.fm, step = rows / frags;
+    const float most = t.bm * t.bn > 128 * 192 ? 0.69f : 0.46f;  // (of what fewer workgroups gain, as above)
+    auto round = [&](float load) { return per * fmaxf(t.fast_us, t.step_us * (1.0f - most * (1.0f - load))) + t.round_us; };
+    const int pieces = (M + step - 1) / step, mt = pieces / frags, left = pieces % frags;
+    const float nt = (float)((N + cols - 1) / cols), slots = (float)t.slots;
+    const float whole = mt * nt * count, full = floorf(whole / slots), over = whole - full * slots;
+    // a short tile's time of a whole one's; alone on the chip it is mostly latency
+    const float each = left == 0 ? 1.0f : fmaxf(0.3f + 0.7f * left / frags, mt > 0 ? 0.0f : 0.75f);
+    float shorts = left ? nt * count : 0.0f, us;
+    us = full * round(1.0f);
+    if (over > 0.0f) {
+      const float beside = fminf(shorts, (slots - over) * floorf(1.0f / each));
+      us += round((over + beside * each) / slots);
+      shorts -= beside;
+    }
+    if (shorts > 0.0f) us += each * ceilf(shorts / slots) * round(fminf(shorts / slots, 1.0f) * each);
+    if (best_us == 0.0f || us < best_us) best_us = us, best.tile = f;
+  }
+  return best;
+}
 
 }  // namespace lga

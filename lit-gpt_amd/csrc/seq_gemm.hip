@@ -2,6 +2,8 @@
 // pipelined tiles of gemm_tiles.h.
 #include "seq_gemm.h"
 
+#include <algorithm>
+
 #include "gemm_tiles.h"
 
 namespace lgs {
@@ -10,39 +12,44 @@ using lga::GemmTile;
 using lga::f32x16_t;
 using lga::gemm_tile;
 
-// grouped rows: this workgroup's tile, z its batch and t its number inside the batch (false: none is left). The batches'
-// tiles are counted side by side over the lanes, and every XCD takes an eighth of those that there are: the grid is the
-// largest number that the groups' sizes allow, of which a third stayed empty and with it the last XCDs (16 groups of 512
-// rows of 2 x 1408 x 2048: 3 rounds on 5 XCDs instead of 2 on all, 216 -> 125 us).
-template <int ROWS>
-__device__ __forceinline__ bool gemm_group(const int* z_start, int batch, int nt, int lane, int* t_at, int* z_at) {
-  auto count = [&](int e0, int* own) {  // tiles of lane's batch and of all up to it
-    const int e = e0 + lane;
-    const int rows = e < batch ? z_start[e + 1] - z_start[e] : 0;
-    *own = (rows + ROWS - 1) / ROWS * nt;
-    int upto = *own;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(upto, o);
-      if (lane >= o) upto += v;
-    }
-    return upto;
+// grouped rows: this workgroup's tile, z its batch and m, n its place inside it (false: none is left). The batches' tiles are
+// counted side by side over the lanes, and every XCD takes an eighth of those that there are: the grid is the largest number that the
+// groups' sizes allow, of which a third stayed empty and with it the last XCDs (16 groups of 512 rows of 2 x 1408 x 2048: 3 rounds on 5
+// XCDs instead of 2 on all, 216 -> 125 us).
+template <int ROWS, int STEP>
+__device__ __forceinline__ bool gemm_group(const int* z_start, int batch, int nt, bool apart, int lane, lga::GemmAt* o) {
+  auto tiles = [&](int e, int* mt) {  // short ones of batch e, and *mt others
+    const int rows = e < batch ? z_start[e + 1] - z_start[e] : 0, all = (rows + ROWS - 1) / ROWS;
+    *mt = apart ? lga::gemm_whole<ROWS, STEP>(rows) : all;
+    return all - *mt;
   };
-  int own, total = 0;
-  for (int e0 = 0; e0 < batch; e0 += 64) total += __shfl(count(e0, &own), 63);
-  const int each = (total + 7) / 8, at = blockIdx.x >> 3;
-  int t = (blockIdx.x & 7) * each + at;
-  if (at >= each || t >= total) return false;
+  auto upto = [&](int v) {  // sum over the lanes up to this one
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(v, d);
+      if (lane >= d) v += u;
+    }
+    return v;
+  };
+  int whole = 0, last = 0, mt, t;
   for (int e0 = 0; e0 < batch; e0 += 64) {
-    const int upto = count(e0, &own);
-    const unsigned long long past = __ballot(upto > t);
+    const int l = tiles(e0 + lane, &mt);
+    whole += __shfl(upto(mt * nt), 63), last += __shfl(upto(l * nt), 63);
+  }
+  const bool first = lga::gemm_xcd(whole, last, &t);
+  if (t < 0) return false;
+  for (int e0 = 0; e0 < batch; e0 += 64) {
+    const int l = tiles(e0 + lane, &mt), own = (first ? mt : l) * nt, sum = upto(own);
+    const unsigned long long past = __ballot(sum > t);
     if (past) {
-      const int l = __ffsll(past) - 1;
-      *z_at = __builtin_amdgcn_readfirstlane(e0 + l);
-      *t_at = __builtin_amdgcn_readfirstlane(t - __shfl(upto - own, l));
+      const int at = __ffsll(past) - 1;
+      mt = __builtin_amdgcn_readfirstlane(__shfl(mt, at));
+      t = __builtin_amdgcn_readfirstlane(t - __shfl(sum - own, at));
+      o->which = __builtin_amdgcn_readfirstlane(e0 + at);
+      o->m = first ? t % mt : mt, o->n = first ? t / mt : t;
       return true;
     }
-    t -= __shfl(upto, 63);
+    t -= __shfl(sum, 63);
   }
   return false;
 }
@@ -55,35 +62,12 @@ constexpr bool kActsFit = FM * FN <= 8;
 // tiles cost 15 us, of 256 x 128 8. Results go straight to memory, past the caches (a lane's rows in 128-byte pieces):
 // turning them in LDS into longer pieces cost 14 us a tile.
 //
-// Workgroup b runs on XCD b % 8, and an XCD takes neighbouring tiles, whose rows of A and W its L2 then holds.
-template <int WM, int WN, int FM, int FN, int RA, int RB>
-__global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, int nt, int batch) {
+// The tile at rows m0 .. of batch z, whose list has Mz rows from r_lo on, and columns n0 ..
+template <int WM, int WN, int FM, int FN, int RA, int RB, bool SHORT, bool ACTS>
+__device__ __forceinline__ void gemm_rows(const LinArgs& p, unsigned char* lds, int z, int split, int r_lo, int Mz, int m0, int n0) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  int z = 0, split = 0, r_lo = 0, Mz = p.M, m, n;
-  if (p.z_start) {
-    if (!gemm_group<T::BM>(p.z_start, batch, nt, lane, &t, &z)) return;
-    r_lo = p.z_start[z];
-    Mz = p.z_start[z + 1] - r_lo;
-    const int mz = (Mz + T::BM - 1) / T::BM;
-    m = t % mz;
-    n = t / mz;
-  } else {
-    const int per = mt * nt;
-    const int which = t / per;
-    if (which >= batch * p.ksplit) return;
-    if (p.ksplit > 1) split = which;
-    else z = which;
-    t -= which * per;
-    const int g = t / (8 * nt), gm = min(8, mt - g * 8);  // groups of up to 8 row tiles
-    t -= g * 8 * nt;
-    m = g * 8 + t % gm;
-    n = t / gm;
-  }
-  const int m0 = m * T::BM, n0 = n * T::BN;
   int nk = p.K / 64, k0 = 0;
   if (p.ksplit > 1) {
     k0 = split * p.kper;
@@ -157,8 +141,10 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, in
   constexpr std::integral_constant<int, 1> one{};
   constexpr std::integral_constant<int, FEW> few{};
   auto put = [&](auto sums, auto past, auto n, auto* y, long ld, auto&& make) __attribute__((always_inline)) {
-    if (inside) each(yes, sums, past, n, y, ld, make);
-    else each(no, sums, past, n, y, ld, make);
+    if constexpr (!SHORT) {
+      if (inside) return each(yes, sums, past, n, y, ld, make);
+    }
+    each(no, sums, past, n, y, ld, make);
   };
   if (p.ksplit > 1) {
     put(no, no, one, p.part + ((size_t)split * p.M + mw) * p.N + nw, p.N, [](int, float v, float) { return v; });
@@ -168,8 +154,8 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, in
 #pragma unroll
   for (int j = 0; j < FN; ++j) bias[j] = p.bias ? p.bias[min(nw + l31 + j * 32, p.N - 1)] : 0.0f;
   const long at = (long)z * p.sy + (long)(r_lo + mw) * p.ldy + nw;
-  if (kActsFit<FM, FN> && p.act != kActNone) {
-    if constexpr (kActsFit<FM, FN>) {
+  if (ACTS && p.act != kActNone) {
+    if constexpr (ACTS) {
       // (a loop of its own for each activation: a choice per result keeps them from standing among one another)
       auto act = [&](auto kind) __attribute__((always_inline)) {
         auto f = [&](int j, float v, float) { return act_f(decltype(kind)::value, v + bias[j]); };
@@ -191,13 +177,44 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int mt, in
   }
 }
 
+// f: fragments along the rows that have one, FM and less
+template <int WM, int WN, int FM, int FN, int MOST, int F = FM - 1>
+__device__ __forceinline__ void gemm_short(const LinArgs& p, unsigned char* lds, int z, int split, int r_lo, int Mz, int m0, int n0, int f) {
+  if constexpr (F > 0) {
+    using S = lga::GemmShort<WM, WN, F, FN, MOST>;
+    if (f == F) gemm_rows<WM, WN, F, FN, S::RA, S::RB, true, kActsFit<FM, FN>>(p, lds, z, split, r_lo, Mz, m0, n0);
+    else gemm_short<WM, WN, FM, FN, MOST, F - 1>(p, lds, z, split, r_lo, Mz, m0, n0, f);
+  }
+}
+
 template <int WM, int WN, int FM, int FN, int RA, int RB>
-static int gemm_go(const LinArgs& p, int batch, hipStream_t stream) {
+__global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int nt, int batch, bool apart) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
-  const int mt = (p.M + T::BM - 1) / T::BM, nt = (p.N + T::BN - 1) / T::BN;
-  const long tiles = p.z_start ? (long)(mt + batch) * nt : (long)mt * nt * batch * p.ksplit;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[FM > 1 ? lga::kGemmLds<T> : T::LDS];
+  lga::GemmAt at;
+  int z = 0, split = 0, r_lo = 0, Mz = p.M;
+  if (p.z_start) {
+    if (!gemm_group<T::BM, WM * 32>(p.z_start, batch, nt, apart, threadIdx.x & 63, &at)) return;
+    z = at.which;
+    r_lo = p.z_start[z];
+    Mz = p.z_start[z + 1] - r_lo;
+  } else {
+    if (!lga::gemm_at<T::BM, WM * 32>(Mz, nt, batch * p.ksplit, apart, &at)) return;
+    if (p.ksplit > 1) split = at.which;
+    else z = at.which;
+  }
+  const int m0 = at.m * T::BM, n0 = at.n * T::BN, f = (Mz - m0 + WM * 32 - 1) / (WM * 32);
+  if (f >= FM) gemm_rows<WM, WN, FM, FN, RA, RB, false, kActsFit<FM, FN>>(p, lds, z, split, r_lo, Mz, m0, n0);
+  else gemm_short<WM, WN, FM, FN, lga::kGemmLds<T>>(p, lds, z, split, r_lo, Mz, m0, n0, f);
+}
+
+template <int WM, int WN, int FM, int FN, int RA, int RB>
+static int gemm_go(const LinArgs& p, int batch, bool apart, hipStream_t stream) {
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
+  const long mt = (p.M + T::BM - 1) / T::BM, nt = (p.N + T::BN - 1) / T::BN;
+  const long tiles = p.z_start ? (mt + batch) * nt : mt * nt * batch * p.ksplit;
   LGA_CHECK_ARG(tiles < (1L << 30), "lgs_linear: too many tiles");
-  gemm_kernel<WM, WN, FM, FN, RA, RB><<<(unsigned)((tiles + 7) / 8 * 8), T::NT, 0, stream>>>(p, mt, nt, batch);
+  gemm_kernel<WM, WN, FM, FN, RA, RB><<<lga::gemm_grid(tiles), T::NT, 0, stream>>>(p, (int)nt, batch, apart);
   return 0;
 }
 
@@ -206,27 +223,11 @@ static int gemm_go(const LinArgs& p, int batch, hipStream_t stream) {
 // twice the width and a launch less than the product and its unit apart, whose bits it gives: 403 us for 2407 rows, twice
 // 11008 columns and K 4096 in a model's prompt (511 on stages of 32 values of K).
 template <int WM, int WN, int FM, int FN, int RA, int RB, bool CLAMPED>
-__global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluForm f, int mt, int nt, int batch) {
+__device__ __forceinline__ void glu_rows(const LinArgs& p, const GluForm& f, unsigned char* lds, int z, int r_lo, int Mz, int m0, int n0) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   static_assert(FM % 2 == 0, "fragments of the two matrices in pairs");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  int z = 0, r_lo = 0, Mz = p.M, m, n;
-  if (p.z_start) {
-    if (!gemm_group<T::BN>(p.z_start, batch, nt, lane, &t, &z)) return;
-    r_lo = p.z_start[z];
-    Mz = p.z_start[z + 1] - r_lo;
-    const int mz = (Mz + T::BN - 1) / T::BN;
-    m = t % mz, n = t / mz;
-  } else {
-    if (t >= mt * nt) return;
-    const int g = t / (8 * nt), gm = min(8, mt - g * 8);  // groups of up to 8 row tiles
-    t -= g * 8 * nt;
-    m = g * 8 + t % gm, n = t / gm;
-  }
-  const int m0 = m * T::BN, n0 = n * (T::BM / 2);
   const unsigned char *src_w[T::PA], *src_x[T::PB];
   int r, c;
 #pragma unroll
@@ -271,37 +272,67 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluFor
   else store([](float g, float u) { return act_f(kActSilu, g) * u; });
 }
 
-template <int WM, int WN, int FM, int FN, int RA, int RB>
-static int glu_go(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
+template <int WM, int WN, int FM, int FN, int MOST, bool CLAMPED, int F = FN - 1>
+__device__ __forceinline__ void glu_short(const LinArgs& p, const GluForm& f, unsigned char* lds, int z, int r_lo, int Mz, int m0, int n0,
+                                          int frags) {
+  if constexpr (F > 0) {
+    using S = lga::GemmShort<WM, WN, FM, F, MOST>;
+    if (frags == F) glu_rows<WM, WN, FM, F, S::RA, S::RB, CLAMPED>(p, f, lds, z, r_lo, Mz, m0, n0);
+    else glu_short<WM, WN, FM, FN, MOST, CLAMPED, F - 1>(p, f, lds, z, r_lo, Mz, m0, n0, frags);
+  }
+}
+
+template <int WM, int WN, int FM, int FN, int RA, int RB, bool CLAMPED>
+__global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluForm f, int nt, int batch, bool apart) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
-  const int mt = (p.M + T::BN - 1) / T::BN, nt = (p.N + T::BM / 2 - 1) / (T::BM / 2);
-  const long tiles = p.z_start ? (long)(mt + batch) * nt : (long)mt * nt;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[FN > 1 ? lga::kGemmLds<T> : T::LDS];
+  lga::GemmAt at;
+  int z = 0, r_lo = 0, Mz = p.M;
+  if (p.z_start) {
+    if (!gemm_group<T::BN, WN * 32>(p.z_start, batch, nt, apart, threadIdx.x & 63, &at)) return;
+    z = at.which;
+    r_lo = p.z_start[z];
+    Mz = p.z_start[z + 1] - r_lo;
+  } else if (!lga::gemm_at<T::BN, WN * 32>(Mz, nt, 1, apart, &at)) {
+    return;
+  }
+  const int m0 = at.m * T::BN, n0 = at.n * (T::BM / 2), frags = (Mz - m0 + WN * 32 - 1) / (WN * 32);
+  if (frags >= FN) glu_rows<WM, WN, FM, FN, RA, RB, CLAMPED>(p, f, lds, z, r_lo, Mz, m0, n0);
+  else glu_short<WM, WN, FM, FN, lga::kGemmLds<T>, CLAMPED>(p, f, lds, z, r_lo, Mz, m0, n0, frags);
+}
+
+template <int WM, int WN, int FM, int FN, int RA, int RB>
+static int glu_go(const LinArgs& p, const GluForm& f, int batch, bool apart, hipStream_t stream) {
+  using T = GemmTile<WM, WN, FM, FN, RA, RB>;
+  const long mt = (p.M + T::BN - 1) / T::BN, nt = (p.N + T::BM / 2 - 1) / (T::BM / 2);
+  const long tiles = p.z_start ? (mt + batch) * nt : mt * nt;
   LGA_CHECK_ARG(tiles < (1L << 30), "lgs_linear_glu: too many tiles");
-  const unsigned grid = (unsigned)((tiles + 7) / 8 * 8);
-  if (f.clamped) gemm_glu_kernel<WM, WN, FM, FN, RA, RB, true><<<grid, T::NT, 0, stream>>>(p, f, mt, nt, batch);
-  else gemm_glu_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(p, f, mt, nt, batch);
+  const unsigned grid = lga::gemm_grid(tiles);
+  if (f.clamped) gemm_glu_kernel<WM, WN, FM, FN, RA, RB, true><<<grid, T::NT, 0, stream>>>(p, f, (int)nt, batch, apart);
+  else gemm_glu_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(p, f, (int)nt, batch, apart);
   return 0;
 }
 
 int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
 #define LGS_CASE(I, SLOTS, US, FAST, ROUND, ...)                                     \
   case I:                                                                            \
-    if constexpr (lga::GemmTile<__VA_ARGS__>::FRAGS % 2 == 0) return glu_go<__VA_ARGS__>(p, f, batch, stream); \
+    if constexpr (lga::kGemmForms[I].fm % 2 == 0) return glu_go<__VA_ARGS__>(p, f, batch, plan.apart, stream); \
     break;
-  switch (lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, lga::kGemmRowsB | lga::kGemmPairs).tile) { LGA_GEMM_FORMS(LGS_CASE) }
+  const GemmPlan plan = lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, lga::kGemmRowsB | lga::kGemmPairs);
+  switch (plan.tile) { LGA_GEMM_FORMS(LGS_CASE) }
 #undef LGS_CASE
   lga_set_error("lgs_linear_glu: no such form");
   return (int)hipErrorInvalidValue;
 }
 
 GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act) {
-  if (grouped && gemm_few_rows(M, batch)) return GemmPlan{-1, 1};
+  if (grouped && gemm_few_rows(M, batch)) return GemmPlan{-1, 1, false};
   return lga::gemm_tile_plan(M, N, K, batch, grouped, ksplit, act != kActNone ? lga::kGemmActs : 0);
 }
 
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream) {
 #define LGS_CASE(I, SLOTS, US, FAST, ROUND, ...) \
-  case I: return gemm_go<__VA_ARGS__>(p, batch, stream);
+  case I: return gemm_go<__VA_ARGS__>(p, batch, plan.apart, stream);
   switch (plan.tile) { LGA_GEMM_FORMS(LGS_CASE) }
 #undef LGS_CASE
   lga_set_error("lgs_linear: no such form");
