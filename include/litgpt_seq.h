@@ -164,7 +164,7 @@ int lgs_moe_down(const float* actbuf, const void* down, int w_f32, const int* id
                  lgs_stream_t stream);
 /* counting sort of the (token, choice) pairs by expert: z_start [E + 1], tok_of [pairs] (token of each sorted entry),
  * where [pairs] (sorted place of each pair); the order inside an expert's range is not fixed. ws: 2 E ints, zero on
- * entry, left zero. */
+ * entry, left zero; up to 8192 pairs it may be NULL. */
 int lgs_moe_sort(const int* ids, int pairs, int top, int E, int* z_start, int* tok_of, int* where, int* ws,
                  lgs_stream_t stream);
 /* x[t] (+)= sum_k wts[t][k] * y[where[t * top + k]]; with ids, a choice with ids[t][k] >= n_real (an identity expert)

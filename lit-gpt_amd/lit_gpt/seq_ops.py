@@ -580,15 +580,18 @@ def moe_down(actbuf: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, wts: t
                                        F, E, _dev(h, "h", F32), N, int(accumulate), _stream()))
 
 
+SORT_PAIRS = 8192  # up to as many, lgs_moe_sort needs no counters
+
+
 def moe_sort(ids: torch.Tensor, E: int):
     T, top = ids.shape
     dev = ids.device
     z_start = torch.empty(E + 1, dtype=I32, device=dev)
     tok_of = torch.empty(T * top, dtype=I32, device=dev)
     where = torch.empty(T * top, dtype=I32, device=dev)
-    ws = torch.zeros(2 * E, dtype=I32, device=dev)
+    ws = torch.zeros(2 * E, dtype=I32, device=dev) if T * top > SORT_PAIRS else None
     _check(load_library().lgs_moe_sort(_dev(ids, "ids", I32), T * top, top, E, z_start.data_ptr(), tok_of.data_ptr(),
-                                       where.data_ptr(), ws.data_ptr(), _stream()))
+                                       where.data_ptr(), _opt(ws, "ws", I32), _stream()))
     return z_start, tok_of, where
 
 
