@@ -268,8 +268,9 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 }
 
 // One row: y = ((x2 W2^T + b2) + (x1 W1^T + b1)) + res, a wave per output, both products in f32_linear_kernel's order. Bound by
-// latency: the weights of a block of 768 columns beside 3072 are in flight at once, x1 and x2 come behind them, and a join of ranges
-// of keys waits for its own loads and the weights ahead of those. Two launches 13.7 us, one 8.0 (8.9 with ranges to join).
+// latency: the weights of a block of 768 columns beside 3072 are in flight at once, x2 and an attention's ranges ahead of them, so that
+// the join waits for nothing else; x2 is read once for a workgroup's four outputs. Two launches 13.7 us, one 8.0; with ranges to join
+// behind the weights 8.8, ahead of them 8.5.
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
   float* y;
@@ -279,30 +280,38 @@ struct F32LinearsSum {
   int parts, hs;
 };
 // x1 of ranges of keys, joined in LDS: the ranges' sums weighted by exp(their largest score - the largest of all)
-__device__ __forceinline__ void f32_join_parts(const F32LinearsSum& a, float* xs, float* wt) {
-  constexpr int E = 4, P = 8;
-  const int H = a.K1 / a.hs;
-  float o[E][P];
+struct F32Parts {
+  static constexpr int E = 4, P = 8;
+  float o[E][P], m[P], l[P];  // (of the thread's first columns, and of head threadIdx.x)
+};
+__device__ __forceinline__ void f32_load_parts(const F32LinearsSum& a, F32Parts& p) {
+  const int H = a.K1 / a.hs, h = min((int)threadIdx.x, H - 1);
 #pragma unroll
-  for (int e = 0; e < E; ++e)
+  for (int s = 0; s < F32Parts::P; ++s) {
+    p.m[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2] : -INFINITY;
+    p.l[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2 + 1] : -1.0f;
+  }
 #pragma unroll
-    for (int s = 0; s < P; ++s) {
+  for (int e = 0; e < F32Parts::E; ++e)
+#pragma unroll
+    for (int s = 0; s < F32Parts::P; ++s) {
       const int i = threadIdx.x + 256 * e;
-      o[e][s] = i < a.K1 && s < a.parts ? a.x1[(size_t)s * a.K1 + i] : 0.0f;
+      p.o[e][s] = i < a.K1 && s < a.parts ? a.x1[(size_t)s * a.K1 + i] : 0.0f;
     }
-  for (int h = threadIdx.x; h < H; h += 256) {
-    float m[P], l[P], most = -INFINITY, sum = 0.0f;
+}
+__device__ __forceinline__ void f32_join_parts(const F32LinearsSum& a, const F32Parts& p, float* xs, float* wt) {
+  constexpr int E = F32Parts::E, P = F32Parts::P;
+  const int H = a.K1 / a.hs;
+  if ((int)threadIdx.x < H) {  // (up to 256 heads)
+    const int h = threadIdx.x;
+    float most = -INFINITY, sum = 0.0f;
+#pragma unroll
+    for (int s = 0; s < P; ++s) most = fmaxf(most, p.m[s]);
 #pragma unroll
     for (int s = 0; s < P; ++s) {
-      m[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2] : -INFINITY;
-      l[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2 + 1] : -1.0f;
-      most = fmaxf(most, m[s]);
-    }
-#pragma unroll
-    for (int s = 0; s < P; ++s) {
-      const bool empty = l[s] < 0.0f;
-      const float w = empty ? -1.0f : (m[s] == -INFINITY ? 0.0f : expf(m[s] - most));
-      if (!empty) sum = fmaf(w, l[s], sum);
+      const bool empty = p.l[s] < 0.0f;
+      const float w = empty ? -1.0f : (p.m[s] == -INFINITY ? 0.0f : expf(p.m[s] - most));
+      if (!empty) sum = fmaf(w, p.l[s], sum);
       wt[h * (P + 1) + s] = w;
     }
     wt[h * (P + 1) + P] = sum;
@@ -319,30 +328,50 @@ __device__ __forceinline__ void f32_join_parts(const F32LinearsSum& a, float* xs
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int i = threadIdx.x + 256 * e;
-    if (i < a.K1) join(i, [&](int s) { return o[e][s]; });
+    if (i < a.K1) join(i, [&](int s) { return p.o[e][s]; });
   }
   for (int i = threadIdx.x + 256 * E; i < a.K1; i += 256) join(i, [&](int s) { return a.x1[(size_t)s * a.K1 + i]; });
   __syncthreads();
 }
-template <bool PARTS>
+// E2: 1024 values each of x2 that LDS takes (0: a longer row, read from memory by every wave)
+template <bool PARTS, int E2>
 __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
-  extern __shared__ __attribute__((aligned(16))) float xs[];  // [K1] the joined row, then the ranges' weights
+  extern __shared__ __attribute__((aligned(16))) float xs[];  // [K1] the joined row, then the ranges' weights; or [K1]; x2
   const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), n = min(row, a.N - 1);
   const float *r1 = a.w1 + (size_t)n * a.K1, *r2 = a.w2 + (size_t)n * a.K2;
+  // the rows first, and what they wait for: the weights behind them arrive while they are joined
+  float4 x2[E2 > 0 ? E2 : 1];
+#pragma unroll
+  for (int e = 0; e < E2; ++e) x2[e] = *(const float4*)(a.x2 + min((int)(threadIdx.x + 256 * e) * 4, a.K2 - 4));
+  F32Parts parts;
+  if (PARTS) f32_load_parts(a, parts);
+  __builtin_amdgcn_sched_barrier(0);
   float4 w1[kF32Chunks], w2[3][kF32Chunks];
   f32_load_chunks(r1, 0, a.K1, lane, w1);
 #pragma unroll
   for (int u = 0; u < 3; ++u) f32_load_chunks(r2, u * kF32Chunks, a.K2, lane, w2[u]);
   const float b1 = a.b1 ? a.b1[n] : 0.0f, b2 = a.b2 ? a.b2[n] : 0.0f, res = a.res[n];
-  const float* x1 = a.x1;
+  __builtin_amdgcn_sched_barrier(0);
+  const float *px1 = a.x1, *px2 = a.x2;
+  if (E2 > 0) {
+    float* to = xs + (PARTS ? a.K1 + (a.K1 / a.hs * 9 + 3) / 4 * 4 : 0);
+#pragma unroll
+    for (int e = 0; e < E2; ++e) {
+      const int k = (threadIdx.x + 256 * e) * 4;
+      if (k < a.K2) *(float4*)(to + k) = x2[e];
+    }
+    px2 = to;
+  }
   if (PARTS) {
-    f32_join_parts(a, xs, xs + a.K1);
-    x1 = xs;
+    f32_join_parts(a, parts, xs, xs + a.K1);
+    px1 = xs;
+  } else if (E2 > 0) {
+    __syncthreads();
   }
   float4 h4 = make_float4(0.f, 0.f, 0.f, 0.f), m4 = h4;
   for (int c0 = 0; c0 * 256 < a.K1; c0 += kF32Chunks) {
     if (c0 > 0) f32_load_chunks(r1, c0, a.K1, lane, w1);
-    f32_dot_chunks(x1, c0, a.K1, lane, w1, h4);
+    f32_dot_chunks(px1, c0, a.K1, lane, w1, h4);
   }
   for (int c0 = 0; c0 * 256 < a.K2; c0 += 3 * kF32Chunks) {
 #pragma unroll
@@ -350,7 +379,7 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
       if (c0 > 0) f32_load_chunks(r2, c0 + u * kF32Chunks, a.K2, lane, w2[u]);
     }
 #pragma unroll
-    for (int u = 0; u < 3; ++u) f32_dot_chunks(a.x2, c0 + u * kF32Chunks, a.K2, lane, w2[u], m4);
+    for (int u = 0; u < 3; ++u) f32_dot_chunks(px2, c0 + u * kF32Chunks, a.K2, lane, w2[u], m4);
   }
   float h = wave_sum((h4.x + h4.y) + (h4.z + h4.w)), m = wave_sum((m4.x + m4.y) + (m4.z + m4.w));
   if (lane == 0 && row < a.N) {
@@ -412,14 +441,6 @@ __global__ void __launch_bounds__(256) f32_rope_kv_kernel(const float* __restric
   }
 }
 
-// x * cos + rotate_half(x) * sin of dim d on the first n_elem dims of one head vector, two roundings
-__device__ __forceinline__ float rope_f32(const float* xs, int d, int n_elem, const float* cr, const float* sr) {
-  if (d >= n_elem) return xs[d];
-  const int half = n_elem / 2;
-  const float r = d < half ? -xs[d + half] : xs[d - half];
-  return add_rn(mul_rn(xs[d], cr[d]), mul_rn(r, sr[d]));
-}
-
 struct F32AttnArgs {
   const float* q;  // [T][H][hs] roped; fused: the token's projection, per group [q_0 .. q_{qpk-1}, k, v]
   float *kc, *vc;  // [G][max_seq][hs] (written by the fused form only)
@@ -447,7 +468,8 @@ __host__ __device__ inline int f32_attention_chunk(int keys, int parts) {
 // caches at position pos[0] and into LDS, in the same launch. Latency-bound at decode sizes (300 keys of 64 per head are
 // 150 KB): one key per wave at a time took 80 us, this form 9 beside the rotation and the append. A workgroup's loads bring some
 // 20 GB/s, so that the fused form takes the keys in ranges side by side (grid (parts, H)), whose sums f32_linears_sum_kernel
-// joins; pythia-160m at 301 keys 12.2 us in one range, 7.8 in five.
+// joins; pythia-160m at 301 keys 12.2 us in one range, 7.7 in five, 6.8 with its
+// first rows loaded beside q and the angles.
 template <int LPK, bool FUSED>
 __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   extern __shared__ float sc[];  // [max_seq] scores, then [8][hs] partial sums
@@ -462,6 +484,14 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   const int L = (int)min(max(p + 1, 1L), (long)a.max_seq);
   // this workgroup's keys, of as many ranges as there are keys for
   const int chunk = FUSED && a.parts > 1 ? f32_attention_chunk(L, a.parts) : L, lo = range * chunk, hi = min(lo + chunk, L);
+  const bool mine = sub * 4 < hs;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto row = [&](const float* base, int j) { return mine ? *(const float4*)(base + (size_t)min(j, L - 1) * hs + sub * 4) : zero; };
+  // the token's q, k, v and angles, and behind them the first keys and values (of a fused range all of them), on their way
+  // together. (The fused form's own row is read here before it is written, and not used.)
+  float4 k[4], v[4];
+  float x[5], cs = 1.0f, sn = 0.0f;
+  const int d0 = min((int)threadIdx.x, hs - 1), half = a.n_elem / 2, d1 = d0 < half ? d0 + half : d0 < a.n_elem ? d0 - half : d0;
   if (FUSED) {
     const long rp = a.rope_pos[0];
     if (p < 0 || p >= a.max_seq || rp < 0 || rp >= a.rope_rows) return;  // host validates; never go out of bounds
@@ -469,16 +499,31 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
       if (threadIdx.x == 0) a.ml[((size_t)range * a.H + h) * 2] = -INFINITY, a.ml[((size_t)range * a.H + h) * 2 + 1] = -1.0f;
       return;
     }
-    const float* src = a.q + (size_t)g * (qpk + 2) * hs;
-    const float *cr = a.cos + (size_t)rp * a.n_elem, *sr = a.sin + (size_t)rp * a.n_elem;
-    for (int d = threadIdx.x; d < hs; d += 512) {
-      qs[d] = rope_f32(src + (size_t)(h % qpk) * hs, d, a.n_elem, cr, sr);
-      const float k = rope_f32(src + (size_t)qpk * hs, d, a.n_elem, cr, sr), v = src[(size_t)(qpk + 1) * hs + d];
-      ks[d] = k;
-      vs[d] = v;
+    const float *src = a.q + (size_t)g * (qpk + 2) * hs, *sq = src + (size_t)(h % qpk) * hs, *sk = src + (size_t)qpk * hs;
+    if ((int)threadIdx.x < hs) {
+      x[0] = sq[d0], x[1] = sq[d1], x[2] = sk[d0], x[3] = sk[d1], x[4] = sk[hs + d0];
+      if (d0 < a.n_elem) cs = a.cos[(size_t)rp * a.n_elem + d0], sn = a.sin[(size_t)rp * a.n_elem + d0];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) k[u] = row(kb, lo + first + u * STEP);
+  if (FUSED) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = row(vb, lo + first + u * STEP);
+    __builtin_amdgcn_sched_barrier(0);
+    if ((int)threadIdx.x < hs) {
+      // x * cos + rotate_half(x) * sin on the first n_elem dims, two roundings
+      auto turned = [&](float own, float mate) {
+        return d0 < a.n_elem ? add_rn(mul_rn(own, cs), mul_rn(d0 < half ? -mate : mate, sn)) : own;
+      };
+      const float kd = turned(x[2], x[3]);
+      qs[d0] = turned(x[0], x[1]);
+      ks[d0] = kd;
+      vs[d0] = x[4];
       if (h % qpk == 0 && hi == L) {
-        kb[(size_t)p * hs + d] = k;
-        vb[(size_t)p * hs + d] = v;
+        kb[(size_t)p * hs + d0] = kd;
+        vb[(size_t)p * hs + d0] = x[4];
       }
     }
   } else {
@@ -486,19 +531,20 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
     for (int d = threadIdx.x; d < hs; d += 512) qs[d] = qr[d];
   }
   __syncthreads();
-  const bool mine = sub * 4 < hs;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
   const float4 q4 = mine ? *(const float4*)(qs + sub * 4) : zero;
-  auto row = [&](const float* base, const float* own, int j) {  // (the fused form's own row is not read back)
-    if (!mine) return zero;
-    if (FUSED && j == L - 1) return *(const float4*)(own + sub * 4);
-    return *(const float4*)(base + (size_t)min(j, L - 1) * hs + sub * 4);
+  auto own = [&](float4 (&x)[4], const float* row, int j0) {
+    if (!FUSED || !mine) return;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (j0 + u * STEP == L - 1) x[u] = *(const float4*)(row + sub * 4);
   };
   float mx = -INFINITY;
   for (int j0 = lo + first; j0 < hi; j0 += 4 * STEP) {
-    float4 k[4];
+    if (j0 != lo + first) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) k[u] = row(kb, ks, j0 + u * STEP);
+      for (int u = 0; u < 4; ++u) k[u] = row(kb, j0 + u * STEP);
+    }
+    own(k, ks, j0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       float d = fmaf(q4.w, k[u].w, fmaf(q4.z, k[u].z, fmaf(q4.y, k[u].y, q4.x * k[u].x)));
@@ -529,9 +575,11 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   sum = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
   float4 o = zero;
   for (int j0 = lo + first; j0 < hi; j0 += 4 * STEP) {
-    float4 v[4];
+    if (!FUSED || j0 != lo + first) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = row(vb, vs, j0 + u * STEP);
+      for (int u = 0; u < 4; ++u) v[u] = row(vb, j0 + u * STEP);
+    }
+    own(v, vs, j0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int j = j0 + u * STEP;
@@ -672,8 +720,18 @@ extern "C" int lga_f32_linears_sum(const float* x1, const float* ml, int parts, 
   LGA_CHECK_ARG(parts == 1 || (parts > 1 && parts <= 8 && ml && hs > 0 && K1 % hs == 0 && K1 <= 8192 && K1 / hs <= 256),
                 "lga_f32_linears_sum: 1 to 8 ranges of up to 256 heads, 8192 columns");
   const lga::F32LinearsSum a{x1, w1, b1, x2, w2, b2, residual, y, N, K1, K2, ml, parts, hs};
-  if (parts > 1) lga::f32_linears_sum_kernel<true><<<(N + 3) / 4, 256, (K1 + K1 / hs * 9) * sizeof(float), stream>>>(a);
-  else lga::f32_linears_sum_kernel<false><<<(N + 3) / 4, 256, 0, stream>>>(a);
+  const size_t joined = parts > 1 ? (size_t)K1 + (K1 / hs * 9 + 3) / 4 * 4 : 0;
+  const unsigned grid = (N + 3) / 4;
+#define LGA_SUM(E2)                                                                                                          \
+  do {                                                                                                                        \
+    const size_t lds = (joined + (E2 > 0 ? K2 : 0)) * sizeof(float);                                                         \
+    if (parts > 1) lga::f32_linears_sum_kernel<true, E2><<<grid, 256, lds, stream>>>(a);                                     \
+    else lga::f32_linears_sum_kernel<false, E2><<<grid, 256, lds, stream>>>(a);                                              \
+  } while (0)
+  if ((joined + K2) * sizeof(float) > 65536 || K2 > 8192) LGA_SUM(0);
+  else if (K2 <= 3072) LGA_SUM(3);
+  else LGA_SUM(8);
+#undef LGA_SUM
   LGA_LAUNCH_RETURN();
 }
 
