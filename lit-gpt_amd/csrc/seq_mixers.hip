@@ -688,6 +688,150 @@ __global__ void __launch_bounds__(256) latent_attention_vec_kernel(LatAttArgs p,
   }
 }
 
+// The same for four heads a workgroup (H % 4 == 0): a cached row is loaded and unpacked once for four, and the four heads' scores
+// of a key end in one row of 16 lanes each, where their softmax takes one instruction for all. The next four keys are on their way
+// while these are worked on. Bound by latency. us of a head a workgroup, with a wave sum through LDS per key and head, / here: 3 tokens
+// of 32 heads over 1200, 731 and 64 rows of 512 + 64 28.8 / 18.3, one of 16 over 2048 18.0 / 16.1, five of 16 over 40 to 2000 46.9 /
+// 21.8, eight of 16 over five 10.5 / 8.6, one over five 9.3 / 10.8.
+template <int CTRL>
+__device__ __forceinline__ float lat_dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+// the sums over 64 lanes of four values: row i of 16 lanes holds that of the i-th
+__device__ __forceinline__ float lat_sum4(const float (&v)[4]) {
+  float s[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = lat_dpp_add<0x140>(lat_dpp_add<0x141>(lat_dpp_add<0x4E>(lat_dpp_add<0xB1>(v[i]))));
+  auto swap16 = [](float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  const float ab = swap16(s[0], s[1]), cd = swap16(s[2], s[3]);
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(ab), __float_as_uint(cd), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float lat_of_row(float v, int row) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), row * 16));
+}
+template <bool CF32>
+__global__ void __launch_bounds__(256) latent_attention_heads_kernel(LatAttArgs p, float* __restrict__ part) {
+  constexpr int U = 4, HP = 4, CV = CF32 ? 2 : 1;
+  __shared__ float sm[4][HP], sl[4][HP];
+  extern __shared__ __attribute__((aligned(16))) float sacc[];  // [4][HP][r]
+  const int t = blockIdx.x, h0 = blockIdx.y * HP, z = blockIdx.z, splits = gridDim.z;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r = p.r, dr = p.dr;
+  const int last = min(p.pos[t], p.max_seq - 1);
+  const int first = p.window > 0 ? max(0, last - p.window + 1) : 0;
+  const int share = (last - first + splits) / splits;  // ceil((last - first + 1) / splits)
+  const int lo = first + z * share, hi = min(last, lo + share - 1);
+  const size_t base = (size_t)p.slot[t] * p.max_seq;
+  const bool live = 8 * lane < r;
+  const int at = live ? 8 * lane : 0, rot[2] = {min(lane, max(dr - 1, 0)), min(lane + 64, max(dr - 1, 0))};
+  uint4 raw[U][CV];
+  float kr[U][2];
+  auto fetch = [&](int j0) {  // (past the end the last key again, without weight)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t row = base + max(min(j0 + 4 * u, hi), 0);
+#pragma unroll
+      for (int c = 0; c < CV; ++c) raw[u][c] = ((const uint4*)((const char*)p.cache_c + (row * r + at) * (CF32 ? 4 : 2)))[c];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) kr[u][e] = dr > 0 ? p.cache_kr[row * dr + rot[e]] : 0.0f;
+    }
+  };
+  fetch(lo + wave);
+  float q[HP][8], qrot[HP][2], acc[HP][8];
+#pragma unroll
+  for (int i = 0; i < HP; ++i) {
+    const float* qc = p.qc + ((size_t)t * p.H + h0 + i) * r + at;
+    const float* qr = p.proj + (size_t)t * p.ld + p.q_off + (size_t)(h0 + i) * (p.d + dr) + p.d;
+    const float4 lo4 = ((const float4*)qc)[0], hi4 = ((const float4*)qc)[1];
+    const float qv[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[i][e] = live ? qv[e] : 0.0f, acc[i][e] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) qrot[i][e] = lane + 64 * e < dr ? qr[lane + 64 * e] : 0.0f;
+  }
+  float m = -INFINITY, l = 0.0f;  // row i of 16 lanes: head i's
+  for (int j0 = lo + wave; j0 <= hi; j0 += 4 * U) {
+    float c[U][8], s[U], mn = m;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if constexpr (CF32) {
+        const uint32_t w[8] = {raw[u][0].x, raw[u][0].y, raw[u][0].z, raw[u][0].w, raw[u][CV - 1].x, raw[u][CV - 1].y, raw[u][CV - 1].z, raw[u][CV - 1].w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[u][e] = __uint_as_float(w[e]);
+      } else {
+        const uint4 w = raw[u][0];
+        c[u][0] = bflo(w.x), c[u][1] = bfhi(w.x), c[u][2] = bflo(w.y), c[u][3] = bfhi(w.y);
+        c[u][4] = bflo(w.z), c[u][5] = bfhi(w.z), c[u][6] = bflo(w.w), c[u][7] = bfhi(w.w);
+      }
+      float dot[HP];
+#pragma unroll
+      for (int i = 0; i < HP; ++i) {
+        dot[i] = 0.0f;
+        if (lane < dr) dot[i] = fmaf(qrot[i][0], kr[u][0], dot[i]);
+        if (lane + 64 < dr) dot[i] = fmaf(qrot[i][1], kr[u][1], dot[i]);
+        if (live)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dot[i] = fmaf(q[i][e], c[u][e], dot[i]);
+      }
+      s[u] = j0 + 4 * u <= hi ? lat_sum4(dot) * p.scale : -INFINITY;
+      mn = fmaxf(mn, s[u]);
+    }
+    fetch(j0 + 4 * U);
+    const float corr = expf(m - mn);
+    m = mn;
+    l *= corr;
+#pragma unroll
+    for (int i = 0; i < HP; ++i) {
+      const float f = lat_of_row(corr, i);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[i][e] *= f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (j0 + 4 * u > hi) break;
+      const float w = expf(s[u] - mn);
+      l += w;
+#pragma unroll
+      for (int i = 0; i < HP; ++i) {
+        const float f = lat_of_row(w, i);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[i][e] = fmaf(f, c[u][e], acc[i][e]);
+      }
+    }
+  }
+  if (lane % 16 == 0) sm[wave][lane / 16] = m, sl[wave][lane / 16] = l;
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < HP; ++i) {
+      float4* to = (float4*)(sacc + ((size_t)wave * HP + i) * r + 8 * lane);
+      to[0] = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]), to[1] = make_float4(acc[i][4], acc[i][5], acc[i][6], acc[i][7]);
+    }
+  }
+  __syncthreads();
+  // a wave a head
+  const bool fin = splits == 1;
+  const float snk = (fin && p.sink) ? p.sink[h0 + wave] : -INFINITY;
+  const float mx = fmaxf(fmaxf(fmaxf(sm[0][wave], sm[1][wave]), fmaxf(sm[2][wave], sm[3][wave])), snk);
+  float f[4], den = (fin && p.sink) ? expf(snk - mx) : 0.0f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    f[w] = sl[w][wave] > 0.0f ? expf(sm[w][wave] - mx) : 0.0f;
+    den += sl[w][wave] * f[w];
+  }
+  const size_t head = (size_t)t * p.H + h0 + wave;
+  float* o = fin ? p.out + head * r : part + (head * splits + z) * (r + 2) + 2;
+  if (!fin && lane == 0) o[-2] = mx, o[-1] = den;
+  const float* x = sacc + (size_t)wave * r;
+  for (int k = lane; k < r; k += 64) {
+    const float v = (x[k] * f[0] + x[(size_t)HP * r + k] * f[1]) + (x[(size_t)2 * HP * r + k] * f[2] + x[(size_t)3 * HP * r + k] * f[3]);
+    o[k] = fin ? v / den : v;
+  }
+}
+
 // The prompt form: 16 consecutive tokens of one sequence and one head per workgroup, key tiles of 16 cached rows
 // staged in LDS as fp32, both products on v_mfma_f32_16x16x4_f32. The four waves split the score product over the
 // latent / rotated dims (partial 16x16 tiles summed through LDS) and the weighted sum over the r output columns
@@ -1019,7 +1163,11 @@ extern "C" int lgs_latent_attention(const float* qc, const float* proj, long ld,
     if (cache_f32) lgs::latent_attention_kernel<true, NR><<<grid, 256, lds, stream>>>(p, part);        \
     else lgs::latent_attention_kernel<false, NR><<<grid, 256, lds, stream>>>(p, part);                 \
   } while (0)
-  if (r % 8 == 0 && r <= 512 && (uintptr_t)cache_c % 16 == 0 && (uintptr_t)qc % 16 == 0) {  // 16-byte row loads
+  const bool vec = r % 8 == 0 && r <= 512 && (uintptr_t)cache_c % 16 == 0 && (uintptr_t)qc % 16 == 0;  // 16-byte row loads
+  if (vec && H % 4 == 0) {
+    if (cache_f32) lgs::latent_attention_heads_kernel<true><<<dim3(T, H / 4, splits), 256, 4 * lds, stream>>>(p, part);
+    else lgs::latent_attention_heads_kernel<false><<<dim3(T, H / 4, splits), 256, 4 * lds, stream>>>(p, part);
+  } else if (vec) {
     if (cache_f32) lgs::latent_attention_vec_kernel<true><<<grid, 256, lds, stream>>>(p, part);
     else lgs::latent_attention_vec_kernel<false><<<grid, 256, lds, stream>>>(p, part);
   } else if (r <= 128) LGS_LAT(2);

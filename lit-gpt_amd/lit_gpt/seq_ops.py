@@ -325,7 +325,8 @@ def latent_attention(qc: torch.Tensor, proj: torch.Tensor, q_off: int, cache_c: 
                      sink: Optional[torch.Tensor], slot: torch.Tensor, pos: torch.Tensor, *, H: int, d: int, dr: int,
                      r: int, scale: float, splits: Optional[int] = None, window: int = 0) -> torch.Tensor:
     """Softmax attention of every (token, head) over its sequence's cached rows up to the token's position (``window``
-    > 0: the last ``window`` of them), in the latent space; the rotated query parts are read from ``proj`` at ``q_off``. ``splits``: workgroups per (token, head); by default enough of them to fill the chip when the
+    > 0: the last ``window`` of them), in the latent space; the rotated query parts are read from ``proj`` at ``q_off``.
+    ``splits``: workgroups per token and head (or four heads); by default enough of them to fill the chip when the
     step has few rows (decode), one when it has many (a prompt)."""
     T, ld = proj.shape
     S = cache_c.shape[1]
@@ -333,7 +334,7 @@ def latent_attention(qc: torch.Tensor, proj: torch.Tensor, q_off: int, cache_c: 
         raise ValueError("latent_attention: shapes")
     out = torch.empty(T, H * r, dtype=F32, device=proj.device)
     if splits is None:
-        splits = max(1, min(32, 1024 // (T * H)))
+        splits = max(1, min(32, (1024 if H % 4 else 1536) // (T * H)))  # (a head a workgroup, or four)
         if window > 0:  # at least one key per wave of a split
             splits = max(1, min(splits, window // 4))
     part = torch.empty(T * H * splits * (r + 2), dtype=F32, device=proj.device) if splits > 1 else None

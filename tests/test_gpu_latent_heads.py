@@ -1,0 +1,37 @@
+"""Latent attention of few tokens, four heads a workgroup and one (csrc/seq_mixers.hip), against float64: ranks and rotated parts at the
+lanes' edges, both caches, windows, sinks, more ranges of keys than keys. Tolerance: sums of some 600 products and the softmax's in fp32
+stay within 2e-6 of the largest value of a row of weighted means."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H", [4, 8, 6, 1])
+@pytest.mark.parametrize("r,dr,d", [(512, 64, 128), (504, 128, 8), (8, 1, 16), (64, 0, 32), (72, 65, 0)])
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("window", [0, 1, 37])
+@pytest.mark.parametrize("splits", [None, 1, 9, 64])
+def test_few_tokens(H, r, dr, d, f32, window, splits):
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(r + H)
+    rand = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    lengths, slots, S = [300, 1, 17, 64, 5], [3, 0, 4, 1, 2], 320
+    T, ld, off = len(lengths), H * (d + dr) + 5, 3
+    c, kr = rand(5, S, r) if f32 else rand(5, S, r).bfloat16(), rand(5, S, max(dr, 1))[..., :dr].contiguous()
+    qc, proj, sink = rand(T, H * r) * r ** -0.5, rand(T, ld), rand(H) if H != 8 else None
+    at = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    got = seq_ops.latent_attention(qc, proj, off, c, kr if dr else rand(5, S, 1), sink, at(slots), at([n - 1 for n in lengths]), H=H, d=d,
+                                   dr=dr, r=r, scale=0.3, splits=splits, window=window)
+    for t, (n, slot) in enumerate(zip(lengths, slots)):
+        lo = max(0, n - window) if window else 0
+        rows, rot = c[slot, lo:n].double(), kr[slot, lo:n].double()
+        q = proj[t, off:off + H * (d + dr)].double().view(H, d + dr)[:, d:]
+        score = (qc[t].double().view(H, r) @ rows.T + q @ rot.T) * 0.3
+        if sink is not None:
+            score = torch.cat([score, sink.double()[:, None]], 1)
+        want = torch.softmax(score, 1)[:, :n - lo] @ rows
+        assert (got[t].double().view(H, r) - want).abs().max() < 2e-6 * max(1.0, float(rows.abs().max())) * 4
