@@ -188,42 +188,46 @@ __global__ void __launch_bounds__(256) lin_glu_row_kernel(const float* __restric
   if (lane == 0) y[col] = glu_f<CLAMPED>(f, g, u);
 }
 
-// the value that the lane eight further on in the row of 16 holds
-__device__ __forceinline__ uint32_t rows_up8(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false);
-}
-// Three to eight rows of A on bf16 weights, on the matrix cores: the operands are the same (A rounded to bf16), and a weight
+// Up to eight rows of A on bf16 weights, on the matrix cores: the operands are the same (A rounded to bf16), and a weight
 // costs no vector instruction however many rows there are. A workgroup owns 16 NR columns; its KW waves each take a
-// range of K, 128 values at a time: PF blocks ahead a lane loads 4 x 16 bytes of its own row of W (256 bytes of a row
-// together) and half of its row of A, of whose 32-value pieces the lanes of the upper eight rows hold every second one.
+// range of K, 128 values at a time: the columns' 256 bytes of W and the MR rows' 512 of A come by LDS-DMA (whole lines,
+// source-swizzled so that fragments are read without bank conflicts) into LDS of the wave's own, so that no barrier is theirs, and are
+// fetched anew as soon as they are in registers. One block's buffers a wave: more workgroups a compute unit hide its trips better than
+// blocks ahead do (8 x 32000 x 2048 30 us, 35 with two blocks' buffers, 36 with three).
 // Sums: two instructions, then vector adds, then the ranges pairwise, so that the error against float64 is what the
 // lanes' sums of lin_gemv_kernel leave (rms of 8 rows at K 2048 / 4096 / 11008: 7.4e-8 / 8.0e-8 / 9.5e-8 of the results,
 // 7.5e-8 / 8.4e-8 / 1.1e-7 there; one chain of instructions 1.5 to 3 times as much).
-// Bound by memory, and by the loads' latency where a wave's range is a few blocks: 8 x 22016 x 4096 51 us (3.5 TB/s), 8 x
-// 4096 x 11008 28 us (3.2 TB/s); a lane's sums 84 and 85.
-template <int NR, int KW>
+// Bound by memory, with few columns by its latency. Loaded into registers as the instructions take them, every lane's 16 bytes lay
+// in a line of their own, and a compute unit got some 17 bytes a ns of W and A together, from whichever cache. us there / here, weights
+// from memory, the same bits: 8 x 2048 x 2048 11.9 / 5.9, x 4096 x 2048 10.1 / 7.6, x 6288 x 2048 14.2 / 9.4, x 32000 x 2048 44.5 / 30.2, x
+// 4096 x 4096 14.4 / 11.3, x 12288 x 4096 35.2 / 23.4, 3 x 12288 x 4096 30.5 / 20.6, x 32000 x 4096 59 / 48.
+template <int NR, int KW, int MR>
 __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
-  constexpr int PF = 3;
-  __shared__ f32x4_t part[KW][NR][64];
+  constexpr int W_BYTES = NR * 4096, A_BYTES = MR * 512, SLOT = W_BYTES + A_BYTES, PW = NR * 4, PA = MR / 2;
+  static_assert(KW * SLOT <= 163840 && NR * 1024 <= SLOT, "LDS");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds_all[KW * SLOT];
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned char* lds = lds_all + wave * SLOT;
   const int z = blockIdx.y, n0 = blockIdx.x * (16 * NR);
   const int nb = p.K / 128, b0 = wave * nb / KW, b1 = (wave + 1) * nb / KW;
-  const float* a = p.a + (size_t)z * p.sa + (size_t)min(l15 & 7, p.M - 1) * p.lda + (l15 >> 3) * 32 + q4 * 8;
-  const uint16_t* w[NR];
+  const unsigned char *w[PW], *a[PA];
 #pragma unroll
-  for (int j = 0; j < NR; ++j)
-    w[j] = (const uint16_t*)p.w + (size_t)z * p.sw + (size_t)min(n0 + j * 16 + l15, p.N - 1) * p.K + q4 * 8;
-  bf16x8_t wr[PF][NR][4];
-  float4 ar[PF][4];
-  auto fetch = [&](int b, int s) {  // (past the range: its last block, never used)
-    const size_t at = (size_t)max(min(b, b1 - 1), 0) * 128;
+  for (int i = 0; i < PW; ++i) {  // four rows of 256 bytes
+    const int row = i * 4 + q4;
+    w[i] = (const unsigned char*)((const uint16_t*)p.w + (size_t)z * p.sw + (size_t)min(n0 + row, p.N - 1) * p.K) + 16 * (l15 ^ (row & 15));
+  }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) ar[s][2 * u] = *(const float4*)(a + at + u * 64), ar[s][2 * u + 1] = *(const float4*)(a + at + u * 64 + 4);
+  for (int i = 0; i < PA; ++i) {  // two rows of 512
+    const int row = i * 2 + (lane >> 5);
+    a[i] = (const unsigned char*)(p.a + (size_t)z * p.sa + (size_t)min(row, p.M - 1) * p.lda) + 16 * ((lane & 31) ^ row);
+  }
+  auto dma = [&](int b) {  // (past the range: its last block, never used)
+    const size_t at = (size_t)max(min(b, b1 - 1), 0) * 256;
 #pragma unroll
-    for (int j = 0; j < NR; ++j)
+    for (int i = 0; i < PW; ++i) lga::gemm_dma16(w[i] + at, lds + i * 1024);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) wr[s][j][m] = *(const bf16x8_t*)(w[j] + at + m * 32);
+    for (int i = 0; i < PA; ++i) lga::gemm_dma16(a[i] + 2 * at, lds + W_BYTES + i * 1024);
   };
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   f32x4_t acc[4][NR];
@@ -231,37 +235,55 @@ __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < NR; ++j) acc[i][j] = zero;
+  dma(b0);
+  const int arow = l15 & (MR - 1), w_at = l15 * 256, a_at = W_BYTES + arow * 512;
+  for (int b = b0; b < b1; b += 2) {
 #pragma unroll
-  for (int s = 0; s < PF; ++s) fetch(b0 + s, s);
-  for (int b = b0; b < b1; b += 2 * PF) {
-#pragma unroll
-    for (int s = 0; s < 2 * PF; ++s) {
+    for (int s = 0; s < 2; ++s) {
       if (b + s < b1) {
+        lga::gemm_wait_vm<0>();
+        bf16x8_t wr[4][NR];
+        float4 x[4][2];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+#pragma unroll
+          for (int j = 0; j < NR; ++j) wr[m][j] = *(const bf16x8_t*)(lds + w_at + j * 4096 + 16 * ((m * 4 + q4) ^ l15));
+#pragma unroll
+          for (int e = 0; e < 2; ++e) x[m][e] = *(const float4*)(lds + a_at + 16 * ((m * 8 + q4 * 2 + e) ^ arow));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before it is filled again)
+        __builtin_amdgcn_sched_barrier(0);
+        dma(b + s + 1);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const float4 lo = ar[s % PF][2 * u], hi = ar[s % PF][2 * u + 1];
-          const uint4 x = make_uint4(pack2(lo.x, lo.y), pack2(lo.z, lo.w), pack2(hi.x, hi.y), pack2(hi.z, hi.w));
-          const uint4 t = make_uint4(rows_up8(x.x), rows_up8(x.y), rows_up8(x.z), rows_up8(x.w));
+          f32x4_t v[NR];
 #pragma unroll
-          for (int j = 0; j < NR; ++j) {
-            f32x4_t v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[s % PF][j][2 * u], __builtin_bit_cast(bf16x8_t, x), zero, 0, 0, 0);
-            v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[s % PF][j][2 * u + 1], __builtin_bit_cast(bf16x8_t, t), v, 0, 0, 0);
-            acc[(s & 1) * 2 + u][j] += v;
+          for (int m = 2 * u; m < 2 * u + 2; ++m) {
+            const uint4 x16 = make_uint4(pack2(x[m][0].x, x[m][0].y), pack2(x[m][0].z, x[m][0].w), pack2(x[m][1].x, x[m][1].y), pack2(x[m][1].z, x[m][1].w));
+#pragma unroll
+            for (int j = 0; j < NR; ++j)
+              v[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[m][j], __builtin_bit_cast(bf16x8_t, x16), m == 2 * u ? zero : v[j], 0, 0, 0);
           }
+#pragma unroll
+          for (int j = 0; j < NR; ++j) acc[s * 2 + u][j] += v[j];
         }
-        fetch(b + s + PF, s % PF);
       }
     }
   }
+  lga::gemm_wait_vm<0>();  // no DMA may outlive its slot
+  __syncthreads();
+  f32x4_t* part = (f32x4_t*)lds_all;  // [KW][NR][64]
 #pragma unroll
-  for (int j = 0; j < NR; ++j) part[wave][j][lane] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
+  for (int j = 0; j < NR; ++j) part[(wave * NR + j) * 64 + lane] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
   __syncthreads();
   if (tid >= NR * 64 || l15 >= p.M) return;
   const int j = NR > 1 ? wave : 0;
   f32x4_t v = zero;
 #pragma unroll
-  for (int k = 0; k < KW; k += 4)
-    v += (part[k][j][lane] + part[k + 1][j][lane]) + (part[k + 2][j][lane] + part[k + 3][j][lane]);
+  for (int k = 0; k < KW; k += 4) {
+    const f32x4_t* at = part + (k * NR + j) * 64 + lane;
+    v += (at[0] + at[NR * 64]) + (at[2 * NR * 64] + at[3 * NR * 64]);
+  }
   float* y = p.y + (size_t)z * p.sy + (size_t)l15 * p.ldy;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -270,6 +292,27 @@ __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
     const float o = act_f(p.act, v[r] + (p.bias ? p.bias[n] : 0.0f));
     y[n] = p.accumulate ? y[n] + o : o;
   }
+}
+// 16 columns a workgroup; 32, which read A half as often, for more than four rows where their workgroups end together: many, or one a
+// compute unit (us of 16 / 32 columns: 8 x 32000 x 2048 31.3 / 30.2, x 22016 x 4096 40.6 / 37.6, x 6288 x 2048 9.8 / 9.4, x 4608 x 4096
+// 13.0 / 12.1, x 8192 x 2048 9.5 / 10.2, x 4096 x 4096 11.3 / 13.4; 3 x 32000 x 4096 48.2 / 50.8). Below 4096 columns eight waves share K.
+template <int NR, int KW>
+static void lin_rows_go(const LinArgs& p, int batch, hipStream_t stream) {
+  const dim3 grid((p.N + 16 * NR - 1) / (16 * NR), batch);
+  if (p.M > 4) lin_rows_kernel<NR, KW, 8><<<grid, KW * 64, 0, stream>>>(p);
+  else lin_rows_kernel<NR, KW, 4><<<grid, KW * 64, 0, stream>>>(p);
+}
+
+// What they gain on a lane's sums (lin_gemv_kernel; us there / here): 5 to 8 rows always (8 x 64 x 512 5.5 / 3.1, 5 x 1024 x 4096 15.3 / 7.2),
+// four but of few columns and long rows (4 x 1024 x 2048 7.4 / 4.4, x 20608 x 2048 34.3 / 18.8; x 256 x 2048 4.1 / 4.0, x 256 x 4096 5.4 /
+// 4.9), two and three of long rows (2 x 2048 x 4096 9.0 / 7.9, 3 x 1024 x 4096 11.4 / 6.6; 3 x 512 x 8192 8.9 / 9.3), one of longer rows and few
+// columns (1 x 2048 x 5632 10.0 / 9.2, x 3072 x 8192 15.7 / 12.3; x 512 x 5632 5.0 / 7.4, x 2048 x 2048 5.2 / 5.4). Two and three shorter
+// rows (2 x 8192 x 2048 12.6 / 9.1) keep the bits that each has alone. columns: of all batches
+static bool lin_rows_pay(int M, long columns, int K) {
+  if (K % 128 != 0 || M > 8) return false;
+  if (M == 1) return K > 4096 && columns > 512 && columns < 4096;
+  if (M <= 3) return K >= 4096 && columns > 512;
+  return M > 4 || columns > 512 || K < 1024;
 }
 
 // ------------------------------------------------------------------------------------------------ MFMA tiles
@@ -684,18 +727,12 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
                  a_bf16 ? (const uint16_t*)a : nullptr, y_bf16 ? (uint16_t*)y : nullptr, bias, nullptr, 1, 0};
   LGA_CHECK_ARG(ksplit >= 1 && (ksplit == 1 || (part && !w_f32 && batch == 1 && !z_start && !a_rows && M > 8 && M <= 65535)),
                 "lgs_linear: K is split for one plain product on the MFMA tiles, with a workspace");
-  // Several rows on the matrix cores (us here / a lane's sums): 5 to 8 rows of at least 2048 columns (8 x 2048 x 2048 11.5 /
-  // 12.4, x 8256 x 2048 21 / 26, x 4096 x 11008 28 / 85, x 32000 x 4096 68 / 104; x 512 x 2048 11.4 / 6.1), 3 and 4 rows
-  // from K 4096 (4 x 4096 x 4096 12.7 / 20.8, x 20608 x 4096 45 / 55; x 10304 x 2048 21 / 19); 2 x 20608 x 4096 44 / 38.
-  // 16 columns a workgroup while that is one to a compute unit, 32 beyond (us of 16 / 32 columns: 8 x 4096 x 4096 14.3 / 18.2,
-  // x 4608 x 4096 23.2 / 19.0, x 20608 x 4096 61 / 49; x 8256 x 2048 21.5 / 22.0), the same sums either way. Below 4096 columns
-  // eight waves share K, not four (8 x 2048 x 2048: 11.8; four would take 9.3 and add in another order). A row's bits are not
-  // those that it has alone: lin_gemv_kernel adds in another order
-  if (!z_start && !a_rows && !w_f32 && M > 2 && M <= 8 && N >= 2048 && (M > 4 || K >= 4096) && K % 128 == 0 && lda % 4 == 0 &&
-      stride_a % 4 == 0 && stride_w % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0) {
-    if (N > 4096) lgs::lin_rows_kernel<2, 4><<<dim3((N + 31) / 32, batch), 256, 0, stream>>>(p);
-    else if (N >= 4096) lgs::lin_rows_kernel<1, 4><<<dim3((N + 15) / 16, batch), 256, 0, stream>>>(p);
-    else lgs::lin_rows_kernel<1, 8><<<dim3((N + 15) / 16, batch), 512, 0, stream>>>(p);
+  // A row's bits are not those that it has alone: lin_gemv_kernel adds in another order
+  if (!z_start && !a_rows && !w_f32 && lgs::lin_rows_pay(M, (long)N * batch, K) && lda % 4 == 0 && stride_a % 4 == 0 &&
+      stride_w % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0) {
+    if (N < 4096) lgs::lin_rows_go<1, 8>(p, batch, stream);
+    else if (M > 4 && (N >= 16384 || (N > 4096 && N < 8192))) lgs::lin_rows_go<2, 4>(p, batch, stream);
+    else lgs::lin_rows_go<1, 4>(p, batch, stream);
     LGA_LAUNCH_RETURN();
   }
   if (M <= 8 && !z_start && !a_rows) {
@@ -795,7 +832,7 @@ extern "C" int lgs_linear_glu(const void* a, long lda, const void* w, long strid
   LGA_LAUNCH_RETURN();
 }
 
-extern "C" int lgs_linear_glu_row_fits(int columns, int K) { return columns > 0 && K > 0 && K % 8 == 0 && !lgs::gemv_deep(columns, K) ? 1 : 0; }
+extern "C" int lgs_linear_glu_row_fits(int columns, int K) { return columns > 0 && K > 0 && K % 8 == 0 && !lgs::gemv_deep(columns, K) && !lgs::lin_rows_pay(1, columns, K) ? 1 : 0; }
 
 extern "C" int lgs_linear_glu_row(const float* a, const void* w, long up_rows, float* y, int n, int K, int act, int clamped,
                                   float alpha, float limit, float shift, hipStream_t stream) {

@@ -165,8 +165,8 @@ def linear(a: torch.Tensor, w: torch.Tensor, *, M: int, N: int, K: int, y: torch
     are ``a_rows`` (or the list places themselves) and whose Y rows are the list places. ``a`` may be a producer's
     bf16 copy (``rmsnorm(bf16_copy=True)``, ``glu(bf16=True)``) for the MFMA tiles with bf16 weights. ``ksplit`` > 1: that
     many ranges of K side by side (MFMA tiles, one plain product), see ``thin_ksplit``; 0: as many as suit a bf16 ``a``,
-    one otherwise. The order of a row's sums depends on the number of rows: up to 2 (4 below K 4096) and 3 (5) to 8 rows of bf16
-    weights, and more, take different kernels, and ``ksplit`` 0 differs with the size, so the bits of a row may too."""
+    one otherwise. The order of a row's sums depends on the number of rows: one, two to eight and more rows
+    of bf16 weights take different kernels by their sizes, and ``ksplit`` 0 differs with the size, so the bits of a row may too."""
     a16 = a.dtype == torch.bfloat16
     ap = _dev(a, "a", torch.bfloat16 if a16 else F32) + (2 if a16 else 4) * a_off
     y16 = y.dtype == torch.bfloat16  # the result feeds another bf16 product
