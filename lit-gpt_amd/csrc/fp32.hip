@@ -18,7 +18,7 @@
 //   lga_f32_attention_decode  the two above for one token in one launch
 // (the token-embedding gather is lga_embedding over the fp32 rows as pairs of 16-bit words — a byte copy; greedy
 // sampling is lga_argmax_f32 in sample.hip)
-#include "common.h"
+#include "gemm_tiles.h"
 
 namespace lga {
 
@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(256) f32_linear_kernel(const float* __restrict
   }
 }
 
-// Prompts, K % 4 == 0: the same sums for eight rows and two outputs a wave. A wave per output read the matrix once a row from L2 and
+// Prompts of other K % 4 == 0: the same sums for eight rows and two outputs a wave. A wave per output read the matrix once a row from L2 and
 // a kilobyte of x for every four products of its lanes; here ten loads stand beside 64. Lane 2 r + o finishes row r of output o.
 // us, a wave per output / here: 300 rows of 3072 x 768 204 / 92, of 768 x 3072 158 / 90, 40 rows 30 / 18, 26 / 17
 __global__ void __launch_bounds__(256) f32_linear_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -113,6 +113,120 @@ __global__ void __launch_bounds__(256) f32_linear_rows_kernel(const float* __res
   y[(size_t)m * N + n] = acc;
 }
 
+typedef float f32x32_t __attribute__((ext_vector_type(32)));
+typedef float f32q_t __attribute__((ext_vector_type(4)));
+
+// Prompts of K % 256 == 0, two rows and more: the same sums once more, on the fp32 matrix cores. f32_linear_kernel's sum is 256 chains
+// (k modulo 256) and a tree over them; a matrix instruction of one k (32x32x1, 16x16x1: 2 or 4 products' blocks side by side)
+// extends one chain of T x T outputs by an fma, so the blocks take the chains that the tree joins first, the four values of a lane's 16
+// bytes four accumulators, and a wave the chains of one 16-byte chunk of every 128-byte line: its part of the tree lies in its own
+// registers, and the last three levels join the eight waves. Rounding, denormals and infinities are fmaf's: the bits of one row alone.
+// A step is 16 KB of x and W by LDS-DMA (whole lines, chunks source-swizzled so that 16 lanes of a fragment read all banks), four on
+// their way, and four instructions a wave. The fragments are read as vectors of the compiler's own: reads of HIP's float4 may alias the
+// DMAs for it, and it waits for all of them before each (T 32: 300 x 768 x 3072 26.5 us so, 20.6 as it is).
+// Bound by the matrix cores (a step without its DMAs takes 0.9 of the time, without its instructions 0.55) and the tree's 256 adds an
+// output; at few rows by one workgroup's chain of steps. us, f32_linear_kernel or f32_linear_rows_kernel / here: 300 rows of 3072 x 768 88 / 31, of
+// 768 x 3072 89 / 21, of 768 x 768 25 / 9.0; 40 rows 16.8 / 9.0, 15.9 / 8.7, 7.6 / 4.6; 16 rows 9.7 / 4.9, 14.3 / 8.3, 5.4 / 4.6; 16 of 50304
+// x 768 100 / 42; 8 of 4096 x 1024 10.9 / 6.3.
+template <int T, int RING>
+__global__ void __launch_bounds__(512, T == 32 ? 2 : 4) f32_linear_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                 const float* __restrict__ b, int act,
+                                                                 const float* __restrict__ res, const float* __restrict__ res2,
+                                                                 float* __restrict__ y, int M, int N, int K) {
+  constexpr int BLK = 64 / T, SETS = 8 / BLK, REG = T * T / 64, STEP = 16384;
+  using Acc = std::conditional_t<T == 32, f32x32_t, f32x16_t>;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING * STEP];
+  static_assert(RING >= 3 && T * T * 32 <= RING * STEP, "one step in use, others on their way; the waves' sums in their place");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tm = (M + T - 1) / T, tn = (N + T - 1) / T, per = (tm * tn + 7) / 8;
+  const int at = (blockIdx.x % 8) * per + blockIdx.x / 8;  // (an XCD's workgroups: neighbouring columns, all rows)
+  if (at >= tm * tn) return;
+  const int m0 = at % tm * T, n0 = at / tm * T;
+  const unsigned char* src[2];
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const int q = (wave * 2 + d) * 8 + (lane >> 3), blk = q / (2 * T), r = q % (2 * T), line = T == 32 ? 4 * blk : 4 * (blk & 1) + 2 * (blk >> 1);
+    const float* row = r < T ? x + (size_t)min(m0 + r, M - 1) * K : w + (size_t)min(n0 + r - T, N - 1) * K;
+    src[d] = (const unsigned char*)row + 128 * line + 16 * ((lane & 7) ^ ((q >> 1) & 7));
+  }
+  const int n = K / 256, last = SETS * n - 1;
+  int set = 0, i = 0;  // of the next step to fetch (past the last: that one again, never used)
+  auto dma = [&](int buffer) {
+    const int at = 128 * (T == 32 ? (set & 1) * 2 + (set >> 1) : set) + 1024 * i;
+#pragma unroll
+    for (int d = 0; d < 2; ++d) gemm_dma16(src[d] + at, lds + buffer * STEP + (wave * 2 + d) * 1024);
+    if (set * n + i < last && ++i == n) i = 0, ++set;
+  };
+  const int row = lane % T, chunk = 16 * (wave ^ ((row >> 1) & 7));
+  const int a_at = (lane / T * 2 * T + row) * 128 + chunk, b_at = a_at + T * 128;
+#pragma unroll
+  for (int s = 0; s < RING; ++s) dma(s);
+  gemm_wait_vm<2 * (RING - 1)>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  f32q_t a = *(const f32q_t*)(lds + a_at), c = *(const f32q_t*)(lds + b_at);
+  int buffer = 0;
+  float t[2][REG];
+#pragma unroll
+  for (int s = 0; s < SETS; ++s) {
+    Acc acc[4];
+    auto step = [&](auto first) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this step's values are in registers, its buffer is free, ...
+      gemm_wait_vm<2 * (RING - 2)>();                      // ... and the next step's have landed
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      const int freed = buffer;
+      buffer = buffer + 1 == RING ? 0 : buffer + 1;
+      const f32q_t a1 = *(const f32q_t*)(lds + buffer * STEP + a_at), c1 = *(const f32q_t*)(lds + buffer * STEP + b_at);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (T == 32) acc[e] = __builtin_amdgcn_mfma_f32_32x32x1f32(a[e], c[e], first ? Acc(0.0f) : acc[e], 0, 0, 0);
+        else acc[e] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], c[e], first ? Acc(0.0f) : acc[e], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (e == 0) dma(freed);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      a = a1, c = c1;
+    };
+    step(std::true_type{});
+#pragma nounroll
+    for (int k = 1; k < n; ++k) step(std::false_type{});
+#pragma unroll
+    for (int r = 0; r < REG; ++r) {
+      float v[BLK];
+#pragma unroll
+      for (int k = 0; k < BLK; ++k) v[k] = (acc[0][k * REG + r] + acc[1][k * REG + r]) + (acc[2][k * REG + r] + acc[3][k * REG + r]);
+      float sum = v[0] + v[1];
+      if constexpr (BLK == 4) sum += v[2] + v[3];
+      if constexpr (T == 32) t[s >> 1][r] = s & 1 ? t[s >> 1][r] + sum : sum;
+      else t[s][r] = sum;
+      asm volatile("" : "+v"(t[T == 32 ? s >> 1 : s][r]));  // (or the sums sink to the end and every set's products stay in registers)
+    }
+  }
+  gemm_wait_vm<0>();  // no DMA may outlive its buffer
+  __syncthreads();
+  float* part = (float*)lds;
+#pragma unroll
+  for (int r = 0; r < REG; ++r) part[(wave * T + (T == 32 ? 8 * (r / 4) : 0) + lane / T * 4 + r % 4) * T + row] = t[0][r] + t[1][r];
+  __syncthreads();
+#pragma unroll
+  for (int e = tid; e < T * T; e += 512) {
+    float p[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) p[k] = part[k * T * T + e];
+    float v = ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
+    const int m = m0 + e / T, o = n0 + e % T;
+    if (m >= M || o >= N) continue;
+    if (b) v += b[o];
+    if (act) v = gelu_f32(v, act == 2);
+    if (res) v += res[(size_t)m * N + o];
+    if (res2) v += res2[(size_t)m * N + o];
+    y[(size_t)m * N + o] = v;
+  }
+}
+
 // From eight rows and some eight waves a CU on, where few of the rows computed are repeated ones or the chip is full several times
 // over. us, a wave per output / here: 8 rows of 4096 x 768 9.3 / 8.3, of 3072 x 768 (1536 waves) 7.6 / 7.9, of 3072 x 3072 21.1 / 23.6; 9
 // rows of 2304 x 256 4.4 / 6.4, of 4096 x 768 10.5 / 11.5, of 8192 x 768 21.1 / 19.1; 12 rows of 2304 x 768 8.2 / 9.2, of 3072 x 768
@@ -120,6 +234,29 @@ __global__ void __launch_bounds__(256) f32_linear_rows_kernel(const float* __res
 static bool f32_linear_in_rows(int M, int N, int K) {
   const long live = (long)M * N / 16, padded = (long)((N + 1) / 2) * ((M + 7) / 8);  // waves' worth of rows, and waves
   return K % 4 == 0 && M >= 8 && live >= 2000 && (live * 10 >= padded * 7 || live >= 4500);
+}
+
+template <int T>
+static long f32_tiles(int M, int N) { return (long)((M + T - 1) / T) * ((N + T - 1) / T); }
+// Whether the matrix cores serve: from some 9000 outputs on they do at every K, below a wave per output ends sooner. us, a wave per output /
+// T 16: 8 x 1024 x 256 3.0 / 3.3, 9 rows 3.3 / 3.2; 5 x 1536 x 512 3.6 / 4.1, 6 rows 4.2 / 4.1; 3 x 2304 x 768 4.0 / 4.7, 4 rows 4.9 / 4.7; 3 x
+// 3072 x 768 5.0 / 4.9; 8 x 1024 x 4096 11.7 / 11.0; 4 x 2048 x 8192 19.5 / 18.2; 2 x 50304 x 768 44 / 36.
+// (2^23 workgroups of 512: as many work-items as a launch holds)
+static bool f32_linear_in_tiles(int M, int N, int K) {
+  return K % 256 == 0 && M > 1 && (long)M * N >= 9000 && f32_tiles<16>(M, N) < (1 << 23) - 8;
+}
+// Tiles of 16 x 16 (two workgroups a CU) or of 32 x 32 (one, four times the outputs in 1.7 times the time): by rounds of the chip, and 16
+// where one of those tiles a CU is enough. us of 16 / 32: 40 x 768 x 3072 8.8 / 20.4, 64 x 3072 x 768 9.0 / 9.2, 96 x 3072 x 768 12.8 / 16.1,
+// 300 x 3072 x 768 32.4 / 30.5, 300 x 768 x 3072 25.7 / 20.6, 64 x 4096 x 1024 14.8 / 11.6.
+static bool f32_tiles_of_16(int M, int N) {
+  const long t16 = f32_tiles<16>(M, N), t32 = f32_tiles<32>(M, N);
+  return t16 <= 256 || (t16 + 511) / 512 * 3 <= (t32 + 255) / 256 * 5;
+}
+template <int T>
+static void f32_linear_tiles(const float* x, const float* w, const float* bias, int act, const float* residual, const float* residual2, float* y,
+                             int M, int N, int K, hipStream_t stream) {
+  const unsigned blocks = 8 * (unsigned)((f32_tiles<T>(M, N) + 7) / 8);
+  f32_linear_tiles_kernel<T, 4><<<blocks, 512, 0, stream>>>(x, w, bias, act, residual, residual2, y, M, N, K);
 }
 
 // Mean and biased variance of a row by a workgroup of 256, the first 256 CPT columns left in r
@@ -687,7 +824,9 @@ extern "C" int lga_f32_linear_act(const float* x, const float* w, const float* b
                                   const float* residual2, float* y, int M, int N, int K, hipStream_t stream) {
   LGA_CHECK_ARG(x && w && y && M > 0 && N > 0 && K > 0 && M <= 65535 && act >= 0 && act <= 2, "lga_f32_linear: bad arguments");
   LGA_CHECK_ARG(((uintptr_t)x | (uintptr_t)w) % 16 == 0 || K % 4 != 0, "lga_f32_linear: 16-B aligned x, w needed");
-  if (lga::f32_linear_in_rows(M, N, K))
+  if (lga::f32_linear_in_tiles(M, N, K))
+    (lga::f32_tiles_of_16(M, N) ? lga::f32_linear_tiles<16> : lga::f32_linear_tiles<32>)(x, w, bias, act, residual, residual2, y, M, N, K, stream);
+  else if (lga::f32_linear_in_rows(M, N, K))
     lga::f32_linear_rows_kernel<<<dim3((N + 7) / 8, (M + 7) / 8), 256, 0, stream>>>(x, w, bias, act, residual, residual2, y, M, N, K);
   else lga::f32_linear_kernel<<<dim3((N + 3) / 4, M), 256, 0, stream>>>(x, w, bias, act, residual, residual2, y, N, K);
   LGA_LAUNCH_RETURN();
