@@ -192,23 +192,26 @@ __global__ void __launch_bounds__(256) lin_glu_row_kernel(const float* __restric
 // costs no vector instruction however many rows there are. A workgroup owns 16 NR columns; its KW waves each take a
 // range of K, 128 values at a time: the columns' 256 bytes of W and the MR rows' 512 of A come by LDS-DMA (whole lines,
 // source-swizzled so that fragments are read without bank conflicts) into LDS of the wave's own, so that no barrier is theirs, and are
-// fetched anew as soon as they are in registers. One block's buffers a wave: more workgroups a compute unit hide its trips better than
-// blocks ahead do (8 x 32000 x 2048 30 us, 35 with two blocks' buffers, 36 with three).
+// fetched anew as soon as they are in registers. One block's buffers a wave where several workgroups share a compute unit: they hide its
+// trips better than blocks ahead do (us with one / two blocks' buffers: 8 x 32000 x 2048 30.2 / 32.8, x 8192 x 2048 9.4 / 10.2, x 8192 x 4096
+// 15.2 / 16.6, 3 x 6144 x 4096 12.6 / 13.5); two where a workgroup of four waves has one alone (8 x 4096 x 4096 11.3 / 9.3, 3 rows 10.0 / 8.7,
+// 11264 long 23.2 / 18.1, 8 x 6144 x 4096 14.7 / 13.4, 8 x 4096 x 2048 7.2 / 6.6; three are no faster, eight waves' 128 KB slower: 8 x 2048 x
+// 2048 5.9 / 6.6). The rows are read as vectors of the compiler's own: a read of HIP's float4 may alias the DMAs for it, and waits for all.
 // Sums: two instructions, then vector adds, then the ranges pairwise, so that the error against float64 is what the
 // lanes' sums of lin_gemv_kernel leave (rms of 8 rows at K 2048 / 4096 / 11008: 7.4e-8 / 8.0e-8 / 9.5e-8 of the results,
 // 7.5e-8 / 8.4e-8 / 1.1e-7 there; one chain of instructions 1.5 to 3 times as much).
 // Bound by memory, with few columns by its latency. Loaded into registers as the instructions take them, every lane's 16 bytes lay
 // in a line of their own, and a compute unit got some 17 bytes a ns of W and A together, from whichever cache. us there / here, weights
-// from memory, the same bits: 8 x 2048 x 2048 11.9 / 5.9, x 4096 x 2048 10.1 / 7.6, x 6288 x 2048 14.2 / 9.4, x 32000 x 2048 44.5 / 30.2, x
-// 4096 x 4096 14.4 / 11.3, x 12288 x 4096 35.2 / 23.4, 3 x 12288 x 4096 30.5 / 20.6, x 32000 x 4096 59 / 48.
-template <int NR, int KW, int MR>
+// from memory, the same bits: 8 x 2048 x 2048 11.9 / 5.9, x 4096 x 2048 10.1 / 6.6, x 6288 x 2048 14.2 / 9.0, x 32000 x 2048 44.5 / 30.2, x
+// 4096 x 4096 14.4 / 9.3, x 12288 x 4096 35.2 / 23.4, 3 x 12288 x 4096 30.5 / 20.6, x 32000 x 4096 59 / 48.
+template <int NR, int KW, int MR, int RB>
 __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
   constexpr int W_BYTES = NR * 4096, A_BYTES = MR * 512, SLOT = W_BYTES + A_BYTES, PW = NR * 4, PA = MR / 2;
-  static_assert(KW * SLOT <= 163840 && NR * 1024 <= SLOT, "LDS");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_all[KW * SLOT];
+  static_assert(KW * RB * SLOT <= 163840 && NR * 1024 <= SLOT, "LDS");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds_all[KW * RB * SLOT];
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  unsigned char* lds = lds_all + wave * SLOT;
+  unsigned char* lds = lds_all + wave * (RB * SLOT);
   const int z = blockIdx.y, n0 = blockIdx.x * (16 * NR);
   const int nb = p.K / 128, b0 = wave * nb / KW, b1 = (wave + 1) * nb / KW;
   const unsigned char *w[PW], *a[PA];
@@ -222,12 +225,12 @@ __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
     const int row = i * 2 + (lane >> 5);
     a[i] = (const unsigned char*)(p.a + (size_t)z * p.sa + (size_t)min(row, p.M - 1) * p.lda) + 16 * ((lane & 31) ^ row);
   }
-  auto dma = [&](int b) {  // (past the range: its last block, never used)
+  auto dma = [&](int b, int slot) {  // (past the range: its last block, never used)
     const size_t at = (size_t)max(min(b, b1 - 1), 0) * 256;
 #pragma unroll
-    for (int i = 0; i < PW; ++i) lga::gemm_dma16(w[i] + at, lds + i * 1024);
+    for (int i = 0; i < PW; ++i) lga::gemm_dma16(w[i] + at, lds + slot + i * 1024);
 #pragma unroll
-    for (int i = 0; i < PA; ++i) lga::gemm_dma16(a[i] + 2 * at, lds + W_BYTES + i * 1024);
+    for (int i = 0; i < PA; ++i) lga::gemm_dma16(a[i] + 2 * at, lds + slot + W_BYTES + i * 1024);
   };
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   f32x4_t acc[4][NR];
@@ -235,25 +238,28 @@ __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < NR; ++j) acc[i][j] = zero;
-  dma(b0);
+#pragma unroll
+  for (int r = 0; r < RB; ++r) dma(b0 + r, r * SLOT);
+  int slot = 0;
   const int arow = l15 & (MR - 1), w_at = l15 * 256, a_at = W_BYTES + arow * 512;
   for (int b = b0; b < b1; b += 2) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       if (b + s < b1) {
-        lga::gemm_wait_vm<0>();
+        lga::gemm_wait_vm<(RB - 1) * (PW + PA)>();
         bf16x8_t wr[4][NR];
-        float4 x[4][2];
+        f32x4_t x[4][2];
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
 #pragma unroll
-          for (int j = 0; j < NR; ++j) wr[m][j] = *(const bf16x8_t*)(lds + w_at + j * 4096 + 16 * ((m * 4 + q4) ^ l15));
+          for (int j = 0; j < NR; ++j) wr[m][j] = *(const bf16x8_t*)(lds + slot + w_at + j * 4096 + 16 * ((m * 4 + q4) ^ l15));
 #pragma unroll
-          for (int e = 0; e < 2; ++e) x[m][e] = *(const float4*)(lds + a_at + 16 * ((m * 8 + q4 * 2 + e) ^ arow));
+          for (int e = 0; e < 2; ++e) x[m][e] = *(const f32x4_t*)(lds + slot + a_at + 16 * ((m * 8 + q4 * 2 + e) ^ arow));
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before it is filled again)
         __builtin_amdgcn_sched_barrier(0);
-        dma(b + s + 1);
+        dma(b + s + RB, slot);
+        slot = slot + SLOT == RB * SLOT ? 0 : slot + SLOT;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           f32x4_t v[NR];
@@ -294,13 +300,20 @@ __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
   }
 }
 // 16 columns a workgroup; 32, which read A half as often, for more than four rows where their workgroups end together: many, or one a
-// compute unit (us of 16 / 32 columns: 8 x 32000 x 2048 31.3 / 30.2, x 22016 x 4096 40.6 / 37.6, x 6288 x 2048 9.8 / 9.4, x 4608 x 4096
-// 13.0 / 12.1, x 8192 x 2048 9.5 / 10.2, x 4096 x 4096 11.3 / 13.4; 3 x 32000 x 4096 48.2 / 50.8). Below 4096 columns eight waves share K.
+// compute unit (us of 16 / 32 columns: 8 x 32000 x 2048 31.3 / 30.2, x 22016 x 4096 40.6 / 37.6, x 6288 x 2048 9.8 / 9.0, x 4608 x 4096
+// 13.0 / 11.5, x 8192 x 2048 9.5 / 10.2, x 4096 x 4096 9.3 / 13.4; 3 x 32000 x 4096 48.2 / 50.8). Below 4096 columns eight waves share K.
 template <int NR, int KW>
 static void lin_rows_go(const LinArgs& p, int batch, hipStream_t stream) {
   const dim3 grid((p.N + 16 * NR - 1) / (16 * NR), batch);
-  if (p.M > 4) lin_rows_kernel<NR, KW, 8><<<grid, KW * 64, 0, stream>>>(p);
-  else lin_rows_kernel<NR, KW, 4><<<grid, KW * 64, 0, stream>>>(p);
+  if constexpr (KW == 4) {
+    if ((long)grid.x * batch <= 256) {
+      if (p.M > 4) lin_rows_kernel<NR, KW, 8, 2><<<grid, KW * 64, 0, stream>>>(p);
+      else lin_rows_kernel<NR, KW, 4, 2><<<grid, KW * 64, 0, stream>>>(p);
+      return;
+    }
+  }
+  if (p.M > 4) lin_rows_kernel<NR, KW, 8, 1><<<grid, KW * 64, 0, stream>>>(p);
+  else lin_rows_kernel<NR, KW, 4, 1><<<grid, KW * 64, 0, stream>>>(p);
 }
 
 // What they gain on a lane's sums (lin_gemv_kernel; us there / here): 5 to 8 rows always (8 x 64 x 512 5.5 / 3.1, 5 x 1024 x 4096 15.3 / 7.2),

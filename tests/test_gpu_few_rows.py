@@ -11,7 +11,7 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("N,K", [(1, 128), (17, 512), (513, 768), (512, 1024), (514, 1024), (1030, 640), (1024, 4224), (3000, 5632), (4095, 896),
-                                 (4097, 256), (8193, 384), (16400, 128), (5000, 1152)])
+                                 (4097, 256), (8193, 384), (16400, 128), (5000, 1152), (4096, 128), (4096, 1408), (8191, 2176)])
 @pytest.mark.parametrize("M", range(1, 9))
 def test_rows(M, N, K):
     from lit_gpt import seq_ops
