@@ -71,6 +71,7 @@ class BatchEngine:
         model.set_kv_cache(max(1, slots), max_seq_length)
         self.pool = SlotPool()
         self.live: Dict[Hashable, Tuple[int, int]] = {}  # request -> (slot, tokens held so far)
+        StepBatch.build([(0, 0, [0])], self.device)  # (the first step finds the tables' pinned memory there)
 
     def step(self, entries: Sequence[Tuple[Hashable, Sequence[int], Sequence[int]]],
              end: Sequence[Hashable] = ()) -> Optional[torch.Tensor]:
@@ -93,9 +94,11 @@ class BatchEngine:
             model.grow_slots(max(self.pool.size, 2 * model.slots))
         out = None
         if table:
-            x = model.forward_step(StepBatch.build(table, self.device))
+            # (the wanted rows go along with the table: a copy after the layers would hold the host until they are through)
+            step = StepBatch.build(table, self.device, rows)
+            x = model.forward_step(step)
             if rows:
-                out = model.logits(x, torch.tensor(rows, dtype=torch.int32).to(self.device))
+                out = model.logits(x, step.rows)
         for req in end:
             slot, _ = self.live.pop(req)
             self.pool.give(slot)

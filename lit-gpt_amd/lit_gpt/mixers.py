@@ -48,10 +48,12 @@ class StepBatch:
     # every sequence starts at position 0 in this step (host side, of the positions as they were when the table was made;
     # False: it may not). Not looked at while a step is captured
     fresh: bool = False
+    rows: Optional[torch.Tensor] = None  # rows of the step whose logits the caller wants, where it said so beforehand
 
     @classmethod
-    def build(cls, entries: Sequence[Tuple[int, int, Sequence[int]]], device: torch.device) -> "StepBatch":
-        """entries: (slot, first position, token ids) per sequence; one host -> device copy for the whole table."""
+    def build(cls, entries: Sequence[Tuple[int, int, Sequence[int]]], device: torch.device,
+              rows: Sequence[int] = ()) -> "StepBatch":
+        """entries: (slot, first position, token ids) per sequence; one host -> device copy for the whole table and ``rows``."""
         if any(isinstance(toks, np.ndarray) for _, _, toks in entries) and all(
                 len(toks) and (isinstance(toks, np.ndarray) or all(type(t) is int for t in toks)) for _, _, toks in entries):
             n = np.array([len(toks) for _, _, toks in entries])
@@ -59,9 +61,11 @@ class StepBatch:
             start = np.concatenate(([0], n.cumsum()))
             T, B = int(start[-1]), len(entries)
             pos = np.arange(T) + np.repeat(spos - start[:-1], n)
-            flat = np.concatenate([*(toks for _, _, toks in entries), np.repeat(sslot, n), pos, start, sslot, spos])
-            parts = torch.split(torch.from_numpy(flat.astype(np.int32)).to(device), [T, T, T, B + 1, B, B])
-            return cls(*parts, T=T, B=B, max_len=int(n.max()), fresh=not spos.any())
+            flat = np.concatenate([*(toks for _, _, toks in entries), np.repeat(sslot, n), pos, start, sslot, spos,
+                                   torch.tensor(rows, dtype=torch.int32).numpy()])
+            flat = _table(torch.from_numpy(flat.astype(np.int32)), device)
+            *parts, wanted = torch.split(flat, [T, T, T, B + 1, B, B, len(rows)])
+            return cls(*parts, T=T, B=B, max_len=int(n.max()), fresh=not spos.any(), rows=wanted if len(rows) else None)
         tokens, slot, pos, start, sslot, spos = [], [], [], [0], [], []
         for s, p0, toks in entries:
             n = len(toks)
@@ -74,10 +78,21 @@ class StepBatch:
             sslot.append(s)
             spos.append(p0)
         T, B = len(tokens), len(entries)
-        flat = torch.tensor(tokens + slot + pos + start + sslot + spos, dtype=torch.int32).to(device)
-        cut = [T, T, T, B + 1, B, B]
-        parts = torch.split(flat, cut)
-        return cls(*parts, T=T, B=B, max_len=max(len(e[2]) for e in entries), fresh=all(p0 == 0 for _, p0, _ in entries))
+        flat = _table(torch.tensor(tokens + slot + pos + start + sslot + spos + list(rows), dtype=torch.int32), device)
+        *parts, wanted = torch.split(flat, [T, T, T, B + 1, B, B, len(rows)])
+        return cls(*parts, T=T, B=B, max_len=max(len(e[2]) for e in entries), fresh=all(p0 == 0 for _, p0, _ in entries),
+                   rows=wanted if len(rows) else None)
+
+
+def _table(host: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """``host`` (int32) on ``device``: by way of pinned memory of its own, so that the copy takes its place in the stream instead of
+    waiting until the stream is empty. While a stream is captured, whose replays would read that memory again, as an ordinary
+    copy (which a capture refuses)."""
+    if torch.device(device).type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return host.to(device)
+    # (a new size of pinned memory costs 75 to 400 us once: all tables of some 1300 tokens share one)
+    pinned = torch.empty(max(host.numel(), 4096), dtype=torch.int32, pin_memory=True)[:host.numel()]
+    return pinned.copy_(host).to(device, non_blocking=True)
 
 
 def _f32(t: torch.Tensor, device) -> torch.Tensor:
