@@ -42,6 +42,10 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 }
 __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
 
+// Until no load of this wave is in flight, in a form that hipcc counts. Ahead of stores that stand under conditions of their own: where
+// a value may still be on its way for all that hipcc knows, it waits for everything before each of them, the store before it included.
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
 // ---- wave-level reductions (64 lanes) ----
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -152,6 +152,7 @@ __global__ void __launch_bounds__(256) ssm_scan_kernel(ScanArgs p) {
     }
     // (the next batch's writes to `part` come after its first barrier, which wave 0 reaches after these reads)
   }
+  lga::wait_loads();  // (or every store waits for the one before)
   if (live) {
 #pragma unroll
     for (int i = 0; i < NR; ++i)
@@ -173,8 +174,9 @@ __global__ void __launch_bounds__(256) ssm_scan_kernel(ScanArgs p) {
 // Of a head only x and the state are staged in LDS, loaded into registers while the head before it is worked on; two
 // workgroups fit a compute unit. Four rows of the inner index at a time are one instruction: lane group q takes rows
 // 16 t + 4 q + e, so that first operands are read 16 bytes at a time. N <= 128.
-// Bound by memory and the fp32 matrix instruction in about equal parts: 2407 tokens of 128 heads of 128 x 64 take 100 us
-// and 210 us, their bytes 50 and 70 (with one head a workgroup, and B, C and four copies of the state's loads, 286 and 717).
+// Bound by memory and the fp32 matrix instruction in about equal parts: 2407 tokens of 128 heads of 128 x 64 take 97 us
+// and 181 us, their bytes 50 and 70 (with one head a workgroup, and B, C and four copies of the state's loads, 286 and 717; D waited for
+// where it is used, and with it every store for the one before, 202).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kSC = 64;
 constexpr int kXS = 68;      // LDS row of x, state and scores: rows 4 apart fall 16 banks apart
@@ -203,6 +205,14 @@ __device__ __forceinline__ float4 ssd_load4(const float* at, int left) {
 }
 __device__ __forceinline__ f32x4_t ssd_mma(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// four rows' values at `at`, of 16 columns each: read for the instructions of the next four rows while those of these run (2407 tokens of
+// 128 heads of 128 x 64: read as they are used, every two instructions wait for LDS first, 189 us; 181 here)
+__device__ __forceinline__ void ssd_read(float (&v)[16], const float* at) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[e * 4 + c] = at[e * kXS + c * 16];
 }
 // lane i's step size d and running sum of log a up to token i, from the raw step size (0 from token n on)
 __device__ __forceinline__ float ssd_decay(const SsdArgs& p, int h, int lane, int n, float raw, float* d) {
@@ -321,7 +331,7 @@ __global__ void __launch_bounds__(256, 2) ssd_out_kernel(SsdArgs p) {
     *(float4*)(Ss + row * kBS + k) = ssd_load4<VEC>(bc + (size_t)min(row, n - 1) * p.ldx + min(k, N - 1), row < n ? N - k : 0);
   }
   float4 xr[4], sr[kTiles];
-  float raw = 0.0f;
+  float raw = 0.0f, Dn = 0.0f;
   auto fetch = [&](int h) {
     const int c = (tid & 15) * 4;
 #pragma unroll
@@ -337,27 +347,29 @@ __global__ void __launch_bounds__(256, 2) ssd_out_kernel(SsdArgs p) {
                              row < N ? dv - col0 - c : 0);
     }
     raw = p.dt[(size_t)(tc + min(lane, n - 1)) * p.ldd + h];
+    Dn = p.D[h];
   };
   fetch(h0);
   __syncthreads();
   f32x4_t cb[4];  // C_i . B_j of this wave's rows, j in piece tj <= ti
 #pragma unroll
-  for (int tj = 0; tj < 4; ++tj) {
-    cb[tj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if (tj > ti) continue;
+  for (int tj = 0; tj < 4; ++tj) cb[tj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      if (t >= tiles) continue;
-      const float4 k4 = *(const float4*)(Ss + (tj * 16 + fr) * kBS + 16 * t + 4 * fk);
-      cb[tj] = ssd_mma(ca[t].x, k4.x, cb[tj]);
-      cb[tj] = ssd_mma(ca[t].y, k4.y, cb[tj]);
-      cb[tj] = ssd_mma(ca[t].z, k4.z, cb[tj]);
-      cb[tj] = ssd_mma(ca[t].w, k4.w, cb[tj]);
-    }
+  for (int t = 0; t < kTiles; ++t) {
+    if (t >= tiles) continue;
+    float4 k4[4];
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj) k4[tj] = *(const float4*)(Ss + (tj * 16 + fr) * kBS + 16 * t + 4 * fk);
+    const float av[4] = {ca[t].x, ca[t].y, ca[t].z, ca[t].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj)
+        if (tj <= ti) cb[tj] = ssd_mma(av[e], e == 0 ? k4[tj].x : (e == 1 ? k4[tj].y : (e == 2 ? k4[tj].z : k4[tj].w)), cb[tj]);
   }
   for (int h = h0; h < h0 + p.hpw; ++h) {
     float d;
-    const float l = ssd_decay(p, h, lane, n, raw, &d);
+    const float l = ssd_decay(p, h, lane, n, raw, &d), Dh = Dn;
     la[wave][lane] = l, dts[wave][lane] = d;
     __syncthreads();  // the head before is done with Xs and Ss (the first: the scores with B)
 #pragma unroll
@@ -382,24 +394,40 @@ __global__ void __launch_bounds__(256, 2) ssd_out_kernel(SsdArgs p) {
     f32x4_t o[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) o[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    auto mul = [&](float4 a, const float* at) {  // += a . four rows
+    auto mul = [&](float4 a, const float (&v)[16]) {  // += a . four rows
       const float av[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) o[c] = ssd_mma(av[e], at[e * kXS + c * 16 + fr], o[c]);
+        for (int c = 0; c < 4; ++c) o[c] = ssd_mma(av[e], v[e * 4 + c], o[c]);
     };
+    // (rows past the last are read all the same, in bounds, and not used: a read under a condition cannot be counted)
+    float v[2][16];
+    float4 ga[4];
+    ssd_read(v[0], Ss + 4 * fk * kXS + fr);
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t)
-      if (t < tiles) mul(ca[t], Ss + (16 * t + 4 * fk) * kXS);
+    for (int t = 0; t < kTiles; ++t) {
+      if (t + 1 < kTiles) ssd_read(v[(t + 1) & 1], Ss + (16 * (t + 1) + 4 * fk) * kXS + fr);
+      else ssd_read(v[0], Xs + 4 * fk * kXS + fr);
+      if (t == kTiles - 1)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ga[u] = *(const float4*)(Gs + (ti * 16 + fr) * kXS + 16 * u + 4 * fk);
+      __builtin_amdgcn_sched_barrier(0);
+      if (t < tiles) mul(ca[t], v[t & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    static_assert(kTiles % 2 == 0, "x follows in v[0]");
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[c][r] *= expf(li[r]);
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-      if (t <= ti) mul(*(const float4*)(Gs + (ti * 16 + fr) * kXS + 16 * t + 4 * fk), Xs + (16 * t + 4 * fk) * kXS);
-    const float Dh = p.D[h];
+    for (int t = 0; t < 4; ++t) {
+      if (t < 3) ssd_read(v[(t + 1) & 1], Xs + (16 * (t + 1) + 4 * fk) * kXS + fr);
+      __builtin_amdgcn_sched_barrier(0);
+      if (t <= ti) mul(ga[t], v[t & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
