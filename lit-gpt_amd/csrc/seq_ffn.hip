@@ -328,6 +328,101 @@ __global__ void __launch_bounds__(256) moe_down_kernel(const float* __restrict__
   }
 }
 
+// dot2 of one pair of weight rows with N tokens' rows at once: the sums of dot2 (its 16-byte form) for each, to the bit
+template <bool WF32, int N>
+__device__ __forceinline__ void dot2_tokens(const float* const (&x)[N], const void* __restrict__ w, size_t r0, size_t r1, int n, int lane,
+                                            float (&a)[N][2]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) a[j][0] = a[j][1] = 0.0f;
+#pragma unroll 2
+  for (int k = lane * 8; k < n; k += 512) {
+    float u[8], v[8];
+    wload8<WF32>(w, r0 + k, u);
+    wload8<WF32>(w, r1 + k, v);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float4 xa = *(const float4*)(x[j] + k), xb = *(const float4*)(x[j] + k + 4);
+      const float xs[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float xe = aop<WF32>(xs[e]);
+        a[j][0] = fmaf(xe, u[e], a[j][0]);
+        a[j][1] = fmaf(xe, v[e], a[j][1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) a[j][0] = wave_sum(a[j][0]), a[j][1] = wave_sum(a[j][1]);
+}
+// the pairs of `mask` up to four at a time; row(pair): its row, put(pair, a0, a1)
+template <bool WF32, class Row, class Put>
+__device__ __forceinline__ void dot2_pairs(uint64_t mask, const void* __restrict__ w, size_t r0, size_t r1, int n, int lane, Row&& row, Put&& put) {
+  auto some = [&](auto count) {
+    constexpr int N = decltype(count)::value;
+    int pair[N];
+    const float* x[N];
+    float a[N][2];
+#pragma unroll
+    for (int j = 0; j < N; ++j) pair[j] = __builtin_ctzll(mask), mask &= mask - 1, x[j] = row(pair[j]);
+    dot2_tokens<WF32, N>(x, w, r0, r1, n, lane, a);
+#pragma unroll
+    for (int j = 0; j < N; ++j) put(pair[j], a[j][0], a[j][1]);
+  };
+  while (mask) {
+    const int left = __builtin_popcountll(mask);
+    if (left >= 4) some(std::integral_constant<int, 4>{});
+    else if (left == 3) some(std::integral_constant<int, 3>{});
+    else if (left == 2) some(std::integral_constant<int, 2>{});
+    else some(std::integral_constant<int, 1>{});
+  }
+}
+
+// moe_up_kernel for several tokens, up to 64 pairs and 16-byte rows: the workgroups of an expert's first pair make the products of
+// all of its pairs, so that a weight is read once however many tokens chose its expert (once a pair it came from L2 or the last cache
+// in turn). Bound by memory. LANES: a lane looks at one pair each, 2 to 3 us ahead of the weights; otherwise the scalar unit does, some
+// four instructions a pair. us, a pair at a time / by scalars / by lanes, 16 experts of 2 x 1408 x 2048: 2 tokens of 4 choices 14.6 / 14.8 / 17.4, 5
+// 35.1 / 35.0 / 36.9, 8 45.6 / 43.4 / 37.8; of 2 x 2752 x 4096: 2 58 / 55 / 66, 3 91 / 75 / 79, 5 134 / 102 / 109, 8 215 / 143 / 138, 16 427 / 283 /
+// 209; 64 of 2 x 512 x 1024 (not taken): 3 7.0 / 8.3 / 7.2, 8 12.2 / 16.6 / 12.7. The eight-wave form of moe_down_kernel that does the same
+// lost: 8 tokens of 2048 x 1408 23.6 / 32.1, of 4096 x 2752 108 / 156.
+template <bool WF32, bool GATED, bool LANES>
+__global__ void __launch_bounds__(256) moe_up_shared_kernel(const float* __restrict__ h, long ldh, const void* __restrict__ up,
+                                                            const int* __restrict__ ids, float* __restrict__ actbuf, int pairs, int top,
+                                                            int F, int K, int act, int n_real) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int f0 = (blockIdx.x * 4 + wave) * (GATED ? 1 : 2);
+  if (f0 >= F) return;
+  const int own = blockIdx.y, e = ids[own];
+  uint64_t mask = 0;
+  if (LANES) {
+    mask = __ballot(lane < pairs && ids[min(lane, pairs - 1)] == e);
+  } else {
+    int p = 0;
+    for (; p + 8 <= pairs; p += 8)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mask |= (uint64_t)(ids[p + j] == e) << (p + j);
+    for (; p < pairs; ++p) mask |= (uint64_t)(ids[p] == e) << p;
+  }
+  if (e >= n_real || __builtin_ctzll(mask) != own) return;
+  const size_t rows = GATED ? 2 * (size_t)F : (size_t)F;
+  const size_t w0 = ((size_t)e * rows + f0) * K, w1 = ((size_t)e * rows + (GATED ? F + f0 : min(f0 + 1, F - 1))) * K;
+  dot2_pairs<WF32>(mask, up, w0, w1, K, lane, [&](int p) { return h + (size_t)(p / top) * ldh; }, [&](int p, float a0, float a1) {
+    if (lane != 0) return;
+    float* out = actbuf + (size_t)p * F + f0;
+    if (GATED) {
+      *out = act_f(act, a0) * a1;
+    } else {
+      out[0] = act_f(act, a0);
+      if (f0 + 1 < F) out[1] = act_f(act, a1);
+    }
+  });
+}
+
+// Several tokens, an expert of 8 MB and more (below, the look at the pairs costs what the second reading does) and few enough experts that
+// tokens share some
+static bool moe_up_shares(int T, int top, long bytes, int n_real) {
+  return T > 1 && T * top <= 64 && bytes >= 8 << 20 && n_real <= 4 * T * top;
+}
+
 // Counting sort of the pairs by expert in three launches. ws: 2 E ints (counts, cursors), zero on entry.
 // z_start[E + 1] expert ranges in the sorted list, tok_of[i] the token (row of h) of sorted entry i, where[pair] the
 // sorted place of a pair. The order inside an expert's range is whatever the atomics give: every row of the grouped
@@ -581,6 +676,19 @@ extern "C" int lgs_moe_up(const float* h, long ldh, const void* up, int w_f32, c
                           int top, int F, int K, int act, int gated, int n_real, hipStream_t stream) {
   LGA_CHECK_ARG(h && up && ids && actbuf && T > 0 && top > 0 && F > 0 && K > 0 && (long)T * top <= 65535 && n_real > 0,
                 "lgs_moe_up: bad arguments");
+  if (lgs::moe_up_shares(T, top, (long)(gated ? 2 : 1) * F * K * (w_f32 ? 4 : 2), n_real) && K % 8 == 0 && ldh % 4 == 0 && (uintptr_t)h % 16 == 0) {
+    const dim3 grid(gated ? (F + 3) / 4 : (F + 7) / 8, T * top);
+    auto go = [&](auto f32, auto glu) {
+      constexpr bool W = decltype(f32)::value, G = decltype(glu)::value;
+      if (T * top > 24) lgs::moe_up_shared_kernel<W, G, true><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, T * top, top, F, K, act, n_real);
+      else lgs::moe_up_shared_kernel<W, G, false><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, T * top, top, F, K, act, n_real);
+    };
+    if (w_f32 && gated) go(std::true_type{}, std::true_type{});
+    else if (w_f32) go(std::true_type{}, std::false_type{});
+    else if (gated) go(std::false_type{}, std::true_type{});
+    else go(std::false_type{}, std::false_type{});
+    LGA_LAUNCH_RETURN();
+  }
   if (gated) {
     const dim3 grid((F + 3) / 4, T * top);
     if (w_f32) lgs::moe_up_kernel<true, true><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, top, F, K, act, n_real);

@@ -1,0 +1,37 @@
+"""Experts of steps with few tokens: several tokens at once give the bits that each token has alone (csrc/seq_ffn.hip:
+moe_up_shared_kernel), at one to all choices of an expert, identity experts, odd sizes, and on both sides of 24 pairs, of 64, of 8 MB
+an expert and of four experts a pair."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("T,top,E,real", [(2, 1, 3, 3), (3, 4, 5, 4), (6, 4, 7, 6), (7, 4, 9, 7), (16, 4, 6, 6), (64, 1, 4, 3), (13, 5, 7, 6),
+                                          (2, 2, 18, 16), (2, 2, 19, 17)])
+@pytest.mark.parametrize("W,F", [(1032, 2045), (1032, 4100), (16, 8), (1031, 2047)])
+def test_tokens_together(dtype, gated, T, top, E, real, W, F):
+    from lit_gpt import seq_ops
+
+    g = torch.Generator(device=DEV).manual_seed(T * E + W)
+    up = (torch.randn(real, (2 if gated else 1) * F, W, generator=g, device=DEV) * W ** -0.5).to(dtype)
+    down = (torch.randn(real, W, F, generator=g, device=DEV) * F ** -0.5).to(dtype)
+    h, x0 = (torch.randn(T, W, generator=g, device=DEV) for _ in range(2))
+    ids = torch.stack([torch.randperm(E, generator=g, device=DEV)[:top] for _ in range(T)]).to(torch.int32)
+    ids[T // 2:] = ids[0]  # (half the tokens choose alike)
+    wts = torch.rand(T, top, generator=g, device=DEV)
+    one = lambda t, i: t[i: i + 1].contiguous()  # noqa: E731
+    for accumulate in (True, False):
+        x = x0.clone()
+        a = seq_ops.moe_up(h, up, ids, seq_ops.ACT_SILU, gated=gated)
+        seq_ops.moe_down(a, down, ids, wts, x, h, accumulate=accumulate)
+        for t in range(T):
+            at = seq_ops.moe_up(one(h, t), up, one(ids, t), seq_ops.ACT_SILU, gated=gated)
+            xt = one(x0, t).clone()
+            seq_ops.moe_down(at, down, one(ids, t), one(wts, t), xt, one(h, t), accumulate=accumulate)
+            live = (ids[t] < real).nonzero().flatten()  # (an identity expert's row is nobody's)
+            assert torch.equal(a.view(T, top, F)[t, live], at.view(top, F)[live]) and torch.equal(x[t], xt[0])
