@@ -382,8 +382,9 @@ __device__ __forceinline__ void dot2_pairs(uint64_t mask, const void* __restrict
 // in turn). Bound by memory. LANES: a lane looks at one pair each, 2 to 3 us ahead of the weights; otherwise the scalar unit does, some
 // four instructions a pair. us, a pair at a time / by scalars / by lanes, 16 experts of 2 x 1408 x 2048: 2 tokens of 4 choices 14.6 / 14.8 / 17.4, 5
 // 35.1 / 35.0 / 36.9, 8 45.6 / 43.4 / 37.8; of 2 x 2752 x 4096: 2 58 / 55 / 66, 3 91 / 75 / 79, 5 134 / 102 / 109, 8 215 / 143 / 138, 16 427 / 283 /
-// 209; 64 of 2 x 512 x 1024 (not taken): 3 7.0 / 8.3 / 7.2, 8 12.2 / 16.6 / 12.7. The eight-wave form of moe_down_kernel that does the same
-// lost: 8 tokens of 2048 x 1408 23.6 / 32.1, of 4096 x 2752 108 / 156.
+// 209; 64 of 2 x 512 x 1024 (not taken): 3 7.0 / 8.3 / 7.2, 8 12.2 / 16.6 / 12.7. Forms of moe_down_kernel
+// that do the same, a workgroup's eight waves on as many experts' rows of two columns, lost: 8 tokens of 2048 x 1408 23.6 / 30.9, of 4096 x
+// 2752 108 / 151, 2 tokens 34 / 52.
 template <bool WF32, bool GATED, bool LANES>
 __global__ void __launch_bounds__(256) moe_up_shared_kernel(const float* __restrict__ h, long ldh, const void* __restrict__ up,
                                                             const int* __restrict__ ids, float* __restrict__ actbuf, int pairs, int top,
