@@ -30,12 +30,13 @@ static __constant__ float kCode4[2][16] = {
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 __device__ __forceinline__ float bflo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bfhi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
-// fp32 -> bf16 round-to-nearest-even in hardware (v_cvt_pk_bf16_f32: one instruction per PAIR, NaN stays NaN);
-// hipcc has no builtin that emits the packed form for two independent values, hence the asm.
+// fp32 -> bf16 round-to-nearest-even in hardware (v_cvt_pk_bf16_f32: one instruction per PAIR, NaN stays NaN), by way of a vector that
+// hipcc converts as one. Not in asm: hipcc keeps two wait states between an instruction that writes a matrix instruction's operand and
+// that one, but not of an asm block, and the operand was then read as it was before.
+typedef float lga_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 lga_bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  uint32_t r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
-  return r;
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((lga_f32x2{lo, hi}), lga_bf16x2));
 }
 __device__ __forceinline__ uint16_t f2bf(float f) {
   return __builtin_bit_cast(unsigned short, static_cast<__bf16>(f));
