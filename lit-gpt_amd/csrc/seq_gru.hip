@@ -7,7 +7,7 @@
 //                     chunk is S -> A S + L with A the product of its 1 - z and L its result from a zero start)
 //   lgs_mingru_step   steps of one token per sequence and few sequences: the three projections of a channel and its
 //                     step in one launch, a wave per channel
-#include "seq_common.h"
+#include "seq_rows.h"
 
 namespace lgs {
 
@@ -183,6 +183,47 @@ __global__ void __launch_bounds__(256) mingru_step_kernel(MinGruStepArgs p) {
   p.out[(size_t)lane * p.n + c] = S * (v[2] * sigmoid_f(v[2]));
 }
 
+// mingru_step_kernel for several sequences and bf16 weights, on the matrix cores (seq_rows.h): a workgroup makes the three projections of 16
+// channels, and a lane finishes four of one sequence. Bound by memory. us, a wave a channel / here: 3 sequences of 4096 channels of 4096 values
+// 27.7 / 19.6, 8 44.1 / 19.8, 8 of 2048 of 2048 20.0 / 11.6, 2 of 8192 of 2048 25.0 / 20.0 (one: 20.6 there).
+template <int KW, int MR, int RB>
+__global__ void __launch_bounds__(KW * 64) mingru_rows_kernel(MinGruStepArgs p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[RowsTile<3, KW, MR, RB>::LDS];
+  const int lane = threadIdx.x & 63, m = lane & 15, c0 = blockIdx.x * 16, c = c0 + (lane >> 4) * 4;
+  const bool fin = threadIdx.x < 64 && m < p.M && c < p.n;
+  const int slot = fin ? p.seq_slot[m] : 0;
+  const bool old = fin && p.seq_pos0[m] > 0;
+  float S0[4], bias[3][4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {  // (channels past the end: the last one's, not used)
+    const int at = min(c + r, p.n - 1);
+    S0[r] = old ? p.state[(size_t)slot * p.n + at] : 0.0f;
+    bias[0][r] = p.bias && fin ? p.bias[p.z0 + at] : 0.0f;
+    bias[1][r] = p.bias && fin ? p.bias[p.u0 + at] : 0.0f;
+    bias[2][r] = p.bias && fin ? p.bias[p.g0 + at] : 0.0f;
+  }
+  const uint16_t* w = (const uint16_t*)p.w;
+  rows_products<3, KW, MR, RB>(lds, [&](int r) {
+    return w + (size_t)((r < 16 ? p.z0 : (r < 32 ? p.u0 : p.g0)) + min(c0 + (r & 15), p.n - 1)) * p.K;
+  }, p.h, p.ldh, p.M, p.K);
+  if (!fin) return;
+  rows_f32x4 v[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) v[j] = rows_sum<3, KW>(lds, j, lane);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (c + r >= p.n) break;
+    float keep;
+    const float S = mingru_next(v[0][r] + bias[0][r], v[1][r] + bias[1][r], S0[r], keep), g = v[2][r] + bias[2][r];
+    p.state[(size_t)slot * p.n + c + r] = S;
+    p.out[(size_t)m * p.n + c + r] = S * (g * sigmoid_f(g));
+  }
+}
+
+// Five sequences and more always, three and four of long rows, two of many channels. us, a wave a channel / matrix cores: 4 of 256 channels of
+// 256 values 5.0 / 5.4, 3 of 1024 of 1024 6.8 / 6.6; 2 of 2048 of 2048 10.4 / 10.9, of 3072 of 2048 13.0 / 11.1, of 5120 of 5120 33.2 / 35.9
+static bool mingru_rows_pay(int M, int K, int n) { return M > 4 || (M > 2 && K >= 1024) || (M == 2 && n > 2048 && K <= 4096); }
+
 }  // namespace lgs
 
 extern "C" int lgs_mingru(const float* z, const float* u, const float* g, long ld, float* state, const int* seq_start,
@@ -212,6 +253,20 @@ extern "C" int lgs_mingru_step(const float* h, long ldh, const void* w, int w_f3
   LGA_CHECK_ARG(z0 >= 0 && u0 >= 0 && g0 >= 0 && (long)z0 + n <= rows && (long)u0 + n <= rows && (long)g0 + n <= rows,
                 "lgs_mingru_step: projections outside the matrix");
   lgs::MinGruStepArgs p{h, ldh, w, bias, z0, u0, g0, M, K, n, state, seq_slot, seq_pos0, out};
+  if (!w_f32 && lgs::mingru_rows_pay(M, K, n) && K % 128 == 0 && ldh % 4 == 0 && ((uintptr_t)h | (uintptr_t)w) % 16 == 0) {
+    const unsigned blocks = (n + 15) / 16;
+    // (a workgroup a compute unit or fewer: eight waves, or two blocks of each of four)
+#define LGS_GRU_ROWS(MR)                                                                            \
+  do {                                                                                              \
+    if (blocks <= 128) lgs::mingru_rows_kernel<8, MR, 1><<<blocks, 512, 0, stream>>>(p);            \
+    else if (blocks <= 256) lgs::mingru_rows_kernel<4, MR, 2><<<blocks, 256, 0, stream>>>(p);       \
+    else lgs::mingru_rows_kernel<4, MR, 1><<<blocks, 256, 0, stream>>>(p);                          \
+  } while (0)
+    if (M > 4) LGS_GRU_ROWS(8);
+    else LGS_GRU_ROWS(4);
+#undef LGS_GRU_ROWS
+    LGA_LAUNCH_RETURN();
+  }
   const unsigned grid = (n + 3) / 4;
 #define LGS_GRU(MT)                                                               \
   do {                                                                            \

@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "seq_gemm.h"
+#include "seq_rows.h"
 
 namespace lgs {
 
@@ -188,108 +189,17 @@ __global__ void __launch_bounds__(256) lin_glu_row_kernel(const float* __restric
   if (lane == 0) y[col] = glu_f<CLAMPED>(f, g, u);
 }
 
-// Up to eight rows of A on bf16 weights, on the matrix cores: the operands are the same (A rounded to bf16), and a weight
-// costs no vector instruction however many rows there are. A workgroup owns 16 NR columns; its KW waves each take a
-// range of K, 128 values at a time: the columns' 256 bytes of W and the MR rows' 512 of A come by LDS-DMA (whole lines,
-// source-swizzled so that fragments are read without bank conflicts) into LDS of the wave's own, so that no barrier is theirs, and are
-// fetched anew as soon as they are in registers. One block's buffers a wave where several workgroups share a compute unit: they hide its
-// trips better than blocks ahead do (us with one / two blocks' buffers: 8 x 32000 x 2048 30.2 / 32.8, x 8192 x 2048 9.4 / 10.2, x 8192 x 4096
-// 15.2 / 16.6, 3 x 6144 x 4096 12.6 / 13.5); two where a workgroup of four waves has one alone (8 x 4096 x 4096 11.3 / 9.3, 3 rows 10.0 / 8.7,
-// 11264 long 23.2 / 18.1, 8 x 6144 x 4096 14.7 / 13.4, 8 x 4096 x 2048 7.2 / 6.6; three are no faster, eight waves' 128 KB slower: 8 x 2048 x
-// 2048 5.9 / 6.6). The rows are read as vectors of the compiler's own: a read of HIP's float4 may alias the DMAs for it, and waits for all.
-// Sums: two instructions, then vector adds, then the ranges pairwise, so that the error against float64 is what the
-// lanes' sums of lin_gemv_kernel leave (rms of 8 rows at K 2048 / 4096 / 11008: 7.4e-8 / 8.0e-8 / 9.5e-8 of the results,
-// 7.5e-8 / 8.4e-8 / 1.1e-7 there; one chain of instructions 1.5 to 3 times as much).
-// Bound by memory, with few columns by its latency. Loaded into registers as the instructions take them, every lane's 16 bytes lay
-// in a line of their own, and a compute unit got some 17 bytes a ns of W and A together, from whichever cache. us there / here, weights
-// from memory, the same bits: 8 x 2048 x 2048 11.9 / 5.9, x 4096 x 2048 10.1 / 6.6, x 6288 x 2048 14.2 / 9.0, x 32000 x 2048 44.5 / 30.2, x
-// 4096 x 4096 14.4 / 9.3, x 12288 x 4096 35.2 / 23.4, 3 x 12288 x 4096 30.5 / 20.6, x 32000 x 4096 59 / 48.
+// seq_rows.h's products, finished here
 template <int NR, int KW, int MR, int RB>
 __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
-  constexpr int W_BYTES = NR * 4096, A_BYTES = MR * 512, SLOT = W_BYTES + A_BYTES, PW = NR * 4, PA = MR / 2;
-  static_assert(KW * RB * SLOT <= 163840 && NR * 1024 <= SLOT, "LDS");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_all[KW * RB * SLOT];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[RowsTile<NR, KW, MR, RB>::LDS];
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, q4 = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  unsigned char* lds = lds_all + wave * (RB * SLOT);
   const int z = blockIdx.y, n0 = blockIdx.x * (16 * NR);
-  const int nb = p.K / 128, b0 = wave * nb / KW, b1 = (wave + 1) * nb / KW;
-  const unsigned char *w[PW], *a[PA];
-#pragma unroll
-  for (int i = 0; i < PW; ++i) {  // four rows of 256 bytes
-    const int row = i * 4 + q4;
-    w[i] = (const unsigned char*)((const uint16_t*)p.w + (size_t)z * p.sw + (size_t)min(n0 + row, p.N - 1) * p.K) + 16 * (l15 ^ (row & 15));
-  }
-#pragma unroll
-  for (int i = 0; i < PA; ++i) {  // two rows of 512
-    const int row = i * 2 + (lane >> 5);
-    a[i] = (const unsigned char*)(p.a + (size_t)z * p.sa + (size_t)min(row, p.M - 1) * p.lda) + 16 * ((lane & 31) ^ row);
-  }
-  auto dma = [&](int b, int slot) {  // (past the range: its last block, never used)
-    const size_t at = (size_t)max(min(b, b1 - 1), 0) * 256;
-#pragma unroll
-    for (int i = 0; i < PW; ++i) lga::gemm_dma16(w[i] + at, lds + slot + i * 1024);
-#pragma unroll
-    for (int i = 0; i < PA; ++i) lga::gemm_dma16(a[i] + 2 * at, lds + slot + W_BYTES + i * 1024);
-  };
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4_t acc[4][NR];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < NR; ++j) acc[i][j] = zero;
-#pragma unroll
-  for (int r = 0; r < RB; ++r) dma(b0 + r, r * SLOT);
-  int slot = 0;
-  const int arow = l15 & (MR - 1), w_at = l15 * 256, a_at = W_BYTES + arow * 512;
-  for (int b = b0; b < b1; b += 2) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if (b + s < b1) {
-        lga::gemm_wait_vm<(RB - 1) * (PW + PA)>();
-        bf16x8_t wr[4][NR];
-        f32x4_t x[4][2];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-#pragma unroll
-          for (int j = 0; j < NR; ++j) wr[m][j] = *(const bf16x8_t*)(lds + slot + w_at + j * 4096 + 16 * ((m * 4 + q4) ^ l15));
-#pragma unroll
-          for (int e = 0; e < 2; ++e) x[m][e] = *(const f32x4_t*)(lds + slot + a_at + 16 * ((m * 8 + q4 * 2 + e) ^ arow));
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before it is filled again)
-        __builtin_amdgcn_sched_barrier(0);
-        dma(b + s + RB, slot);
-        slot = slot + SLOT == RB * SLOT ? 0 : slot + SLOT;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          f32x4_t v[NR];
-#pragma unroll
-          for (int m = 2 * u; m < 2 * u + 2; ++m) {
-            const uint4 x16 = make_uint4(pack2(x[m][0].x, x[m][0].y), pack2(x[m][0].z, x[m][0].w), pack2(x[m][1].x, x[m][1].y), pack2(x[m][1].z, x[m][1].w));
-#pragma unroll
-            for (int j = 0; j < NR; ++j)
-              v[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[m][j], __builtin_bit_cast(bf16x8_t, x16), m == 2 * u ? zero : v[j], 0, 0, 0);
-          }
-#pragma unroll
-          for (int j = 0; j < NR; ++j) acc[s * 2 + u][j] += v[j];
-        }
-      }
-    }
-  }
-  lga::gemm_wait_vm<0>();  // no DMA may outlive its slot
-  __syncthreads();
-  f32x4_t* part = (f32x4_t*)lds_all;  // [KW][NR][64]
-#pragma unroll
-  for (int j = 0; j < NR; ++j) part[(wave * NR + j) * 64 + lane] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
-  __syncthreads();
+  const uint16_t* w = (const uint16_t*)p.w + (size_t)z * p.sw;
+  rows_products<NR, KW, MR, RB>(lds, [&](int r) { return w + (size_t)min(n0 + r, p.N - 1) * p.K; }, p.a + (size_t)z * p.sa, p.lda, p.M, p.K);
   if (tid >= NR * 64 || l15 >= p.M) return;
-  const int j = NR > 1 ? wave : 0;
-  f32x4_t v = zero;
-#pragma unroll
-  for (int k = 0; k < KW; k += 4) {
-    const f32x4_t* at = part + (k * NR + j) * 64 + lane;
-    v += (at[0] + at[NR * 64]) + (at[2 * NR * 64] + at[3 * NR * 64]);
-  }
+  const int j = NR > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
+  const rows_f32x4 v = rows_sum<NR, KW>(lds, j, lane);
   float* y = p.y + (size_t)z * p.sy + (size_t)l15 * p.ldy;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
