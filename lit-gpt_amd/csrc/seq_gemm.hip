@@ -153,6 +153,9 @@ __device__ __forceinline__ void gemm_rows(const LinArgs& p, unsigned char* lds, 
   float bias[FN];
 #pragma unroll
   for (int j = 0; j < FN; ++j) bias[j] = p.bias ? p.bias[min(nw + l31 + j * 32, p.N - 1)] : 0.0f;
+  // (or, in tiles that rows or columns end in, every store waits for the one before. us: 1000 rows of 6288 x 2048 36.3 / 29.6, 1500
+  // 52.0 / 41.6, of 4096 x 4096 53.8 / 49.7, 2407 of 2048 x 2048 29.4 / 25.1)
+  lga::wait_loads();
   const long at = (long)z * p.sy + (long)(r_lo + mw) * p.ldy + nw;
   if (ACTS && p.act != kActNone) {
     if constexpr (ACTS) {
