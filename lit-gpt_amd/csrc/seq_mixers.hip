@@ -690,9 +690,13 @@ __global__ void __launch_bounds__(256) latent_attention_vec_kernel(LatAttArgs p,
 
 // The same for four heads a workgroup (H % 4 == 0): a cached row is loaded and unpacked once for four, and the four heads' scores
 // of a key end in one row of 16 lanes each, where their softmax takes one instruction for all. The next four keys are on their way
-// while these are worked on. Bound by latency. us of a head a workgroup, with a wave sum through LDS per key and head, / here: 3 tokens
-// of 32 heads over 1200, 731 and 64 rows of 512 + 64 28.8 / 18.3, one of 16 over 2048 18.0 / 16.1, five of 16 over 40 to 2000 46.9 /
-// 21.8, eight of 16 over five 10.5 / 8.6, one over five 9.3 / 10.8.
+// while these are worked on. Bound by latency, of which short caches are nothing else: a range without keys says so and leaves its row
+// alone, values of lanes past a row are zeros instead of branches around each product, and the waves' sums are read and stored four
+// columns a lane; with the combination's columns side by side none of 24 forms of 1 to 16 tokens of 4 to 64 heads is slower than a head
+// a workgroup. us of that, with a wave sum through LDS per key and head, / here with branches, stores of a column and every range
+// written / here, both launches, rows of 512 + 64 from caches: one token of 8 heads over one 8.4 / 10.6 / 7.5, over 64 8.6 / 10.8 /
+// 8.7, over 600 11.1 / 12.7 / 10.3, over 2000 21.5 / 16.1 / 13.8; of 16 over five 9.5 / 10.9 / 7.9, over 2000 23.2 / 16.9 / 14.8; of 64
+// over 64 12.4 / 10.3 / 8.8; eight of 16 over five 10.7 / 8.1 / 7.1, over 2000 65 / 32.8 / 30.9; 3 of 32 over 600 21.9 / 15.8 / 13.9.
 template <int CTRL>
 __device__ __forceinline__ float lat_dpp_add(float v) {
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
@@ -728,6 +732,13 @@ __global__ void __launch_bounds__(256) latent_attention_heads_kernel(LatAttArgs 
   const size_t base = (size_t)p.slot[t] * p.max_seq;
   const bool live = 8 * lane < r;
   const int at = live ? 8 * lane : 0, rot[2] = {min(lane, max(dr - 1, 0)), min(lane + 64, max(dr - 1, 0))};
+  if (lo > hi && splits > 1) {  // (no keys: a sum of zero, whose row the combination does not read)
+    if (lane == 0) {
+      float* o = part + (((size_t)t * p.H + h0 + wave) * splits + z) * (r + 2);
+      o[0] = -INFINITY, o[1] = 0.0f;
+    }
+    return;
+  }
   uint4 raw[U][CV];
   float kr[U][2];
   auto fetch = [&](int j0) {  // (past the end the last key again, without weight)
@@ -751,7 +762,10 @@ __global__ void __launch_bounds__(256) latent_attention_heads_kernel(LatAttArgs 
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[i][e] = live ? qv[e] : 0.0f, acc[i][e] = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 2; ++e) qrot[i][e] = lane + 64 * e < dr ? qr[lane + 64 * e] : 0.0f;
+    for (int e = 0; e < 2; ++e) {
+      const float v = dr > 0 ? qr[rot[e]] : 0.0f;
+      qrot[i][e] = lane + 64 * e < dr ? v : 0.0f;
+    }
   }
   float m = -INFINITY, l = 0.0f;  // row i of 16 lanes: head i's
   for (int j0 = lo + wave; j0 <= hi; j0 += 4 * U) {
@@ -767,20 +781,24 @@ __global__ void __launch_bounds__(256) latent_attention_heads_kernel(LatAttArgs 
         c[u][0] = bflo(w.x), c[u][1] = bfhi(w.x), c[u][2] = bflo(w.y), c[u][3] = bfhi(w.y);
         c[u][4] = bflo(w.z), c[u][5] = bfhi(w.z), c[u][6] = bflo(w.w), c[u][7] = bfhi(w.w);
       }
+      // (lanes past a row: zeros on both sides)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) c[u][e] = live ? c[u][e] : 0.0f;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) kr[u][e] = lane + 64 * e < dr ? kr[u][e] : 0.0f;
       float dot[HP];
 #pragma unroll
       for (int i = 0; i < HP; ++i) {
         dot[i] = 0.0f;
-        if (lane < dr) dot[i] = fmaf(qrot[i][0], kr[u][0], dot[i]);
-        if (lane + 64 < dr) dot[i] = fmaf(qrot[i][1], kr[u][1], dot[i]);
-        if (live)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) dot[i] = fmaf(q[i][e], c[u][e], dot[i]);
+        for (int e = 0; e < 2; ++e) dot[i] = fmaf(qrot[i][e], kr[u][e], dot[i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot[i] = fmaf(q[i][e], c[u][e], dot[i]);
       }
       s[u] = j0 + 4 * u <= hi ? lat_sum4(dot) * p.scale : -INFINITY;
       mn = fmaxf(mn, s[u]);
     }
-    fetch(j0 + 4 * U);
+    if (j0 + 4 * U <= hi) fetch(j0 + 4 * U);
     const float corr = expf(m - mn);
     m = mn;
     l *= corr;
@@ -825,10 +843,17 @@ __global__ void __launch_bounds__(256) latent_attention_heads_kernel(LatAttArgs 
   const size_t head = (size_t)t * p.H + h0 + wave;
   float* o = fin ? p.out + head * r : part + (head * splits + z) * (r + 2) + 2;
   if (!fin && lane == 0) o[-2] = mx, o[-1] = den;
-  const float* x = sacc + (size_t)wave * r;
-  for (int k = lane; k < r; k += 64) {
-    const float v = (x[k] * f[0] + x[(size_t)HP * r + k] * f[1]) + (x[(size_t)2 * HP * r + k] * f[2] + x[(size_t)3 * HP * r + k] * f[3]);
-    o[k] = fin ? v / den : v;
+  for (int k = 4 * lane; k < r; k += 256) {
+    float4 x[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) x[w] = *(const float4*)(sacc + ((size_t)w * HP + wave) * r + k);
+    const float v[4] = {(x[0].x * f[0] + x[1].x * f[1]) + (x[2].x * f[2] + x[3].x * f[3]),
+                        (x[0].y * f[0] + x[1].y * f[1]) + (x[2].y * f[2] + x[3].y * f[3]),
+                        (x[0].z * f[0] + x[1].z * f[1]) + (x[2].z * f[2] + x[3].z * f[3]),
+                        (x[0].w * f[0] + x[1].w * f[1]) + (x[2].w * f[2] + x[3].w * f[3])};
+#pragma unroll
+    for (int e = 0; e < 4; e += 2)  // (a range's row starts on eight bytes)
+      *(float2*)(o + k + e) = fin ? make_float2(v[e] / den, v[e + 1] / den) : make_float2(v[e], v[e + 1]);
   }
 }
 
@@ -1017,7 +1042,8 @@ __global__ void __launch_bounds__(256) latent_attention_tile_kernel(LatTileArgs 
   }
 }
 
-// grid (T, H): merges the splits' partial softmaxes and the sink
+// grid (T, H, ceil(r / 256)): merges the splits' partial softmaxes and the sink, a column a thread (two one after the other, whose
+// rows are fetched eight at a time: 1.1 us more for 32 splits of 512 columns)
 __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __restrict__ part, const float* __restrict__ sink,
                                                              float* __restrict__ out, int H, int r, int splits) {
   const int t = blockIdx.x, h = blockIdx.y;
@@ -1035,15 +1061,15 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
   const float f = lz > 0.0f ? expf(mz - mx) : 0.0f;
   wz[z0] = f;
   const float den = block_sum_256(lz * f, red) + (sink ? expf(snk - mx) : 0.0f);
-  for (int i = threadIdx.x; i < r; i += 256) {
-    float a = 0.0f;
+  const int i = threadIdx.x + 256 * blockIdx.z;
+  if (i >= r) return;
+  float a = 0.0f;
 #pragma unroll 8
-    for (int z = 0; z < splits; ++z) {
-      const float v = pp[(size_t)z * (r + 2) + 2 + i];
-      a = fmaf(wz[z], wz[z] > 0.0f ? v : 0.0f, a);  // (an empty split's row is not written)
-    }
-    out[((size_t)t * H + h) * r + i] = a / den;
+  for (int z = 0; z < splits; ++z) {
+    const float v = pp[(size_t)z * (r + 2) + 2 + i];
+    a = fmaf(wz[z], wz[z] > 0.0f ? v : 0.0f, a);  // (an empty split's row is not written)
   }
+  out[((size_t)t * H + h) * r + i] = a / den;
 }
 
 }  // namespace lgs
@@ -1164,7 +1190,10 @@ extern "C" int lgs_latent_attention(const float* qc, const float* proj, long ld,
     else lgs::latent_attention_kernel<false, NR><<<grid, 256, lds, stream>>>(p, part);                 \
   } while (0)
   const bool vec = r % 8 == 0 && r <= 512 && (uintptr_t)cache_c % 16 == 0 && (uintptr_t)qc % 16 == 0;  // 16-byte row loads
-  if (vec && H % 4 == 0) {
+  // (few heads of short rows leave most of a wave idle either way, and four in one then wait longer: us of a head a workgroup / four, one
+  // token of 8 heads over 64 rows of 256 + 64 7.4 / 8.2, of 128 7.2 / 7.9, of 512 8.6 / 8.3; of 32 heads of 256 9.5 / 8.7, of 128 8.4 / 8.1)
+  const bool heads = H % 4 == 0 && (r > 256 || (long)T * H >= 32) && (uintptr_t)(splits > 1 ? part : out) % 8 == 0;
+  if (vec && heads) {
     if (cache_f32) lgs::latent_attention_heads_kernel<true><<<dim3(T, H / 4, splits), 256, 4 * lds, stream>>>(p, part);
     else lgs::latent_attention_heads_kernel<false><<<dim3(T, H / 4, splits), 256, 4 * lds, stream>>>(p, part);
   } else if (vec) {
@@ -1175,7 +1204,7 @@ extern "C" int lgs_latent_attention(const float* qc, const float* proj, long ld,
   else if (r <= 512) LGS_LAT(8);
   else LGS_LAT(16);
 #undef LGS_LAT
-  if (splits > 1) lgs::latent_combine_kernel<<<dim3(T, H), 256, 0, stream>>>(part, sink, out, H, r, splits);
+  if (splits > 1) lgs::latent_combine_kernel<<<dim3(T, H, (r + 255) / 256), 256, 0, stream>>>(part, sink, out, H, r, splits);
   LGA_LAUNCH_RETURN();
 }
 

@@ -334,7 +334,9 @@ def latent_attention(qc: torch.Tensor, proj: torch.Tensor, q_off: int, cache_c: 
         raise ValueError("latent_attention: shapes")
     out = torch.empty(T, H * r, dtype=F32, device=proj.device)
     if splits is None:
-        splits = max(1, min(32, (1024 if H % 4 else 1536) // (T * H)))  # (a head a workgroup, or four)
+        # (1536, with four heads a workgroup: one token of 64 heads over 64 rows 8.8 -> 10.0 us, eight of 16 7.6 -> 8.5, 20 of
+        # 32, which then take a second launch, 10.1 -> 13.1; from 600 rows on 61 -> 52 there, one to two in a hundred elsewhere)
+        splits = max(1, min(32, 1024 // (T * H)))
         if window > 0:  # at least one key per wave of a split
             splits = max(1, min(splits, window // 4))
     part = torch.empty(T * H * splits * (r + 2), dtype=F32, device=proj.device) if splits > 1 else None

@@ -35,3 +35,23 @@ def test_few_tokens(H, r, dr, d, f32, window, splits):
             score = torch.cat([score, sink.double()[:, None]], 1)
         want = torch.softmax(score, 1)[:, :n - lo] @ rows
         assert (got[t].double().view(H, r) - want).abs().max() < 2e-6 * max(1.0, float(rows.abs().max())) * 4
+
+
+@pytest.mark.parametrize("splits", [None, 9])
+def test_ranges_without_keys(splits):
+    """Their rows are never written: whatever memory they get, here NaN, is not read."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(2)
+    H, r, dr, d = 8, 264, 16, 8
+    c, kr = torch.randn(1, 40, r, generator=g, device=dev), torch.randn(1, 40, dr, generator=g, device=dev)
+    qc, proj = torch.randn(1, H * r, generator=g, device=dev), torch.randn(1, H * (d + dr), generator=g, device=dev)
+    at = lambda n: torch.tensor([n], dtype=torch.int32, device=dev)  # noqa: E731
+    for keys in (1, 2, 5):
+        held = [torch.full((n,), float("nan"), device=dev) for n in (H * r, *[H * 32 * (r + 2), H * 9 * (r + 2)] * 2)]
+        del held  # (the workspace comes from these)
+        got = seq_ops.latent_attention(qc, proj, 0, c, kr, None, at(0), at(keys - 1), H=H, d=d, dr=dr, r=r, scale=0.1, splits=splits)
+        q = proj.double().view(H, d + dr)[:, d:]
+        score = (qc.double().view(H, r) @ c[0, :keys].double().T + q @ kr[0, :keys].double().T) * 0.1
+        assert (got.double().view(H, r) - torch.softmax(score, 1) @ c[0, :keys].double()).abs().max() < 1e-5
