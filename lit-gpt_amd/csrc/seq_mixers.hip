@@ -490,6 +490,10 @@ struct LatAttArgs {
   int window;  // a query sees the last `window` rows (0: all up to its own)
 };
 
+// what an online softmax subtracts from its scores: their largest so far, or 0 while that is minus infinity, so that such keys weigh
+// nothing (and not NaN)
+__device__ __forceinline__ float lat_from(float most) { return most == -INFINITY ? 0.0f : most; }
+
 // grid (T, H, splits): split z of (token, head) owns an equal share of the keys it sees; its wave w walks keys
 // lo + w, lo + w + 4, ... four at a time (their loads in flight together) with an online softmax; lanes hold dims
 // lane + 64 e. One split finishes in place (the sink joins the denominator); several leave (max, sum, weighted sum)
@@ -547,7 +551,7 @@ __global__ void __launch_bounds__(256) latent_attention_kernel(LatAttArgs p, flo
     for (int u = 0; u < U; ++u) {
       if (j0 + 4 * u > hi) break;
       const float mn = fmaxf(m, dot[u]);
-      const float corr = expf(m - mn), w = expf(dot[u] - mn);
+      const float from = lat_from(mn), corr = expf(m - from), w = expf(dot[u] - from);
       l = l * corr + w;
 #pragma unroll
       for (int e = 0; e < NR; ++e) acc[e] = acc[e] * corr + w * c[u][e];
@@ -648,7 +652,7 @@ __global__ void __launch_bounds__(256) latent_attention_vec_kernel(LatAttArgs p,
     for (int u = 0; u < U; ++u) {
       if (j0 + 4 * u > hi) break;
       const float mn = fmaxf(m, dot[u]);
-      const float corr = expf(m - mn), w = expf(dot[u] - mn);
+      const float from = lat_from(mn), corr = expf(m - from), w = expf(dot[u] - from);
       l = l * corr + w;
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[e] = acc[e] * corr + w * c[u][e];
@@ -799,7 +803,7 @@ __global__ void __launch_bounds__(256) latent_attention_heads_kernel(LatAttArgs 
       mn = fmaxf(mn, s[u]);
     }
     if (j0 + 4 * U <= hi) fetch(j0 + 4 * U);
-    const float corr = expf(m - mn);
+    const float from = lat_from(mn), corr = expf(m - from);
     m = mn;
     l *= corr;
 #pragma unroll
@@ -811,7 +815,7 @@ __global__ void __launch_bounds__(256) latent_attention_heads_kernel(LatAttArgs 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (j0 + 4 * u > hi) break;
-      const float w = expf(s[u] - mn);
+      const float w = expf(s[u] - from);
       l += w;
 #pragma unroll
       for (int i = 0; i < HP; ++i) {

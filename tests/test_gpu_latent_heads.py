@@ -55,3 +55,28 @@ def test_ranges_without_keys(splits):
         q = proj.double().view(H, d + dr)[:, d:]
         score = (qc.double().view(H, r) @ c[0, :keys].double().T + q @ kr[0, :keys].double().T) * 0.1
         assert (got.double().view(H, r) - torch.softmax(score, 1) @ c[0, :keys].double()).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("H,r", [(8, 264), (6, 264), (6, 260), (8, 8)])
+@pytest.mark.parametrize("splits", [1, 3, 32])
+@pytest.mark.parametrize("sink", [False, True])
+def test_scores_of_minus_infinity(H, r, splits, sink):
+    """Keys with such a score weigh nothing, first or last of a wave's keys, of a range or of all; in all three kernels."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(r + splits)
+    dr, d, n = 4, 8, 50
+    c, kr = torch.randn(4, n, r, generator=g, device=dev), torch.randn(4, n, dr, generator=g, device=dev)
+    qc, proj = torch.randn(4, H * r, generator=g, device=dev), torch.randn(4, H, d + dr, generator=g, device=dev)
+    proj[..., d] = proj[..., d].abs() + 0.1
+    for slot, none in enumerate([[0], [*range(0, n, 4), 1, 6], list(range(20)), [*range(17), *range(34, n)]]):
+        kr[slot, none, 0] = float("-inf")
+    s = torch.randn(H, generator=g, device=dev) if sink else None
+    at = torch.arange(4, dtype=torch.int32, device=dev)
+    got = seq_ops.latent_attention(qc, proj.view(4, -1), 0, c, kr, s, at, torch.full_like(at, n - 1), H=H, d=d, dr=dr, r=r, scale=0.1,
+                                   splits=splits)
+    score = (qc.double().view(4, H, r) @ c.double().transpose(1, 2) + proj[..., d:].double() @ kr.double().transpose(1, 2)) * 0.1
+    if sink:
+        score = torch.cat([score, s.double()[:, None].expand(4, H, 1)], 2)
+    assert (got.double().view(4, H, r) - torch.softmax(score, 2)[..., :n] @ c.double()).abs().max() < 1e-5
