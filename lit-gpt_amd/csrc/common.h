@@ -43,9 +43,17 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 }
 __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
 
-// Until no load of this wave is in flight, in a form that hipcc counts. Ahead of stores that stand under conditions of their own: where
-// a value may still be on its way for all that hipcc knows, it waits for everything before each of them, the store before it included.
+// Ahead of stores that stand under conditions of their own. Where a register that they use or write may be a load's for all that hipcc
+// knows, on any way that leads there, it waits for everything in flight before each of them, the store before it included; behind a
+// wait that it counts it knows better. (The wait is for earlier stores as well: not for between stores.)
 __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// The same for values of their own, whose loads then cannot move behind the wait
+template <int N>
+__device__ __forceinline__ void wait_loads(float (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+  wait_loads();
+}
 
 // ---- wave-level reductions (64 lanes) ----
 __device__ __forceinline__ float wave_sum(float v) {

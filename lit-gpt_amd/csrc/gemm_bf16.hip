@@ -14,7 +14,6 @@ namespace lga {
 struct BfArgs {
   Q4dArgs a;
   int nt, splits, kper;  // tiles over columns; ranges of K of kper stages of 64 values
-  bool apart;            // (gemm_at)
 };
 
 // the tile at rows m0 .. and columns n0 .. of range `split`
@@ -68,7 +67,7 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(BfArgs k) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[FN > 1 ? kGemmLds<T> : T::LDS];
   GemmAt at;
-  if (!gemm_at<T::BN, WN * 32>(k.a.M, k.nt, k.splits, k.apart, &at)) return;
+  if (!gemm_at<T::BN, WN * 32>(k.a.M, k.nt, k.splits, &at)) return;
   const int m0 = at.m * T::BN, n0 = at.n * (DUAL ? T::BM / 2 : T::BM), frags = (k.a.M - m0 + WN * 32 - 1) / (WN * 32);
   if (frags >= FN) bf16_rows<WM, WN, FM, FN, RA, RB, DUAL>(k, lds, at.which, m0, n0);
   else bf16_short<WM, WN, FM, FN, kGemmLds<T>, DUAL>(k, lds, at.which, m0, n0, frags);
@@ -91,7 +90,7 @@ static void bf16_go(BfArgs k, bool dual, hipStream_t stream) {
 // (2^26). More than 1024 rows that fill the chip keep K whole.
 GemmPlan bf16_plan(int M, int N, int K, bool dual) {
   const long cols = dual ? 2L * N : N;
-  if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1, false};
+  if (M <= 32 && cols * K < 1L << 26) return GemmPlan{-1, 1};
   const bool full = M > 1024 && (M + 255) / 256 * (cols / 128) >= 256;
   return gemm_tile_plan(M, (int)cols, K, 1, false, full ? 1 : 0, kGemmRowsB | (dual ? kGemmPairs : 0));
 }
@@ -102,7 +101,7 @@ size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {
 
 int bf16_run(const Q4dArgs& a, const GemmPlan& p, bool dual, hipStream_t stream) {
   const int steps = a.K / 64, kper = (steps + p.ksplit - 1) / p.ksplit;
-  const BfArgs k{a, 0, (steps + kper - 1) / kper, kper, p.apart};
+  const BfArgs k{a, 0, (steps + kper - 1) / kper, kper};
   switch (p.tile) {
 #define LGA_CASE(I, SLOTS, US, FAST, ROUND, ...) \
   case I: bf16_go<__VA_ARGS__>(k, dual, stream); break;

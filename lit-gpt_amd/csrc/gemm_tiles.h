@@ -176,14 +176,13 @@ __device__ __forceinline__ bool gemm_xcd(int whole, int last, int* t) {
   return false;
 }
 inline unsigned gemm_grid(long tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
-// Where a workgroup's tile lies among those of `count` products (batches or ranges of K). apart: the short tiles behind all whole ones,
-// or else each beside the whole tiles of its columns
+// Where a workgroup's tile lies among those of `count` products (batches or ranges of K), the short tiles behind all whole ones
 struct GemmAt {
   int which, m, n;
 };
 template <int ROWS, int STEP>
-__device__ __forceinline__ bool gemm_at(int rows, int nt, int count, bool apart, GemmAt* o) {
-  const int all = (rows + ROWS - 1) / ROWS, mt = apart ? gemm_whole<ROWS, STEP>(rows) : all, per = mt * nt;
+__device__ __forceinline__ bool gemm_at(int rows, int nt, int count, GemmAt* o) {
+  const int all = (rows + ROWS - 1) / ROWS, mt = gemm_whole<ROWS, STEP>(rows), per = mt * nt;
   int t;
   if (gemm_xcd(count * per, count * (all - mt) * nt, &t)) {
     o->which = t / per;
@@ -225,7 +224,6 @@ constexpr int kGemmFormCount = sizeof(kGemmForms) / sizeof(kGemmForms[0]);
 // Which form, and how many ranges of K (ksplit 0: the plan's own choice); tile -1: K is no multiple of 64.
 struct GemmPlan {
   int tile, ksplit;
-  bool apart;
 };
 enum {
   kGemmRowsB = 1,  // the rows are the tile's B, the columns its A
@@ -239,7 +237,7 @@ inline bool gemm_form_fits(const GemmForm& t, int flags) {
 // Against all forms and ranges on 24 products of 64 to 4096 rows, weights from memory, the choice was the fastest or within 7 % of it
 // before there were short tiles. It still says the ranges, and with them the order of a product's sums, and the forms of grouped products.
 inline GemmPlan gemm_whole_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int flags) {
-  GemmPlan best{-1, 1, false};
+  GemmPlan best{-1, 1};
   if (K % 64 != 0 || M <= 0) return best;
   const int steps = K / 64;
   float best_us = 0.0f;
@@ -279,7 +277,6 @@ inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int
   if (best.tile < 0 || grouped) return best;
   const int steps = K / 64, per = (steps + best.ksplit - 1) / best.ksplit, count = batch * ((steps + per - 1) / per);
   float best_us = 0.0f;
-  best.apart = true;
   for (int f = 0; f < kGemmFormCount; ++f) {
     const GemmForm& t = kGemmForms[f];
     if (!gemm_form_fits(t, flags)) continue;

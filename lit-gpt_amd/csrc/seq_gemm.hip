@@ -12,44 +12,38 @@ using lga::GemmTile;
 using lga::f32x16_t;
 using lga::gemm_tile;
 
-// grouped rows: this workgroup's tile, z its batch and m, n its place inside it (false: none is left). The batches' tiles are
+// grouped rows: this workgroup's tile, z its batch and m, n its place inside it, a short one beside the whole ones of its columns
+// (false: none is left). The batches' tiles are
 // counted side by side over the lanes, and every XCD takes an eighth of those that there are: the grid is the largest number that the
 // groups' sizes allow, of which a third stayed empty and with it the last XCDs (16 groups of 512 rows of 2 x 1408 x 2048: 3 rounds on 5
 // XCDs instead of 2 on all, 216 -> 125 us).
-template <int ROWS, int STEP>
-__device__ __forceinline__ bool gemm_group(const int* z_start, int batch, int nt, bool apart, int lane, lga::GemmAt* o) {
-  auto tiles = [&](int e, int* mt) {  // short ones of batch e, and *mt others
-    const int rows = e < batch ? z_start[e + 1] - z_start[e] : 0, all = (rows + ROWS - 1) / ROWS;
-    *mt = apart ? lga::gemm_whole<ROWS, STEP>(rows) : all;
-    return all - *mt;
-  };
-  auto upto = [&](int v) {  // sum over the lanes up to this one
+template <int ROWS>
+__device__ __forceinline__ bool gemm_group(const int* z_start, int batch, int nt, int lane, lga::GemmAt* o) {
+  auto count = [&](int e, int* mt) {  // batch e's *mt row tiles, and the tiles of those of this lane and of all before it
+    *mt = e < batch ? (z_start[e + 1] - z_start[e] + ROWS - 1) / ROWS : 0;
+    int upto = *mt * nt;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-      const int u = __shfl_up(v, d);
-      if (lane >= d) v += u;
+      const int u = __shfl_up(upto, d);
+      if (lane >= d) upto += u;
     }
-    return v;
+    return upto;
   };
-  int whole = 0, last = 0, mt, t;
+  int total = 0, mt, t;
+  for (int e0 = 0; e0 < batch; e0 += 64) total += __shfl(count(e0 + lane, &mt), 63);
+  if (!lga::gemm_xcd(total, 0, &t)) return false;
   for (int e0 = 0; e0 < batch; e0 += 64) {
-    const int l = tiles(e0 + lane, &mt);
-    whole += __shfl(upto(mt * nt), 63), last += __shfl(upto(l * nt), 63);
-  }
-  const bool first = lga::gemm_xcd(whole, last, &t);
-  if (t < 0) return false;
-  for (int e0 = 0; e0 < batch; e0 += 64) {
-    const int l = tiles(e0 + lane, &mt), own = (first ? mt : l) * nt, sum = upto(own);
-    const unsigned long long past = __ballot(sum > t);
+    const int upto = count(e0 + lane, &mt);
+    const unsigned long long past = __ballot(upto > t);
     if (past) {
       const int at = __ffsll(past) - 1;
+      t = __builtin_amdgcn_readfirstlane(t - __shfl(upto - mt * nt, at));
       mt = __builtin_amdgcn_readfirstlane(__shfl(mt, at));
-      t = __builtin_amdgcn_readfirstlane(t - __shfl(sum - own, at));
       o->which = __builtin_amdgcn_readfirstlane(e0 + at);
-      o->m = first ? t % mt : mt, o->n = first ? t / mt : t;
+      o->m = t % mt, o->n = t / mt;
       return true;
     }
-    t -= __shfl(sum, 63);
+    t -= __shfl(upto, 63);
   }
   return false;
 }
@@ -104,6 +98,7 @@ __device__ __forceinline__ void gemm_rows(const LinArgs& p, unsigned char* lds, 
     constexpr int R = decltype(rows_at_once)::value;
     const unsigned at = (unsigned)(hi * 4 * (int)ld + l31);
     const int rows = Mz - 1 - mw - hi * 4, cols = p.N - 1 - nw - l31;  // a lane's last ones
+    if constexpr (!SUMS) lga::wait_loads();
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -153,9 +148,10 @@ __device__ __forceinline__ void gemm_rows(const LinArgs& p, unsigned char* lds, 
   float bias[FN];
 #pragma unroll
   for (int j = 0; j < FN; ++j) bias[j] = p.bias ? p.bias[min(nw + l31 + j * 32, p.N - 1)] : 0.0f;
-  // (or, in tiles that rows or columns end in, every store waits for the one before. us: 1000 rows of 6288 x 2048 36.3 / 29.6, 1500
-  // 52.0 / 41.6, of 4096 x 4096 53.8 / 49.7, 2407 of 2048 x 2048 29.4 / 25.1)
-  lga::wait_loads();
+  // (here and at each list of stores: or, in tiles that rows or columns end in, every store waits for the one before. us: 1000 rows of
+  // 6288 x 2048 36.3 / 29.6, 1500 52.0 / 41.6, of 4096 x 4096 53.8 / 49.7, 2407 of 2048 x 2048 29.4 / 25.1; 16 groups of 512 rows of 1024
+  // x 1024 41.5 / 29.4)
+  lga::wait_loads(bias);
   const long at = (long)z * p.sy + (long)(r_lo + mw) * p.ldy + nw;
   if (ACTS && p.act != kActNone) {
     if constexpr (ACTS) {
@@ -191,18 +187,18 @@ __device__ __forceinline__ void gemm_short(const LinArgs& p, unsigned char* lds,
 }
 
 template <int WM, int WN, int FM, int FN, int RA, int RB>
-__global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int nt, int batch, bool apart) {
+__global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int nt, int batch) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[FM > 1 ? lga::kGemmLds<T> : T::LDS];
   lga::GemmAt at;
   int z = 0, split = 0, r_lo = 0, Mz = p.M;
   if (p.z_start) {
-    if (!gemm_group<T::BM, WM * 32>(p.z_start, batch, nt, apart, threadIdx.x & 63, &at)) return;
+    if (!gemm_group<T::BM>(p.z_start, batch, nt, threadIdx.x & 63, &at)) return;
     z = at.which;
     r_lo = p.z_start[z];
     Mz = p.z_start[z + 1] - r_lo;
   } else {
-    if (!lga::gemm_at<T::BM, WM * 32>(Mz, nt, batch * p.ksplit, apart, &at)) return;
+    if (!lga::gemm_at<T::BM, WM * 32>(Mz, nt, batch * p.ksplit, &at)) return;
     if (p.ksplit > 1) split = at.which;
     else z = at.which;
   }
@@ -212,12 +208,12 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_kernel(LinArgs p, int nt, in
 }
 
 template <int WM, int WN, int FM, int FN, int RA, int RB>
-static int gemm_go(const LinArgs& p, int batch, bool apart, hipStream_t stream) {
+static int gemm_go(const LinArgs& p, int batch, hipStream_t stream) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   const long mt = (p.M + T::BM - 1) / T::BM, nt = (p.N + T::BN - 1) / T::BN;
   const long tiles = p.z_start ? (mt + batch) * nt : mt * nt * batch * p.ksplit;
   LGA_CHECK_ARG(tiles < (1L << 30), "lgs_linear: too many tiles");
-  gemm_kernel<WM, WN, FM, FN, RA, RB><<<lga::gemm_grid(tiles), T::NT, 0, stream>>>(p, (int)nt, batch, apart);
+  gemm_kernel<WM, WN, FM, FN, RA, RB><<<lga::gemm_grid(tiles), T::NT, 0, stream>>>(p, (int)nt, batch);
   return 0;
 }
 
@@ -286,17 +282,17 @@ __device__ __forceinline__ void glu_short(const LinArgs& p, const GluForm& f, un
 }
 
 template <int WM, int WN, int FM, int FN, int RA, int RB, bool CLAMPED>
-__global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluForm f, int nt, int batch, bool apart) {
+__global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluForm f, int nt, int batch) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[FN > 1 ? lga::kGemmLds<T> : T::LDS];
   lga::GemmAt at;
   int z = 0, r_lo = 0, Mz = p.M;
   if (p.z_start) {
-    if (!gemm_group<T::BN, WN * 32>(p.z_start, batch, nt, apart, threadIdx.x & 63, &at)) return;
+    if (!gemm_group<T::BN>(p.z_start, batch, nt, threadIdx.x & 63, &at)) return;
     z = at.which;
     r_lo = p.z_start[z];
     Mz = p.z_start[z + 1] - r_lo;
-  } else if (!lga::gemm_at<T::BN, WN * 32>(Mz, nt, 1, apart, &at)) {
+  } else if (!lga::gemm_at<T::BN, WN * 32>(Mz, nt, 1, &at)) {
     return;
   }
   const int m0 = at.m * T::BN, n0 = at.n * (T::BM / 2), frags = (Mz - m0 + WN * 32 - 1) / (WN * 32);
@@ -305,21 +301,21 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_glu_kernel(LinArgs p, GluFor
 }
 
 template <int WM, int WN, int FM, int FN, int RA, int RB>
-static int glu_go(const LinArgs& p, const GluForm& f, int batch, bool apart, hipStream_t stream) {
+static int glu_go(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
   using T = GemmTile<WM, WN, FM, FN, RA, RB>;
   const long mt = (p.M + T::BN - 1) / T::BN, nt = (p.N + T::BM / 2 - 1) / (T::BM / 2);
   const long tiles = p.z_start ? (mt + batch) * nt : mt * nt;
   LGA_CHECK_ARG(tiles < (1L << 30), "lgs_linear_glu: too many tiles");
   const unsigned grid = lga::gemm_grid(tiles);
-  if (f.clamped) gemm_glu_kernel<WM, WN, FM, FN, RA, RB, true><<<grid, T::NT, 0, stream>>>(p, f, (int)nt, batch, apart);
-  else gemm_glu_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(p, f, (int)nt, batch, apart);
+  if (f.clamped) gemm_glu_kernel<WM, WN, FM, FN, RA, RB, true><<<grid, T::NT, 0, stream>>>(p, f, (int)nt, batch);
+  else gemm_glu_kernel<WM, WN, FM, FN, RA, RB, false><<<grid, T::NT, 0, stream>>>(p, f, (int)nt, batch);
   return 0;
 }
 
 int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
 #define LGS_CASE(I, SLOTS, US, FAST, ROUND, ...)                                     \
   case I:                                                                            \
-    if constexpr (lga::kGemmForms[I].fm % 2 == 0) return glu_go<__VA_ARGS__>(p, f, batch, plan.apart, stream); \
+    if constexpr (lga::kGemmForms[I].fm % 2 == 0) return glu_go<__VA_ARGS__>(p, f, batch, stream); \
     break;
   const GemmPlan plan = lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, lga::kGemmRowsB | lga::kGemmPairs);
   switch (plan.tile) { LGA_GEMM_FORMS(LGS_CASE) }
@@ -329,13 +325,13 @@ int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t s
 }
 
 GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act) {
-  if (grouped && gemm_few_rows(M, batch)) return GemmPlan{-1, 1, false};
+  if (grouped && gemm_few_rows(M, batch)) return GemmPlan{-1, 1};
   return lga::gemm_tile_plan(M, N, K, batch, grouped, ksplit, act != kActNone ? lga::kGemmActs : 0);
 }
 
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream) {
 #define LGS_CASE(I, SLOTS, US, FAST, ROUND, ...) \
-  case I: return gemm_go<__VA_ARGS__>(p, batch, plan.apart, stream);
+  case I: return gemm_go<__VA_ARGS__>(p, batch, stream);
   switch (plan.tile) { LGA_GEMM_FORMS(LGS_CASE) }
 #undef LGS_CASE
   lga_set_error("lgs_linear: no such form");

@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(256) lin_mfma_kernel(LinArgs p) {
   float bias[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) bias[e] = p.bias && !split ? p.bias[min(n + e, p.N - 1)] : 0.0f;
-  lga::wait_loads();  // (or every store waits for the one before)
+  lga::wait_loads(bias);  // (or every store waits for the one before)
 #pragma unroll
   for (int part = 0; part < 2; ++part) {
 #pragma unroll

@@ -152,7 +152,7 @@ __global__ void __launch_bounds__(256) ssm_scan_kernel(ScanArgs p) {
     }
     // (the next batch's writes to `part` come after its first barrier, which wave 0 reaches after these reads)
   }
-  lga::wait_loads();  // (or every store waits for the one before)
+  lga::wait_loads(S);  // (or every store waits for the one before)
   if (live) {
 #pragma unroll
     for (int i = 0; i < NR; ++i)
