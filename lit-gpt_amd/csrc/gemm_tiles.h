@@ -17,6 +17,7 @@
 // 8192 950 -> 804. Both give the same bits.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -233,30 +234,42 @@ enum {
 inline bool gemm_form_fits(const GemmForm& t, int flags) {
   return !((flags & kGemmActs && t.bm * t.bn > 256 * 128) || (flags & kGemmPairs && t.fm % 2));
 }
+// (a plan is made at every launch: no library call for a rounding, nothing of the ranges for each form anew. us a plan, mean of 66 sizes,
+// with both / here: ranges to choose 2.34 / 0.85, given 0.45 / 0.14)
+// (of 0 to 2^63)
+inline float gemm_floor(float v) { return (float)(long)v; }
+inline float gemm_ceil(float v) { return gemm_floor(v) + (gemm_floor(v) < v ? 1.0f : 0.0f); }
 // Counted in whole tiles: rounds of workgroups times what one takes; several ranges of K cost a second launch that reads them all.
 // Against all forms and ranges on 24 products of 64 to 4096 rows, weights from memory, the choice was the fastest or within 7 % of it
 // before there were short tiles. It still says the ranges, and with them the order of a product's sums, and the forms of grouped products.
 inline GemmPlan gemm_whole_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int flags) {
   GemmPlan best{-1, 1};
   if (K % 64 != 0 || M <= 0) return best;
-  const int steps = K / 64;
+  constexpr int kMost = 16;
+  const int steps = K / 64, s_lo = ksplit > 0 ? ksplit : 1, s_hi = ksplit > 0 ? ksplit : (batch > 1 || grouped ? 1 : kMost);
+  int each[kMost], count = 0;  // steps of a range, by the number of ranges asked for
+  float made[kMost];           // ranges that there are
+  for (int s = s_lo; s <= s_hi && (s == s_lo || steps / s >= 4); ++s, ++count) {
+    each[count] = (steps + s - 1) / s;
+    made[count] = (float)((steps + each[count] - 1) / each[count]);
+  }
   float best_us = 0.0f;
+#pragma unroll
   for (int f = 0; f < kGemmFormCount; ++f) {
     const GemmForm& t = kGemmForms[f];
     if (!gemm_form_fits(t, flags)) continue;
     const int rows = flags & kGemmRowsB ? t.bn : t.bm, cols = flags & kGemmRowsB ? t.bm : t.bn;
     const float nt = (float)((N + cols - 1) / cols);
     // a range of the list ends somewhere in its last tile, and has one
-    const float mt = grouped ? fmaxf((float)M / rows + 0.5f * batch, (float)min(batch, M)) : (float)((M + rows - 1) / rows) * batch;
-    const int s_lo = ksplit > 0 ? ksplit : 1, s_hi = ksplit > 0 ? ksplit : (batch > 1 || grouped ? 1 : 16);
-    for (int s = s_lo; s <= s_hi && (s == s_lo || steps / s >= 4); ++s) {
-      const int per = (steps + s - 1) / s;
-      const float rounds = mt * nt * (float)((steps + per - 1) / per) / (float)t.slots, whole = floorf(rounds);
+    const float mt = grouped ? std::max((float)M / rows + 0.5f * batch, (float)std::min(batch, M)) : (float)((M + rows - 1) / rows) * batch;
+    for (int i = 0; i < count; ++i) {
+      const int s = s_lo + i, per = each[i];
+      const float rounds = mt * nt * made[i] / (float)t.slots, whole = gemm_floor(rounds);
       float us = (grouped && rounds > 1.0f ? rounds + 0.5f : whole) * (per * t.step_us + t.round_us);
       if (grouped ? rounds <= 1.0f : rounds > whole) {
         // few workgroups have a higher clock: 160 of 256 x 256 take 0.74 of 256's time; smaller tiles, which draw less, 0.82
         const float most = t.bm * t.bn > 128 * 192 ? 0.7f : 0.5f;
-        us += per * fmaxf(t.fast_us, t.step_us * (1.0f - most * (1.0f - (rounds - whole)))) + t.round_us;
+        us += per * std::max(t.fast_us, t.step_us * (1.0f - most * (1.0f - (rounds - whole)))) + t.round_us;
       }
       if (s > 1) us += 2.0f + (float)M * N * 4.0f * (s + 1) / 5.5e6f;
       if (best.tile < 0 || us < best_us) best_us = us, best.tile = f, best.ksplit = s;
@@ -270,33 +283,37 @@ inline GemmPlan gemm_whole_plan(int M, int N, int K, int batch, bool grouped, in
 // the form that counts whole tiles 2.0 %. us of whole tiles alone / here: 2407 x 20608 x 4096 448 / 381, 517 x 11008 x 4096 with SwiGLU
 // 109 / 101, 40 rows of it 37 / 33.
 // A grouped product's short tiles stand beside the whole ones of their columns, whose weights they would otherwise fetch anew (16 groups of
-// 278 rows of twice 2752 x 4096 302 behind, 260 beside): 546 products of 16 groups, 160 to 16384 rows in all, in 0.96 of the time of
-// whole tiles (450 rows each of 2048 x 1408 70 / 67, of 4096 x 2752 227 / 210), none more than 7 % slower.
+// 278 rows of twice 2752 x 4096 302 behind, 260 beside): 480 products of 8 to 18 groups, 144 to 16384 rows in all, weights from memory,
+// take 0.93 of the time that whole tiles took (gated units 0.98), none more than 3 % more. (Weights that stay in the last cache from
+// call to call gain less, up to 6 % lost.)
 inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int flags) {
-  GemmPlan best = gemm_whole_plan(M, N, K, batch, grouped, ksplit, flags);
-  if (best.tile < 0 || grouped) return best;
+  GemmPlan best{-1, 1};
+  if (grouped) return gemm_whole_plan(M, N, K, batch, true, ksplit, flags);
+  if (K % 64 != 0 || M <= 0) return best;
+  best.ksplit = ksplit > 0 ? ksplit : batch > 1 ? 1 : gemm_whole_plan(M, N, K, 1, false, 0, flags).ksplit;
   const int steps = K / 64, per = (steps + best.ksplit - 1) / best.ksplit, count = batch * ((steps + per - 1) / per);
   float best_us = 0.0f;
+#pragma unroll
   for (int f = 0; f < kGemmFormCount; ++f) {
     const GemmForm& t = kGemmForms[f];
     if (!gemm_form_fits(t, flags)) continue;
     const bool rows_b = flags & kGemmRowsB;
     const int rows = rows_b ? t.bn : t.bm, cols = rows_b ? t.bm : t.bn, frags = rows_b ? t.fn : t.fm, step = rows / frags;
-    const float most = t.bm * t.bn > 128 * 192 ? 0.69f : 0.46f;  // (of what fewer workgroups gain, as above)
-    auto round = [&](float load) { return per * fmaxf(t.fast_us, t.step_us * (1.0f - most * (1.0f - load))) + t.round_us; };
+    const float most = t.bm * t.bn > 128 * 192 ? 0.69f : 0.46f;  // (of what fewer workgroups gain: 0.7 and 0.5 above, fitted anew on these products)
+    auto round = [&](float load) { return per * std::max(t.fast_us, t.step_us * (1.0f - most * (1.0f - load))) + t.round_us; };
     const int pieces = (M + step - 1) / step, mt = pieces / frags, left = pieces % frags;
     const float nt = (float)((N + cols - 1) / cols), slots = (float)t.slots;
-    const float whole = mt * nt * count, full = floorf(whole / slots), over = whole - full * slots;
+    const float whole = mt * nt * count, full = gemm_floor(whole / slots), over = whole - full * slots;
     // a short tile's time of a whole one's; alone on the chip it is mostly latency
-    const float each = left == 0 ? 1.0f : fmaxf(0.3f + 0.7f * left / frags, mt > 0 ? 0.0f : 0.75f);
+    const float each = left == 0 ? 1.0f : std::max(0.3f + 0.7f * left / frags, mt > 0 ? 0.0f : 0.75f);
     float shorts = left ? nt * count : 0.0f, us;
     us = full * round(1.0f);
     if (over > 0.0f) {
-      const float beside = fminf(shorts, (slots - over) * floorf(1.0f / each));
+      const float beside = std::min(shorts, (slots - over) * gemm_floor(1.0f / each));
       us += round((over + beside * each) / slots);
       shorts -= beside;
     }
-    if (shorts > 0.0f) us += each * ceilf(shorts / slots) * round(fminf(shorts / slots, 1.0f) * each);
+    if (shorts > 0.0f) us += each * gemm_ceil(shorts / slots) * round(std::min(shorts / slots, 1.0f) * each);
     if (best_us == 0.0f || us < best_us) best_us = us, best.tile = f;
   }
   return best;
