@@ -186,8 +186,8 @@ __global__ void __launch_bounds__(256) mingru_step_kernel(MinGruStepArgs p) {
 // mingru_step_kernel for several sequences and bf16 weights, on the matrix cores (seq_rows.h): a workgroup makes the three projections of 16
 // channels, and a lane finishes four of one sequence. Bound by memory. us, a wave a channel / here: 3 sequences of 4096 channels of 4096 values
 // 27.7 / 19.6, 8 44.1 / 19.8, 8 of 2048 of 2048 20.0 / 11.6, 2 of 8192 of 2048 25.0 / 20.0 (one: 20.6 there).
-template <int KW, int MR, int RB>
-__global__ void __launch_bounds__(KW * 64) mingru_rows_kernel(MinGruStepArgs p) {
+template <int KW, int MR, int RB, bool ONE>
+__global__ void __launch_bounds__(KW * 64, 2) mingru_rows_kernel(MinGruStepArgs p) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[RowsTile<3, KW, MR, RB>::LDS];
   const int lane = threadIdx.x & 63, m = lane & 15, c0 = blockIdx.x * 16, c = c0 + (lane >> 4) * 4;
   const bool fin = threadIdx.x < 64 && m < p.M && c < p.n;
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(KW * 64) mingru_rows_kernel(MinGruStepArgs p) 
     bias[2][r] = p.bias && fin ? p.bias[p.g0 + at] : 0.0f;
   }
   const uint16_t* w = (const uint16_t*)p.w;
-  rows_products<3, KW, MR, RB>(lds, [&](int r) {
+  rows_products<3, KW, MR, RB, ONE>(lds, [&](int r) {
     return w + (size_t)((r < 16 ? p.z0 : (r < 32 ? p.u0 : p.g0)) + min(c0 + (r & 15), p.n - 1)) * p.K;
   }, p.h, p.ldh, p.M, p.K);
   if (!fin) return;
@@ -256,14 +256,19 @@ extern "C" int lgs_mingru_step(const float* h, long ldh, const void* w, int w_f3
   if (!w_f32 && lgs::mingru_rows_pay(M, K, n) && K % 128 == 0 && ldh % 4 == 0 && ((uintptr_t)h | (uintptr_t)w) % 16 == 0) {
     const unsigned blocks = (n + 15) / 16;
     // (a workgroup a compute unit or fewer: eight waves, or two blocks of each of four)
-#define LGS_GRU_ROWS(MR)                                                                            \
+#define LGS_GRU_ROWS(MR, ONE)                                                                       \
   do {                                                                                              \
-    if (blocks <= 128) lgs::mingru_rows_kernel<8, MR, 1><<<blocks, 512, 0, stream>>>(p);            \
-    else if (blocks <= 256) lgs::mingru_rows_kernel<4, MR, 2><<<blocks, 256, 0, stream>>>(p);       \
-    else lgs::mingru_rows_kernel<4, MR, 1><<<blocks, 256, 0, stream>>>(p);                          \
+    if (blocks <= 128) lgs::mingru_rows_kernel<8, MR, 1, ONE><<<blocks, 512, 0, stream>>>(p);       \
+    else if (blocks <= 256) lgs::mingru_rows_kernel<4, MR, 2, ONE><<<blocks, 256, 0, stream>>>(p);  \
+    else lgs::mingru_rows_kernel<4, MR, 1, ONE><<<blocks, 256, 0, stream>>>(p);                     \
   } while (0)
-    if (M > 4) LGS_GRU_ROWS(8);
-    else LGS_GRU_ROWS(4);
+    if (lgs::rows_one(K)) {
+      if (M > 4) LGS_GRU_ROWS(8, true);
+      else LGS_GRU_ROWS(4, true);
+    } else {
+      if (M > 4) LGS_GRU_ROWS(8, false);
+      else LGS_GRU_ROWS(4, false);
+    }
 #undef LGS_GRU_ROWS
     LGA_LAUNCH_RETURN();
   }

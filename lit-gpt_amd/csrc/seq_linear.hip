@@ -190,13 +190,13 @@ __global__ void __launch_bounds__(256) lin_glu_row_kernel(const float* __restric
 }
 
 // seq_rows.h's products, finished here
-template <int NR, int KW, int MR, int RB>
+template <int NR, int KW, int MR, int RB, bool ONE>
 __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[RowsTile<NR, KW, MR, RB>::LDS];
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, q4 = lane >> 4;
   const int z = blockIdx.y, n0 = blockIdx.x * (16 * NR);
   const uint16_t* w = (const uint16_t*)p.w + (size_t)z * p.sw;
-  rows_products<NR, KW, MR, RB>(lds, [&](int r) { return w + (size_t)min(n0 + r, p.N - 1) * p.K; }, p.a + (size_t)z * p.sa, p.lda, p.M, p.K);
+  rows_products<NR, KW, MR, RB, ONE>(lds, [&](int r) { return w + (size_t)min(n0 + r, p.N - 1) * p.K; }, p.a + (size_t)z * p.sa, p.lda, p.M, p.K);
   if (tid >= NR * 64 || l15 >= p.M) return;
   const int j = NR > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
   const rows_f32x4 v = rows_sum<NR, KW>(lds, j, lane);
@@ -212,18 +212,18 @@ __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
 // 16 columns a workgroup; 32, which read A half as often, for more than four rows where their workgroups end together: many, or one a
 // compute unit (us of 16 / 32 columns: 8 x 32000 x 2048 31.3 / 30.2, x 22016 x 4096 40.6 / 37.6, x 6288 x 2048 9.8 / 9.0, x 4608 x 4096
 // 13.0 / 11.5, x 8192 x 2048 9.5 / 10.2, x 4096 x 4096 9.3 / 13.4; 3 x 32000 x 4096 48.2 / 50.8). Below 4096 columns eight waves share K.
-template <int NR, int KW>
+template <int NR, int KW, int MR, bool ONE>
 static void lin_rows_go(const LinArgs& p, int batch, hipStream_t stream) {
   const dim3 grid((p.N + 16 * NR - 1) / (16 * NR), batch);
   if constexpr (KW == 4) {
-    if ((long)grid.x * batch <= 256) {
-      if (p.M > 4) lin_rows_kernel<NR, KW, 8, 2><<<grid, KW * 64, 0, stream>>>(p);
-      else lin_rows_kernel<NR, KW, 4, 2><<<grid, KW * 64, 0, stream>>>(p);
-      return;
-    }
+    if ((long)grid.x * batch <= 256) return lin_rows_kernel<NR, KW, MR, 2, ONE><<<grid, KW * 64, 0, stream>>>(p);
   }
-  if (p.M > 4) lin_rows_kernel<NR, KW, 8, 1><<<grid, KW * 64, 0, stream>>>(p);
-  else lin_rows_kernel<NR, KW, 4, 1><<<grid, KW * 64, 0, stream>>>(p);
+  lin_rows_kernel<NR, KW, MR, 1, ONE><<<grid, KW * 64, 0, stream>>>(p);
+}
+template <int NR, int KW>
+static void lin_rows_go(const LinArgs& p, int batch, hipStream_t stream) {
+  if (rows_one(p.K)) (p.M > 4 ? lin_rows_go<NR, KW, 8, true> : lin_rows_go<NR, KW, 4, true>)(p, batch, stream);
+  else (p.M > 4 ? lin_rows_go<NR, KW, 8, false> : lin_rows_go<NR, KW, 4, false>)(p, batch, stream);
 }
 
 // What they gain on a lane's sums (lin_gemv_kernel; us there / here): 5 to 8 rows always (8 x 64 x 512 5.5 / 3.1, 5 x 1024 x 4096 15.3 / 7.2),

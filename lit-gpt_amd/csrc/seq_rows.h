@@ -18,9 +18,10 @@ typedef float rows_f32x4 __attribute__((ext_vector_type(4)));
 // 15.2 / 16.6, 3 x 6144 x 4096 12.6 / 13.5); two where a workgroup of four waves has one alone (8 x 4096 x 4096 11.3 / 9.3, 3 rows 10.0 / 8.7,
 // 11264 long 23.2 / 18.1, 8 x 6144 x 4096 14.7 / 13.4, 8 x 4096 x 2048 7.2 / 6.6; three are no faster, eight waves' 128 KB slower: 8 x 2048 x
 // 2048 5.9 / 6.6). The rows are read as vectors of the compiler's own: a read of HIP's float4 may alias the DMAs for it, and waits for all.
-// Sums: two instructions, then vector adds, then the ranges pairwise, so that the error against float64 is what the
-// lanes' sums of lin_gemv_kernel leave (rms of 8 rows at K 2048 / 4096 / 11008: 7.4e-8 / 8.0e-8 / 9.5e-8 of the results,
-// 7.5e-8 / 8.4e-8 / 1.1e-7 there; one chain of instructions 1.5 to 3 times as much).
+// Sums: two instructions (one below K 2048), then vector adds, then the ranges pairwise, so that the error against float64 is at most
+// what the lanes' sums of lin_gemv_kernel leave: rms of 8 rows at K 128 / 512 / 1024 / 2048 / 4096 / 11008 4.8e-8 / 6.1e-8 / 6.7e-8 / 7.4e-8
+// / 8.0e-8 / 9.5e-8 of the results, 4.8e-8 / 6.2e-8 / 6.8e-8 / 7.5e-8 / 8.4e-8 / 1.1e-7 there. (Two instructions at K 128 / 512 / 1024 5.0e-8 /
+// 6.3e-8 / 6.9e-8, one at 4096 / 11008 8.3e-8 / 1.1e-7; one chain of instructions 1.5 to 3 times as much.)
 // Bound by memory, with few columns by its latency. Loaded into registers as the instructions take them, every lane's 16 bytes lay
 // in a line of their own, and a compute unit got some 17 bytes a ns of W and A together, from whichever cache. us there / here, weights
 // from memory, the same bits: 8 x 2048 x 2048 11.9 / 5.9, x 4096 x 2048 10.1 / 6.6, x 6288 x 2048 14.2 / 9.0, x 32000 x 2048 44.5 / 30.2, x
@@ -31,9 +32,12 @@ struct RowsTile {
   static_assert(LDS <= 163840 && NR * 1024 <= SLOT, "LDS");
 };
 
+// Whether a sum takes one instruction
+inline bool rows_one(int K) { return K < 2048; }
+
 // weights(r): the K values of column r of the workgroup's 16 NR; x0: M rows, ldx apart. The ranges' sums are left in LDS, for rows_sum
 // behind the barrier that ends this.
-template <int NR, int KW, int MR, int RB, class Weights>
+template <int NR, int KW, int MR, int RB, bool ONE, class Weights>
 __device__ __forceinline__ void rows_products(unsigned char* lds_all, Weights&& weights, const float* x0, long ldx, int M, int K) {
   using T = RowsTile<NR, KW, MR, RB>;
   constexpr int W_BYTES = T::W_BYTES, SLOT = T::SLOT, PW = NR * 4, PA = MR / 2;
@@ -89,16 +93,19 @@ __device__ __forceinline__ void rows_products(unsigned char* lds_all, Weights&& 
         slot = slot + SLOT == RB * SLOT ? 0 : slot + SLOT;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          rows_f32x4 v[NR];
+          rows_f32x4 v[2][NR];
 #pragma unroll
-          for (int m = 2 * u; m < 2 * u + 2; ++m) {
+          for (int e = 0; e < 2; ++e) {
+            const int m = 2 * u + e;
             const uint4 x16 = make_uint4(pack2(x[m][0].x, x[m][0].y), pack2(x[m][0].z, x[m][0].w), pack2(x[m][1].x, x[m][1].y), pack2(x[m][1].z, x[m][1].w));
 #pragma unroll
             for (int j = 0; j < NR; ++j)
-              v[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[m][j], __builtin_bit_cast(rows_bf16x8, x16), m == 2 * u ? zero : v[j], 0, 0, 0);
+              v[e][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[m][j], __builtin_bit_cast(rows_bf16x8, x16), ONE || e == 0 ? zero : v[0][j], 0, 0, 0);
           }
 #pragma unroll
-          for (int j = 0; j < NR; ++j) acc[s * 2 + u][j] += v[j];
+          for (int e = ONE ? 0 : 1; e < 2; ++e)
+#pragma unroll
+            for (int j = 0; j < NR; ++j) acc[s * 2 + u][j] += v[e][j];
         }
       }
     }
