@@ -220,9 +220,13 @@ __global__ void __launch_bounds__(KW * 64, 2) mingru_rows_kernel(MinGruStepArgs 
   }
 }
 
-// Five sequences and more always, three and four of long rows, two of many channels. us, a wave a channel / matrix cores: 4 of 256 channels of
-// 256 values 5.0 / 5.4, 3 of 1024 of 1024 6.8 / 6.6; 2 of 2048 of 2048 10.4 / 10.9, of 3072 of 2048 13.0 / 11.1, of 5120 of 5120 33.2 / 35.9
-static bool mingru_rows_pay(int M, int K, int n) { return M > 4 || (M > 2 && K >= 1024) || (M == 2 && n > 2048 && K <= 4096); }
+// Five sequences and more always, three and four of long rows, two of many channels whose workgroups end together. us, a wave a channel /
+// matrix cores: 4 of 256 channels of 256 values 5.1 / 5.5, 3 of 1024 of 1024 6.8 / 6.4; 2 of 2048 of 2048 10.5 / 11.3, of 3072 of 2048 13.1 /
+// 11.3, of 2560 of 512 6.3 / 6.5, of 4096 of 512 7.2 / 7.1, of 5120 of 3072 21.9 / 23.3, of 8192 of 256 9.2 / 7.5, of 4096 42.7 / 37.3
+static bool mingru_rows_pay(int M, int K, int n) {
+  if (M == 2) return K >= 256 && K <= 4096 && (n >= 7168 || (n > 2048 && n <= 4096 && (long)n * K >= 1L << 21));
+  return M > 4 || (M > 2 && K >= 1024);
+}
 
 }  // namespace lgs
 

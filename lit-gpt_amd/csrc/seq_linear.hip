@@ -211,7 +211,8 @@ __global__ void __launch_bounds__(KW * 64) lin_rows_kernel(LinArgs p) {
 }
 // 16 columns a workgroup; 32, which read A half as often, for more than four rows where their workgroups end together: many, or one a
 // compute unit (us of 16 / 32 columns: 8 x 32000 x 2048 31.3 / 30.2, x 22016 x 4096 40.6 / 37.6, x 6288 x 2048 9.8 / 9.0, x 4608 x 4096
-// 13.0 / 11.5, x 8192 x 2048 9.5 / 10.2, x 4096 x 4096 9.3 / 13.4; 3 x 32000 x 4096 48.2 / 50.8). Below 4096 columns eight waves share K.
+// 13.0 / 11.5, x 8192 x 2048 9.5 / 10.2, x 4096 x 4096 9.3 / 13.4, x 5120 x 1024 5.4 / 5.8; 3 x 32000 x 4096 48.2 / 50.8). Below 4096 columns
+// eight waves share K.
 template <int NR, int KW, int MR, bool ONE>
 static void lin_rows_go(const LinArgs& p, int batch, hipStream_t stream) {
   const dim3 grid((p.N + 16 * NR - 1) / (16 * NR), batch);
@@ -230,10 +231,14 @@ static void lin_rows_go(const LinArgs& p, int batch, hipStream_t stream) {
 // four but of few columns and long rows (4 x 1024 x 2048 7.4 / 4.4, x 20608 x 2048 34.3 / 18.8; x 256 x 2048 4.1 / 4.0, x 256 x 4096 5.4 /
 // 4.9), two and three of long rows (2 x 2048 x 4096 9.0 / 7.9, 3 x 1024 x 4096 11.4 / 6.6; 3 x 512 x 8192 8.9 / 9.3), one of longer rows and few
 // columns (1 x 2048 x 5632 10.0 / 9.2, x 3072 x 8192 15.7 / 12.3; x 512 x 5632 5.0 / 7.4, x 2048 x 2048 5.2 / 5.4). Two and three shorter
-// rows (2 x 8192 x 2048 12.6 / 9.1) keep the bits that each has alone. columns: of all batches
+// rows (2 x 8192 x 2048 12.6 / 9.1) keep the bits that each has alone, and two of large matrices whose rows lie a multiple of 16 KB apart,
+// in the same channels of memory, go faster side by side (2 x 16384 x 8192 55.4 / 57.8, x 14336 x 16384 91 / 104; x 11008 x 8192 39.8 /
+// 37.3, x 14336 x 11008 76 / 65). Of short rows: 5 x 2048 x 128 3.5 / 3.3, 4 x 512 x 128 4.0 / 3.2, of 16 heads 8 x 512 x 128 9.3 / 4.0.
+// columns: of all batches
 static bool lin_rows_pay(int M, long columns, int K) {
   if (K % 128 != 0 || M > 8) return false;
   if (M == 1) return K > 4096 && columns > 512 && columns < 4096;
+  if (M == 2 && K % 8192 == 0 && columns > 12288) return false;
   if (M <= 3) return K >= 4096 && columns > 512;
   return M > 4 || columns > 512 || K < 1024;
 }
@@ -655,7 +660,7 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
   if (!z_start && !a_rows && !w_f32 && lgs::lin_rows_pay(M, (long)N * batch, K) && lda % 4 == 0 && stride_a % 4 == 0 &&
       stride_w % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0) {
     if (N < 4096) lgs::lin_rows_go<1, 8>(p, batch, stream);
-    else if (M > 4 && (N >= 16384 || (N > 4096 && N < 8192))) lgs::lin_rows_go<2, 4>(p, batch, stream);
+    else if (M > 4 && (N >= 16384 || (N > 4096 && N < 8192 && K >= 2048))) lgs::lin_rows_go<2, 4>(p, batch, stream);
     else lgs::lin_rows_go<1, 4>(p, batch, stream);
     LGA_LAUNCH_RETURN();
   }

@@ -57,7 +57,7 @@ __device__ __forceinline__ void rows_products(unsigned char* lds_all, Weights&& 
     a[i] = (const unsigned char*)(x0 + (size_t)min(row, M - 1) * ldx) + 16 * ((lane & 31) ^ row);
   }
   auto dma = [&](int b, int slot) {  // (past the range: its last block, never used)
-    const size_t at = (size_t)max(min(b, b1 - 1), 0) * 256;
+    const size_t at = (size_t)min(b, b1 - 1) * 256;
 #pragma unroll
     for (int i = 0; i < PW; ++i) lga::gemm_dma16(w[i] + at, lds + slot + i * 1024);
 #pragma unroll
@@ -69,8 +69,10 @@ __device__ __forceinline__ void rows_products(unsigned char* lds_all, Weights&& 
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < NR; ++j) acc[i][j] = zero;
+  if (b0 < b1) {  // (fewer blocks than waves: those without one fetch nothing)
 #pragma unroll
-  for (int r = 0; r < RB; ++r) dma(b0 + r, r * SLOT);
+    for (int r = 0; r < RB; ++r) dma(b0 + r, r * SLOT);
+  }
   int slot = 0;
   const int arow = l15 & (MR - 1), w_at = l15 * 256, a_at = W_BYTES + arow * 512;
   for (int b = b0; b < b1; b += 2) {
@@ -89,7 +91,7 @@ __device__ __forceinline__ void rows_products(unsigned char* lds_all, Weights&& 
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before it is filled again)
         __builtin_amdgcn_sched_barrier(0);
-        dma(b + s + RB, slot);
+        if (RB > 1 || b + s + RB < b1) dma(b + s + RB, slot);  // (several are counted by the wait: one more always)
         slot = slot + SLOT == RB * SLOT ? 0 : slot + SLOT;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
