@@ -405,9 +405,13 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 }
 
 // One row: y = ((x2 W2^T + b2) + (x1 W1^T + b1)) + res, a wave per output, both products in f32_linear_kernel's order. Bound by
-// latency: the weights of a block of 768 columns beside 3072 are in flight at once, x2 and an attention's ranges ahead of them, so that
-// the join waits for nothing else; x2 is read once for a workgroup's four outputs. Two launches 13.7 us, one 8.0; with ranges to join
-// behind the weights 8.8, ahead of them 8.5.
+// latency: the weights of a block of 768 columns beside 3072 are in flight at once. Two launches 13.7 us, one 8.0. AHEAD: x2 and an
+// attention's ranges come ahead of the weights, so that the join waits for nothing else, and x2 is read once for a workgroup's four
+// outputs; the weights then start later, and a workgroup holds LDS, which rows of up to 3072 values make up for in a model's chain of
+// launches and longer ones do not (us a token behind 300 keys, weights first / AHEAD: pythia-160m 307.9 / 303.6, pythia-410m 694 / 742,
+// pythia-1b 1234 / 1318; alone, weights from memory, 768 columns beside 3072 7.4 / 8.2, 1024 beside 4096 9.7 / 12.5, 2048 beside 8192
+// 31.3 / 35.9).
+constexpr int kF32AheadMost = 3072;  // (values of x2)
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
   float* y;
@@ -470,18 +474,17 @@ __device__ __forceinline__ void f32_join_parts(const F32LinearsSum& a, const F32
   for (int i = threadIdx.x + 256 * E; i < a.K1; i += 256) join(i, [&](int s) { return a.x1[(size_t)s * a.K1 + i]; });
   __syncthreads();
 }
-// E2: 1024 values each of x2 that LDS takes (0: a longer row, read from memory by every wave)
-template <bool PARTS, int E2>
+template <bool PARTS, bool AHEAD>
 __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
   extern __shared__ __attribute__((aligned(16))) float xs[];  // [K1] the joined row, then the ranges' weights; or [K1]; x2
   const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), n = min(row, a.N - 1);
   const float *r1 = a.w1 + (size_t)n * a.K1, *r2 = a.w2 + (size_t)n * a.K2;
-  // the rows first, and what they wait for: the weights behind them arrive while they are joined
+  constexpr int E2 = AHEAD ? kF32AheadMost / 1024 : 0;
   float4 x2[E2 > 0 ? E2 : 1];
 #pragma unroll
   for (int e = 0; e < E2; ++e) x2[e] = *(const float4*)(a.x2 + min((int)(threadIdx.x + 256 * e) * 4, a.K2 - 4));
   F32Parts parts;
-  if (PARTS) f32_load_parts(a, parts);
+  if (PARTS && AHEAD) f32_load_parts(a, parts);
   __builtin_amdgcn_sched_barrier(0);
   float4 w1[kF32Chunks], w2[3][kF32Chunks];
   f32_load_chunks(r1, 0, a.K1, lane, w1);
@@ -489,8 +492,9 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
   for (int u = 0; u < 3; ++u) f32_load_chunks(r2, u * kF32Chunks, a.K2, lane, w2[u]);
   const float b1 = a.b1 ? a.b1[n] : 0.0f, b2 = a.b2 ? a.b2[n] : 0.0f, res = a.res[n];
   __builtin_amdgcn_sched_barrier(0);
+  if (PARTS && !AHEAD) f32_load_parts(a, parts);
   const float *px1 = a.x1, *px2 = a.x2;
-  if (E2 > 0) {
+  if (AHEAD) {
     float* to = xs + (PARTS ? a.K1 + (a.K1 / a.hs * 9 + 3) / 4 * 4 : 0);
 #pragma unroll
     for (int e = 0; e < E2; ++e) {
@@ -502,7 +506,7 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
   if (PARTS) {
     f32_join_parts(a, parts, xs, xs + a.K1);
     px1 = xs;
-  } else if (E2 > 0) {
+  } else if (AHEAD) {
     __syncthreads();
   }
   float4 h4 = make_float4(0.f, 0.f, 0.f, 0.f), m4 = h4;
@@ -860,17 +864,10 @@ extern "C" int lga_f32_linears_sum(const float* x1, const float* ml, int parts, 
                 "lga_f32_linears_sum: 1 to 8 ranges of up to 256 heads, 8192 columns");
   const lga::F32LinearsSum a{x1, w1, b1, x2, w2, b2, residual, y, N, K1, K2, ml, parts, hs};
   const size_t joined = parts > 1 ? (size_t)K1 + (K1 / hs * 9 + 3) / 4 * 4 : 0;
-  const unsigned grid = (N + 3) / 4;
-#define LGA_SUM(E2)                                                                                                          \
-  do {                                                                                                                        \
-    const size_t lds = (joined + (E2 > 0 ? K2 : 0)) * sizeof(float);                                                         \
-    if (parts > 1) lga::f32_linears_sum_kernel<true, E2><<<grid, 256, lds, stream>>>(a);                                     \
-    else lga::f32_linears_sum_kernel<false, E2><<<grid, 256, lds, stream>>>(a);                                              \
-  } while (0)
-  if ((joined + K2) * sizeof(float) > 65536 || K2 > 8192) LGA_SUM(0);
-  else if (K2 <= 3072) LGA_SUM(3);
-  else LGA_SUM(8);
-#undef LGA_SUM
+  const bool ahead = K2 <= lga::kF32AheadMost;
+  const size_t lds = (joined + (ahead ? K2 : 0)) * sizeof(float);
+  (parts > 1 ? (ahead ? lga::f32_linears_sum_kernel<true, true> : lga::f32_linears_sum_kernel<true, false>)
+             : (ahead ? lga::f32_linears_sum_kernel<false, true> : lga::f32_linears_sum_kernel<false, false>))<<<(N + 3) / 4, 256, lds, stream>>>(a);
   LGA_LAUNCH_RETURN();
 }
 
