@@ -697,10 +697,11 @@ __global__ void __launch_bounds__(256) latent_attention_vec_kernel(LatAttArgs p,
 // while these are worked on. Bound by latency, of which short caches are nothing else: a range without keys says so and leaves its row
 // alone, values of lanes past a row are zeros instead of branches around each product, and the waves' sums are read and stored four
 // columns a lane; with the combination's columns side by side none of 24 forms of 1 to 16 tokens of 4 to 64 heads is slower than a head
-// a workgroup. us of that, with a wave sum through LDS per key and head, / here with branches, stores of a column and every range
-// written / here, both launches, rows of 512 + 64 from caches: one token of 8 heads over one 8.4 / 10.6 / 7.5, over 64 8.6 / 10.8 /
-// 8.7, over 600 11.1 / 12.7 / 10.3, over 2000 21.5 / 16.1 / 13.8; of 16 over five 9.5 / 10.9 / 7.9, over 2000 23.2 / 16.9 / 14.8; of 64
-// over 64 12.4 / 10.3 / 8.8; eight of 16 over five 10.7 / 8.1 / 7.1, over 2000 65 / 32.8 / 30.9; 3 of 32 over 600 21.9 / 15.8 / 13.9.
+// a workgroup, but for 17 to 24 tokens' 32 heads over caches of up to 30 rows, which take a second launch (20 over one 6.9 / 8.6). us of
+// that, with a wave sum through LDS per key and head, / here with branches, stores of a column and every range written / here, both
+// launches, rows of 512 + 64 from caches: one token of 8 heads over one 8.4 / 10.6 / 7.5, over 64 8.6 / 10.9 / 8.3, over 600 11.1 / 12.5 /
+// 10.1, over 2000 21.5 / 16.2 / 13.6; of 16 over five 9.5 / 10.9 / 7.8, over 2000 23.2 / 16.9 / 14.8; of 64 over 64 12.4 / 12.1 / 10.0;
+// eight of 16 over five 10.7 / 9.2 / 7.3, over 2000 65 / 34.7 / 32.6; 3 of 32 over 600 21.9 / 16.8 / 14.8.
 template <int CTRL>
 __device__ __forceinline__ float lat_dpp_add(float v) {
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));

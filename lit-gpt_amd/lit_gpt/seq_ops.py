@@ -334,9 +334,10 @@ def latent_attention(qc: torch.Tensor, proj: torch.Tensor, q_off: int, cache_c: 
         raise ValueError("latent_attention: shapes")
     out = torch.empty(T, H * r, dtype=F32, device=proj.device)
     if splits is None:
-        # (1536, with four heads a workgroup: one token of 64 heads over 64 rows 8.8 -> 10.0 us, eight of 16 7.6 -> 8.5, 20 of
-        # 32, which then take a second launch, 10.1 -> 13.1; from 600 rows on 61 -> 52 there, one to two in a hundred elsewhere)
-        splits = max(1, min(32, 1024 // (T * H)))
+        # (four heads a workgroup take half as many ranges more: the longest sequence of a step is worked on to its end. us of 1024 /
+        # 1536: 19 tokens of 32 heads over 3 to 1500 rows 257 / 151, six of 16 over 2 to 1305 19.5 / 16.6; where all are short, 20 of 32
+        # over 64 rows 10.1 / 13.1)
+        splits = max(1, min(32, (1024 if H % 4 else 1536) // (T * H)))
         if window > 0:  # at least one key per wave of a split
             splits = max(1, min(splits, window // 4))
     part = torch.empty(T * H * splits * (r + 2), dtype=F32, device=proj.device) if splits > 1 else None
