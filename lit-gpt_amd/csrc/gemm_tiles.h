@@ -282,6 +282,10 @@ inline GemmPlan gemm_whole_plan(int M, int N, int K, int batch, bool grouped, in
 // the chip's idle part. Of 1491 products of 33 to 2600 rows, weights from memory, it is 1.1 % from the fastest form in the mean, and
 // the form that counts whole tiles 2.0 %. us of whole tiles alone / here: 2407 x 20608 x 4096 448 / 381, 517 x 11008 x 4096 with SwiGLU
 // 109 / 101, 40 rows of it 37 / 33.
+// Rows as the tile's B: at least nine steps, and a fortieth gained, or else the form that counts whole tiles. (Ends of tiles are most
+// of shorter products, and of 64 x 128 they are less than the sums here say: 990 products for which the two choose otherwise, the sums' choice
+// alone 1.04 times the time of whole tiles' for plain ones, 1.06 for gated units, with the line 0.99 and 0.99; 120 x 768 x 3072 10.8 / 12.1, 2849
+// x twice 5524 x 512 53 / 62. Rows as A 0.93, at every length.)
 // A grouped product's short tiles stand beside the whole ones of their columns, whose weights they would otherwise fetch anew (16 groups of
 // 278 rows of twice 2752 x 4096 302 behind, 260 beside): 480 products of 8 to 18 groups, 144 to 16384 rows in all, weights from memory,
 // take 0.93 of the time that whole tiles took (gated units 0.98), none more than 3 % more. (Weights that stay in the last cache from
@@ -290,14 +294,17 @@ inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int
   GemmPlan best{-1, 1};
   if (grouped) return gemm_whole_plan(M, N, K, batch, true, ksplit, flags);
   if (K % 64 != 0 || M <= 0) return best;
-  best.ksplit = ksplit > 0 ? ksplit : batch > 1 ? 1 : gemm_whole_plan(M, N, K, 1, false, 0, flags).ksplit;
+  const bool rows_b = flags & kGemmRowsB;
+  if (rows_b || (ksplit <= 0 && batch == 1)) best = gemm_whole_plan(M, N, K, batch, false, ksplit, flags);
+  else best.ksplit = ksplit > 0 ? ksplit : 1;
   const int steps = K / 64, per = (steps + best.ksplit - 1) / best.ksplit, count = batch * ((steps + per - 1) / per);
-  float best_us = 0.0f;
+  if (rows_b && per < 9) return best;
+  const int kept = best.tile;
+  float best_us = 0.0f, kept_us = 0.0f;
 #pragma unroll
   for (int f = 0; f < kGemmFormCount; ++f) {
     const GemmForm& t = kGemmForms[f];
     if (!gemm_form_fits(t, flags)) continue;
-    const bool rows_b = flags & kGemmRowsB;
     const int rows = rows_b ? t.bn : t.bm, cols = rows_b ? t.bm : t.bn, frags = rows_b ? t.fn : t.fm, step = rows / frags;
     const float most = t.bm * t.bn > 128 * 192 ? 0.69f : 0.46f;  // (of what fewer workgroups gain: 0.7 and 0.5 above, fitted anew on these products)
     auto round = [&](float load) { return per * std::max(t.fast_us, t.step_us * (1.0f - most * (1.0f - load))) + t.round_us; };
@@ -315,7 +322,9 @@ inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int
     }
     if (shorts > 0.0f) us += each * gemm_ceil(shorts / slots) * round(std::min(shorts / slots, 1.0f) * each);
     if (best_us == 0.0f || us < best_us) best_us = us, best.tile = f;
+    if (f == kept) kept_us = us;
   }
+  if (rows_b && best_us > 0.975f * kept_us) best.tile = kept;
   return best;
 }
 
