@@ -251,7 +251,8 @@ __device__ __forceinline__ int swz(int row, int chunk) { return row * 128 + 16 *
 
 // VEC: K % 8 == 0 and 16-B aligned rows of A and W (vector loads); otherwise element loads with k guards.
 // A16: A arrives as bf16 (half the operand traffic of the fp32 stream; the same values the fp32 path would round to)
-template <bool VEC, bool A16>
+// NARROW: up to 18 columns (a router's)
+template <bool VEC, bool A16, bool NARROW>
 __global__ void __launch_bounds__(256) lin_mfma_kernel(LinArgs p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * 2 * TILE_BYTES];  // [buf][A|W]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -361,8 +362,35 @@ __global__ void __launch_bounds__(256) lin_mfma_kernel(LinArgs p) {
     __syncthreads();
   }
 
+  if constexpr (NARROW) {  // as the accumulators lie, and only those that hold columns
+    if (wn > 0) return;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int n = j * 16 + fr;
+      if (n >= p.N) continue;
+      const float bias = p.bias ? p.bias[n] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + wm * 64 + i * 16 + fk * 4 + r;
+          if (m >= Mz) continue;
+          if (p.ksplit > 1) {
+            p.part[((size_t)blockIdx.z * p.M + m) * p.N + n] = acc[i][j][r];
+            continue;
+          }
+          const size_t at = (size_t)z * p.sy + (size_t)(r_lo + m) * p.ldy + n;
+          const float v = act_f(p.act, acc[i][j][r] + bias);
+          if (p.y16) p.y16[at] = f2bf(v);
+          else p.y[at] = p.accumulate ? p.y[at] + v : v;
+        }
+    }
+    return;
+  }
   // a wave turns 32 rows of its 64 x 64 results at a time in LDS of its own and stores them four columns a lane, 256 bytes of a row
-  // together (as the accumulators lie, 64: 2048 x 2048 x 64, all of it results, 22.0 -> 13.4 us)
+  // together (as the accumulators lie, 64: 2048 x 2048 x 64, all of it results, 22.0 -> 13.4 us; of a few columns most of that would be work
+  // for none, us turned / as they lie: 1725 x 16 x 512 into sums 25.0 / 19.1, 2048 x 16 x 2048 60.5 / 54.6, 300 x 18 x
+  // 2048 61.0 / 58.3, 58 x 16 x 64 8.7 / 6.5, 1211 x 20 x 64 9.5 / 11.0)
   constexpr int RS = 68;
   float* turned = (float*)(lds + wave * 16384);
   const int c4 = fr * 4, n = n0 + wn * 64 + c4, cols = p.N - n;
@@ -722,13 +750,16 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
   }
   const dim3 grid((N + lgs::BN - 1) / lgs::BN, (M + lgs::BM - 1) / lgs::BM, p.ksplit > 1 ? p.ksplit : batch);
   LGA_CHECK_ARG(grid.y <= 65535, "lgs_linear: too many rows");
-  if (a_bf16) {
-    if (vec) lgs::lin_mfma_kernel<true, true><<<grid, 256, 0, stream>>>(p);
-    else lgs::lin_mfma_kernel<false, true><<<grid, 256, 0, stream>>>(p);
-  } else {
-    if (vec) lgs::lin_mfma_kernel<true, false><<<grid, 256, 0, stream>>>(p);
-    else lgs::lin_mfma_kernel<false, false><<<grid, 256, 0, stream>>>(p);
-  }
+#define LGS_MFMA(NARROW)                                                                    \
+  do {                                                                                      \
+    if (a_bf16 && vec) lgs::lin_mfma_kernel<true, true, NARROW><<<grid, 256, 0, stream>>>(p); \
+    else if (a_bf16) lgs::lin_mfma_kernel<false, true, NARROW><<<grid, 256, 0, stream>>>(p); \
+    else if (vec) lgs::lin_mfma_kernel<true, false, NARROW><<<grid, 256, 0, stream>>>(p);   \
+    else lgs::lin_mfma_kernel<false, false, NARROW><<<grid, 256, 0, stream>>>(p);           \
+  } while (0)
+  if (N <= 18) LGS_MFMA(true);
+  else LGS_MFMA(false);
+#undef LGS_MFMA
   if (p.ksplit > 1) lgs::lin_sum_kernel<<<dim3((N + 255) / 256, M), 256, 0, stream>>>(p);
   LGA_LAUNCH_RETURN();
 }

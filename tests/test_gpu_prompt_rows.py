@@ -110,7 +110,7 @@ def test_queries_and_keys(T, H, G, d, dv, rot, interleaved):
     assert (k[0] == 7).all() and (k[1, :2] == 7).all() and (k[1, T + 2:] == 7).all() and (v[0] == 7).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(9, 1, 8), (130, 131, 64), (300, 513, 72), (128, 128, 64), (257, 66, 136)])
+@pytest.mark.parametrize("M,N,K", [(9, 1, 8), (130, 131, 64), (300, 513, 72), (128, 128, 64), (257, 66, 136), (129, 16, 72), (70, 18, 64), (140, 19, 64)])
 @pytest.mark.parametrize("kind", ["fp32", "bf16", "sums"])
 @pytest.mark.parametrize("ldy", [0, 1])
 def test_products_of_fp32_rows(M, N, K, kind, ldy):
