@@ -55,8 +55,8 @@ __device__ __forceinline__ float cload(const void* c, size_t i) {
   return CF32 ? ((const float*)c)[i] : bf2f(((const uint16_t*)c)[i]);
 }
 
-// grid (T, parts): threads walk (vector, pair) items: 2 H query maps, then 2 G key maps, then the value columns
-template <bool CF32>
+// grid (T, parts; ONE: T): threads walk (vector, pair) items: 2 H query maps, then 2 G key maps, then the value columns
+template <bool CF32, bool ONE>
 __global__ void __launch_bounds__(256) diffattn_prepare_kernel(AttnPrepArgs p) {
   const size_t t = blockIdx.x;
   const int pos = p.pos[t];
@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) diffattn_prepare_kernel(AttnPrepArgs p) {
   const int d = p.d, half = d / 2 + (d & 1), rp = p.rot_dims / 2;
   const int nq = 2 * p.H * half, nk = p.k_off >= 0 ? 2 * p.G * half : 0;
   const size_t crow = ((size_t)p.slot[t] * p.S + pos) * p.G;
-  const int first = threadIdx.x + 256 * blockIdx.y, step = 256 * gridDim.y;
+  const int first = threadIdx.x + (ONE ? 0 : 256 * blockIdx.y), step = ONE ? 256 : 256 * gridDim.y;
   for (int it = first; it < nq + nk; it += step) {
     const bool isk = it >= nq;
     const int e = isk ? it - nq : it;
@@ -132,12 +132,12 @@ __device__ __forceinline__ void pool_block(const void* cache_k, const void* cach
   }
 }
 
-// grid (T, parts; 1 with a joint norm or pooled blocks): the waves take the vectors in turn, those of the H query heads (normed, rotated
+// grid (T, parts; ONE: T, so with a joint norm or pooled blocks): the waves take the vectors in turn, those of the H query heads (normed, rotated
 // and multiplied by the
 // position's query temperature, in place) and of the G key heads (normed and rotated on their way into the cache);
 // then all threads copy the values into the cache. The value columns may be the key columns themselves (values = the
 // keys as projected): the keys are never changed in place.
-template <bool CF32>
+template <bool CF32, bool ONE>
 __global__ void __launch_bounds__(256) normattn_prepare_kernel(NormPrepArgs p) {
   __shared__ float red[4];
   const size_t t = blockIdx.x;
@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(256) normattn_prepare_kernel(NormPrepArgs p) {
     kf = 1.0f / sqrtf(sk / (float)(p.G * d) + p.eps);
   }
   const int st = p.interleaved ? 2 : 1, mate = p.interleaved ? 1 : half;  // pair i: elements st i and st i + mate
-  for (int vec = wave + 4 * blockIdx.y; vec < p.H + p.G; vec += 4 * gridDim.y) {
+  for (int vec = wave + (ONE ? 0 : 4 * blockIdx.y); vec < p.H + p.G; vec += ONE ? 4 : 4 * gridDim.y) {
     const bool isk = vec >= p.H;
     float* x = row + (isk ? p.k_off + (size_t)(vec - p.H) * d : p.q_off + (size_t)vec * d);
     const float* w = isk ? p.k_w : p.q_w;
@@ -198,7 +198,8 @@ __global__ void __launch_bounds__(256) normattn_prepare_kernel(NormPrepArgs p) {
       else x[i] = u;
     }
   }
-  const int nv = p.G * p.dv, first = threadIdx.x + 256 * blockIdx.y, step = 256 * gridDim.y;
+  if (ONE) __syncthreads();  // (the values' columns side by side, not each wave's when it is through)
+  const int nv = p.G * p.dv, first = threadIdx.x + (ONE ? 0 : 256 * blockIdx.y), step = ONE ? 256 : 256 * gridDim.y;
   if (p.v_freq) {
     const int hv = p.dv / 2, vmate = p.interleaved ? 1 : hv;
     for (int i = first; i < p.G * hv; i += step) {
@@ -768,10 +769,14 @@ extern "C" int lgs_diffattn_prepare(float* proj, long ld, int q_off, int k_off, 
                 "lgs_diffattn_prepare: keys or values outside the row");
   lgs::AttnPrepArgs p{proj, ld, q_off, k_off, v_off, cache_k, cache_v, inv_freq, slot, pos, H, G, d, dv, rot_dims, max_seq};
   const long items = ((long)H + (k_off >= 0 ? G : 0)) * 2 * (d / 2 + (d & 1));
-  // (a thread an item: 3 tokens of 32 + 8 heads 7.1 -> 2.3 us, 2407 25.9 -> 23.0)
-  const dim3 grid(T, (unsigned)std::min((items + 255) / 256, 65535L));
-  if (cache_f32) lgs::diffattn_prepare_kernel<true><<<grid, 256, 0, stream>>>(p);
-  else lgs::diffattn_prepare_kernel<false><<<grid, 256, 0, stream>>>(p);
+  // A thread an item (us of one workgroup a token / here: 3 tokens of 32 + 8 heads 7.1 / 2.3, 2407 25.5 / 22.2); of prompts no workgroup for
+  // the last few, and one a token where the chip holds nearly all at once or there is no angle to wait for (4096 tokens 33.0 / 35.1, 2000 not
+  // rotated 16.6 / 18.0, of 8 + 2 heads of 32 4.3 / 4.7)
+  const long parts = T <= 640 ? (items + 255) / 256 : T > 3500 || (rot_dims == 0 && T > 900) ? 1 : std::max(items / 256, 1L);
+  const dim3 grid(T, (unsigned)std::min(parts, 65535L));
+  const bool one = grid.y == 1;
+  (cache_f32 ? (one ? lgs::diffattn_prepare_kernel<true, true> : lgs::diffattn_prepare_kernel<true, false>)
+             : (one ? lgs::diffattn_prepare_kernel<false, true> : lgs::diffattn_prepare_kernel<false, false>))<<<grid, 256, 0, stream>>>(p);
   LGA_LAUNCH_RETURN();
 }
 
@@ -828,9 +833,13 @@ extern "C" int lgs_normattn_prepare(float* proj, long ld, int q_off, int k_off, 
                       pool_rows};
   // A wave's vectors wait for one another: few tokens' get waves of their own, up to 4096 workgroups (us of one workgroup per token / here:
   // 8 tokens of 16 + 4 heads 7.2 / 3.2, 3 of 32 + 8 15.2 / 3.5, 300 of 16 + 4 7.9 / 4.9; five workgroups a token at 2048 19.7 / 20.1)
-  const dim3 grid(T, norm == 2 || pool > 0 ? 1 : std::min((H + G + 3) / 4, std::max(4096 / T, 1)));
-  if (cache_f32) lgs::normattn_prepare_kernel<true><<<grid, 256, 0, stream>>>(p);
-  else lgs::normattn_prepare_kernel<false><<<grid, 256, 0, stream>>>(p);
+  // Not where there is little to do beside the copies, nor for prompts whose workgroups of one a token the chip holds at once and of three
+  // it does not (8 + 8 heads of 64, neither normed nor rotated, 900 tokens 5.0 / 6.0; 16 + 4 of 128, rotated, 1300 10.5 / 11.2, 700 8.4 / 7.6)
+  const bool few = norm == 0 && rot_dims == 0 && (H + G) * d < 2560 && T > 512, held = T > 1024 && T < 1700 && (norm == 0 || rot_dims == 0);
+  const dim3 grid(T, norm == 2 || pool > 0 || few || held ? 1 : std::min((H + G + 3) / 4, std::max(4096 / T, 1)));
+  const bool one = grid.y == 1;
+  (cache_f32 ? (one ? lgs::normattn_prepare_kernel<true, true> : lgs::normattn_prepare_kernel<true, false>)
+             : (one ? lgs::normattn_prepare_kernel<false, true> : lgs::normattn_prepare_kernel<false, false>))<<<grid, 256, 0, stream>>>(p);
   LGA_LAUNCH_RETURN();
 }
 
