@@ -418,10 +418,13 @@ __global__ void __launch_bounds__(256) moe_up_shared_kernel(const float* __restr
   });
 }
 
-// Several tokens, an expert of 8 MB and more (below, the look at the pairs costs what the second reading does) and few enough experts that
-// tokens share some
+// Several tokens, an expert of 8 MB and more (below, the look at the pairs costs what the second reading does), few enough experts that
+// tokens share some, and as many pairs as make up for those that have an expert alone (us, a pair at a time / shared, experts of 2 x 1408 x
+// 2048: 3 tokens of two of 8 9.2 / 11.4, 4 of two 14.8 / 13.2; 5 of two of 16 18.5 / 19.3, 6 of two 21.3 / 18.5; of 2 x 2816 x 2048 4 of one of 16
+// 15.6 / 16.0, 3 of two 21.0 / 19.4; of 2 x 2752 x 4096 3 of one of 16 21.7 / 21.7)
 static bool moe_up_shares(int T, int top, long bytes, int n_real) {
-  return T > 1 && T * top <= 64 && bytes >= 8 << 20 && n_real <= 4 * T * top;
+  const int pairs = T * top;
+  return T > 1 && pairs <= 64 && bytes >= 8 << 20 && n_real <= 4 * pairs && bytes * pairs >= (n_real <= 8 ? 80L : 128L) << 20;
 }
 
 // Counting sort of the pairs by expert in three launches. ws: 2 E ints (counts, cursors), zero on entry.

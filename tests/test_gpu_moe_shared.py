@@ -1,6 +1,6 @@
 """Experts of steps with few tokens: several tokens at once give the bits that each token has alone (csrc/seq_ffn.hip:
-moe_up_shared_kernel), at one to all choices of an expert, identity experts, odd sizes, and on both sides of 24 pairs, of 64, of 8 MB
-an expert and of four experts a pair."""
+moe_up_shared_kernel), at one to all choices of an expert, identity experts, odd sizes, and on both sides of 24 pairs, of 64, of the bytes
+of all pairs from which they share and of four experts a pair."""
 
 import pytest
 import torch
