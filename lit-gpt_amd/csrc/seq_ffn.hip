@@ -546,7 +546,8 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const float* __restric
 }
 
 // The same, four columns a thread and the rows of four choices on their way together: 2048 tokens' 4 of 2048 columns 15.7 us (24.4 a column
-// a thread, row after row), 4096 29.6 (42.2)
+// a thread, row after row), 4096 29.6 (42.2); of one or two choices from 200000 values on (one of 64 tokens of 2048 2.14 us a column a thread,
+// 2.31 here, of 100 2.33 either way)
 __global__ void __launch_bounds__(256) moe_combine4_kernel(const float* __restrict__ y, const int* __restrict__ where,
                                                            const float* __restrict__ wts, float* __restrict__ x, long ldx,
                                                            int top, int N, const int* __restrict__ ids, int n_real,
@@ -742,7 +743,7 @@ extern "C" int lgs_moe_combine(const float* y, const int* where, const float* wt
                                hipStream_t stream) {
   LGA_CHECK_ARG(y && where && wts && x && T > 0 && T <= 65535 && top > 0 && N > 0, "lgs_moe_combine: bad arguments");
   LGA_CHECK_ARG(!ids || hin, "lgs_moe_combine: identity experts need the tokens' inputs");
-  if (N % 4 == 0 && ldx % 4 == 0 && (!ids || ldh % 4 == 0) && ((uintptr_t)y | (uintptr_t)x | (uintptr_t)(ids ? hin : nullptr)) % 16 == 0) {
+  if ((top > 2 || (long)T * N >= 200000) && N % 4 == 0 && ldx % 4 == 0 && (!ids || ldh % 4 == 0) && ((uintptr_t)y | (uintptr_t)x | (uintptr_t)(ids ? hin : nullptr)) % 16 == 0) {
     lgs::moe_combine4_kernel<<<dim3((N / 4 + 255) / 256, T), 256, 0, stream>>>(y, where, wts, x, ldx, top, N, ids, n_real, hin, ldh,
                                                                                 accumulate);
     LGA_LAUNCH_RETURN();

@@ -59,7 +59,7 @@ def test_sorted_pairs(T, top, E):
         assert torch.equal(torch.searchsorted(start[1:].contiguous(), place, right=True).int(), ids.flatten()[pair.long()])
 
 
-@pytest.mark.parametrize("T,top,N", [(33, 4, 2048), (5, 1, 4), (17, 3, 2052), (9, 9, 1028), (7, 4, 2050), (3, 5, 31)])
+@pytest.mark.parametrize("T,top,N", [(33, 4, 2048), (5, 1, 4), (17, 3, 2052), (9, 9, 1028), (7, 4, 2050), (3, 5, 31), (97, 2, 2064), (96, 1, 2084)])
 @pytest.mark.parametrize("identity", [False, True])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_combined_pairs(T, top, N, identity, accumulate):
