@@ -1140,7 +1140,8 @@ extern "C" int lgs_head_gate(float* o, const float* g, long ldg, int T, int H, i
                              int g2_f32, hipStream_t stream) {
   LGA_CHECK_ARG(o && g && T > 0 && H > 0 && H <= 65535 && dv > 0 && (!w_g2 || (rank > 0 && rank <= 512)),
                 "lgs_head_gate: bad arguments (inner size of a low-rank gate 1..512)");
-  if (dv == 128 && (long)T * H >= 4096 && (!w_g2 || rank % 8 == 0)) {  // (values of a map one by one: 260 tokens of 16 heads, rank 20, 6.0 / 6.7)
+  if (dv == 128 && (long)T * H >= 4096 && (!w_g2 || rank % 8 == 0 || (long)T * H >= 5600)) {
+    // (off eight a map's values come one by one: 260 tokens of 16 heads, rank 20, 6.0 / 6.7, 362 9.2 / 8.1, 1975 of 32 80 / 46)
     const dim3 grid((T + lgs::kGateTokens - 1) / lgs::kGateTokens, H);
     const size_t lds = w_g2 ? (size_t)lgs::kGateTokens * rank * sizeof(float) : 0;
     if (g2_f32)
