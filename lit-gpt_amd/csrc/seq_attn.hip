@@ -771,8 +771,8 @@ extern "C" int lgs_diffattn_prepare(float* proj, long ld, int q_off, int k_off, 
   const long items = ((long)H + (k_off >= 0 ? G : 0)) * 2 * (d / 2 + (d & 1));
   // A thread an item (us of one workgroup a token / here: 3 tokens of 32 + 8 heads 7.1 / 2.3, 2407 25.5 / 22.2); of prompts no workgroup for
   // the last few, and one a token where the chip holds nearly all at once or there is no angle to wait for (4096 tokens 33.0 / 35.1, 2000 not
-  // rotated 16.6 / 18.0, of 8 + 2 heads of 32 4.3 / 4.7)
-  const long parts = T <= 640 ? (items + 255) / 256 : T > 3500 || (rot_dims == 0 && T > 900) ? 1 : std::max(items / 256, 1L);
+  // rotated 16.6 / 18.0, of 8 + 2 heads of 32 4.3 / 4.7; heads of 128 gain all the same, 1026 not rotated 20.8 / 18.4)
+  const long parts = T <= 640 ? (items + 255) / 256 : T > 3500 || (rot_dims == 0 && d < 128 && T > 900) ? 1 : std::max(items / 256, 1L);
   const dim3 grid(T, (unsigned)std::min(parts, 65535L));
   const bool one = grid.y == 1;
   (cache_f32 ? (one ? lgs::diffattn_prepare_kernel<true, true> : lgs::diffattn_prepare_kernel<true, false>)
@@ -834,8 +834,10 @@ extern "C" int lgs_normattn_prepare(float* proj, long ld, int q_off, int k_off, 
   // A wave's vectors wait for one another: few tokens' get waves of their own, up to 4096 workgroups (us of one workgroup per token / here:
   // 8 tokens of 16 + 4 heads 7.2 / 3.2, 3 of 32 + 8 15.2 / 3.5, 300 of 16 + 4 7.9 / 4.9; five workgroups a token at 2048 19.7 / 20.1)
   // Not where there is little to do beside the copies, nor for prompts whose workgroups of one a token the chip holds at once and of three
-  // it does not (8 + 8 heads of 64, neither normed nor rotated, 900 tokens 5.0 / 6.0; 16 + 4 of 128, rotated, 1300 10.5 / 11.2, 700 8.4 / 7.6)
-  const bool few = norm == 0 && rot_dims == 0 && (H + G) * d < 2560 && T > 512, held = T > 1024 && T < 1700 && (norm == 0 || rot_dims == 0);
+  // it does not (8 + 8 heads of 64, neither normed nor rotated, 900 tokens 5.0 / 6.0, 32 + 32 of 128, 1219 27.9 / 31.3; 16 + 4 of 128,
+  // rotated, 1300 10.5 / 11.2, 700 8.4 / 7.6; but 32 + 32 of 128, rotated, 1544 42.3 / 36.1)
+  const bool bare = norm == 0 && rot_dims == 0, few = bare && T > ((H + G) * d < 2560 ? 512 : 1024);
+  const bool held = !bare && T > 1024 && T < 1700 && (H + G) * d <= 2560 && (norm == 0 || rot_dims == 0);
   const dim3 grid(T, norm == 2 || pool > 0 || few || held ? 1 : std::min((H + G + 3) / 4, std::max(4096 / T, 1)));
   const bool one = grid.y == 1;
   (cache_f32 ? (one ? lgs::normattn_prepare_kernel<true, true> : lgs::normattn_prepare_kernel<true, false>)
