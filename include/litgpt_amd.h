@@ -84,6 +84,8 @@ size_t lga_q4f_workspace_bytes(int M, int N, int K, int swiglu);
  * to be zero (else it need be neither cleared nor kept), the bits above the workspace's bytes. A matter of the sizes and the format
  * alone: a larger workspace changes nothing. */
 size_t lga_q4f_plan(int M, int N, int K, int swiglu, int fmt);
+/* of form 2 the tile (its number among the forms of csrc/gemm_tiles.h) and, behind eight bits, the ranges of K; -1: another form */
+int lga_bf16_gemm_form(int M, int N, int K, int swiglu);
 int lga_q4_gemm_fused(const void* x, const void* weight, const void* scales, const void* bias, const void* residual,
                       void* y, int M, int N, int K, int group, int fmt, void* workspace, size_t workspace_bytes,
                       lga_stream_t stream);

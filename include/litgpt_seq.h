@@ -61,6 +61,9 @@ int lgs_linear_glu_row(const float* a, const void* w, long up_rows, float* y, in
                        float limit, float shift, lgs_stream_t stream);
 /* ranges of K that a plain product of a bf16 A on bf16 weights (M > 8 rows) is best made in; 1: as one */
 int lgs_linear_ksplit(int M, int N, int K);
+/* the tile (its number among the forms of csrc/gemm_tiles.h) that a product of a bf16 A on bf16 weights is made with, by ksplit ranges
+ * of K, or with gated != 0 the unit of lgs_linear_glu of N columns; -1: not on those tiles */
+int lgs_linear_form(int M, int N, int K, int batch, int grouped, int ksplit, int act, int gated);
 /* x[t] = table[tokens[t]] * scale */
 int lgs_embed(const int* tokens, const void* table, int w_f32, float scale, float* x, int T, int W, int vocab,
               lgs_stream_t stream);

@@ -95,6 +95,13 @@ GemmPlan bf16_plan(int M, int N, int K, bool dual) {
   return gemm_tile_plan(M, (int)cols, K, 1, false, full ? 1 : 0, kGemmRowsB | (dual ? kGemmPairs : 0));
 }
 
+// (its number among the forms, and behind eight bits the ranges of K; -1: not on these tiles)
+extern "C" int lga_bf16_gemm_form(int M, int N, int K, int swiglu) {
+  if (M <= 0 || N <= 0 || K <= 0) return -1;
+  const GemmPlan p = bf16_plan(M, N, K, swiglu != 0);
+  return p.tile < 0 ? -1 : p.tile | p.ksplit << 8;
+}
+
 size_t bf16_workspace(const GemmPlan& p, int M, int N, bool dual) {
   return p.ksplit > 1 ? 4096 + (size_t)p.ksplit * (dual ? 2 : 1) * M * N * 4 : 0;
 }

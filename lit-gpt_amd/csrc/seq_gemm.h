@@ -28,6 +28,7 @@ struct LinArgs {
 // -1: not one of theirs (K is no multiple of 64). Rows of A and W start on 16 bytes. ksplit 0: the plan's own choice.
 using lga::GemmPlan;
 GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act = kActNone);
+GemmPlan gemm_glu_plan(int M, int n, int K, int batch, bool grouped);
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream);
 
 // A grouped product whose list is one tile of lgs_linear's older kernel and whose groups have two rows or less: that kernel

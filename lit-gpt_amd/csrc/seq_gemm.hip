@@ -312,12 +312,16 @@ static int glu_go(const LinArgs& p, const GluForm& f, int batch, hipStream_t str
   return 0;
 }
 
+GemmPlan gemm_glu_plan(int M, int n, int K, int batch, bool grouped) {
+  return lga::gemm_tile_plan(M, 2 * n, K, batch, grouped, 1, lga::kGemmRowsB | lga::kGemmPairs);
+}
+
 int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t stream) {
 #define LGS_CASE(I, SLOTS, US, FAST, ROUND, ...)                                     \
   case I:                                                                            \
     if constexpr (lga::kGemmForms[I].fm % 2 == 0) return glu_go<__VA_ARGS__>(p, f, batch, stream); \
     break;
-  const GemmPlan plan = lga::gemm_tile_plan(p.M, 2 * p.N, p.K, batch, p.z_start != nullptr, 1, lga::kGemmRowsB | lga::kGemmPairs);
+  const GemmPlan plan = gemm_glu_plan(p.M, p.N, p.K, batch, p.z_start != nullptr);
   switch (plan.tile) { LGA_GEMM_FORMS(LGS_CASE) }
 #undef LGS_CASE
   lga_set_error("lgs_linear_glu: no such form");

@@ -817,6 +817,12 @@ extern "C" int lgs_linear_glu_row(const float* a, const void* w, long up_rows, f
 extern "C" int lgs_linear_ksplit(int M, int N, int K) {
   return M > 8 && M <= 65535 && N > 0 && K > 0 ? lgs::gemm_plan(M, N, K, 1, false, 0).ksplit : 1;
 }
+// the tile (LGA_GEMM_FORMS) that such a product is made with, by ksplit ranges of K or (gated) with its unit; -1: none of them
+extern "C" int lgs_linear_form(int M, int N, int K, int batch, int grouped, int ksplit, int act, int gated) {
+  if (M <= 8 || N <= 0 || K <= 0 || batch <= 0 || ksplit <= 0) return -1;
+  if (gated) return glu_served(M, N, K) ? lgs::gemm_glu_plan(M, N, K, batch, grouped != 0).tile : -1;
+  return lgs::gemm_plan(M, N, K, batch, grouped != 0, ksplit, act).tile;
+}
 
 extern "C" int lgs_embed(const int* tokens, const void* table, int w_f32, float scale, float* x, int T, int W,
                          int vocab, hipStream_t stream) {

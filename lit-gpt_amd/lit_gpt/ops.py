@@ -49,6 +49,7 @@ SIGNATURES = {
     "lga_q4f_fits": [_I, _I, _I, _I, _I],
     "lga_q4f_workspace_bytes": [_I, _I, _I, _I],
     "lga_q4f_plan": [_I, _I, _I, _I, _I],
+    "lga_bf16_gemm_form": [_I, _I, _I, _I],
     "lga_q4_gemm_fused": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P],
     "lga_q4_gemm_swiglu": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P],
     "lga_q4_dequantize": [_P, _P, _P, _I, _I, _I, _I, _P],

@@ -33,6 +33,7 @@ SIGNATURES = {
     "lgs_last_error_string": [],
     "lgs_linear": [_P, _L, _L, _P, _I, _L, _P, _L, _L, _I, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _P, _I, _P],
     "lgs_linear_ksplit": [_I, _I, _I],
+    "lgs_linear_form": [_I] * 8,
     "lgs_linear_glu_fits": [_I, _I, _I, _I],
     "lgs_linear_glu_row_fits": [_I, _I],
     "lgs_linear_glu_row": [_P, _P, _L, _P, _I, _I, _I, _I, _F, _F, _F, _P],

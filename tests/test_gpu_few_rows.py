@@ -60,3 +60,21 @@ def test_error_of_rows_together(M, N, K):
         errs[0] += float((y.double() - ref).square().mean())
         errs[1] += float((alone.double() - ref).square().mean())
     assert errs[0] ** 0.5 <= 1.015 * errs[1] ** 0.5
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 600, 4096), (4, 1030, 640), (5, 300, 128), (8, 4097, 2048), (8, 8193, 2176)])
+def test_values_that_are_not_ordinary(M, N, K):
+    """Infinities and NaN: in their own rows and columns, as one row alone has them."""
+    from lit_gpt import seq_ops
+
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a = torch.randn(M, K, generator=g, device=DEV)
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(torch.bfloat16)
+    a[0, K - 1], a[M - 1, 5] = float("inf"), float("nan")
+    w[N - 1, 0], w[16, K // 2] = float("-inf"), float("nan")
+    y = torch.empty(M, N, device=DEV)
+    seq_ops.linear(a, w, M=M, N=N, K=K, y=y, lda=K, ldy=N)
+    ref = a.to(torch.bfloat16).double() @ w.double().t()
+    assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf()) and ref[1].isfinite().sum() == N - 2
+    assert torch.equal(y[y.isinf()].sign().double(), ref[ref.isinf()].sign())
+    assert float((y - ref)[ref.isfinite()].abs().max()) <= 2 ** -20 * 6

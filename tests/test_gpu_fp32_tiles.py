@@ -14,9 +14,10 @@ def rows(x, w, **kw):
     return torch.cat([ops.f32_linear(x[i: i + 1], w, **{k: one(v, i) for k, v in kw.items()}) for i in range(x.shape[0])])
 
 
-# (16 x 16 tiles: the first five and the last; 32 x 32: the others, one of them with a last row alone)
+# (32 x 32 tiles: 17 x 4097, 300 x 768 and the last four, each of these with a last row alone; 16 x 16: the others)
 @pytest.mark.parametrize("M,N,K", [(2, 4500, 256), (16, 577, 768), (17, 4097, 256), (9, 1000, 512), (31, 300, 3072), (33, 8191, 256), (97, 2049, 512),
-                                   (128, 2304, 768), (300, 768, 1024), (15, 601, 2048)])
+                                   (128, 2304, 768), (300, 768, 1024), (15, 601, 2048), (33, 3001, 768), (65, 1999, 768), (97, 1801, 1024),
+                                   (129, 1001, 512)])
 def test_rows_to_the_bit(M, N, K):
     from lit_gpt import ops
 

@@ -109,8 +109,21 @@ def test_strided_batch():
 
 # every tile form with a partial last tile of rows and of columns, rows as the tile's A (tests of products with rows as its
 # B: below); few values of K, so that rings are refilled past the end from the first step on
-@pytest.mark.parametrize("M,N,K", [(1279, 12031, 256), (1023, 10753, 128), (3327, 2305, 1024), (385, 12289, 256),
-                                   (257, 10943, 128), (769, 6913, 128), (257, 6529, 128), (65, 127, 128), (769, 9471, 128)])
+PLAIN = [(1279, 12031, 256), (1023, 10753, 128), (3327, 2305, 1024), (385, 12289, 256),
+         (257, 10943, 128), (769, 6913, 128), (257, 6529, 128), (65, 127, 128), (769, 9471, 128)]
+PROMPT = [(1279, 12032, 256), (575, 13056, 128), (769, 6656, 1024), (1023, 5376, 256), (769, 4608, 128),
+          (769, 6528, 128), (257, 5504, 128), (129, 64, 128), (769, 9408, 128), (769, 9360, 576), (257, 16640, 576)]
+
+
+def test_the_sizes_take_every_form():
+    from lit_gpt import ops, seq_ops
+
+    lib = seq_ops.load_library()
+    assert {lib.lgs_linear_form(M, N, K, 1, 0, lib.lgs_linear_ksplit(M, N, K), 0, 0) for M, N, K in PLAIN} == set(range(9))
+    assert {ops.load_library().lga_bf16_gemm_form(M, N, K, 0) & 255 for M, N, K in PROMPT} == set(range(9))
+
+
+@pytest.mark.parametrize("M,N,K", PLAIN)
 def test_every_form_at_its_edges(M, N, K):
     from lit_gpt import seq_ops
 
@@ -122,8 +135,7 @@ def test_every_form_at_its_edges(M, N, K):
     assert (y[:M].double() - want).abs().max() < TOL and y[M:].isnan().all()
 
 
-@pytest.mark.parametrize("M,N,K", [(1279, 12032, 256), (575, 13056, 128), (769, 6656, 1024), (1023, 5376, 256), (769, 4608, 128),
-                                   (769, 6528, 128), (257, 5504, 128), (129, 64, 128), (769, 9408, 128)])
+@pytest.mark.parametrize("M,N,K", PROMPT)
 def test_every_form_of_prompt_products(M, N, K):
     """bf16 weights of the GPT models: one rounding of the sum to bf16."""
     from lit_gpt import ops

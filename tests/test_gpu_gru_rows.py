@@ -39,3 +39,26 @@ def test_step(n, K, M, biased):
     assert (out.view(M, n).double() - want).abs().max() <= 2 ** -19 * size * (1 + gate.abs().max())
     rest = [i for i in range(M + 3) if i not in slot.tolist()]
     assert torch.equal(state[rest], before[rest])
+
+
+@pytest.mark.parametrize("n,K,M", [(100, 1152, 3), (2056, 640, 8)])
+def test_values_that_are_not_ordinary(n, K, M):
+    """Infinities and NaN in a sequence, a weight and a state: where one sequence alone has them too."""
+    from lit_gpt import seq_ops
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    h = torch.randn(M, K, generator=g, device=DEV)
+    w = (torch.randn(3 * n, K, generator=g, device=DEV) * K ** -0.5).to(torch.bfloat16)
+    state = torch.randn(M, n, generator=g, device=DEV)
+    h[0, 3], h[1, K - 1] = float("inf"), float("nan")
+    w[5, 7], w[n + 16, 0], w[3 * n - 1, 1] = float("-inf"), float("inf"), float("nan")
+    state[2, 9], state[2, n - 2] = float("inf"), float("nan")
+    slot, pos0 = torch.arange(M, dtype=torch.int32, device=DEV), torch.full((M,), 7, dtype=torch.int32, device=DEV)
+    together, alone = state.clone(), state.clone()
+    out = seq_ops.mingru_step(h, w, None, 0, n, 2 * n, together, slot, pos0).view(M, n)
+    one = torch.cat([seq_ops.mingru_step(h[m: m + 1], w, None, 0, n, 2 * n, alone, slot[m: m + 1], pos0[m: m + 1]).view(1, n) for m in range(M)])
+    for got, want in ((out, one), (together, alone)):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        assert torch.equal(got[got.isinf()], want[want.isinf()]) and want[2].isfinite().sum() >= n - 5
+        assert (got - want)[want.isfinite()].abs().max() <= 2 ** -18 * 64  # (both within test_step's 2^-19 of the same)
+    assert out[1].isnan().all()

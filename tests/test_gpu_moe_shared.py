@@ -35,3 +35,22 @@ def test_tokens_together(dtype, gated, T, top, E, real, W, F):
             seq_ops.moe_down(at, down, one(ids, t), one(wts, t), xt, one(h, t), accumulate=accumulate)
             live = (ids[t] < real).nonzero().flatten()  # (an identity expert's row is nobody's)
             assert torch.equal(a.view(T, top, F)[t, live], at.view(top, F)[live]) and torch.equal(x[t], xt[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("gated", [True, False])
+def test_values_that_are_not_ordinary(dtype, gated):
+    """Infinities and NaN of a token and of an expert's weights: where that token has them alone."""
+    from lit_gpt import seq_ops
+
+    T, top, E, W, F = 16, 4, 6, 1032, 4100
+    g = torch.Generator(device=DEV).manual_seed(5)
+    up = (torch.randn(E, (2 if gated else 1) * F, W, generator=g, device=DEV) * W ** -0.5).to(dtype)
+    h = torch.randn(T, W, generator=g, device=DEV)
+    ids = torch.stack([torch.randperm(E, generator=g, device=DEV)[:top] for _ in range(T)]).to(torch.int32)
+    h[3, 5], h[T - 1, W - 1] = float("nan"), float("inf")
+    up[2, 7, 0], up[4, F - 1, W - 1] = float("-inf"), float("nan")
+    a = seq_ops.moe_up(h, up, ids, seq_ops.ACT_SILU, gated=gated).view(T, -1)
+    one = torch.cat([seq_ops.moe_up(h[t: t + 1], up, ids[t: t + 1], seq_ops.ACT_SILU, gated=gated).view(1, -1) for t in range(T)])
+    assert torch.equal(a.isnan(), one.isnan()) and torch.equal(a.nan_to_num(0.0, 3e38, -3e38), one.nan_to_num(0.0, 3e38, -3e38))
+    assert a[3].isnan().all() and a[0].isfinite().sum() >= top * F - 2 and not a.isfinite().all(1).all()
