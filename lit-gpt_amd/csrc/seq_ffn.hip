@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(64) moe_route_kernel(const float* __restrict__
     const float w = expf(best - first);  // the first pick is the maximum
     den += w;
     if (lane == 0) {
-      ids[(size_t)t * top + k] = bi;
+      ids[(size_t)t * top + k] = min(bi, E - 1);  // (where all are NaN, none is best)
       wts[(size_t)t * top + k] = w;
     }
 #pragma unroll
@@ -209,7 +209,7 @@ __device__ __forceinline__ void route_scores_wave(const float* z, int E, int top
       }
     }
     if (lane == 0) {
-      ids[k] = bi;
+      ids[k] = min(bi, E - 1);  // (where all are NaN, none is best)
       wts[k] = (square ? bs * bs : bs) * wscale;
     }
 #pragma unroll

@@ -127,3 +127,23 @@ def test_products_of_fp32_rows(M, N, K, kind, ldy):
     want = z * torch.sigmoid(z) + (old[:, :N].double() if kind == "sums" else 0.0)
     assert ((y[:, :N].double() - want).abs() <= (2.0 ** -8 * want.abs() if kind == "bf16" else 0.0) + 2e-5).all()
     assert torch.equal(y[:, N:], old[:, N:].to(y.dtype))
+
+
+@pytest.mark.parametrize("T", [1, 700, 5000])
+@pytest.mark.parametrize("scores", [False, True])
+def test_tokens_whose_logits_are_nan_choose_experts_that_there_are(T, scores):
+    """(T top 10 and 7000: the sort in one launch, 50000: in three.)"""
+    from lit_gpt import seq_ops
+
+    dev, E, top = torch.device("cuda", 0), 18, 10
+    z = torch.randn(T, E, generator=torch.Generator(device=dev).manual_seed(T), device=dev)
+    route = seq_ops.moe_route_scores if scores else seq_ops.moe_route
+    plain = route(z, 0, E, top)[0]
+    z[T // 2] = float("nan")
+    ids = route(z, 0, E, top)[0]
+    rest = torch.arange(T, device=dev) != T // 2
+    assert ids.min() >= 0 and ids.max() < E and torch.equal(ids[rest], plain[rest])
+    z_start, tok_of, where = seq_ops.moe_sort(ids, E)
+    assert torch.equal(z_start[1:] - z_start[:-1], torch.bincount(ids.flatten().long(), minlength=E).int())
+    assert torch.equal(where.sort().values, torch.arange(T * top, dtype=torch.int32, device=dev))
+    assert torch.equal(tok_of[where.long()], torch.arange(T * top, dtype=torch.int32, device=dev) // top)
