@@ -16,7 +16,7 @@ def close(got, want, size=None, extra=0.0):
     assert ((got.double() - want).abs() <= EPS * size + extra + 1e-30).all()
 
 
-@pytest.mark.parametrize("T,H,dv", [(512, 8, 128), (511, 8, 128), (517, 8, 128), (4097, 1, 128), (300, 16, 64), (9, 16, 128)])
+@pytest.mark.parametrize("T,H,dv", [(512, 8, 128), (511, 8, 128), (517, 8, 128), (709, 8, 128), (4097, 1, 128), (300, 16, 64), (9, 16, 128)])
 @pytest.mark.parametrize("rank", [0, 64, 20])
 @pytest.mark.parametrize("unit", [False, True])
 def test_head_gate(T, H, dv, rank, unit):
@@ -108,6 +108,27 @@ def test_queries_and_keys(T, H, G, d, dv, rot, interleaved):
     close(k[1, 2:T + 2], x[:, H:], size[:, H:])
     assert torch.equal(v[1, 2:T + 2], before[:, (H + G) * d:].view(T, G, dv)) and torch.equal(proj[:, H * d:], before[:, H * d:])
     assert (k[0] == 7).all() and (k[1, :2] == 7).all() and (k[1, T + 2:] == 7).all() and (v[0] == 7).all()
+
+
+@pytest.mark.parametrize("T", [640, 641, 1000, 3501])
+@pytest.mark.parametrize("H,G,d,dv,rot", [(9, 3, 64, 100, 0), (9, 3, 64, 100, 30), (4, 4, 128, 256, 0), (1, 1, 10, 12, 10)])
+def test_two_maps_a_head(T, H, G, d, dv, rot):
+    """Tokens together give the bits that they have in a step of few, in all forms of the launch."""
+    from lit_gpt import seq_ops
+
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    proj = torch.randn(T, 2 * (H + G) * d + G * dv, generator=g, device=DEV)
+    slot, pos = torch.zeros(T, dtype=torch.int32, device=DEV), torch.arange(T, dtype=torch.int32, device=DEV)
+    freq = torch.rand(rot // 2, generator=g, device=DEV) if rot else None
+
+    def prepare(step):
+        p, k, v = proj.clone(), torch.zeros(1, T, G, 2 * d, device=DEV), torch.zeros(1, T, G, dv, device=DEV)
+        for t in range(0, T, step):
+            at = slice(t, min(t + step, T))
+            seq_ops.diffattn_prepare(p[at], 0, 2 * H * d, 2 * (H + G) * d, k, v, freq, slot[at], pos[at], H=H, G=G, d=d, dv=dv, rot_dims=rot)
+        return p, k, v
+
+    assert all(torch.equal(a, b) for a, b in zip(prepare(T), prepare(100)))
 
 
 @pytest.mark.parametrize("M,N,K", [(9, 1, 8), (130, 131, 64), (300, 513, 72), (128, 128, 64), (257, 66, 136), (129, 16, 72), (70, 18, 64), (140, 19, 64)])
