@@ -866,8 +866,9 @@ extern "C" int lga_f32_linears_sum(const float* x1, const float* ml, int parts, 
   const size_t joined = parts > 1 ? (size_t)K1 + (K1 / hs * 9 + 3) / 4 * 4 : 0;
   const bool ahead = K2 <= lga::kF32AheadMost;
   const size_t lds = (joined + (ahead ? K2 : 0)) * sizeof(float);
-  (parts > 1 ? (ahead ? lga::f32_linears_sum_kernel<true, true> : lga::f32_linears_sum_kernel<true, false>)
-             : (ahead ? lga::f32_linears_sum_kernel<false, true> : lga::f32_linears_sum_kernel<false, false>))<<<(N + 3) / 4, 256, lds, stream>>>(a);
+  const auto kernel = parts > 1 ? (ahead ? lga::f32_linears_sum_kernel<true, true> : lga::f32_linears_sum_kernel<true, false>)
+                                : (ahead ? lga::f32_linears_sum_kernel<false, true> : lga::f32_linears_sum_kernel<false, false>);
+  kernel<<<(N + 3) / 4, 256, lds, stream>>>(a);
   LGA_LAUNCH_RETURN();
 }
 

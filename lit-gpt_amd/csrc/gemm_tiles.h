@@ -306,7 +306,8 @@ inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int
     const GemmForm& t = kGemmForms[f];
     if (!gemm_form_fits(t, flags)) continue;
     const int rows = rows_b ? t.bn : t.bm, cols = rows_b ? t.bm : t.bn, frags = rows_b ? t.fn : t.fm, step = rows / frags;
-    const float most = t.bm * t.bn > 128 * 192 ? 0.69f : 0.46f;  // (of what fewer workgroups gain: 0.7 and 0.5 above, fitted anew on these products)
+    // (of what fewer workgroups gain: 0.7 and 0.5 above, fitted anew on these products)
+    const float most = t.bm * t.bn > 128 * 192 ? 0.69f : 0.46f;
     auto round = [&](float load) { return per * std::max(t.fast_us, t.step_us * (1.0f - most * (1.0f - load))) + t.round_us; };
     const int pieces = (M + step - 1) / step, mt = pieces / frags, left = pieces % frags;
     const float nt = (float)((N + cols - 1) / cols), slots = (float)t.slots;

@@ -132,11 +132,10 @@ __device__ __forceinline__ void pool_block(const void* cache_k, const void* cach
   }
 }
 
-// grid (T, parts; ONE: T, so with a joint norm or pooled blocks): the waves take the vectors in turn, those of the H query heads (normed, rotated
-// and multiplied by the
-// position's query temperature, in place) and of the G key heads (normed and rotated on their way into the cache);
-// then all threads copy the values into the cache. The value columns may be the key columns themselves (values = the
-// keys as projected): the keys are never changed in place.
+// grid (T, parts; ONE: T, so with a joint norm or pooled blocks): the waves take the vectors in turn, those of the H query
+// heads (normed, rotated and multiplied by the position's query temperature, in place) and of the G key heads (normed and
+// rotated on their way into the cache); then all threads copy the values into the cache. The value columns may be the key
+// columns themselves (values = the keys as projected): the keys are never changed in place.
 template <bool CF32, bool ONE>
 __global__ void __launch_bounds__(256) normattn_prepare_kernel(NormPrepArgs p) {
   __shared__ float red[4];
@@ -775,8 +774,9 @@ extern "C" int lgs_diffattn_prepare(float* proj, long ld, int q_off, int k_off, 
   const long parts = T <= 640 ? (items + 255) / 256 : T > 3500 || (rot_dims == 0 && d < 128 && T > 900) ? 1 : std::max(items / 256, 1L);
   const dim3 grid(T, (unsigned)std::min(parts, 65535L));
   const bool one = grid.y == 1;
-  (cache_f32 ? (one ? lgs::diffattn_prepare_kernel<true, true> : lgs::diffattn_prepare_kernel<true, false>)
-             : (one ? lgs::diffattn_prepare_kernel<false, true> : lgs::diffattn_prepare_kernel<false, false>))<<<grid, 256, 0, stream>>>(p);
+  const auto kernel = cache_f32 ? (one ? lgs::diffattn_prepare_kernel<true, true> : lgs::diffattn_prepare_kernel<true, false>)
+                                : (one ? lgs::diffattn_prepare_kernel<false, true> : lgs::diffattn_prepare_kernel<false, false>);
+  kernel<<<grid, 256, 0, stream>>>(p);
   LGA_LAUNCH_RETURN();
 }
 
@@ -840,8 +840,9 @@ extern "C" int lgs_normattn_prepare(float* proj, long ld, int q_off, int k_off, 
   const bool held = !bare && T > 1024 && T < 1700 && (H + G) * d <= 2560 && (norm == 0 || rot_dims == 0);
   const dim3 grid(T, norm == 2 || pool > 0 || few || held ? 1 : std::min((H + G + 3) / 4, std::max(4096 / T, 1)));
   const bool one = grid.y == 1;
-  (cache_f32 ? (one ? lgs::normattn_prepare_kernel<true, true> : lgs::normattn_prepare_kernel<true, false>)
-             : (one ? lgs::normattn_prepare_kernel<false, true> : lgs::normattn_prepare_kernel<false, false>))<<<grid, 256, 0, stream>>>(p);
+  const auto kernel = cache_f32 ? (one ? lgs::normattn_prepare_kernel<true, true> : lgs::normattn_prepare_kernel<true, false>)
+                                : (one ? lgs::normattn_prepare_kernel<false, true> : lgs::normattn_prepare_kernel<false, false>);
+  kernel<<<grid, 256, 0, stream>>>(p);
   LGA_LAUNCH_RETURN();
 }
 

@@ -743,7 +743,8 @@ extern "C" int lgs_moe_combine(const float* y, const int* where, const float* wt
                                hipStream_t stream) {
   LGA_CHECK_ARG(y && where && wts && x && T > 0 && T <= 65535 && top > 0 && N > 0, "lgs_moe_combine: bad arguments");
   LGA_CHECK_ARG(!ids || hin, "lgs_moe_combine: identity experts need the tokens' inputs");
-  if ((top > 2 || (long)T * N >= 200000) && N % 4 == 0 && ldx % 4 == 0 && (!ids || ldh % 4 == 0) && ((uintptr_t)y | (uintptr_t)x | (uintptr_t)(ids ? hin : nullptr)) % 16 == 0) {
+  if ((top > 2 || (long)T * N >= 200000) && N % 4 == 0 && ldx % 4 == 0 && (!ids || ldh % 4 == 0) &&
+      ((uintptr_t)y | (uintptr_t)x | (uintptr_t)(ids ? hin : nullptr)) % 16 == 0) {
     lgs::moe_combine4_kernel<<<dim3((N / 4 + 255) / 256, T), 256, 0, stream>>>(y, where, wts, x, ldx, top, N, ids, n_real, hin, ldh,
                                                                                 accumulate);
     LGA_LAUNCH_RETURN();

@@ -197,7 +197,8 @@ __global__ void __launch_bounds__(KW * 64, NR == 2 && RB == 1 ? 3 : 1) lin_rows_
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, q4 = lane >> 4;
   const int z = blockIdx.y, n0 = blockIdx.x * (16 * NR);
   const uint16_t* w = (const uint16_t*)p.w + (size_t)z * p.sw;
-  rows_products<NR, KW, MR, RB, ONE>(lds, [&](int r) { return w + (size_t)min(n0 + r, p.N - 1) * p.K; }, p.a + (size_t)z * p.sa, p.lda, p.M, p.K);
+  rows_products<NR, KW, MR, RB, ONE>(lds, [&](int r) { return w + (size_t)min(n0 + r, p.N - 1) * p.K; }, p.a + (size_t)z * p.sa,
+                                     p.lda, p.M, p.K);
   if (tid >= NR * 64 || l15 >= p.M) return;
   const int j = NR > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
   const rows_f32x4 v = rows_sum<NR, KW>(lds, j, lane);

@@ -102,7 +102,8 @@ __device__ __forceinline__ void rows_products(unsigned char* lds_all, Weights&& 
             const uint4 x16 = make_uint4(pack2(x[m][0].x, x[m][0].y), pack2(x[m][0].z, x[m][0].w), pack2(x[m][1].x, x[m][1].y), pack2(x[m][1].z, x[m][1].w));
 #pragma unroll
             for (int j = 0; j < NR; ++j)
-              v[e][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[m][j], __builtin_bit_cast(rows_bf16x8, x16), ONE || e == 0 ? zero : v[0][j], 0, 0, 0);
+              v[e][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[m][j], __builtin_bit_cast(rows_bf16x8, x16),
+                                                                ONE || e == 0 ? zero : v[0][j], 0, 0, 0);
           }
 #pragma unroll
           for (int e = ONE ? 0 : 1; e < 2; ++e)
