@@ -422,9 +422,15 @@ __global__ void __launch_bounds__(256) moe_up_shared_kernel(const float* __restr
 // tokens share some, and as many pairs as make up for those that have an expert alone (us, a pair at a time / shared, experts of 2 x 1408 x
 // 2048: 3 tokens of two of 8 9.2 / 11.4, 4 of two 14.8 / 13.2; 5 of two of 16 18.5 / 19.3, 6 of two 21.3 / 18.5; of 2 x 2816 x 2048 4 of one of 16
 // 15.6 / 16.0, 3 of two 21.0 / 19.4; of 2 x 2752 x 4096 3 of one of 16 21.7 / 21.7)
-static bool moe_up_shares(int T, int top, long bytes, int n_real) {
+//
+// Rows below 2048 values are over before the look at the pairs is paid for, unless there are pairs enough of an expert; a few hundred
+// workgroups do not fill the chip. Of 1254 calls of all this, gated 4 in 5, from 2 to 64 experts' pairs, those on this side take 0.72 of
+// a pair at a time's time, those on the other 1.17 (6 tokens of 4 of 8, 2 x 5136 x 448 35.0 / 63.4; 2 of 8 of 16, 2 x 3952 x 576 30.1 /
+// 44.3; 8 of two of 8, 832 x 5056 16.9 / 24.2; 14 of one of 8, 2 x 4096 x 512 19.5 / 29.8).
+static bool moe_up_shares(int T, int top, long bytes, int n_real, int K, int blocks) {
   const int pairs = T * top;
-  return T > 1 && pairs <= 64 && bytes >= 8 << 20 && n_real <= 4 * pairs && bytes * pairs >= (n_real <= 8 ? 80L : 128L) << 20;
+  if (T == 1 || pairs > 64 || bytes < 8 << 20 || n_real > 4 * pairs || bytes * pairs < (n_real <= 8 ? 80L : 128L) << 20) return false;
+  return (K >= 2048 || (K >= 1024 && pairs * (K - 640) >= 768 * n_real)) && (long)blocks * std::min(pairs, n_real) >= 640;
 }
 
 // Counting sort of the pairs by expert in three launches. ws: 2 E ints (counts, cursors), zero on entry.
@@ -681,8 +687,10 @@ extern "C" int lgs_moe_up(const float* h, long ldh, const void* up, int w_f32, c
                           int top, int F, int K, int act, int gated, int n_real, hipStream_t stream) {
   LGA_CHECK_ARG(h && up && ids && actbuf && T > 0 && top > 0 && F > 0 && K > 0 && (long)T * top <= 65535 && n_real > 0,
                 "lgs_moe_up: bad arguments");
-  if (lgs::moe_up_shares(T, top, (long)(gated ? 2 : 1) * F * K * (w_f32 ? 4 : 2), n_real) && K % 8 == 0 && ldh % 4 == 0 && (uintptr_t)h % 16 == 0) {
-    const dim3 grid(gated ? (F + 3) / 4 : (F + 7) / 8, T * top);
+  const int blocks = gated ? (F + 3) / 4 : (F + 7) / 8;
+  if (lgs::moe_up_shares(T, top, (long)(gated ? 2 : 1) * F * K * (w_f32 ? 4 : 2), n_real, K, blocks) && K % 8 == 0 && ldh % 4 == 0 &&
+      (uintptr_t)h % 16 == 0) {
+    const dim3 grid(blocks, T * top);
     auto go = [&](auto f32, auto glu) {
       constexpr bool W = decltype(f32)::value, G = decltype(glu)::value;
       if (T * top > 24) lgs::moe_up_shared_kernel<W, G, true><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, T * top, top, F, K, act, n_real);
@@ -694,12 +702,11 @@ extern "C" int lgs_moe_up(const float* h, long ldh, const void* up, int w_f32, c
     else go(std::false_type{}, std::false_type{});
     LGA_LAUNCH_RETURN();
   }
+  const dim3 grid(blocks, T * top);
   if (gated) {
-    const dim3 grid((F + 3) / 4, T * top);
     if (w_f32) lgs::moe_up_kernel<true, true><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, top, F, K, act, n_real);
     else lgs::moe_up_kernel<false, true><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, top, F, K, act, n_real);
   } else {
-    const dim3 grid((F + 7) / 8, T * top);
     if (w_f32) lgs::moe_up_kernel<true, false><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, top, F, K, act, n_real);
     else lgs::moe_up_kernel<false, false><<<grid, 256, 0, stream>>>(h, ldh, up, ids, actbuf, top, F, K, act, n_real);
   }
