@@ -252,7 +252,7 @@ __device__ __forceinline__ int swz(int row, int chunk) { return row * 128 + 16 *
 
 // VEC: K % 8 == 0 and 16-B aligned rows of A and W (vector loads); otherwise element loads with k guards.
 // A16: A arrives as bf16 (half the operand traffic of the fp32 stream; the same values the fp32 path would round to)
-// NARROW: up to 18 columns (a router's)
+// NARROW: up to 32 columns, those of a router
 template <bool VEC, bool A16, bool NARROW>
 __global__ void __launch_bounds__(256) lin_mfma_kernel(LinArgs p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * 2 * TILE_BYTES];  // [buf][A|W]
@@ -391,7 +391,8 @@ __global__ void __launch_bounds__(256) lin_mfma_kernel(LinArgs p) {
   // a wave turns 32 rows of its 64 x 64 results at a time in LDS of its own and stores them four columns a lane, 256 bytes of a row
   // together (as the accumulators lie, 64: 2048 x 2048 x 64, all of it results, 22.0 -> 13.4 us; of a few columns most of that would be work
   // for none, us turned / as they lie: 1725 x 16 x 512 into sums 25.0 / 19.1, 2048 x 16 x 2048 60.5 / 54.6, 300 x 18 x
-  // 2048 61.0 / 58.3, 58 x 16 x 64 8.7 / 6.5, 1211 x 20 x 64 9.5 / 11.0)
+  // 2048 61.0 / 58.3, 58 x 16 x 64 8.7 / 6.5, 1211 x 20 x 64 9.5 / 11.0; of 19 to 31 columns that do not lie in fours, 118 products into
+  // sums 1.03 in the mean and up to 1.12, 1530 x 27 x 384 26.2 / 24.2, others the same)
   constexpr int RS = 68;
   float* turned = (float*)(lds + wave * 16384);
   const int c4 = fr * 4, n = n0 + wn * 64 + c4, cols = p.N - n;
@@ -758,7 +759,7 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
     else if (vec) lgs::lin_mfma_kernel<true, false, NARROW><<<grid, 256, 0, stream>>>(p);   \
     else lgs::lin_mfma_kernel<false, false, NARROW><<<grid, 256, 0, stream>>>(p);           \
   } while (0)
-  if (N <= 18) LGS_MFMA(true);
+  if (N <= 18 || (N < 32 && (p.ksplit > 1 ? N : ldy) % 4 != 0)) LGS_MFMA(true);
   else LGS_MFMA(false);
 #undef LGS_MFMA
   if (p.ksplit > 1) lgs::lin_sum_kernel<<<dim3((N + 255) / 256, M), 256, 0, stream>>>(p);

@@ -131,7 +131,8 @@ def test_two_maps_a_head(T, H, G, d, dv, rot):
     assert all(torch.equal(a, b) for a, b in zip(prepare(T), prepare(100)))
 
 
-@pytest.mark.parametrize("M,N,K", [(9, 1, 8), (130, 131, 64), (300, 513, 72), (128, 128, 64), (257, 66, 136), (129, 16, 72), (70, 18, 64), (140, 19, 64)])
+@pytest.mark.parametrize("M,N,K", [(9, 1, 8), (130, 131, 64), (300, 513, 72), (128, 128, 64), (257, 66, 136), (129, 16, 72), (70, 18, 64), (140, 19, 64),
+                                   (77, 31, 64), (130, 28, 72), (129, 33, 64)])
 @pytest.mark.parametrize("kind", ["fp32", "bf16", "sums"])
 @pytest.mark.parametrize("ldy", [0, 1])
 def test_products_of_fp32_rows(M, N, K, kind, ldy):
