@@ -229,7 +229,8 @@ struct GemmPlan {
 enum {
   kGemmRowsB = 1,  // the rows are the tile's B, the columns its A
   kGemmPairs = 2,  // A's fragments are those of two matrices in turn: forms with an even number of them
-  kGemmActs = 4    // forms whose code holds activations
+  kGemmActs = 4,   // forms whose code holds activations
+  kGemmSums = 8    // results go into sums
 };
 inline bool gemm_form_fits(const GemmForm& t, int flags) {
   return !((flags & kGemmActs && t.bm * t.bn > 256 * 128) || (flags & kGemmPairs && t.fm % 2));
@@ -285,7 +286,8 @@ inline GemmPlan gemm_whole_plan(int M, int N, int K, int batch, bool grouped, in
 // Rows as the tile's B: at least nine steps, and a fortieth gained, or else the form that counts whole tiles. (Ends of tiles are most
 // of shorter products, and of 64 x 128 they are less than the sums here say: 990 products for which the two choose otherwise, the sums' choice
 // alone 1.04 times the time of whole tiles' for plain ones, 1.06 for gated units, with the line 0.99 and 0.99; 120 x 768 x 3072 10.8 / 12.1, 2849
-// x twice 5524 x 512 53 / 62. Rows as A 0.93, at every length.)
+// x twice 5524 x 512 53 / 62. Rows as A 0.93, at every length; but activations into sums, where ends of tiles are the most work, need nine
+// steps too: 2084 x 3159 x 256 24.1 / 33.8, 291 x 17493 x 192 22.6 / 30.2.)
 // A grouped product's short tiles stand beside the whole ones of their columns, whose weights they would otherwise fetch anew (16 groups of
 // 278 rows of twice 2752 x 4096 302 behind, 260 beside): 480 products of 8 to 18 groups, 144 to 16384 rows in all, weights from memory,
 // take 0.93 of the time that whole tiles took (gated units 0.98), none more than 3 % more. (Weights that stay in the last cache from
@@ -294,11 +296,11 @@ inline GemmPlan gemm_tile_plan(int M, int N, int K, int batch, bool grouped, int
   GemmPlan best{-1, 1};
   if (grouped) return gemm_whole_plan(M, N, K, batch, true, ksplit, flags);
   if (K % 64 != 0 || M <= 0) return best;
-  const bool rows_b = flags & kGemmRowsB;
-  if (rows_b || (ksplit <= 0 && batch == 1)) best = gemm_whole_plan(M, N, K, batch, false, ksplit, flags);
+  const bool rows_b = flags & kGemmRowsB, acts_sums = flags & kGemmActs && flags & kGemmSums;
+  if (rows_b || acts_sums || (ksplit <= 0 && batch == 1)) best = gemm_whole_plan(M, N, K, batch, false, ksplit, flags);
   else best.ksplit = ksplit > 0 ? ksplit : 1;
   const int steps = K / 64, per = (steps + best.ksplit - 1) / best.ksplit, count = batch * ((steps + per - 1) / per);
-  if (rows_b && per < 9) return best;
+  if ((rows_b || acts_sums) && per < 9) return best;
   const int kept = best.tile;
   float best_us = 0.0f, kept_us = 0.0f;
 #pragma unroll

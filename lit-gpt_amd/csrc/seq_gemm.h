@@ -27,7 +27,7 @@ struct LinArgs {
 // Which tile form and how many ranges of K a product of bf16 A and W takes on the pipelined tiles (seq_gemm.hip); tile
 // -1: not one of theirs (K is no multiple of 64). Rows of A and W start on 16 bytes. ksplit 0: the plan's own choice.
 using lga::GemmPlan;
-GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act = kActNone);
+GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act = kActNone, bool sums = false);
 GemmPlan gemm_glu_plan(int M, int n, int K, int batch, bool grouped);
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream);
 

@@ -155,14 +155,18 @@ __device__ __forceinline__ void gemm_rows(const LinArgs& p, unsigned char* lds, 
   const long at = (long)z * p.sy + (long)(r_lo + mw) * p.ldy + nw;
   if (ACTS && p.act != kActNone) {
     if constexpr (ACTS) {
-      // (a loop of its own for each activation: a choice per result keeps them from standing among one another)
+      // (a loop of its own for each activation: a choice per result keeps them from standing among one another. Into sums: 2084 rows of
+      // 3159 x 256, silu, 46.1 -> 33.8 us, 832 of 9600 x 1408 97 -> 77.7, 264 of 20528 x 1152 59.7 -> 46.2)
       auto act = [&](auto kind) __attribute__((always_inline)) {
         auto f = [&](int j, float v, float) { return act_f(decltype(kind)::value, v + bias[j]); };
         if (p.y16) each(no, no, no, few, p.y16 + at, p.ldy, [&](int j, float v, float) { return f2bf(f(j, v, 0.0f)); });
+        else if (p.accumulate) each(no, yes, no, few, p.y + at, p.ldy, [&](int j, float v, float old) {
+#pragma clang fp contract(off)
+          return old + f(j, v, 0.0f);
+        });
         else each(no, no, no, few, p.y + at, p.ldy, f);
       };
-      if (p.accumulate) each(no, yes, no, few, p.y + at, p.ldy, [&](int j, float v, float old) { return old + act_f(p.act, v + bias[j]); });
-      else if (p.act == kActRelu2) act(std::integral_constant<int, kActRelu2>{});
+      if (p.act == kActRelu2) act(std::integral_constant<int, kActRelu2>{});
       else if (p.act == kActGeluTanh) act(std::integral_constant<int, kActGeluTanh>{});
       else if (p.act == kActSilu) act(std::integral_constant<int, kActSilu>{});
       else act(std::integral_constant<int, kActSigmoid>{});
@@ -328,9 +332,9 @@ int gemm_glu_launch(const LinArgs& p, const GluForm& f, int batch, hipStream_t s
   return (int)hipErrorInvalidValue;
 }
 
-GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act) {
+GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int act, bool sums) {
   if (grouped && gemm_few_rows(M, batch)) return GemmPlan{-1, 1};
-  return lga::gemm_tile_plan(M, N, K, batch, grouped, ksplit, act != kActNone ? lga::kGemmActs : 0);
+  return lga::gemm_tile_plan(M, N, K, batch, grouped, ksplit, (act != kActNone ? lga::kGemmActs : 0) | (sums ? lga::kGemmSums : 0));
 }
 
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream) {
