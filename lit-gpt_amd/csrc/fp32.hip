@@ -410,7 +410,7 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 // outputs; the weights then start later, and a workgroup holds LDS, which rows of up to 3072 values make up for in a model's chain of
 // launches and longer ones do not (us a token behind 300 keys, weights first / AHEAD: pythia-160m 307.9 / 303.6, pythia-410m 694 / 742,
 // pythia-1b 1234 / 1318; alone, weights from memory, 768 columns beside 3072 7.4 / 8.2, 1024 beside 4096 9.7 / 12.5, 2048 beside 8192
-// 31.3 / 35.9).
+// 31.3 / 35.9). Nor where x1 is longer than the block: 2240 columns beside 1280 9.8 / 13.0, 2560 beside 704 10.5 / 14.0.
 constexpr int kF32AheadMost = 3072;  // (values of x2)
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
@@ -864,7 +864,7 @@ extern "C" int lga_f32_linears_sum(const float* x1, const float* ml, int parts, 
                 "lga_f32_linears_sum: 1 to 8 ranges of up to 256 heads, 8192 columns");
   const lga::F32LinearsSum a{x1, w1, b1, x2, w2, b2, residual, y, N, K1, K2, ml, parts, hs};
   const size_t joined = parts > 1 ? (size_t)K1 + (K1 / hs * 9 + 3) / 4 * 4 : 0;
-  const bool ahead = K2 <= lga::kF32AheadMost;
+  const bool ahead = K1 <= 768 && K2 <= lga::kF32AheadMost;
   const size_t lds = (joined + (ahead ? K2 : 0)) * sizeof(float);
   const auto kernel = parts > 1 ? (ahead ? lga::f32_linears_sum_kernel<true, true> : lga::f32_linears_sum_kernel<true, false>)
                                 : (ahead ? lga::f32_linears_sum_kernel<false, true> : lga::f32_linears_sum_kernel<false, false>);
