@@ -191,6 +191,14 @@ int lgs_streams_step(float* x, const float* y, const float* mix, const float* ou
                      const float* norm_w, float* h, void* h_bf16, float eps, int T, int W, int streams,
                      lgs_stream_t stream);
 
+/* The read of lgs_streams_step on streams that are made anew in registers: from table[tokens[t]] * scale (tokens given) or from
+ * base [T][streams][W], then for k = 0 .. count - 1 x_j <- sum_i mix[k][i * streams + j] x_i + out[k][j] y[k] (y, mix, out: host
+ * arrays of device pointers). x: where the streams are stored (may be base), or NULL. h or h_bf16 may be left out. W <= 4096, 2 to 4
+ * streams, count <= 2 streams on tokens, 1 to 3 on base. */
+int lgs_streams_held(const int* tokens, const void* table, int w_f32, float scale, int vocab, const float* base, float* x,
+                     const float* const* y, const float* const* mix, const float* const* out, int count, const float* in,
+                     const float* norm_w, float* h, void* h_bf16, float eps, int T, int W, int streams, lgs_stream_t stream);
+
 /* ---- differential attention ---- */
 /* Per token: rotary (interleaved pairs 2i, 2i + 1 of the first rot_dims dims of every map; angle = position *
  * inv_freq[i]) on the 2 H query maps at proj[q_off ..] in place and on the 2 G key maps at proj[k_off ..] on their way

@@ -7,6 +7,8 @@
 //   lgs_embed_streams   x[t][j] = table[tokens[t]] * scale for every stream j
 //   lgs_streams_step    one launch per sublayer boundary: the write-back of the sublayer that just ran (optional)
 //                       followed by the read + norm of the next one (optional), so the streams are read once
+//   lgs_streams_held    a boundary of a prompt that makes the streams anew from the embedding (or stored streams) and the
+//                       sublayers' outputs since, instead of storing and reading them
 //   lgs_sandwich_step   the boundary of layers with one residual whose sublayers are normed on the way in (and
 //                       optionally out): the norms and the average of up to two branch outputs, the output norm times
 //                       the layer scale, the residual add, a learned average over the depth at a layer's end or what
@@ -187,6 +189,186 @@ static bool streams_step_reg(const StreamArgs& p, int T, hipStream_t stream) {
   else if (p.W <= 4096 && SMAX <= 4) streams_step_reg_kernel<SMAX, 16, 256><<<T, 256, 0, stream>>>(p);
   else return false;
   return true;
+}
+
+// A boundary of a prompt without the write-back: the streams are made anew, in registers, from where they last stood (the embedding, or
+// streams that were stored) and the outputs of the K sublayers since, and stored only where `x` is given. The values are
+// those of K steps of the kernels above, operation by operation; thread i owns columns i, i + 256, ... as there, so the sums
+// of squares are theirs too.
+//
+// Bound by memory: 2407 rows of 4096, four streams, us (and TB/s) with 0, 1, 4 and 8 outputs since the embedding 16.6 (2.4), 23 (3.4),
+// 43 (4.6), 79 (4.7), where a step that stores took 92 (4.1); the embedding's own 50 are gone. Storing s streams costs 2 s rows of
+// fp32 a boundary, reading what they are made of one row per sublayer since, so four streams go on from the embedding (half a
+// row) for eight sublayers and from stored streams for three (seq_ops.streams_hold). Columns come in two portions in turn, the next
+// one's loads ahead of the sums.
+constexpr int kMaxHeld = 8;
+struct HeldArgs {
+  const int* tokens;  // embedding base: x_j = table[tokens[t]] * scale
+  const void* table;
+  int w_f32;
+  float scale;
+  const float* base;  // stored base [T][s][W]
+  float* x;           // where the streams are stored (null: nowhere; base itself or another place)
+  const float* y[kMaxHeld];
+  const float* mix[kMaxHeld];
+  const float* out[kMaxHeld];
+  const float *in, *w;  // w null: the weighted sum itself is the result
+  float* h;             // fp32 result (may be null beside h16)
+  uint16_t* h16;
+  float eps;
+  int W;
+};
+
+// FROM: the embedding in bf16 (0) or fp32 (1), or stored streams (2)
+template <int S, int K, int FROM>
+__global__ void __launch_bounds__(256) streams_held_kernel(HeldArgs p) {
+  constexpr int CPT = 16, ROWS = K + (FROM == 2 ? S : 1);          // columns of a thread (W <= 4096); rows that they are made of
+  constexpr int CH = ROWS <= 2 ? 16 : ROWS <= 4 ? 8 : 4;           // ... at a time
+  __shared__ float us[CPT * 256];  // the weighted sums, until the norm is known (every thread its own)
+  __shared__ float red[4];
+  const int tid = threadIdx.x, W = p.W;
+  const size_t t = blockIdx.x;
+  const float* base = FROM == 2 ? p.base + t * S * W : nullptr;
+  const size_t row = FROM == 2 ? 0 : (size_t)p.tokens[t] * W;
+  const float* table32 = (const float*)p.table + row;
+  const uint16_t* table16 = (const uint16_t*)p.table + row;
+  struct Columns {
+    float y[K + 1][CH], v[FROM == 2 ? S : 1][CH];
+  };
+  auto load = [&](int i0, Columns& o) {  // (columns past the end repeat the last one, never stored or summed)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      int at = k;
+      asm volatile("" : "+s"(at));  // (all outputs' addresses at once are too many scalars)
+      const float* y = p.y[at] + t * W;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) o.y[k][c] = y[min(i0 + 256 * c, W - 1)];
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int i = min(i0 + 256 * c, W - 1);
+      if constexpr (FROM == 2) {
+#pragma unroll
+        for (int j = 0; j < S; ++j) o.v[j][c] = base[(size_t)j * W + i];
+      } else if constexpr (FROM == 1) {
+        o.v[0][c] = table32[i];
+      } else {
+        o.v[0][c] = __uint_as_float((uint32_t)table16[i]);
+      }
+    }
+  };
+  // A sublayer's links come as scalars, for all columns at a time and one sublayer ahead (read from LDS five operations need a
+  // read). The index is hidden from the compiler, or it fetches all sublayers' first, more than there are scalar registers.
+  using Scalars = const __attribute__((address_space(4))) float*;
+  struct Links {
+    float mix[S * S], out[S];
+  };
+  auto fetch = [&](int k, Links& o) {
+    asm volatile("" : "+s"(k));
+    const Scalars mix = (Scalars)p.mix[k], out = (Scalars)p.out[k];
+#pragma unroll
+    for (int e = 0; e < S * S; ++e) o.mix[e] = mix[e];
+#pragma unroll
+    for (int e = 0; e < S; ++e) o.out[e] = out[e];
+  };
+  float ss = 0.0f;
+  auto work = [&](int i0, const Columns& a) {
+    float v[CH][S];
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int j = 0; j < S; ++j) {
+        if constexpr (FROM == 2) v[c][j] = a.v[j][c];
+        else if constexpr (FROM == 1) v[c][j] = a.v[0][c] * p.scale;
+        else v[c][j] = __uint_as_float(__float_as_uint(a.v[0][c]) << 16) * p.scale;
+      }
+    Links l[2];
+    if constexpr (K > 0) fetch(0, l[0]);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k + 1 < K) fetch(k + 1, l[(k + 1) & 1]);
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        float nv[S];
+#pragma unroll
+        for (int j = 0; j < S; ++j) {
+          float acc = 0.0f;
+#pragma unroll
+          for (int f = 0; f < S; ++f) acc = fmaf(l[k & 1].mix[f * S + j], v[c][f], acc);
+          nv[j] = fmaf(l[k & 1].out[j], a.y[k][c], acc);
+        }
+#pragma unroll
+        for (int j = 0; j < S; ++j) v[c][j] = nv[j];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int i = i0 + 256 * c;
+      float r = 0.0f;
+#pragma unroll
+      for (int j = 0; j < S; ++j) r = fmaf(((Scalars)p.in)[j], v[c][j], r);
+      us[i] = r;  // (without a branch, or the sums above move behind it, and behind all the links' loads)
+      const float more = fmaf(r, r, ss);
+      ss = i < W ? more : ss;
+    }
+    if (p.x) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+        if (i0 + 256 * c < W) {
+#pragma unroll
+          for (int j = 0; j < S; ++j) p.x[(t * S + j) * W + i0 + 256 * c] = v[c][j];
+        }
+    }
+  };
+  constexpr int STEP = CH * 256;
+  Columns a, b;  // (two in turn: a copy would wait for the loads ahead)
+  load(tid, a);
+#pragma unroll 1
+  for (int i0 = tid; i0 < W; i0 += 2 * STEP) {
+    if (CH < CPT) load(i0 + STEP, b);
+    __builtin_amdgcn_sched_barrier(0);
+    work(i0, a);
+    if (CH == CPT || i0 + STEP >= W) break;
+    load(i0 + 2 * STEP, a);
+    __builtin_amdgcn_sched_barrier(0);
+    work(i0 + STEP, b);
+  }
+  float rstd = 1.0f, nw[CPT];
+  if (p.w) {
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) nw[c] = p.w[min(tid + 256 * c, W - 1)];
+    ss = wave_sum(ss);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    ss = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) ss += red[w];
+    rstd = 1.0f / sqrtf(ss / (float)W + p.eps);
+  }
+#pragma unroll
+  for (int c = 0; c < CPT; ++c) {
+    const int i = tid + 256 * c;
+    if (i >= W) break;
+    const float r = p.w ? us[i] * rstd * nw[c] : us[i];
+    if (p.h) p.h[t * W + i] = r;
+    if (p.h16) p.h16[t * W + i] = f2bf(r);
+  }
+}
+
+template <int S, int FROM, int K = FROM == 2 ? 1 : 0>
+static bool streams_held(const HeldArgs& p, int T, int count, hipStream_t stream) {
+  if (count == K) {
+    streams_held_kernel<S, K, FROM><<<T, 256, 0, stream>>>(p);
+    return true;
+  }
+  if constexpr (K < (FROM == 2 ? 3 : 2 * S)) return streams_held<S, FROM, K + 1>(p, T, count, stream);
+  return false;
+}
+template <int S>
+static bool streams_held_from(const HeldArgs& p, int T, int count, hipStream_t stream) {
+  return p.base ? streams_held<S, 2>(p, T, count, stream)
+                : p.w_f32 ? streams_held<S, 1>(p, T, count, stream) : streams_held<S, 0>(p, T, count, stream);
 }
 
 // ------------------------------------------------------------------------------------------------ sandwich norms
@@ -418,6 +600,33 @@ extern "C" int lgs_streams_step(float* x, const float* y, const float* mix, cons
   else if (streams <= 4) done = lgs::streams_step_reg<4>(p, T, stream);
   else done = lgs::streams_step_reg<8>(p, T, stream);
   if (!done) lgs::streams_step_kernel<<<T, 256, 0, stream>>>(p);  // wide rows: column blocks one after the other
+  LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lgs_streams_held(const int* tokens, const void* table, int w_f32, float scale, int vocab, const float* base,
+                                float* x, const float* const* y, const float* const* mix, const float* const* out, int count,
+                                const float* in, const float* norm_w, float* h, void* h_bf16, float eps, int T, int W,
+                                int streams, hipStream_t stream) {
+  LGA_CHECK_ARG(T > 0 && W > 0 && W <= 4096, "lgs_streams_held: rows of up to 4096 columns");
+  LGA_CHECK_ARG(streams >= 2 && streams <= 4, "lgs_streams_held: 2 to 4 streams");
+  LGA_CHECK_ARG((base != nullptr) != (tokens != nullptr), "lgs_streams_held: stored streams, or tokens");
+  LGA_CHECK_ARG(!tokens || (table && vocab > 0), "lgs_streams_held: tokens without a table");
+  LGA_CHECK_ARG(count >= (base ? 1 : 0) && count <= (base ? 3 : 2 * streams),
+                "lgs_streams_held: 1 to 3 outputs on stored streams, up to 2 s on the embedding");
+  LGA_CHECK_ARG(count == 0 || (y && mix && out), "lgs_streams_held: an output needs its mix matrix and weights");
+  LGA_CHECK_ARG(in && (h || h_bf16) && (norm_w || !h_bf16), "lgs_streams_held: a read with a place for it (bf16: made by the norm)");
+  lgs::HeldArgs p{};
+  p.tokens = tokens, p.table = table, p.w_f32 = w_f32, p.scale = scale, p.base = base, p.x = x;
+  for (int k = 0; k < count; ++k) {
+    LGA_CHECK_ARG(y[k] && mix[k] && out[k], "lgs_streams_held: an output needs its mix matrix and weights");
+    p.y[k] = y[k], p.mix[k] = mix[k], p.out[k] = out[k];
+  }
+  p.in = in, p.w = norm_w, p.h = h, p.h16 = (uint16_t*)h_bf16, p.eps = eps, p.W = W;
+  bool done = false;
+  if (streams == 2) done = lgs::streams_held_from<2>(p, T, count, stream);
+  else if (streams == 3) done = lgs::streams_held_from<3>(p, T, count, stream);
+  else done = lgs::streams_held_from<4>(p, T, count, stream);
+  LGA_CHECK_ARG(done, "lgs_streams_held: no such form");
   LGA_LAUNCH_RETURN();
 }
 

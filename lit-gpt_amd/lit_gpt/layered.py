@@ -136,13 +136,14 @@ class Sublayer(nn.Module):
         return rows > 8 and self.w_in.dtype == torch.bfloat16
 
     def forward(self, h: torch.Tensor, h16: Optional[torch.Tensor], step: StepBatch, cache) -> torch.Tensor:
-        """h (T, width): the normed read of the streams. Returns the sublayer's output (T, width) fp32."""
+        """h (T, width): the normed read of the streams (may be missing beside its bf16 copy h16). Returns the sublayer's output
+        (T, width) fp32."""
         n_in, W = self.w_in.shape
-        y = torch.empty(step.T, W, dtype=torch.float32, device=h.device)
+        y = torch.empty(step.T, W, dtype=torch.float32, device=self.w_in.device)
         if cache is None and self.b_in is None and not hooked(self.module) and \
                 self.module.forward_in(h if h16 is None else h16, self.w_in, y):
             return y
-        proj = torch.empty(step.T, n_in, dtype=torch.float32, device=h.device)
+        proj = torch.empty(step.T, n_in, dtype=torch.float32, device=self.w_in.device)
         seq_ops.linear(h if h16 is None else h16, self.w_in, M=step.T, N=n_in, K=W, y=proj, lda=W, ldy=n_in,
                        bias=self.b_in, ksplit=self.module.in_ksplit)
         if cache is None:
@@ -793,9 +794,12 @@ class LayeredGPT(nn.Module):
         last boundary reads the plain sum of the streams, which is returned. ``after_layer(run, x)``: a hook that
         sees the streams (T, s, width) after each layer run (for tests; it costs one extra launch per layer)."""
         eps = self.config.norm_eps
-        x = seq_ops.embed_streams(step.tokens, self.embed, self.config.embedding_scale, self.config.streams)
         chain = [(run, sub, self.caches[run] if k == 0 else None)
                  for run, layer in enumerate(self.runs) for k, sub in enumerate(self.blocks[layer].sublayers())]
+        if after_layer is None and seq_ops.streams_hold(step.T, self.config.width, self.config.streams, False) and \
+                not any(hooked(sub, sub.module) for _, sub, _ in chain):
+            return self._forward_held(step, chain)
+        x = seq_ops.embed_streams(step.tokens, self.embed, self.config.embedding_scale, self.config.streams)
         first = chain[0][1]
         got = seq_ops.streams_step(x, read=first.links.read, norm_w=first.norm_w, eps=eps,
                                    bf16_copy=first.wants_bf16(step.T))
@@ -813,6 +817,29 @@ class LayeredGPT(nn.Module):
             got = seq_ops.streams_step(x, read=nxt[1].links.read, norm_w=nxt[1].norm_w, eps=eps,
                                        bf16_copy=nxt[1].wants_bf16(step.T), **kw)
         raise AssertionError("unreachable")
+
+    def _forward_held(self, step: StepBatch, chain) -> torch.Tensor:
+        """The same values for prompts whose streams are seldom stored: a boundary makes them anew from where they last stood and
+        the sublayers' outputs since (none of which a hook sees). A bf16 input is all that a sublayer here reads."""
+        cfg, s = self.config, self.config.streams
+        T, W, eps = step.T, cfg.width, cfg.norm_eps
+        x, held = None, []
+
+        def boundary(sub, store):
+            nonlocal x, held
+            into = torch.empty(T, s, W, dtype=torch.float32, device=self.device) if store and x is None else x
+            b16 = sub is not None and sub.wants_bf16(T)
+            kw = dict(read=self.stream_ones) if sub is None else dict(read=sub.links.read, norm_w=sub.norm_w, eps=eps)
+            got = seq_ops.streams_held(step.tokens, self.embed, cfg.embedding_scale, x, held, want_f32=not b16, bf16_copy=b16,
+                                       store=into if store else None, **kw)
+            if store:
+                x, held = into, []
+            return got
+
+        for n, (_, sub, cache) in enumerate(chain):
+            h, h16 = boundary(sub, len(held) > 0 and len(held) == seq_ops.streams_hold(T, W, s, x is not None))
+            held.append((sub(h, h16, step, cache), sub.links.mix, sub.links.write))
+        return boundary(None, False)[0]
 
     @torch.inference_mode()
     def logits(self, x: torch.Tensor, rows: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -62,6 +62,7 @@ SIGNATURES = {
     "lgs_token_side": [_P, _P, _P, _I, _L, _I, _P, _P, _P, _I, _I, _I, _I, _F, _P],
     "lgs_embed_streams": [_P, _P, _I, _F, _P, _I, _I, _I, _I, _P],
     "lgs_streams_step": [_P, _P, _P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _P],
+    "lgs_streams_held": [_P, _P, _I, _F, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _F, _I, _I, _I, _P],
     "lgs_diffattn_prepare": [_P, _L, _I, _I, _I, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "lgs_attn_one_heads": [_I, _I, _I, _I, _I, _I],
     "lgs_diffattn": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _F,
@@ -659,6 +660,42 @@ def streams_step(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, mix: Opti
     if read is None:
         return None
     return (h, h16) if bf16_copy else h
+
+
+def streams_hold(T: int, W: int, streams: int, stored: bool) -> int:
+    """After how many sublayers a prompt's streams are stored: until then ``streams_held`` makes them anew (0: every boundary
+    stores them, by ``streams_step``). A boundary that stores reads and writes a row per stream, one that does not reads a row per
+    sublayer since: with s streams the fewest bytes are moved by storing every sqrt(2 s) sublayers, and, from the embedding, not
+    before 2 s. us of the embedding and nine boundaries of four streams, stored each / held: 2407 rows of 4096 926 / 425, 256 217 / 123,
+    33 197 / 119; of 2048 columns 423 / 277, 142 / 97, 125 / 97; five of two streams of 4096 281 / 139, 81 / 51, 62 / 50. Up to 32 rows
+    keep the step that gives a row 1024 threads."""
+    if T <= 32 or W > 4096 or not 2 <= streams <= 4:
+        return 0
+    return (2 if streams == 2 else 3) if stored else 2 * streams
+
+
+def streams_held(tokens: Optional[torch.Tensor], table: torch.Tensor, scale: float, base: Optional[torch.Tensor], held, *,
+                 read: torch.Tensor, norm_w: Optional[torch.Tensor] = None, eps: float = 0.0, want_f32: bool = True,
+                 bf16_copy: bool = False, store: Optional[torch.Tensor] = None):
+    """The next sublayer's input (h fp32 or None, h_bf16 or None) of a multi-stream residual that is not in memory: it stands at
+    ``base`` (T, s, W), or without one at the embedding of ``tokens`` in every stream, and ``held`` lists (y, mix, out) of the
+    sublayers since. ``store`` (T, s, W), which may be ``base``: the streams are stored there."""
+    s, W = read.numel(), table.shape[1]
+    T = base.shape[0] if base is not None else tokens.numel()
+    if not (want_f32 or bf16_copy) or (bf16_copy and norm_w is None) or (norm_w is not None and norm_w.numel() != W):
+        raise ValueError("streams_held: read shapes")
+    if any(t is not None and t.shape != (T, s, W) for t in (base, store)):
+        raise ValueError("streams_held: (rows, streams, width) expected")
+    if any(y.shape != (T, W) or mix.numel() != s * s or out.numel() != s for y, mix, out in held):
+        raise ValueError("streams_held: write-back shapes")
+    h = torch.empty(T, W, dtype=F32, device=read.device) if want_f32 else None
+    h16 = torch.empty(T, W, dtype=torch.bfloat16, device=read.device) if bf16_copy else None
+    ys, mixes, outs = ((_P * max(len(held), 1))(*(_dev(e[i], "held", F32) for e in held)) for i in range(3))
+    _check(load_library().lgs_streams_held(
+        None if base is not None else _dev(tokens, "tokens", I32), _dev(table, "table"), _wf32(table, "table"), float(scale),
+        table.shape[0], _opt(base, "base", F32), _opt(store, "store", F32), ys, mixes, outs, len(held), _dev(read, "read", F32),
+        _opt(norm_w, "norm_w", F32), _opt(h, "h", F32), _opt(h16, "h_bf16", torch.bfloat16), float(eps), T, W, s, _stream()))
+    return h, h16
 
 
 def diffattn_prepare(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, cache_k: Optional[torch.Tensor],

@@ -596,3 +596,67 @@ def test_checkpoint_folder_through_registry_and_runner(tmp_path):
     assert rel_err(got0, wa[[3, 9]]).max() < TOL32
     assert rel_err(got1, torch.stack([wa[10], wb[5]])).max() < TOL32
     assert rel_err(got3, wa[13:14]).max() < TOL32
+
+
+@pytest.mark.parametrize("T", [1, 37])
+@pytest.mark.parametrize("s,W", [(2, 300), (3, 1025), (4, 1024), (4, 4096), (2, 2049), (3, 4095)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_streams_held(s, W, T, dtype):
+    """Streams made anew from the embedding, or from stored ones, and the outputs since: the bits of a boundary after the other
+    (the 256-thread form, which takes 33 rows and more), stored or not, over ends of column blocks and every count of outputs."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(s + W)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device=dev)  # noqa: E731
+    table, tokens = draw(9, W).to(dtype), torch.randint(0, 9, (40,), generator=g, device=dev, dtype=torch.int32)
+    read, nw = draw(s), draw(W)
+    held = [(draw(40, W), 0.5 * draw(s, s), draw(s)) for _ in range(2 * s)]
+    x = seq_ops.embed_streams(tokens, table, 0.7, s)
+    want = [(seq_ops.streams_step(x, read=read, norm_w=nw, eps=1e-5, bf16_copy=True), x.clone())]
+    for y, mix, out in held:
+        want.append((seq_ops.streams_step(x, y=y, mix=mix, out=out, read=read, norm_w=nw, eps=1e-5, bf16_copy=True), x.clone()))
+    rows = lambda e: tuple(t[:T].contiguous() for t in e)  # noqa: E731
+    for base in range(2 * s):
+        for n in range(base + (base > 0), 2 * s + 1 if base == 0 else min(2 * s, base + 3) + 1):
+            start = want[base][1][:T].clone() if base else None
+            since = [(y[:T].contiguous(), mix, out) for y, mix, out in held[base:n]]
+            (h, h16), stands = rows(want[n][0]), want[n][1][:T]
+            form = dict(read=read, norm_w=nw, eps=1e-5)
+            got = seq_ops.streams_held(tokens[:T], table, 0.7, start, since, bf16_copy=True, **form)
+            assert torch.equal(got[0], h) and torch.equal(got[1], h16), (base, n)
+            if start is not None:
+                assert torch.equal(start, want[base][1][:T])
+            store = start if start is not None else torch.empty(T, s, W, device=dev)
+            got = seq_ops.streams_held(tokens[:T], table, 0.7, start, since, bf16_copy=True, want_f32=False, store=store, **form)
+            assert got[0] is None and torch.equal(got[1], h16) and torch.equal(store, stands), (base, n)
+    plain = seq_ops.streams_held(tokens[:T], table, 0.7, None, [(y[:T].contiguous(), m, o) for y, m, o in held], read=read)
+    assert torch.equal(plain[0], seq_ops.streams_step(x, read=read)[:T]) and plain[1] is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("streams,T", [(2, 33), (4, 33), (4, 300)])
+def test_prompt_whose_streams_are_not_stored(streams, dtype, T, monkeypatch):
+    """More sublayers than are gone through from the embedding and from two places where the streams were stored: the residual
+    of the boundaries that store each time, to the bit; a hook keeps those."""
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import StepBatch
+
+    cfg = make_cfg(MIXED * 3, streams=streams)
+    model, _ = build(cfg, dtype=dtype)
+    assert sum(len(b.sublayers()) for b in model.blocks) > 2 * streams + 6
+    toks = tokens_of(T, cfg["vocab"])
+    model.set_kv_cache(1, 320)
+    with torch.inference_mode():
+        step = StepBatch.build([(0, 0, toks)], model.device)
+        calls = []
+        whole, one = seq_ops.streams_step, seq_ops.streams_held
+        monkeypatch.setattr(seq_ops, "streams_held", lambda *a, **k: calls.append("held") or one(*a, **k))
+        monkeypatch.setattr(seq_ops, "streams_step", lambda *a, **k: calls.append("step") or whole(*a, **k))
+        got = model.forward_step(step)
+        assert set(calls) == {"held"}
+        handle = model.blocks[0].sub1.register_forward_hook(lambda *_: None)
+        hooked = model.forward_step(step)
+        handle.remove()
+        assert set(calls[len(calls) // 2:]) == {"step"}
+    assert torch.equal(got, hooked)
