@@ -234,20 +234,27 @@ __device__ __forceinline__ void attn_body(const uint16_t* __restrict__ q, uint16
     }
   }
   // merge the RGW row groups of this wave (lanes differing in the bits above log2(LPR))
-#pragma unroll
-  for (int off = LPR; off < 64; off <<= 1) {
+  auto merge = [&](auto distance) {
+    constexpr int D = decltype(distance)::value;  // (the lanes that count, below LPR, are the pairs' first ones)
 #pragma unroll
     for (int h = 0; h < QPK; ++h) {
-      const float mo = __shfl_xor(m[h], off), lo = __shfl_xor(l[h], off);
-      const float mn = fmaxf(m[h], mo);
-      const float ca = __builtin_amdgcn_exp2f(m[h] - mn);  // m >= kMFloor: finite, never exp(-inf - -inf)
-      const float cb = __builtin_amdgcn_exp2f(mo - mn);
-      l[h] = l[h] * ca + lo * cb;
+      const LanePair mp = lane_pair<D>(m[h]), lp = lane_pair<D>(l[h]);
+      const float mn = fmaxf(mp.a, mp.b);
+      const float ca = __builtin_amdgcn_exp2f(mp.a - mn);  // m >= kMFloor: finite, never exp(-inf - -inf)
+      const float cb = __builtin_amdgcn_exp2f(mp.b - mn);
+      l[h] = lp.a * ca + lp.b * cb;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[h][i] = o[h][i] * ca + __shfl_xor(o[h][i], off) * cb;
+      for (int i = 0; i < 8; ++i) {
+        const LanePair op = lane_pair<D>(o[h][i]);
+        o[h][i] = op.a * ca + op.b * cb;
+      }
       m[h] = mn;
     }
-  }
+  };
+  static_assert(LPR == 8 || LPR == 16, "lanes of a key row");
+  if constexpr (LPR == 8) merge(std::integral_constant<int, 8>{});
+  merge(std::integral_constant<int, 16>{});
+  merge(std::integral_constant<int, 32>{});
   __shared__ float sm[NW][QPK], sl[NW][QPK];
   __shared__ __attribute__((aligned(16))) float so[NW][QPK][HS];
   __shared__ unsigned s_ticket;

@@ -56,22 +56,98 @@ __device__ __forceinline__ void wait_loads(float (&v)[N]) {
 }
 
 // ---- wave-level reductions (64 lanes) ----
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+// Every lane's value and its partner's, lane ^ D away, in either order; in registers, where a shuffle goes through LDS, whose latency
+// a wave sum then has six times. All lanes of the wave take part. One-token steps, us by shuffles / here: pythia-160m fp32 303 / 291, 8
+// sequences of the 2048-wide delta-rule model 545 / 532, one of the state-space one 286 / 277, Llama-2-7B int4 1288 / 1270.
+struct LanePair {
+  float a, b;
+};
+template <int CTRL, int BANKS = 0xf>
+__device__ __forceinline__ float lane_dpp(float old, float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, 0xf, BANKS, false));
+}
+template <int D>
+__device__ __forceinline__ LanePair lane_pair(float v) {
+  static_assert(D == 32 || D == 16 || D == 8 || D == 4 || D == 2 || D == 1, "a power of two");
+  if constexpr (D == 32) {
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return {__uint_as_float(h[0]), __uint_as_float(h[1])};
+  } else if constexpr (D == 16) {
+    const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return {__uint_as_float(h[0]), __uint_as_float(h[1])};
+  } else if constexpr (D == 8) {
+    return {v, lane_dpp<0x128>(v, v)};  // row_ror:8
+  } else if constexpr (D == 4) {  // row_shl:4 in the even groups of four, row_shr:4 in the odd ones
+    return {v, lane_dpp<0x114, 0xa>(lane_dpp<0x104, 0x5>(v, v), v)};
+  } else {
+    return {v, lane_dpp<D == 2 ? 0x4E : 0xB1>(v, v)};  // quad_perm
+  }
+}
+// of two values at once: lanes with bit D clear get x's pair, the others y's
+template <int D>
+__device__ __forceinline__ LanePair lane_swap(float x, float y) {
+  static_assert(D == 32 || D == 16, "whole rows of 16 lanes");
+  if constexpr (D == 32) {
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return {__uint_as_float(h[0]), __uint_as_float(h[1])};
+  } else {
+    const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return {__uint_as_float(h[0]), __uint_as_float(h[1])};
+  }
+}
+// f over aligned groups of W lanes, the partners W / 2, ..., 2, 1 away: the same bits as by shuffles (f is commutative)
+template <int W, class F>
+__device__ __forceinline__ float lanes_fold(float v, F&& f) {
+  static_assert(W == 64 || W == 32 || W == 16 || W == 8 || W == 4 || W == 2, "a power of two");
+  auto step = [&](LanePair p) { return f(p.a, p.b); };
+  if constexpr (W >= 64) v = step(lane_pair<32>(v));
+  if constexpr (W >= 32) v = step(lane_pair<16>(v));
+  if constexpr (W >= 16) v = step(lane_pair<8>(v));
+  if constexpr (W >= 16) v = f(v, lane_dpp<0x124>(v, v));  // (row_ror:4: lanes 8 apart are equal by now)
+  else if constexpr (W >= 8) v = step(lane_pair<4>(v));
+  if constexpr (W >= 4) v = step(lane_pair<2>(v));
+  return step(lane_pair<1>(v));
+}
+// f over the lanes that share the bits below FROM, nearest first; f(a, b) of lanes without the bit: their own value, then the other's
+template <int FROM, class F>
+__device__ __forceinline__ float lanes_join(float v, F&& f) {
+  auto step = [&](LanePair p) { return f(p.a, p.b); };
+  if constexpr (FROM <= 1) v = step(lane_pair<1>(v));
+  if constexpr (FROM <= 2) v = step(lane_pair<2>(v));
+  if constexpr (FROM <= 4) v = step(lane_pair<4>(v));
+  if constexpr (FROM <= 8) v = step(lane_pair<8>(v));
+  if constexpr (FROM <= 16) v = step(lane_pair<16>(v));
+  if constexpr (FROM <= 32) v = step(lane_pair<32>(v));
   return v;
 }
+template <int FROM>
+__device__ __forceinline__ float lanes_join_sum(float v) {
+  return lanes_join<FROM>(v, [](float a, float b) { return a + b; });
+}
+// the largest value of the wave and its place (the lowest among equals), in every lane
+__device__ __forceinline__ void wave_best(float& v, int& i) {
+  auto step = [&](LanePair p, LanePair q) {
+    const int x = __float_as_int(q.a), y = __float_as_int(q.b);
+    const bool second = p.b > p.a || (p.b == p.a && y < x);
+    v = second ? p.b : p.a, i = second ? y : x;
+  };
+  step(lane_pair<32>(v), lane_pair<32>(__int_as_float(i)));
+  step(lane_pair<16>(v), lane_pair<16>(__int_as_float(i)));
+  step(lane_pair<8>(v), lane_pair<8>(__int_as_float(i)));
+  step(lane_pair<4>(v), lane_pair<4>(__int_as_float(i)));
+  step(lane_pair<2>(v), lane_pair<2>(__int_as_float(i)));
+  step(lane_pair<1>(v), lane_pair<1>(__int_as_float(i)));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  return lanes_fold<64>(v, [](float a, float b) { return a + b; });
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
+  return lanes_fold<64>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 // sum over aligned groups of `W` lanes (W power of two <= 64)
 template <int W>
 __device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  return lanes_fold<W>(v, [](float a, float b) { return a + b; });
 }
 
 // exact-order (no FMA contraction) helpers used where the reference's CPU math does mul then add. HIP's

@@ -50,16 +50,18 @@ __device__ __forceinline__ float butterfly(float* a, int lane) {
     const bool h = lane & D;
 #pragma unroll
     for (int i = 0; i < n; ++i) {
-      // the pair as register values first: on two loads of the array, LLVM folds the selects below into ONE load
-      // through a selected pointer, and the dynamically indexed array then lives in scratch (a store + load round
-      // trip per level in every wave's tail; round 6)
-      float lo = a[i], hi = a[i + n];
-      asm volatile("" : "+v"(lo), "+v"(hi));
-      const float send = h ? lo : hi, keep = h ? hi : lo;
-      float recv;
-      if (D == 8) recv = LGA_DPP(send, 0x128);  // row_ror:8 == xor 8 inside a 16-lane row
-      else recv = __shfl_xor(send, D);
-      a[i] = keep + recv;
+      if (D >= 16) {  // lanes without bit D keep a[i], the others a[i + n]: one exchange and one sum
+        const LanePair p = D == 32 ? lane_swap<32>(a[i], a[i + n]) : lane_swap<16>(a[i], a[i + n]);
+        a[i] = p.a + p.b;
+      } else {
+        // the pair as register values first: on two loads of the array, LLVM folds the selects below into ONE load
+        // through a selected pointer, and the dynamically indexed array then lives in scratch (a store + load round
+        // trip per level in every wave's tail)
+        float lo = a[i], hi = a[i + n];
+        asm volatile("" : "+v"(lo), "+v"(hi));
+        const float send = h ? lo : hi, keep = h ? hi : lo;
+        a[i] = keep + LGA_DPP(send, 0x128);  // row_ror:8 == xor 8 inside a 16-lane row
+      }
     }
   }
   float d = a[0];
@@ -68,7 +70,10 @@ __device__ __forceinline__ float butterfly(float* a, int lane) {
   d += LGA_DPP(d, 0x4E);
   d += LGA_DPP(d, 0x141);  // 8-lane groups done (R = 8)
   if (R <= 4) d += LGA_DPP(d, 0x140);  // 16-lane groups (R = 4)
-  if (R <= 2) d += __shfl_xor(d, 16);  // 32-lane groups (R = 2)
+  if (R <= 2) {  // 32-lane groups (R = 2)
+    const LanePair p = lane_pair<16>(d);
+    d = p.a + p.b;
+  }
   return d;
 }
 template <int R>

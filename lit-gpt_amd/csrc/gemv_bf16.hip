@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(256) gemv_bf16_kernel(GemvBArgs a) {
   if (DUAL) {
     // value index = 2*row + matrix: the fc_2 partner of a row sits in the lane whose value index differs in bit 0
     constexpr int PD = RB == 8 ? 8 : (RB == 4 ? 16 : 32);
-    const float other = PD == 8 ? LGA_DPP(tot, 0x128) : __shfl_xor(tot, PD);
+    const float other = lane_pair<PD>(tot).b;  // (used in lanes without that bit)
     const int row = row0 + (vi >> 1);
     if ((lane & (GROUP - 1)) == 0 && (vi & 1) == 0 && row < a.N) {
       const float g = round_bf(silu_f(round_bf(tot)));  // silu(bf16(fc_1 x)) -> bf16

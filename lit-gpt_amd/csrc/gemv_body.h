@@ -237,7 +237,7 @@ __device__ __forceinline__ void gemv_q4_body(GemvArgs a, int blk, unsigned char*
   if (DUAL) {
     // partner value (other matrix, same row) sits in the lane whose value index differs in bit 0
     constexpr int PD = R == 8 ? 8 : (R == 4 ? 16 : 32);
-    const float other = PD == 8 ? LGA_DPP(tot, 0x128) : __shfl_xor(tot, PD);
+    const float other = lane_pair<PD>(tot).b;  // (used in lanes without that bit)
     const int row = row0 + (vi >> 1);
     const float g = round_bf(silu_f(round_bf(tot)));  // silu(bf16(fc_1 x)) -> bf16
     const uint16_t ob = f2bf(__fmul_rn(g, round_bf(other)));  // * bf16(fc_2 x)

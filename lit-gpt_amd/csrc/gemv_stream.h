@@ -175,7 +175,7 @@ __device__ __forceinline__ void gemv_q4_stream(GemvArgs a, unsigned char* smem, 
     const int row0 = tile * RT;
     if (DUAL) {
       constexpr int PD = R == 8 ? 8 : (R == 4 ? 16 : 32);
-      const float other = PD == 8 ? LGA_DPP(tot, 0x128) : __shfl_xor(tot, PD);
+      const float other = lane_pair<PD>(tot).b;  // (used in lanes without that bit)
       const int row = row0 + (vi >> 1);
       const float gs = round_bf(silu_f(round_bf(tot)));
       const uint16_t ob = f2bf(__fmul_rn(gs, round_bf(other)));

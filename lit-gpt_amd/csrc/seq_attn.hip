@@ -537,6 +537,18 @@ __device__ __forceinline__ float attn_lanes_sum(float v) {
   return W == 16 ? attn_dpp<0x140>(v) : v;
 }
 
+// A value of map f, whose lanes are the first (f 0) or the last eight of sixteen and hold it alike, in all sixteen
+template <int MAPS>
+__device__ __forceinline__ float of_map(int f, float v) {
+  if (MAPS == 1) return v;
+  return f == 0 ? lane_dpp<0x128, 0xc>(v, v) : lane_dpp<0x128, 0x3>(v, v);  // row_ror:8 into the other half
+}
+
+// x f over the wave's four groups of 16 lanes, for the lanes of the first one
+__device__ __forceinline__ float groups_sum(float x, float f) {
+  return lanes_join_sum<32>(fmaf(x, f, lane_pair<16>(mul_rn(x, f)).b));
+}
+
 // One token per sequence over bf16 caches whose key and value rows are 128 values (MAPS maps of 128 / MAPS, dv 128): grid
 // (B, H / HG, splits), HG query heads of one key head per workgroup. A key belongs to 16 lanes, 16 bytes of its key and
 // of its value row each; each of the workgroup's 16 such groups takes every 16th key, four at a time, whose loads are
@@ -612,15 +624,14 @@ __global__ void __launch_bounds__(256) attn_one_kernel(AttnArgs p) {
       l[h] = l[h] * a + sum;
       m[h] = mn;
 #pragma unroll
-      for (int f = 0; f < MAPS; ++f) {  // (the other map's weights lie with the lanes eight away)
+      for (int f = 0; f < MAPS; ++f) {
         const int r = h * MAPS + f;
-        const int src = (lane & ~15) | (f * 8);
-        const float ar = MAPS == 2 ? __shfl(a, src) : a;
+        const float ar = of_map<MAPS>(f, a);
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[r][e] *= ar;
 #pragma unroll
         for (int i = 0; i < U; ++i) {
-          const float wr = MAPS == 2 ? __shfl(w[h][i], src) : w[h][i];
+          const float wr = of_map<MAPS>(f, w[h][i]);
           const float vv[8] = {bflo(v4[i].x), bfhi(v4[i].x), bflo(v4[i].y), bfhi(v4[i].y),
                                bflo(v4[i].z), bfhi(v4[i].z), bflo(v4[i].w), bfhi(v4[i].w)};
 #pragma unroll
@@ -631,21 +642,17 @@ __global__ void __launch_bounds__(256) attn_one_kernel(AttnArgs p) {
   }
 #pragma unroll
   for (int h = 0; h < HG; ++h) {  // the wave's four groups
-    const float top = fmaxf(fmaxf(m[h], __shfl_xor(m[h], 16)), fmaxf(__shfl_xor(m[h], 32), __shfl_xor(m[h], 48)));
+    const float top = lanes_join<16>(m[h], [](float x, float y) { return fmaxf(x, y); });
     const float a = m[h] == -INFINITY ? 0.0f : expf(m[h] - top);
-    float s = l[h] * a;
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
+    const float s = groups_sum(l[h], a);
 #pragma unroll
     for (int f = 0; f < MAPS; ++f) {
-      const int r = h * MAPS + f, src = (lane & ~15) | (f * 8);
-      const float ar = MAPS == 2 ? __shfl(a, src) : a, tr = MAPS == 2 ? __shfl(top, src) : top, sr = MAPS == 2 ? __shfl(s, src) : s;
+      const int r = h * MAPS + f;
+      const float ar = of_map<MAPS>(f, a), tr = of_map<MAPS>(f, top), sr = of_map<MAPS>(f, s);
       if (lane == 0) ml[wave][r][0] = tr, ml[wave][r][1] = sr;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        float v = acc[r][e] * ar;
-        v += __shfl_xor(v, 16);
-        v += __shfl_xor(v, 32);
+        const float v = groups_sum(acc[r][e], ar);
         if (lane < 16) sums[wave][r][l16 * 8 + e] = v;
       }
     }

@@ -100,15 +100,7 @@ __global__ void __launch_bounds__(64) moe_route_kernel(const float* __restrict__
         bi = i;
       }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ob > best || (ob == best && oi < bi)) {
-        best = ob;
-        bi = oi;
-      }
-    }
+    wave_best(best, bi);
     if (k == 0) first = best;
     const float w = expf(best - first);  // the first pick is the maximum
     den += w;
@@ -187,27 +179,22 @@ __device__ __forceinline__ void route_scores_wave(const float* z, int E, int top
     }
   }
   for (int k = 0; k < top; ++k) {
-    float best = -INFINITY, bs = 0.0f;
+    float best = -INFINITY;
     int bi = 0x7fffffff;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = lane + 64 * e;
       if (i < E && (c[e] > best || (c[e] == best && i < bi))) {
         best = c[e];
-        bs = s[e];
         bi = i;
       }
     }
+    wave_best(best, bi);
+    const int at = __builtin_amdgcn_readfirstlane(bi);
+    float bs = 0.0f;  // the chosen one's score, out of its lane
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o), os = __shfl_xor(bs, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ob > best || (ob == best && oi < bi)) {
-        best = ob;
-        bs = os;
-        bi = oi;
-      }
-    }
+    for (int e = 0; e < 4; ++e)
+      if (at >> 6 == e) bs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[e]), at & 63));
     if (lane == 0) {
       ids[k] = min(bi, E - 1);  // (where all are NaN, none is best)
       wts[k] = (square ? bs * bs : bs) * wscale;

@@ -1003,14 +1003,11 @@ __global__ void __launch_bounds__(256) latent_attention_tile_kernel(LatTileArgs 
       const int key = kt * 16 + fr;
       if (key > prow[j] || (p.window > 0 && key + p.window <= prow[j])) sc = -INFINITY;
       float mx = sc;
-#pragma unroll
-      for (int x = 8; x > 0; x >>= 1) mx = fmaxf(mx, __shfl_xor(mx, x));
+      mx = lanes_fold<16>(mx, [](float a, float b) { return fmaxf(a, b); });
       const float mn = fmaxf(m[j], mx);
       // (a window's first tile may hold no key of a row: its maximum is then still -inf)
       const float w = mn == -INFINITY ? 0.0f : expf(sc - mn);
-      float sum = w;
-#pragma unroll
-      for (int x = 8; x > 0; x >>= 1) sum += __shfl_xor(sum, x);
+      const float sum = group_sum<16>(w);
       corr[j] = mn == -INFINITY ? 0.0f : expf(m[j] - mn);
       l[j] = l[j] * corr[j] + sum;
       m[j] = mn;

@@ -561,8 +561,7 @@ __global__ void __launch_bounds__(256) channel_scan_kernel(ChanArgs p) {
             for (int r = part; r < p.rank; r += L) acc = fmaf(xr[r], wload<WF32>(p.w_dt, (size_t)c * p.rank + r), acc);
           }
         }
-#pragma unroll
-        for (int x = CW; x < 64; x <<= 1) acc += __shfl_xor(acc, x);
+        acc = lanes_join_sum<CW>(acc);
         d = acc + bias;
       }
       d = softplus_f(d);
@@ -576,8 +575,7 @@ __global__ void __launch_bounds__(256) channel_scan_kernel(ChanArgs p) {
         if (MODE != 1) acc = fmaf(S[i], Bt[NP + i], acc);
       }
       if (MODE != 1) {
-#pragma unroll
-        for (int x = CW; x < 64; x <<= 1) acc += __shfl_xor(acc, x);
+        acc = lanes_join_sum<CW>(acc);
         if (part == 0 && live) {
           const float zz = zv[t];
           const float v = fmaf(Dc, xv[t], acc) * (zz / (1.0f + expf(-zz)));
