@@ -18,6 +18,8 @@
 //   lga_f32_attention_decode  the two above for one token in one launch
 // (the token-embedding gather is lga_embedding over the fp32 rows as pairs of 16-bit words — a byte copy; greedy
 // sampling is lga_argmax_f32 in sample.hip)
+#include <type_traits>
+
 #include "gemm_tiles.h"
 
 namespace lga {
@@ -263,15 +265,16 @@ static void f32_linear_tiles(const float* x, const float* w, const float* bias, 
 template <int CPT>
 __device__ __forceinline__ void f32_row_stats(const float* __restrict__ xr, int n, float (&r)[CPT], float (&red)[4],
                                               float& mean, float& var) {
+  const int at = threadIdx.x;
   float s = 0.0f;
 #pragma unroll
   for (int e = 0; e < CPT; ++e) {
-    const int i = threadIdx.x + 256 * e;
+    const int i = at + 256 * e;
     r[e] = i < n ? xr[i] : 0.0f;
   }
 #pragma unroll
   for (int e = 0; e < CPT; ++e) s += r[e];
-  for (int i = threadIdx.x + 256 * CPT; i < n; i += 256) s += xr[i];
+  for (int i = at + 256 * CPT; i < n; i += 256) s += xr[i];
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
@@ -280,10 +283,10 @@ __device__ __forceinline__ void f32_row_stats(const float* __restrict__ xr, int 
   float ss = 0.0f;
 #pragma unroll
   for (int e = 0; e < CPT; ++e) {
-    const float d = threadIdx.x + 256 * e < n ? r[e] - mean : 0.0f;
+    const float d = at + 256 * e < n ? r[e] - mean : 0.0f;
     ss = fmaf(d, d, ss);
   }
-  for (int i = threadIdx.x + 256 * CPT; i < n; i += 256) {
+  for (int i = at + 256 * CPT; i < n; i += 256) {
     const float d = xr[i] - mean;
     ss = fmaf(d, d, ss);
   }
@@ -329,9 +332,9 @@ __global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restr
 }
 
 // One row, K a multiple of 4: up to two products of a norm of the row each (f32_linear_kernel of f32_layernorm_kernel's row, to
-// the bit). A workgroup makes its norm anew, in LDS, a wave then one output after the other. The first weights are loaded ahead of the
-// row, and loads return in order: the statistics wait for both, the sums for nothing more. pythia-160m (768 -> 2304 and 3072):
-// norms and products in three launches 16.2 us, in this one 7.6.
+// the bit), a wave one output after the other. The first weights are loaded ahead of the row, and loads return in order: the
+// statistics wait for both, the sums for nothing more. pythia-160m (768 -> 2304 and 3072): norms and products in three launches 16.2
+// us, in this one 7.6 with a workgroup's norm in LDS and 7.3 with a wave's in registers.
 struct F32NormLinear {
   const float *nw, *nb;
   float eps;
@@ -346,55 +349,113 @@ struct F32NormLinears {
   F32NormLinear p[2];
 };
 constexpr int kF32Chunks = 4;  // 256 columns each: a wave's loads in flight
-__device__ __forceinline__ void f32_load_chunks(const float* row, int c0, int K, int lane, float4 (&v)[kF32Chunks]) {
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
+typedef float f32x2_any_t __attribute__((ext_vector_type(2), aligned(4)));
+// 16 bytes of a row, or of a vector, whose address (of any float) is the same for the wave; k: a lane's columns, those past the last four
+// are theirs
+__device__ __forceinline__ f32x4_t f32_load4(const float* row, int k, int K) {
+  return *(const f32x4_any_t*)((const char*)row + (unsigned)min(k, K - 4) * 4u);
+}
+__device__ __forceinline__ void f32_load_chunks(const float* row, int c0, int K, int lane, f32x4_t (&v)[kF32Chunks]) {
+#pragma unroll
+  for (int c = 0; c < kF32Chunks; ++c)
+    if ((c0 + c) * 256 < K) v[c] = f32_load4(row, (c0 + c) * 256 + lane * 4, K);
+}
+__device__ __forceinline__ void f32_fma4(const f32x4_t& x, const f32x4_t& w, f32x4_t& acc) {
+  acc.x = fmaf(x.x, w.x, acc.x), acc.y = fmaf(x.y, w.y, acc.y), acc.z = fmaf(x.z, w.z, acc.z), acc.w = fmaf(x.w, w.w, acc.w);
+}
+__device__ __forceinline__ void f32_dot_chunks(const float* xr, int c0, int K, int lane, const f32x4_t (&w)[kF32Chunks], f32x4_t& acc) {
 #pragma unroll
   for (int c = 0; c < kF32Chunks; ++c) {
     const int k = (c0 + c) * 256 + lane * 4;
-    if (k < K) v[c] = *(const float4*)(row + k);
+    if (k < K) f32_fma4(*(const f32x4_t*)(xr + k), w[c], acc);
   }
 }
-__device__ __forceinline__ void f32_dot_chunks(const float* xr, int c0, int K, int lane, const float4 (&w)[kF32Chunks], float4& acc) {
+__device__ __forceinline__ float f32_dot_end(const f32x4_t& a) { return wave_sum((a.x + a.y) + (a.z + a.w)); }
+// the sum of f32_row_stats over a wave's row, whose lanes hold four neighbouring columns of every 256: s[j] belongs to thread 4 lane + j
+__device__ __forceinline__ float f32_row_sum(f32x4_t s) {
 #pragma unroll
-  for (int c = 0; c < kF32Chunks; ++c) {
-    const int k = (c0 + c) * 256 + lane * 4;
-    if (k < K) f32_fma4(*(const float4*)(xr + k), w[c], acc);
+  for (int j = 0; j < 4; ++j) {
+    const LanePair p = lane_pair<8>(s[j]);
+    float v = p.a + p.b;
+    v += lane_dpp<0x124>(v, v);  // (row_ror:4: lanes eight apart are equal)
+    v += lane_pair<2>(v).b;
+    s[j] = v + lane_pair<1>(v).b;
   }
+  return lanes_join_sum<16>((s[0] + s[2]) + (s[1] + s[3]));
 }
+
+// Up to 1024 columns (CPT 4) every wave makes the norm for itself, in registers, with no barrier among them; longer rows stand in LDS
 template <int CPT>
 __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a) {
   extern __shared__ __attribute__((aligned(16))) float xn[];  // [K]
-  __shared__ float red[4];
   const bool second = (int)blockIdx.x >= a.p[0].blocks;
   const F32NormLinear p = second ? a.p[1] : a.p[0];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, K = a.K;
-  int n = ((int)blockIdx.x - (second ? a.p[0].blocks : 0)) * 4 + wave;
-  float4 w[kF32Chunks];
+  const int block = (int)blockIdx.x - (second ? a.p[0].blocks : 0), K = a.K;
+  const float* x = a.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  int n = block * 4 + wave;
+  f32x4_t w[kF32Chunks];
   if (n < p.N) f32_load_chunks(p.w + (size_t)n * K, 0, K, lane, w);
   float bias = n < p.N && p.b ? p.b[n] : 0.0f;
-  float r[CPT], nw[CPT], nb[CPT], mean, var;
+  f32x4_t v[kF32Chunks];
+  if constexpr (CPT == kF32Chunks) {
+    if (n >= p.N) return;
+    f32x4_t nw[kF32Chunks], nb[kF32Chunks], s = {0.0f, 0.0f, 0.0f, 0.0f}, ss = s;
+    f32_load_chunks(x, 0, K, lane, v);
+    f32_load_chunks(p.nw, 0, K, lane, nw);
+    if (p.nb) f32_load_chunks(p.nb, 0, K, lane, nb);
 #pragma unroll
-  for (int e = 0; e < CPT; ++e) {
-    const int i = threadIdx.x + 256 * e;
-    nw[e] = i < K ? p.nw[i] : 0.0f;
-    nb[e] = i < K && p.nb ? p.nb[i] : 0.0f;
-  }
-  f32_row_stats<CPT>(a.x, K, r, red, mean, var);
-  const float rstd = 1.0f / sqrtf(var + p.eps);
+    for (int c = 0; c < kF32Chunks; ++c)
+      if (c * 256 + lane * 4 < K) s += v[c];
+    const float mean = f32_row_sum(s) / (float)K;
 #pragma unroll
-  for (int e = 0; e < CPT; ++e) {
-    const int i = threadIdx.x + 256 * e;
-    if (i < K) xn[i] = f32_normed(r[e], mean, rstd, nw[e], p.nb, nb[e]);
+    for (int c = 0; c < kF32Chunks; ++c)
+      if (c * 256 + lane * 4 < K) {
+        const f32x4_t d = v[c] - mean;
+        f32_fma4(d, d, ss);
+      }
+    const float rstd = 1.0f / sqrtf(f32_row_sum(ss) / (float)K + p.eps);
+#pragma unroll
+    for (int c = 0; c < kF32Chunks; ++c)
+      if (c * 256 < K)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[c][j] = f32_normed(v[c][j], mean, rstd, nw[c][j], p.nb, p.nb ? nb[c][j] : 0.0f);
+  } else {
+    __shared__ float red[4];
+    const int at = threadIdx.x;
+    float r[CPT], nw[CPT], nb[CPT], mean, var;
+#pragma unroll
+    for (int e = 0; e < CPT; ++e) {
+      const int i = at + 256 * e;
+      nw[e] = i < K ? p.nw[i] : 0.0f;
+      nb[e] = i < K && p.nb ? p.nb[i] : 0.0f;
+    }
+    f32_row_stats<CPT>(x, K, r, red, mean, var);
+    const float rstd = 1.0f / sqrtf(var + p.eps);
+#pragma unroll
+    for (int e = 0; e < CPT; ++e) {
+      const int i = at + 256 * e;
+      if (i < K) xn[i] = f32_normed(r[e], mean, rstd, nw[e], p.nb, nb[e]);
+    }
+    for (int i = at + 256 * CPT; i < K; i += 256) xn[i] = f32_normed(x[i], mean, rstd, p.nw[i], p.nb, p.nb ? p.nb[i] : 0.0f);
+    __syncthreads();
   }
-  for (int i = threadIdx.x + 256 * CPT; i < K; i += 256) xn[i] = f32_normed(a.x[i], mean, rstd, p.nw[i], p.nb, p.nb ? p.nb[i] : 0.0f);
-  __syncthreads();
   for (const int step = p.blocks * 4; n < p.N; n += step) {
-    float4 a4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    f32x4_t a4 = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int c0 = 0; c0 * 256 < K; c0 += kF32Chunks) {
-      f32_dot_chunks(xn, c0, K, lane, w, a4);
+      if constexpr (CPT == kF32Chunks) {
+#pragma unroll
+        for (int c = 0; c < kF32Chunks; ++c)
+          if (c * 256 + lane * 4 < K) f32_fma4(v[c], w[c], a4);
+      } else {
+        f32_dot_chunks(xn, c0, K, lane, w, a4);
+      }
       const bool more = (c0 + kF32Chunks) * 256 < K;
       if (more || n + step < p.N) f32_load_chunks(p.w + (size_t)(more ? n : n + step) * K, more ? c0 + kF32Chunks : 0, K, lane, w);
     }
-    float acc = wave_sum((a4.x + a4.y) + (a4.z + a4.w));
+    float acc = f32_dot_end(a4);
     if (lane == 0) {
       if (p.b) acc += bias;
       if (p.act) acc = gelu_f32(acc, p.act == 2);
@@ -405,13 +466,13 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 }
 
 // One row: y = ((x2 W2^T + b2) + (x1 W1^T + b1)) + res, a wave per output, both products in f32_linear_kernel's order. Bound by
-// latency: the weights of a block of 768 columns beside 3072 are in flight at once. Two launches 13.7 us, one 8.0. AHEAD: x2 and an
+// latency: the weights of a block of 768 columns beside 3072 are in flight at once. E2 > 0: x2 (of up to 1024 E2 values) and an
 // attention's ranges come ahead of the weights, so that the join waits for nothing else, and x2 is read once for a workgroup's four
-// outputs; the weights then start later, and a workgroup holds LDS, which rows of up to 3072 values make up for in a model's chain of
-// launches and longer ones do not (us a token behind 300 keys, weights first / AHEAD: pythia-160m 307.9 / 303.6, pythia-410m 694 / 742,
-// pythia-1b 1234 / 1318; alone, weights from memory, 768 columns beside 3072 7.4 / 8.2, 1024 beside 4096 9.7 / 12.5, 2048 beside 8192
-// 31.3 / 35.9). Nor where x1 is longer than the block: 2240 columns beside 1280 9.8 / 13.0, 2560 beside 704 10.5 / 14.0.
-constexpr int kF32AheadMost = 3072;  // (values of x2)
+// outputs (kept in registers until LDS has them: as an array of HIP's float4 they went through scratch memory, a trip of their own
+// ahead of all weights). Weights from memory, an attention in five ranges, us without / with: 768 columns beside 3072 9.4 / 9.5, 1024
+// beside 4096 10.2 / 9.6, 1600 beside 6400 24.2 / 18.1, 2048 beside 8192 30.0 / 24.3, in one range 23.3 / 18.2; a token behind 300 keys:
+// pythia-160m 300 / 275, pythia-410m 676 / 606, pythia-1b 1101 / 1008. Not where x1 is no shorter than half of x2: 4096 beside 4096 in
+// five ranges 47.8 / 66.4, 2240 beside 1280 9.8 / 10.3.
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
   float* y;
@@ -426,19 +487,20 @@ struct F32Parts {
   float o[E][P], m[P], l[P];  // (of the thread's first columns, and of head threadIdx.x)
 };
 __device__ __forceinline__ void f32_load_parts(const F32LinearsSum& a, F32Parts& p) {
-  const int H = a.K1 / a.hs, h = min((int)threadIdx.x, H - 1);
+  const int H = a.K1 / a.hs;
+  const unsigned h = (unsigned)min((int)threadIdx.x, H - 1) * 8u;
+  unsigned at[F32Parts::E];  // (columns past the last one are its)
+#pragma unroll
+  for (int e = 0; e < F32Parts::E; ++e) at[e] = (unsigned)min((int)threadIdx.x + 256 * e, a.K1 - 1) * 4u;
 #pragma unroll
   for (int s = 0; s < F32Parts::P; ++s) {
-    p.m[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2] : -INFINITY;
-    p.l[s] = s < a.parts ? a.ml[((size_t)s * H + h) * 2 + 1] : -1.0f;
+    p.m[s] = -INFINITY, p.l[s] = -1.0f;
+    if (s >= a.parts) continue;
+    const f32x2_any_t ml = *(const f32x2_any_t*)((const char*)(a.ml + (size_t)s * H * 2) + h);
+    p.m[s] = ml.x, p.l[s] = ml.y;
+#pragma unroll
+    for (int e = 0; e < F32Parts::E; ++e) p.o[e][s] = *(const float*)((const char*)(a.x1 + (size_t)s * a.K1) + at[e]);
   }
-#pragma unroll
-  for (int e = 0; e < F32Parts::E; ++e)
-#pragma unroll
-    for (int s = 0; s < F32Parts::P; ++s) {
-      const int i = threadIdx.x + 256 * e;
-      p.o[e][s] = i < a.K1 && s < a.parts ? a.x1[(size_t)s * a.K1 + i] : 0.0f;
-    }
 }
 __device__ __forceinline__ void f32_join_parts(const F32LinearsSum& a, const F32Parts& p, float* xs, float* wt) {
   constexpr int E = F32Parts::E, P = F32Parts::P;
@@ -474,19 +536,19 @@ __device__ __forceinline__ void f32_join_parts(const F32LinearsSum& a, const F32
   for (int i = threadIdx.x + 256 * E; i < a.K1; i += 256) join(i, [&](int s) { return a.x1[(size_t)s * a.K1 + i]; });
   __syncthreads();
 }
-template <bool PARTS, bool AHEAD>
+template <bool PARTS, int E2>
 __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
   extern __shared__ __attribute__((aligned(16))) float xs[];  // [K1] the joined row, then the ranges' weights; or [K1]; x2
-  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), n = min(row, a.N - 1);
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = min(row, a.N - 1);
   const float *r1 = a.w1 + (size_t)n * a.K1, *r2 = a.w2 + (size_t)n * a.K2;
-  constexpr int E2 = AHEAD ? kF32AheadMost / 1024 : 0;
-  float4 x2[E2 > 0 ? E2 : 1];
+  constexpr bool AHEAD = E2 > 0;
+  f32x4_t x2[E2 > 0 ? E2 : 1];
 #pragma unroll
-  for (int e = 0; e < E2; ++e) x2[e] = *(const float4*)(a.x2 + min((int)(threadIdx.x + 256 * e) * 4, a.K2 - 4));
+  for (int e = 0; e < E2; ++e) x2[e] = f32_load4(a.x2, (threadIdx.x + 256 * e) * 4, a.K2);
   F32Parts parts;
   if (PARTS && AHEAD) f32_load_parts(a, parts);
   __builtin_amdgcn_sched_barrier(0);
-  float4 w1[kF32Chunks], w2[3][kF32Chunks];
+  f32x4_t w1[kF32Chunks], w2[3][kF32Chunks];
   f32_load_chunks(r1, 0, a.K1, lane, w1);
 #pragma unroll
   for (int u = 0; u < 3; ++u) f32_load_chunks(r2, u * kF32Chunks, a.K2, lane, w2[u]);
@@ -499,7 +561,7 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
 #pragma unroll
     for (int e = 0; e < E2; ++e) {
       const int k = (threadIdx.x + 256 * e) * 4;
-      if (k < a.K2) *(float4*)(to + k) = x2[e];
+      if (k < a.K2) *(f32x4_t*)(to + k) = x2[e];
     }
     px2 = to;
   }
@@ -509,7 +571,7 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
   } else if (AHEAD) {
     __syncthreads();
   }
-  float4 h4 = make_float4(0.f, 0.f, 0.f, 0.f), m4 = h4;
+  f32x4_t h4 = {0.0f, 0.0f, 0.0f, 0.0f}, m4 = h4;
   for (int c0 = 0; c0 * 256 < a.K1; c0 += kF32Chunks) {
     if (c0 > 0) f32_load_chunks(r1, c0, a.K1, lane, w1);
     f32_dot_chunks(px1, c0, a.K1, lane, w1, h4);
@@ -522,7 +584,7 @@ __global__ void __launch_bounds__(256) f32_linears_sum_kernel(F32LinearsSum a) {
 #pragma unroll
     for (int u = 0; u < 3; ++u) f32_dot_chunks(px2, c0 + u * kF32Chunks, a.K2, lane, w2[u], m4);
   }
-  float h = wave_sum((h4.x + h4.y) + (h4.z + h4.w)), m = wave_sum((m4.x + m4.y) + (m4.z + m4.w));
+  float h = f32_dot_end(h4), m = f32_dot_end(m4);
   if (lane == 0 && row < a.N) {
     if (a.b1) h += b1;
     if (a.b2) m += b2;
@@ -626,8 +688,11 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   // this workgroup's keys, of as many ranges as there are keys for
   const int chunk = FUSED && a.parts > 1 ? f32_attention_chunk(L, a.parts) : L, lo = range * chunk, hi = min(lo + chunk, L);
   const bool mine = sub * 4 < hs;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto row = [&](const float* base, int j) { return mine ? *(const float4*)(base + (size_t)min(j, L - 1) * hs + sub * 4) : zero; };
+  // (the last columns again for a lane past them, its values cleared: a choice of addresses, one of them a constant's, makes the compiler load
+  // through the generic aperture, in two pieces; pythia-160m at 301 keys 6.7 us so, 5.3 as it is)
+  const int at = mine ? sub * 4 : hs - 4;
+  auto kept = [&](float4 v) { return make_float4(mine ? v.x : 0.0f, mine ? v.y : 0.0f, mine ? v.z : 0.0f, mine ? v.w : 0.0f); };
+  auto row = [&](const float* base, int j) { return kept(*(const float4*)(base + (size_t)min(j, L - 1) * hs + at)); };
   // the token's q, k, v and angles, and behind them the first keys and values (of a fused range all of them), on their way
   // together. (The fused form's own row is read here before it is written, and not used.)
   float4 k[4], v[4];
@@ -672,12 +737,12 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
     for (int d = threadIdx.x; d < hs; d += 512) qs[d] = qr[d];
   }
   __syncthreads();
-  const float4 q4 = mine ? *(const float4*)(qs + sub * 4) : zero;
+  const float4 q4 = kept(*(const float4*)(qs + at));
   auto own = [&](float4 (&x)[4], const float* row, int j0) {
     if (!FUSED || !mine) return;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (j0 + u * STEP == L - 1) x[u] = *(const float4*)(row + sub * 4);
+      if (j0 + u * STEP == L - 1) x[u] = kept(*(const float4*)(row + at));
   };
   float mx = -INFINITY;
   for (int j0 = lo + first; j0 < hi; j0 += 4 * STEP) {
@@ -714,7 +779,7 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
   if (lane == 0) red[wave] = sum;
   __syncthreads();
   sum = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
-  float4 o = zero;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int j0 = lo + first; j0 < hi; j0 += 4 * STEP) {
     if (!FUSED || j0 != lo + first) {
 #pragma unroll
@@ -728,13 +793,14 @@ __global__ void __launch_bounds__(512) f32_attention_vec_kernel(F32AttnArgs a) {
       if (j < hi) o.x = fmaf(w, v[u].x, o.x), o.y = fmaf(w, v[u].y, o.y), o.z = fmaf(w, v[u].z, o.z), o.w = fmaf(w, v[u].w, o.w);
     }
   }
-#pragma unroll
-  for (int x = 32; x >= LPK; x >>= 1) {
-    o.x += __shfl_xor(o.x, x);
-    o.y += __shfl_xor(o.y, x);
-    o.z += __shfl_xor(o.z, x);
-    o.w += __shfl_xor(o.w, x);
-  }
+  auto fold = [&](float v) {  // over the lanes of other keys, the farthest first
+    auto add = [](LanePair p) { return p.a + p.b; };
+    if constexpr (LPK <= 32) v = add(lane_pair<32>(v));
+    if constexpr (LPK <= 16) v = add(lane_pair<16>(v));
+    return v;
+  };
+  static_assert(LPK >= 16, "lanes of a key");
+  o = make_float4(fold(o.x), fold(o.y), fold(o.z), fold(o.w));
   __syncthreads();  // the weights are read
   float* part = sc;
   if (lane < LPK && mine) *(float4*)(part + wave * hs + sub * 4) = o;
@@ -845,8 +911,13 @@ extern "C" int lga_f32_norm_linears(const float* x, int K, const float* nw1, con
                 "lga_f32_norm_linears: bad arguments");
   LGA_CHECK_ARG(K % 4 == 0 && K <= 8192 && ((uintptr_t)w1 | (uintptr_t)w2) % 16 == 0,
                 "lga_f32_norm_linears: K a multiple of 4 up to 8192 and 16-B aligned weights needed");
-  // (2048 workgroups fill the chip: beyond, a workgroup's norm serves several outputs a wave)
-  auto blocks = [](int N) { return std::min((N + 3) / 4, 2048); };
+  // One output a wave up to 2048 workgroups; beyond, a wave makes as many outputs as any other or one less, on workgroups that stand on the
+  // chip side by side. Weights from memory, 50304 outputs of 768, 1024, 2048 and 2560 columns, us in 2048 / 1280 workgroups: 34.3 / 29.7,
+  // 40.2 / 36.3, 87 / 70, 109 / 88 (1536 as 2048 or worse, 3072 within 2 % of 1280); 6144 and 8192 of 2048 in two each lose 4 %.
+  auto blocks = [](int N) {
+    const int all = (N + 3) / 4, each = all > 2048 ? (all + 1279) / 1280 : 1;
+    return (all + each - 1) / each;
+  };
   const lga::F32NormLinears a{x, K, {{nw1, nb1, eps1, w1, b1, act1, y1, N1, blocks(N1)}, {nw2, nb2, eps2, w2, b2, act2, y2, N2, blocks(N2)}}};
   const unsigned grid = (unsigned)(blocks(N1) + blocks(N2));
   if (K <= 1024) lga::f32_norm_linears_kernel<4><<<grid, 256, K * sizeof(float), stream>>>(a);
@@ -864,10 +935,13 @@ extern "C" int lga_f32_linears_sum(const float* x1, const float* ml, int parts, 
                 "lga_f32_linears_sum: 1 to 8 ranges of up to 256 heads, 8192 columns");
   const lga::F32LinearsSum a{x1, w1, b1, x2, w2, b2, residual, y, N, K1, K2, ml, parts, hs};
   const size_t joined = parts > 1 ? (size_t)K1 + (K1 / hs * 9 + 3) / 4 * 4 : 0;
-  const bool ahead = K1 <= 768 && K2 <= lga::kF32AheadMost;
+  const int ahead = K1 > K2 / 2 || K2 > 8192 ? 0 : K2 <= 4096 ? 4 : 8;
   const size_t lds = (joined + (ahead ? K2 : 0)) * sizeof(float);
-  const auto kernel = parts > 1 ? (ahead ? lga::f32_linears_sum_kernel<true, true> : lga::f32_linears_sum_kernel<true, false>)
-                                : (ahead ? lga::f32_linears_sum_kernel<false, true> : lga::f32_linears_sum_kernel<false, false>);
+  auto go = [&](auto many) {
+    constexpr bool PARTS = decltype(many)::value;
+    return ahead == 0 ? lga::f32_linears_sum_kernel<PARTS, 0> : ahead == 4 ? lga::f32_linears_sum_kernel<PARTS, 4> : lga::f32_linears_sum_kernel<PARTS, 8>;
+  };
+  const auto kernel = parts > 1 ? go(std::true_type{}) : go(std::false_type{});
   kernel<<<(N + 3) / 4, 256, lds, stream>>>(a);
   LGA_LAUNCH_RETURN();
 }

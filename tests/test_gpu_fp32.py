@@ -97,6 +97,10 @@ def test_one_row_norms_and_products(K, N1, N2, bias):
     parts = [(norms[0], linears[0], None)] + [(norms[1], linears[1], "tanh")] * (N2 > 0)
     for y, (norm, linear, gelu) in zip(ops.f32_norm_linears(x, *parts), parts):
         assert torch.equal(y, ops.f32_linear(ops.layernorm(x, norm.weight, norm.bias, norm.eps), linear.weight, linear.bias, gelu=gelu))
+    off = [torch.cat([t.new_zeros(1), t.flatten()])[1:] for t in (x, norms[0].weight)]  # vectors that begin on no 16 bytes
+    shifted = Part(weight=off[1], bias=norms[0].bias, eps=norms[0].eps)
+    assert off[0].data_ptr() % 16 == 4
+    assert torch.equal(ops.f32_norm_linears(off[0].view(1, K), (shifted, linears[0], None))[0], ops.f32_norm_linears(x, parts[0])[0])
     x2, res = draw(1, 3 * K), draw(1, N1)
     wide = Part(weight=draw(N1, 3 * K) * K ** -0.5, bias=draw(N1) if bias else None)
     h = ops.f32_linear(x, linears[0].weight, linears[0].bias)

@@ -8,7 +8,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N,K1,K2", [(5, 4, 4), (768, 768, 3072), (10, 832, 3072), (33, 1024, 3076), (7, 1028, 4096), (9, 64, 8192), (6, 256, 8196), (130, 8192, 8192)])
+@pytest.mark.parametrize("N,K1,K2", [(5, 4, 4), (768, 768, 3072), (10, 832, 3072), (33, 1024, 3076), (7, 1028, 4096), (9, 64, 8192), (6, 256, 8196), (130, 8192, 8192),
+                                     (35, 2048, 4096), (35, 2052, 4100), (3, 4096, 8192), (9, 1024, 4100), (10, 2052, 4096), (2, 4, 8)])
 @pytest.mark.parametrize("parts,hs", [(1, 4), (2, 4), (8, 64)])
 def test_two_products_of_a_row(N, K1, K2, parts, hs):
     from lit_gpt import ops
