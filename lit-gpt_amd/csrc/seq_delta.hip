@@ -18,6 +18,9 @@
 //                       inside those lanes with DPP adds (no LDS, no barrier);
 //                       q, k, g, v, beta of 16 tokens at a time are staged in LDS, the next 16 prefetched in registers
 //                       (8 at a time for key dims above 256)
+#include <utility>
+
+#include "gemm_tiles.h"
 #include "seq_common.h"
 
 namespace lgs {
@@ -544,27 +547,63 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
 // The same recurrence for key dims of 128 with 32 lanes a column, to the bits of gated_delta_kernel<2, 16>: of the four partial
 // sums per product there, ka + kb stand in one lane and kc + kd in its neighbour, whose sum is the first of the lane sums.
 //
-// A lone wave issues an instruction each five clocks, and a token is a chain of some 70 there, 490 clocks. With half of the rows
-// a lane has 48, 310 clocks, and a prompt of 16 heads one wave on each SIMD of the chip instead of one on every other. q, k and decays lie
-// in LDS as the lanes hold them (one 16-byte read each), v, beta and k . q of a token and column side by side. 2048 tokens of 16
-// heads of 128 x 128: 430 us before, 270 to 280 here; one token 6.6 / 5.2. Beyond 512 workgroups the waves share their
-// SIMDs unevenly and the fewer instructions of the other form count: 2048 tokens of 32 heads 432 / 388, 1024 of 48 heads 259 / 302, 404
-// of 5 sequences' 8 heads of 100 columns, which are 13 workgroups each, 92 / 107.
+// Bound by the instructions of a lone wave on each SIMD, four clocks each, and by LDS. Three things keep a token short. The key's product is
+// summed over the lanes at once, but the query's is not needed before the output: eight tokens' partial sums go through the same
+// tree together, two tokens at a time in the two halves of a group of lanes, then four, then eight, which leaves every token's sum in
+// lanes of its own, while the next eight tokens' chains run: an instruction's result reaches a DPP or a lane swap two instructions
+// later, and those places are filled with the query's product and the tree (left to the compiler they were waits of eight clocks, five a
+// token). The lanes are numbered for it: the tree's levels are, from the rows' lowest bit on, the mirrored eight, the mirrored
+// sixteen, the other sixteen, neighbours and pairs, of which a DPP's bank mask tells the first two apart and a lane swap the third. The
+// operands come by LDS-DMA, batches of eight tokens in a ring of six, and are read two tokens ahead, over the ends of batches too.
 //
-// grid (B * H * ceil(dv / 8) rounded up to 8). Lane l of a column: rows 64 j + 2 l + e, j, e < 2.
-// (PC: a decay per channel. The loads ahead carry no branches: behind one, every batch would wait for the next one's loads.)
+// us of 2048 tokens with heads of 128 x 128, when 32 tokens were staged through registers and every sum ran at its token / here: 16
+// heads with a decay per channel 304 / 258, 8 heads with one each 271 / 235, 32 heads (two workgroups on a CU) 408 / 344; 1024 and 512
+// tokens together of 16 heads 194 / 165. LDS by the lanes' 16 bytes in a row, which only DMAs of four bytes a lane can lay out: 288 of 16
+// heads, 435 of 32. The reads between the sums' steps instead of ahead of them: 259 and 254. Beyond 512 workgroups (two on each CU) a
+// third would wait for a whole chain, and the form of 16 lanes is the better one: 2048 tokens of 48 heads.
+//
+// grid (B * H * ceil(dv / 8) rounded up to 8). A column's lane p is number l of the rows 64 j + 2 l + e, j, e < 2.
+// (PC: a decay per channel; otherwise it stands beside the betas.)
+template <bool PC>
 struct DeltaWide {
-  static constexpr int D = 128, CW = 8, TB = 32, ROW = 3 * D + 4 * CW;  // staged floats per token: q | k | g | (v, beta, k . q, -) per column
-  static constexpr int STAGED = (TB + 1) * ROW, LDS = (STAGED + TB * CW) * 4;  // (a batch's last token reads one row ahead)
-  static constexpr int ALONE = 28 * 1024;  // more of it that nobody uses (gated_delta_wide_launch)
+  static constexpr int D = 128, CW = 8, TB = 8, RING = 6, PARTS = PC ? 3 : 2;
+  // a batch in floats: the tokens' q | k, their decays, a value of each column and token, then beta, k . q and decays by token
+  static constexpr int G = TB * 2 * D, V = TB * PARTS * D, SC = V + TB * CW, SLOT = SC + (PC ? 2 : 3) * 64, LDS = RING * SLOT * 4;
+  static constexpr int LOADS = PARTS + 1;  // DMAs of a wave and batch: 1 KB of q and k each of two tokens, and decays of two; values or scalars
+  // more of it that nobody uses (gated_delta_wide_launch)
+  static constexpr int ALONE = (kCuLds / 2 + 4096 - LDS) / 1024 * 1024;
+  static_assert(2 * LDS <= kCuLds, "two on a CU");
   static_assert(2 * (LDS + ALONE) > kCuLds && LDS + ALONE + kPromptAttnLds > kCuLds, "alone on a CU");
 };
+typedef float delta_f2 __attribute__((ext_vector_type(2)));  // (the compiler's own: reads of HIP's would wait for every DMA)
+typedef float delta_f4 __attribute__((ext_vector_type(4)));
+// SIZE bytes a lane into LDS. Through a buffer resource: behind a flat-encoded load the compiler waits for every read of LDS in flight
+// wherever it needs one; and what lies past the resource's bytes is not read (zeros)
+template <int SIZE>
+__device__ __forceinline__ void delta_dma(const void* base, int bytes, unsigned off, unsigned char* lds) {
+#ifdef __HIP_DEVICE_COMPILE__  // (a device builtin: the host pass only type-checks the body)
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, bytes, 0x00020000);
+  if constexpr (SIZE == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, off, 0, 0, 0);
+#endif
+}
+template <int... I, class F>
+__device__ __forceinline__ void delta_steps(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N>  // until at most N of this wave's LDS operations are on their way
+__device__ __forceinline__ void delta_wait_lds() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
 template <bool DELTA, bool PC>
 __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
-  constexpr int D = DeltaWide::D, CW = DeltaWide::CW, TB = DeltaWide::TB, ROW = DeltaWide::ROW;
-  __shared__ __attribute__((aligned(16))) float st[DeltaWide::STAGED];
-  __shared__ float os[TB * CW];
-  const int tid = threadIdx.x, l = tid & 31, cw = tid >> 5;
+  using T = DeltaWide<PC>;
+  constexpr int D = T::D, CW = T::CW, TB = T::TB, RING = T::RING, PARTS = T::PARTS, SLOT = T::SLOT;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[T::LDS];
+  const int tid = threadIdx.x, lane = tid & 31, cw = tid >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (lane = the levels' distances 7, 15, 16, 1, 2 by the bits of l)
+  const int l = ((lane >> 2 ^ lane >> 3) & 1) | (lane >> 3 & 1) << 1 | (lane >> 4 & 1) << 2 | ((lane ^ lane >> 2) & 1) << 3 |
+                ((lane >> 1 ^ lane >> 2) & 1) << 4;
   const int per_xcd = (p.items + 7) / 8;  // (a head's column blocks on one XCD, as above)
   const int item = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (item >= p.items) return;
@@ -582,100 +621,247 @@ __global__ void __launch_bounds__(256) gated_delta_wide_kernel(DeltaArgs p) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(S[i]));  // (as above: the loads of S end here)
 
-  // a thread stages the tokens cw, cw + 8, ... of a batch: q, k and decays of the rows of lane l; and one column's v, beta, k . q
-  // of one token
-  const float* qk = p.qkv + (size_t)r0 * p.ld;
-  const float* dec = p.dec + ((size_t)r0 * H + hd) * (PC ? D : 1);
-  const long dstep = (long)H * (PC ? D : 1);
-  const int vt = tid / CW, vc = cblk * CW + tid % CW;
-  float2 pre[TB / 8][3][2];
-  float vpre, bpre = 0.0f, kqpre;
-  auto prefetch = [&](int t0) {  // (past the end: the last token again)
+  // A wave brings q and k of the tokens 2 w and 2 w + 1 of a batch, their decays, and the values (wave 0), betas (1), k . q (2) or decays of a
+  // head (3) of all eight. Addresses go on batch by batch; rows past the sequence's end are past the resource's bytes.
+  const int lane64 = tid & 63;
+  const char* qk = (const char*)(p.qkv + (size_t)r0 * p.ld + (size_t)g * D);
+  const char* dec = (const char*)(p.dec + ((size_t)r0 * H + hd) * (PC ? D : 1));
+  const char* few = (const char*)(p.kq + (size_t)r0 * p.G + g);
+  const int ld4 = (int)p.ld * 4, dstep = H * (PC ? D : 1) * 4;
+  int fstep = p.G * 4, few_end = 4;  // bytes of a row, and those read of the last one
+  if (wave == 0) {
+    few = (const char*)(p.qkv + (size_t)r0 * p.ld + (size_t)2 * p.G * D + (size_t)hd * dv + cblk * CW);
+    fstep = ld4, few_end = 4 * min(CW, dv - cblk * CW);
+  }
+  if (wave == 1 && DELTA) few = (const char*)(p.beta + (size_t)r0 * H + hd), fstep = H * 4;
+  if (wave == 3 && !PC) few = dec, fstep = dstep;
+  const int few_to = (wave == 0 ? T::V : T::SC + (wave == 1 ? 0 : wave == 3 && !PC ? 2 : 1) * 64) * 4;
+  const unsigned qk_off = (lane64 >> 5) * (unsigned)(p.G * D * 4) + 16 * (lane64 & 31);
+  const unsigned g_off = (2 * wave + (lane64 >> 5)) * (unsigned)dstep + 16 * (lane64 & 31);
+  const unsigned few_off = (wave == 0 ? lane64 >> 3 : lane64 & 7) * (unsigned)fstep + (wave == 0 ? 4 * (lane64 & 7) : 0);
+  auto slot_at = [&](int slot) { return lds + slot * (SLOT * 4); };
+  int left = n;  // rows that are not loaded yet
+  auto load = [&](int slot) {
+    unsigned char* to = slot_at(slot);
+    const int rows = __builtin_amdgcn_readfirstlane(min(max(left, 0), TB));
 #pragma unroll
-    for (int u = 0; u < TB / 8; ++u) {
-      const int t = min(t0 + u * 8 + cw, n - 1);
-      const float *q = qk + t * p.ld + (size_t)g * D + 2 * l, *k = q + (size_t)p.G * D, *d = dec + t * dstep;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        pre[u][0][j] = *(const float2*)(q + 64 * j);
-        pre[u][1][j] = *(const float2*)(k + 64 * j);
-        if constexpr (PC) pre[u][2][j] = *(const float2*)(d + 64 * j + 2 * l);
-        else pre[u][2][j].x = d[0];
-      }
+    for (int i = 0; i < 2; ++i) {
+      const int t = 2 * wave + i;
+      delta_dma<16>(qk + (long)t * ld4, t < rows ? (p.G + 1) * D * 4 : 0, qk_off, to + t * 1024);
     }
-    const int t = min(t0 + vt, n - 1);
-    vpre = qk[t * p.ld + (size_t)2 * p.G * D + (size_t)hd * dv + min(vc, dv - 1)];
-    if constexpr (DELTA) bpre = p.beta[(size_t)(r0 + t) * H + hd];
-    kqpre = p.kq[(size_t)(r0 + t) * p.G + g];
+    if constexpr (PC) delta_dma<16>(dec, max(rows * dstep - (dstep - D * 4), 0), g_off, to + (T::G + 2 * wave * D) * 4);
+    delta_dma<4>(few, max(rows * fstep - (fstep - few_end), 0), few_off, to + few_to);
+    left -= TB;
+    qk += (long)TB * ld4, dec += (long)TB * dstep, few += (long)TB * fstep;
   };
-  if (n > 0) prefetch(0);
 
   struct Token {
-    float4 k, g, q, c;
+    delta_f2 q[2], k[2], g[2];
   };
-  auto fetch = [&](const float* row, Token& x) {
-    x.g = *(const float4*)(row + 2 * D + 4 * l);
-    x.k = *(const float4*)(row + D + 4 * l);
-    x.q = *(const float4*)(row + 4 * l);
-    x.c = *(const float4*)(row + 3 * D + 4 * cw);
+  // A batch's vectors as this lane reads them: six addresses that the compiler cannot tell apart from strangers, or it joins two reads of 8
+  // bytes into one instruction, whose two places fall on the same banks (64 clocks of four waves where two reads take 21, measured)
+  struct Places {
+    unsigned q[2], k[2], g[2];
   };
-  auto one = [&](const Token& x) {
-    S[0] *= x.g.x, S[1] *= x.g.y, S[2] *= x.g.z, S[3] *= x.g.w;
-    float ks = 0.0f;
-    if (DELTA) ks = fmaf(S[2], x.k.z, fmaf(S[0], x.k.x, 0.0f)) + fmaf(S[3], x.k.w, fmaf(S[1], x.k.y, 0.0f));
-    float qs = fmaf(S[2], x.q.z, fmaf(S[0], x.q.x, 0.0f)) + fmaf(S[3], x.q.w, fmaf(S[1], x.q.y, 0.0f));
-    lanes_sum2<16>(ks, qs);
-    // the two rows of 16 lanes, both sums in one swap: even rows then hold ks of either row, odd ones qs; and back to all lanes
-    const auto halves = __builtin_amdgcn_permlane16_swap(__float_as_uint(ks), __float_as_uint(qs), false, false);
-    const float both = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
-    const auto sums = __builtin_amdgcn_permlane16_swap(__float_as_uint(both), __float_as_uint(both), false, false);
-    ks = __uint_as_float(sums[0]), qs = __uint_as_float(sums[1]);
-    const float u = DELTA ? x.c.y * (x.c.x - ks) : x.c.x;
-    S[0] = fmaf(x.k.x, u, S[0]), S[1] = fmaf(x.k.y, u, S[1]), S[2] = fmaf(x.k.z, u, S[2]), S[3] = fmaf(x.k.w, u, S[3]);
-    return fmaf(u, x.c.z, qs);
-  };
-  for (int t0 = 0; t0 < n; t0 += TB) {
-    const int nb = min(TB, n - t0);
-    __syncthreads();  // the previous batch's reads of st and os are done
+  auto places = [&](int slot, Places& o) {
 #pragma unroll
-    for (int u = 0; u < TB / 8; ++u)
-#pragma unroll
-      for (int part = 0; part < 3; ++part) {
-        const float2 a = pre[u][part][0], c = pre[u][part][1];
-        *(float4*)(st + (u * 8 + cw) * ROW + part * D + 4 * l) =
-            part < 2 || PC ? make_float4(a.x, a.y, c.x, c.y) : make_float4(a.x, a.x, a.x, a.x);
-      }
-    *(float4*)(st + vt * ROW + 3 * D + 4 * (tid % CW)) = make_float4(vpre, bpre, kqpre, 0.0f);
-    __syncthreads();
-    if (t0 + TB < n) prefetch(t0 + TB);
-    Token x[2];
-    const float* row = st;
-    fetch(row, x[0]);
-    float keep = 0.0f;
-    if (nb == TB) {
-#pragma unroll 4
-      for (int t = 0; t < TB; t += 2) {
-        fetch(row + ROW, x[1]);
-        float o = one(x[0]);
-        if (t == l) keep = o;
-        row += 2 * ROW;
-        fetch(row, x[0]);
-        o = one(x[1]);
-        if (t + 1 == l) keep = o;
-      }
-    } else {
-      for (int t = 0; t < nb; ++t) {
-        row += ROW;
-        fetch(row, x[1]);
-        const float o = one(x[0]);
-        if (t == l) keep = o;
-        x[0] = x[1];
+    for (int j = 0; j < 2; ++j) {
+      o.q[j] = slot * (SLOT * 4) + 256 * j + 8 * l;
+      o.k[j] = o.q[j] + 512;
+      asm volatile("" : "+v"(o.q[j]), "+v"(o.k[j]));
+      if constexpr (PC) {
+        o.g[j] = slot * (SLOT * 4) + T::G * 4 + 256 * j + 8 * l;
+        asm volatile("" : "+v"(o.g[j]));
       }
     }
-    os[l * CW + cw] = keep;
-    __syncthreads();
-    if (vt < nb && vc < dv) p.out[(size_t)(r0 + t0 + vt) * H * dv + (size_t)hd * dv + vc] = os[tid];
+  };
+  auto fetch = [&](const Places& at, int t, Token& x) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (PC) x.g[j] = *(const delta_f2*)(lds + at.g[j] + t * 512);
+      x.k[j] = *(const delta_f2*)(lds + at.k[j] + t * 1024);
+      x.q[j] = *(const delta_f2*)(lds + at.q[j] + t * 1024);
+    }
+  };
+  auto add16 = [](float v) {
+    const LanePair rows = lane_pair<16>(v);
+    return rows.a + rows.b;
+  };
+  auto pin = [] { __builtin_amdgcn_sched_barrier(0); };
+  auto here = [](float& v) { asm volatile("" : "+v"(v)); };  // (made here, not where it is used)
+  // One token: the decayed state's product with the key over all lanes and, between its steps, that with the query, left as this lane's
+  // share, and what `fill` does at five places; then the correction and the write. Returns u.
+  auto one = [&](const Token& x, float v, float beta, float gate, float& qs, auto&& fill) {
+    S[0] *= PC ? x.g[0].x : gate, S[1] *= PC ? x.g[0].y : gate, S[2] *= PC ? x.g[1].x : gate, S[3] *= PC ? x.g[1].y : gate;
+    float u = v;
+    if constexpr (DELTA) {
+      float ks = fmaf(S[2], x.k[1].x, S[0] * x.k[0].x) + fmaf(S[3], x.k[1].y, S[1] * x.k[0].y);
+      pin();
+      float a = S[0] * x.q[0].x, c = S[1] * x.q[0].y;
+      here(a), here(c);
+      pin();
+      ks += dpp_f<0x141>(ks);  // mirrored eight, then sixteen
+      pin();
+      a = fmaf(S[2], x.q[1].x, a), c = fmaf(S[3], x.q[1].y, c);
+      here(a), here(c);
+      pin();
+      ks += dpp_f<0x140>(ks);
+      float mate = ks;
+      here(mate);  // (a copy)
+      pin();
+      qs = a + c;
+      here(qs);
+      fill(std::integral_constant<int, 0>{});
+      pin();
+      const LanePair rows = lane_swap<16>(ks, mate);
+      ks = rows.a + rows.b;
+      pin();
+      fill(std::integral_constant<int, 1>{});
+      fill(std::integral_constant<int, 2>{});
+      pin();
+      ks += dpp_f<0xB1>(ks);
+      pin();
+      fill(std::integral_constant<int, 3>{});
+      fill(std::integral_constant<int, 4>{});
+      pin();
+      ks += dpp_f<0x4E>(ks);
+      u = beta * (v - ks);
+    } else {
+      qs = fmaf(S[2], x.q[1].x, S[0] * x.q[0].x) + fmaf(S[3], x.q[1].y, S[1] * x.q[0].y);
+      here(qs);
+      fill(std::integral_constant<int, 0>{});
+      fill(std::integral_constant<int, 1>{});
+      fill(std::integral_constant<int, 2>{});
+      fill(std::integral_constant<int, 3>{});
+      fill(std::integral_constant<int, 4>{});
+    }
+    S[0] = fmaf(x.k[0].x, u, S[0]), S[1] = fmaf(x.k[0].y, u, S[1]), S[2] = fmaf(x.k[1].x, u, S[2]), S[3] = fmaf(x.k[1].y, u, S[3]);
+    return u;
+  };
+  const int own = lane >> 2;  // of eight tokens the one whose sum this lane gets
+  const long ostep = (long)H * dv * 4;
+  char* out = (char*)(p.out + (size_t)r0 * H * dv + (size_t)hd * dv);
+  const unsigned o_off = own * (unsigned)ostep + 4 * col;
+  // eight tokens whose output is still to be made, and the tree over them in 31 steps (some empty: five to a token)
+  struct Eight {
+    float q[8], a[8], two[4], b[4], four[2], sum, u, kq;
+  } eight;
+  auto tree = [&](auto at, Eight& o) {
+    constexpr int I = decltype(at)::value;
+    if constexpr (I < 8) o.a[I] = o.q[I] + dpp_f<0x141>(o.q[I]), here(o.a[I]);
+    else if constexpr (I < 12) o.two[I - 8] = lane_dpp<0xE4, 0xa>(o.a[2 * (I - 8)], o.a[2 * (I - 8) + 1]), here(o.two[I - 8]);
+    else if constexpr (I < 16) o.b[I - 12] = o.two[I - 12] + dpp_f<0x128>(o.two[I - 12]), here(o.b[I - 12]);
+    else if constexpr (I < 18) o.four[I - 16] = lane_dpp<0xE4, 0xc>(o.b[2 * (I - 16)], o.b[2 * (I - 16) + 1]), here(o.four[I - 16]);
+    else if constexpr (I == 20) {
+      const LanePair rows = lane_swap<16>(o.four[0], o.four[1]);
+      o.sum = rows.a + rows.b, here(o.sum);
+    } else if constexpr (I == 25) o.sum += dpp_f<0xB1>(o.sum), here(o.sum);
+    else if constexpr (I == 30) o.sum += dpp_f<0x4E>(o.sum), here(o.sum);
+  };
+  auto finish = [&] {  // (out: of the tokens behind them)
+    if (live) *(float*)(out - TB * ostep + o_off) = fmaf(eight.u, eight.kq, eight.sum);  // (four lanes alike)
+  };
+
+  // batch t0 is worked on in slot `slot`; the five behind it are in LDS or on their way there
+  int slot = 0;
+  Token x[4];
+  Places at;
+  float cv[8], cb[8], cg[8];
+  auto scalars = [&](const unsigned char* from, int half) {  // four tokens' v, beta and decay
+#pragma unroll
+    for (int t = 4 * half; t < 4 * half + 4; ++t) cv[t] = *(const float*)(from + (T::V + t * CW + cw) * 4);
+    if constexpr (DELTA) {
+      const delta_f4 v = *(const delta_f4*)(from + (T::SC + 4 * half) * 4);
+      cb[4 * half] = v.x, cb[4 * half + 1] = v.y, cb[4 * half + 2] = v.z, cb[4 * half + 3] = v.w;
+    }
+    if constexpr (!PC) {
+      const delta_f4 v = *(const delta_f4*)(from + (T::SC + 128 + 4 * half) * 4);
+      cg[4 * half] = v.x, cg[4 * half + 1] = v.y, cg[4 * half + 2] = v.z, cg[4 * half + 3] = v.w;
+    }
+  };
+  // this wave's DMAs of the next batch have landed, and it has read all that it reads of the batch before (what it issued since are
+  // the reads of the two tokens ahead); and so has everyone
+  auto begin = [&] {
+    lga::gemm_wait_vm<3 * T::LOADS>();
+    delta_wait_lds<4 * PARTS>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  if (n > TB) {
+#pragma unroll
+    for (int i = 0; i < RING - 1; ++i) load(i);
+    begin();
+    places(0, at);
+    fetch(at, 0, x[0]);
+    fetch(at, 1, x[1]);
+    scalars(slot_at(0), 0);
+  } else if (n > 0) {
+    load(0);
+    lga::gemm_wait_vm<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   }
+  bool any = false;  // eight tokens before these
+#pragma unroll
+  for (int i = 0; i < 8; ++i) eight.q[i] = 0.0f;
+  int t0 = 0;
+  auto next_slot = [&](int s) { return s == RING - 1 ? 0 : s + 1; };
+  for (; t0 + TB <= n && n > TB; t0 += TB) {
+    if (t0 > 0) begin();
+    load(slot == 0 ? RING - 1 : slot - 1);
+    const int ns = next_slot(slot);
+    Places behind;
+    places(ns, behind);
+    float us = 0.0f, qs[8];
+    const float kq_own = *(const float*)(slot_at(slot) + (T::SC + 64 + own) * 4);
+    auto token = [&](auto i) {
+      constexpr int I = decltype(i)::value;
+      fetch(I < 6 ? at : behind, (I + 2) & 7, x[(I + 2) & 3]);
+      if constexpr (I == 1) scalars(slot_at(slot), 1);
+      if constexpr (I == 5) scalars(slot_at(ns), 0);
+      pin();
+      const float u = one(x[I & 3], cv[I], cb[I], cg[I], qs[I], [&](auto f) { tree(std::integral_constant<int, I * 5 + decltype(f)::value>{}, eight); });
+      us = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(us), __float_as_int(u), 0xE4, I < 4 ? 0x5 : 0xa, 1 << (I & 3), false));
+    };
+    token(std::integral_constant<int, 0>{});
+    token(std::integral_constant<int, 1>{});
+    token(std::integral_constant<int, 2>{});
+    token(std::integral_constant<int, 3>{});
+    token(std::integral_constant<int, 4>{});
+    token(std::integral_constant<int, 5>{});
+    token(std::integral_constant<int, 6>{});
+    token(std::integral_constant<int, 7>{});
+    if (any) finish();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) eight.q[i] = qs[i];
+    eight.u = us, eight.kq = kq_own, any = true;
+    out += TB * ostep;
+    slot = ns, at = behind;
+  }
+  if (any) {
+    delta_steps(std::make_integer_sequence<int, 31>{}, [&](auto at) { tree(at, eight); });
+    finish();
+  }
+  if (t0 < n) {  // fewer than eight are left, or are all there are
+    if (n > TB) begin();
+    const unsigned char* from = slot_at(slot);
+    places(slot, at);
+    for (int t = 0; t < n - t0; ++t) {
+      Token y;
+      fetch(at, t, y);
+      float qs;
+      const float u = one(y, *(const float*)(from + (T::V + t * CW + cw) * 4), DELTA ? *(const float*)(from + (T::SC + t) * 4) : 0.0f,
+                          PC ? 0.0f : *(const float*)(from + (T::SC + 128 + t) * 4), qs, [](auto) {});
+      const float kq_t = *(const float*)(from + (T::SC + 64 + t) * 4);
+      qs += dpp_f<0x141>(qs);
+      qs += dpp_f<0x140>(qs);
+      qs = add16(qs);
+      qs += dpp_f<0xB1>(qs);
+      qs += dpp_f<0x4E>(qs);
+      if (live && lane == 0) *(float*)(out + (size_t)t * ostep + 4 * col) = fmaf(u, kq_t, qs);
+    }
+  }
+  lga::gemm_wait_vm<0>();  // no DMA may outlive the workgroup's LDS
   if (live) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) sp[(size_t)row_of(i) * dv + col] = S[i];
@@ -688,9 +874,10 @@ static void gated_delta_wide_launch(DeltaArgs p, int B, bool plain, hipStream_t 
   p.items = B * p.H * p.ncb;
   const unsigned grid = (unsigned)((p.items + 7) / 8 * 8);
   // Up to half as many workgroups as the chip has CUs: LDS that nobody uses keeps a CU from two of them and from one beside a
-  // workgroup of the prompts' attention (kPromptAttnLds). The rule of 8 heads runs beside its layer's attention on another stream: 354
-  // to 424 us of 2048 tokens where they share CUs, 274 on its own ones (a raised wave priority changed nothing).
-  const unsigned alone = p.items <= 128 ? DeltaWide::ALONE : 0;
+  // workgroup of the prompts' attention (kPromptAttnLds). The rule of 8 heads runs beside its layer's attention on another stream: with
+  // 32 tokens staged at a time 354 to 424 us of 2048 tokens where they shared CUs, 274 on its own ones (235 now; a raised wave
+  // priority changed nothing).
+  const unsigned alone = p.items > 128 ? 0 : p.per_channel ? DeltaWide<true>::ALONE : DeltaWide<false>::ALONE;
   if (p.per_channel) {
     if (plain) gated_delta_wide_kernel<false, true><<<grid, 256, alone, stream>>>(p);
     else gated_delta_wide_kernel<true, true><<<grid, 256, alone, stream>>>(p);
@@ -796,7 +983,8 @@ extern "C" int lgs_gated_delta(const float* qkv, long ld, const float* dec, cons
   // lanes per column: more lanes shorten a token's dependent chain and multiply the waves; by default as many as
   // keep the launch within about two waves per SIMD, and at least enough for 32 rows per lane
   int lpc = lanes;
-  const bool pairs = ld % 2 == 0 && ((uintptr_t)qkv | (uintptr_t)dec) % 8 == 0;  // (loaded two floats at a time)
+  // (even rows: only they gained; rows below 2^24 floats: eight of them are offsets of 32 bits)
+  const bool pairs = ld % 2 == 0 && ld < (1 << 24) && ((uintptr_t)qkv | (uintptr_t)dec) % 8 == 0;
   if (lanes == 0 && d == 128 && pairs && (long)B * H * ((dv + 7) / 8) <= lgs::kDeltaWideItems) {
     lgs::gated_delta_wide_launch(p, B, plain != 0, stream);
     LGA_LAUNCH_RETURN();

@@ -459,6 +459,34 @@ def test_delta_rule_of_wide_heads_to_the_bit(H, G, dv, extra, lens, per_channel,
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
 
 
+@pytest.mark.parametrize("per_channel,plain", [(True, False), (False, False), (True, True), (False, True)])
+@pytest.mark.parametrize("H,G,dv,before,after,lens", [(2, 1, 17, 2, 4, [1, 7, 8, 9, 10, 15, 16, 17]), (3, 3, 8, 0, 2, [24, 41, 47, 48]),
+                                                      (4, 2, 25, 6, 0, [55, 57, 8, 64])])
+def test_delta_rule_of_wide_heads_by_eights_to_the_bit(H, G, dv, before, after, lens, per_channel, plain):
+    """Sequences about the eight tokens of a batch and the six batches of the ring, fresh and continued, packed side by side, whose rows
+    start off 16 bytes inside wider ones (``before`` + q | k | v + ``after``): the bits of 16 lanes a column. What lies past a sequence
+    or a head's columns is infinite where nobody owns it, so a term too many would show."""
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import StepBatch
+
+    dev, d, T = torch.device("cuda", 0), 128, sum(lens)
+    g = torch.Generator(device=dev).manual_seed(dv + T)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev)  # noqa: E731
+    step = StepBatch.build([(s, 4 * (s % 2), [0] * n) for s, n in enumerate(lens)], dev)
+    qkv = torch.full((T, before + 2 * G * d + H * dv + (before + after + H * dv) % 2 + after), float("inf"), device=dev)
+    qkv[:, before : before + 2 * G * d + H * dv] = draw(T, 2 * G * d + H * dv) * d ** -0.5
+    state = draw(len(lens), H, d, dv)
+    dec = torch.rand(T, H * d if per_channel else H, generator=g, device=dev) * 0.5 + 0.5
+    beta, kq, res = torch.rand(T, H, generator=g, device=dev), draw(T, G), []
+    for lanes in (0, 16):
+        s = state.clone()
+        out = seq_ops.gated_delta(qkv, dec, None if plain else beta, kq, s, step.seq_start, step.seq_slot, step.seq_pos0, H=H, G=G,
+                                  d=d, dv=dv, per_channel=per_channel, lanes=lanes, plain=plain, qkv_off=before)
+        res.append((out, s))
+    assert torch.isfinite(res[0][0]).all()
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+
+
 @pytest.mark.parametrize("H,G,d,per_channel,rank,unit,form", [(4, 2, 128, True, 64, True, 0), (4, 4, 40, False, 0, True, 0),
                                                               (2, 1, 130, True, 12, True, 0), (3, 3, 512, True, 3, False, 1),
                                                               (16, 16, 64, True, 0, True, 1)])
