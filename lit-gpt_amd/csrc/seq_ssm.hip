@@ -7,6 +7,7 @@
 //                        S <- a S + dt B x^T (S is N x dv, fp32, one per cache slot), y = S^T C + D x;
 //                        heads share B and C in groups. Token by token (decode, short portions), or for prompts
 //                        in chunks of 64 tokens as fp32 matrix products with the chunks side by side
+//   lgs_ssm_walk         the same with a sequence's chunks one after another and the state in registers
 //   lgs_channel_scan     the selective scan with a diagonal state matrix per channel (the Mamba form):
 //                        s_n <- 2^(dt a2_n) s_n + (dt x) B_n per channel, output (s . C + D x) silu(z);
 //                        token by token, or for prompts in chunks of 64 tokens side by side
@@ -458,6 +459,299 @@ __global__ void __launch_bounds__(256) ssd_carry_kernel(SsdArgs p) {
   *st = s;
 }
 
+// The prompt form with the chunks one after another: a workgroup walks a sequence through 64 columns of one head with the state in
+// registers, so that no chunk's state goes to memory. Wave w owns columns 16 w .. + 15 and all NT * 16 rows. With rows 16 t + 4 q + e in
+// lane group q a matrix instruction's result is laid out as its operands are read: the state's accumulators are the operand of C S, x is
+// loaded in the layout of the outputs and serves the scores' product, and the scores (B C^T, made once a group by
+// ssd_scores_kernel) become the operand of theirs. C and B of a chunk are staged in LDS while the chunk before is worked on. The sums
+// stand in the order of the kernels above, so the results have their bits.
+// Bound by the fp32 matrix instruction: 296 of 32 clocks a chunk and wave for N = 128, two thirds of the time it takes (6.1 us a chunk
+// and workgroup). 1500 + 777 + 130 tokens of 128 heads of 128 x 64 take 180 us, the three kernels above 340 (their chunks' states are
+// 640 MB written and read); four times 500 tokens of 64 heads 66 against 110; one chunk 16 to 19 against 24 to 29 whatever the heads.
+// With everything a chunk needs loaded and written at the start of a half 188, with decays and scores' exponentials made by every
+// wave 240, with row offsets held in registers (and spilled) 450.
+struct WalkArgs {
+  SsdArgs s;
+  float* scores;  // [B * max_chunks][groups][10][64][4]
+  float* decays;  // [B * max_chunks][heads][4][64]: l, d, exp(l_last - l) d, exp(l)
+};
+constexpr int kScoreTiles = 10;  // 16 x 16 pieces (ti, tj), tj <= ti, at ti (ti + 1) / 2 + tj
+
+// grid (B * max_chunks, groups + ceil(heads / 4)): the scores of a group, or the decays of four heads, a wave each
+template <int NT>
+__global__ void __launch_bounds__(256) ssd_scores_kernel(WalkArgs a) {
+  const SsdArgs& p = a.s;
+  const int b = blockIdx.x / p.max_chunks, cidx = blockIdx.x % p.max_chunks, g = blockIdx.y;
+  const int lane = threadIdx.x & 63, fr = lane & 15, fk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tc = p.seq_start[b] + cidx * kSC, n = min(kSC, p.seq_start[b + 1] - tc);
+  if (n <= 0) return;
+  if (g >= p.groups) {
+    const int h = (g - p.groups) * 4 + wave;
+    if (h >= p.heads) return;
+    float d;
+    const float l = ssd_decay(p, h, lane, n, p.dt[(size_t)(tc + min(lane, n - 1)) * p.ldd + h], &d), last = __shfl(l, n - 1);
+    float* out = a.decays + ((size_t)blockIdx.x * p.heads + h) * 4 * kSC + lane;
+    out[0] = l, out[kSC] = d, out[2 * kSC] = expf(last - l) * d, out[3 * kSC] = expf(l);
+    if (lane == 0) p.wdec[(size_t)blockIdx.x * p.heads + h] = expf(last);
+    return;
+  }
+  const float* bc = p.xbc + (size_t)tc * p.ldx + (size_t)p.heads * p.dv + (size_t)g * p.N + 4 * fk;
+  float4* out = (float4*)a.scores + ((size_t)blockIdx.x * p.groups + g) * kScoreTiles * 64 + lane;
+  for (int i = wave; i < kScoreTiles; i += 4) {
+    const int ti = i >= 6 ? 3 : (i >= 3 ? 2 : (i >= 1 ? 1 : 0)), tj = i - ti * (ti + 1) / 2;
+    const int ri = ti * 16 + fr, rj = tj * 16 + fr;
+    const float* bj = bc + (size_t)min(rj, n - 1) * p.ldx;
+    const float* ci = bc + (size_t)min(ri, n - 1) * p.ldx + (size_t)p.groups * p.N;
+    float4 bv[NT], cv[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      bv[t] = ssd_load4<true>(bj + 16 * t, rj < n ? 4 : 0);
+      cv[t] = ssd_load4<true>(ci + 16 * t, ri < n ? 4 : 0);
+    }
+    f32x4_t s = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      s = ssd_mma(bv[t].x, cv[t].x, s);
+      s = ssd_mma(bv[t].y, cv[t].y, s);
+      s = ssd_mma(bv[t].z, cv[t].z, s);
+      s = ssd_mma(bv[t].w, cv[t].w, s);
+    }
+    out[i * 64] = make_float4(s[0], s[1], s[2], s[3]);
+  }
+}
+
+// grid (heads, ceil(dv / 64), B)
+template <int NT>
+__global__ void __launch_bounds__(256, 2) ssd_walk_kernel(WalkArgs a) {
+  constexpr int N = NT * 16, LS = N + 4, KV = NT * 4, LD = kSC * KV / 256;  // KV: 16-byte pieces of a row, LD: of a thread
+  __shared__ __attribute__((aligned(16))) float Cs[kSC * LS], Bs[kSC * LS], Gs[12 * 256];  // (two pieces of Gs are not read)
+  __shared__ __attribute__((aligned(16))) float el[kSC], wgt[kSC];
+  const SsdArgs& p = a.s;
+  const int H = p.heads, dv = p.dv, b = blockIdx.z, inner = H * dv;
+  // an XCD takes neighbouring heads, which share B and C
+  const int h = H % 8 == 0 ? (blockIdx.x % 8) * (H / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int g = h / (H / p.groups);
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = __builtin_amdgcn_readfirstlane(p.seq_start[b]), len = __builtin_amdgcn_readfirstlane(p.seq_start[b + 1]) - r0;
+  const int col = blockIdx.y * 64 + wave * 16 + fr;
+  const bool live = col < dv;
+  const float Dh = p.D[h];
+  // a chunk's rows through buffer descriptors that end after its last row: rows past it read as zeros and are not written. Addresses
+  // are a step after the one before (as multiples of the row they would be held in registers, and spilled)
+  auto rows = [&](const float* base, int ld, int n) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, n * ld * 4, 0x00020000);
+  };
+  auto step = [](unsigned& at, unsigned by) {
+    at += by;
+    asm volatile("" : "+v"(at));
+  };
+  const int ldx = (int)p.ldx;
+  constexpr unsigned dead = 0x7ffffff0;  // (past every descriptor's end, with 64 rows added too)
+  const unsigned at_bc = ((tid / KV) * ldx + tid % KV * 4) * 4, at_x = live ? (4 * fk * ldx + col) * 4 : dead;
+  const unsigned at_y = live ? (4 * fk * inner + col) * 4 : dead;
+  f32x4_t cr[LD], br[LD], sc[3], lj[3], dj[3];
+  float x[16], li[3], dec = 0.0f, whole = 0.0f;
+  const float *Bp = p.xbc + inner + (size_t)g * N, *Cp = Bp + (size_t)p.groups * N, *Xp = p.xbc + (size_t)h * dv;
+  auto chunk_of = [&](const float* from, int c) { return rows(from + (size_t)(r0 + c * kSC) * ldx, ldx, min(kSC, len - c * kSC)); };
+  auto fetch_row = [&](f32x4_t& v, const auto& rs, unsigned& at) {  // a piece of a chunk's B or C
+    v = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+    step(at, 256 / KV * 4 * ldx);
+  };
+  auto fetch_x = [&](int k, const auto& rs, unsigned& at) {  // token 16 (k / 4) + 4 fk + k % 4
+    x[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0));
+    step(at, (k % 4 == 3 ? 13 : 1) * 4 * ldx);
+  };
+  // this wave's pieces of the scores (ti, tj) = wave, wave + 4, wave + 8 and what decays them
+  auto piece = [&](int k, int& ti, int& tj) {
+    const int i = min(wave + 4 * k, kScoreTiles - 1);
+    ti = i >= 6 ? 3 : (i >= 3 ? 2 : (i >= 1 ? 1 : 0)), tj = i - ti * (ti + 1) / 2;
+    return i;
+  };
+  auto fetch_score = [&](int k, size_t at) {
+    const f32x4_t* from = (const f32x4_t*)a.scores + (at * p.groups + g) * kScoreTiles * 64;
+    const float* de = a.decays + (at * H + h) * 4 * kSC;
+    int ti, tj;
+    const int i = piece(k, ti, tj);
+    sc[k] = (from + i * 64)[(unsigned)lane];
+    li[k] = (de + ti * 16)[(unsigned)fr];
+    lj[k] = ((const f32x4_t*)(de + tj * 16))[(unsigned)fk];
+    dj[k] = ((const f32x4_t*)(de + kSC + tj * 16))[(unsigned)fk];
+  };
+  auto fetch_decay = [&](size_t at) {
+    dec = (a.decays + ((at * H + h) * 4 + 2) * kSC)[(unsigned)(tid & 127)];
+    whole = p.wdec[at * H + h];
+  };
+  auto decay_scores = [&](int k) {  // in place
+    int ti, tj;
+    piece(k, ti, tj);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float v = sc[k][r] * expf(li[k] - lj[k][r]) * dj[k][r];
+      sc[k][r] = ti > tj || 4 * fk + r <= fr ? v : 0.0f;
+    }
+  };
+  // the state at the sequence's start: zeros (a descriptor that ends before its first value) at position 0
+  f32x4_t S[NT];
+  const int slot = __builtin_amdgcn_readfirstlane(p.seq_slot[b]), old = __builtin_amdgcn_readfirstlane(p.seq_pos0[b]) > 0;
+  float* st = p.state + ((size_t)slot * H + h) * N * dv;
+  const auto sr = rows(st, dv, old ? N : 0);
+  const unsigned at_s = live ? (4 * fk * dv + col) * 4 : dead;
+  {
+    unsigned at = at_s;
+#pragma unroll
+    for (int k = 0; k < 4 * NT; ++k) {
+      S[k / 4][k % 4] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, at, 0, 0));
+      step(at, (k % 4 == 3 ? 13 : 1) * 4 * dv);
+    }
+  }
+  const int chunks = (len + kSC - 1) / kSC;
+  auto put_row = [&](float* to, const f32x4_t& v, int k) {
+    const int i = tid + 256 * k;
+    *(f32x4_t*)(to + i / KV * LS + i % KV * 4) = v;
+  };
+  auto put_scores = [&](int k) {
+    decay_scores(k);
+    *(f32x4_t*)(Gs + ((wave + 4 * k) * 64 + lane) * 4) = sc[k];
+  };
+  auto put_el = [&]() {
+    if (tid >= kSC && tid < 2 * kSC) el[tid - kSC] = dec;
+  };
+  const size_t at0 = (size_t)b * p.max_chunks;
+  if (chunks > 0) {
+    const auto bs = chunk_of(Bp, 0), cs = chunk_of(Cp, 0);
+    unsigned ab = at_bc, ac = at_bc;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) fetch_score(k, at0);
+    fetch_decay(at0);
+#pragma unroll
+    for (int k = 0; k < LD; ++k) fetch_row(cr[k], cs, ac), fetch_row(br[k], bs, ab);
+#pragma unroll
+    for (int k = 0; k < LD; ++k) put_row(Cs, cr[k], k);
+    put_el();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) put_scores(k);
+  }
+  // Of a chunk, C and the scores are read before the middle barrier and B after it: the next chunk's are written in the other half.
+  // Loads and writes stand one or two behind every four matrix instructions (all together at the start of a half, the matrix cores
+  // waited for their issue). The next chunk's loads are those of this one again where it is the last: under a condition they could
+  // not be counted, and would be waited for as one.
+  for (int c = 0; c < chunks; ++c) {
+    const int next = min(c + 1, chunks - 1);
+    const auto xs = chunk_of(Xp, c), cs = chunk_of(Cp, next), bs = chunk_of(Bp, next);
+    const auto ys = rows(p.y + (size_t)(r0 + c * kSC) * inner + (size_t)h * dv, inner, min(kSC, len - c * kSC));
+    unsigned ax = at_x, ac = at_bc, ab = at_bc, ay = at_y;
+    f32x4_t o[4], ca[2][4];
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) o[ti] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const float held = whole;
+    __syncthreads();
+    auto read_c = [&](f32x4_t& v, int t, int ti) { v = *(const f32x4_t*)(Cs + (ti * 16 + fr) * LS + 16 * t + 4 * fk); };
+    auto read_g = [&](f32x4_t& v, int tj, int ti) {
+      if (ti >= tj) v = *(const f32x4_t*)(Gs + ((ti * (ti + 1) / 2 + tj) * 64 + lane) * 4);
+    };
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) read_c(ca[0][ti], 0, ti);
+    if (tid < kSC) wgt[tid] = dec;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * t + e;
+#pragma unroll
+        for (int ti = 0; ti < 4; ++ti) o[ti] = ssd_mma(ca[t & 1][ti][e], S[t][e], o[ti]);
+        if (t + 1 < NT) read_c(ca[(t + 1) & 1][e], t + 1, e);
+        else read_g(ca[(t + 1) & 1][e], 0, e);
+        if (i < 8) fetch_x(2 * i, xs, ax), fetch_x(2 * i + 1, xs, ax);
+        if (i < LD) put_row(Bs, br[i], i);
+        if (i >= 8 && i < 8 + LD) fetch_row(cr[i - 8], cs, ac);
+        if (i >= 4 * NT - 4 && i < 4 * NT - 1) fetch_score(i - 4 * NT + 4, at0 + next);
+        if (i == 4 * NT - 1) fetch_decay(at0 + next);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) {
+      const f32x4_t e = *(const f32x4_t*)&el[ti * 16 + 4 * fk];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[ti][r] *= e[r];
+    }
+    static_assert(NT % 2 == 0, "the scores follow in ca[0]");
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (tj < 3) read_g(ca[(tj + 1) & 1][e], tj + 1, e);
+#pragma unroll
+        for (int ti = 0; ti < 4; ++ti)
+          if (ti >= tj) o[ti] = ssd_mma(ca[tj & 1][ti][e], x[tj * 4 + e], o[ti]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    __syncthreads();
+    // the state: this chunk's sum onto the decayed state before it
+    f32x4_t s[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) s[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float bv[2][NT];
+    auto read_b = [&](float (&v)[NT], int k) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) v[t] = Bs[(16 * (k >> 2) + 4 * fk + (k & 3)) * LS + 16 * t + fr];
+    };
+    read_b(bv[0], 0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const f32x4_t w = *(const f32x4_t*)&wgt[16 * u + 4 * fk];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[u][e] = fmaf(Dh, x[u * 4 + e], o[u][e]);
+        x[u * 4 + e] *= w[e];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+#pragma unroll
+      for (int t = 0; t < NT / 2; ++t) s[t] = ssd_mma(bv[k & 1][t], x[k], s[t]);
+      if (k + 1 < 16) read_b(bv[(k + 1) & 1], k + 1);
+      if (k % 4 != 3) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = NT / 2; t < NT; ++t) s[t] = ssd_mma(bv[k & 1][t], x[k], s[t]);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[k / 4][k % 4]), ys, ay, 0, 0);
+      step(ay, (k % 4 == 3 ? 13 : 1) * 4 * inner);
+      if (k < LD) {
+        put_row(Cs, cr[k], k);
+        fetch_row(br[k], bs, ab);
+      }
+      if (k == 8) put_el();
+      if (k % 4 == 3 && k < 12) {  // the next chunk's scores in the gaps of the matrix instructions
+        put_scores(k / 4);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 96 / NT, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[t][r] = fmaf(held, S[t][r], s[t][r]);
+  }
+  const auto sw = rows(st, dv, N);
+  unsigned at = at_s;
+#pragma unroll
+  for (int k = 0; k < 4 * NT; ++k) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[k / 4][k % 4]), sw, at, 0, 0);
+    step(at, (k % 4 == 3 ? 13 : 1) * 4 * dv);
+  }
+}
+
+template <int NT>
+static void ssd_walk_launch(const WalkArgs& a, int B, hipStream_t stream) {
+  ssd_scores_kernel<NT><<<dim3(B * a.s.max_chunks, a.s.groups + (a.s.heads + 3) / 4), 256, 0, stream>>>(a);
+  ssd_walk_kernel<NT><<<dim3(a.s.heads, (a.s.dv + 63) / 64, B), 256, 0, stream>>>(a);
+}
+
 // ------------------------------------------------------------------------------------------------ channel scan
 // Selective scan with a step size per channel and a diagonal state matrix (channels x N): nothing is shared between
 // channels but B and C, and every (channel, state) pair decays at a rate of its own, so the work is
@@ -710,6 +1004,28 @@ extern "C" int lgs_ssm_scan(const float* xbc, long ldx, const float* dt, long ld
   else if (nr <= 16) lgs::ssm_scan_kernel<16><<<grid, 256, 0, stream>>>(p);
   else if (nr <= 32) lgs::ssm_scan_kernel<32><<<grid, 256, 0, stream>>>(p);
   else lgs::ssm_scan_kernel<64><<<grid, 256, 0, stream>>>(p);
+  LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lgs_ssm_walk(const float* xbc, long ldx, const float* dt, long ldd, const float* dt_bias,
+                            const float* A_log, const float* D, float* state, const int* seq_start,
+                            const int* seq_slot, const int* seq_pos0, float* y, int B, int heads, int groups, int N,
+                            int dv, float* ws, int max_chunks, hipStream_t stream) {
+  LGA_CHECK_ARG(xbc && dt && dt_bias && A_log && D && state && seq_start && seq_slot && seq_pos0 && y && ws,
+                "lgs_ssm_walk: null pointer");
+  LGA_CHECK_ARG(B > 0 && B <= 65535 && heads > 0 && groups > 0 && heads % groups == 0 && groups + (heads + 3) / 4 <= 65535,
+                "lgs_ssm_walk: heads must be a multiple of the groups");
+  LGA_CHECK_ARG((N == 64 || N == 128) && dv > 0 && (dv + 63) / 64 <= 65535, "lgs_ssm_walk: state size 64 or 128");
+  LGA_CHECK_ARG(ldx >= (long)heads * dv + 2L * groups * N && ldd >= heads, "lgs_ssm_walk: rows shorter than their parts");
+  LGA_CHECK_ARG(ldx < (1L << 22) && ldd < (1L << 22), "lgs_ssm_walk: 64 rows are more than 32 bits address");
+  LGA_CHECK_ARG(dv % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)xbc | (uintptr_t)ws) % 16 == 0, "lgs_ssm_walk: rows in 16 bytes");
+  LGA_CHECK_ARG(max_chunks > 0 && (long)B * max_chunks < (1L << 31), "lgs_ssm_walk: too many chunks");
+  const size_t chunks = (size_t)B * max_chunks;
+  float* decays = ws + chunks * groups * lgs::kScoreTiles * 256;
+  lgs::WalkArgs a{{xbc, ldx, dt, ldd, dt_bias, A_log, D, state, seq_start, seq_slot, seq_pos0, y, nullptr,
+                   decays + chunks * heads * 4 * lgs::kSC, heads, groups, N, dv, max_chunks, 1}, ws, decays};
+  if (N == 128) lgs::ssd_walk_launch<8>(a, B, stream);
+  else lgs::ssd_walk_launch<4>(a, B, stream);
   LGA_LAUNCH_RETURN();
 }
 

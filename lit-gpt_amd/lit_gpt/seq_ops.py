@@ -69,6 +69,7 @@ SIGNATURES = {
                      _F, _P],
     "lgs_conv_silu": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "lgs_ssm_scan": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P],
+    "lgs_ssm_walk": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P],
     "lgs_gated_group_norm": [_P, _P, _L, _P, _F, _P, _P, _I, _I, _I, _P],
     "lgs_glu_clamped": [_P, _P, _L, _P, _I, _I, _I, _F, _F, _F, _P],
     "lgs_embed_pos": [_P, _P, _P, _P, _I, _F, _P, _P, _I, _I, _I, _I, _P],
@@ -783,14 +784,25 @@ def conv_silu(proj: torch.Tensor, off: int, weight: torch.Tensor, bias: torch.Te
     return out
 
 
+def _ssm_walks(T: int, max_chunks: int, heads: int, N: int, dv: int, ldx: int, ldd: int) -> bool:
+    """Whether a prompt step's scan walks the chunks of a sequence one after another. A walk takes 6.1 us for every chunk of the
+    longest sequence however few its workgroups are (a head's 64 columns each, 256 in 6.1 us); the chunks side by side
+    take 0.045 us and more for every workgroup's chunk. us side by side / walked: 128 heads 2048 tokens 219 / 206, 64 heads of as
+    many 114 / 203, four times 500 tokens 110 / 66 and of 32 heads 71 / 64, of 16 51 / 63; one chunk of 16 to 128 heads 26 to 29 /
+    18, two of 16 27 / 24, three 30 / 31."""
+    if N not in (64, 128) or dv % 4 or ldx % 4 or max(ldx, ldd) >= 1 << 22 or heads >= 1 << 15:
+        return False
+    return max_chunks <= 2 or heads * -(-dv // 64) * T >= 112 * 64 * max_chunks
+
+
 def ssm_scan(xbc: torch.Tensor, proj: torch.Tensor, dt_off: int, dt_bias: torch.Tensor, A_log: torch.Tensor,
              D: torch.Tensor, state: torch.Tensor, seq_start: torch.Tensor, seq_slot: torch.Tensor,
              seq_pos0: torch.Tensor, *, heads: int, groups: int, N: int, dv: int, max_len: int = 0,
              chunked: Optional[bool] = None) -> torch.Tensor:
     """The selective scan over a packed batch: xbc (T, heads dv + 2 groups N) after the convolution, raw step sizes
     in the ``heads`` columns of ``proj`` at ``dt_off``; state (slots, heads, N, dv) fp32. Returns y (T, heads dv).
-    ``chunked`` picks the prompt form (64-token chunks as matrix products, all chunks side by side; N <= 128) over
-    the token-by-token walk; by default steps in which a sequence brings more than 16 tokens (``max_len``) take it."""
+    ``chunked`` picks the prompt form (64-token chunks as matrix products, side by side or one after another, to the
+    same bits; N <= 128) over the token-by-token walk; by default steps in which a sequence brings more than 16 tokens (``max_len``) take it."""
     T, ldx = xbc.shape
     B = seq_slot.numel()
     if ldx != heads * dv + 2 * groups * N or tuple(state.shape[1:]) != (heads, N, dv) or proj.shape[0] != T:
@@ -805,6 +817,16 @@ def ssm_scan(xbc: torch.Tensor, proj: torch.Tensor, dt_off: int, dt_bias: torch.
         if not 0 < max_len <= T or N > 128:
             raise ValueError("ssm_scan: the prompt form needs the longest sequence's token count and N <= 128")
         max_chunks = (max_len + 63) // 64
+        # (xbc is a tensor of its own or a part of one: its rows may lie off 16 bytes)
+        if _ssm_walks(T, max_chunks, heads, N, dv, ldx, proj.shape[1]) and xbc.data_ptr() % 16 == 0:
+            ws = torch.empty(B * max_chunks * (2560 * groups + 257 * heads), dtype=F32, device=xbc.device)
+            _check(load_library().lgs_ssm_walk(_dev(xbc, "xbc", F32), ldx, _dev(proj, "proj", F32) + 4 * dt_off,
+                                               proj.shape[1], _dev(dt_bias, "dt_bias", F32), _dev(A_log, "A_log", F32),
+                                               _dev(D, "D", F32), _dev(state, "state", F32),
+                                               _dev(seq_start, "seq_start", I32), _dev(seq_slot, "seq_slot", I32),
+                                               _dev(seq_pos0, "seq_pos0", I32), y.data_ptr(), B, heads, groups, N, dv,
+                                               ws.data_ptr(), max_chunks, _stream()))
+            return y
         ws = torch.empty(B * max_chunks * heads * N * dv, dtype=F32, device=xbc.device)
         wdec = torch.empty(B * max_chunks * heads, dtype=F32, device=xbc.device)
     _check(load_library().lgs_ssm_scan(_dev(xbc, "xbc", F32), ldx, _dev(proj, "proj", F32) + 4 * dt_off,

@@ -31,3 +31,33 @@ def test_prompt_form_against_token_walk(heads, groups, N, dv):
     assert float((y[True] - y[False]).abs().max()) < 4e-5 * float(y[False].abs().max())
     assert float((state[True] - state[False]).abs().max()) < 4e-5 * max(1.0, float(state[False].abs().max()))
     assert torch.equal(state[True][-1], stale[-1])
+
+
+@pytest.mark.parametrize("heads,groups,N,dv", [(16, 2, 128, 64), (24, 1, 64, 72), (6, 3, 64, 40), (3, 3, 128, 4), (8, 8, 128, 132)])
+@pytest.mark.parametrize("lens", [[1], [64], [65, 1, 130, 128], [1000, 300]])
+def test_chunks_walked_against_side_by_side(heads, groups, N, dv, lens, monkeypatch):
+    """A sequence's chunks one after another (ssd_walk_kernel) and side by side: the same sums in the same order, so the same
+    bits; heads that are and are not multiples of eight, columns that end inside a wave's sixteen, an infinite input."""
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import StepBatch
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(N + dv)
+    pos0 = [9, 0, 3, 0][:len(lens)]
+    T, inner = sum(lens), heads * dv
+    rand = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    xbc, raw = rand(T, inner + 2 * groups * N) * 0.5, rand(T, heads + 3)
+    xbc[T // 2, 1] = float("inf")
+    dt_bias, A_log, D = rand(heads) - 1.0, rand(heads), rand(heads)
+    stale = rand(len(lens) + 1, heads, N, dv)
+    step = StepBatch.build([(i, p0, [0] * n) for i, (n, p0) in enumerate(zip(lens, pos0))], dev)
+    y, state = {}, {}
+    for walk in (False, True):
+        monkeypatch.setattr(seq_ops, "_ssm_walks", lambda *a, walk=walk: walk)
+        state[walk] = stale.clone()
+        y[walk] = seq_ops.ssm_scan(xbc, raw, 2, dt_bias, A_log, D, state[walk], step.seq_start, step.seq_slot, step.seq_pos0,
+                                   heads=heads, groups=groups, N=N, dv=dv, max_len=max(lens), chunked=True)
+    torch.testing.assert_close(y[True], y[False], rtol=0, atol=0, equal_nan=True)
+    torch.testing.assert_close(state[True], state[False], rtol=0, atol=0, equal_nan=True)
+    assert torch.equal(state[True][-1], stale[-1])
+    assert torch.isfinite(y[True]).any()
