@@ -309,7 +309,8 @@ int lgs_ssm_scan(const float* xbc, long ldx, const float* dt, long ldd, const fl
 int lgs_ssm_walk(const float* xbc, long ldx, const float* dt, long ldd, const float* dt_bias, const float* A_log,
                  const float* D, float* state, const int* seq_start, const int* seq_slot, const int* seq_pos0,
                  float* y, int B, int heads, int groups, int N, int dv, float* ws, int max_chunks, lgs_stream_t stream);
-/* out = v / sqrt(mean over the group of v^2 + eps) * w, v = y * silu(z); `groups` equal parts of `inner` columns */
+/* out = v / sqrt(mean over the group of v^2 + eps) * w, v = y * silu(z); `groups` equal parts of `inner` columns. out may be
+ * NULL beside out_bf16 in groups of up to 2048 columns. */
 int lgs_gated_group_norm(const float* y, const float* z, long ldz, const float* w, float eps, float* out,
                          void* out_bf16, int T, int inner, int groups, lgs_stream_t stream);
 /* out[t][i] = g sigmoid(alpha g) (u + shift), g = min(a[t ld + i], limit), u = clamp(b[t ld + i], -limit, limit)

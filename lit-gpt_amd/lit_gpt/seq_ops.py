@@ -885,10 +885,11 @@ def gated_group_norm(y: torch.Tensor, proj: torch.Tensor, z_off: int, weight: to
     T, inner = y.shape
     if z_off + inner > proj.shape[1] or weight.numel() != inner or inner % groups:
         raise ValueError("gated_group_norm: shapes")
-    out = torch.empty(T, inner, dtype=F32, device=y.device)
+    # (wider groups are made in two passes over the fp32 result)
+    out = torch.empty(T, inner, dtype=F32, device=y.device) if not bf16_copy or inner > 2048 * groups else None
     out16 = torch.empty(T, inner, dtype=torch.bfloat16, device=y.device) if bf16_copy else None
     _check(load_library().lgs_gated_group_norm(_dev(y, "y", F32), _dev(proj, "proj", F32) + 4 * z_off, proj.shape[1],
-                                               _dev(weight, "weight", F32), float(eps), out.data_ptr(),
+                                               _dev(weight, "weight", F32), float(eps), _opt(out, "out", F32),
                                                _opt(out16, "out_bf16", torch.bfloat16), T, inner, groups, _stream()))
     return out16 if bf16_copy else out
 
