@@ -31,6 +31,9 @@ GemmPlan gemm_plan(int M, int N, int K, int batch, bool grouped, int ksplit, int
 GemmPlan gemm_glu_plan(int M, int n, int K, int batch, bool grouped);
 int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t stream);
 
+// Up to 32 columns on a kernel of their own: false where it does not take the product (nothing is launched)
+bool gemm_narrow(const LinArgs& p, int batch, hipStream_t stream);
+
 // A grouped product whose list is one tile of lgs_linear's older kernel and whose groups have two rows or less: that kernel
 // finds a group's rows by its place in the grid, where every workgroup here looks the list's groups through and most have
 // nothing to do. us there / here of top-4 routed tokens, up and down products: 64 experts of 512 x 2048, 13 tokens 45 + 30 / 60

@@ -346,4 +346,20 @@ int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t s
   return (int)hipErrorInvalidValue;
 }
 
+// 32 rows and up to 32 columns by one wave, eight steps ahead: a router's logits, whole in K. The sums are those of the tiles above, to the
+// same bits, but there are more workgroups and none of their waves works on columns that are not there. Bound by the latency of a step.
+// us, the tiles of 64 x 128 / here: 2048 x 18 x 2048 13.8 / 10.4 (in a model's prompt 16.4 / 12.0), 4096 x 16 x 2048 14.0 / 10.8, 2407 x 16
+// x 4096 23.0 / 17.2, 300 x 32 x 1024 8.7 / 6.7; past 8192 rows both have work for the chip (16000 x 18 x 2048 16.3 / 17.7). With the
+// operands in registers as the instructions take them 9.9 and 16.0, but only for K a multiple of 512.
+__global__ void __launch_bounds__(64) gemm_narrow_kernel(LinArgs p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[GemmTile<1, 1, 1, 1, 8, 8>::LDS];
+  gemm_rows<1, 1, 1, 1, 8, 8, true, true>(p, lds, blockIdx.y, 0, 0, p.M, blockIdx.x * 32, 0);
+}
+
+bool gemm_narrow(const LinArgs& p, int batch, hipStream_t stream) {
+  if (p.N > 32 || p.M > 8192 || p.K % 64 != 0 || p.ksplit > 1 || p.z_start) return false;
+  gemm_narrow_kernel<<<dim3((p.M + 31) / 32, batch), 64, 0, stream>>>(p);
+  return true;
+}
+
 }  // namespace lgs

@@ -742,6 +742,7 @@ extern "C" int lgs_linear(const void* a_any, long lda, long stride_a, const void
     p.ksplit = (nk + p.kper - 1) / p.kper;  // (no empty range)
   }
   if (a_bf16 && vec && std::max(ldy, (long)N) < (1L << 28)) {  // (a lane's place in four rows of Y: 32 bits)
+    if (lgs::gemm_narrow(p, batch, stream)) LGA_LAUNCH_RETURN();
     const lgs::GemmPlan plan = lgs::gemm_plan(M, N, K, batch, z_start != nullptr, p.ksplit, act, accumulate != 0);
     if (plan.tile >= 0) {
       const int rc = lgs::gemm_launch(p, plan, batch, stream);
