@@ -77,6 +77,44 @@ __device__ __forceinline__ float lowrank_dot(const void* w, size_t i, const floa
   return acc;
 }
 
+// The products of 16 rows of the map's inner values with TILES x 16 rows of its bf16 weights, on the matrix cores: lane group fk, lane fr
+// holds rows 4 fk + r of column 16 j + fr in out[j][r]. a: row t at a + t lda (fp32, rounded to bf16), w: row i at w + i rank. Rows past
+// the last repeat it. rank % 64 == 0, a, lda and w on 16 bytes. The operands and the order of their sums are those of lgs_linear's product
+// of an fp32 A and bf16 weights in more than 8 rows, and so are the bits.
+typedef __bf16 map_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float map_f32x4 __attribute__((ext_vector_type(4)));
+template <int TILES>
+__device__ __forceinline__ void lowrank_tiles(const float* a, long lda, int t0, int T, const uint16_t* w, int i0, int n, int rank, int lane,
+                                              map_f32x4 (&out)[TILES]) {
+  const int fr = lane & 15, fk = lane >> 4;
+  const float* ar = a + (size_t)min(t0 + fr, T - 1) * lda + fk * 8;
+  const uint16_t* wr[TILES];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) {
+    wr[j] = w + (size_t)min(i0 + 16 * j + fr, n - 1) * rank + fk * 8;
+    out[j] = map_f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int k = 0; k < rank; k += 64) {
+    uint4 wv[2][TILES], av[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const float4 lo = *(const float4*)(ar + k + 32 * s), hi = *(const float4*)(ar + k + 32 * s + 4);
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) wv[s][j] = *(const uint4*)(wr[j] + k + 32 * s);
+      av[s] = make_uint4(pack2(lo.x, lo.y), pack2(lo.z, lo.w), pack2(hi.x, hi.y), pack2(hi.z, hi.w));
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < TILES; ++j)
+        out[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(map_bf16x8, av[s]),
+                                                         __builtin_bit_cast(map_bf16x8, wv[s][j]), out[j], 0, 0, 0);
+  }
+}
+inline bool lowrank_tiles_fit(const void* a, long lda, const void* w, int w_f32, int rank) {
+  return w && !w_f32 && rank % 64 == 0 && lda % 4 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
+}
+
 // sum over the 256 threads of a workgroup (4 waves); `red` holds 4 floats; every thread gets the sum
 __device__ __forceinline__ float block_sum_256(float v, float* red) {
   v = wave_sum(v);

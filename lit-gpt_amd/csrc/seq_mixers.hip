@@ -351,15 +351,17 @@ __global__ void __launch_bounds__(256) head_gate_kernel(float* __restrict__ o, c
 // of them, whose values are on their way together; a row of a low-rank gate's second map is read once for its four tokens.
 // 2048 tokens of 16 heads: 13.8 us (31.6 for a workgroup per token and head, half of which had no column), of 8 8.3 (15.3), 256 of 16
 // 4.4 (5.4), of 8 3.8 (3.7), 65 of 16 4.1 (3.2): from 4096 tokens' heads on
-constexpr int kGateTokens = 8;
-template <bool G2F32>
+// MAP: the gate's inputs by lowrank_tiles, 16 tokens a workgroup. In a prompt of 2048 tokens of 16 heads, 64 inner values: a product's
+// launch 13 us and the gate behind it 16, here 20.
+constexpr int kGateTokens = 8, kGateMapTokens = 16;
+template <bool G2F32, bool MAP>
 __global__ void __launch_bounds__(256) head_gate_rows_kernel(float* __restrict__ o, const float* __restrict__ g, long ldg, int T, int H,
                                                              int unit, float eps, int act, const float* __restrict__ w, float post,
                                                              uint16_t* __restrict__ o16, const void* __restrict__ w_g2, int rank) {
-  constexpr int dv = 128, U = kGateTokens / 2;
+  constexpr int dv = 128, TOKENS = MAP ? kGateMapTokens : kGateTokens, U = TOKENS / 2;
   __shared__ float red[U][4];
-  extern __shared__ float g1[];  // [kGateTokens][rank]
-  const int t0 = blockIdx.x * kGateTokens, h = blockIdx.y, i = threadIdx.x & 127, half = threadIdx.x >> 7;
+  extern __shared__ float g1[];  // [kGateTokens][rank], MAP: [kGateMapTokens][dv]
+  const int t0 = blockIdx.x * TOKENS, h = blockIdx.y, i = threadIdx.x & 127, half = threadIdx.x >> 7;
   float v[U], gin[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {  // (past the end the last token again, never stored)
@@ -367,7 +369,18 @@ __global__ void __launch_bounds__(256) head_gate_rows_kernel(float* __restrict__
     v[u] = o[(t * H + h) * dv + i];
     gin[u] = w_g2 ? 0.0f : g[t * ldg + (size_t)h * dv + i];
   }
-  if (w_g2) {
+  if constexpr (MAP) {
+    const int lane = threadIdx.x & 63, c0 = (threadIdx.x >> 6) * 32;
+    map_f32x4 m[2];
+    lowrank_tiles<2>(g, ldg, t0, T, (const uint16_t*)w_g2, h * dv + c0, H * dv, rank, lane, m);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) g1[((lane >> 4) * 4 + r) * dv + c0 + 16 * j + (lane & 15)] = m[j][r];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) gin[u] = g1[(2 * u + half) * dv + i];
+  } else if (w_g2) {
     for (int x = threadIdx.x; x < kGateTokens * rank; x += 256) g1[x] = aop<G2F32>(g[(size_t)min(t0 + x / rank, T - 1) * ldg + x % rank]);
     __syncthreads();
     const size_t row = (size_t)h * dv + i;
@@ -1139,13 +1152,19 @@ extern "C" int lgs_head_gate(float* o, const float* g, long ldg, int T, int H, i
                 "lgs_head_gate: bad arguments (inner size of a low-rank gate 1..512)");
   if (dv == 128 && (long)T * H >= 4096 && (!w_g2 || rank % 8 == 0 || (long)T * H >= 5600)) {
     // (off eight a map's values come one by one: 260 tokens of 16 heads, rank 20, 6.0 / 6.7, 362 9.2 / 8.1, 1975 of 32 80 / 46)
+    if (lgs::lowrank_tiles_fit(g, ldg, w_g2, g2_f32, rank)) {
+      constexpr int N = lgs::kGateMapTokens;
+      lgs::head_gate_rows_kernel<false, true><<<dim3((T + N - 1) / N, H), 256, N * 128 * sizeof(float), stream>>>(
+          o, g, ldg, T, H, unit_norm, eps, act, weight, post, (uint16_t*)o_bf16, w_g2, rank);
+      LGA_LAUNCH_RETURN();
+    }
     const dim3 grid((T + lgs::kGateTokens - 1) / lgs::kGateTokens, H);
     const size_t lds = w_g2 ? (size_t)lgs::kGateTokens * rank * sizeof(float) : 0;
     if (g2_f32)
-      lgs::head_gate_rows_kernel<true><<<grid, 256, lds, stream>>>(o, g, ldg, T, H, unit_norm, eps, act, weight, post, (uint16_t*)o_bf16,
+      lgs::head_gate_rows_kernel<true, false><<<grid, 256, lds, stream>>>(o, g, ldg, T, H, unit_norm, eps, act, weight, post, (uint16_t*)o_bf16,
                                                                    w_g2, rank);
     else
-      lgs::head_gate_rows_kernel<false><<<grid, 256, lds, stream>>>(o, g, ldg, T, H, unit_norm, eps, act, weight, post, (uint16_t*)o_bf16,
+      lgs::head_gate_rows_kernel<false, false><<<grid, 256, lds, stream>>>(o, g, ldg, T, H, unit_norm, eps, act, weight, post, (uint16_t*)o_bf16,
                                                                     w_g2, rank);
     LGA_LAUNCH_RETURN();
   }

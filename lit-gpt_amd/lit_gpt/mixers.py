@@ -542,17 +542,20 @@ class GatedDelta(InputReader):
         else:
             qkv = seq_ops.conv_silu(proj, self.off["qkv"], self.conv_w, self.conv_b, cache.conv, *tables,
                                     step.max_len or T)
-            if self.per_channel:
-                ra, rg = self.w_a2.shape[1], self.w_g2.shape[1]
-                a = torch.empty(T, H * d, dtype=torch.float32, device=proj.device)
-                seq_ops.linear(proj, self.w_a2, M=T, N=H * d, K=ra, y=a, a_off=self.off["a1"], lda=ld, ldy=H * d)
-                gate = torch.empty(T, H * dv, dtype=torch.float32, device=proj.device)
-                seq_ops.linear(proj, self.w_g2, M=T, N=H * dv, K=rg, y=gate, a_off=self.off["g1"], lda=ld, ldy=H * dv)
-                a_off, g_off = 0, 0
+            a2 = g2 = None
+            if self.per_channel:  # the second maps inside the launches that use them, or as products
+                a, a_off, a2 = proj, self.off["a1"], self.w_a2
+                if not seq_ops.decay_map_inside(proj, a_off, a2, H=H, d=d):
+                    a, a_off, a2 = torch.empty(T, H * d, dtype=torch.float32, device=proj.device), 0, None
+                    seq_ops.linear(proj, self.w_a2, M=T, N=H * d, K=self.w_a2.shape[1], y=a, a_off=self.off["a1"], lda=ld, ldy=H * d)
+                gate, g_off, g2 = proj, self.off["g1"], self.w_g2
+                if not seq_ops.gate_map_inside(proj, g_off, g2, H=H, dv=dv):
+                    gate, g_off, g2 = torch.empty(T, H * dv, dtype=torch.float32, device=proj.device), 0, None
+                    seq_ops.linear(proj, self.w_g2, M=T, N=H * dv, K=self.w_g2.shape[1], y=gate, a_off=self.off["g1"], lda=ld,
+                                   ldy=H * dv)
             else:
                 a, a_off, gate, g_off = proj, self.off["a"], proj, self.off["g"]
-            g2 = None
-            dec, beta, kq = seq_ops.delta_prepare(qkv, a, a_off, proj, self.off["b"], self.A_log, self.dt_bias, **kw)
+            dec, beta, kq = seq_ops.delta_prepare(qkv, a, a_off, proj, self.off["b"], self.A_log, self.dt_bias, w_a2=a2, **kw)
         o = seq_ops.gated_delta(qkv, dec, beta, kq, cache.s, *tables, H=H, G=G, d=d, dv=dv,
                                 per_channel=self.per_channel)
         act = seq_ops.ACT_SIGMOID if self.per_channel else seq_ops.ACT_SILU

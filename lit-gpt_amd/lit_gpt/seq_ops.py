@@ -269,6 +269,23 @@ def retention(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, state: tor
     return out
 
 
+def _map_fits(proj: torch.Tensor, off: int, w: torch.Tensor) -> bool:
+    return w.dtype == torch.bfloat16 and w.shape[1] % 64 == 0 and w.shape[1] <= 512 and proj.shape[1] % 4 == 0 and \
+        (proj.data_ptr() + 4 * off) % 16 == 0 and w.data_ptr() % 16 == 0
+
+
+def decay_map_inside(proj: torch.Tensor, off: int, w_a2: torch.Tensor, *, H: int, d: int) -> bool:
+    """Whether ``delta_prepare`` makes the second map of a prompt's decays itself, to the bits of the product (rows that it prepares
+    side by side, inner values in 64s)."""
+    T = proj.shape[0]
+    return (T >= 2048 or (T > 64 and H * d >= 1024)) and d <= 512 and _map_fits(proj, off, w_a2)
+
+
+def gate_map_inside(proj: torch.Tensor, off: int, w_g2: torch.Tensor, *, H: int, dv: int) -> bool:
+    """Whether ``head_gate`` makes the second map of a prompt's gates itself, to the bits of the product."""
+    return dv == 128 and proj.shape[0] > 8 and proj.shape[0] * H >= 4096 and _map_fits(proj, off, w_g2)
+
+
 def head_gate(o: torch.Tensor, proj: torch.Tensor, g_off: int, *, H: int, dv: int, unit_norm: bool, eps: float,
               act: int, bf16_copy: bool = False, weight: Optional[torch.Tensor] = None,
               post: float = 1.0, w_g2: Optional[torch.Tensor] = None) -> torch.Tensor:
