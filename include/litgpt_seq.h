@@ -304,6 +304,10 @@ int lgs_ssm_scan(const float* xbc, long ldx, const float* dt, long ldd, const fl
                  const float* D, float* state, const int* seq_start, const int* seq_slot, const int* seq_pos0,
                  float* y, int B, int heads, int groups, int N, int dv, float* ws, float* wdec, int max_chunks,
                  lgs_stream_t stream);
+/* Every sequence brings one token: the same bits as token by token. N <= 128. */
+int lgs_ssm_one(const float* xbc, long ldx, const float* dt, long ldd, const float* dt_bias, const float* A_log,
+                const float* D, float* state, const int* seq_start, const int* seq_slot, const int* seq_pos0, float* y,
+                int B, int heads, int groups, int N, int dv, lgs_stream_t stream);
 /* The prompt form with a sequence's chunks one after another, the state in registers, to the same bits: N 64 or 128, dv and
  * ldx multiples of 4, xbc and ws on 16 bytes. ws: B max_chunks (2560 groups + 257 heads) floats. */
 int lgs_ssm_walk(const float* xbc, long ldx, const float* dt, long ldd, const float* dt_bias, const float* A_log,

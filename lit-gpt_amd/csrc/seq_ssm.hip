@@ -7,6 +7,7 @@
 //                        S <- a S + dt B x^T (S is N x dv, fp32, one per cache slot), y = S^T C + D x;
 //                        heads share B and C in groups. Token by token (decode, short portions), or for prompts
 //                        in chunks of 64 tokens as fp32 matrix products with the chunks side by side
+//   lgs_ssm_one          the same for steps of one token a sequence
 //   lgs_ssm_walk         the same with a sequence's chunks one after another and the state in registers
 //   lgs_channel_scan     the selective scan with a diagonal state matrix per channel (the Mamba form):
 //                        s_n <- 2^(dt a2_n) s_n + (dt x) B_n per channel, output (s . C + D x) silu(z);
@@ -216,6 +217,60 @@ __global__ void __launch_bounds__(256) ssm_scan_kernel(ScanArgs p) {
     for (int i = 0; i < NR; ++i)
       if (n0 + i < N) st[(size_t)(n0 + i) * dv + col] = S[i];
   }
+}
+
+// Steps of one token a sequence, to the bits of ssm_scan_kernel: a wave takes 16 columns of a head, its lane groups the quarters of the
+// rows, and everything that it needs is on its way at once (there, the step size, x, B and C, and the state come one behind the other, on a
+// quarter as many compute units). Bound by latency. us, there / here: 64 heads of 128 x 64 of one
+// sequence 7.0 / 3.2, of three 8.5 / 5.5, 128 heads 7.3 / 3.7. Where there are many, memory bounds both and rows of 64 bytes are the worse
+// ones: eight sequences of 64 heads 10.8 / 11.9, of 128 14.4 / 19.2, so up to 1024 waves.
+// grid (ceil(dv / 16), heads, B), 64 threads; VEC: N = 4 NR, rows of B and C on 16 bytes
+template <int NR, bool VEC>
+__global__ void __launch_bounds__(64) ssm_one_kernel(ScanArgs p) {
+  const int lane = threadIdx.x, hd = blockIdx.y, b = blockIdx.z, n0 = (lane >> 4) * NR;
+  const int N = p.N, dv = p.dv, H = p.heads, inner = H * dv, g = hd / (H / p.groups);
+  const int col = blockIdx.x * 16 + (lane & 15), cc = min(col, dv - 1);
+  const size_t r = p.seq_start[b];
+  const bool fresh = p.seq_pos0[b] == 0;
+  float* st = p.state + (((size_t)p.seq_slot[b] * H + hd) * N) * dv;
+  const float* row = p.xbc + r * p.ldx;
+  const float *Bp = row + inner + (size_t)g * N, *Cp = Bp + (size_t)p.groups * N;
+  float S[NR], Bt[NR], Ct[NR];
+  if constexpr (VEC) {
+    typedef float four_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int i = 0; i < NR; i += 4) {
+      const four_t bv = *(const four_t*)(Bp + n0 + i), cv = *(const four_t*)(Cp + n0 + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) Bt[i + e] = bv[e], Ct[i + e] = cv[e];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) Bt[i] = Bp[min(n0 + i, N - 1)], Ct[i] = Cp[min(n0 + i, N - 1)];
+  }
+  const float raw = p.dt[r * p.ldd + hd], bias = p.dt_bias[hd], rate = expf(p.A_log[hd]), Dh = p.D[hd], x = row[hd * dv + cc];
+  if (fresh) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) S[i] = 0.0f;
+  } else {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) S[i] = st[(size_t)min(n0 + i, N - 1) * dv + cc];
+  }
+  const float d = softplus_f(raw + bias), a = expf(-rate * d), dx = d * x;
+  float acc = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    if (!VEC && n0 + i >= N) break;
+    S[i] = fmaf(a, S[i], Bt[i] * dx);
+    acc = fmaf(S[i], Ct[i], acc);
+  }
+  acc = lga::lanes_join_sum<16>(acc);  // (the quarters' sums in twos, then those)
+  lga::wait_loads(S);
+  if (col >= dv) return;
+  if (lane < 16) p.y[r * inner + hd * dv + col] = fmaf(Dh, x, acc);
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+    if (VEC || n0 + i < N) st[(size_t)(n0 + i) * dv + col] = S[i];
 }
 
 // The prompt form of the scan: chunks of 64 tokens as fp32 matrix products (v_mfma_f32_16x16x4_f32), all chunks of
@@ -1100,6 +1155,27 @@ extern "C" int lgs_ssm_scan(const float* xbc, long ldx, const float* dt, long ld
   else if (nr <= 16) lgs::ssm_scan_kernel<16><<<grid, 256, 0, stream>>>(p);
   else if (nr <= 32) lgs::ssm_scan_kernel<32><<<grid, 256, 0, stream>>>(p);
   else lgs::ssm_scan_kernel<64><<<grid, 256, 0, stream>>>(p);
+  LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lgs_ssm_one(const float* xbc, long ldx, const float* dt, long ldd, const float* dt_bias, const float* A_log,
+                           const float* D, float* state, const int* seq_start, const int* seq_slot, const int* seq_pos0,
+                           float* y, int B, int heads, int groups, int N, int dv, hipStream_t stream) {
+  LGA_CHECK_ARG(xbc && dt && dt_bias && A_log && D && state && seq_start && seq_slot && seq_pos0 && y,
+                "lgs_ssm_one: null pointer");
+  LGA_CHECK_ARG(B > 0 && B <= 65535 && heads > 0 && heads <= 65535 && groups > 0 && heads % groups == 0,
+                "lgs_ssm_one: heads must be a multiple of the groups");
+  LGA_CHECK_ARG(N > 0 && N <= 128 && dv > 0, "lgs_ssm_one: state size 1 to 128");
+  LGA_CHECK_ARG(ldx >= (long)heads * dv + 2L * groups * N && ldd >= heads, "lgs_ssm_one: rows shorter than their parts");
+  lgs::ScanArgs p{xbc, ldx, dt, ldd, dt_bias, A_log, D, state, seq_start, seq_slot, seq_pos0, y, heads, groups, N, dv};
+  const dim3 grid((dv + 15) / 16, heads, B);
+  const bool vec = ldx % 4 == 0 && (heads * dv) % 4 == 0 && (uintptr_t)xbc % 16 == 0;
+  const int nr = (N + 3) / 4;
+  if (vec && N == 128) lgs::ssm_one_kernel<32, true><<<grid, 64, 0, stream>>>(p);
+  else if (vec && N == 64) lgs::ssm_one_kernel<16, true><<<grid, 64, 0, stream>>>(p);
+  else if (nr <= 8) lgs::ssm_one_kernel<8, false><<<grid, 64, 0, stream>>>(p);
+  else if (nr <= 16) lgs::ssm_one_kernel<16, false><<<grid, 64, 0, stream>>>(p);
+  else lgs::ssm_one_kernel<32, false><<<grid, 64, 0, stream>>>(p);
   LGA_LAUNCH_RETURN();
 }
 

@@ -69,6 +69,7 @@ SIGNATURES = {
                      _F, _P],
     "lgs_conv_silu": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "lgs_ssm_scan": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P],
+    "lgs_ssm_one": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "lgs_ssm_walk": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P],
     "lgs_gated_group_norm": [_P, _P, _L, _P, _F, _P, _P, _I, _I, _I, _P],
     "lgs_glu_clamped": [_P, _P, _L, _P, _I, _I, _I, _F, _F, _F, _P],
@@ -830,6 +831,13 @@ def ssm_scan(xbc: torch.Tensor, proj: torch.Tensor, dt_off: int, dt_bias: torch.
     if chunked is None:
         chunked = max_len > 16 and N <= 128
     ws, wdec, max_chunks = None, None, 0
+    if not chunked and max_len == 1 and T == B and N <= 128 and B * heads * -(-dv // 16) <= 1024:
+        _check(load_library().lgs_ssm_one(_dev(xbc, "xbc", F32), ldx, _dev(proj, "proj", F32) + 4 * dt_off, proj.shape[1],
+                                          _dev(dt_bias, "dt_bias", F32), _dev(A_log, "A_log", F32), _dev(D, "D", F32),
+                                          _dev(state, "state", F32), _dev(seq_start, "seq_start", I32),
+                                          _dev(seq_slot, "seq_slot", I32), _dev(seq_pos0, "seq_pos0", I32), y.data_ptr(), B,
+                                          heads, groups, N, dv, _stream()))
+        return y
     if chunked:
         if not 0 < max_len <= T or N > 128:
             raise ValueError("ssm_scan: the prompt form needs the longest sequence's token count and N <= 128")

@@ -61,3 +61,24 @@ def test_chunks_walked_against_side_by_side(heads, groups, N, dv, lens, monkeypa
     torch.testing.assert_close(state[True], state[False], rtol=0, atol=0, equal_nan=True)
     assert torch.equal(state[True][-1], stale[-1])
     assert torch.isfinite(y[True]).any()
+
+
+@pytest.mark.parametrize("heads,groups,N,dv,B", [(64, 8, 128, 64, 3), (6, 3, 23, 40, 3), (16, 2, 64, 72, 5), (8, 8, 100, 130, 2), (1, 1, 1, 1, 1)])
+def test_one_token_a_sequence(heads, groups, N, dv, B):
+    """ssm_one_kernel against the walk of tokens: the same bits, fresh sequences and continued ones, rows off 16 bytes too."""
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import StepBatch
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(N + dv)
+    rand = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    xbc, raw = rand(B, heads * dv + 2 * groups * N), rand(B, heads + 3)
+    dt_bias, A_log, D = rand(heads) - 1.0, rand(heads), rand(heads)
+    stale = rand(B + 1, heads, N, dv)
+    step = StepBatch.build([(i, i, [0]) for i in range(B)], dev)
+    y, state = {}, {}
+    for max_len in (0, 1):  # 0: not known to be one token each
+        state[max_len] = stale.clone()
+        y[max_len] = seq_ops.ssm_scan(xbc, raw, 2, dt_bias, A_log, D, state[max_len], step.seq_start, step.seq_slot, step.seq_pos0,
+                                      heads=heads, groups=groups, N=N, dv=dv, max_len=max_len)
+    assert torch.equal(y[0], y[1]) and torch.equal(state[0], state[1]) and torch.equal(state[1][-1], stale[-1])
