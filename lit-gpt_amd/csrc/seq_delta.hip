@@ -366,12 +366,15 @@ __device__ __forceinline__ void lanes_sum2(float& a, float& b) {
 
 // grid (B * H * ceil(dv / CW) rounded up to 8), CW = 256 / LPC columns per workgroup. Lane l of a wave: r = l % LPC, column
 // l / LPC of the wave's 64 / LPC; the lane holds the rows 4 (r + LPC j) + e, j < NR4, e < 4, of its column.
-template <int NR4, int LPC, bool DELTA>
+// ONE: sequences of one token (of more, too, but slowly): nothing is staged for tokens that do not come, and the state is on its way
+// beside the rows. us, the general form / this, a decay per channel: 8 sequences of 16 heads of 128 x 128 9.3 / 7.1, 3 7.7 / 6.3, 1 4.3 /
+// 3.7, 32 19.9 / 15.1, 8 of 32 heads 11.0 / 8.7, 4 of 4 heads of 256 x 256 8.5 / 6.9, 3 of 512 x 64 11.8 / 10.6.
+template <int NR4, int LPC, bool DELTA, bool ONE>
 __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
   constexpr int DP = 4 * NR4 * LPC;      // rows, padded
   constexpr int CW = 256 / LPC;          // columns per workgroup
   constexpr int ROW = 3 * DP + CW + 4;   // staged floats per token: q | k | g | v | beta (rows stay 16-byte aligned)
-  constexpr int kDeltaTB = DP > 256 ? 8 : (DP > 128 ? 16 : 32);  // tokens staged at a time
+  constexpr int kDeltaTB = ONE ? 1 : DP > 256 ? 8 : (DP > 128 ? 16 : 32);  // tokens staged at a time
   constexpr int EPT = (ROW + 255) / 256;       // staged entries per thread and token
   constexpr int KEEP = (kDeltaTB + LPC - 1) / LPC;  // outputs of a batch that a lane keeps
   __shared__ __attribute__((aligned(16))) float st[(kDeltaTB + 1) * ROW];  // (a batch's last token reads one row ahead)
@@ -398,13 +401,15 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 4 * (r + LPC * j) + e;
-      S[j][e] = (!fresh && live && row < d) ? sp[(size_t)row * dv + col] : 0.0f;
+      if (ONE) S[j][e] = sp[(size_t)min(row, d - 1) * dv + min(col, dv - 1)];
+      else S[j][e] = (!fresh && live && row < d) ? sp[(size_t)row * dv + col] : 0.0f;
     }
   // (the loads of S end here: left to the token loop's first use, every batch there would wait for the next one's loads)
+  if constexpr (!ONE)
 #pragma unroll
-  for (int j = 0; j < NR4; ++j)
+    for (int j = 0; j < NR4; ++j)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(S[j][e]));
+      for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(S[j][e]));
   // Entry e = tid + 256 i of a token's staged row comes from one place whatever the token: a pointer to it at the
   // sequence's first row, the distance to the next token's, and the value of an entry that has no source (padding).
   // (an entry without a source loads a valid address all the same, so that the loads carry no branches)
@@ -445,6 +450,12 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
       }
   };
   prefetch(0);
+  if constexpr (ONE)
+#pragma unroll
+    for (int j = 0; j < NR4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (fresh || !live || 4 * (r + LPC * j) + e >= d) S[j][e] = 0.0f;
 
   struct Token {
     float4 k[NR4], g[NR4], q[NR4];
@@ -517,7 +528,7 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
     // every LPC-th token stays in one lane's register instead of a branch and a store per token. 2048 tokens of 16 heads
     // of 128 x 128: 438 us, one token's reads after the other's work 667; with 32 rows a lane the second set of operands
     // does not fit the registers (8 x 512 tokens of 8 heads of 256 x 256: 623 us against 462).
-    if (NR4 <= 4 && nb == kDeltaTB) {
+    if (!ONE && NR4 <= 4 && nb == kDeltaTB) {
       Token x[2];
       const float* row = st;
       fetch(row, x[0]);
@@ -556,6 +567,7 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
         p.out[(size_t)(r0 + t0 + t) * H * dv + (size_t)hd * dv + cblk * CW + c] = os[t][c];
     }
   }
+  lga::wait_loads();
   if (live) {
 #pragma unroll
     for (int j = 0; j < NR4; ++j)
@@ -910,16 +922,16 @@ static void gated_delta_wide_launch(DeltaArgs p, int B, bool plain, hipStream_t 
   }
 }
 
-template <int LPC, bool DELTA>
+template <int LPC, bool DELTA, bool ONE>
 static bool gated_delta_launch(DeltaArgs p, int B, hipStream_t stream) {
   p.ncb = (p.dv + 256 / LPC - 1) / (256 / LPC);
   p.items = B * p.H * p.ncb;
   const dim3 grid((p.items + 7) / 8 * 8);
   const int nr4 = (p.d + 4 * LPC - 1) / (4 * LPC);
-  if (nr4 <= 1) gated_delta_kernel<1, LPC, DELTA><<<grid, 256, 0, stream>>>(p);
-  else if (nr4 <= 2) gated_delta_kernel<2, LPC, DELTA><<<grid, 256, 0, stream>>>(p);
-  else if (nr4 <= 4) gated_delta_kernel<4, LPC, DELTA><<<grid, 256, 0, stream>>>(p);
-  else if (nr4 <= 8) gated_delta_kernel<8, LPC, DELTA><<<grid, 256, 0, stream>>>(p);
+  if (nr4 <= 1) gated_delta_kernel<1, LPC, DELTA, ONE><<<grid, 256, 0, stream>>>(p);
+  else if (nr4 <= 2) gated_delta_kernel<2, LPC, DELTA, ONE><<<grid, 256, 0, stream>>>(p);
+  else if (nr4 <= 4) gated_delta_kernel<4, LPC, DELTA, ONE><<<grid, 256, 0, stream>>>(p);
+  else if (nr4 <= 8) gated_delta_kernel<8, LPC, DELTA, ONE><<<grid, 256, 0, stream>>>(p);
   else return false;
   return true;
 }
@@ -996,10 +1008,9 @@ extern "C" int lgs_delta_step_prepare(const float* u, long ldu, const void* conv
   LGA_LAUNCH_RETURN();
 }
 
-extern "C" int lgs_gated_delta(const float* qkv, long ld, const float* dec, const float* beta, const float* kq,
-                               float* state, const int* seq_start, const int* seq_slot, const int* seq_pos0, float* out,
-                               int B, int H, int G, int d, int dv, int per_channel, int lanes, int plain,
-                               hipStream_t stream) {
+static int gated_delta_any(const float* qkv, long ld, const float* dec, const float* beta, const float* kq, float* state,
+                           const int* seq_start, const int* seq_slot, const int* seq_pos0, float* out, int B, int H, int G, int d,
+                           int dv, int per_channel, int lanes, int plain, bool one, hipStream_t stream) {
   LGA_CHECK_ARG(qkv && dec && (beta || plain) && kq && state && seq_start && seq_slot && seq_pos0 && out,
                 "lgs_gated_delta: null pointer");
   LGA_CHECK_ARG(B > 0 && H > 0 && G > 0 && H % G == 0 && d > 0 && d <= 512 && dv > 0,
@@ -1024,10 +1035,31 @@ extern "C" int lgs_gated_delta(const float* qkv, long ld, const float* dec, cons
   }
   while (lpc < 16 && d > 32 * lpc) lpc <<= 1;
   bool ok;
-  if (lpc == 4) ok = plain ? lgs::gated_delta_launch<4, false>(p, B, stream) : lgs::gated_delta_launch<4, true>(p, B, stream);
-  else if (lpc == 8) ok = plain ? lgs::gated_delta_launch<8, false>(p, B, stream) : lgs::gated_delta_launch<8, true>(p, B, stream);
-  else if (lpc == 16) ok = plain ? lgs::gated_delta_launch<16, false>(p, B, stream) : lgs::gated_delta_launch<16, true>(p, B, stream);
+  auto go = [&](auto n) {
+    constexpr int L = decltype(n)::value;
+    if (one) return plain ? lgs::gated_delta_launch<L, false, true>(p, B, stream) : lgs::gated_delta_launch<L, true, true>(p, B, stream);
+    return plain ? lgs::gated_delta_launch<L, false, false>(p, B, stream) : lgs::gated_delta_launch<L, true, false>(p, B, stream);
+  };
+  if (lpc == 4) ok = go(std::integral_constant<int, 4>{});
+  else if (lpc == 8) ok = go(std::integral_constant<int, 8>{});
+  else if (lpc == 16) ok = go(std::integral_constant<int, 16>{});
   else ok = false;
   LGA_CHECK_ARG(ok, "lgs_gated_delta: lanes per column must be 4, 8 or 16 and cover the key dim");
   LGA_LAUNCH_RETURN();
+}
+
+extern "C" int lgs_gated_delta(const float* qkv, long ld, const float* dec, const float* beta, const float* kq,
+                               float* state, const int* seq_start, const int* seq_slot, const int* seq_pos0, float* out,
+                               int B, int H, int G, int d, int dv, int per_channel, int lanes, int plain,
+                               hipStream_t stream) {
+  return gated_delta_any(qkv, ld, dec, beta, kq, state, seq_start, seq_slot, seq_pos0, out, B, H, G, d, dv, per_channel, lanes, plain,
+                         false, stream);
+}
+
+extern "C" int lgs_gated_delta_one(const float* qkv, long ld, const float* dec, const float* beta, const float* kq,
+                                   float* state, const int* seq_start, const int* seq_slot, const int* seq_pos0, float* out,
+                                   int B, int H, int G, int d, int dv, int per_channel, int lanes, int plain,
+                                   hipStream_t stream) {
+  return gated_delta_any(qkv, ld, dec, beta, kq, state, seq_start, seq_slot, seq_pos0, out, B, H, G, d, dv, per_channel, lanes, plain,
+                         true, stream);
 }

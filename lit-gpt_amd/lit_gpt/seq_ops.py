@@ -90,6 +90,7 @@ SIGNATURES = {
     "lgs_mingru": [_P, _P, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _P, _I, _P],
     "lgs_mingru_step": [_P, _L, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P],
     "lgs_gated_delta": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
+    "lgs_gated_delta_one": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
 }
 _RESTYPES = {"lgs_last_error_string": ctypes.c_char_p}
 
@@ -1208,10 +1209,10 @@ def gated_delta(qkv: torch.Tensor, dec: torch.Tensor, beta: Optional[torch.Tenso
             kq.shape != (T, G):
         raise ValueError("gated_delta: shapes")
     out = torch.empty(T, H * dv, dtype=F32, device=qkv.device)
-    _check(load_library().lgs_gated_delta(_dev(qkv, "qkv", F32) + 4 * qkv_off, ld, _dev(dec, "dec", F32),
-                                          _opt(beta, "beta", F32) if plain else _dev(beta, "beta", F32),
-                                          _dev(kq, "kq", F32), _dev(state, "state", F32), _dev(seq_start, "seq_start", I32),
-                                          _dev(seq_slot, "seq_slot", I32), _dev(seq_pos0, "seq_pos0", I32),
-                                          out.data_ptr(), B, H, G, d, dv, int(per_channel), int(lanes), int(plain),
-                                          _stream()))
+    lib = load_library()
+    rule = lib.lgs_gated_delta_one if T == B else lib.lgs_gated_delta
+    _check(rule(_dev(qkv, "qkv", F32) + 4 * qkv_off, ld, _dev(dec, "dec", F32),
+                _opt(beta, "beta", F32) if plain else _dev(beta, "beta", F32), _dev(kq, "kq", F32), _dev(state, "state", F32),
+                _dev(seq_start, "seq_start", I32), _dev(seq_slot, "seq_slot", I32), _dev(seq_pos0, "seq_pos0", I32),
+                out.data_ptr(), B, H, G, d, dv, int(per_channel), int(lanes), int(plain), _stream()))
     return out

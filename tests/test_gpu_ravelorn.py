@@ -810,3 +810,28 @@ def test_two_streams_equal_one():
         ParallelMixer.overlap = True
     for a, b in zip(one, two):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,G,d,dv,B,per_channel,plain", [(16, 16, 128, 128, 8, True, False), (8, 4, 64, 72, 5, True, True),
+                                                          (4, 2, 100, 36, 6, False, False), (4, 4, 256, 256, 4, True, False),
+                                                          (2, 2, 16, 40, 2, True, False), (3, 1, 512, 64, 3, True, False)])
+def test_one_token_a_sequence(H, G, d, dv, B, per_channel, plain, monkeypatch):
+    """The delta rule's form for steps of one token a sequence against the general one: the same bits; one and two lanes' rows past the
+    key dim, columns that end inside a workgroup's, a fresh sequence over a slot with stale contents."""
+    from lit_gpt import seq_ops
+    from lit_gpt.mixers import StepBatch
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(d + dv)
+    rand = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    qkv, kq, stale = rand(B, 2 * G * d + H * dv) * d ** -0.5, rand(B, G), rand(B + 1, H, d, dv)
+    dec, beta = (torch.rand(B, n, generator=g, device=dev) for n in (H * d if per_channel else H, H))
+    step = StepBatch.build([(i, i, [0]) for i in range(B)], dev)
+    lib, got = seq_ops.load_library(), []
+    for rule in (lib.lgs_gated_delta_one, lib.lgs_gated_delta):
+        monkeypatch.setattr(lib, "lgs_gated_delta_one", rule)
+        state = stale.clone()
+        o = seq_ops.gated_delta(qkv, dec, None if plain else beta, kq, state, step.seq_start, step.seq_slot, step.seq_pos0, H=H, G=G,
+                                d=d, dv=dv, per_channel=per_channel, plain=plain)
+        got.append((o, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][1][-1], stale[-1])
