@@ -108,23 +108,36 @@ template <int SMAX, int CPT, int NT>
 __global__ void __launch_bounds__(NT) streams_step_reg_kernel(StreamArgs p) {
   __shared__ float red[NT / 64];
   __shared__ float cm[kMaxStreams * kMaxStreams], cb[kMaxStreams], ca[kMaxStreams];
-  const int s = p.s, W = p.W;
-  if (threadIdx.x < s * s) cm[threadIdx.x] = p.mix ? p.mix[threadIdx.x] : 0.0f;
-  if (threadIdx.x < s) {
-    cb[threadIdx.x] = p.out ? p.out[threadIdx.x] : 0.0f;
-    ca[threadIdx.x] = p.in ? p.in[threadIdx.x] : 0.0f;
-  }
+  const int s = p.s, W = p.W, tid = threadIdx.x;
   float* xt = p.x + (size_t)blockIdx.x * s * W;
   const float* yt = p.y ? p.y + (size_t)blockIdx.x * W : nullptr;
-  float v[SMAX][CPT], y[CPT], nw[CPT];
+  // (streams and columns past the last: those again, left out below; a load under a condition of its own is a branch. One token of four
+  // streams of 2048: 5.1 us with branches and the links' loads ahead, 4.5 here)
+  float v[SMAX][CPT], y[CPT], nw[CPT], mix = 0.0f, wr = 0.0f, rd = 0.0f;
 #pragma unroll
-  for (int c = 0; c < CPT; ++c) {
-    const int i = threadIdx.x + NT * c;
+  for (int c = 0; c < CPT; ++c)
 #pragma unroll
-    for (int j = 0; j < SMAX; ++j) v[j][c] = (j < s && i < W) ? xt[(size_t)j * W + i] : 0.0f;
-    y[c] = (yt && i < W) ? yt[i] : 0.0f;
-    nw[c] = (p.in && p.w && i < W) ? p.w[i] : 1.0f;
+    for (int j = 0; j < SMAX; ++j) v[j][c] = xt[(size_t)min(j, s - 1) * W + min(tid + NT * c, W - 1)];
+  if (yt) {
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) y[c] = yt[min(tid + NT * c, W - 1)];
   }
+  if (p.in && p.w) {
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) nw[c] = p.w[min(tid + NT * c, W - 1)];
+  }
+  if (p.mix) mix = p.mix[min(tid, s * s - 1)];
+  if (p.out) wr = p.out[min(tid, s - 1)];
+  if (p.in) rd = p.in[min(tid, s - 1)];
+  if (tid < s * s) cm[tid] = mix;
+  if (tid < s) cb[tid] = wr, ca[tid] = rd;
+#pragma unroll
+  for (int c = 0; c < CPT; ++c)
+    if (tid + NT * c >= W) {
+      y[c] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < SMAX; ++j) v[j][c] = 0.0f;
+    }
   __syncthreads();
   float u[CPT], ss = 0.0f;
 #pragma unroll
