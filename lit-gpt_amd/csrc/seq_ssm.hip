@@ -578,10 +578,10 @@ __global__ void __launch_bounds__(256) ssd_carry_kernel(SsdArgs p) {
 // ssd_scores_kernel) become the operand of theirs. C and B of a chunk are staged in LDS while the chunk before is worked on. The sums
 // stand in the order of the kernels above, so the results have their bits.
 // Bound by the fp32 matrix instruction: 296 of 32 clocks a chunk and wave for N = 128, two thirds of the time it takes (6.1 us a chunk
-// and workgroup). 1500 + 777 + 130 tokens of 128 heads of 128 x 64 take 180 us, the three kernels above 340 (their chunks' states are
-// 640 MB written and read); four times 500 tokens of 64 heads 66 against 110; one chunk 16 to 19 against 24 to 29 whatever the heads.
-// With everything a chunk needs loaded and written at the start of a half 188, with decays and scores' exponentials made by every
-// wave 240, with row offsets held in registers (and spilled) 450.
+// and workgroup). 1500 + 777 + 130 tokens of 128 heads of 128 x 64 take 177 us, the three kernels above 340 (their chunks' states are
+// 640 MB written and read); four times 500 tokens of 64 heads 65 against 110; one chunk 16 to 19 against 24 to 29 whatever the heads.
+// With operands read as late as the instruction group before 180, with everything a chunk needs loaded and written at the start of a half
+// 188, with decays and scores' exponentials made by every wave 240, with row offsets held in registers (and spilled) 450.
 struct WalkArgs {
   SsdArgs s;
   float* scores;  // [B * max_chunks][groups][10][64][4]
@@ -771,10 +771,14 @@ __global__ void __launch_bounds__(256, 2) ssd_walk_kernel(WalkArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 4 * t + e;
+        if (e == 0)
+#pragma unroll
+          for (int ti = 0; ti < 4; ++ti) {
+            if (t + 1 < NT) read_c(ca[(t + 1) & 1][ti], t + 1, ti);
+            else read_g(ca[(t + 1) & 1][ti], 0, ti);
+          }
 #pragma unroll
         for (int ti = 0; ti < 4; ++ti) o[ti] = ssd_mma(ca[t & 1][ti][e], S[t][e], o[ti]);
-        if (t + 1 < NT) read_c(ca[(t + 1) & 1][e], t + 1, e);
-        else read_g(ca[(t + 1) & 1][e], 0, e);
         if (i < 8) fetch_x(2 * i, xs, ax), fetch_x(2 * i + 1, xs, ax);
         if (i < LD) put_row(Bs, br[i], i);
         if (i >= 8 && i < 8 + LD) fetch_row(cr[i - 8], cs, ac);
@@ -793,7 +797,9 @@ __global__ void __launch_bounds__(256, 2) ssd_walk_kernel(WalkArgs a) {
     for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        if (tj < 3) read_g(ca[(tj + 1) & 1][e], tj + 1, e);
+        if (tj < 3 && e == 0)
+#pragma unroll
+          for (int ti = 0; ti < 4; ++ti) read_g(ca[(tj + 1) & 1][ti], tj + 1, ti);
 #pragma unroll
         for (int ti = 0; ti < 4; ++ti)
           if (ti >= tj) o[ti] = ssd_mma(ca[tj & 1][ti][e], x[tj * 4 + e], o[ti]);
@@ -821,9 +827,9 @@ __global__ void __launch_bounds__(256, 2) ssd_walk_kernel(WalkArgs a) {
     }
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
+      if (k + 1 < 16) read_b(bv[(k + 1) & 1], k + 1);
 #pragma unroll
       for (int t = 0; t < NT / 2; ++t) s[t] = ssd_mma(bv[k & 1][t], x[k], s[t]);
-      if (k + 1 < 16) read_b(bv[(k + 1) & 1], k + 1);
       if (k % 4 != 3) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int t = NT / 2; t < NT; ++t) s[t] = ssd_mma(bv[k & 1][t], x[k], s[t]);
@@ -1066,8 +1072,8 @@ __global__ void __launch_bounds__(256) gated_group_norm_kernel(const float* __re
 }
 
 // The same for groups of up to 256 NV columns: the values stay in registers, where the kernel above writes `out`, reads it again and
-// writes it twice; beside a bf16 copy `out` may be null. The same sums in the same order. us, the kernel above / this: 2407 tokens of 8 groups of 1024,
-// bf16 alone 76.4 / 29.9, 2000 of 4 of 2048, fp32 49.8 / 30.2, 2048 of 8 of 512 26.5 / 17.4, one token 2.6 / 2.2.
+// writes it twice; beside a bf16 copy `out` may be null. The same sums in the same order. us, the kernel above / this: 2407 tokens of 8
+// groups of 1024, bf16 alone 76.4 / 29.9, 2000 of 4 of 2048, fp32 49.8 / 30.2, 2048 of 8 of 512 26.5 / 17.4, one token 2.6 / 2.2.
 template <int NV>
 __global__ void __launch_bounds__(256) gated_group_norm_reg_kernel(const float* __restrict__ y, const float* __restrict__ z,
                                                                    long ldz, const float* __restrict__ w, float eps,
