@@ -651,6 +651,7 @@ def test_prompt_whose_streams_are_not_stored(streams, dtype, T, monkeypatch):
         step = StepBatch.build([(0, 0, toks)], model.device)
         calls = []
         whole, one = seq_ops.streams_step, seq_ops.streams_held
+        monkeypatch.setattr(type(model), "HELD_FROM", 0)
         monkeypatch.setattr(seq_ops, "streams_held", lambda *a, **k: calls.append("held") or one(*a, **k))
         monkeypatch.setattr(seq_ops, "streams_step", lambda *a, **k: calls.append("step") or whole(*a, **k))
         got = model.forward_step(step)
