@@ -286,7 +286,8 @@ int lgs_delta_step_prepare(const float* u, long ldu, const void* conv_w, int con
 int lgs_gated_delta(const float* qkv, long ld, const float* dec, const float* beta, const float* kq, float* state,
                     const int* seq_start, const int* seq_slot, const int* seq_pos0, float* out, int B, int H, int G, int d,
                     int dv, int per_channel, int lanes, int plain, lgs_stream_t stream);
-/* The same, to the same bits, for steps in which every sequence brings one token (others are walked, slowly). */
+/* The same, to the same bits, for steps in which every sequence brings one token (others are walked, slowly; one without tokens
+ * keeps its state, or gets zeros at position 0, in either). */
 int lgs_gated_delta_one(const float* qkv, long ld, const float* dec, const float* beta, const float* kq, float* state,
                         const int* seq_start, const int* seq_slot, const int* seq_pos0, float* out, int B, int H, int G, int d,
                         int dv, int per_channel, int lanes, int plain, lgs_stream_t stream);

@@ -391,7 +391,8 @@ __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
   const int d = p.d, dv = p.dv, H = p.H;
   const bool live = col < dv;
   const int g = hd / (H / p.G);
-  const int r0 = p.seq_start[b], n = p.seq_start[b + 1] - r0;
+  // (a sequence without tokens loads the first row ahead, for nothing: its own place may be past the last one)
+  const int first = p.seq_start[b], n = p.seq_start[b + 1] - first, r0 = n > 0 ? first : 0;
   const int dc = p.per_channel ? d : 1;
   float* sp = p.state + (((size_t)p.seq_slot[b] * H + hd) * d) * dv;
   const bool fresh = p.seq_pos0[b] == 0;

@@ -835,3 +835,41 @@ def test_one_token_a_sequence(H, G, d, dv, B, per_channel, plain, monkeypatch):
                                 d=d, dv=dv, per_channel=per_channel, plain=plain)
         got.append((o, state))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][1][-1], stale[-1])
+
+
+@pytest.mark.parametrize("H,G,d,dv,per_channel,plain", [(4, 4, 128, 128, True, False), (40, 8, 128, 128, True, False), (2, 1, 64, 72, False, False),
+                                                        (4, 2, 100, 36, False, True), (2, 2, 256, 48, True, False), (3, 1, 512, 64, True, False)])
+@pytest.mark.parametrize("lens", [[2, 0], [0, 1, 2, 3, 0, 0], [3, 0, 0, 1, 4, 0, 0, 0], [0, 0, 0, 4]])
+def test_one_token_form_over_other_lengths(H, G, d, dv, per_channel, plain, lens):
+    """As many tokens as sequences, which is what chooses the form for one token each, but not one each: walked to the bits of the general
+    form and of 16 lanes a column, which take the sequences that have tokens alone; those without keep their states, the last ones too,
+    behind whose place no row is."""
+    from lit_gpt import seq_ops
+
+    dev, T, B = torch.device("cuda", 0), sum(lens), len(lens)
+    g = torch.Generator(device=dev).manual_seed(d + B)
+    rand = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    qkv, kq, stale = rand(T, 2 * G * d + H * dv) * d ** -0.5, rand(T, G), rand(B, H, d, dv)
+    dec, beta = (torch.rand(T, n, generator=g, device=dev) for n in (H * d if per_channel else H, H))
+    table = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    start = [sum(lens[:b]) for b in range(B + 1)]
+    pos0 = [5 * (b % 2) for b in range(B)]
+    lib, got = seq_ops.load_library(), []
+
+    def rule(function, some, lanes):
+        out, state = torch.full((T, H * dv), 7.0, device=dev), stale.clone()
+        starts, slots, first = table([start[b] for b in some] + [T]), table(some), table([pos0[b] for b in some])
+        seq_ops._check(function(qkv.data_ptr(), qkv.shape[1], dec.data_ptr(), None if plain else beta.data_ptr(), kq.data_ptr(),
+                                state.data_ptr(), starts.data_ptr(), slots.data_ptr(), first.data_ptr(), out.data_ptr(), len(some), H, G,
+                                d, dv, int(per_channel), lanes, int(plain), seq_ops._stream()))
+        return out, state
+
+    want, want_state = rule(lib.lgs_gated_delta, [b for b in range(B) if lens[b]], 16)
+    for b in range(B):
+        if not lens[b] and not pos0[b]:
+            want_state[b] = 0.0
+    for function in (lib.lgs_gated_delta_one, lib.lgs_gated_delta):
+        out, state = rule(function, list(range(B)), 16)
+        assert torch.equal(out, want) and torch.equal(state, want_state)
+        got.append(rule(function, list(range(B)), 0))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
