@@ -180,7 +180,8 @@ int lgs_token_side(float* x, const int* tokens, const void* table, int w_f32, lo
                    float eps, lgs_stream_t stream);
 
 /* ---- several residual streams (hyper-connections) ---- */
-/* x[t][j] = table[tokens[t]] * scale for each of `streams` streams: x is [T][streams][W] */
+/* x[t][j] = table[tokens[t]] * scale for each of `streams` streams: x is [T][streams][W]. An id outside the table's `vocab` rows takes
+ * its first or last one, here and below. */
 int lgs_embed_streams(const int* tokens, const void* table, int w_f32, float scale, float* x, int T, int W, int vocab,
                       int streams, lgs_stream_t stream);
 /* One sublayer boundary on x [T][streams][W], in place. With y [T][W] (a sublayer's output):

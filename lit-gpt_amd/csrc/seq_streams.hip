@@ -22,9 +22,9 @@ constexpr int kMaxStreams = 8;
 
 template <bool WF32>
 __global__ void __launch_bounds__(256) embed_streams_kernel(const int* __restrict__ tokens, const void* __restrict__ table,
-                                                            float scale, float* __restrict__ x, int W, int streams) {
+                                                            float scale, float* __restrict__ x, int W, int vocab, int streams) {
   const size_t t = blockIdx.x;
-  const size_t src = (size_t)tokens[t] * W;
+  const size_t src = (size_t)min(max(tokens[t], 0), vocab - 1) * W;  // (the host validates ids; never read out of bounds)
   for (int i = blockIdx.y * 256 + threadIdx.x; i < W; i += gridDim.y * 256) {
     const float v = wload<WF32>(table, src + i) * scale;
     for (int j = 0; j < streams; ++j) x[(t * streams + j) * W + i] = v;
@@ -218,7 +218,7 @@ constexpr int kMaxHeld = 8;
 struct HeldArgs {
   const int* tokens;  // embedding base: x_j = table[tokens[t]] * scale
   const void* table;
-  int w_f32;
+  int w_f32, vocab;
   float scale;
   const float* base;  // stored base [T][s][W]
   float* x;           // where the streams are stored (null: nowhere; base itself or another place)
@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(256) streams_held_kernel(HeldArgs p) {
   const int tid = threadIdx.x, W = p.W;
   const size_t t = blockIdx.x;
   const float* base = FROM == 2 ? p.base + t * S * W : nullptr;
-  const size_t row = FROM == 2 ? 0 : (size_t)p.tokens[t] * W;
+  const size_t row = FROM == 2 ? 0 : (size_t)min(max(p.tokens[t], 0), p.vocab - 1) * W;  // (as above)
   const float* table32 = (const float*)p.table + row;
   const uint16_t* table16 = (const uint16_t*)p.table + row;
   struct Columns {
@@ -599,8 +599,8 @@ extern "C" int lgs_embed_streams(const int* tokens, const void* table, int w_f32
   LGA_CHECK_ARG(tokens && table && x && T > 0 && W > 0 && vocab > 0, "lgs_embed_streams: bad arguments");
   LGA_CHECK_ARG(streams >= 1 && streams <= lgs::kMaxStreams, "lgs_embed_streams: 1 to 8 streams");
   const dim3 grid = lgs::embed_grid(T, W);
-  if (w_f32) lgs::embed_streams_kernel<true><<<grid, 256, 0, stream>>>(tokens, table, scale, x, W, streams);
-  else lgs::embed_streams_kernel<false><<<grid, 256, 0, stream>>>(tokens, table, scale, x, W, streams);
+  if (w_f32) lgs::embed_streams_kernel<true><<<grid, 256, 0, stream>>>(tokens, table, scale, x, W, vocab, streams);
+  else lgs::embed_streams_kernel<false><<<grid, 256, 0, stream>>>(tokens, table, scale, x, W, vocab, streams);
   LGA_LAUNCH_RETURN();
 }
 
@@ -636,7 +636,7 @@ extern "C" int lgs_streams_held(const int* tokens, const void* table, int w_f32,
   LGA_CHECK_ARG(count == 0 || (y && mix && out), "lgs_streams_held: an output needs its mix matrix and weights");
   LGA_CHECK_ARG(in && (h || h_bf16) && (norm_w || !h_bf16), "lgs_streams_held: a read with a place for it (bf16: made by the norm)");
   lgs::HeldArgs p{};
-  p.tokens = tokens, p.table = table, p.w_f32 = w_f32, p.scale = scale, p.base = base, p.x = x;
+  p.tokens = tokens, p.table = table, p.w_f32 = w_f32, p.vocab = vocab, p.scale = scale, p.base = base, p.x = x;
   for (int k = 0; k < count; ++k) {
     LGA_CHECK_ARG(y[k] && mix[k] && out[k], "lgs_streams_held: an output needs its mix matrix and weights");
     p.y[k] = y[k], p.mix[k] = mix[k], p.out[k] = out[k];

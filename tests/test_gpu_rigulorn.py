@@ -634,6 +634,26 @@ def test_streams_held(s, W, T, dtype):
     assert torch.equal(plain[0], seq_ops.streams_step(x, read=read)[:T]) and plain[1] is None
 
 
+@pytest.mark.parametrize("s,W", [(2, 300), (4, 1025)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_streams_of_ids_outside_the_table(s, W, dtype):
+    """Ids that the table has no row for take its first or last one, stored and held, as the plain embedding's do."""
+    from lit_gpt import seq_ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(W)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device=dev)  # noqa: E731
+    table, read, nw = draw(9, W).to(dtype), draw(s), draw(W)
+    ids, held = torch.tensor([-1, 0, 9, 8, -2 ** 31, 2 ** 31 - 1, 4], dtype=torch.int32, device=dev), []
+    x = seq_ops.embed_streams(ids, table, 0.7, s)
+    assert torch.equal(x, seq_ops.embed_streams(ids.clamp(0, 8), table, 0.7, s)) and torch.equal(x[:, 0], seq_ops.embed(ids, table, 0.7))
+    for _ in range(2):
+        form = dict(read=read, norm_w=nw, eps=1e-5)
+        got, want = (seq_ops.streams_held(i, table, 0.7, None, held, **form)[0] for i in (ids, ids.clamp(0, 8)))
+        assert torch.equal(got, want)
+        held.append((draw(7, W), draw(s, s), draw(s)))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("streams,T", [(2, 33), (4, 33), (4, 300)])
 def test_prompt_whose_streams_are_not_stored(streams, dtype, T, monkeypatch):
