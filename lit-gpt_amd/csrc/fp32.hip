@@ -332,9 +332,11 @@ __global__ void __launch_bounds__(256) f32_layernorm_kernel(const float* __restr
 }
 
 // One row, K a multiple of 4: up to two products of a norm of the row each (f32_linear_kernel of f32_layernorm_kernel's row, to
-// the bit), a wave one output after the other. The first weights are loaded ahead of the row, and loads return in order: the
-// statistics wait for both, the sums for nothing more. pythia-160m (768 -> 2304 and 3072): norms and products in three launches 16.2
-// us, in this one 7.6 with a workgroup's norm in LDS and 7.3 with a wave's in registers.
+// the bit). A workgroup makes its norm anew, in LDS, a wave then one output after the other. The first weights are loaded ahead of the
+// row, and loads return in order: the statistics wait for both, the sums for nothing more. pythia-160m (768 -> 2304 and 3072):
+// norms and products in three launches 16.2 us, in this one 7.0. With a norm of each wave's own in registers, and no barrier, 8.1: four times
+// the loads of the row and its weights (weights from memory, LDS / registers: 512 -> 8192 6.9 / 8.8, 1024 -> 3072 and 4096 8.8 / 10.1, 256 ->
+// 50304 14.0 / 19.7; a token behind 300 keys of pythia-160m 268 / 279, of pythia-410m 582 / 613).
 struct F32NormLinear {
   const float *nw, *nb;
   float eps;
@@ -373,23 +375,10 @@ __device__ __forceinline__ void f32_dot_chunks(const float* xr, int c0, int K, i
   }
 }
 __device__ __forceinline__ float f32_dot_end(const f32x4_t& a) { return wave_sum((a.x + a.y) + (a.z + a.w)); }
-// the sum of f32_row_stats over a wave's row, whose lanes hold four neighbouring columns of every 256: s[j] belongs to thread 4 lane + j
-__device__ __forceinline__ float f32_row_sum(f32x4_t s) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const LanePair p = lane_pair<8>(s[j]);
-    float v = p.a + p.b;
-    v += lane_dpp<0x124>(v, v);  // (row_ror:4: lanes eight apart are equal)
-    v += lane_pair<2>(v).b;
-    s[j] = v + lane_pair<1>(v).b;
-  }
-  return lanes_join_sum<16>((s[0] + s[2]) + (s[1] + s[3]));
-}
-
-// Up to 1024 columns (CPT 4) every wave makes the norm for itself, in registers, with no barrier among them; longer rows stand in LDS
 template <int CPT>
 __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a) {
   extern __shared__ __attribute__((aligned(16))) float xn[];  // [K]
+  __shared__ float red[4];
   const bool second = (int)blockIdx.x >= a.p[0].blocks;
   const F32NormLinear p = second ? a.p[1] : a.p[0];
   const int block = (int)blockIdx.x - (second ? a.p[0].blocks : 0), K = a.K;
@@ -399,59 +388,27 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
   f32x4_t w[kF32Chunks];
   if (n < p.N) f32_load_chunks(p.w + (size_t)n * K, 0, K, lane, w);
   float bias = n < p.N && p.b ? p.b[n] : 0.0f;
-  f32x4_t v[kF32Chunks];
-  if constexpr (CPT == kF32Chunks) {
-    if (n >= p.N) return;
-    f32x4_t nw[kF32Chunks], nb[kF32Chunks], s = {0.0f, 0.0f, 0.0f, 0.0f}, ss = s;
-    f32_load_chunks(x, 0, K, lane, v);
-    f32_load_chunks(p.nw, 0, K, lane, nw);
-    if (p.nb) f32_load_chunks(p.nb, 0, K, lane, nb);
+  const int at = threadIdx.x;
+  float r[CPT], nw[CPT], nb[CPT], mean, var;
 #pragma unroll
-    for (int c = 0; c < kF32Chunks; ++c)
-      if (c * 256 + lane * 4 < K) s += v[c];
-    const float mean = f32_row_sum(s) / (float)K;
-#pragma unroll
-    for (int c = 0; c < kF32Chunks; ++c)
-      if (c * 256 + lane * 4 < K) {
-        const f32x4_t d = v[c] - mean;
-        f32_fma4(d, d, ss);
-      }
-    const float rstd = 1.0f / sqrtf(f32_row_sum(ss) / (float)K + p.eps);
-#pragma unroll
-    for (int c = 0; c < kF32Chunks; ++c)
-      if (c * 256 < K)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[c][j] = f32_normed(v[c][j], mean, rstd, nw[c][j], p.nb, p.nb ? nb[c][j] : 0.0f);
-  } else {
-    __shared__ float red[4];
-    const int at = threadIdx.x;
-    float r[CPT], nw[CPT], nb[CPT], mean, var;
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) {
-      const int i = at + 256 * e;
-      nw[e] = i < K ? p.nw[i] : 0.0f;
-      nb[e] = i < K && p.nb ? p.nb[i] : 0.0f;
-    }
-    f32_row_stats<CPT>(x, K, r, red, mean, var);
-    const float rstd = 1.0f / sqrtf(var + p.eps);
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) {
-      const int i = at + 256 * e;
-      if (i < K) xn[i] = f32_normed(r[e], mean, rstd, nw[e], p.nb, nb[e]);
-    }
-    for (int i = at + 256 * CPT; i < K; i += 256) xn[i] = f32_normed(x[i], mean, rstd, p.nw[i], p.nb, p.nb ? p.nb[i] : 0.0f);
-    __syncthreads();
+  for (int e = 0; e < CPT; ++e) {
+    const int i = at + 256 * e;
+    nw[e] = i < K ? p.nw[i] : 0.0f;
+    nb[e] = i < K && p.nb ? p.nb[i] : 0.0f;
   }
+  f32_row_stats<CPT>(x, K, r, red, mean, var);
+  const float rstd = 1.0f / sqrtf(var + p.eps);
+#pragma unroll
+  for (int e = 0; e < CPT; ++e) {
+    const int i = at + 256 * e;
+    if (i < K) xn[i] = f32_normed(r[e], mean, rstd, nw[e], p.nb, nb[e]);
+  }
+  for (int i = at + 256 * CPT; i < K; i += 256) xn[i] = f32_normed(x[i], mean, rstd, p.nw[i], p.nb, p.nb ? p.nb[i] : 0.0f);
+  __syncthreads();
   for (const int step = p.blocks * 4; n < p.N; n += step) {
     f32x4_t a4 = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int c0 = 0; c0 * 256 < K; c0 += kF32Chunks) {
-      if constexpr (CPT == kF32Chunks) {
-#pragma unroll
-        for (int c = 0; c < kF32Chunks; ++c)
-          if (c * 256 + lane * 4 < K) f32_fma4(v[c], w[c], a4);
-      } else {
-        f32_dot_chunks(xn, c0, K, lane, w, a4);
-      }
+      f32_dot_chunks(xn, c0, K, lane, w, a4);
       const bool more = (c0 + kF32Chunks) * 256 < K;
       if (more || n + step < p.N) f32_load_chunks(p.w + (size_t)(more ? n : n + step) * K, more ? c0 + kF32Chunks : 0, K, lane, w);
     }
@@ -471,7 +428,7 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 // outputs (kept in registers until LDS has them: as an array of HIP's float4 they went through scratch memory, a trip of their own
 // ahead of all weights). Weights from memory, an attention in five ranges, us without / with: 768 columns beside 3072 9.4 / 9.5, 1024
 // beside 4096 10.2 / 9.6, 1600 beside 6400 24.2 / 18.1, 2048 beside 8192 30.0 / 24.3, in one range 23.3 / 18.2; a token behind 300 keys:
-// pythia-160m 300 / 275, pythia-410m 676 / 606, pythia-1b 1101 / 1008. Not where x1 is no shorter than half of x2: 4096 beside 4096 in
+// pythia-160m 292 / 267, pythia-410m 652 / 581, pythia-1b 1109 / 1013. Not where x1 is no shorter than half of x2: 4096 beside 4096 in
 // five ranges 47.8 / 66.4, 2240 beside 1280 9.8 / 10.3.
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;
@@ -911,12 +868,16 @@ extern "C" int lga_f32_norm_linears(const float* x, int K, const float* nw1, con
                 "lga_f32_norm_linears: bad arguments");
   LGA_CHECK_ARG(K % 4 == 0 && K <= 8192 && ((uintptr_t)w1 | (uintptr_t)w2) % 16 == 0,
                 "lga_f32_norm_linears: K a multiple of 4 up to 8192 and 16-B aligned weights needed");
-  // One output a wave up to 2048 workgroups; beyond, a wave makes as many outputs as any other or one less, on workgroups that stand on the
-  // chip side by side. Weights from memory, 50304 outputs of 768, 1024, 2048 and 2560 columns, us in 2048 / 1280 workgroups: 34.3 / 29.7,
-  // 40.2 / 36.3, 87 / 70, 109 / 88 (1536 as 2048 or worse, 3072 within 2 % of 1280); 6144 and 8192 of 2048 in two each lose 4 %.
-  auto blocks = [](int N) {
-    const int all = (N + 3) / 4, each = all > 2048 ? (all + 1279) / 1280 : 1;
-    return (all + each - 1) / each;
+  // One output a wave up to 2048 workgroups. Beyond, a wave makes several, in as many workgroups as stand on the chip side by side: rows of
+  // 1024 values and more let five (their LDS, at 8192 values, four) stand on a compute unit, and the others of 2048 come behind them; shorter
+  // ones are done before that counts. Weights from memory, us in 2048 / 1280 workgroups: 256 values to 14000 and 50304 outputs 6.4 / 7.0, 14.0 /
+  // 16.6, 768 to 8500, 20480 and 50304 8.2 / 7.6, 12.1 / 13.1, 27.0 / 28.2, 1024 to those 9.4 / 8.4, 16.0 / 15.7, 36.2 / 35.1, 2048 to 8500
+  // and 50304 18.1 / 16.8, 81 / 70, 4096 to 14000 51 / 44; 8192 to 8500 and 14000 in 2048 / 1280 / 1024 86 / 84 / 73, 108 / 126 / 102. (As many
+  // outputs a wave as any other or one less: 8192 to 14000 in 1167 134.)
+  const int most = K < 1024 ? 2048 : (K + 4) * 4 <= 160 * 1024 / 5 ? 1280 : 1024;
+  auto blocks = [&](int N) {
+    const int all = (N + 3) / 4;
+    return all > 2048 ? most : all;
   };
   const lga::F32NormLinears a{x, K, {{nw1, nb1, eps1, w1, b1, act1, y1, N1, blocks(N1)}, {nw2, nb2, eps2, w2, b2, act2, y2, N2, blocks(N2)}}};
   const unsigned grid = (unsigned)(blocks(N1) + blocks(N2));

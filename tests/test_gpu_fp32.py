@@ -108,6 +108,27 @@ def test_one_row_norms_and_products(K, N1, N2, bias):
     assert torch.equal(ops.f32_linears_sum(x, linears[0], x2, wide, res), want)
 
 
+@pytest.mark.parametrize("K", [4, 1020, 1024, 8188, 8192])
+def test_one_row_of_more_outputs_than_waves(K):
+    """The outputs of 2048 workgroups and one more, and of three rounds of the fewest that longer rows take, bit by bit: rows on both
+    sides of what decides how many workgroups there are."""
+    from types import SimpleNamespace as Part
+
+    from lit_gpt import ops
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(K)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev)  # noqa: E731
+    x, norm = draw(1, K), Part(weight=draw(K), bias=draw(K), eps=1e-5)
+    whole = Part(weight=draw(16389, K) * K ** -0.5, bias=draw(16389))
+    want = ops.f32_linear(ops.layernorm(x, norm.weight, norm.bias, norm.eps), whole.weight, whole.bias)
+    for N in (8192, 8193, 8197, 16389):
+        linear = Part(weight=whole.weight[:N], bias=whole.bias[:N])
+        other = Part(weight=whole.weight[-5:], bias=None)
+        first, second = ops.f32_norm_linears(x, (norm, linear, None), (norm, other, None))
+        assert torch.equal(first, want[:, :N]) and torch.equal(second + whole.bias[-5:], want[:, -5:])
+
+
 def test_one_token_past_the_modules():
     """A block's three launches give the bits of its modules called one by one (a hook keeps them apart), behind up to 64 keys."""
     from generate.base import build_model
