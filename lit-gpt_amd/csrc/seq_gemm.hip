@@ -349,15 +349,19 @@ int gemm_launch(const LinArgs& p, const GemmPlan& plan, int batch, hipStream_t s
 // 32 rows and up to 32 columns by one wave, eight steps ahead: a router's logits, whole in K. The sums are those of the tiles above, to the
 // same bits, but there are more workgroups and none of their waves works on columns that are not there. Bound by the latency of a step.
 // us, the tiles of 64 x 128 / here: 2048 x 18 x 2048 13.8 / 10.4 (in a model's prompt 16.4 / 12.0), 4096 x 16 x 2048 14.0 / 10.8, 2407 x 16
-// x 4096 23.0 / 17.2, 300 x 32 x 1024 8.7 / 6.7; past 8192 rows both have work for the chip (16000 x 18 x 2048 16.3 / 17.7). With the
-// operands in registers as the instructions take them 9.9 and 16.0, but only for K a multiple of 512.
+// x 4096 23.0 / 17.2, 300 x 32 x 1024 8.7 / 6.7; past 8192 rows both have work for the chip (16000 x 18 x 2048 16.3 / 17.7), the rows of
+// all batches together (4 of 8192 x 32 x 64 4.8 / 6.1, 64 of 512 x 16 x 512 9.1 / 12.7), or 16384 where there are few batches or K is short
+// (8 of 2048 x 16 x 2048 15.3 / 13.9, 16 of 1024 15.4 / 14.4, 64 of 256 x 16 x 512 6.9 / 5.2; x 32 x 1024 9.9 / 13.0). With the operands
+// in registers as the instructions take them 9.9 and 16.0, but only for K a multiple of 512.
 __global__ void __launch_bounds__(64) gemm_narrow_kernel(LinArgs p) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[GemmTile<1, 1, 1, 1, 8, 8>::LDS];
   gemm_rows<1, 1, 1, 1, 8, 8, true, true>(p, lds, blockIdx.y, 0, 0, p.M, blockIdx.x * 32, 0);
 }
 
 bool gemm_narrow(const LinArgs& p, int batch, hipStream_t stream) {
-  if (p.N > 32 || p.M > 8192 || p.K % 64 != 0 || p.ksplit > 1 || p.z_start) return false;
+  const long rows = (long)p.M * batch;
+  const bool idle = p.M <= 8192 && (rows <= 8192 || (rows <= 16384 && (batch <= 16 || p.K <= 512)));
+  if (p.N > 32 || !idle || p.K % 64 != 0 || p.ksplit > 1 || p.z_start) return false;
   gemm_narrow_kernel<<<dim3((p.M + 31) / 32, batch), 64, 0, stream>>>(p);
   return true;
 }
