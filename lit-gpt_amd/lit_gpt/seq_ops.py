@@ -284,8 +284,12 @@ def decay_map_inside(proj: torch.Tensor, off: int, w_a2: torch.Tensor, *, H: int
 
 
 def gate_map_inside(proj: torch.Tensor, off: int, w_g2: torch.Tensor, *, H: int, dv: int) -> bool:
-    """Whether ``head_gate`` makes the second map of a prompt's gates itself, to the bits of the product."""
-    return dv == 128 and proj.shape[0] > 8 and proj.shape[0] * H >= 4096 and _map_fits(proj, off, w_g2)
+    """Whether ``head_gate`` makes the second map of a prompt's gates itself, to the bits of the product. Its workgroups read a head's part
+    of the map for 16 tokens each, so long maps of many heads' tokens stay products. us, a product and the gate / inside: 32 heads of
+    256 values, 2048 tokens 55 / 49, 4096 94 / 89; of 384, 1500 tokens 52.0 / 51.2, 2048 60.8 / 65.7; of 512, 1024 tokens 50 / 46, 2048
+    67 / 82, 4096 122 / 156; 48 of 320, 2048 tokens 85 / 82, 4096 144 / 156."""
+    pairs = proj.shape[0] * H
+    return dv == 128 and proj.shape[0] > 8 and pairs >= 4096 and (w_g2.shape[1] - 192) * pairs <= 11 << 20 and _map_fits(proj, off, w_g2)
 
 
 def head_gate(o: torch.Tensor, proj: torch.Tensor, g_off: int, *, H: int, dv: int, unit_norm: bool, eps: float,

@@ -54,3 +54,15 @@ def test_maps_off_sixteen_bytes_stay_products():
     for args in ((proj, 3, w), (proj[:, :126].contiguous(), 4, w), (proj, 4, w[:, :60].contiguous()), (proj, 4, w.float())):
         assert not seq_ops.decay_map_inside(*args, H=16, d=128) and not seq_ops.gate_map_inside(*args, H=16, dv=128)
     assert not seq_ops.decay_map_inside(proj[:64], 4, w, H=16, d=128) and not seq_ops.gate_map_inside(proj[:255], 4, w, H=16, dv=128)
+
+
+def test_long_maps_of_many_tokens_stay_products():
+    """Both sides of the line, where the gate makes the map of rows that share it with others, and where a product does."""
+    from lit_gpt import seq_ops
+
+    def inside(T, H, rank):
+        proj, w = torch.empty(T, rank, device=DEV), torch.empty(H * 128, rank, dtype=torch.bfloat16, device=DEV)
+        return seq_ops.gate_map_inside(proj, 0, w, H=H, dv=128)
+
+    assert inside(16384, 32, 192) and inside(5632, 32, 256) and inside(1024, 32, 512)
+    assert not inside(5633, 32, 256) and not inside(2048, 32, 384) and not inside(1127, 32, 512)
