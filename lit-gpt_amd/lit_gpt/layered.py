@@ -788,9 +788,16 @@ class LayeredGPT(nn.Module):
                 after_layer(run, x)
         return x
 
-    # Values of a stream from which prompts hold their streams: shorter ones wait for the host, whose share is the larger then (a step
-    # of 100 tokens of 2048 columns 589 us stored, 620 held; of 1050 1366 stored, 1297 held with all else that made it faster)
+    # A prompt whose streams have more values than these each holds them: shorter ones wait for the host, which does more for a boundary
+    # that holds. us a step of the layers above 2048 columns, stored / held: 4 streams, 100 tokens 588 / 610, 200 638 / 662, 257 654 / 639,
+    # 1050 1361 / 1326, 2400 2321 / 2189 (captured, without the host, 463 / 447, 555 / 533, 618 / 591, 1331 / 1316, 2247 / 2127), of 4096 129
+    # tokens 1006 / 942. Two streams are two rows of four that are not moved, and of 2048 columns gain nothing below eight times as many:
+    # ten layers, 257 tokens 1598 / 1616, 800 2998 / 2991, 2400 4537 / 4445; of 4096 columns 129 tokens 1734 / 1715.
     HELD_FROM = 1 << 19
+
+    def _holds(self, T: int) -> bool:
+        W, s = self.config.width, self.config.streams
+        return T * W > self.HELD_FROM * (8 if s == 2 and W <= 2048 else 1) and seq_ops.streams_hold(T, W, s, False) > 0
 
     def _forward_streams(self, step: StepBatch, after_layer=None) -> torch.Tensor:
         """The sequential layers over the residual streams. Every boundary between two sublayers is one launch: the
@@ -800,9 +807,7 @@ class LayeredGPT(nn.Module):
         eps = self.config.norm_eps
         chain = [(run, sub, self.caches[run] if k == 0 else None)
                  for run, layer in enumerate(self.runs) for k, sub in enumerate(self.blocks[layer].sublayers())]
-        if after_layer is None and step.T * self.config.width > self.HELD_FROM and \
-                seq_ops.streams_hold(step.T, self.config.width, self.config.streams, False) and \
-                not any(hooked(sub, sub.module) for _, sub, _ in chain):
+        if after_layer is None and self._holds(step.T) and not any(hooked(sub, sub.module) for _, sub, _ in chain):
             return self._forward_held(step, chain)
         x = seq_ops.embed_streams(step.tokens, self.embed, self.config.embedding_scale, self.config.streams)
         first = chain[0][1]

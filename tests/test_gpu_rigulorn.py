@@ -681,3 +681,26 @@ def test_prompt_whose_streams_are_not_stored(streams, dtype, T, monkeypatch):
         handle.remove()
         assert set(calls[len(calls) // 2:]) == {"step"}
     assert torch.equal(got, hooked)
+
+
+@pytest.mark.parametrize("streams,eighths", [(2, 8), (3, 1), (4, 1)])
+def test_line_between_stored_and_held_streams(streams, eighths, monkeypatch):
+    """The last prompt whose streams are stored and the first whose are held, by the rule's own line: eight times as far for two narrow
+    streams."""
+    from lit_gpt import seq_ops
+    from lit_gpt.layered import LayeredGPT
+    from lit_gpt.mixers import StepBatch
+
+    cfg = make_cfg(MIXED, streams=streams)
+    model, _ = build(cfg)
+    W, calls = model.config.width, []
+    monkeypatch.setattr(LayeredGPT, "HELD_FROM", 64 * W // eighths)
+    held, step = seq_ops.streams_held, seq_ops.streams_step
+    monkeypatch.setattr(seq_ops, "streams_held", lambda *a, **k: calls.append("held") or held(*a, **k))
+    monkeypatch.setattr(seq_ops, "streams_step", lambda *a, **k: calls.append("step") or step(*a, **k))
+    model.set_kv_cache(1, 80)
+    for T, want in ((64, "step"), (65, "held")):
+        with torch.inference_mode():
+            model.forward_step(StepBatch.build([(0, 0, tokens_of(T, cfg["vocab"]))], model.device))
+        assert set(calls) == {want}
+        calls.clear()

@@ -765,3 +765,18 @@ def test_fazolorn_plain_implementation():
     assert u.item() == pytest.approx(0.0)
     u = orc.clamped_feed_forward(one, {"gate": 3 * one, "up": 7 * one, "down": one}, 1.0)
     assert u.item() == pytest.approx(2.0 / (1.0 + math.exp(-1.702)))
+
+
+def test_prompts_that_hold_their_streams():
+    """Which prompts make their residual streams anew: enough values a stream, more of them for two narrow ones; never few rows, one stream,
+    more than four or rows past the kernel's."""
+    from types import SimpleNamespace
+
+    from lit_gpt.layered import LayeredGPT
+
+    def holds(T, W, s):
+        return LayeredGPT._holds(SimpleNamespace(config=SimpleNamespace(width=W, streams=s), HELD_FROM=LayeredGPT.HELD_FROM), T)
+
+    assert not holds(256, 2048, 4) and holds(257, 2048, 4) and holds(257, 2048, 3) and not holds(128, 4096, 2) and holds(129, 4096, 2)
+    assert not holds(2048, 2048, 2) and holds(2049, 2048, 2) and holds(256, 2049, 2)
+    assert not any(holds(5000, W, s) for W, s in ((2048, 1), (2048, 5), (4097, 4)))
