@@ -686,16 +686,26 @@ def streams_step(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, mix: Opti
     return (h, h16) if bf16_copy else h
 
 
+HELD_BYTES = 1 << 30  # of sublayers' outputs that a prompt keeps for its streams
+
+
 def streams_hold(T: int, W: int, streams: int, stored: bool) -> int:
     """After how many sublayers a prompt's streams are stored: until then ``streams_held`` makes them anew (0: every boundary
     stores them, by ``streams_step``). A boundary that stores reads and writes a row per stream, one that does not reads a row per
     sublayer since: with s streams the fewest bytes are moved by storing every sqrt(2 s) sublayers, and, from the embedding, not
-    before 2 s. us of the embedding and nine boundaries of four streams, stored each / held: 2407 rows of 4096 926 / 425, 256 217 / 123,
-    33 197 / 119; of 2048 columns 423 / 277, 142 / 97, 125 / 97; five of two streams of 4096 281 / 139, 81 / 51, 62 / 50. Up to 32 rows
-    keep the step that gives a row 1024 threads."""
+    before 2 s. us of the launches of the embedding and nine boundaries of four streams, stored each / held: 2407 rows of 4096 926 / 425, 256
+    217 / 123, 33 197 / 119; of 2048 columns 423 / 277, 142 / 97, 125 / 97; five of two streams of 4096 281 / 139, 81 / 51, 62 / 50 (what a
+    whole step gains stands with the models' rule). Up to 32 rows keep the step that gives a row 1024 threads.
+
+    The outputs that are held take memory that boundaries which store do not: with four streams up to eight rows of W, and four more where
+    they are stored at last, in place of four and the read in fp32. A step's peak, MB, stored / held, 4096 tokens of 4096 columns: ten layers
+    of attention and feed-forwards with 4 streams 672 / 832, with 3 608 / 640, with 2 544 / 448; where a state-space mixer's own rows are the
+    peak 1122 / 1122. So at most ``HELD_BYTES`` of outputs are held, fewer of longer prompts, and from two on or none: the first of these
+    models at 8192 tokens 1344 / 1664 and 36.5 / 34.3 ms, at 16384, which hold four and then three, 2688 / 2688 and 73.2 / 69.2."""
     if T <= 32 or W > 4096 or not 2 <= streams <= 4:
         return 0
-    return (2 if streams == 2 else 3) if stored else 2 * streams
+    most = HELD_BYTES // (4 * T * W)
+    return min(most, (2 if streams == 2 else 3) if stored else 2 * streams) if most >= 2 else 0
 
 
 class HeldOutputs:

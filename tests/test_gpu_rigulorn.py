@@ -704,3 +704,26 @@ def test_line_between_stored_and_held_streams(streams, eighths, monkeypatch):
             model.forward_step(StepBatch.build([(0, 0, tokens_of(T, cfg["vocab"]))], model.device))
         assert set(calls) == {want}
         calls.clear()
+
+
+@pytest.mark.parametrize("streams", [2, 3, 4])
+@pytest.mark.parametrize("most", [2, 3, 5])
+def test_prompt_that_holds_fewer_outputs(streams, most, monkeypatch):
+    """Memory for fewer outputs than move the fewest bytes: the residual of the boundaries that store each time, to the bit."""
+    from lit_gpt import seq_ops
+    from lit_gpt.layered import LayeredGPT
+    from lit_gpt.mixers import StepBatch
+
+    cfg, T = make_cfg(MIXED * 2, streams=streams), 50
+    model, _ = build(cfg)
+    model.set_kv_cache(1, 64)
+    step = StepBatch.build([(0, 0, tokens_of(T, cfg["vocab"]))], model.device)
+    monkeypatch.setattr(seq_ops, "HELD_BYTES", 4 * T * model.config.width * most)
+    counts, one = [], seq_ops.streams_held
+    monkeypatch.setattr(seq_ops, "streams_held", lambda *a, **k: counts.append(len(a[4])) or one(*a, **k))
+    with torch.inference_mode():
+        stored = model.forward_step(step)
+        assert not counts
+        monkeypatch.setattr(LayeredGPT, "HELD_FROM", 0)
+        held = model.forward_step(step)
+    assert max(counts) == min(most, 2 * streams) and torch.equal(stored, held)

@@ -780,3 +780,16 @@ def test_prompts_that_hold_their_streams():
     assert not holds(256, 2048, 4) and holds(257, 2048, 4) and holds(257, 2048, 3) and not holds(128, 4096, 2) and holds(129, 4096, 2)
     assert not holds(2048, 2048, 2) and holds(2049, 2048, 2) and holds(256, 2049, 2)
     assert not any(holds(5000, W, s) for W, s in ((2048, 1), (2048, 5), (4097, 4)))
+
+
+def test_outputs_that_are_held_are_bounded():
+    """As many sublayers' outputs as move the fewest bytes, and never more than HELD_BYTES of them."""
+    from lit_gpt import seq_ops
+
+    assert [seq_ops.streams_hold(8192, 4096, s, False) for s in (1, 2, 3, 4, 5)] == [0, 4, 6, 8, 0]
+    assert [seq_ops.streams_hold(8192, 4096, s, True) for s in (2, 3, 4)] == [2, 3, 3]
+    assert [seq_ops.streams_hold(T, 4096, 4, False) for T in (32, 33, 8193, 16384, 32768, 32769)] == [0, 8, 7, 4, 2, 0]
+    for T in (33, 5000, 10000, 21845, 21846, 32768, 60000):
+        for s in (2, 3, 4):
+            first, later = (seq_ops.streams_hold(T, 4096, s, stored) for stored in (False, True))
+            assert 4 * T * 4096 * max(first, later) <= seq_ops.HELD_BYTES and (first >= 2) == (later >= 2)
