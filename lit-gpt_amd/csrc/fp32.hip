@@ -428,7 +428,7 @@ __global__ void __launch_bounds__(256) f32_norm_linears_kernel(F32NormLinears a)
 // outputs (kept in registers until LDS has them: as an array of HIP's float4 they went through scratch memory, a trip of their own
 // ahead of all weights). Weights from memory, an attention in five ranges, us without / with: 768 columns beside 3072 9.4 / 9.5, 1024
 // beside 4096 10.2 / 9.6, 1600 beside 6400 24.2 / 18.1, 2048 beside 8192 30.0 / 24.3, in one range 23.3 / 18.2; a token behind 300 keys:
-// pythia-160m 292 / 267, pythia-410m 652 / 581, pythia-1b 1109 / 1013. Not where x1 is no shorter than half of x2: 4096 beside 4096 in
+// pythia-160m 292 / 267, pythia-410m 652 / 581, pythia-1b 1109 / 1013. Not where x1 is longer than half of x2: 4096 beside 4096 in
 // five ranges 47.8 / 66.4, 2240 beside 1280 9.8 / 10.3.
 struct F32LinearsSum {
   const float *x1, *w1, *b1, *x2, *w2, *b2, *res;

@@ -367,8 +367,8 @@ __device__ __forceinline__ void lanes_sum2(float& a, float& b) {
 // grid (B * H * ceil(dv / CW) rounded up to 8), CW = 256 / LPC columns per workgroup. Lane l of a wave: r = l % LPC, column
 // l / LPC of the wave's 64 / LPC; the lane holds the rows 4 (r + LPC j) + e, j < NR4, e < 4, of its column.
 // ONE: sequences of one token (of more, too, but slowly): nothing is staged for tokens that do not come, and the state is on its way
-// beside the rows. us, the general form / this, a decay per channel: 8 sequences of 16 heads of 128 x 128 9.3 / 7.1, 3 7.7 / 6.3, 1 4.3 /
-// 3.7, 32 19.9 / 15.1, 8 of 32 heads 11.0 / 8.7, 4 of 4 heads of 256 x 256 8.5 / 6.9, 3 of 512 x 64 11.8 / 10.6.
+// beside the rows. us, the general form / this, a decay per channel: 8 sequences of 16 heads of 128 x 128 9.3 / 7.1, 3 7.7 / 6.3, 32 19.9 /
+// 15.1, 8 of 32 heads 11.0 / 8.7, 4 of 4 heads of 256 x 256 8.5 / 6.9, 3 of 512 x 64 11.8 / 10.6.
 template <int NR4, int LPC, bool DELTA, bool ONE>
 __global__ void __launch_bounds__(256) gated_delta_kernel(DeltaArgs p) {
   constexpr int DP = 4 * NR4 * LPC;      // rows, padded
@@ -1023,6 +1023,8 @@ static int gated_delta_any(const float* qkv, long ld, const float* dec, const fl
   // lanes per column: more lanes shorten a token's dependent chain and multiply the waves; by default as many as
   // keep the launch within about two waves per SIMD, and at least enough for 32 rows per lane
   int lpc = lanes;
+  // Steps of one token take the wide form too, up to its workgroups. us of 128 x 128, wide / ONE with 16 lanes: one sequence of 1 to 16 heads 3.6
+  // to 3.9 / 4.1 to 4.5; past 256 workgroups, two to a CU, three of 8 heads 4.7 / 4.3, two of 16 4.9 / 4.3, one of 32 4.8 / 4.3.
   // (even rows: only they gained; rows below 2^24 floats: eight of them are offsets of 32 bits)
   const bool pairs = ld % 2 == 0 && ld < (1 << 24) && ((uintptr_t)qkv | (uintptr_t)dec) % 8 == 0;
   if (lanes == 0 && d == 128 && pairs && (long)B * H * ((dv + 7) / 8) <= lgs::kDeltaWideItems) {
