@@ -869,12 +869,12 @@ extern "C" int lga_f32_norm_linears(const float* x, int K, const float* nw1, con
   LGA_CHECK_ARG(K % 4 == 0 && K <= 8192 && ((uintptr_t)w1 | (uintptr_t)w2) % 16 == 0,
                 "lga_f32_norm_linears: K a multiple of 4 up to 8192 and 16-B aligned weights needed");
   // One output a wave up to 2048 workgroups. Beyond, a wave makes several, in as many workgroups as stand on the chip side by side: rows of
-  // 1024 values and more let five (their LDS, at 8192 values, four) stand on a compute unit, and the others of 2048 come behind them; shorter
-  // ones are done before that counts. Weights from memory, us in 2048 / 1280 workgroups: 256 values to 14000 and 50304 outputs 6.4 / 7.0, 14.0 /
-  // 16.6, 768 to 8500, 20480 and 50304 8.2 / 7.6, 12.1 / 13.1, 27.0 / 28.2, 1024 to those 9.4 / 8.4, 16.0 / 15.7, 36.2 / 35.1, 2048 to 8500
-  // and 50304 18.1 / 16.8, 81 / 70, 4096 to 14000 51 / 44; 8192 to 8500 and 14000 in 2048 / 1280 / 1024 86 / 84 / 73, 108 / 126 / 102. (As many
-  // outputs a wave as any other or one less: 8192 to 14000 in 1167 134.)
-  const int most = K < 1024 ? 2048 : (K + 4) * 4 <= 160 * 1024 / 5 ? 1280 : 1024;
+  // 1024 values and more let five (past 7996 values four: a workgroup's LDS comes in pieces of 1280 bytes) stand on a compute unit, and the
+  // others of 2048 come behind them; shorter ones are done before that counts. Weights from memory, us in 2048 / 1280 workgroups: 256 values
+  // to 14000 and 50304 outputs 6.4 / 7.0, 14.0 / 16.6, 768 to 8500, 20480 and 50304 8.2 / 7.6, 12.1 / 13.1, 27.0 / 28.2, 1024 to those 9.4 / 8.4,
+  // 16.0 / 15.7, 36.2 / 35.1, 2048 to 8500 and 50304 18.1 / 16.8, 81 / 70, 4096 to 14000 51 / 44; 8192 to 8500 and 14000 in 2048 / 1280 / 1024
+  // 86 / 84 / 73, 108 / 126 / 102, 8188 to 14000 109 / 129 / 104. (As many outputs a wave as any other or one less: 8192 to 14000 in 1167 134.)
+  const int most = K < 1024 ? 2048 : (K + 4) * 4 <= 25 * 1280 ? 1280 : 1024;
   auto blocks = [&](int N) {
     const int all = (N + 3) / 4;
     return all > 2048 ? most : all;
